@@ -115,9 +115,8 @@ int ll_update_kv_index(int32_t* table, const void* b_req_idx, const void* b_seq_
  * 32 floats per (row, head, partition) -- batch * hq * nparts * 32 -- one cache line per record.
  * Same values either way. */
 int ll_flash_decoding_num_partitions(int64_t max_len);
-/* Waves of the one-workgroup-per-(row, KV head) decode form for contexts of up to max_len tokens launched as `workgroups` = batch x
- * KV heads (x head groups) workgroups (2 .. 8 partitions: a wave per partition; more: 8 waves that walk the partitions, when the
- * launch has >= 128 workgroups); 0: the form does not apply -- ll_decode_attention_partials needs it. */
+/* Waves of a workgroup where ll_decode_attention_partials serves contexts of up to max_len tokens at `workgroups` = batch x KV heads
+ * (x head groups) pairs: 2 .. 8 partitions a wave per partition, more (>= 64 pairs) 8 waves that walk the partitions; 0: not served. */
 int ll_flash_decoding_group_waves(int64_t max_len, int64_t workgroups);
 int ll_flash_decoding(void* out, const void* q, const void* k_cache, const void* v_cache,
                       const int32_t* table, const void* b_req_idx, const void* b_seq_len,
@@ -154,7 +153,8 @@ int ll_decode_attention(void* out, const void* q, const void* kv_new, int64_t kv
 /* ll_decode_attention whose q / k_new / v_new arrive as the fp32 split-K partials [s_count][batch][(hq + 2 hkv) * d] of the
  * fused q|k|v projection (ll_w4a16_matmul_prepacked epilogue 2) plus the projection bias (or NULL): every workgroup adds
  * the partials of its (row, KV head), rounds once to the pool dtype -- the value the projection would have stored -- and
- * continues as ll_decode_attention.  Contexts of 2..8 partitions (129..1024 tokens); LL_ERR_SHAPE otherwise.
+ * continues as ll_decode_attention.  Served where ll_flash_decoding_group_waves says so; LL_ERR_SHAPE otherwise.
+ * mid_o / mid_lse / counters as for ll_decode_attention: needed past 8 partitions below 128 (row, KV head) pairs, else NULL.
  * int32_a_scale [batch] / int32_w_scale [row width] (both or both NULL; fp16, d == 128): the planes are the exact int32 sums
  * of a smoothquant projection (ll_dense_partials wfmt 3); the value summed is fp16(((float)sum * a_scale[row]) * w_scale[col]
  * (+ bias)), what ll_w8a8_matmul stores. */
@@ -166,7 +166,8 @@ int ll_decode_attention_partials(void* out, const float* qkv_partials, int s_cou
                                  int64_t v_stride_t, int64_t v_stride_h, int64_t o_stride_b, int64_t o_stride_h,
                                  int64_t table_stride_b, int dtype, int req_width, int seq_width,
                                  const void* q_norm_weight, const void* k_norm_weight, float norm_eps,
-                                 const float* int32_a_scale, const float* int32_w_scale, void* stream);
+                                 const float* int32_a_scale, const float* int32_w_scale, float* mid_o, float* mid_lse,
+                                 int32_t* counters, void* stream);
 
 /* ---- a6: flash_attention2_no_pad  (kernels/flashattention2_nopad.py:175-231) --
  * Varlen causal prefill over freshly projected q/k/v (exp2 softmax; sm_scale

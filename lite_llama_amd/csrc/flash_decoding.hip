@@ -247,7 +247,10 @@ __global__ __launch_bounds__(GROUPED ? 64 * FD_GROUP_MAX : 64) void fd_stage1(
   const int wave = GROUPED ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : 0;
   uint16_t* lds_v = lds_all + wave * (32 * VSTR);  // this wave's V staging tile
   const int t = lane & 15, c = lane >> 4;
-  const int part = GROUPED ? wave : (int)blockIdx.x;
+  // GROUPED: gridDim.x workgroups share a row's partitions (1 unless the launch would leave most of the chip idle, fd_plan): wave
+  // ``part`` of all of them walks partitions part, part + walkers, ...
+  const int walkers = GROUPED ? (int)(gridDim.x * (blockDim.x >> 6)) : 1;
+  const int part = GROUPED ? (int)(blockIdx.x * (blockDim.x >> 6)) + wave : (int)blockIdx.x;
   const int kvh = blockIdx.y % hkv;
   const int hg = blockIdx.y / hkv;
   const int b = blockIdx.z;
@@ -342,8 +345,20 @@ __global__ __launch_bounds__(GROUPED ? 64 * FD_GROUP_MAX : 64) void fd_stage1(
 
   // (requested together: the table row address needs req, the partition bounds need seq_len -- one round trip, not two)
   const int64_t req = fd_load_idx(b_req_idx, b, req_w);
-  const int64_t seq_len = fd_load_idx(b_seq_len, b, seq_w);
-  int64_t start = (int64_t)part * FD_PART;  // (GROUPED: the wave's FIRST partition; it walks part, part + waves, ... below)
+  int64_t seq_len = fd_load_idx(b_seq_len, b, seq_w);
+  // (a stale / too small max length: there may be more walkers than launched partitions, and none reads past them)
+  if (GROUPED && seq_len > (int64_t)nparts * FD_PART) seq_len = (int64_t)nparts * FD_PART;
+  // Tokens of a partition.  Where several workgroups share a row they share it evenly, in tiles of 32 (27 rows of 1500 - 3000 tokens on
+  // 4 x 8 waves: 96 each and no second walk; 718 us a step against 741 with 128); one workgroup keeps whole partitions, where smaller
+  // ones lost (batch 1 x ctx 300: 697 -> 712 us, batch 64 x ctx 700: 972 -> 981).
+  int ptok = FD_PART;
+  if constexpr (GROUPED) {
+    if (gridDim.x > 1 && seq_len < (int64_t)walkers * FD_PART) ptok = (((int)seq_len + walkers * 32 - 1) / (walkers * 32)) * 32;
+  }
+  int64_t start = (int64_t)part * ptok;  // (GROUPED: the wave's FIRST partition; it walks part, part + walkers, ... below)
+  if constexpr (GROUPED) {
+    if (blockIdx.x > 0 && start - (int64_t)wave * ptok >= seq_len) return;  // a split past the row's end: no wave has work, none merges
+  }
   if (start >= seq_len) {  // empty partition stores nothing (flashdecoding.py:141-161)
     publish_q();
     if constexpr (FUSE) {
@@ -354,10 +369,12 @@ __global__ __launch_bounds__(GROUPED ? 64 * FD_GROUP_MAX : 64) void fd_stage1(
         for (int dd = c; dd < D; dd += 4) out[b * o_sb + (int64_t)head * o_sh + dd] = from_f32<DT>(nan);
       }
     }
-    if constexpr (GROUPED) __syncthreads();  // the workgroup's one barrier (the waves with tokens meet here before the merge)
-    return;
+    if constexpr (!GROUPED) return;
   }
-  int64_t end = seq_len < start + FD_PART ? seq_len : start + FD_PART;
+  const bool live = start < seq_len;  // (GROUPED: waves without tokens still merge)
+  if (GROUPED && !live) __syncthreads();
+  if (!GROUPED || live) {
+  int64_t end = seq_len < start + ptok ? seq_len : start + ptok;
   const int32_t* trow = table + req * t_sb;
   // Pool rows of the whole partition, requested now (the K/V gathers depend on them; everything up to the first
   // gather overlaps this round trip)
@@ -402,9 +419,10 @@ __global__ __launch_bounds__(GROUPED ? 64 * FD_GROUP_MAX : 64) void fd_stage1(
     }
     // the new token lives in the last non-empty partition; head group 0 owns the write
     // (clamped to the launched partitions: a stale / too small max length then still stores the row)
-    const int wpart = (int)((seq_len - 1) / FD_PART) < nparts - 1 ? (int)((seq_len - 1) / FD_PART) : nparts - 1;
+    const int wpart = GROUPED ? (int)(seq_len - 1) / ptok
+                              : (int)((seq_len - 1) / FD_PART) < nparts - 1 ? (int)((seq_len - 1) / FD_PART) : nparts - 1;
     // (GROUPED with more partitions than waves: the wave that WILL gather partition wpart -- it is its only reader -- writes now)
-    if (hg == 0 && (GROUPED ? wave == wpart % (int)(blockDim.x >> 6) : part == wpart)) {
+    if (hg == 0 && (GROUPED ? part == wpart % walkers : part == wpart)) {
       const int64_t dstrow = fd_load_idx(rp.sel, b, rp.sel_w);
       const uint16_t* kn = qpart ? q_lds + groups * D : rp.kv_new + b * rp.kv_rs + (int64_t)kvh * D;
       const uint16_t* vn = qpart ? q_lds + groups * D + D : rp.kv_new + b * rp.kv_rs + (int64_t)(hkv + kvh) * D;
@@ -686,10 +704,7 @@ __global__ __launch_bounds__(GROUPED ? 64 * FD_GROUP_MAX : 64) void fd_stage1(
     // Contexts of more partitions than waves (round 6): the wave walks partitions part + W, part + 2 W, ... with the SAME running
     // maximum / denominator / accumulators -- the online softmax does not care where a partition ends -- so the one-workgroup form
     // (partials of the q|k|v projection summed in the prologue, merge through LDS, no global round trip) serves any context.
-    const int W_ = (int)(blockDim.x >> 6);
-    for (int pn = part + W_; pn < nparts; pn += W_) {
-      const int64_t st_ = (int64_t)pn * FD_PART;
-      if (st_ >= seq_len) break;
+    for (int64_t st_ = start + (int64_t)walkers * FD_PART; st_ < seq_len; st_ += (int64_t)walkers * FD_PART) {  // (only with whole partitions)
       start = st_;
       end = seq_len < start + FD_PART ? seq_len : start + FD_PART;
       const int64_t last_ = end - 1;
@@ -714,13 +729,11 @@ __global__ __launch_bounds__(GROUPED ? 64 * FD_GROUP_MAX : 64) void fd_stage1(
 #undef FD_WAVE_SYNC
 
   if constexpr (GROUPED) {
-    int np = (int)((seq_len + FD_PART - 1) / FD_PART);  // records = waves with tokens
-    if (np > nparts) np = nparts;
-    if (np > (int)(blockDim.x >> 6)) np = (int)(blockDim.x >> 6);
     constexpr int REC = 32 * VSTR / 2;  // floats per wave record: [16 heads][D] normalised partial + [16] log-sum-exp
-    if (np > 1 && head_ok) {
+    if (head_ok) {
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the last tile's V reads are done: the tile becomes the record
       float* rec = reinterpret_cast<float*>(lds_v);
+      static_assert(REC * 4 == 32 * VSTR * 2, "a record is a wave's V tile");
       const float inv = (KV8 ? rp.v_scale : 1.0f) / d_i;
 #pragma unroll
       for (int dt = 0; dt < NT; ++dt) {
@@ -731,56 +744,7 @@ __global__ __launch_bounds__(GROUPED ? 64 * FD_GROUP_MAX : 64) void fd_stage1(
       if (c == 0) rec[16 * D + t] = m_i * 0.69314718055994530942f + logf(d_i);
     }
     __syncthreads();
-    if (wave != 0) return;
-    if (np == 1) {
-      // single partition: stage 2 computes (0*0 + 1*(o/d)) / (0*0 + 1) -- the same value
-      if (!head_ok) return;
-      uint16_t* orow = out + b * o_sb + (int64_t)head * o_sh + 4 * c;
-      const float inv = (KV8 ? rp.v_scale : 1.0f) / d_i;
-#pragma unroll
-      for (int dt = 0; dt < NT; ++dt) {
-        uint16_t o4[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) o4[e] = from_f32<DT>(ot[dt][e] * inv);
-        *reinterpret_cast<uint2*>(orow + dt * 16) =
-            uint2{(uint32_t)o4[0] | ((uint32_t)o4[1] << 16), (uint32_t)o4[2] | ((uint32_t)o4[3] << 16)};
-      }
-      return;
-    }
-    // merge the np records in partition order: the recurrence of fd_stage2, element by element (same values as
-    // the global-memory merge below and as the two-launch form)
-    constexpr int D4 = D / 4;
-    constexpr int NSL = (GS * D4 + 63) / 64;
-    const int nvalid = groups - hg * 16 < 16 ? groups - hg * 16 : 16;
-    uint16_t* out_g = out + b * o_sb + (int64_t)(kvh * groups + hg * 16) * o_sh;
-    const float* recs = reinterpret_cast<const float*>(lds_all);
-#pragma unroll
-    for (int j = 0; j < NSL; ++j) {
-      const int sidx = lane + 64 * j;
-      const int hl_s = sidx / D4, d4 = sidx % D4;
-      if (hl_s >= nvalid) continue;
-      float mm = -INFINITY, dd = 0.f;
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-      for (int pp = 0; pp < np; ++pp) {
-        const float* rec = recs + pp * REC;
-        const f32x4 v = *reinterpret_cast<const f32x4*>(rec + hl_s * D + d4 * 4);
-        const float l = rec[16 * D + hl_s];
-        const float m_new = fmaxf(mm, l);
-        const float alpha = expf(mm - m_new), w = expf(l - m_new);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc[e] = acc[e] * alpha + w * v[e];
-        dd = dd * alpha + w;
-        mm = m_new;
-      }
-      uint16_t o4[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) o4[e] = from_f32<DT>(acc[e] / dd);
-      *reinterpret_cast<uint2*>(out_g + (int64_t)hl_s * o_sh + d4 * 4) =
-          uint2{(uint32_t)o4[0] | ((uint32_t)o4[1] << 16), (uint32_t)o4[2] | ((uint32_t)o4[3] << 16)};
-    }
-    return;
-  }
-  if constexpr (!FUSE) {
+  } else if constexpr (!FUSE) {
     if (head_ok) {
       const float inv = (KV8 ? rp.v_scale : 1.0f) / d_i;
       float* mo = mid_o + (((int64_t)b * hq + head) * nparts + part) * D;
@@ -909,6 +873,107 @@ __global__ __launch_bounds__(GROUPED ? 64 * FD_GROUP_MAX : 64) void fd_stage1(
           uint2{(uint32_t)o4[0] | ((uint32_t)o4[1] << 16), (uint32_t)o4[2] | ((uint32_t)o4[3] << 16)};
     }
   }
+  }  // (the waves with tokens)
+
+  if constexpr (GROUPED) {
+    // Merge of the workgroup's records, in partition order, with the recurrence of fd_stage2 element by element (same values as the
+    // global-memory merge above and as the two-launch form).  EVERY wave merges: heads x D / 4 slots over all threads, so a slot's
+    // serial chain (two expf per record) runs once per thread -- on wave 0 alone it ran 4 times (GQA 7), 1.4 us of the launch's tail.
+    constexpr int D4 = D / 4;
+    constexpr int REC = 32 * VSTR / 2;
+    const int W = (int)(blockDim.x >> 6);
+    const int np = seq_len > 0 ? ((int)seq_len + ptok - 1) / ptok : 0;
+    const int first = (int)blockIdx.x * W;
+    const int nrec = np - first < W ? np - first : W;                 // waves of this workgroup with tokens
+    const int splits = (np + W - 1) / W < (int)gridDim.x ? (np + W - 1) / W : (int)gridDim.x;  // workgroups of this row with tokens
+    const int nvalid = groups - hg * 16 < 16 ? groups - hg * 16 : 16;
+    const int head0 = kvh * groups + hg * 16;
+    uint16_t* out_g = out + b * o_sb + (int64_t)head0 * o_sh;
+    const float* recs = reinterpret_cast<const float*>(lds_all);
+    if (np == 0) return;                                              // (a zero-length row: its 0/0 is written above)
+    const int64_t hr0 = ((int64_t)b * hq + head0) * nparts + blockIdx.x;  // this split's record of the group's first head
+    for (int sidx = (int)threadIdx.x; sidx < nvalid * D4; sidx += (int)blockDim.x) {
+      const int hl_s = sidx / D4, d4 = sidx % D4;
+      float mm = -INFINITY, dd = 0.f;
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+      for (int pp = 0; pp < nrec; ++pp) {
+        const float* rec = recs + pp * REC;
+        const f32x4 v = *reinterpret_cast<const f32x4*>(rec + hl_s * D + d4 * 4);
+        const float l = rec[16 * D + hl_s];
+        const float m_new = fmaxf(mm, l);
+        const float alpha = expf(mm - m_new), w = expf(l - m_new);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] = acc[e] * alpha + w * v[e];
+        dd = dd * alpha + w;
+        mm = m_new;
+      }
+      if (splits == 1) {
+        uint16_t o4[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o4[e] = from_f32<DT>(acc[e] / dd);
+        *reinterpret_cast<uint2*>(out_g + (int64_t)hl_s * o_sh + d4 * 4) =
+            uint2{(uint32_t)o4[0] | ((uint32_t)o4[1] << 16), (uint32_t)o4[2] | ((uint32_t)o4[3] << 16)};
+      } else {
+        // the split's own normalised partial and log-sum-exp, written through (agent scope) for the workgroup that arrives last
+        unsigned long long* mo = reinterpret_cast<unsigned long long*>(mid_o + (hr0 + (int64_t)hl_s * nparts) * D + d4 * 4);
+#pragma unroll
+        for (int e = 0; e < 4; e += 2) {
+          const float lo = acc[e] / dd, hi = acc[e + 1] / dd;
+          __hip_atomic_store(mo + e / 2, (unsigned long long)__float_as_uint(lo) | ((unsigned long long)__float_as_uint(hi) << 32),
+                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (d4 == 0)
+          __hip_atomic_store(mid_lse + (hr0 + (int64_t)hl_s * nparts) * FD_LSE_PAD, mm + logf(dd), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+    if (splits == 1) return;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's records are out ..
+    __syncthreads();                                   // .. and every thread's, before the counter moves
+    int* lds_old = reinterpret_cast<int*>(lds_all);    // (the wave records were read before the barrier)
+    if (threadIdx.x == 0) {
+      int32_t* ctr = counters + (int64_t)b * gridDim.y + blockIdx.y;
+      const int old = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (old == splits - 1) __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // ready for the next launch
+      *lds_old = old;
+    }
+    __syncthreads();
+    if (*lds_old != splits - 1) return;
+    const int64_t hra = ((int64_t)b * hq + head0) * nparts;
+    for (int sidx = (int)threadIdx.x; sidx < nvalid * D4; sidx += (int)blockDim.x) {
+      const int hl_s = sidx / D4, d4 = sidx % D4;
+      float mm = -INFINITY, dd = 0.f;
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+      constexpr int PB = 8;  // records requested together: one memory round trip per eight splits
+      for (int p0 = 0; p0 < splits; p0 += PB) {
+        unsigned long long v[PB][2];
+        float l[PB];
+#pragma unroll
+        for (int u = 0; u < PB; ++u) {
+          const int64_t rr = hra + (int64_t)hl_s * nparts + (p0 + u < splits ? p0 + u : splits - 1);  // clamped; dropped below
+          const unsigned long long* mo = reinterpret_cast<const unsigned long long*>(mid_o + rr * D + d4 * 4);
+          v[u][0] = __hip_atomic_load(mo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          v[u][1] = __hip_atomic_load(mo + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          l[u] = __hip_atomic_load(mid_lse + rr * FD_LSE_PAD, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+#pragma unroll
+        for (int u = 0; u < PB; ++u) {
+          if (p0 + u >= splits) break;
+          const float m_new = fmaxf(mm, l[u]);
+          const float alpha = expf(mm - m_new), w = expf(l[u] - m_new);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            acc[e] = acc[e] * alpha + w * __uint_as_float((uint32_t)(v[u][e >> 1] >> (32 * (e & 1))));
+          dd = dd * alpha + w;
+          mm = m_new;
+        }
+      }
+      uint16_t o4[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o4[e] = from_f32<DT>(acc[e] / dd);
+      *reinterpret_cast<uint2*>(out_g + (int64_t)hl_s * o_sh + d4 * 4) =
+          uint2{(uint32_t)o4[0] | ((uint32_t)o4[1] << 16), (uint32_t)o4[2] | ((uint32_t)o4[3] << 16)};
+    }
+  }
 }
 
 // grid = (hq, batch), block = D threads
@@ -953,18 +1018,29 @@ __global__ void fd_stage2(uint16_t* __restrict__ out, const float* __restrict__ 
 extern "C" int ll_flash_decoding_num_partitions(int64_t max_len) {
   return (int)((max_len + FD_PART - 1) / FD_PART);
 }
-// Waves of the one-workgroup-per-(row, KV head group) decode form for contexts of up to max_len tokens, launched as `workgroups`
-// = batch x KV heads x head groups workgroups; 0: the form does not apply.  Up to FD_GROUP_MAX partitions: a wave per partition
-// (whatever the batch: round 2's measurement).  More (round 6): FD_GROUP_MAX waves that walk the partitions -- taken when the
-// launch alone fills half the chip (128 workgroups); smaller batches keep a workgroup per partition + the counter merge, which
-// spreads ONE row's context over many CUs.
+// The grouped decode form for contexts of up to max_len tokens, (batch x KV heads x head groups) = `workgroups` (row, group) pairs:
+// waves per workgroup and workgroups per pair; {0, 0}: the form does not apply.  Up to FD_GROUP_MAX partitions: one workgroup, a
+// wave per partition.  More: FD_GROUP_MAX waves that walk the partitions, in ONE workgroup where the pairs alone fill half the chip,
+// else in as many as bring the launch to one workgroup per CU.  (A one-wave workgroup per partition, whose last arriver merges every
+// partition's record from memory by itself, took
+// 49 us where this form takes 27: 27 rows of 1500 - 3000 tokens, 2 KV heads of 128, bf16.)
 #define FD_LOOP_MAX 256  // partitions (32 768 tokens)
-extern "C" int ll_flash_decoding_group_waves(int64_t max_len, int64_t workgroups) {
-  static const bool no_loop = getenv("LL_FD_NO_LOOP") != nullptr;  // A/B knob, read once
+struct FdPlan {
+  int waves, splits;
+};
+static FdPlan fd_plan(int64_t max_len, int64_t workgroups) {
   const int64_t np = (max_len + FD_PART - 1) / FD_PART;
-  if (np < 2) return 0;
-  if (np <= FD_GROUP_MAX) return (int)np;
-  return (!no_loop && np <= FD_LOOP_MAX && workgroups >= 128) ? FD_GROUP_MAX : 0;
+  if (np < 2 || np > FD_LOOP_MAX || workgroups < 1) return {0, 0};
+  if (np <= FD_GROUP_MAX) return {(int)np, 1};
+  if (workgroups >= 128) return {FD_GROUP_MAX, 1};
+  const int64_t most = (np + FD_GROUP_MAX - 1) / FD_GROUP_MAX, fill = 256 / workgroups;
+  return {FD_GROUP_MAX, (int)(most < fill ? most : fill)};
+}
+// Waves of a workgroup where the grouped form also takes q|k|v as split-K partials (every workgroup of a pair adds them up again:
+// past FD_GROUP_MAX partitions that is declined below 64 pairs); 0: it does not.
+extern "C" int ll_flash_decoding_group_waves(int64_t max_len, int64_t workgroups) {
+  const FdPlan pl = fd_plan(max_len, workgroups);
+  return pl.splits > 1 && workgroups < 64 ? 0 : pl.waves;
 }
 
 template <int DT>
@@ -986,13 +1062,13 @@ static int launch_fd(void* out, const void* q, const void* kc, const void* vc, c
   rp.v_scale = v_scale;
   const bool qkn = rope && (rp.qnw || rp.knw);
   if (qkn && (!rp.qnw || !rp.knw || d != 128 || kv8 || !(rp.nrm_eps >= 0.f))) return LL_ERR_SHAPE;
-  const int gw = ll_flash_decoding_group_waves(max_len, (int64_t)batch * hkv * hgroups);  // waves of a grouped workgroup; 0: not grouped
-  const bool grouped_ok = fuse && gw >= 2;
+  const FdPlan plan = fd_plan(max_len, (int64_t)batch * hkv * hgroups);
+  const int gw = plan.waves;  // waves of a grouped workgroup; 0: not grouped
+  const bool grouped_ok = fuse && gw >= 2 && (plan.splits == 1 || (mid_o && mid_lse));
   // split-K partial inputs need the grouped form and two float4 slots per lane: (groups + 2) * d / 4 <= 2 * 64 * waves
   static const bool ungrouped_env = getenv("LL_FD_UNGROUPED") != nullptr;  // A/B knob, read once
   if (rope && rp.qp && (!grouped_ok || rp.qs < 1 || rp.qs > FD_QS_MAX || (groups + 2) * d / 4 > 128 * gw || ungrouped_env))
     return LL_ERR_SHAPE;
-  // one workgroup per (row, KV head group) with a wave per partition while the context fits FD_GROUP_MAX partitions
   const bool grouped = grouped_ok && !ungrouped_env;
 #define LL_FD1X(DD, FU, RO, GG, GR) LL_FD1XK(DD, FU, RO, GG, GR, false, false, false)
 #define LL_FD1XK(DD, FU, RO, GG, GR, K8, QN, QI)                                                            \
@@ -1006,7 +1082,7 @@ static int launch_fd(void* out, const void* q, const void* kc, const void* vc, c
         attr_ = true;                                                                                \
       }                                                                                              \
     }                                                                                                \
-    fd_stage1<DT, DD, FU, RO, GG, GR, K8, QN, QI><<<(GR) ? dim3(1, grid.y, grid.z) : grid, (GR) ? 64 * gw : 64, \
+    fd_stage1<DT, DD, FU, RO, GG, GR, K8, QN, QI><<<(GR) ? dim3((unsigned)plan.splits, grid.y, grid.z) : grid, (GR) ? 64 * gw : 64, \
                                         ((GR) ? gw : 1) * tile_bytes_ + ((GR) ? 18 * DD * 2 : 0), st>>>( \
         (const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc, table, req, seq, mid_o, mid_lse, hq, hkv, nparts, \
         scale, q_sb, q_sh, k_st, k_sh, v_st, v_sh, t_sb, req_w, seq_w, (uint16_t*)out, o_sb, o_sh, counters, rp); \
@@ -1193,7 +1269,8 @@ extern "C" int ll_decode_attention_partials(void* out, const float* qkv_partials
                                             int64_t v_stride_h, int64_t o_stride_b, int64_t o_stride_h,
                                             int64_t table_stride_b, int dtype, int req_width, int seq_width,
                                             const void* q_norm_weight, const void* k_norm_weight, float norm_eps,
-                                            const float* int32_a_scale, const float* int32_w_scale, void* stream) {
+                                            const float* int32_a_scale, const float* int32_w_scale, float* mid_o, float* mid_lse,
+                                            int32_t* counters, void* stream) {
   if (!qkv_partials || !cos_t || !sin_t || !positions || !select_index) return LL_ERR_ARG;
   if ((int32_a_scale != nullptr) != (int32_w_scale != nullptr) || !ll_aligned16(int32_w_scale)) return LL_ERR_ARG;
   if ((q_norm_weight != nullptr) != (k_norm_weight != nullptr) || !ll_aligned16(q_norm_weight) || !ll_aligned16(k_norm_weight))
@@ -1202,7 +1279,11 @@ extern "C" int ll_decode_attention_partials(void* out, const float* qkv_partials
   if (cs_row_stride % 8 != 0 || !ll_aligned16(qkv_partials) || !ll_aligned16(cos_t) || !ll_aligned16(sin_t) || d % 4 != 0)
     return LL_ERR_ARG;
   const int64_t row_w = (int64_t)(hq + 2 * hkv) * d;
-  static int32_t dummy_counters = 0;  // the grouped form never touches the counters; fd_entry only wants a non-null pointer
+  static int32_t dummy_counters = 0;  // one workgroup per pair never touches the counters; fd_entry only wants a non-null pointer
+  if (!counters || !mid_o || !mid_lse) {
+    counters = &dummy_counters;
+    mid_o = mid_lse = nullptr;          // (launches that split a pair need them: LL_ERR_SHAPE)
+  }
   FdRope rp{nullptr, 0, (const uint16_t*)cos_t, (const uint16_t*)sin_t, cs_row_stride, positions, select_index,
             sel_width, (uint16_t*)k_cache, (uint16_t*)v_cache, qkv_partials, s_count, (int64_t)batch * row_w, row_w,
             (const uint16_t*)qkv_bias};
@@ -1212,7 +1293,7 @@ extern "C" int ll_decode_attention_partials(void* out, const float* qkv_partials
   rp.q_as = int32_a_scale;
   rp.q_ws = int32_w_scale;
   // q pointer / strides are unused in this mode; pass the pool (aligned, non-null) to satisfy the argument checks
-  return fd_entry(out, k_cache, k_cache, v_cache, table, b_req_idx, b_seq_len, nullptr, nullptr, batch, hq, hkv, d, max_len,
+  return fd_entry(out, k_cache, k_cache, v_cache, table, b_req_idx, b_seq_len, mid_o, mid_lse, batch, hq, hkv, d, max_len,
                   qk_scale, 8, 8, k_stride_t, k_stride_h, v_stride_t, v_stride_h, o_stride_b, o_stride_h, table_stride_b,
-                  dtype, req_width, seq_width, &dummy_counters, &rp, stream);
+                  dtype, req_width, seq_width, counters, &rp, stream);
 }

@@ -190,9 +190,8 @@ def decode_attention(q, kv, cos_table, sin_table, positions, select_index, kv_bu
 
 
 def decode_attention_partials_supported(max_actual_seq_len, num_heads: int, num_kv_heads: int, head_dim: int, batch: int = 1) -> bool:
-    """Whether :func:`decode_attention_partials` serves this step (known before the projection is launched): the
-    one-workgroup-per-(row, KV head) form -- contexts of 129 .. 1024 tokens at any batch, longer ones (round 6: the waves walk the
-    partitions) when ``batch x KV heads`` alone fills half the chip."""
+    """Whether :func:`decode_attention_partials` serves this step (known before the projection is launched): contexts of 129 ..
+    1024 tokens at any batch, longer ones from 64 (row, KV head) pairs."""
     waves = L.lib().ll_flash_decoding_group_waves(int(max_actual_seq_len), int(batch) * int(num_kv_heads))
     return (waves >= 2 and head_dim >= 64 and head_dim % 32 == 0 and num_heads % num_kv_heads == 0
             and num_heads // num_kv_heads <= 16 and (num_heads // num_kv_heads + 2) * head_dim // 4 <= 128 * waves)
@@ -207,7 +206,7 @@ def decode_attention_partials(parts, bias, num_heads: int, num_kv_heads: int, he
     partials of its (row, KV head) -- plus bias, one rounding to the pool dtype: the value the projection itself would
     have stored -- and continues as ``decode_attention`` (``qk_norm`` as there).  ``parts`` may also be the
     ``ScaledInt32Partials`` of a smoothquant projection (fp16, head_dim 128): the launch applies the scale epilogue.  Returns ``None`` when the shape is not served (contexts of
-    129..1024 tokens -- any longer one when batch x KV heads >= 128 workgroups --, head_dim >= 64, <= 16 query heads per KV head):
+    129..1024 tokens -- any longer one from 64 (row, KV head) pairs --, head_dim >= 64, <= 16 query heads per KV head):
     finish the sums and call ``decode_attention``."""
     p = parts.parts
     scaled = p.dtype == torch.int32  # smoothquant: exact int32 planes + per-token / per-channel scales (ScaledInt32Partials)
@@ -229,11 +228,19 @@ def decode_attention_partials(parts, bias, num_heads: int, num_kv_heads: int, he
             or not _head_norm_ok(qk_norm, head_dim, dt)):
         return None
     max_len = int(max_actual_seq_len)
-    waves = L.lib().ll_flash_decoding_group_waves(max_len, batchs * num_kv_heads)  # the one-workgroup form (0: not applicable)
+    waves = L.lib().ll_flash_decoding_group_waves(max_len, batchs * num_kv_heads)  # (0: not applicable)
     if waves < 2 or (num_heads // num_kv_heads + 2) * head_dim // 4 > 128 * waves:
         return None
     k_cache, v_cache = kv_buffer[:, :num_kv_heads], kv_buffer[:, num_kv_heads:]
     out = torch.empty((batchs, num_heads, head_dim), dtype=dt, device=p.device)
+    mid_o = mid_lse = counters = None
+    if max_len > 1024 and batchs * num_kv_heads < 128:  # several workgroups share a row: scratch of their merge
+        counters = _merge_counters(p.device, batchs * num_kv_heads)
+        if counters is None:
+            return None
+        nparts = L.lib().ll_flash_decoding_num_partitions(max_len)
+        mid_o = torch.empty((batchs, num_heads, nparts, head_dim), dtype=torch.float32, device=p.device)
+        mid_lse = torch.empty((batchs, num_heads, nparts, 32), dtype=torch.float32, device=p.device)
     L.check(
         L.lib().ll_decode_attention_partials(
             out.data_ptr(), p.data_ptr(), s_count, L.ptr(bias), cos_table.data_ptr(), sin_table.data_ptr(),
@@ -244,7 +251,7 @@ def decode_attention_partials(parts, bias, num_heads: int, num_kv_heads: int, he
             b_req_tokens_table.stride(0), L.dtype_code(dt), L.index_width(b_req_idx), L.index_width(b_seq_len),
             L.ptr(None if qk_norm is None else qk_norm[0]), L.ptr(None if qk_norm is None else qk_norm[1]),
             0.0 if qk_norm is None else float(qk_norm[2]), parts.a_scale.data_ptr() if scaled else 0,
-            parts.w_scale.data_ptr() if scaled else 0, L.stream_ptr(),
+            parts.w_scale.data_ptr() if scaled else 0, L.ptr(mid_o), L.ptr(mid_lse), L.ptr(counters), L.stream_ptr(),
         ),
         "decode_attention_partials",
     )
