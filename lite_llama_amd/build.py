@@ -32,7 +32,7 @@ FILE_FLAGS = {"gemm_short.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"],
               "seq_mix.hip": _NO_PACKED_FP32, "ragged_attn.hip": _NO_PACKED_FP32, "ragged_attn_mfma.hip": _NO_PACKED_FP32,
               "group_norm.hip": _NO_PACKED_FP32, "latent_attn.hip": _NO_PACKED_FP32, "moe_sparse.hip": _NO_PACKED_FP32,
               "linear_mix.hip": _NO_PACKED_FP32, "delta_scan.hip": _NO_PACKED_FP32, "stream_norm.hip": _NO_PACKED_FP32,
-              "retention.hip": _NO_PACKED_FP32}
+              "retention.hip": _NO_PACKED_FP32, "gemm_tile256.hip": _NO_PACKED_FP32}
 
 
 # part libraries: the sources ONE model family needs (a fresh checkout serving only that family builds nothing else)

@@ -18,6 +18,7 @@
 #include <stdlib.h>
 
 #include "common.h"
+#include "gemm_tile256.h"
 #include "gemm_w4_common.h"
 
 #define PF_BN 256
@@ -266,12 +267,18 @@ extern "C" int ll_w4a16_matmul_prepacked_mtiled(void* out, const void* x, const 
   if (!out || !x || !wpacked || !spacked) return LL_ERR_ARG;
   if (!ll_aligned16(out) || !ll_aligned16(x) || !ll_aligned16(wpacked) || !ll_aligned16(spacked)) return LL_ERR_ARG;
   if ((m - 1) * x_stride_m * 2 + k * 2 >= (1ll << 31)) return LL_ERR_SHAPE;  // 32-bit activation offsets
+  int sh = 0;
+  while ((128 << sh) < group_size) ++sh;
+  if (tile256_wants(m, n, k, 0)) {  // (gemm_tile256.hip: both engines' figures beside the rule)
+    T2Params t{};
+    t.out = (uint16_t*)out; t.x = (const unsigned char*)x; t.w = (const unsigned char*)wpacked; t.sp = spacked; t.bias = (const uint16_t*)bias;
+    t.m = m; t.n = n; t.k = k; t.x_stride = x_stride_m * 2; t.chunks = (int)(k / 128); t.gshift = sh; t.epi = epilogue;
+    return tile256_launch(t, 0, stream);
+  }
   PfParams p{};
   p.out = (uint16_t*)out; p.x = (const uint16_t*)x; p.wp = wpacked; p.sp = spacked; p.bias = (const uint16_t*)bias;
   p.m = m; p.n = n; p.k = k; p.x_stride = x_stride_m;
   p.chunks = (int)(k / 128);
-  int sh = 0;
-  while ((128 << sh) < group_size) ++sh;
   p.gshift = sh;
   p.epi = epilogue;
   static const int wmh_env = getenv("LL_PF_WMH") ? atoi(getenv("LL_PF_WMH")) : 0;  // A/B knob, read once (1 / 2: force the tile height)

@@ -17,6 +17,7 @@
 #include <stdlib.h>
 
 #include "common.h"
+#include "gemm_tile256.h"
 #include "gemm_w4_common.h"
 #include "gemm_w8_common.h"
 
@@ -304,6 +305,14 @@ extern "C" int ll_w8_mtiled_try(void* out, const void* x, const void* w, const f
   if (wfmt == 3 && (!a_scale || !scales || !ll_aligned16(scales) || (acc_out && !ll_aligned16(acc_out)))) return 0;
   if (wfmt != 3 && !scales) return 0;
   if (bias && (reinterpret_cast<uintptr_t>(bias) & 7u)) return 0;
+  if (tile256_wants(m, n, k, wfmt)) {  // (gemm_tile256.hip; the kernel below keeps k that is no multiple of 128, for int8 x int8 256)
+    T2Params t{};
+    t.out = (uint16_t*)out; t.x = (const unsigned char*)x; t.w = (const unsigned char*)w; t.scales = scales; t.a_scale = a_scale;
+    t.bias = (const uint16_t*)bias; t.acc_out = acc_out;
+    t.m = m; t.n = n; t.k = k; t.x_stride = x_stride * eb; t.w_stride = w_stride;
+    t.s_stride_n = s_stride_n; t.s_stride_k = s_stride_k; t.group_k = group_k; t.group_n = group_n > 0 ? group_n : 1;
+    return tile256_launch(t, wfmt, stream) == LL_OK ? 1 : LL_ERR_LAUNCH;
+  }
   P8Params p{};
   p.out = (uint16_t*)out; p.x = (const unsigned char*)x; p.w = (const unsigned char*)w; p.scales = scales; p.a_scale = a_scale;
   p.bias = (const uint16_t*)bias; p.acc_out = acc_out;

@@ -12,6 +12,7 @@
 #include <stdlib.h>
 
 #include "common.h"
+#include "gemm_tile256.h"
 
 struct alignas(16) Q4 {
   uint32_t x, y, z, w;
@@ -743,13 +744,30 @@ extern "C" int ll_moe_gemm(void* c, const void* a, const void* w, const float* w
                            int64_t s_stride_k, int dtype, void* stream) {
   if (dtype != LL_F16) return LL_ERR_DTYPE;  // the reference MoE path is fp16 end to end
   if (wfmt != LL_W_F16 && wfmt != LL_W_FP8E4M3 && wfmt != LL_W_INT8) return LL_ERR_DTYPE;
-  if (block_m != 16 && block_m != 32 && block_m != 64 && block_m != 128) return LL_ERR_SHAPE;
+  if (block_m != 16 && block_m != 32 && block_m != 64 && block_m != 128 && block_m != 256) return LL_ERR_SHAPE;
   if (n <= 0 || k <= 0 || top_k <= 0 || k % 8 != 0 || a_stride_m % 8 != 0) return LL_ERR_SHAPE;
   if (mul_routed_weight < 0 || mul_routed_weight > 3 || ((mul_routed_weight & 2) && (n & 1))) return LL_ERR_SHAPE;
   if (wfmt != LL_W_F16 && (!w_scale || group_n <= 0 || group_k <= 0)) return LL_ERR_ARG;
   if (wfmt != LL_W_F16 && group_k < k && group_k % 8 != 0) return LL_ERR_SHAPE;  // a scale block spans whole 8-k MFMA steps
   if (wfmt == LL_W_F16 ? (w_stride_n % 8 != 0) : (w_stride_n % 8 != 0)) return LL_ERR_SHAPE;
   if (num_slots == 0) return LL_OK;
+  if (block_m == 256) {
+    // prefill-sized inputs over 8-bit experts: the 256 x 256 tiles of the dense projections (gemm_tile256.hip)
+    const int64_t rows = (num_slots + top_k - 1) / top_k;
+    if (wfmt == LL_W_F16 || k % 128 != 0 || k < 256 || n % 32 != 0 || (group_k < k && group_k % 64 != 0) || w_stride_n % 16 != 0 ||
+        w_stride_e % 16 != 0 || !ll_aligned16(a) || !ll_aligned16(w) || !ll_aligned16(c) || num_slots >= (1ll << 30) || n >= (1ll << 30) ||
+        rows * a_stride_m * 2 >= (1ll << 32) || n * w_stride_n >= (1ll << 32) || n * s_stride_n * 4 >= (1ll << 32))
+      return LL_ERR_SHAPE;
+    T2Params t{};
+    t.out = (uint16_t*)c; t.x = (const unsigned char*)a; t.w = (const unsigned char*)w; t.scales = w_scale;
+    t.m = num_slots; t.n = n; t.k = k; t.x_stride = a_stride_m * 2; t.w_stride = w_stride_n;
+    t.s_stride_n = s_stride_n; t.s_stride_k = s_stride_k; t.group_k = group_k; t.group_n = group_n;
+    t.epi = mul_routed_weight & 2 ? 1 : 0;
+    t.sorted_ids = sorted_ids; t.expert_ids = expert_ids; t.num_post = num_post;
+    t.topk_w = mul_routed_weight & 1 ? (const uint16_t*)topk_w : nullptr;
+    t.w_stride_e = w_stride_e; t.s_stride_e = s_stride_e; t.num_slots = (int)num_slots; t.top_k = top_k;
+    return tile256_grouped_launch(t, wfmt, stream);
+  }
   MoeParams p{};
   p.c = (uint16_t*)c; p.a = (const uint16_t*)a; p.w = w; p.w_scale = w_scale; p.topk_w = (const uint16_t*)topk_w;
   p.sorted_ids = sorted_ids; p.expert_ids = expert_ids; p.num_post = num_post;

@@ -49,6 +49,15 @@ def _block_m(num_tokens: int) -> int:
     return 64
 
 
+def _tiles_256(x, slots, w1, w2, s1, s2, g1, g2) -> bool:
+    """Whether ``ll_moe_gemm`` takes both products in blocks of 256 slots (its 32-bit offsets and 16-byte loads)."""
+    if x.data_ptr() % 16 or slots >= 2 ** 30 or max((x.shape[0] + 1) * x.stride(0), slots * w2.shape[2]) >= 2 ** 31:
+        return False
+    return all(w.shape[2] % 128 == 0 and w.shape[2] >= 256 and w.shape[1] % 32 == 0 and (gk >= w.shape[2] or gk % 64 == 0)
+               and w.stride(0) % 16 == 0 and w.stride(1) % 16 == 0 and w.data_ptr() % 16 == 0 and w.shape[1] * w.stride(1) < 2 ** 32
+               and s.dim() == 3 and w.shape[1] * s.stride(1) < 2 ** 30 for w, s, (_, gk) in ((w1, s1, g1), (w2, s2, g2)))
+
+
 def fused_moe_block_m(num_tokens: int) -> int:
     """The row-block size :func:`fused_moe` aligns ``num_tokens`` tokens to."""
     return _block_m(num_tokens)
@@ -145,7 +154,11 @@ def fused_moe(
     flat_weights = topk_weights.reshape(-1).to(dtype).contiguous()
 
     block_m = _block_m(num_tokens)
-    if (num_tokens * top_k >= 256 * num_experts and hidden % 128 == 0 and intermediate % 128 == 0
+    if wfmt and num_tokens * top_k >= 128 * num_experts and _tiles_256(hidden_states, num_tokens * top_k, w1, w2, w1_scale, w2_scale, g1, g2):
+        # 8-bit experts, 128+ rows each on average: blocks of 256 slots on the 256 x 256 tiles.  128 experts of 2048 / 768, us with blocks of
+        # 64 / 128 / 256: 1024 tokens 315 / 325 / 339, 2048 503 / 463 / 376, 8192 1576 / 1383 / 963
+        block_m = 256
+    elif (num_tokens * top_k >= 256 * num_experts and hidden % 128 == 0 and intermediate % 128 == 0
             and (not wfmt or all(gk >= kdim or gk % 64 == 0 for gk, kdim in ((g1[1], hidden), (g2[1], intermediate))))
             and w1.stride(1) % 16 == 0 and w2.stride(1) % 16 == 0 and w1.stride(0) % 16 == 0 and w2.stride(0) % 16 == 0):
         # (extension, round 6) prefill-sized inputs -- 256+ rows per expert on average: 128-row blocks on the full-line grouped GEMM

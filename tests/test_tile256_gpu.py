@@ -1,0 +1,130 @@
+"""The 256 x 256 tiles for many rows (csrc/gemm_tile256.hip): dense projections over int4 / fp8 / int8 weights and int8 x int8, and the
+expert products over blocks of 256 slots, against 64-bit products of the dequantised operands."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def gen(seed):
+    return torch.Generator(device=DEV).manual_seed(seed)
+
+
+def near(got, want):
+    """fp32 sums of fp16 products of unit size, rounded once to fp16: half a unit of the result plus the sums' own rounding."""
+    bar = 2.0 ** -11 * want.abs() + 2.0 ** -13 * want.abs().amax()
+    assert ((got.double() - want).abs() <= bar).all(), ((got.double() - want).abs() - bar).max()
+
+
+# rows at the edges of a tile, of a 32-row fragment, of a workgroup's next tile; int4: more than 16 column tiles or 144 tiles (the dispatch rule)
+ROWS = [(65, 4352), (129, 49152), (257, 24832), (1057, 12288), (2600, 3584)]
+
+
+@pytest.mark.parametrize("m,n", ROWS)
+@pytest.mark.parametrize("k", [256, 640])
+def test_int4(m, n, k):
+    import lite_llama_amd.kernels.quantization as Q
+
+    g = gen(m)
+    q = torch.randint(0, 16, (n, k // 8, 8), generator=g, device=DEV, dtype=torch.int32)
+    words = sum(q[..., j] << (4 * j) for j in range(8)).to(torch.int32)
+    scale = torch.rand(n, k // 128, generator=g, device=DEV) * 0.01 + 0.01
+    zero = torch.randint(0, 16, (n, k // 128), generator=g, device=DEV).float()
+    x = torch.randn(m, k, generator=g, device=DEV).half()
+    bias = torch.randn(n, generator=g, device=DEV).half()
+    pw, ps = Q.pack_w4a16_weights(words), Q.pack_w4a16_scales(scale, zero)
+    s16, nzs = scale.half().double(), (-zero * scale).half().double()
+    w = (q.view(n, k // 128, 128).double() * s16[..., None] + nzs[..., None]).half().double().view(n, k)   # one rounding, as the kernel's fma
+    want = x.double() @ w.T
+    near(Q.w4a16_matmul_prepacked_rows(x, pw, ps, bias=bias), want + bias.double())
+    pairs = want.half().double()
+    act = Q.w4a16_matmul_prepacked_rows(x, pw, ps, gate_up_swiglu=True)
+    ref = torch.nn.functional.silu(pairs[:, 0::2]) * pairs[:, 1::2]
+    # gate and up are rounded to fp16 first: a unit of each, times the other
+    bar = 2.0 ** -9 * (ref.abs() + pairs[:, 0::2].abs() + pairs[:, 1::2].abs() + 1)
+    assert ((act.double() - ref).abs() <= bar).all()
+
+
+@pytest.mark.parametrize("m,n", [(65, 32), (129, 49152 - 32), (257, 24832 + 96), (1057, 12288)])
+@pytest.mark.parametrize("fmt,gn,gk", [("fp8", 128, 128), ("int8", 1, 1 << 30), ("fp8", 1, 128)])
+@pytest.mark.parametrize("k", [256, 640])
+def test_8bit_weights(m, n, fmt, gn, gk, k):
+    from lite_llama_amd import kernels as K
+
+    g = gen(n)
+    gk = min(gk, k)
+    if fmt == "fp8":
+        w = (torch.randn(n, k, generator=g, device=DEV) * 60).clamp(-448, 448).to(torch.float8_e4m3fn)
+        codes, wide, unit = w.view(torch.uint8), w.double(), 1 / 60
+    else:
+        codes = torch.randint(-127, 128, (n, k), generator=g, device=DEV, dtype=torch.int8)
+        wide, unit = codes.double(), 1 / 64
+    scale = ((torch.rand(-(-n // gn), k // gk, generator=g, device=DEV) + 0.5) * unit).half().float()
+    x = torch.randn(m, k, generator=g, device=DEV).half()
+    bias = torch.randn(n, generator=g, device=DEV).half()
+    full = scale.double().repeat_interleave(gn, 0)[:n].repeat_interleave(gk, 1)
+    # weight times scale is rounded to fp16 once (fp8: the widened value, 2^-8 of it, times 256 scales)
+    w16 = (wide * full).half().double() if fmt == "int8" else ((wide / 256).half().double() * (scale * 256).half().double().repeat_interleave(gn, 0)[:n].repeat_interleave(gk, 1)).half().double()
+    near(K.w8a16_matmul(x, codes, scale, group_n=gn, group_k=gk, bias=bias), x.double() @ w16.T + bias.double())
+
+
+@pytest.mark.parametrize("m,n,k", [(65, 32, 512), (129, 49152 - 32, 512), (257, 24832, 768), (1057, 12288 + 64, 512)])
+def test_int8_by_int8(m, n, k):
+    from lite_llama_amd import kernels as K
+    from lite_llama_amd.kernels.quantization import quantize_activations_int8
+
+    g = gen(k)
+    w = torch.randint(-127, 128, (n, k), generator=g, device=DEV, dtype=torch.int8)
+    scale = torch.rand(n, 1, generator=g, device=DEV) * 0.01
+    x = torch.randn(m, k, generator=g, device=DEV).half()
+    qa, a = quantize_activations_int8(x)
+    sums = qa.double() @ w.double().T                 # exact
+    want = (sums.float() * a.view(-1, 1)) * scale.view(1, -1)
+    assert torch.equal(K.smoothquant_matmul(x, w, scale), want.half())
+
+
+@pytest.mark.parametrize("fmt", ["fp8", "int8"])
+@pytest.mark.parametrize("tokens,experts,top", [(1100, 4, 2), (2049, 5, 2), (1500, 3, 1)])
+@pytest.mark.parametrize("interleaved", [False, True])
+def test_expert_products(fmt, tokens, experts, top, interleaved):
+    """Experts of very different loads: none, one slot, one slot into a block, whole blocks; the router's weights."""
+    from lite_llama_amd import kernels as K
+
+    hidden, inter = 256, 384
+    g = gen(tokens)
+    load = torch.rand(experts, generator=g, device=DEV) ** 3
+    load[1] = 0
+    ids = torch.multinomial(load.expand(tokens, experts) + 1e-9, top, generator=g)
+    ids[0, 0], ids[1:, 0] = 1, torch.where(ids[1:, 0] == 1, torch.full_like(ids[1:, 0], 2), ids[1:, 0])
+    wts = torch.softmax(torch.randn(tokens, top, generator=g, device=DEV), -1).half()
+    x = torch.randn(tokens, hidden, generator=g, device=DEV).half()
+    ws, scales, wide = [], [], []
+    for out, inp in ((2 * inter, hidden), (hidden, inter)):
+        w = torch.randn(experts, out, inp, generator=g, device=DEV)
+        sc = (torch.rand(experts, out, inp // 128, generator=g, device=DEV) + 0.5) * inp ** -0.5
+        if fmt == "fp8":
+            code = (w * 60).clamp(-448, 448).to(torch.float8_e4m3fn)
+            sc = sc / 60
+            wide.append(((code.double() / 256).half().double() * (sc * 256).half().double().repeat_interleave(128, 2)).half().double())
+            ws.append(code.view(torch.uint8))
+        else:
+            code = (w * 32).round().clamp(-127, 127).to(torch.int8)
+            sc = sc / 32
+            wide.append((code.double() * sc.half().double().repeat_interleave(128, 2)).half().double())
+            ws.append(code)
+        scales.append(sc)
+    want = torch.zeros(tokens, hidden, dtype=torch.float64, device=DEV)
+    for e in range(experts):
+        rows, slot = (ids == e).nonzero(as_tuple=True)
+        gu = (x[rows].double() @ wide[0][e].T).half().double()
+        gate, up = (gu[:, :inter], gu[:, inter:]) if not interleaved else (gu[:, 0::2], gu[:, 1::2])
+        y = ((torch.nn.functional.silu(gate) * up).half().double() @ wide[1][e].T) * wts[rows, slot].double()[:, None]
+        want.index_add_(0, rows, y.half().double())
+    got = K.fused_moe(x, ws[0], ws[1], wts, ids, w1_scale=scales[0], w2_scale=scales[1], group_n=1, group_k=128, w1_group=(1, 128),
+                      w2_group=(1, 128), w1_interleaved=interleaved)
+    # a unit of fp16 at each of three roundings (gate / up, the activation, a slot's result) and of the sum over the slots
+    bar = 2.0 ** -8 * want.abs().amax()
+    assert (got.double() - want).abs().max() <= bar
+    assert (got.double() - want).norm() <= 2.0 ** -10 * want.norm()
