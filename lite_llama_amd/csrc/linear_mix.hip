@@ -55,7 +55,10 @@ __device__ __forceinline__ float act_sigmoid(float v) {
 }
 
 // ln(sigmoid(z)) without cancellation on either side
-__device__ __forceinline__ float log_sigmoid(float z) { return z >= 0.f ? -log1pf(expf(-z)) : z - log1pf(expf(z)); }
+__device__ __forceinline__ float log_sigmoid(float z) {   // (one evaluation for both signs: lanes of a wave differ in them)
+  const float l = log1pf(expf(-fabsf(z)));
+  return z >= 0.f ? -l : z - l;
+}
 __device__ __forceinline__ float softplus(float z) { return z > 20.f ? z : log1pf(expf(z)); }
 // sigmoid(z)^(1 / tau): ONE definition for the scan and for the pass that evaluates a step's decays ahead of it
 __device__ __forceinline__ float entry_decay(float z, float inv_tau) { return expf(log_sigmoid(z) * inv_tau); }
@@ -104,28 +107,40 @@ __global__ __launch_bounds__(256) void entry_decay_kernel(float* __restrict__ ou
 // rows kg, kg + 16, ... in registers.  Tokens are taken tb at a time: decay, key and query of every key entry are staged in
 // LDS as one 16-byte record (all transcendental work happens here, once per token and entry), the slice's values beside
 // them; every thread then walks the tb tokens over its rows (state update + partial read-out), and the partials of the 16 row
-// groups are added in group order.  The walk is the same token-by-token expression whatever the step's cut.
-template <int DT, int RMAX, bool EXACT>   // EXACT: dk == 16 RMAX, every thread owns RMAX rows (no per-row guards)
+// groups are added in group order.  The walk is the same token-by-token expression whatever the cut of its steps.
+// CV: state columns per thread.  4 (one decoded token per sequence, dv a multiple of 4): 64 columns per workgroup, the state moves in
+// 16-byte pieces -- the same sums in the same order.  32 sequences, 8 heads of 128 x 256 (64 MB of state both ways): 21.1 -> 12.1 us.
+template <int DT, int RMAX, bool EXACT, int CV>   // EXACT: dk == 16 RMAX, every thread owns RMAX rows (no per-row guards)
 __global__ __launch_bounds__(256) void linear_scan_kernel(const ScanArgs a) {
   extern __shared__ float lds[];
-  const int b = blockIdx.x, head = blockIdx.y, c0 = blockIdx.z * 16;
-  const int tid = threadIdx.x, col = tid & 15, kg = tid >> 4;
+  const int b = blockIdx.x, head = blockIdx.y, c0 = blockIdx.z * 16 * CV;
+  constexpr int CW = 16 * CV;
+  const int tid = threadIdx.x, col = (tid & 15) * CV, kg = tid >> 4;
   const int dk = a.dk, dv = a.dv, tb = a.tb, heads = a.heads;
   const bool active = c0 + col < dv && kg < dk;
   const int rows = kg < dk ? (dk - kg + 15) / 16 : 0;
   f32x4* sg = reinterpret_cast<f32x4*>(lds);   // [tb][dk] (decay, key, query, -)
-  float* sv = lds + 4 * tb * dk;                // [tb][16] what enters the state: value (times the step size)
-  float* sx = sv + tb * 16;                     // [tb][16] skip path: skip_h * value
-  float* sp = sx + tb * 16;                     // [tb][16 groups][16] partial read-outs
-  float* sd = sp + tb * 256;                    // [tb][2] kind 2: (decay, step size) of the token
+  float* sv = lds + 4 * tb * dk;                // [tb][CW] what enters the state: value (times the step size)
+  float* sx = sv + tb * CW;                     // [tb][CW] skip path: skip_h * value
+  float* sp = sx + tb * CW;                     // [tb][16 groups][CW] partial read-outs
+  float* sd = sp + tb * 16 * CW;                    // [tb][2] kind 2: (decay, step size) of the token
   const int t0 = a.seq_start[b], t1 = a.seq_start[b + 1];
   float* st = a.state + ((int64_t)a.seq_slot[b] * heads + head) * dk * dv + c0 + col;
   const bool carry = a.seq_first_pos[b] > 0;
   const int qh = head / a.qk_rep;
   const int kind = a.kind;
-  float S[RMAX];
+  float S[RMAX][CV];
 #pragma unroll
-  for (int r = 0; r < RMAX; ++r) S[r] = (active && r < rows && carry) ? st[(int64_t)(kg + 16 * r) * dv] : 0.f;
+  for (int r = 0; r < RMAX; ++r) {
+    const bool in = active && r < rows && carry;
+    if constexpr (CV == 4) {
+      const f32x4 old = in ? *reinterpret_cast<const f32x4*>(st + (int64_t)(kg + 16 * r) * dv) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) S[r][e] = old[e];
+    } else {
+      S[r][0] = in ? st[(int64_t)(kg + 16 * r) * dv] : 0.f;
+    }
+  }
   for (int base = t0; base < t1; base += tb) {
     const int nt = t1 - base < tb ? t1 - base : tb;
     __syncthreads();
@@ -154,8 +169,8 @@ __global__ __launch_bounds__(256) void linear_scan_kernel(const ScanArgs a) {
       else dec = sd[2 * tt];
       sg[i] = f32x4{dec, kv, qv * a.q_scale, 0.f};
     }
-    for (int i = tid; i < nt * 16; i += 256) {
-      const int tt = i >> 4, cc = i & 15;
+    for (int i = tid; i < nt * CW; i += 256) {
+      const int tt = i / CW, cc = i % CW;
       float x = c0 + cc < dv ? ldv<DT>(a.v, (int64_t)(base + tt) * a.v_ld + head * dv + c0 + cc) : 0.f;
       if (a.act) x *= act_sigmoid<DT>(x);
       sv[i] = kind == 2 ? sd[2 * tt + 1] * x : x;
@@ -163,30 +178,374 @@ __global__ __launch_bounds__(256) void linear_scan_kernel(const ScanArgs a) {
     }
     __syncthreads();
     for (int tt = 0; tt < nt; ++tt) {
-      const float val = sv[tt * 16 + col];
-      float acc = 0.f;
+      float val[CV], acc[CV];
+#pragma unroll
+      for (int e = 0; e < CV; ++e) {
+        val[e] = sv[tt * CW + col + e];
+        acc[e] = 0.f;
+      }
 #pragma unroll
       for (int r = 0; r < RMAX; ++r) {
         if (EXACT || r < rows) {
           const f32x4 g = sg[tt * dk + kg + 16 * r];
-          S[r] = __builtin_fmaf(g[0], S[r], g[1] * val);
-          acc = __builtin_fmaf(S[r], g[2], acc);
+#pragma unroll
+          for (int e = 0; e < CV; ++e) {
+            S[r][e] = __builtin_fmaf(g[0], S[r][e], g[1] * val[e]);
+            acc[e] = __builtin_fmaf(S[r][e], g[2], acc[e]);
+          }
         }
       }
-      sp[(tt * 16 + kg) * 16 + col] = acc;
+#pragma unroll
+      for (int e = 0; e < CV; ++e) sp[(tt * 16 + kg) * CW + col + e] = acc[e];
     }
     __syncthreads();
-    for (int i = tid; i < nt * 16; i += 256) {
-      const int tt = i >> 4, cc = i & 15;
+    for (int i = tid; i < nt * CW; i += 256) {
+      const int tt = i / CW, cc = i % CW;
       float o = 0.f;
 #pragma unroll
-      for (int g2 = 0; g2 < 16; ++g2) o += sp[(tt * 16 + g2) * 16 + cc];
+      for (int g2 = 0; g2 < 16; ++g2) o += sp[(tt * 16 + g2) * CW + cc];
       if (c0 + cc < dv) a.o[((int64_t)(base + tt) * heads + head) * dv + c0 + cc] = o + sx[i];
     }
   }
 #pragma unroll
-  for (int r = 0; r < RMAX; ++r)
-    if (active && r < rows) st[(int64_t)(kg + 16 * r) * dv] = S[r];
+  for (int r = 0; r < RMAX; ++r) {
+    if (!(active && r < rows)) continue;
+    if constexpr (CV == 4) *reinterpret_cast<f32x4*>(st + (int64_t)(kg + 16 * r) * dv) = f32x4{S[r][0], S[r][1], S[r][2], S[r][3]};
+    else st[(int64_t)(kg + 16 * r) * dv] = S[r][0];
+  }
+}
+
+// ------------------------------------------------------------------------------------------------------------------------
+// runs of many tokens: chunks of 16 tokens as matrix products on the fp32 matrix cores.  With D_t the product of the decays of a chunk's
+// tokens up to t, R(u, t) that of the tokens behind u up to t, and S the state in front of the chunk,
+//
+//   o_t = (q_t D_t)^T S + sum_(u <= t) [sum_i q_t[i] k_u[i] R(u, t)[i]] v_u,      S <- D_15 S + sum_u (k_u R(u, 15)) v_u^T
+//
+// Every factor is a running product of decays (no quotient), so nothing leaves the range the walk token by token stays in.
+//   chunk_terms_kernel   everything that does not depend on the state, for all chunks at once: activations, decays, decayed queries and
+//                        keys, the 16 x 16 scores -- stored in the order in which the second kernel's lanes take operands
+//   chunk_scan_kernel    a wave per (sequence, head, 16 columns) carries its state columns through the chunks in registers
+// The walk is bound by LDS (a 16-byte record per 16 columns of a key entry and token) and by its three fp32 operations per state entry
+// and token; here a wave runs 2 dk / 4 + 4 matrix instructions per 16 tokens.  us, walk -> chunks (both kernels), 8 runs of 256 - 512 tokens
+// | one of 1024: per entry, 8 heads of 128 x 256: 536 -> 95 (terms 31) | 417 -> 130; fixed, 16 of 128 x 128: 439 -> 105 | 340 -> 137; per
+// token, 32 of 128 x 64: 443 -> 88 | 344 -> 140.  Of the 66 us of the first scan 33 are its matrix instructions; the rest waits for
+// operands, requested half a chunk ahead.  Products of decays, which meet the state once per chunk, are taken in 64 bits and what a chunk
+// adds is summed apart: the error against 64 bits is the walk's or below it (fixed: 7.8e-8 against 9.2e-8 of the result's norm).
+// ------------------------------------------------------------------------------------------------------------------------
+constexpr int kCT = 16;      // tokens per chunk
+constexpr int kRec = 320;    // floats per (chunk, head): scores 256, then kinds 0 and 2: D_t, R(u, 15) b_u, b_u (16 each)
+
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+struct ChunkBufs {
+  float* q;      // [chunk][terms head][KT][64 lanes][4]: decayed queries (kinds 0 and 2: queries)
+  float* k;      // likewise keys, token-major inside a lane
+  float* last;   // kind 1: [chunk][head][16 KT] D_15 per key entry
+  float* rec;    // [chunk][head][kRec]
+};
+
+// One workgroup per (chunk of the longest run, sequence, terms head): a head for kind 1, else a query / key head with all its value heads.
+template <int DT, int KT, bool ENTRY>
+__global__ __launch_bounds__(256) void chunk_terms_kernel(const ScanArgs a, const ChunkBufs w) {
+  constexpr int W = 16 * KT, LD = W + 4;
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  __shared__ float vec[16][kCT], steps[16][kCT];
+  float* sq = lds;
+  float* sk = sq + kCT * LD;
+  float* sa = sk + kCT * LD;   // ENTRY
+  const int b = blockIdx.y, th = blockIdx.z, tid = threadIdx.x;
+  const int t0 = a.seq_start[b], t1 = a.seq_start[b + 1];
+  const int base = t0 + kCT * (int)blockIdx.x;
+  if (base >= t1) return;
+  const int n = t1 - base < kCT ? t1 - base : kCT;
+  const int64_t slot = t0 / kCT + b + blockIdx.x;
+  const int heads = a.heads;
+  constexpr int dk = W;
+  const int qh = ENTRY ? th / a.qk_rep : th;
+  const int tnum = ENTRY ? heads : heads / a.qk_rep;
+#pragma unroll
+  for (int i0 = 0; i0 < kCT * W; i0 += 256) {
+    const int i = i0 + tid, tt = i / W, kk = i - tt * W;
+    float qv = 0.f, kv = 0.f, dec = 1.f;
+    if (tt < n) {
+      const int64_t row = base + tt;
+      qv = ldv<DT>(a.q, row * a.q_ld + (int64_t)qh * dk + kk);
+      kv = ldv<DT>(a.k, row * a.k_ld + (int64_t)qh * dk + kk);
+      if (a.act) {
+        qv *= act_sigmoid<DT>(qv);
+        kv *= act_sigmoid<DT>(kv);
+      }
+      qv *= a.q_scale;
+      if constexpr (ENTRY)
+        dec = entry_decay(ldv<DT>(a.gate, row * a.gate_ld + (int64_t)th * dk + kk) + ldv<DT>(a.gate_bias, th * dk + kk), a.inv_tau);
+    }
+    sq[tt * LD + kk] = qv;
+    sk[tt * LD + kk] = kv;
+    if constexpr (ENTRY) sa[tt * LD + kk] = dec;
+  }
+  __syncthreads();
+  // scores: thread (key token u, entries 4 g + 64 j ..) against all queries behind it
+  const int u = tid >> 4, g = tid & 15, u0 = __builtin_amdgcn_readfirstlane(tid >> 6) * 4;   // u0: the wave's first key token
+  float acc[kCT];
+#pragma unroll
+  for (int t = 0; t < kCT; ++t) acc[t] = 0.f;
+#pragma unroll
+  for (int j = 0; j < KT / 4; ++j) {
+    const int at = 4 * g + 64 * j;
+    f32x4 m = *reinterpret_cast<const f32x4*>(sk + u * LD + at);
+#pragma unroll
+    for (int t = 0; t < kCT; ++t) {
+      if (t < u0) continue;
+      const f32x4 qv = *reinterpret_cast<const f32x4*>(sq + t * LD + at);
+      if constexpr (ENTRY) {
+        const f32x4 av = *reinterpret_cast<const f32x4*>(sa + t * LD + at);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) m[e] = t > u ? m[e] * av[e] : m[e];
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[t] = __builtin_fmaf(qv[e], m[e], acc[t]);
+    }
+  }
+  __syncthreads();
+  if constexpr (ENTRY) {
+    if (tid < W) {
+      double p = 1.0;
+#pragma unroll
+      for (int t = 0; t < kCT; ++t) {
+        p *= sa[t * LD + tid];
+        sq[t * LD + tid] *= (float)p;
+      }
+      w.last[(slot * tnum + th) * W + tid] = (float)p;
+      p = 1.0;
+#pragma unroll
+      for (int t = kCT - 1; t >= 0; --t) {
+        sk[t * LD + tid] *= (float)p;
+        p *= sa[t * LD + tid];
+      }
+    }
+    __syncthreads();
+  }
+  // operands in lane order: lane (t, c) of piece s takes query t's entries 16 s + 4 c .. and key entry 16 s + t of tokens 4 c ..
+  for (int i = tid; i < KT * 64; i += 256) {
+    const int s = i >> 6, t = i & 15, c = (i >> 4) & 3;
+    const int64_t at = ((slot * tnum + th) * KT * 64 + i) * 4;
+    *reinterpret_cast<f32x4*>(w.q + at) = *reinterpret_cast<const f32x4*>(sq + t * LD + 16 * s + 4 * c);
+    f32x4 kv;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) kv[e] = sk[(4 * c + e) * LD + 16 * s + t];
+    *reinterpret_cast<f32x4*>(w.k + at) = kv;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < kCT; ++t) lds[tid * 17 + t] = acc[t];
+  __syncthreads();
+  const int t = tid & 15;
+  float part[16];
+#pragma unroll
+  for (int j = 0; j < 16; ++j) part[j] = lds[(u * 16 + j) * 17 + t];
+#pragma unroll
+  for (int j = 8; j > 0; j >>= 1)
+#pragma unroll
+    for (int i = 0; i < j; ++i) part[i] += part[i + j];
+  const float p = part[0];
+  const int rec_at = ((u >> 2) * 16 + t) * 4 + (u & 3);   // lane (t, c) takes query t's scores against tokens 4 c ..
+  if constexpr (ENTRY) {
+    w.rec[(slot * heads + th) * kRec + rec_at] = t >= u ? p : 0.f;
+    return;
+  }
+  for (int r0 = 0; r0 < a.qk_rep; r0 += 16) {   // value heads, 16 at a time
+    __syncthreads();
+    const int hn = a.qk_rep - r0 < 16 ? a.qk_rep - r0 : 16;
+    const int h0 = th * a.qk_rep + r0;
+    if (u < hn) {   // (thread (value head, token))
+      float dec = 1.f, step = 1.f;
+      if (t < n) {
+        if (a.kind == 0) {
+          dec = a.head_decay[h0 + u];
+        } else {
+          step = softplus(ldv<DT>(a.dt, (int64_t)(base + t) * a.dt_ld + h0 + u) + ldv<DT>(a.dt_bias, h0 + u));
+          dec = expf(-expf(ldv<DT>(a.a_log, h0 + u)) * step);
+        }
+      }
+      vec[u][t] = dec;
+      steps[u][t] = step;
+    }
+    __syncthreads();
+    if (u < hn) {
+      double d = 1.0, e = 1.0;
+#pragma unroll
+      for (int x = 0; x < kCT; ++x) {
+        d = x <= t ? d * vec[u][x] : d;
+        e = x > t ? e * vec[u][x] : e;
+      }
+      float* rec = w.rec + (slot * heads + h0 + u) * kRec + 256;
+      rec[t] = (float)d;
+      rec[16 + t] = (float)(e * steps[u][t]);
+      rec[32 + t] = steps[u][t];
+    }
+    for (int h = 0; h < hn; ++h) {   // (thread (key token, query token))
+      double r = 1.0;
+#pragma unroll
+      for (int x = 1; x < kCT; ++x) r = x > u && x <= t ? r * vec[h][x] : r;
+      w.rec[(slot * heads + h0 + h) * kRec + rec_at] = t >= u ? p * (float)r : 0.f;
+    }
+  }
+}
+
+// A wave per (sequence, head, 16 state columns), no LDS and no barrier: lane (t, c), element r of piece s holds the state of key entry
+// 16 s + 4 c + r and column t -- the layout in which v_mfma_f32_16x16x4 leaves results AND takes its second operand when a contraction's
+// entries are taken in the order (element, c).  Queries of the next chunk are requested behind the read-out, under the state's
+// products; keys behind those, under the next read-out.  The waves of a head are dealt to one XCD: they read the same operands.
+template <int DT, int KT, bool ENTRY>
+__global__ __launch_bounds__(256) void chunk_scan_kernel(const ScanArgs a, const ChunkBufs w, int pairs, int tiles) {
+  constexpr int W = 16 * KT;
+  const int wid = blockIdx.x;
+  const int groups = (tiles + 3) >> 2, xcd = wid & 7, rest = wid >> 3;
+  const int pair = rest / groups * 8 + xcd, tile = rest % groups * 4 + (threadIdx.x >> 6);
+  if (pair >= pairs || tile >= tiles) return;
+  const int b = pair / a.heads, head = pair - b * a.heads, lane = threadIdx.x & 63, t = lane & 15, c = lane >> 4;
+  const int dv = a.dv, heads = a.heads, col = tile * 16 + t;
+  const int t0 = a.seq_start[b], t1 = a.seq_start[b + 1];
+  if (t0 >= t1) return;
+  const int tnum = ENTRY ? heads : heads / a.qk_rep, th = ENTRY ? head : head / a.qk_rep;
+  const bool carry = a.seq_first_pos[b] > 0, live = col < dv;
+  float* st = a.state + ((int64_t)a.seq_slot[b] * heads + head) * W * dv + col;
+  f32x4 S[KT];
+#pragma unroll
+  for (int s = 0; s < KT; ++s)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int kk = 16 * s + 4 * c + r;
+      S[s][r] = (carry && live) ? st[(int64_t)kk * dv] : 0.f;
+    }
+  const bool skips = !ENTRY && a.kind == 2 && a.skip;
+  const float skip = skips ? ldv<DT>(a.skip, head) : 0.f;
+  const int chunks = (t1 - t0 + kCT - 1) / kCT;
+  const int64_t slot = t0 / kCT + b;
+  const float* qp = w.q + ((slot * tnum + th) * KT * 64 + lane) * 4;
+  const float* kp = w.k + ((slot * tnum + th) * KT * 64 + lane) * 4;
+  const float* lp = ENTRY ? w.last + (slot * tnum + th) * W + 4 * c : nullptr;
+  const float* rp = w.rec + (slot * heads + head) * kRec;
+  const int64_t qk_step = (int64_t)tnum * KT * 256, last_step = (int64_t)tnum * W, rec_step = (int64_t)heads * kRec;
+  f32x4 qf[KT], kf[KT], lf[ENTRY ? KT : 1], pf, df, wf, sf;
+  uint32_t raw[4];   // the values' bits: converted where they are used, so that nothing waits for them here
+  auto get_q = [&]() {
+#pragma unroll
+    for (int s = 0; s < KT; ++s) qf[s] = *reinterpret_cast<const f32x4*>(qp + 256 * s);
+    pf = *reinterpret_cast<const f32x4*>(rp + 4 * lane);
+    if constexpr (!ENTRY) {
+      df = *reinterpret_cast<const f32x4*>(rp + 256 + 4 * c);
+      wf = *reinterpret_cast<const f32x4*>(rp + 272 + 4 * c);
+      sf = *reinterpret_cast<const f32x4*>(rp + 288 + 4 * c);
+    }
+  };
+  auto get_k = [&]() {
+#pragma unroll
+    for (int s = 0; s < KT; ++s) kf[s] = *reinterpret_cast<const f32x4*>(kp + 256 * s);
+    if constexpr (ENTRY) {
+#pragma unroll
+      for (int s = 0; s < KT; ++s) lf[s] = *reinterpret_cast<const f32x4*>(lp + 16 * s);
+    }
+  };
+  auto get_v = [&](int base) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int tok = base + 4 * c + r < t1 ? base + 4 * c + r : t1 - 1;
+      const int64_t at = (int64_t)tok * a.v_ld + (int64_t)head * dv + (live ? col : 0);
+      if constexpr (DT == LL_F32) raw[r] = ((const uint32_t*)a.v)[at];
+      else raw[r] = ((const uint16_t*)a.v)[at];
+    }
+  };
+  get_q();
+  get_v(t0);
+  __builtin_amdgcn_sched_barrier(0);   // (the loop's order of requests, so that its waits count the same in its first pass)
+  get_k();
+  __builtin_amdgcn_sched_barrier(0);
+  for (int j = 0; j < chunks; ++j) {
+    const int base = t0 + kCT * j;
+    const bool more = j + 1 < chunks;   // (the last chunk requests its own operands again: no branch around the loads)
+    f32x4 v, x;
+    bool odd = false;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const bool in = live && base + 4 * c + r < t1;
+      if constexpr (DT == LL_F32) x[r] = in ? __uint_as_float(raw[r]) : 0.f;
+      else x[r] = in ? to_f32<DT>((uint16_t)raw[r]) : 0.f;
+      if (a.act) x[r] *= act_sigmoid<DT>(x[r]);
+      v[r] = !ENTRY && a.kind == 2 ? sf[r] * x[r] : x[r];
+      odd |= !(fabsf(v[r]) < INFINITY);
+    }
+    f32x4 part[8];   // eight short sums, then pairs of them
+#pragma unroll
+    for (int i = 0; i < 8; ++i) part[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < KT; ++s)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) part[(4 * s + e) & 7] = mfma4(qf[s][e], S[s][e], part[(4 * s + e) & 7]);
+#pragma unroll
+    for (int i = 4; i > 0; i >>= 1)
+#pragma unroll
+      for (int y = 0; y < i; ++y) part[y] += part[y + i];
+    f32x4 o = part[0];
+    const float dlast = ENTRY ? 0.f : __shfl(df[3], 48);   // D_15: all decays of the chunk
+    f32x4 vw = x;
+    f32x4 near = {0.f, 0.f, 0.f, 0.f};
+    if (__ballot(odd) == 0) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) near = mfma4(pf[e], v[e], near);
+    } else {   // a value that is not finite must not meet the zero scores of the tokens in front of it
+#pragma unroll 1
+      for (int uu = 0; uu < kCT; ++uu) {
+        const float val = __shfl(v[0], (uu >> 2) * 16 + t), val1 = __shfl(v[1], (uu >> 2) * 16 + t);
+        const float val2 = __shfl(v[2], (uu >> 2) * 16 + t), val3 = __shfl(v[3], (uu >> 2) * 16 + t);
+        const float vu = (uu & 3) == 0 ? val : (uu & 3) == 1 ? val1 : (uu & 3) == 2 ? val2 : val3;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int tok = 4 * c + r;
+          if (uu <= tok) near[r] = __builtin_fmaf(rp[((uu >> 2) * 16 + tok) * 4 + (uu & 3)], vu, near[r]);
+        }
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      o[r] = ENTRY ? o[r] + near[r] : __builtin_fmaf(o[r], df[r], near[r]);
+      if constexpr (!ENTRY) vw[r] *= wf[r];
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int tok = base + 4 * c + r;
+      if (live && tok < t1) a.o[((int64_t)tok * heads + head) * dv + col] = skips ? o[r] + skip * x[r] : o[r];
+    }
+    qp += more ? qk_step : 0;
+    rp += more ? rec_step : 0;
+    get_q();
+    get_v(more ? base + kCT : base);
+    __builtin_amdgcn_sched_barrier(0);   // (the requests stay in front of the products that hide them)
+    f32x4 add[KT];   // what the chunk adds, summed by itself: the state is rounded once per chunk
+#pragma unroll
+    for (int s = 0; s < KT; ++s) add[s] = mfma4(kf[s][0], vw[0], f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+    for (int e = 1; e < 4; ++e)
+#pragma unroll
+      for (int s = 0; s < KT; ++s) add[s] = mfma4(kf[s][e], vw[e], add[s]);
+#pragma unroll
+    for (int s = 0; s < KT; ++s) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) S[s][r] = __builtin_fmaf(ENTRY ? lf[s][r] : dlast, S[s][r], add[s][r]);
+    }
+    kp += more ? qk_step : 0;
+    if constexpr (ENTRY) lp += more ? last_step : 0;
+    __builtin_amdgcn_sched_barrier(0);
+    get_k();
+    __builtin_amdgcn_sched_barrier(0);
+  }
+#pragma unroll
+  for (int s = 0; s < KT; ++s)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int kk = 16 * s + 4 * c + r;
+      if (live) st[(int64_t)kk * dv] = S[s][r];
+    }
 }
 
 // One wave per (token, part): out = [o * act(gate)] / sqrt(mean_part(.^2) + eps) * w [* act(gate)] * out_scale.
@@ -587,6 +946,9 @@ __global__ __launch_bounds__(256) void rownorm_rope_cache_vec_kernel(
 
 }  // namespace
 
+constexpr int64_t kChunkRun = 64, kChunkRunFull = 24;   // least longest run of a step for the chunk form (see its scratch)
+constexpr int64_t kChunkFloats = 1ll << 28;     // largest scratch of the chunk form (1 GiB)
+
 #define LL_BY_DTYPE(dtype, CALL)                  \
   do {                                            \
     if (dtype == LL_F16) { CALL(LL_F16); }        \
@@ -596,12 +958,27 @@ __global__ __launch_bounds__(256) void rownorm_rope_cache_vec_kernel(
 
 extern "C" int ll_linear_scan_supported(int64_t dk, int64_t dv) { return dk >= 1 && dk <= 256 && dv >= 1 ? 1 : 0; }
 
-extern "C" int ll_linear_scan(const void* q, int64_t q_ld, const void* k, int64_t k_ld, const void* v, int64_t v_ld, int64_t heads,
+// Floats of scratch for the chunk form, 0 where the walk serves: heads of whole 64-entry groups (16 KT entries, no padding), and a longest run
+// of 64 tokens, or of 24 where the walk's workgroups are enough to fill the chip.  The chunk form costs two launches and about 12 us
+// ahead of its first token, the walk 0.2 - 0.3 us a token when alone; us, walk / chunks: one run of 64 31 / 22 (per entry), 25 / 19
+// (fixed), 25 / 23 (per token), of 32 19 / 19, 14 / 15, 15 / 20; eight of 24 30 / 21, 25 / 18, 26 / 22, four of 24 18 / 20, 14 / 16, 15 / 21.
+extern "C" int64_t ll_linear_scan_chunk_floats(int64_t n, int64_t batch, int64_t heads, int64_t dk, int64_t dv, int64_t qk_rep, int kind,
+                                               int64_t longest_run) {
+  if (n < 1 || batch < 1 || batch > 65535 || heads < 1 || heads > 65535 || dk < 64 || dk > 256 || dk % 64 || dv < 1 || qk_rep < 1 ||
+      heads % qk_rep || longest_run < kChunkRunFull ||
+      (longest_run < kChunkRun && batch * heads * ((dv + 15) / 16) < 1024))
+    return 0;
+  const int64_t slots = n / kCT + batch, terms = kind == 1 ? heads : heads / qk_rep;
+  const int64_t per = terms * (2 * kCT * dk + (kind == 1 ? dk : 0)) + heads * kRec;
+  return per > kChunkFloats / slots ? 0 : slots * per;
+}
+
+static int linear_scan(const void* q, int64_t q_ld, const void* k, int64_t k_ld, const void* v, int64_t v_ld, int64_t heads,
                               int64_t dk, int64_t dv, int64_t qk_rep, int kind, int act, float q_scale, const float* head_decay,
                               const void* gate, int64_t gate_ld, const void* gate_bias, float inv_tau, const void* dt, int64_t dt_ld,
                               const void* dt_bias, const void* a_log, const void* skip, float* o, int64_t batch,
                               const int32_t* seq_start, const int32_t* seq_first_pos, const int32_t* seq_slot, float* state,
-                              float* decay_scratch, int64_t n, int64_t longest_run, int dtype, void* stream) {
+                              float* decay_scratch, float* chunk_scratch, int64_t n, int64_t longest_run, int dtype, void* stream) {
   if (dtype != LL_F16 && dtype != LL_BF16 && dtype != LL_F32) return LL_ERR_DTYPE;
   if (batch < 0 || heads < 1 || heads > 65535 || !ll_linear_scan_supported(dk, dv) || qk_rep < 1 || heads % qk_rep || kind < 0 ||
       kind > 2 || (dv + 15) / 16 > 65535)
@@ -619,11 +996,50 @@ extern "C" int ll_linear_scan(const void* q, int64_t q_ld, const void* k, int64_
   a.head_decay = head_decay; a.gate = gate; a.gate_ld = gate_ld; a.gate_bias = gate_bias; a.inv_tau = inv_tau;
   a.decay_pre = nullptr;
   a.dt = dt; a.dt_ld = dt_ld; a.dt_bias = dt_bias; a.a_log = a_log; a.skip = skip; a.o = o;
+  if (chunk_scratch) {
+    const int64_t floats = ll_linear_scan_chunk_floats(n, batch, heads, dk, dv, qk_rep, kind, longest_run);
+    if (floats <= 0 || !ll_aligned16(chunk_scratch)) return LL_ERR_SHAPE;
+    const int64_t slots = n / kCT + batch, terms = kind == 1 ? heads : heads / qk_rep;
+    ChunkBufs w;
+    w.q = chunk_scratch;
+    w.k = w.q + slots * terms * kCT * dk;
+    w.rec = w.k + slots * terms * kCT * dk;
+    w.last = w.rec + slots * heads * kRec;
+    const int tiles = (int)((dv + 15) / 16), groups = (tiles + 3) / 4;
+    const int64_t pairs = batch * heads, waves = (pairs + 7) / 8 * 8 * groups;
+    if (waves > 0x7fffffffll) return LL_ERR_SHAPE;
+    const dim3 tgrid((unsigned)((longest_run + kCT - 1) / kCT), (unsigned)batch, (unsigned)terms);
+    hipStream_t cst = (hipStream_t)stream;
+    const size_t full = (size_t)3 * kCT * (dk + 4) * sizeof(float), sums = (size_t)256 * 17 * sizeof(float);
+    const size_t clds = full > sums ? full : sums;
+#define CALL_C(DT, KT, EN)                                                                                    \
+  do {                                                                                                        \
+    chunk_terms_kernel<DT, KT, EN><<<tgrid, 256, clds, cst>>>(a, w);                                          \
+    chunk_scan_kernel<DT, KT, EN><<<dim3((unsigned)waves), 256, 0, cst>>>(a, w, (int)pairs, tiles);           \
+  } while (0)
+#define CALL_K(DT, KT) \
+  if (kind == 1) CALL_C(DT, KT, true); \
+  else CALL_C(DT, KT, false)
+#define CALL(DT)                      \
+  if (dk == 64) { CALL_K(DT, 4); }     \
+  else if (dk == 128) { CALL_K(DT, 8); } \
+  else if (dk == 192) { CALL_K(DT, 12); } \
+  else { CALL_K(DT, 16); }
+    LL_BY_DTYPE(dtype, CALL);
+#undef CALL
+#undef CALL_K
+#undef CALL_C
+    return LL_LAUNCH_CHECK();
+  }
   a.tb = dk <= 128 ? 16 : 8;   // tokens staged per pass; a step of short runs asks for less LDS and fits more workgroups per CU
   if (longest_run > 0 && longest_run < a.tb) a.tb = (int)longest_run;
   a.seq_start = seq_start; a.seq_first_pos = seq_first_pos; a.seq_slot = seq_slot; a.state = state;
-  const size_t lds = sizeof(float) * (size_t)(a.tb * (4 * dk + 16 + 16 + 256 + 2));
-  const dim3 grid((unsigned)batch, (unsigned)heads, (unsigned)((dv + 15) / 16));
+  // decoded tokens: 64 columns per workgroup from 128 such workgroups on (8 heads of 128 x 256, us, 16 / 64 columns: 4 sequences 6.4 / 6.0, 32
+  // 21.1 / 12.1; below, 16 heads of 128 x 128: 1 sequence 4.8 / 5.0)
+  const bool wide = longest_run == 1 && dv % 4 == 0 && ll_aligned16(state) && batch * heads * ((dv + 63) / 64) >= 128;
+  const int cw = wide ? 64 : 16;
+  const size_t lds = sizeof(float) * (size_t)(a.tb * (4 * dk + 18 * cw + 2));
+  const dim3 grid((unsigned)batch, (unsigned)heads, (unsigned)((dv + cw - 1) / cw));
   hipStream_t st = (hipStream_t)stream;
   if (kind == 1 && decay_scratch && n > 0) {   // decays once per token and entry, ahead of the scan: fp32 [n, heads dk]
     const int64_t total = n * heads * dk;
@@ -635,7 +1051,11 @@ extern "C" int ll_linear_scan(const void* q, int64_t q_ld, const void* k, int64_
     a.decay_pre = decay_scratch;
   }
   const int rmax = (int)((dk + 15) / 16);
-#define CALL_W(DT, R, E) linear_scan_kernel<DT, R, E><<<grid, 256, lds, st>>>(a)
+#define CALL_W(DT, R, E)                                               \
+  do {                                                                 \
+    if (wide) linear_scan_kernel<DT, R, E, 4><<<grid, 256, lds, st>>>(a); \
+    else linear_scan_kernel<DT, R, E, 1><<<grid, 256, lds, st>>>(a);   \
+  } while (0)
 #define CALL(DT)                                \
   if (dk == 64) CALL_W(DT, 4, true);            \
   else if (dk == 128) CALL_W(DT, 8, true);      \
@@ -647,6 +1067,29 @@ extern "C" int ll_linear_scan(const void* q, int64_t q_ld, const void* k, int64_
 #undef CALL
 #undef CALL_W
   return LL_LAUNCH_CHECK();
+}
+
+extern "C" int ll_linear_scan(const void* q, int64_t q_ld, const void* k, int64_t k_ld, const void* v, int64_t v_ld, int64_t heads,
+                              int64_t dk, int64_t dv, int64_t qk_rep, int kind, int act, float q_scale, const float* head_decay,
+                              const void* gate, int64_t gate_ld, const void* gate_bias, float inv_tau, const void* dt, int64_t dt_ld,
+                              const void* dt_bias, const void* a_log, const void* skip, float* o, int64_t batch,
+                              const int32_t* seq_start, const int32_t* seq_first_pos, const int32_t* seq_slot, float* state,
+                              float* decay_scratch, int64_t n, int64_t longest_run, int dtype, void* stream) {
+  return linear_scan(q, q_ld, k, k_ld, v, v_ld, heads, dk, dv, qk_rep, kind, act, q_scale, head_decay, gate, gate_ld, gate_bias, inv_tau, dt, dt_ld,
+                     dt_bias, a_log, skip, o, batch, seq_start, seq_first_pos, seq_slot, state, decay_scratch, nullptr, n,
+                     longest_run, dtype, stream);
+}
+
+extern "C" int ll_linear_scan_chunks(const void* q, int64_t q_ld, const void* k, int64_t k_ld, const void* v, int64_t v_ld, int64_t heads,
+                                     int64_t dk, int64_t dv, int64_t qk_rep, int kind, int act, float q_scale, const float* head_decay,
+                                     const void* gate, int64_t gate_ld, const void* gate_bias, float inv_tau, const void* dt, int64_t dt_ld,
+                                     const void* dt_bias, const void* a_log, const void* skip, float* o, int64_t batch,
+                                     const int32_t* seq_start, const int32_t* seq_first_pos, const int32_t* seq_slot, float* state,
+                                     float* chunk_scratch, int64_t n, int64_t longest_run, int dtype, void* stream) {
+  if (!chunk_scratch) return LL_ERR_ARG;
+  return linear_scan(q, q_ld, k, k_ld, v, v_ld, heads, dk, dv, qk_rep, kind, act, q_scale, head_decay, gate, gate_ld, gate_bias, inv_tau, dt, dt_ld,
+                     dt_bias, a_log, skip, o, batch, seq_start, seq_first_pos, seq_slot, state, nullptr, chunk_scratch, n,
+                     longest_run, dtype, stream);
 }
 
 extern "C" int ll_gated_out_norm(void* out, int64_t out_ld, const float* o, const void* gate, int64_t gate_ld, int gate_kind,

@@ -186,7 +186,10 @@ def linear_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, heads: int, d
         ``a = exp(-exp(a_log) dt')``, ``b = dt'``.
 
     ``state [slots, heads, dk, dv]`` fp32: a sequence whose run starts at position 0 starts from zeros, every run leaves its
-    final state.  Decays, step sizes, state and read-out are fp32.  Returns ``o`` fp32 ``[n, heads dv]``."""
+    final state.  Decays, step sizes, state and read-out are fp32.  Returns ``o`` fp32 ``[n, heads dv]``.
+
+    Short runs are walked token by token, in the same bits however a prompt is cut; long runs of heads with ``dk`` a multiple of 64 are
+    matrix products over chunks of 16 tokens, whose sums round in another order."""
     L.require_cuda(q, k, v, state, head_decay, gate, gate_bias, dt, dt_bias, a_log, skip)
     n, st = q.shape[0], q.dtype
     qk_heads = heads if qk_heads is None else qk_heads
@@ -226,15 +229,20 @@ def linear_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, heads: int, d
         if dt.dtype != st or dt.shape[0] != n:
             raise ValueError("linear_scan: step sizes in the rows' dtype, one row per token")
     o = torch.empty(n, heads * dv, dtype=torch.float32, device=q.device)
-    # runs of several tokens: the decays per key entry are evaluated once per token ahead of the scan (its column workgroups
-    # would each evaluate them again); decode steps evaluate them in the scan
-    pre = torch.empty(n, heads * dk, dtype=torch.float32, device=q.device) if (kind == 1 and step.longest_run != 1 and dv > 16) else None
-    L.check(L.lib().ll_linear_scan(
+    # long runs: chunks as matrix products.  Other runs of several tokens: the decays per key entry are evaluated once per token ahead of
+    # the scan (its column workgroups would each evaluate them again); decode steps evaluate them in the scan
+    floats = int(L.lib().ll_linear_scan_chunk_floats(n, step.num_seqs, heads, dk, dv, heads // qk_heads, kind, int(step.longest_run)))
+    if floats:
+        scratch, fn = torch.empty(floats, dtype=torch.float32, device=q.device), L.lib().ll_linear_scan_chunks
+    else:
+        ahead = kind == 1 and step.longest_run != 1 and dv > 16
+        scratch, fn = torch.empty(n, heads * dk, dtype=torch.float32, device=q.device) if ahead else None, L.lib().ll_linear_scan
+    L.check(fn(
         q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0), heads, dk, dv, heads // qk_heads, kind,
         1 if act else 0, float(q_scale), L.ptr(head_decay), L.ptr(gate), gate.stride(0) if gate is not None else 0, L.ptr(gate_bias),
         1.0 / float(tau), L.ptr(dt), dt.stride(0) if dt is not None else 0, L.ptr(dt_bias), L.ptr(a_log), L.ptr(skip), o.data_ptr(),
         step.num_seqs, step.seq_start.data_ptr(), step.seq_first_pos.data_ptr(), step.seq_slot.data_ptr(), state.data_ptr(),
-        L.ptr(pre), n, int(step.longest_run), L.dtype_code(st), L.stream_ptr()), "linear_scan")
+        L.ptr(scratch), n, int(step.longest_run), L.dtype_code(st), L.stream_ptr()), "linear_scan")
     return o
 
 

@@ -1,0 +1,112 @@
+"""Linear attention with a decay over runs of many tokens (csrc/linear_mix.hip: chunks of 16 as matrix products) and decoded tokens in
+64-column workgroups, against 64 bits and against the walk token by token, which serves a step whose longest run is not known."""
+
+import dataclasses
+
+import pytest
+import torch
+
+from tests.test_layered_gpu import _step
+
+pytestmark = pytest.mark.gpu
+DEV, F64 = "cuda", torch.float64
+
+
+def _inputs(kind, heads, qk_heads, dk, dv, n, dtype, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+
+    def r(*s):
+        return torch.randn(*s, generator=g, device=DEV).to(dtype)
+
+    # (rows of a fused projection: column ranges, starts off every 16-byte border)
+    rows = r(n, 2 * qk_heads * dk + heads * dv + 3)
+    q, k, v = rows[:, 1:1 + qk_heads * dk], rows[:, 2 + qk_heads * dk:2 + 2 * qk_heads * dk], rows[:, 3 + 2 * qk_heads * dk:]
+    if kind == "fixed":
+        kw = dict(act=True, head_decay=torch.linspace(1.0, 0.25, heads, device=DEV))
+    elif kind == "entry":
+        kw = dict(q_scale=dk ** -0.5, gate=r(n, heads * dk), gate_bias=r(heads * dk), tau=4.0)
+    else:
+        kw = dict(dt=r(n, heads), dt_bias=r(heads), a_log=r(heads), skip=r(heads))
+    return q, k, v, dict(kw, qk_heads=qk_heads)
+
+
+def _exact(q, k, v, heads, dk, dv, runs, state, kw):
+    qk_heads = kw["qk_heads"]
+    q, k, v = q.to(F64).reshape(-1, qk_heads, dk), k.to(F64).reshape(-1, qk_heads, dk), v.to(F64).reshape(-1, heads, dv)
+    b = torch.ones(v.shape[0], heads, 1, dtype=F64, device=DEV)
+    if "head_decay" in kw:
+        q, k, v = (torch.nn.functional.silu(t) for t in (q, k, v))
+        a = kw["head_decay"].to(F64).view(1, heads, 1).expand(v.shape[0], heads, dk)
+    elif "gate" in kw:
+        q = q * float(torch.tensor(kw["q_scale"], dtype=torch.float32))
+        a = torch.exp(torch.nn.functional.logsigmoid(kw["gate"].to(F64) + kw["gate_bias"].to(F64)) / kw["tau"]).view(-1, heads, dk)
+    else:
+        b = torch.nn.functional.softplus(kw["dt"].to(F64) + kw["dt_bias"].to(F64)).unsqueeze(-1)
+        a = torch.exp(-torch.exp(kw["a_log"].to(F64)).view(1, heads, 1) * b).expand(-1, heads, dk)
+    q, k = q.repeat_interleave(heads // qk_heads, 1), k.repeat_interleave(heads // qk_heads, 1)
+    out, state, at = torch.empty_like(v), state.to(F64).clone(), 0
+    for i, (first, count) in enumerate(runs):
+        s = state[i] if first else torch.zeros_like(state[i])
+        for t in range(at, at + count):
+            s = a[t].unsqueeze(-1) * s + k[t].unsqueeze(-1) * (b[t] * v[t]).unsqueeze(1)
+            out[t] = torch.einsum("hkv,hk->hv", s, q[t])
+        state[i], at = s, at + count
+    if "skip" in kw:
+        out += kw["skip"].to(F64).view(1, heads, 1) * v
+    return out.reshape(-1, heads * dv), state
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("kind,heads,qk_heads,dk,dv", [("fixed", 3, 3, 64, 17), ("fixed", 2, 1, 128, 64), ("entry", 2, 2, 128, 40),
+                                                     ("entry", 4, 2, 192, 9), ("token", 34, 2, 64, 4), ("token", 3, 1, 256, 80)])
+@pytest.mark.parametrize("runs", [[(0, 64)], [(5, 1), (9, 79), (0, 16), (3, 17), (0, 1)], [(2, 95), (0, 33)]])
+def test_runs_of_many_tokens(dtype, kind, heads, qk_heads, dk, dv, runs):
+    """Runs that end on and off a chunk of 16, beside single tokens; carried and fresh states; values off every tile of 16 columns."""
+    from lite_llama_amd import _lib
+    from lite_llama_amd.kernels.recurrent import linear_scan
+
+    n = sum(c for _, c in runs)
+    q, k, v, kw = _inputs(kind, heads, qk_heads, dk, dv, n, dtype, dk + dv)
+    step = _step([(i, f, c, 0) for i, (f, c) in enumerate(runs)], None)
+    assert _lib.lib().ll_linear_scan_chunk_floats(n, len(runs), heads, dk, dv, heads // qk_heads, ["fixed", "entry", "token"].index(kind),
+                                                  step.longest_run) > 0
+    start = torch.randn(len(runs), heads, dk, dv, device=DEV)
+    want, want_state = _exact(q, k, v, heads, dk, dv, runs, start, kw)
+    for longest in (step.longest_run, 0):
+        state = start.clone()
+        got = linear_scan(q, k, v, heads, dk, dv, dataclasses.replace(step, longest_run=longest), state, **kw)
+        # fp32 throughout: a few units of rounding per token of a run and per entry of a sum, against the largest result
+        for x, y in ((got, want), (state, want_state)):
+            assert (x.to(F64) - y).abs().max() <= 64 * 2.0 ** -24 * y.abs().max()
+
+
+@pytest.mark.parametrize("kind", ["fixed", "entry", "token"])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("where", [0, 37, 63])
+def test_a_value_that_is_not_finite_leaves_the_tokens_in_front_of_it_alone(kind, bad, where):
+    from lite_llama_amd.kernels.recurrent import linear_scan
+
+    heads, dk, dv, n = 2, 64, 24, 70
+    q, k, v, kw = _inputs(kind, heads, heads, dk, dv, n, torch.bfloat16, 3)
+    step = _step([(0, 0, n, 0)], None)
+    clean = linear_scan(q, k, v, heads, dk, dv, step, torch.zeros(1, heads, dk, dv, device=DEV), **kw)
+    v[where, 5] = bad
+    got = linear_scan(q, k, v, heads, dk, dv, step, torch.zeros(1, heads, dk, dv, device=DEV), **kw)
+    fine = torch.ones(n, heads * dv, dtype=torch.bool, device=DEV)
+    fine[where:, 5] = False
+    # (the chunk of the value adds its scores in another order)
+    assert (got - clean)[fine].abs().max() <= 64 * 2.0 ** -24 * clean.abs().max()
+    assert not got[where:, 5].isfinite().any()
+
+
+@pytest.mark.parametrize("kind,heads,qk_heads,dk,dv", [("fixed", 5, 5, 64, 68), ("entry", 4, 4, 24, 40), ("token", 64, 2, 136, 4)])
+def test_decoded_tokens_are_bit_equal_in_either_workgroup(kind, heads, qk_heads, dk, dv):
+    from lite_llama_amd.kernels.recurrent import linear_scan
+
+    for batch in (1, 40):   # 16-column and 64-column workgroups; the walk where the longest run is not known
+        q, k, v, kw = _inputs(kind, heads, qk_heads, dk, dv, batch, torch.bfloat16, batch)
+        step = _step([(i, i % 3, 1, 0) for i in range(batch)], None)
+        start = torch.randn(batch, heads, dk, dv, device=DEV)
+        states = [start.clone(), start.clone()]
+        outs = [linear_scan(q, k, v, heads, dk, dv, dataclasses.replace(step, longest_run=m), s, **kw) for m, s in zip((1, 0), states)]
+        assert torch.equal(outs[0], outs[1]) and torch.equal(states[0], states[1])
