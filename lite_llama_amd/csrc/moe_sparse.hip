@@ -299,14 +299,15 @@ __global__ __launch_bounds__(256) void moe_rows_gemm_kernel(const void* __restri
                                                             const float* __restrict__ slot_weight, void* __restrict__ out,
                                                             int64_t out_ld, const int32_t* __restrict__ sorted,
                                                             const int32_t* __restrict__ block_expert,
-                                                            const int32_t* __restrict__ num_post, int num_slots, float glu_limit) {
+                                                            const int32_t* __restrict__ num_post, int num_slots, float glu_limit, int shift) {
   constexpr bool GLU = MODE == 1;
   constexpr int BM = 32, BN = 64, BK = 32;
   __shared__ float As[BM][BK + 1];
   __shared__ int rows[BM];
   const int block = blockIdx.x;
   if (block * BM >= num_post[0]) return;
-  const int e = block_expert[block];
+  const int e = block_expert[block >> shift];   // (sorted in blocks of 32 << shift rows)
+  if (sorted[block * BM] >= num_slots) return;
   const int tid = threadIdx.x, tx = tid & 63, ty = tid >> 6;
   if (tid < BM) rows[tid] = sorted[block * BM + tid];
   const int col = blockIdx.y * BN + tx;
@@ -354,202 +355,171 @@ __global__ __launch_bounds__(256) void moe_rows_gemm_kernel(const void* __restri
   }
 }
 
-// ------------------------------------------------------------------------------------------------------------------------
-// grouped products, MFMA form (16-bit storage, K a multiple of 8, 16-byte aligned rows): one wave per 32 sorted rows x 32
-// columns (gate and up: 32 + 32).  Both operands are contraction-contiguous, so a lane's fragment is ONE 16-byte load: lane
-// (t, c) holds entries 8 c .. 8 c + 7 (+ 32 per pass) of row / column t.  Rows = columns of the MFMA (B operand), weight rows
-// = MFMA rows (A operand): the accumulator of lane (t, c) holds weight rows 4 c .. 4 c + 3 of sorted row t.
-// ------------------------------------------------------------------------------------------------------------------------
 struct alignas(16) Q4 {
   uint32_t x, y, z, w;
 };
+
+// ------------------------------------------------------------------------------------------------------------------------
+// grouped products, LDS-tiled MFMA form for blocks of 128 sorted rows: a workgroup of four waves owns a block's rows x 128 weight rows
+// (gate|up: 64 output columns, their gate rows and up rows) and walks the contraction in steps of 64.
+//   * Both tiles go global -> LDS by LDS-DMA as 128-byte row pieces, slot s of row r at s ^ ((r >> 1) & 7) (through the source address):
+//     fragment reads are bank-conflict free.  Weights sit three steps deep, rows two (80 KB: two workgroups per CU): 32 KB of weights of
+//     a CU are always on their way, which is what streaming them from memory needs.  One barrier per step.
+//   * Row tiles without a slot are not multiplied; wave (wr, wc) owns row tiles wr and wr + 2 (of 32 rows) and two weight tiles, so that
+//     a half-full block still keeps every matrix core busy.
+//   * Tiles are dealt to the XCDs in contiguous ranges of the tiles that exist (num_post, a device value), four blocks side by side under
+//     one weight tile: blocks of one expert read it from the XCD's own L2.
+// us for both products, 32 experts of 2048 / 704 with 384 / 706 rows each: 362 / 602 with one buffer filled through registers and two barriers
+// per step, 254 / 427 here (0.48 PFLOP/s: two operand tiles per 128 x 128 results through L2); at 70 rows each 95 us, of which the weights
+// alone need 55.
+// ------------------------------------------------------------------------------------------------------------------------
+__device__ const uint32_t moe_zeros[4] __attribute__((aligned(16))) = {0, 0, 0, 0};   // what pieces behind the contraction's end read
+
+// 64 lanes x 16 bytes from per-lane addresses to 1 KB of LDS at byte `dst` (counted by vmcnt, which the compiler does not see)
+__device__ __forceinline__ void dma16(uint32_t dst, const void* src) {
+  dst = __builtin_amdgcn_readfirstlane(dst);
+  uint32_t keep;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep) : "s"(dst), "v"(src) : "memory");
+}
 template <int DT>
-__device__ __forceinline__ f32x4 mfma16(const Q4& a, const Q4& b, f32x4 c) {
+__device__ __forceinline__ f32x16 mfma32(const Q4& a, const Q4& b, f32x16 c) {
   if constexpr (DT == LL_F16)
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
   else
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
 }
 
 template <int DT, int MODE>
-__global__ __launch_bounds__(64) void moe_rows_gemm_mfma_kernel(const uint16_t* __restrict__ a, int64_t a_ld, int a_div,
-                                                                const uint16_t* __restrict__ w, int64_t w_stride_e, int K, int N,
-                                                                const float* __restrict__ slot_weight, uint16_t* __restrict__ out,
-                                                                int64_t out_ld, const int32_t* __restrict__ sorted,
-                                                                const int32_t* __restrict__ block_expert,
-                                                                const int32_t* __restrict__ num_post, int num_slots, float glu_limit) {
+__global__ __launch_bounds__(256, 2) void moe_rows_gemm_tiled_kernel(const uint16_t* __restrict__ a, int64_t a_ld, int a_div,
+                                                                     const uint16_t* __restrict__ w, int64_t w_stride_e, int K, int N,
+                                                                     const float* __restrict__ slot_weight, uint16_t* __restrict__ out,
+                                                                     int64_t out_ld, const int32_t* __restrict__ sorted,
+                                                                     const int32_t* __restrict__ block_expert,
+                                                                     const int32_t* __restrict__ num_post, int num_slots, float glu_limit,
+                                                                     int tiles_n, int wide) {
   constexpr bool GLU = MODE == 1;
-  constexpr int BM = 32, BN = 32;
-  constexpr int NW = GLU ? 4 : 2;   // weight-row tiles of 16: gate 0..1, up 2..3
-  const int block = blockIdx.x;
-  if (block * BM >= num_post[0]) return;
-  const int e = block_expert[block];
-  const int lane = threadIdx.x, t = lane & 15, c = lane >> 4;
-  const int n0 = blockIdx.y * BN;
-  int slot[2];
-  const uint16_t* arow[2];
+  constexpr int CW = GLU ? 64 : 128, TILE = 128 * 128;   // output columns; bytes of a stage's operand
+  extern __shared__ __attribute__((aligned(16))) unsigned char tile_lds[];   // rows x 2, weights x 3
+  const int blocks = num_post[0] / 128;
+  const int total = blocks * tiles_n;   // (below 2^31: checked on the host for the largest count)
+  const int xcd = blockIdx.x & 7;
+  const int first = (int)((int64_t)total * xcd / 8), last = (int)((int64_t)total * (xcd + 1) / 8);
+  const int at = first + (int)(blockIdx.x >> 3);
+  if (at >= last) return;
+  const int per = 4 * tiles_n, g4 = at / per, in4 = at - g4 * per;
+  const int side = blocks - 4 * g4 < 4 ? blocks - 4 * g4 : 4;
+  const int nt = in4 / side, block = 4 * g4 + (in4 - nt * side);
+  const int e = block_expert[block], n0 = nt * CW;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wr = wave & 1, wc = wave >> 1, tl = lane & 31, h = lane >> 5;
+  const int32_t* srt = sorted + (int64_t)block * 128;
+  // what this thread requests of a step: row (and weight row) 8 (4 wave + j) + lane / 8, one swizzled 16-byte piece of it
+  const char* aptr[4];
+  const char* wptr[4];
+  int piece[4];
 #pragma unroll
-  for (int m = 0; m < 2; ++m) {
-    slot[m] = sorted[block * BM + 16 * m + t];
-    arow[m] = slot[m] < num_slots ? a + (int64_t)(slot[m] / a_div) * a_ld : nullptr;
+  for (int j = 0; j < 4; ++j) {
+    const int r = (wave * 4 + j) * 8 + (lane >> 3);
+    piece[j] = ((lane & 7) ^ ((r >> 1) & 7)) * 8;
+    const int slot = srt[r];   // (rows without a slot read row 0, columns >= N the last: they feed only unstored results)
+    aptr[j] = (const char*)(a + (slot < num_slots ? (int64_t)(slot / a_div) * a_ld : 0) + piece[j]);
+    int col = GLU ? n0 + (r & 63) : n0 + r;
+    col = col < N ? col : N - 1;
+    wptr[j] = (const char*)(w + (int64_t)e * w_stride_e + (GLU && r >= 64 ? (int64_t)N + col : (int64_t)col) * K + piece[j]);
   }
-  const uint16_t* wrow[NW];
+  auto get_a = [&](int s) {
 #pragma unroll
-  for (int j = 0; j < NW; ++j) {
-    const int col = n0 + 16 * (j & 1) + t;
-    const int64_t r = (GLU && j >= 2) ? (int64_t)N + col : col;
-    wrow[j] = col < N ? w + (int64_t)e * w_stride_e + r * K : nullptr;
-  }
-  f32x4 acc[NW][2];
-#pragma unroll
-  for (int j = 0; j < NW; ++j) acc[j][0] = acc[j][1] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // the fragments of the next two contraction steps are requested before the products of the current one: with a handful of
-  // rows per expert (decoding) the launch streams every weight row once, and only loads in flight hide that latency
-  constexpr int AHEAD = 2;
-  Q4 af[AHEAD + 1][2], wf[AHEAD + 1][NW];
-  auto fetch = [&](int k0, Q4 (&fa)[2], Q4 (&fw)[NW]) {
-    const int ch = k0 + 8 * c;
-    const bool in = ch < K;
-#pragma unroll
-    for (int m = 0; m < 2; ++m) fa[m] = (in && arow[m]) ? *reinterpret_cast<const Q4*>(arow[m] + ch) : Q4{0, 0, 0, 0};
-#pragma unroll
-    for (int j = 0; j < NW; ++j) fw[j] = (in && wrow[j]) ? *reinterpret_cast<const Q4*>(wrow[j] + ch) : Q4{0, 0, 0, 0};
+    for (int j = 0; j < 4; ++j)
+      dma16((uint32_t)((s & 1) * TILE + (wave * 4 + j) * 1024), s * 64 + piece[j] < K ? aptr[j] + (int64_t)s * 128 : (const char*)moe_zeros);
   };
+  auto get_w = [&](int s, int buf) {
 #pragma unroll
-  for (int a2 = 0; a2 < AHEAD; ++a2) fetch(32 * a2, af[a2], wf[a2]);
-  for (int k0 = 0; k0 < K; k0 += 32 * (AHEAD + 1)) {
+    for (int j = 0; j < 4; ++j)
+      dma16((uint32_t)((2 + buf) * TILE + (wave * 4 + j) * 1024), s * 64 + piece[j] < K ? wptr[j] + (int64_t)s * 128 : (const char*)moe_zeros);
+  };
+  const bool act0 = srt[32 * wr] < num_slots, act1 = srt[32 * (wr + 2)] < num_slots;   // (an expert's empty rows stand last)
+  f32x16 acc[2][2];
 #pragma unroll
-    for (int u = 0; u <= AHEAD; ++u) {   // (slot u holds step k0 + 32 u; the slot just freed receives step + AHEAD)
-      fetch(k0 + 32 * (u + AHEAD), af[(u + AHEAD) % (AHEAD + 1)], wf[(u + AHEAD) % (AHEAD + 1)]);
+  for (int m = 0; m < 2; ++m)
 #pragma unroll
-      for (int j = 0; j < NW; ++j) {
-        acc[j][0] = mfma16<DT>(wf[u][j], af[u][0], acc[j][0]);
-        acc[j][1] = mfma16<DT>(wf[u][j], af[u][1], acc[j][1]);
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[m][j][r] = 0.f;
+  const int sw = (tl >> 1) & 7;
+  const unsigned char* arow = tile_lds + (32 * wr + tl) * 128;
+  const unsigned char* wrow0 = tile_lds + 2 * TILE + ((GLU ? 32 * wc : 64 * wc) + tl) * 128;
+  const int wrow1 = (GLU ? 64 : 32) * 128;
+  get_a(0);
+  get_w(0, 0);
+  get_w(1, 1);
+  const int steps = (K + 63) / 64;
+  int buf = 0;
+  for (int s = 0; s < steps; ++s) {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0074);   // all but the last four requests (the weights of step s + 1); own fragment reads
+    __builtin_amdgcn_s_barrier();
+    get_a(s + 1);
+    get_w(s + 2, buf == 0 ? 2 : buf - 1);   // (the buffer step s - 1 has been read from)
+    const unsigned char* ap = arow + (s & 1) * TILE;
+    const unsigned char* wp = wrow0 + buf * TILE;
+    if (act0) {
+      Q4 w0[4], w1[4], a0[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int o = ((2 * q + h) ^ sw) * 16;
+        w0[q] = *reinterpret_cast<const Q4*>(wp + o);
+        w1[q] = *reinterpret_cast<const Q4*>(wp + wrow1 + o);
+        a0[q] = *reinterpret_cast<const Q4*>(ap + o);
+      }
+      if (act1) {
+        Q4 a1[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) a1[q] = *reinterpret_cast<const Q4*>(ap + 64 * 128 + ((2 * q + h) ^ sw) * 16);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          acc[0][0] = mfma32<DT>(w0[q], a0[q], acc[0][0]);
+          acc[0][1] = mfma32<DT>(w1[q], a0[q], acc[0][1]);
+          acc[1][0] = mfma32<DT>(w0[q], a1[q], acc[1][0]);
+          acc[1][1] = mfma32<DT>(w1[q], a1[q], acc[1][1]);
+        }
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          acc[0][0] = mfma32<DT>(w0[q], a0[q], acc[0][0]);
+          acc[0][1] = mfma32<DT>(w1[q], a0[q], acc[0][1]);
+        }
       }
     }
+    buf = buf == 2 ? 0 : buf + 1;
   }
+  __builtin_amdgcn_s_waitcnt(0x0070);   // (requests past the end have landed before the LDS is given back)
+  if (!act0) return;
 #pragma unroll
   for (int m = 0; m < 2; ++m) {
-    if (slot[m] >= num_slots) continue;
-    const float sw = (!GLU && slot_weight) ? slot_weight[slot[m]] : 1.0f;
-    uint16_t* orow = out + (int64_t)slot[m] * out_ld;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int col = n0 + 16 * j + 4 * c + r;
-        if (col >= N) continue;
-        float v;
-        if (GLU) {
-          const float g = acc[j][m][r];
-          v = glu_pair<DT>(g, acc[j + 2][m][r], glu_limit);
-        } else {
-          v = slot_value<MODE>(acc[j][m][r], sw);
-        }
-        orow[col] = from_f32<DT>(v);
-      }
-    }
-  }
-}
-
-// ------------------------------------------------------------------------------------------------------------------------
-// grouped products, LDS-tiled MFMA form for prompt-sized inputs: a workgroup of four waves owns 128 sorted rows x 128 weight
-// rows (gate|up: 64 output columns, gate rows and up rows of the same columns side by side) and walks the contraction in steps
-// of 64.  Both tiles are fetched ONCE per workgroup (global -> registers -> LDS, the next step's loads in flight under the
-// products); a wave multiplies all eight row tiles with two weight tiles (its gate and its up tile), so every A fragment read
-// from LDS feeds two MFMAs and every weight fragment eight.
-// ------------------------------------------------------------------------------------------------------------------------
-template <int DT, int MODE>
-__global__ __launch_bounds__(256) void moe_rows_gemm_tiled_kernel(const uint16_t* __restrict__ a, int64_t a_ld, int a_div,
-                                                                  const uint16_t* __restrict__ w, int64_t w_stride_e, int K, int N,
-                                                                  const float* __restrict__ slot_weight, uint16_t* __restrict__ out,
-                                                                  int64_t out_ld, const int32_t* __restrict__ sorted,
-                                                                  const int32_t* __restrict__ block_expert,
-                                                                  const int32_t* __restrict__ num_post, int num_slots, float glu_limit) {
-  constexpr bool GLU = MODE == 1;
-  constexpr int BM = 128, WN = 128, BK = 64, STR = BK + 8, CW = GLU ? 64 : 128;
-  __shared__ __attribute__((aligned(16))) uint16_t lds_a[BM * STR];
-  __shared__ __attribute__((aligned(16))) uint16_t lds_w[WN * STR];
-  __shared__ int rows_s[BM];
-  const int block = blockIdx.x;
-  if (block * BM >= num_post[0]) return;
-  const int e = block_expert[block];
-  const int n0 = blockIdx.y * CW;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, t = lane & 15, c = lane >> 4;
-  if (tid < BM) rows_s[tid] = sorted[block * BM + tid];
-  __syncthreads();
-  const uint16_t* aptr[4];
-  const uint16_t* wptr[4];
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int i = tid + 256 * u, row = i >> 3, pc = i & 7;
-    const int slot = rows_s[row];
-    aptr[u] = slot < num_slots ? a + (int64_t)(slot / a_div) * a_ld + 8 * pc : nullptr;
-    const int col = GLU ? n0 + (row & 63) : n0 + row;
-    const int64_t grow = (GLU && row >= 64) ? (int64_t)N + col : col;
-    wptr[u] = col < N ? w + (int64_t)e * w_stride_e + grow * K + 8 * pc : nullptr;
-  }
-  Q4 ra[4], rw[4];
-#define LL_FETCH(K0)                                                                                        \
-  _Pragma("unroll") for (int u = 0; u < 4; ++u) {                                                           \
-    const bool in = (K0) + 8 * ((tid + 256 * u) & 7) < K;                                                   \
-    ra[u] = (in && aptr[u]) ? *reinterpret_cast<const Q4*>(aptr[u] + (K0)) : Q4{0, 0, 0, 0};                \
-    rw[u] = (in && wptr[u]) ? *reinterpret_cast<const Q4*>(wptr[u] + (K0)) : Q4{0, 0, 0, 0};                \
-  }
-#define LL_STAGE()                                                                                          \
-  _Pragma("unroll") for (int u = 0; u < 4; ++u) {                                                           \
-    const int i = tid + 256 * u, row = i >> 3, pc = i & 7;                                                  \
-    *reinterpret_cast<Q4*>(&lds_a[row * STR + 8 * pc]) = ra[u];                                             \
-    *reinterpret_cast<Q4*>(&lds_w[row * STR + 8 * pc]) = rw[u];                                             \
-  }
-  const int tile0 = GLU ? wave : 2 * wave, tile1 = GLU ? 4 + wave : 2 * wave + 1;
-  f32x4 acc[2][8];
-#pragma unroll
-  for (int m = 0; m < 8; ++m) acc[0][m] = acc[1][m] = f32x4{0.f, 0.f, 0.f, 0.f};
-  LL_FETCH(0)
-  LL_STAGE()
-  __syncthreads();
-  for (int k0 = 0; k0 < K; k0 += BK) {
-    if (k0 + BK < K) { LL_FETCH(k0 + BK) }
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      const Q4 w0 = *reinterpret_cast<const Q4*>(&lds_w[(16 * tile0 + t) * STR + 32 * ks + 8 * c]);
-      const Q4 w1 = *reinterpret_cast<const Q4*>(&lds_w[(16 * tile1 + t) * STR + 32 * ks + 8 * c]);
-#pragma unroll
-      for (int m = 0; m < 8; ++m) {
-        const Q4 af = *reinterpret_cast<const Q4*>(&lds_a[(16 * m + t) * STR + 32 * ks + 8 * c]);
-        acc[0][m] = mfma16<DT>(w0, af, acc[0][m]);
-        acc[1][m] = mfma16<DT>(w1, af, acc[1][m]);
-      }
-    }
-    __syncthreads();   // everybody has read this step's tiles
-    if (k0 + BK < K) { LL_STAGE() }
-    __syncthreads();
-  }
-#undef LL_FETCH
-#undef LL_STAGE
-#pragma unroll
-  for (int m = 0; m < 8; ++m) {
-    const int slot = rows_s[16 * m + t];
+    const int slot = srt[32 * (wr + 2 * m) + tl];
     if (slot >= num_slots) continue;
+    const float weight = !GLU && slot_weight ? slot_weight[slot] : 1.0f;
     uint16_t* orow = out + (int64_t)slot * out_ld;
-    if (GLU) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int col = n0 + 16 * wave + 4 * c + r;
-        const float g = acc[0][m][r];
-        if (col < N) orow[col] = from_f32<DT>(glu_pair<DT>(g, acc[1][m][r], glu_limit));
-      }
-    } else {
-      const float sw = slot_weight ? slot_weight[slot] : 1.0f;
+    for (int j = 0; j < (GLU ? 1 : 2); ++j)
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int q = 0; q < 4; ++q) {   // result 4 q + i of the lane: weight row 8 q + 4 h + i of the tile
+        const int col = n0 + (GLU ? 32 * wc : 64 * wc + 32 * j) + 8 * q + 4 * h;
+        uint16_t y[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int col = n0 + 16 * (2 * wave + j) + 4 * c + r;
-          if (col < N) orow[col] = from_f32<DT>(slot_value<MODE>(acc[j][m][r], sw));
+        for (int i = 0; i < 4; ++i) {
+          const float v = acc[m][j][4 * q + i];
+          y[i] = from_f32<DT>(GLU ? glu_pair<DT>(v, acc[m][1][4 * q + i], glu_limit) : slot_value<MODE>(v, weight));
         }
-    }
+        if (wide) {
+          if (col < N) *reinterpret_cast<uint2*>(orow + col) = uint2{(uint32_t)y[0] | (uint32_t)y[1] << 16, (uint32_t)y[2] | (uint32_t)y[3] << 16};
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (col + i < N) orow[col + i] = y[i];
+        }
+      }
   }
 }
 
@@ -622,11 +592,14 @@ extern "C" int ll_group_router(const void* h, int64_t h_ld, const void* w_router
   return LL_LAUNCH_CHECK();
 }
 
-// rows per sorted block: 128 (the LDS-tiled form) when the experts average at least 128 slots each and the 16-bit matrix-core
-// forms apply, else 32
+// rows per sorted block: 128 (the LDS-tiled form) where a 16-bit matrix-core product applies to either contraction, else 32.  At any number of
+// rows: a form of one wave per 32 rows x 32 columns straight from memory, which it replaced, was slower down to a few decoded tokens (both
+// products, us, that form -> this one: 64 experts of 3072 / 512, 6 tokens with 8 experts each 123 -> 98, 32 163 -> 134, 128 196 -> 145, 800
+// 559 -> 200; 32 experts of 2048 / 704, 32 tokens with 4 each 81 -> 74, 600 205 -> 95)
 extern "C" int64_t ll_moe_rows_block(int64_t num_slots, int64_t experts, int64_t width, int64_t ff, int dtype) {
-  static const bool small = getenv("LL_MOE_ROWS_SMALL") != nullptr;   // A/B knob, read once
-  return (!small && dtype != LL_F32 && width % 8 == 0 && ff % 8 == 0 && num_slots >= 128 * experts) ? 128 : 32;
+  (void)num_slots;
+  (void)experts;
+  return dtype != LL_F32 && (width % 8 == 0 || ff % 8 == 0) ? 128 : 32;
 }
 
 // counts: int32 scratch [experts].  sorted [num_slots + experts * (block - 1)], block_expert [ceil(that / block)], num_post [1]
@@ -659,37 +632,40 @@ extern "C" int ll_moe_rows_gemm(const void* a, int64_t a_ld, int64_t a_div, cons
     return LL_ERR_SHAPE;
   if (num_slots == 0) return LL_OK;
   if (!a || !w || !out || !sorted || !block_expert || !num_post) return LL_ERR_ARG;
-  const int64_t max_blocks = (num_slots + experts * (block - 1) + block - 1) / block;
+  const int64_t max_rows = num_slots + experts * (block - 1);
   hipStream_t st = (hipStream_t)stream;
   static const bool no_mfma = getenv("LL_MOE_ROWS_VALU") != nullptr;   // A/B knob, read once
   const bool mfma = !no_mfma && dtype != LL_F32 && K % 8 == 0 && a_ld % 8 == 0 && w_stride_e % 8 == 0 && ll_aligned16(a) && ll_aligned16(w);
-  if (block == 128) {
-    if (!mfma) return LL_ERR_SHAPE;   // (blocks of 128 rows are only sorted for the tiled matrix-core form)
-    const dim3 grid((unsigned)max_blocks, (unsigned)((N + (mode == 1 ? 63 : 127)) / (mode == 1 ? 64 : 128)));
-#define CALL_T(DT, G)                                                                                                          \
-  moe_rows_gemm_tiled_kernel<DT, G><<<grid, 256, 0, st>>>((const uint16_t*)a, a_ld, (int)a_div, (const uint16_t*)w, w_stride_e, \
-                                                          (int)K, (int)N, slot_weight, (uint16_t*)out, out_ld, sorted, block_expert, \
-                                                          num_post, (int)num_slots, glu_limit)
+  if (block == 128 && mfma) {
+    const int64_t tiles_n = (N + (mode == 1 ? 63 : 127)) / (mode == 1 ? 64 : 128), max_tiles = (max_rows + 127) / 128 * tiles_n;
+    if (max_tiles > 0x7ffffff0ll) return LL_ERR_SHAPE;
+    const unsigned grid = (unsigned)((max_tiles + 7) / 8 * 8 + 8);   // (a range of an XCD may hold one tile more than an eighth)
+    const int wide = N % 4 == 0 && out_ld % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & 7u) == 0;
+    constexpr int bytes = 5 * 128 * 128;
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+#define CALL_T(DT, G)                                                                                                             \
+  do {                                                                                                                            \
+    static bool attr[16] = {false};                                                                                               \
+    if (dev >= 0 && dev < 16 && !attr[dev]) {                                                                                     \
+      (void)hipFuncSetAttribute((const void*)moe_rows_gemm_tiled_kernel<DT, G>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes); \
+      attr[dev] = true;                                                                                                           \
+    }                                                                                                                             \
+    moe_rows_gemm_tiled_kernel<DT, G><<<dim3(grid), 256, bytes, st>>>((const uint16_t*)a, a_ld, (int)a_div, (const uint16_t*)w,   \
+                                                                      w_stride_e, (int)K, (int)N, slot_weight, (uint16_t*)out, out_ld, \
+                                                                      sorted, block_expert, num_post, (int)num_slots, glu_limit, \
+                                                                      (int)tiles_n, wide);                                        \
+  } while (0)
     if (dtype == LL_F16) { if (mode == 1) CALL_T(LL_F16, 1); else if (mode == 2) CALL_T(LL_F16, 2); else CALL_T(LL_F16, 0); }
     else { if (mode == 1) CALL_T(LL_BF16, 1); else if (mode == 2) CALL_T(LL_BF16, 2); else CALL_T(LL_BF16, 0); }
 #undef CALL_T
     return LL_LAUNCH_CHECK();
   }
-  if (mfma) {
-    const dim3 grid((unsigned)max_blocks, (unsigned)((N + 31) / 32));
-#define CALL_M(DT, G)                                                                                                         \
-  moe_rows_gemm_mfma_kernel<DT, G><<<grid, 64, 0, st>>>((const uint16_t*)a, a_ld, (int)a_div, (const uint16_t*)w, w_stride_e, \
-                                                        (int)K, (int)N, slot_weight, (uint16_t*)out, out_ld, sorted, block_expert, \
-                                                        num_post, (int)num_slots, glu_limit)
-    if (dtype == LL_F16) { if (mode == 1) CALL_M(LL_F16, 1); else if (mode == 2) CALL_M(LL_F16, 2); else CALL_M(LL_F16, 0); }
-    else { if (mode == 1) CALL_M(LL_BF16, 1); else if (mode == 2) CALL_M(LL_BF16, 2); else CALL_M(LL_BF16, 0); }
-#undef CALL_M
-    return LL_LAUNCH_CHECK();
-  }
+  const int64_t max_blocks = (max_rows + 31) / 32;   // (the plain form takes either order: blocks of 128 rows are four of its own)
   const dim3 grid((unsigned)max_blocks, (unsigned)((N + 63) / 64));
 #define CALL_P(DT, G)                                                                                                        \
   moe_rows_gemm_kernel<DT, G><<<grid, 256, 0, st>>>(a, a_ld, (int)a_div, w, w_stride_e, (int)K, (int)N, slot_weight, out, out_ld, sorted, \
-                                                    block_expert, num_post, (int)num_slots, glu_limit)
+                                                    block_expert, num_post, (int)num_slots, glu_limit, block == 128 ? 2 : 0)
 #define CALL(DT)                        \
   if (mode == 1) CALL_P(DT, 1);         \
   else if (mode == 2) CALL_P(DT, 2);    \

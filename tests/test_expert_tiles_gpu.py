@@ -1,0 +1,53 @@
+"""Grouped expert products over sorted blocks of 128 rows (csrc/moe_sparse.hip) against 64-bit products of the same operands: experts
+whose last block holds one row, a row tile, a row more; contractions and widths off every tile; the plain form over the same order."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV, F64 = "cuda", torch.float64
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("width,ff", [(8, 8), (72, 200), (136, 64), (192, 132), (100, 72), (256, 24)])
+@pytest.mark.parametrize("form", ["silu", "clamped", "square"])
+def test_experts_of_every_load(dtype, width, ff, form):
+    from lite_llama_amd.kernels.fused_moe import sparse_glu_experts, sparse_square_experts
+
+    loads = [1, 0, 31, 32, 33, 64, 65, 96, 127, 128, 129, 300]
+    experts, top = len(loads), 2
+    g = torch.Generator(device=DEV).manual_seed(width + ff)
+
+    def r(*s, std=1.0):
+        return (torch.randn(*s, generator=g, device=DEV) * std).to(dtype)
+
+    ids = torch.cat([torch.full((c,), e) for e, c in enumerate(loads)] + [torch.full((sum(loads) % 2,), 11)])
+    ids = ids[torch.randperm(ids.numel(), generator=torch.Generator().manual_seed(1))].view(-1, top).to(torch.int32).to(DEV)
+    if form != "square":
+        ids[5, 1] = experts + 3          # a slot that no expert serves
+    n = ids.shape[0]
+    h, weights = r(n, width), torch.rand(n, top, generator=g, device=DEV) + 0.1
+    up = r(experts, ff if form == "square" else 2 * ff, width, std=width ** -0.5)
+    down = r(experts, width, ff, std=ff ** -0.5)
+    if form == "square":
+        got = sparse_square_experts(h, up, down, ids, weights)
+    else:
+        got = sparse_glu_experts(h, up, down, ids, weights, limit=1.5 if form == "clamped" else None, skipped_ids=True)
+    want, mid = torch.zeros(n, top, width, dtype=F64, device=DEV), torch.zeros(n, top, 1, dtype=F64, device=DEV)
+    for e in range(experts):
+        at = (ids == e).nonzero(as_tuple=True)
+        x, wt = h[at[0]].to(F64), weights[at].to(F64)[:, None]
+        if form == "square":
+            act, wt = torch.relu(x @ up[e].to(F64).T * wt) ** 2, torch.ones_like(wt)
+        else:
+            gate, u = (x @ w.to(F64).T for w in (up[e, :ff], up[e, ff:]))
+            if form == "clamped":
+                gate, u = gate.clamp(max=1.5), u.clamp(-1.5, 1.5) + 1
+                act = gate * torch.sigmoid(1.702 * gate) * u
+            else:
+                act = torch.nn.functional.silu(gate) * u
+        want[at] = (act @ down[e].to(F64).T) * wt
+        mid[at] = act.norm(dim=1, keepdim=True) * wt * ff ** -0.5
+    # two roundings to 16 bits: the activations' (each a half unit, met by weights of std ff^-1/2: 6 deviations) and the result's own
+    unit = 2.0 ** (-11 if dtype == torch.float16 else -8)
+    assert ((got.to(F64) - want).abs() <= unit * (want.abs() + 6 * mid) + 2.0 ** -14 * unit).all()
