@@ -203,8 +203,10 @@ def has(name: str) -> bool:
     return hasattr(lib(), name)
 
 
-def stream_ptr() -> int:
-    return torch.cuda.current_stream().cuda_stream
+def stream_ptr(index: int | None = None) -> int:
+    """The current stream of the device ``index`` (the current device).  The handle straight from the runtime: building a
+    ``torch.cuda.Stream`` around it costs about 5 us, on every launch."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def dtype_code(dt: torch.dtype) -> int:
@@ -267,7 +269,7 @@ def scratch_keys(device: torch.device):
     cap = (device.type, idx, "capture")
     if torch.cuda.is_current_stream_capturing():
         return cap, cap
-    return (device.type, idx, torch.cuda.current_stream(idx).cuda_stream), cap
+    return (device.type, idx, stream_ptr(idx)), cap
 
 
 def _grow_gemm_ws(key, device, floats: int, ints: int):

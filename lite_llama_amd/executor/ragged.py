@@ -13,6 +13,7 @@ from __future__ import annotations
 from collections.abc import Sequence
 from dataclasses import dataclass, field
 
+import numpy as np
 import torch
 
 from .paged_kv import PagedStateCache
@@ -125,10 +126,11 @@ class RaggedRunner:
         slots = [s for s, _ in entries]
         if len(set(slots)) != len(slots):
             raise ValueError("a request rides at most once in a step")
-        counts = [len(t) for _, t in entries]
+        tokens = [[int(t) for t in toks] for _, toks in entries]
+        counts = [len(t) for t in tokens]
         if min(counts) < 1:
             raise ValueError("every entry brings at least one token")
-        if self.vocab_size and not all(0 <= int(t) < self.vocab_size for _, toks in entries for t in toks):
+        if self.vocab_size and not all(0 <= min(t) and max(t) < self.vocab_size for t in tokens):
             raise ValueError(f"token ids lie in 0 .. {self.vocab_size - 1}")
         first = [self._len[s] for s in slots]
         new_len = [f + c for f, c in zip(first, counts)]
@@ -137,20 +139,30 @@ class RaggedRunner:
         need = sum(self.blocks_for(n) - self.blocks_for(f) for n, f in zip(new_len, first))
         if self.blocks_held() + need > self.total_blocks:
             raise RuntimeError(f"the block pool is exhausted: {self.blocks_held()} of {self.total_blocks} blocks held, {need} more asked")
-        starts, tok_seq, tok_pos, pick, tokens = [0], [], [], [], []
         longest = max(counts)
-        for i, ((_, toks), f, c) in enumerate(zip(entries, first, counts)):
+        starts, tok_seq, tok_pos, pick, flat = [0], [], [], [], []
+        for i, (toks, f, c) in enumerate(zip(tokens, first, counts)):
             starts.append(starts[-1] + c)
-            tok_seq += [i] * c
-            tok_pos += range(f, f + c)
-            pick += range(i * longest + longest - c, (i + 1) * longest)
-            tokens += [int(t) for t in toks]
-        parts = [tok_seq, tok_pos, starts, first, slots, [self._parity[s] for s in slots], new_len, pick, tokens]
+            tok_seq.append(np.full(c, i, np.int32))
+            tok_pos.append(np.arange(f, f + c, dtype=np.int32))
+            pick.append(np.arange(i * longest + longest - c, (i + 1) * longest, dtype=np.int32))
+            flat += toks
+        parts = [np.concatenate(tok_seq), np.concatenate(tok_pos), starts, first, slots, [self._parity[s] for s in slots], new_len,
+                 np.concatenate(pick), flat]
+        parts = [np.asarray(p, dtype=np.int32) for p in parts]
         for s, n in zip(slots, new_len):
             self._len[s] = n
             self._parity[s] ^= 1
         self._all_start = not any(first)
         return parts, longest, max(new_len)
+
+    def _host(self, parts) -> torch.Tensor:
+        """The parts as one int32 host tensor: page-locked for a GPU, so that its copy waits for nothing that is queued there (the
+        allocator keeps the memory until the copy is done)."""
+        sizes = [len(p) for p in parts]
+        host = torch.empty(sum(sizes), dtype=torch.int32, pin_memory=self.device.type == "cuda")
+        np.concatenate(parts, out=host.numpy())
+        return host
 
     @staticmethod
     def _views(packed: torch.Tensor, sizes):
@@ -163,12 +175,18 @@ class RaggedRunner:
     def build_step(self, entries: Sequence[tuple[int, Sequence[int]]]) -> tuple[RaggedStep, torch.Tensor]:
         """The step's device vectors: every one of them crosses to the device in ONE copy (a packed int32 tensor, sliced into
         views); blocks for the new tokens are reserved on the device."""
+        return self._build(entries, [])[:2]
+
+    def _build(self, entries, logits_rows):
+        """:meth:`build_step` and the listed rows (int64, ``None`` for an empty list), which ride in the same copy."""
         parts, longest, longest_context = self._plan(entries)
-        packed = torch.tensor([v for part in parts for v in part], dtype=torch.int32).to(self.device, non_blocking=True)
-        return self._step_from(packed, [len(p) for p in parts], len(entries), longest, longest_context)
+        parts.append(np.asarray(logits_rows, dtype=np.int32))
+        packed = self._host(parts).to(self.device, non_blocking=True)
+        step, token_ids = self._step_from(packed, [len(p) for p in parts], len(entries), longest, longest_context)
+        return step, token_ids, packed[packed.numel() - len(logits_rows):].long() if logits_rows else None
 
     def _step_from(self, packed, sizes, num_seqs, longest, longest_context):
-        v_tok_seq, v_tok_pos, v_starts, v_first, v_slots, v_parity, v_new_len, v_pick, v_tokens = self._views(packed, sizes)
+        v_tok_seq, v_tok_pos, v_starts, v_first, v_slots, v_parity, v_new_len, v_pick, v_tokens = self._views(packed, sizes)[:9]
         rows = self.cache.extend(v_slots, v_new_len, longest, self.token_table)
         select = rows.reshape(-1)[v_pick].contiguous() if longest > 1 else rows.reshape(-1)
         step = RaggedStep(num_tokens=v_tokens.numel(), num_seqs=num_seqs, tok_seq=v_tok_seq, tok_pos=v_tok_pos, select=select,
@@ -191,8 +209,7 @@ class RaggedRunner:
         if (self.capture_decode and collect_layers is None and all(len(t) == 1 for _, t in entries)
                 and logits_rows == list(range(len(entries)))):
             return self._decode_step_captured(entries)
-        step, token_ids = self.build_step(entries)
-        rows = torch.tensor(logits_rows, dtype=torch.long, device=self.device) if logits_rows else None
+        step, token_ids, rows = self._build(entries, logits_rows)
         return self.model(token_ids, step, self.cache, self.token_table, logits_rows=rows, collect_layers=collect_layers)
 
     # ------------------------------------------------------------------ captured decode steps ---- #
@@ -207,7 +224,7 @@ class RaggedRunner:
         part = int(L.lib().ll_ragged_attention_partition()) if L.has("ll_ragged_attention_partition") else 256
         parts, longest, longest_context = self._plan(entries)
         key = (tuple(s for s, _ in entries), -(-longest_context // part))
-        host = torch.tensor([v for p in parts for v in p], dtype=torch.int32)
+        host = self._host(parts)
         cell = self._cells.get(key)
         if cell is None:
             self._sightings[key] = self._sightings.get(key, 0) + 1
@@ -216,7 +233,7 @@ class RaggedRunner:
                 rows = torch.arange(len(entries), device=self.device)
                 return self.model(token_ids, step, self.cache, self.token_table, logits_rows=rows)
             cell = self._capture_cell(key, host, [len(p) for p in parts], len(entries), key[1] * part)
-        cell.packed.copy_(host)   # (pageable source: the copy has left the host buffer when this returns)
+        cell.packed.copy_(host, non_blocking=True)   # (behind the graph's previous replay; the next step is planned meanwhile)
         cell.graph.replay()
         self.replays += 1
         return cell.logits
