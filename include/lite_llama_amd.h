@@ -742,8 +742,8 @@ int ll_moe_rows_gemm(const void* a, int64_t a_ld, int64_t a_div, const void* w, 
  * from zeros.  decay_scratch (kind 1; fp32 [n, heads dk] for the step's n tokens, or NULL): the decays are evaluated once per
  * token and entry ahead of the scan instead of by every column workgroup (same values).  longest_run: most tokens a sequence
  * of the step brings (0: unknown); sizes the staging buffers, and 1 selects the form for decoded tokens.
- * ll_linear_scan_chunks: the same over runs of many tokens, in chunks of 16 as fp32 matrix products: fp32 sums in another order than the
- * walk's.  longest_run exact; chunk_scratch: ll_linear_scan_chunk_floats(...) fp32, 16-byte aligned (0: not served, use ll_linear_scan).
+ * ll_linear_scan_walk: the same bits over runs of many tokens, in two kernels.  walk_scratch: ll_linear_scan_walk_floats(...) fp32,
+ * 16-byte aligned (0: not served, use ll_linear_scan).
  * ll_gated_out_norm: o fp32 [n, width] -> RMS norm over `parts` equal consecutive parts, times w[(channel) mod w_len] (NULL:
  * none), times act(gate) (gate_kind 0 none, 1 silu, 2 sigmoid; gate_first: before the norm), times out_scale -> out rows of
  * stride out_ld.
@@ -760,14 +760,14 @@ int ll_linear_scan(const void* q, int64_t q_ld, const void* k, int64_t k_ld, con
                    const void* dt_bias, const void* a_log, const void* skip, float* o, int64_t batch,
                    const int32_t* seq_start, const int32_t* seq_first_pos, const int32_t* seq_slot, float* state,
                    float* decay_scratch, int64_t n, int64_t longest_run, int dtype, void* stream);
-int64_t ll_linear_scan_chunk_floats(int64_t n, int64_t batch, int64_t heads, int64_t dk, int64_t dv, int64_t qk_rep, int kind,
+int64_t ll_linear_scan_walk_floats(int64_t n, int64_t batch, int64_t heads, int64_t dk, int64_t dv, int64_t qk_rep, int kind,
                                     int64_t longest_run);
-int ll_linear_scan_chunks(const void* q, int64_t q_ld, const void* k, int64_t k_ld, const void* v, int64_t v_ld, int64_t heads,
+int ll_linear_scan_walk(const void* q, int64_t q_ld, const void* k, int64_t k_ld, const void* v, int64_t v_ld, int64_t heads,
                    int64_t dk, int64_t dv, int64_t qk_rep, int kind, int act, float q_scale, const float* head_decay,
                    const void* gate, int64_t gate_ld, const void* gate_bias, float inv_tau, const void* dt, int64_t dt_ld,
                    const void* dt_bias, const void* a_log, const void* skip, float* o, int64_t batch,
                    const int32_t* seq_start, const int32_t* seq_first_pos, const int32_t* seq_slot, float* state,
-                   float* chunk_scratch, int64_t n, int64_t longest_run, int dtype, void* stream);
+                   float* walk_scratch, int64_t n, int64_t longest_run, int dtype, void* stream);
 int ll_gated_out_norm(void* out, int64_t out_ld, const float* o, const void* gate, int64_t gate_ld, int gate_kind,
                       int gate_first, const void* w, int64_t w_len, float eps, float out_scale, int64_t n, int64_t width,
                       int64_t parts, int dtype, void* stream);

@@ -137,8 +137,8 @@ SIGNATURES = {
     "ll_moe_rows_gemm": [P, L, L, P, L, L, L, I, P, P, L, P, P, P, L, L, L, F, I, P],
     "ll_linear_scan_supported": [L, L],
     "ll_linear_scan": [P, L, P, L, P, L, L, L, L, L, I, I, F, P, P, L, P, F, P, L, P, P, P, P, L, P, P, P, P, P, L, L, I, P],
-    "ll_linear_scan_chunk_floats": [L, L, L, L, L, L, I, L],
-    "ll_linear_scan_chunks": [P, L, P, L, P, L, L, L, L, L, I, I, F, P, P, L, P, F, P, L, P, P, P, P, L, P, P, P, P, P, L, L, I, P],
+    "ll_linear_scan_walk_floats": [L, L, L, L, L, L, I, L],
+    "ll_linear_scan_walk": [P, L, P, L, P, L, L, L, L, L, I, I, F, P, P, L, P, F, P, L, P, P, P, P, L, P, P, P, P, P, L, L, I, P],
     "ll_retention_supported": [L, L],
     "ll_retention": [P, L, P, L, P, L, L, L, L, P, L, L, F, P, P, P, P, P, P, P, L, F, P, L, L, L, I, P],
     "ll_gated_out_norm": [P, L, P, P, L, I, I, P, L, F, F, L, L, L, I, P],
@@ -152,7 +152,7 @@ SIGNATURES = {
     "ll_stream_norm": [P, L, L, P, P, L, P, P, P, P, P, P, P, F, F, P, L, L, L, I, P],
 }
 
-_RETURNS_I64 = {"ll_linear_scan_chunk_floats", "ll_rglru_scan_scratch_floats", "ll_delta_scan_scratch_floats", "ll_ragged_attention_partition", "ll_mingru_scan_scratch_floats", "ll_moe_rows_block", "ll_kv_alloc_scratch_bytes", "ll_tp_oneshot_flag_words", "ll_moe_router_workspace_floats", "ll_moe_align_workspace_ints"}
+_RETURNS_I64 = {"ll_linear_scan_walk_floats", "ll_rglru_scan_scratch_floats", "ll_delta_scan_scratch_floats", "ll_ragged_attention_partition", "ll_mingru_scan_scratch_floats", "ll_moe_rows_block", "ll_kv_alloc_scratch_bytes", "ll_tp_oneshot_flag_words", "ll_moe_router_workspace_floats", "ll_moe_align_workspace_ints"}
 _lib = None
 
 

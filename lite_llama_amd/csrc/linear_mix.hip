@@ -216,336 +216,237 @@ __global__ __launch_bounds__(256) void linear_scan_kernel(const ScanArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------------------------------------
-// runs of many tokens: chunks of 16 tokens as matrix products on the fp32 matrix cores.  With D_t the product of the decays of a chunk's
-// tokens up to t, R(u, t) that of the tokens behind u up to t, and S the state in front of the chunk,
-//
-//   o_t = (q_t D_t)^T S + sum_(u <= t) [sum_i q_t[i] k_u[i] R(u, t)[i]] v_u,      S <- D_15 S + sum_u (k_u R(u, 15)) v_u^T
-//
-// Every factor is a running product of decays (no quotient), so nothing leaves the range the walk token by token stays in.
-//   chunk_terms_kernel   everything that does not depend on the state, for all chunks at once: activations, decays, decayed queries and
-//                        keys, the 16 x 16 scores -- stored in the order in which the second kernel's lanes take operands
-//   chunk_scan_kernel    a wave per (sequence, head, 16 columns) carries its state columns through the chunks in registers
-// The walk is bound by LDS (a 16-byte record per 16 columns of a key entry and token) and by its three fp32 operations per state entry
-// and token; here a wave runs 2 dk / 4 + 4 matrix instructions per 16 tokens.  us, walk -> chunks (both kernels), 8 runs of 256 - 512 tokens
-// | one of 1024: per entry, 8 heads of 128 x 256: 536 -> 95 (terms 31) | 417 -> 130; fixed, 16 of 128 x 128: 439 -> 105 | 340 -> 137; per
-// token, 32 of 128 x 64: 443 -> 88 | 344 -> 140.  Of the 66 us of the first scan 33 are its matrix instructions; the rest waits for
-// operands, requested half a chunk ahead.  Products of decays, which meet the state once per chunk, are taken in 64 bits and what a chunk
-// adds is summed apart: the error against 64 bits is the walk's or below it (fixed: 7.8e-8 against 9.2e-8 of the result's norm).
+// runs of many tokens: the walk above, with the same bits, in two kernels.  Token by token it is three fp32 operations per state entry; what
+// it spent its time on was everything around them -- per 16 columns of a head the rows were loaded, activated and written to LDS again,
+// eight 16-byte records were read for 24 operations, and every 16 tokens waited for their rows from memory.
+//   scan_terms_kernel    per token, once: (key, query) pairs behind activation and scale, decays per key entry, (decay, step size) pairs
+//   linear_walk_kernel   a workgroup per (sequence, head, 16 CV columns): thread (kg, piece) owns CV neighbouring columns of the state rows kg,
+//                        kg + 16, ...; eight tokens at a time come to LDS by DMA under the walk over the eight in front of them, a token's
+//                        records are read under the products of the one in front of it, and the partial read-outs of eight tokens are
+//                        added at once (row groups in order, as in the walk above): only the walk's own instructions stand between its tokens
+// us, before -> both kernels, 8 runs of 256 - 512 tokens | one of 1024: per entry, 8 heads of 128 x 256: 536 -> 182 | 417 -> 196; fixed, 16 of
+// 128 x 128: 439 -> 153 | 340 -> 166; per token, 32 of 128 x 64: 443 -> 147 | 344 -> 164 (the terms take 10 - 21 of each).  The longest run's
+// own operations need 70 (two columns per thread).  Sums over chunks of 16 tokens as matrix products took 95 | 130, but round in another order.
 // ------------------------------------------------------------------------------------------------------------------------
-constexpr int kCT = 16;      // tokens per chunk
-constexpr int kRec = 320;    // floats per (chunk, head): scores 256, then kinds 0 and 2: D_t, R(u, 15) b_u, b_u (16 each)
+constexpr int kTB = 8;   // tokens per stage of the walk
 
-__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-
-struct ChunkBufs {
-  float* q;      // [chunk][terms head][KT][64 lanes][4]: decayed queries (kinds 0 and 2: queries)
-  float* k;      // likewise keys, token-major inside a lane
-  float* last;   // kind 1: [chunk][head][16 KT] D_15 per key entry
-  float* rec;    // [chunk][head][kRec]
-};
-
-// One workgroup per (chunk of the longest run, sequence, terms head): a head for kind 1, else a query / key head with all its value heads.
-template <int DT, int KT, bool ENTRY>
-__global__ __launch_bounds__(256) void chunk_terms_kernel(const ScanArgs a, const ChunkBufs w) {
-  constexpr int W = 16 * KT, LD = W + 4;
-  extern __shared__ __attribute__((aligned(16))) float lds[];
-  __shared__ float vec[16][kCT], steps[16][kCT];
-  float* sq = lds;
-  float* sk = sq + kCT * LD;
-  float* sa = sk + kCT * LD;   // ENTRY
-  const int b = blockIdx.y, th = blockIdx.z, tid = threadIdx.x;
-  const int t0 = a.seq_start[b], t1 = a.seq_start[b + 1];
-  const int base = t0 + kCT * (int)blockIdx.x;
-  if (base >= t1) return;
-  const int n = t1 - base < kCT ? t1 - base : kCT;
-  const int64_t slot = t0 / kCT + b + blockIdx.x;
-  const int heads = a.heads;
-  constexpr int dk = W;
-  const int qh = ENTRY ? th / a.qk_rep : th;
-  const int tnum = ENTRY ? heads : heads / a.qk_rep;
-#pragma unroll
-  for (int i0 = 0; i0 < kCT * W; i0 += 256) {
-    const int i = i0 + tid, tt = i / W, kk = i - tt * W;
-    float qv = 0.f, kv = 0.f, dec = 1.f;
-    if (tt < n) {
-      const int64_t row = base + tt;
-      qv = ldv<DT>(a.q, row * a.q_ld + (int64_t)qh * dk + kk);
-      kv = ldv<DT>(a.k, row * a.k_ld + (int64_t)qh * dk + kk);
-      if (a.act) {
-        qv *= act_sigmoid<DT>(qv);
-        kv *= act_sigmoid<DT>(kv);
-      }
-      qv *= a.q_scale;
-      if constexpr (ENTRY)
-        dec = entry_decay(ldv<DT>(a.gate, row * a.gate_ld + (int64_t)th * dk + kk) + ldv<DT>(a.gate_bias, th * dk + kk), a.inv_tau);
+template <int DT>
+__global__ __launch_bounds__(256) void scan_terms_kernel(const ScanArgs a, float2* __restrict__ kq, float* __restrict__ decay,
+                                                         float2* __restrict__ td, int64_t n, int64_t total) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= total) return;
+  const int heads = a.heads, qk_heads = heads / a.qk_rep, dk = a.dk;
+  const int cols = (a.kind == 1 ? heads : qk_heads) * dk;
+  const int64_t row = i / cols;
+  const int c = (int)(i - row * cols);
+  if (a.kind == 1)
+    decay[i] = entry_decay(ldv<DT>(a.gate, row * a.gate_ld + c) + ldv<DT>(a.gate_bias, c), a.inv_tau);
+  if (row < n && c < qk_heads * dk) {
+    float qv = ldv<DT>(a.q, row * a.q_ld + c), kv = ldv<DT>(a.k, row * a.k_ld + c);
+    if (a.act) {
+      qv *= act_sigmoid<DT>(qv);
+      kv *= act_sigmoid<DT>(kv);
     }
-    sq[tt * LD + kk] = qv;
-    sk[tt * LD + kk] = kv;
-    if constexpr (ENTRY) sa[tt * LD + kk] = dec;
+    kq[row * qk_heads * dk + c] = float2{kv, qv * a.q_scale};
   }
-  __syncthreads();
-  // scores: thread (key token u, entries 4 g + 64 j ..) against all queries behind it
-  const int u = tid >> 4, g = tid & 15, u0 = __builtin_amdgcn_readfirstlane(tid >> 6) * 4;   // u0: the wave's first key token
-  float acc[kCT];
-#pragma unroll
-  for (int t = 0; t < kCT; ++t) acc[t] = 0.f;
-#pragma unroll
-  for (int j = 0; j < KT / 4; ++j) {
-    const int at = 4 * g + 64 * j;
-    f32x4 m = *reinterpret_cast<const f32x4*>(sk + u * LD + at);
-#pragma unroll
-    for (int t = 0; t < kCT; ++t) {
-      if (t < u0) continue;
-      const f32x4 qv = *reinterpret_cast<const f32x4*>(sq + t * LD + at);
-      if constexpr (ENTRY) {
-        const f32x4 av = *reinterpret_cast<const f32x4*>(sa + t * LD + at);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) m[e] = t > u ? m[e] * av[e] : m[e];
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) acc[t] = __builtin_fmaf(qv[e], m[e], acc[t]);
-    }
-  }
-  __syncthreads();
-  if constexpr (ENTRY) {
-    if (tid < W) {
-      double p = 1.0;
-#pragma unroll
-      for (int t = 0; t < kCT; ++t) {
-        p *= sa[t * LD + tid];
-        sq[t * LD + tid] *= (float)p;
-      }
-      w.last[(slot * tnum + th) * W + tid] = (float)p;
-      p = 1.0;
-#pragma unroll
-      for (int t = kCT - 1; t >= 0; --t) {
-        sk[t * LD + tid] *= (float)p;
-        p *= sa[t * LD + tid];
-      }
-    }
-    __syncthreads();
-  }
-  // operands in lane order: lane (t, c) of piece s takes query t's entries 16 s + 4 c .. and key entry 16 s + t of tokens 4 c ..
-  for (int i = tid; i < KT * 64; i += 256) {
-    const int s = i >> 6, t = i & 15, c = (i >> 4) & 3;
-    const int64_t at = ((slot * tnum + th) * KT * 64 + i) * 4;
-    *reinterpret_cast<f32x4*>(w.q + at) = *reinterpret_cast<const f32x4*>(sq + t * LD + 16 * s + 4 * c);
-    f32x4 kv;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) kv[e] = sk[(4 * c + e) * LD + 16 * s + t];
-    *reinterpret_cast<f32x4*>(w.k + at) = kv;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int t = 0; t < kCT; ++t) lds[tid * 17 + t] = acc[t];
-  __syncthreads();
-  const int t = tid & 15;
-  float part[16];
-#pragma unroll
-  for (int j = 0; j < 16; ++j) part[j] = lds[(u * 16 + j) * 17 + t];
-#pragma unroll
-  for (int j = 8; j > 0; j >>= 1)
-#pragma unroll
-    for (int i = 0; i < j; ++i) part[i] += part[i + j];
-  const float p = part[0];
-  const int rec_at = ((u >> 2) * 16 + t) * 4 + (u & 3);   // lane (t, c) takes query t's scores against tokens 4 c ..
-  if constexpr (ENTRY) {
-    w.rec[(slot * heads + th) * kRec + rec_at] = t >= u ? p : 0.f;
-    return;
-  }
-  for (int r0 = 0; r0 < a.qk_rep; r0 += 16) {   // value heads, 16 at a time
-    __syncthreads();
-    const int hn = a.qk_rep - r0 < 16 ? a.qk_rep - r0 : 16;
-    const int h0 = th * a.qk_rep + r0;
-    if (u < hn) {   // (thread (value head, token))
-      float dec = 1.f, step = 1.f;
-      if (t < n) {
-        if (a.kind == 0) {
-          dec = a.head_decay[h0 + u];
-        } else {
-          step = softplus(ldv<DT>(a.dt, (int64_t)(base + t) * a.dt_ld + h0 + u) + ldv<DT>(a.dt_bias, h0 + u));
-          dec = expf(-expf(ldv<DT>(a.a_log, h0 + u)) * step);
-        }
-      }
-      vec[u][t] = dec;
-      steps[u][t] = step;
-    }
-    __syncthreads();
-    if (u < hn) {
-      double d = 1.0, e = 1.0;
-#pragma unroll
-      for (int x = 0; x < kCT; ++x) {
-        d = x <= t ? d * vec[u][x] : d;
-        e = x > t ? e * vec[u][x] : e;
-      }
-      float* rec = w.rec + (slot * heads + h0 + u) * kRec + 256;
-      rec[t] = (float)d;
-      rec[16 + t] = (float)(e * steps[u][t]);
-      rec[32 + t] = steps[u][t];
-    }
-    for (int h = 0; h < hn; ++h) {   // (thread (key token, query token))
-      double r = 1.0;
-#pragma unroll
-      for (int x = 1; x < kCT; ++x) r = x > u && x <= t ? r * vec[h][x] : r;
-      w.rec[(slot * heads + h0 + h) * kRec + rec_at] = t >= u ? p * (float)r : 0.f;
-    }
+  if (a.kind == 2 && i < n * heads) {
+    const int64_t t = i / heads;
+    const int h = (int)(i - t * heads);
+    const float step = softplus(ldv<DT>(a.dt, t * a.dt_ld + h) + ldv<DT>(a.dt_bias, h));
+    td[i] = float2{expf(-expf(ldv<DT>(a.a_log, h)) * step), step};
   }
 }
 
-// A wave per (sequence, head, 16 state columns), no LDS and no barrier: lane (t, c), element r of piece s holds the state of key entry
-// 16 s + 4 c + r and column t -- the layout in which v_mfma_f32_16x16x4 leaves results AND takes its second operand when a contraction's
-// entries are taken in the order (element, c).  Queries of the next chunk are requested behind the read-out, under the state's
-// products; keys behind those, under the next read-out.  The waves of a head are dealt to one XCD: they read the same operands.
-template <int DT, int KT, bool ENTRY>
-__global__ __launch_bounds__(256) void chunk_scan_kernel(const ScanArgs a, const ChunkBufs w, int pairs, int tiles) {
-  constexpr int W = 16 * KT;
-  const int wid = blockIdx.x;
-  const int groups = (tiles + 3) >> 2, xcd = wid & 7, rest = wid >> 3;
-  const int pair = rest / groups * 8 + xcd, tile = rest % groups * 4 + (threadIdx.x >> 6);
-  if (pair >= pairs || tile >= tiles) return;
-  const int b = pair / a.heads, head = pair - b * a.heads, lane = threadIdx.x & 63, t = lane & 15, c = lane >> 4;
-  const int dv = a.dv, heads = a.heads, col = tile * 16 + t;
+// 64 lanes x 16 bytes from per-lane addresses to 1 KB of LDS at byte `dst` (counted by vmcnt, which the compiler does not see)
+__device__ __forceinline__ void dma16(uint32_t dst, const void* src) {
+  dst = __builtin_amdgcn_readfirstlane(dst);
+  uint32_t keep;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep) : "s"(dst), "v"(src) : "memory");
+}
+
+// dk == 16 RMAX.  dt: the values' storage dtype (a few conversions per eight tokens: no form of its own)
+template <int RMAX, int CV, int KIND>
+__global__ __launch_bounds__(256) void linear_walk_kernel(const ScanArgs a, const float2* __restrict__ kq, const float2* __restrict__ td, int dt) {
+  constexpr int dk = 16 * RMAX, CW = 16 * CV, NV = (kTB * CW + 255) / 256, NB = kTB * dk * 2;
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  float* skq = lds;                                    // [2][kTB][dk] (key, query)
+  float* sdec = skq + 2 * NB;                          // KIND 1: [2][kTB][dk] decays; 2: [2][kTB]
+  float* sv = sdec + 2 * kTB * (KIND == 1 ? dk : 1);   // [2][kTB][CW] what enters the state
+  float* sp = sv + 2 * kTB * CW;                       // [kTB][16 groups][CW] partial read-outs
+  const int b = blockIdx.y, head = blockIdx.x, c0 = blockIdx.z * CW;   // (heads over the XCDs: sequences differ in length)
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), col = (tid & 15) * CV, kg = tid >> 4;
+  const int dv = a.dv, heads = a.heads, qh = head / a.qk_rep, qk_heads = heads / a.qk_rep;
+  const bool active = c0 + col < dv;
   const int t0 = a.seq_start[b], t1 = a.seq_start[b + 1];
   if (t0 >= t1) return;
-  const int tnum = ENTRY ? heads : heads / a.qk_rep, th = ENTRY ? head : head / a.qk_rep;
-  const bool carry = a.seq_first_pos[b] > 0, live = col < dv;
-  float* st = a.state + ((int64_t)a.seq_slot[b] * heads + head) * W * dv + col;
-  f32x4 S[KT];
+  float* st = a.state + ((int64_t)a.seq_slot[b] * heads + head) * dk * dv + c0 + col;
+  const bool carry = a.seq_first_pos[b] > 0;
+  float S[RMAX][CV];
 #pragma unroll
-  for (int s = 0; s < KT; ++s)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int kk = 16 * s + 4 * c + r;
-      S[s][r] = (carry && live) ? st[(int64_t)kk * dv] : 0.f;
+  for (int r = 0; r < RMAX; ++r) {
+    const bool in = active && carry;
+    const float* at = st + (int64_t)(kg + 16 * r) * dv;
+    if constexpr (CV == 2) {
+      const float2 old = in ? *reinterpret_cast<const float2*>(at) : float2{0.f, 0.f};
+      S[r][0] = old.x;
+      S[r][1] = old.y;
+    } else {
+      S[r][0] = in ? at[0] : 0.f;
     }
-  const bool skips = !ENTRY && a.kind == 2 && a.skip;
-  const float skip = skips ? ldv<DT>(a.skip, head) : 0.f;
-  const int chunks = (t1 - t0 + kCT - 1) / kCT;
-  const int64_t slot = t0 / kCT + b;
-  const float* qp = w.q + ((slot * tnum + th) * KT * 64 + lane) * 4;
-  const float* kp = w.k + ((slot * tnum + th) * KT * 64 + lane) * 4;
-  const float* lp = ENTRY ? w.last + (slot * tnum + th) * W + 4 * c : nullptr;
-  const float* rp = w.rec + (slot * heads + head) * kRec;
-  const int64_t qk_step = (int64_t)tnum * KT * 256, last_step = (int64_t)tnum * W, rec_step = (int64_t)heads * kRec;
-  f32x4 qf[KT], kf[KT], lf[ENTRY ? KT : 1], pf, df, wf, sf;
-  uint32_t raw[4];   // the values' bits: converted where they are used, so that nothing waits for them here
-  auto get_q = [&]() {
+  }
+  const float fixed = KIND == 0 ? a.head_decay[head] : 0.f;
+  const bool skips = KIND == 2 && a.skip;
+  const float skip = !skips ? 0.f : dt == LL_F32 ? ldv<LL_F32>(a.skip, head) : dt == LL_F16 ? ldv<LL_F16>(a.skip, head) : ldv<LL_BF16>(a.skip, head);
+  // eight tokens' pairs (and decays) to LDS: 16-byte pieces in token order; a token behind the run repeats its last row
+  auto request = [&](int base, int buf) {
 #pragma unroll
-    for (int s = 0; s < KT; ++s) qf[s] = *reinterpret_cast<const f32x4*>(qp + 256 * s);
-    pf = *reinterpret_cast<const f32x4*>(rp + 4 * lane);
-    if constexpr (!ENTRY) {
-      df = *reinterpret_cast<const f32x4*>(rp + 256 + 4 * c);
-      wf = *reinterpret_cast<const f32x4*>(rp + 272 + 4 * c);
-      sf = *reinterpret_cast<const f32x4*>(rp + 288 + 4 * c);
+    for (int j = 0; j < RMAX; j += 4) {
+      const int p = (wave + j) * 64 + lane, tt = p / (dk / 2), at = p - tt * (dk / 2);
+      const int row = base + tt < t1 ? base + tt : t1 - 1;
+      dma16((uint32_t)((buf * NB) * 4 + (wave + j) * 1024), kq + ((int64_t)row * qk_heads + qh) * dk + 2 * at);
     }
-  };
-  auto get_k = [&]() {
+    if constexpr (KIND == 1) {
 #pragma unroll
-    for (int s = 0; s < KT; ++s) kf[s] = *reinterpret_cast<const f32x4*>(kp + 256 * s);
-    if constexpr (ENTRY) {
-#pragma unroll
-      for (int s = 0; s < KT; ++s) lf[s] = *reinterpret_cast<const f32x4*>(lp + 16 * s);
-    }
-  };
-  auto get_v = [&](int base) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int tok = base + 4 * c + r < t1 ? base + 4 * c + r : t1 - 1;
-      const int64_t at = (int64_t)tok * a.v_ld + (int64_t)head * dv + (live ? col : 0);
-      if constexpr (DT == LL_F32) raw[r] = ((const uint32_t*)a.v)[at];
-      else raw[r] = ((const uint16_t*)a.v)[at];
-    }
-  };
-  get_q();
-  get_v(t0);
-  __builtin_amdgcn_sched_barrier(0);   // (the loop's order of requests, so that its waits count the same in its first pass)
-  get_k();
-  __builtin_amdgcn_sched_barrier(0);
-  for (int j = 0; j < chunks; ++j) {
-    const int base = t0 + kCT * j;
-    const bool more = j + 1 < chunks;   // (the last chunk requests its own operands again: no branch around the loads)
-    f32x4 v, x;
-    bool odd = false;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const bool in = live && base + 4 * c + r < t1;
-      if constexpr (DT == LL_F32) x[r] = in ? __uint_as_float(raw[r]) : 0.f;
-      else x[r] = in ? to_f32<DT>((uint16_t)raw[r]) : 0.f;
-      if (a.act) x[r] *= act_sigmoid<DT>(x[r]);
-      v[r] = !ENTRY && a.kind == 2 ? sf[r] * x[r] : x[r];
-      odd |= !(fabsf(v[r]) < INFINITY);
-    }
-    f32x4 part[8];   // eight short sums, then pairs of them
-#pragma unroll
-    for (int i = 0; i < 8; ++i) part[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < KT; ++s)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) part[(4 * s + e) & 7] = mfma4(qf[s][e], S[s][e], part[(4 * s + e) & 7]);
-#pragma unroll
-    for (int i = 4; i > 0; i >>= 1)
-#pragma unroll
-      for (int y = 0; y < i; ++y) part[y] += part[y + i];
-    f32x4 o = part[0];
-    const float dlast = ENTRY ? 0.f : __shfl(df[3], 48);   // D_15: all decays of the chunk
-    f32x4 vw = x;
-    f32x4 near = {0.f, 0.f, 0.f, 0.f};
-    if (__ballot(odd) == 0) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) near = mfma4(pf[e], v[e], near);
-    } else {   // a value that is not finite must not meet the zero scores of the tokens in front of it
-#pragma unroll 1
-      for (int uu = 0; uu < kCT; ++uu) {
-        const float val = __shfl(v[0], (uu >> 2) * 16 + t), val1 = __shfl(v[1], (uu >> 2) * 16 + t);
-        const float val2 = __shfl(v[2], (uu >> 2) * 16 + t), val3 = __shfl(v[3], (uu >> 2) * 16 + t);
-        const float vu = (uu & 3) == 0 ? val : (uu & 3) == 1 ? val1 : (uu & 3) == 2 ? val2 : val3;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int tok = 4 * c + r;
-          if (uu <= tok) near[r] = __builtin_fmaf(rp[((uu >> 2) * 16 + tok) * 4 + (uu & 3)], vu, near[r]);
-        }
+      for (int j = 0; j < RMAX / 2; j += 4) {
+        if (wave + j >= RMAX / 2) break;
+        const int p = (wave + j) * 64 + lane, tt = p / (dk / 4), at = p - tt * (dk / 4);
+        const int row = base + tt < t1 ? base + tt : t1 - 1;
+        dma16((uint32_t)((2 * NB + buf * kTB * dk) * 4 + (wave + j) * 1024), a.decay_pre + ((int64_t)row * heads + head) * dk + 4 * at);
       }
     }
+  };
+  // values of a stage: entries tid + 256 j of [kTB][CW], bits first
+  uint32_t raw[NV];
+  float2 rt[NV];
+  float sx[NV];
+  auto fetch = [&](int base) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      o[r] = ENTRY ? o[r] + near[r] : __builtin_fmaf(o[r], df[r], near[r]);
-      if constexpr (!ENTRY) vw[r] *= wf[r];
+    for (int j = 0; j < NV; ++j) {
+      const int i = tid + 256 * j, tt = i / CW, cc = i % CW;
+      const int row = base + tt < t1 ? base + tt : t1 - 1;
+      const int64_t at = (int64_t)row * a.v_ld + (int64_t)head * dv + (c0 + cc < dv ? c0 + cc : 0);
+      raw[j] = dt == LL_F32 ? ((const uint32_t*)a.v)[at] : ((const uint16_t*)a.v)[at];
+      if constexpr (KIND == 2) rt[j] = td[(int64_t)row * heads + head];
     }
+  };
+  auto stage = [&](int buf) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int tok = base + 4 * c + r;
-      if (live && tok < t1) a.o[((int64_t)tok * heads + head) * dv + col] = skips ? o[r] + skip * x[r] : o[r];
+    for (int j = 0; j < NV; ++j) {
+      const int i = tid + 256 * j, tt = i / CW, cc = i % CW;
+      float x = dt == LL_F32 ? __uint_as_float(raw[j]) : dt == LL_F16 ? to_f32<LL_F16>((uint16_t)raw[j]) : to_f32<LL_BF16>((uint16_t)raw[j]);
+      if (c0 + cc >= dv) x = 0.f;
+      if (a.act) x *= dt == LL_F32 ? act_sigmoid<LL_F32>(x) : act_sigmoid<LL_BF16>(x);
+      sx[j] = skips ? skip * x : 0.f;
+      if (i >= kTB * CW) continue;
+      sv[buf * kTB * CW + i] = KIND == 2 ? rt[j].y * x : x;
+      if (KIND == 2 && cc == 0) sdec[buf * kTB + tt] = rt[j].x;
     }
-    qp += more ? qk_step : 0;
-    rp += more ? rec_step : 0;
-    get_q();
-    get_v(more ? base + kCT : base);
-    __builtin_amdgcn_sched_barrier(0);   // (the requests stay in front of the products that hide them)
-    f32x4 add[KT];   // what the chunk adds, summed by itself: the state is rounded once per chunk
-#pragma unroll
-    for (int s = 0; s < KT; ++s) add[s] = mfma4(kf[s][0], vw[0], f32x4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-    for (int e = 1; e < 4; ++e)
-#pragma unroll
-      for (int s = 0; s < KT; ++s) add[s] = mfma4(kf[s][e], vw[e], add[s]);
-#pragma unroll
-    for (int s = 0; s < KT; ++s) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) S[s][r] = __builtin_fmaf(ENTRY ? lf[s][r] : dlast, S[s][r], add[s][r]);
+  };
+  struct Token {   // what a thread reads of a token
+    float2 g[RMAX];
+    float dec[KIND == 1 ? RMAX : 1], v[CV];
+  };
+  auto read = [&](int buf, int tt, Token& k) {
+    const float* val = sv + (buf * kTB + tt) * CW + col;
+    const float* kp = skq + buf * NB + (tt * dk + kg) * 2;
+    const float* dp = sdec + (KIND == 1 ? (buf * kTB + tt) * dk + kg : buf * kTB + tt);
+    if constexpr (CV == 2) {
+      const float2 w = *reinterpret_cast<const float2*>(val);
+      k.v[0] = w.x;
+      k.v[1] = w.y;
+    } else {
+      k.v[0] = val[0];
     }
-    kp += more ? qk_step : 0;
-    if constexpr (ENTRY) lp += more ? last_step : 0;
-    __builtin_amdgcn_sched_barrier(0);
-    get_k();
-    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (KIND == 0) k.dec[0] = fixed;
+    if constexpr (KIND == 2) k.dec[0] = dp[0];
+#pragma unroll
+    for (int r = 0; r < RMAX; ++r) {
+      k.g[r] = *reinterpret_cast<const float2*>(kp + 32 * r);
+      if constexpr (KIND == 1) k.dec[r] = dp[16 * r];
+    }
+  };
+  auto walk = [&](const Token& k, float (&acc)[CV]) {
+#pragma unroll
+    for (int e = 0; e < CV; ++e) acc[e] = 0.f;
+#pragma unroll
+    for (int r = 0; r < RMAX; ++r)
+#pragma unroll
+      for (int e = 0; e < CV; ++e) {
+        S[r][e] = __builtin_fmaf(k.dec[KIND == 1 ? r : 0], S[r][e], k.g[r].x * k.v[e]);
+        acc[e] = __builtin_fmaf(S[r][e], k.g[r].y, acc[e]);
+      }
+  };
+  auto leave = [&](int tt, const float (&acc)[CV]) {
+    float* at = sp + (tt * 16 + kg) * CW + col;
+    if constexpr (CV == 2) *reinterpret_cast<float2*>(at) = float2{acc[0], acc[1]};
+    else at[0] = acc[0];
+  };
+  auto add_up = [&](int base, const float (&x)[NV]) {
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      const int i = tid + 256 * j, tt = i / CW, cc = i % CW;
+      if (i >= kTB * CW || base + tt >= t1) continue;
+      float o = 0.f;
+#pragma unroll
+      for (int g2 = 0; g2 < 16; ++g2) o += sp[(tt * 16 + g2) * CW + cc];
+      if (c0 + cc < dv) a.o[((int64_t)(base + tt) * heads + head) * dv + c0 + cc] = o + x[j];
+    }
+  };
+  fetch(t0);
+  request(t0, 0);
+  stage(0);
+  int buf = 0;
+  for (int base = t0; base < t1; base += kTB) {
+    const int nt = t1 - base < kTB ? t1 - base : kTB;
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0070);   // this stage's pairs and values are there; the partial sums have been read
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    float x_now[NV];
+#pragma unroll
+    for (int j = 0; j < NV; ++j) x_now[j] = sx[j];
+    const bool more = base + kTB < t1;
+    if (more) {
+      request(base + kTB, buf ^ 1);
+      fetch(base + kTB);
+    }
+    if (nt == kTB) {
+      float acc[kTB][CV];   // (written behind the last token: a write to LDS between them would hold the reads of the next)
+      Token k[2];
+      read(buf, 0, k[0]);
+#pragma unroll
+      for (int tt = 0; tt < kTB; ++tt) {
+        if (tt + 1 < kTB) read(buf, tt + 1, k[(tt + 1) & 1]);
+        __builtin_amdgcn_sched_barrier(0);   // (the next token's reads stay in front of this one's products)
+        walk(k[tt & 1], acc[tt]);
+      }
+#pragma unroll
+      for (int tt = 0; tt < kTB; ++tt) leave(tt, acc[tt]);
+    } else {
+      for (int tt = 0; tt < nt; ++tt) {
+        float acc[CV];
+        Token k;
+        read(buf, tt, k);
+        walk(k, acc);
+        leave(tt, acc);
+      }
+    }
+    if (more) stage(buf ^ 1);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xc07f);   // (LDS only: the next stage may still be on its way)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    add_up(base, x_now);
+    buf ^= 1;
   }
 #pragma unroll
-  for (int s = 0; s < KT; ++s)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int kk = 16 * s + 4 * c + r;
-      if (live) st[(int64_t)kk * dv] = S[s][r];
-    }
+  for (int r = 0; r < RMAX; ++r) {
+    if (!active) continue;
+    float* at = st + (int64_t)(kg + 16 * r) * dv;
+    if constexpr (CV == 2) *reinterpret_cast<float2*>(at) = float2{S[r][0], S[r][1]};
+    else at[0] = S[r][0];
+  }
 }
 
 // One wave per (token, part): out = [o * act(gate)] / sqrt(mean_part(.^2) + eps) * w [* act(gate)] * out_scale.
@@ -946,8 +847,7 @@ __global__ __launch_bounds__(256) void rownorm_rope_cache_vec_kernel(
 
 }  // namespace
 
-constexpr int64_t kChunkRun = 64, kChunkRunFull = 24;   // least longest run of a step for the chunk form (see its scratch)
-constexpr int64_t kChunkFloats = 1ll << 28;     // largest scratch of the chunk form (1 GiB)
+constexpr int64_t kWalkFloats = 1ll << 28;   // largest scratch of the two-kernel walk (1 GiB)
 
 #define LL_BY_DTYPE(dtype, CALL)                  \
   do {                                            \
@@ -958,19 +858,16 @@ constexpr int64_t kChunkFloats = 1ll << 28;     // largest scratch of the chunk 
 
 extern "C" int ll_linear_scan_supported(int64_t dk, int64_t dv) { return dk >= 1 && dk <= 256 && dv >= 1 ? 1 : 0; }
 
-// Floats of scratch for the chunk form, 0 where the walk serves: heads of whole 64-entry groups (16 KT entries, no padding), and a longest run
-// of 64 tokens, or of 24 where the walk's workgroups are enough to fill the chip.  The chunk form costs two launches and about 12 us
-// ahead of its first token, the walk 0.2 - 0.3 us a token when alone; us, walk / chunks: one run of 64 31 / 22 (per entry), 25 / 19
-// (fixed), 25 / 23 (per token), of 32 19 / 19, 14 / 15, 15 / 20; eight of 24 30 / 21, 25 / 18, 26 / 22, four of 24 18 / 20, 14 / 16, 15 / 21.
-extern "C" int64_t ll_linear_scan_chunk_floats(int64_t n, int64_t batch, int64_t heads, int64_t dk, int64_t dv, int64_t qk_rep, int kind,
-                                               int64_t longest_run) {
-  if (n < 1 || batch < 1 || batch > 65535 || heads < 1 || heads > 65535 || dk < 64 || dk > 256 || dk % 64 || dv < 1 || qk_rep < 1 ||
-      heads % qk_rep || longest_run < kChunkRunFull ||
-      (longest_run < kChunkRun && batch * heads * ((dv + 15) / 16) < 1024))
+// Floats of scratch for the two-kernel walk, 0 where the one above serves: heads of 64, 128 or 256 entries (whole 16-byte pieces and DMA
+// rounds) and a longest run of 24 tokens.  One run, us, one kernel / two: of 24 16 / 10 (per entry), 12 / 9 (fixed and per token), 8.1 / 7.6 (fixed,
+// 24 heads of 64 x 128); of 16 12 / 8, 9.0 / 7.4, 9.2 / 8.3, but 6.5 / 6.8, and 6.8 / 7.5 for 48 heads of 64 x 64.
+extern "C" int64_t ll_linear_scan_walk_floats(int64_t n, int64_t batch, int64_t heads, int64_t dk, int64_t dv, int64_t qk_rep, int kind,
+                                              int64_t longest_run) {
+  if (n < 1 || batch < 1 || batch > 65535 || heads < 1 || heads > 65535 || (dk != 64 && dk != 128 && dk != 256) || dv < 1 || qk_rep < 1 || heads % qk_rep ||
+      longest_run < 24)
     return 0;
-  const int64_t slots = n / kCT + batch, terms = kind == 1 ? heads : heads / qk_rep;
-  const int64_t per = terms * (2 * kCT * dk + (kind == 1 ? dk : 0)) + heads * kRec;
-  return per > kChunkFloats / slots ? 0 : slots * per;
+  const int64_t per = heads / qk_rep * dk * 2 + (kind == 1 ? heads * dk : 0) + (kind == 2 ? heads * 2 : 0);
+  return per > kWalkFloats / n ? 0 : n * per;
 }
 
 static int linear_scan(const void* q, int64_t q_ld, const void* k, int64_t k_ld, const void* v, int64_t v_ld, int64_t heads,
@@ -978,7 +875,7 @@ static int linear_scan(const void* q, int64_t q_ld, const void* k, int64_t k_ld,
                               const void* gate, int64_t gate_ld, const void* gate_bias, float inv_tau, const void* dt, int64_t dt_ld,
                               const void* dt_bias, const void* a_log, const void* skip, float* o, int64_t batch,
                               const int32_t* seq_start, const int32_t* seq_first_pos, const int32_t* seq_slot, float* state,
-                              float* decay_scratch, float* chunk_scratch, int64_t n, int64_t longest_run, int dtype, void* stream) {
+                              float* decay_scratch, float* walk_scratch, int64_t n, int64_t longest_run, int dtype, void* stream) {
   if (dtype != LL_F16 && dtype != LL_BF16 && dtype != LL_F32) return LL_ERR_DTYPE;
   if (batch < 0 || heads < 1 || heads > 65535 || !ll_linear_scan_supported(dk, dv) || qk_rep < 1 || heads % qk_rep || kind < 0 ||
       kind > 2 || (dv + 15) / 16 > 65535)
@@ -996,39 +893,53 @@ static int linear_scan(const void* q, int64_t q_ld, const void* k, int64_t k_ld,
   a.head_decay = head_decay; a.gate = gate; a.gate_ld = gate_ld; a.gate_bias = gate_bias; a.inv_tau = inv_tau;
   a.decay_pre = nullptr;
   a.dt = dt; a.dt_ld = dt_ld; a.dt_bias = dt_bias; a.a_log = a_log; a.skip = skip; a.o = o;
-  if (chunk_scratch) {
-    const int64_t floats = ll_linear_scan_chunk_floats(n, batch, heads, dk, dv, qk_rep, kind, longest_run);
-    if (floats <= 0 || !ll_aligned16(chunk_scratch)) return LL_ERR_SHAPE;
-    const int64_t slots = n / kCT + batch, terms = kind == 1 ? heads : heads / qk_rep;
-    ChunkBufs w;
-    w.q = chunk_scratch;
-    w.k = w.q + slots * terms * kCT * dk;
-    w.rec = w.k + slots * terms * kCT * dk;
-    w.last = w.rec + slots * heads * kRec;
-    const int tiles = (int)((dv + 15) / 16), groups = (tiles + 3) / 4;
-    const int64_t pairs = batch * heads, waves = (pairs + 7) / 8 * 8 * groups;
-    if (waves > 0x7fffffffll) return LL_ERR_SHAPE;
-    const dim3 tgrid((unsigned)((longest_run + kCT - 1) / kCT), (unsigned)batch, (unsigned)terms);
-    hipStream_t cst = (hipStream_t)stream;
-    const size_t full = (size_t)3 * kCT * (dk + 4) * sizeof(float), sums = (size_t)256 * 17 * sizeof(float);
-    const size_t clds = full > sums ? full : sums;
-#define CALL_C(DT, KT, EN)                                                                                    \
-  do {                                                                                                        \
-    chunk_terms_kernel<DT, KT, EN><<<tgrid, 256, clds, cst>>>(a, w);                                          \
-    chunk_scan_kernel<DT, KT, EN><<<dim3((unsigned)waves), 256, 0, cst>>>(a, w, (int)pairs, tiles);           \
-  } while (0)
-#define CALL_K(DT, KT) \
-  if (kind == 1) CALL_C(DT, KT, true); \
-  else CALL_C(DT, KT, false)
-#define CALL(DT)                      \
-  if (dk == 64) { CALL_K(DT, 4); }     \
-  else if (dk == 128) { CALL_K(DT, 8); } \
-  else if (dk == 192) { CALL_K(DT, 12); } \
-  else { CALL_K(DT, 16); }
+  if (walk_scratch) {
+    const int64_t floats = ll_linear_scan_walk_floats(n, batch, heads, dk, dv, qk_rep, kind, longest_run);
+    if (floats <= 0 || !ll_aligned16(walk_scratch)) return LL_ERR_SHAPE;
+    const int64_t pairs = n * (heads / qk_rep) * dk;
+    float2* kq = reinterpret_cast<float2*>(walk_scratch);
+    float* decay = walk_scratch + 2 * pairs;
+    float2* td = reinterpret_cast<float2*>(decay);
+    int64_t total = kind == 1 ? n * heads * dk : pairs;
+    if (kind == 2 && total < n * heads) total = n * heads;
+    if ((total + 255) / 256 > 0x7fffffffll || n >= (1ll << 31)) return LL_ERR_SHAPE;
+    hipStream_t wst = (hipStream_t)stream;
+#define CALL(DT) scan_terms_kernel<DT><<<dim3((unsigned)((total + 255) / 256)), 256, 0, wst>>>(a, kq, decay, td, n, total)
     LL_BY_DTYPE(dtype, CALL);
 #undef CALL
+    a.decay_pre = decay;
+    // two columns per thread once there is more than a workgroup of one column per CU (sequences counted by the longest run's length: decoded
+    // tokens beside a portion weigh nothing): a record read serves twice the products.  us, one / two: runs of 64, per entry, 8 heads of
+    // 128 x 256: one sequence 17 / 20, two (256 workgroups) 19 / 21, four 25 / 23, eight 44 / 32; 12 heads: two (384) 24 / 22
+    const int cv = dv % 2 == 0 && (reinterpret_cast<uintptr_t>(state) & 7u) == 0 &&
+                           (n + longest_run - 1) / longest_run * heads * ((dv + 15) / 16) > 320 ? 2 : 1;
+    const int cw = 16 * cv;
+    const size_t wlds = sizeof(float) * (size_t)(2 * kTB * (2 * dk + (kind == 1 ? dk : 1) + 9 * cw));
+    const dim3 wgrid((unsigned)heads, (unsigned)batch, (unsigned)((dv + cw - 1) / cw));
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+#define CALL_W(R, C, KD)                                                                                                               \
+  do {                                                                                                                                 \
+    static bool attr[16] = {false};                                                                                                    \
+    if (dev >= 0 && dev < 16 && !attr[dev]) {                                                                                          \
+      (void)hipFuncSetAttribute((const void*)linear_walk_kernel<R, C, KD>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);    \
+      attr[dev] = true;                                                                                                                \
+    }                                                                                                                                  \
+    linear_walk_kernel<R, C, KD><<<wgrid, 256, wlds, wst>>>(a, kq, td, dtype);                                                         \
+  } while (0)
+#define CALL_C(R, KD)                 \
+  if (cv == 2) CALL_W(R, 2, KD); \
+  else CALL_W(R, 1, KD)
+#define CALL_K(R)                     \
+  if (kind == 0) { CALL_C(R, 0); }    \
+  else if (kind == 1) { CALL_C(R, 1); } \
+  else { CALL_C(R, 2); }
+    if (dk == 64) { CALL_K(4) }
+    else if (dk == 128) { CALL_K(8) }
+    else { CALL_K(16) }
 #undef CALL_K
 #undef CALL_C
+#undef CALL_W
     return LL_LAUNCH_CHECK();
   }
   a.tb = dk <= 128 ? 16 : 8;   // tokens staged per pass; a step of short runs asks for less LDS and fits more workgroups per CU
@@ -1080,15 +991,15 @@ extern "C" int ll_linear_scan(const void* q, int64_t q_ld, const void* k, int64_
                      longest_run, dtype, stream);
 }
 
-extern "C" int ll_linear_scan_chunks(const void* q, int64_t q_ld, const void* k, int64_t k_ld, const void* v, int64_t v_ld, int64_t heads,
+extern "C" int ll_linear_scan_walk(const void* q, int64_t q_ld, const void* k, int64_t k_ld, const void* v, int64_t v_ld, int64_t heads,
                                      int64_t dk, int64_t dv, int64_t qk_rep, int kind, int act, float q_scale, const float* head_decay,
                                      const void* gate, int64_t gate_ld, const void* gate_bias, float inv_tau, const void* dt, int64_t dt_ld,
                                      const void* dt_bias, const void* a_log, const void* skip, float* o, int64_t batch,
                                      const int32_t* seq_start, const int32_t* seq_first_pos, const int32_t* seq_slot, float* state,
-                                     float* chunk_scratch, int64_t n, int64_t longest_run, int dtype, void* stream) {
-  if (!chunk_scratch) return LL_ERR_ARG;
+                                     float* walk_scratch, int64_t n, int64_t longest_run, int dtype, void* stream) {
+  if (!walk_scratch) return LL_ERR_ARG;
   return linear_scan(q, q_ld, k, k_ld, v, v_ld, heads, dk, dv, qk_rep, kind, act, q_scale, head_decay, gate, gate_ld, gate_bias, inv_tau, dt, dt_ld,
-                     dt_bias, a_log, skip, o, batch, seq_start, seq_first_pos, seq_slot, state, nullptr, chunk_scratch, n,
+                     dt_bias, a_log, skip, o, batch, seq_start, seq_first_pos, seq_slot, state, nullptr, walk_scratch, n,
                      longest_run, dtype, stream);
 }
 

@@ -186,10 +186,8 @@ def linear_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, heads: int, d
         ``a = exp(-exp(a_log) dt')``, ``b = dt'``.
 
     ``state [slots, heads, dk, dv]`` fp32: a sequence whose run starts at position 0 starts from zeros, every run leaves its
-    final state.  Decays, step sizes, state and read-out are fp32.  Returns ``o`` fp32 ``[n, heads dv]``.
-
-    Short runs are walked token by token, in the same bits however a prompt is cut; long runs of heads with ``dk`` a multiple of 64 are
-    matrix products over chunks of 16 tokens, whose sums round in another order."""
+    final state.  Decays, step sizes, state and read-out are fp32.  Returns ``o`` fp32 ``[n, heads dv]``.  The
+    results are the same bits however a prompt is cut."""
     L.require_cuda(q, k, v, state, head_decay, gate, gate_bias, dt, dt_bias, a_log, skip)
     n, st = q.shape[0], q.dtype
     qk_heads = heads if qk_heads is None else qk_heads
@@ -229,11 +227,11 @@ def linear_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, heads: int, d
         if dt.dtype != st or dt.shape[0] != n:
             raise ValueError("linear_scan: step sizes in the rows' dtype, one row per token")
     o = torch.empty(n, heads * dv, dtype=torch.float32, device=q.device)
-    # long runs: chunks as matrix products.  Other runs of several tokens: the decays per key entry are evaluated once per token ahead of
+    # long runs: the tokens' terms ahead of the walk.  Other runs of several tokens: the decays per key entry are evaluated once per token ahead of
     # the scan (its column workgroups would each evaluate them again); decode steps evaluate them in the scan
-    floats = int(L.lib().ll_linear_scan_chunk_floats(n, step.num_seqs, heads, dk, dv, heads // qk_heads, kind, int(step.longest_run)))
+    floats = int(L.lib().ll_linear_scan_walk_floats(n, step.num_seqs, heads, dk, dv, heads // qk_heads, kind, int(step.longest_run)))
     if floats:
-        scratch, fn = torch.empty(floats, dtype=torch.float32, device=q.device), L.lib().ll_linear_scan_chunks
+        scratch, fn = torch.empty(floats, dtype=torch.float32, device=q.device), L.lib().ll_linear_scan_walk
     else:
         ahead = kind == 1 and step.longest_run != 1 and dv > 16
         scratch, fn = torch.empty(n, heads * dk, dtype=torch.float32, device=q.device) if ahead else None, L.lib().ll_linear_scan

@@ -1,5 +1,5 @@
-"""Linear attention with a decay over runs of many tokens (csrc/linear_mix.hip: chunks of 16 as matrix products) and decoded tokens in
-64-column workgroups, against 64 bits and against the walk token by token, which serves a step whose longest run is not known."""
+"""Linear attention with a decay over runs of many tokens (csrc/linear_mix.hip: the tokens' terms ahead of the walk) and decoded tokens in
+64-column workgroups, against 64 bits and bit for bit against the walk in one kernel, which serves a step whose longest run is not known."""
 
 import dataclasses
 
@@ -58,45 +58,27 @@ def _exact(q, k, v, heads, dk, dv, runs, state, kw):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("kind,heads,qk_heads,dk,dv", [("fixed", 3, 3, 64, 17), ("fixed", 2, 1, 128, 64), ("entry", 2, 2, 128, 40),
-                                                     ("entry", 4, 2, 192, 9), ("token", 34, 2, 64, 4), ("token", 3, 1, 256, 80)])
-@pytest.mark.parametrize("runs", [[(0, 64)], [(5, 1), (9, 79), (0, 16), (3, 17), (0, 1)], [(2, 95), (0, 33)]])
+                                                     ("entry", 4, 2, 256, 9), ("token", 34, 2, 64, 4), ("token", 3, 1, 256, 80), ("entry", 20, 20, 64, 272)])
+@pytest.mark.parametrize("runs", [[(0, 24)], [(5, 1), (9, 79), (0, 16), (3, 17), (0, 1)], [(2, 95), (0, 33)]])
 def test_runs_of_many_tokens(dtype, kind, heads, qk_heads, dk, dv, runs):
-    """Runs that end on and off a chunk of 16, beside single tokens; carried and fresh states; values off every tile of 16 columns."""
+    """Runs that end on and off eight tokens, beside single tokens; carried and fresh states; values off every tile of columns; one column
+    per thread and two."""
     from lite_llama_amd import _lib
     from lite_llama_amd.kernels.recurrent import linear_scan
 
     n = sum(c for _, c in runs)
     q, k, v, kw = _inputs(kind, heads, qk_heads, dk, dv, n, dtype, dk + dv)
     step = _step([(i, f, c, 0) for i, (f, c) in enumerate(runs)], None)
-    assert _lib.lib().ll_linear_scan_chunk_floats(n, len(runs), heads, dk, dv, heads // qk_heads, ["fixed", "entry", "token"].index(kind),
+    assert _lib.lib().ll_linear_scan_walk_floats(n, len(runs), heads, dk, dv, heads // qk_heads, ["fixed", "entry", "token"].index(kind),
                                                   step.longest_run) > 0
     start = torch.randn(len(runs), heads, dk, dv, device=DEV)
     want, want_state = _exact(q, k, v, heads, dk, dv, runs, start, kw)
-    for longest in (step.longest_run, 0):
-        state = start.clone()
-        got = linear_scan(q, k, v, heads, dk, dv, dataclasses.replace(step, longest_run=longest), state, **kw)
-        # fp32 throughout: a few units of rounding per token of a run and per entry of a sum, against the largest result
-        for x, y in ((got, want), (state, want_state)):
-            assert (x.to(F64) - y).abs().max() <= 64 * 2.0 ** -24 * y.abs().max()
-
-
-@pytest.mark.parametrize("kind", ["fixed", "entry", "token"])
-@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
-@pytest.mark.parametrize("where", [0, 37, 63])
-def test_a_value_that_is_not_finite_leaves_the_tokens_in_front_of_it_alone(kind, bad, where):
-    from lite_llama_amd.kernels.recurrent import linear_scan
-
-    heads, dk, dv, n = 2, 64, 24, 70
-    q, k, v, kw = _inputs(kind, heads, heads, dk, dv, n, torch.bfloat16, 3)
-    step = _step([(0, 0, n, 0)], None)
-    clean = linear_scan(q, k, v, heads, dk, dv, step, torch.zeros(1, heads, dk, dv, device=DEV), **kw)
-    v[where, 5] = bad
-    got = linear_scan(q, k, v, heads, dk, dv, step, torch.zeros(1, heads, dk, dv, device=DEV), **kw)
-    fine = torch.ones(n, heads * dv, dtype=torch.bool, device=DEV)
-    fine[where:, 5] = False
-    # (the chunk of the value adds its scores in another order)
-    assert (got - clean)[fine].abs().max() <= 64 * 2.0 ** -24 * clean.abs().max()
-    assert not got[where:, 5].isfinite().any()
+    states = [start.clone(), start.clone()]
+    outs = [linear_scan(q, k, v, heads, dk, dv, dataclasses.replace(step, longest_run=m), s, **kw) for m, s in zip((step.longest_run, 0), states)]
+    # fp32 throughout: a few units of rounding per token of a run and per entry of a sum, against the largest result
+    for x, y in ((outs[0], want), (states[0], want_state)):
+        assert (x.to(F64) - y).abs().max() <= 64 * 2.0 ** -24 * y.abs().max()
+    assert torch.equal(outs[0], outs[1]) and torch.equal(states[0], states[1])
 
 
 @pytest.mark.parametrize("kind,heads,qk_heads,dk,dv", [("fixed", 5, 5, 64, 68), ("entry", 4, 4, 24, 40), ("token", 64, 2, 136, 4)])
