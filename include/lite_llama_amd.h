@@ -716,7 +716,9 @@ int ll_rotate_pairs(const void* q, int64_t q_tok_stride, int64_t q_head_stride, 
  * weights are the chosen sigmoid scores themselves.  scoring 4: scores = softmax over all logits, a group's score is its largest,
  * weights as in 0.
  * ll_moe_sort: slots sorted by expert in blocks of `block` = ll_moe_rows_block(...) rows, 32 or 128 (counts: int32 scratch
- * [experts]; sorted [num_slots + experts (block - 1)], block_expert [ceil(that / block)], num_post [1]).
+ * [experts]; sorted [num_slots + experts (block - 1)], block_expert [ceil(that / block)], num_post [1]).  ll_moe_sort_skipped (up to 8192
+ * experts): slots whose id lies outside 0 .. experts - 1 follow in a run of their own under expert -1 (arrays for experts + 1 runs);
+ * ll_moe_rows_gemm writes zeros for them where glu == 0 or 3, nothing where it makes gated activations.
  * ll_moe_rows_gemm: glu != 0: w [experts][2 N][K] (gate rows, then up rows), out[slot] = silu(a Wg^T) * (a Wu^T) with
  * a = row slot / a_div (glu == 2: g' sigmoid(1.702 g') (u' + 1) with g' = min(g, limit), u' = clamp(u, -limit, limit));
  * glu == 0: w [experts][N][K], out[slot] = (a W^T) * slot_weight[slot]; glu == 3: w [experts][N][K],
@@ -728,6 +730,8 @@ int ll_group_router(const void* h, int64_t h_ld, const void* w_router, const voi
 int64_t ll_moe_rows_block(int64_t num_slots, int64_t experts, int64_t width, int64_t ff, int dtype);
 int ll_moe_sort(const int32_t* ids, int64_t num_slots, int64_t experts, int64_t block, int32_t* counts, int32_t* sorted,
                 int32_t* block_expert, int32_t* num_post, void* stream);
+int ll_moe_sort_skipped(const int32_t* ids, int64_t num_slots, int64_t experts, int64_t block, int32_t* counts, int32_t* sorted,
+                        int32_t* block_expert, int32_t* num_post, void* stream);
 int ll_moe_rows_gemm(const void* a, int64_t a_ld, int64_t a_div, const void* w, int64_t w_stride_e, int64_t K, int64_t N,
                      int glu, const float* slot_weight, void* out, int64_t out_ld, const int32_t* sorted,
                      const int32_t* block_expert, const int32_t* num_post, int64_t num_slots, int64_t experts, int64_t block,

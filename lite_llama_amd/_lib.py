@@ -134,6 +134,7 @@ SIGNATURES = {
     "ll_group_router": [P, L, P, P, L, L, L, L, L, L, F, I, P, P, P, P, P, L, I, P],
     "ll_moe_rows_block": [L, L, L, L, I],
     "ll_moe_sort": [P, L, L, L, P, P, P, P, P],
+    "ll_moe_sort_skipped": [P, L, L, L, P, P, P, P, P],
     "ll_moe_rows_gemm": [P, L, L, P, L, L, L, I, P, P, L, P, P, P, L, L, L, F, I, P],
     "ll_linear_scan_supported": [L, L],
     "ll_linear_scan": [P, L, P, L, P, L, L, L, L, L, I, I, F, P, P, L, P, F, P, L, P, P, P, P, L, P, P, P, P, P, L, L, I, P],

@@ -303,16 +303,21 @@ def group_router(h: torch.Tensor, router_weight: torch.Tensor, top: int, group_c
     return ids, weights, extra
 
 
-def _sort_slots(ids: torch.Tensor, slots: int, experts: int, width: int, ff: int, dt):
-    """Slots sorted by expert in row blocks: ``(rows per block, sorted slots, expert of every block, [padded count])``."""
+_SKIPPED_RUN = 8192   # most experts beside which ll_moe_sort_skipped sorts skipped slots
+
+
+def _sort_slots(ids: torch.Tensor, slots: int, experts: int, width: int, ff: int, dt, skipped: bool = False):
+    """Slots sorted by expert in row blocks: ``(rows per block, sorted slots, expert of every block, [padded count])``.  ``skipped``:
+    slots whose id is no expert's follow in blocks of expert -1."""
     lib = L.lib()
     block = int(lib.ll_moe_rows_block(slots, experts, width, ff, L.dtype_code(dt)))
-    padded = slots + experts * (block - 1)
+    padded = slots + (experts + (1 if skipped else 0)) * (block - 1)
     meta = torch.empty(experts + padded + -(-padded // block) + 1, dtype=torch.int32, device=ids.device)
     counts, sorted_ids = meta[:experts], meta[experts:experts + padded]
     block_expert, num_post = meta[experts + padded:-1], meta[-1:]
-    L.check(lib.ll_moe_sort(ids.data_ptr(), slots, experts, block, counts.data_ptr(), sorted_ids.data_ptr(), block_expert.data_ptr(),
-                            num_post.data_ptr(), L.stream_ptr()), "moe_sort")
+    sort = lib.ll_moe_sort_skipped if skipped else lib.ll_moe_sort
+    L.check(sort(ids.data_ptr(), slots, experts, block, counts.data_ptr(), sorted_ids.data_ptr(), block_expert.data_ptr(),
+                 num_post.data_ptr(), L.stream_ptr()), "moe_sort")
     return block, sorted_ids, block_expert, num_post
 
 
@@ -339,9 +344,10 @@ def sparse_glu_experts(h: torch.Tensor, w_gate_up: torch.Tensor, w_down: torch.T
         raise ValueError("sparse_glu_experts: int32 ids and fp32 weights [n, top]")
     lib = L.lib()
     slots = n * top
-    block, sorted_ids, block_expert, num_post = _sort_slots(ids, slots, experts, width, ff, dt)
+    run = skipped_ids and experts <= _SKIPPED_RUN    # (the last product writes the skipped slots' zeros)
+    block, sorted_ids, block_expert, num_post = _sort_slots(ids, slots, experts, width, ff, dt, run)
     act = torch.empty(slots, ff, dtype=dt, device=h.device)
-    out = (torch.zeros if skipped_ids else torch.empty)(n, top, width, dtype=dt, device=h.device)
+    out = (torch.zeros if skipped_ids and not run else torch.empty)(n, top, width, dtype=dt, device=h.device)
     code, st = L.dtype_code(dt), L.stream_ptr()
     glu, lim = (1, 0.0) if limit is None else (2, float(limit))
     L.check(lib.ll_moe_rows_gemm(h.data_ptr(), h.stride(0), top, w_gate_up.data_ptr(), w_gate_up.stride(0), width, ff, glu, 0,

@@ -51,3 +51,31 @@ def test_experts_of_every_load(dtype, width, ff, form):
     # two roundings to 16 bits: the activations' (each a half unit, met by weights of std ff^-1/2: 6 deviations) and the result's own
     unit = 2.0 ** (-11 if dtype == torch.float16 else -8)
     assert ((got.to(F64) - want).abs() <= unit * (want.abs() + 6 * mid) + 2.0 ** -14 * unit).all()
+
+
+@pytest.mark.parametrize("slots,experts,block", [(1, 1, 32), (7, 5, 32), (256, 34, 128), (257, 300, 32), (5000, 64, 128), (13057, 3, 128), (900, 9000, 32)])
+@pytest.mark.parametrize("skipped", [False, True])
+def test_slots_sorted_by_expert(slots, experts, block, skipped):
+    """Every expert's slots in their order, padded to blocks; with a run of their own, the slots that no expert serves behind them."""
+    from lite_llama_amd import _lib as L
+
+    if skipped and experts > 8192:
+        pytest.skip("a run of skipped slots stands beside 8192 experts at most")
+    g = torch.Generator().manual_seed(slots)
+    ids = torch.randint(-1, experts + 2, (slots,), generator=g, dtype=torch.int32)
+    runs = [(e, (ids == e).nonzero()[:, 0].tolist()) for e in range(experts)]
+    if skipped:
+        runs.append((-1, ((ids < 0) | (ids >= experts)).nonzero()[:, 0].tolist()))
+    want, want_expert = [], []
+    for e, run in runs:
+        blocks = -(-len(run) // block)
+        want += run + [slots] * (blocks * block - len(run))
+        want_expert += [e] * blocks
+    room = slots + (experts + 1) * (block - 1)
+    dev = ids.to(DEV)
+    counts, out = (torch.empty(k, dtype=torch.int32, device=DEV) for k in (experts, room))
+    expert, post = torch.empty(-(-room // block), dtype=torch.int32, device=DEV), torch.empty(1, dtype=torch.int32, device=DEV)
+    sort = L.lib().ll_moe_sort_skipped if skipped else L.lib().ll_moe_sort
+    L.check(sort(dev.data_ptr(), slots, experts, block, counts.data_ptr(), out.data_ptr(), expert.data_ptr(), post.data_ptr(),
+                 L.stream_ptr()), "moe_sort")
+    assert post.item() == len(want) and out[:len(want)].tolist() == want and expert[:len(want_expert)].tolist() == want_expert
