@@ -286,6 +286,11 @@ int ll_w8a8_matmul(void* out, const int8_t* qa, const float* a_scale, const int8
  * w8a8.py:151-217); this predicate says whether a shape is served (1 / 0; otherwise the 64-row weight-streaming tile loops
  * over M).  wfmt: 1 fp8 e4m3 / 2 int8 weights under fp16 activations, 3 int8 x int8.  n % 32 == 0; k % 64 (128 for wfmt 3). */
 int ll_w8_mtiled_supported(int64_t m, int64_t n, int64_t k, int wfmt, int64_t group_k);
+/* The int8 x int8 product of an interleaved (gate_j, up_j) weight with silu(gate) * up in its epilogue: out fp16 [m, n / 2], the values of
+ * ll_w8a8_matmul followed by ll_silu_and_mul_pairs.  supported: 1 / 0 (more than 64 rows, k % 256 == 0, k >= 512, n % 32 == 0). */
+int ll_w8a8_mtiled_swiglu_supported(int64_t m, int64_t n, int64_t k);
+int ll_w8a8_mtiled_swiglu(void* out, const int8_t* qa, const float* a_scale, const int8_t* qweight, const float* w_scale, int64_t m,
+                          int64_t n, int64_t k, int64_t qw_stride_n, void* stream);
 
 /* Split-K partial mode of the decode-shaped 8-bit / 16-bit engine (no reference counterpart; the int4 engine's epilogue 2 for
  * the other formats): partials [S][M][N] fp32 with the block scales applied, summed by the projection's consumer

@@ -74,6 +74,8 @@ SIGNATURES = {
     "ll_quant_act_cached_try": [P, P, P, L, L, L, P],
     "ll_w8a8_matmul": [P, P, P, P, P, P, L, L, L, L, P, P, P, P],
     "ll_w8_mtiled_supported": [L, L, L, I, L],
+    "ll_w8a8_mtiled_swiglu_supported": [L, L, L],
+    "ll_w8a8_mtiled_swiglu": [P, P, P, P, P, L, L, L, L, P],
     "ll_moe_align_block_size": [P, I, L, I, I, P, P, P, P],
     "ll_moe_align_workspace_ints": [L, I],
     "ll_moe_align_block_size_ws": [P, I, L, I, I, P, P, P, P, L, P],

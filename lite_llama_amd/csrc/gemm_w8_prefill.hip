@@ -352,3 +352,22 @@ extern "C" int ll_w8_mtiled_try(void* out, const void* x, const void* w, const f
 #undef P8_GO
   return hipGetLastError() == hipSuccess ? 1 : LL_ERR_LAUNCH;
 }
+
+// silu(gate) * up of an int8 x int8 gate|up projection whose rows are interleaved (gate_j, up_j): out [m][n / 2], both sums scaled and rounded
+// to fp16 first -- the values of the product and ll_silu_and_mul_pairs over it, in the product's epilogue (5000 rows of 2 x 14336: the
+// activation's launch took 78 us to read and write 430 MB, and the product another 143 MB of stores).
+extern "C" int ll_w8a8_mtiled_swiglu_supported(int64_t m, int64_t n, int64_t k) {
+  return ll_w8_mtiled_supported(m, n, k, 3, k) && tile256_wants(m, n, k, 3) ? 1 : 0;
+}
+
+extern "C" int ll_w8a8_mtiled_swiglu(void* out, const int8_t* qa, const float* a_scale, const int8_t* qweight, const float* w_scale, int64_t m,
+                                     int64_t n, int64_t k, int64_t qw_stride_n, void* stream) {
+  if (!ll_w8a8_mtiled_swiglu_supported(m, n, k) || qw_stride_n % 16 != 0 || qw_stride_n < k || (n - 1) * qw_stride_n + k >= (1ll << 32))
+    return LL_ERR_SHAPE;
+  if (!out || !qa || !a_scale || !qweight || !w_scale || !ll_aligned16(out) || !ll_aligned16(qa) || !ll_aligned16(qweight) || !ll_aligned16(w_scale))
+    return LL_ERR_ARG;
+  T2Params t{};
+  t.out = (uint16_t*)out; t.x = (const unsigned char*)qa; t.w = (const unsigned char*)qweight; t.scales = w_scale; t.a_scale = a_scale;
+  t.m = m; t.n = n; t.k = k; t.x_stride = k; t.w_stride = qw_stride_n; t.group_k = k; t.group_n = 1; t.epi = 1;
+  return tile256_launch(t, 3, stream);
+}

@@ -6,6 +6,7 @@ over the HIP C-ABI.  Same signatures, same ValueErrors, same on-device weight fo
 
 from __future__ import annotations
 
+import math
 import os
 
 import torch
@@ -440,6 +441,31 @@ def smoothquant_gate_up_swiglu(x, qweight, weight_scales, *, max_splits: int = 1
     L.check(L.lib().ll_w8a8_finish_swiglu(out.data_ptr(), parts.data_ptr(), s, a_scale.data_ptr(),
                                           _w8a8_scales(weight_scales).data_ptr(), m, n, L.stream_ptr()),
             "smoothquant_gate_up_swiglu")
+    return out.view(*x.shape[:-1], n // 2)
+
+
+def smoothquant_prefill_swiglu(x, qweight, weight_scales):
+    """:func:`smoothquant_gate_up_swiglu` for prefill shapes (csrc/gemm_tile256.hip): the activation in the GEMM's epilogue, the same
+    values.  ``None`` when not served (up to 64 rows, shapes off the tiles' grid)."""
+    from .norm_act import Int8Rows
+    n, k = qweight.shape
+    m = math.prod(x.shape[:-1]) if x.shape[-1] == k else 0
+    if (qweight.dtype != torch.int8 or qweight.stride(1) != 1 or qweight.stride(0) % 16 or qweight.data_ptr() % 16
+            or not L.lib().ll_w8a8_mtiled_swiglu_supported(m, n, k) or (n - 1) * qweight.stride(0) + k >= 2 ** 32):
+        return None
+    if isinstance(x, Int8Rows):
+        qa, a_scale = x.q, x.scale
+    elif x.is_cuda and x.dtype == torch.float16:
+        a = x.reshape(-1, k)
+        qa, a_scale = quantize_activations_int8(a if a.stride(-1) == 1 else a.contiguous())
+    else:
+        return None
+    ws = _w8a8_scales(weight_scales)
+    if not qa.is_contiguous() or qa.data_ptr() % 16 or ws.data_ptr() % 16 or ws.numel() != n:
+        return None
+    out = torch.empty((m, n // 2), dtype=torch.float16, device=qa.device)
+    L.check(L.lib().ll_w8a8_mtiled_swiglu(out.data_ptr(), qa.data_ptr(), a_scale.data_ptr(), qweight.data_ptr(), ws.data_ptr(), m, n, k,
+                                          qweight.stride(0), L.stream_ptr()), "smoothquant_prefill_swiglu")
     return out.view(*x.shape[:-1], n // 2)
 
 

@@ -85,6 +85,27 @@ def test_int8_by_int8(m, n, k):
     assert torch.equal(K.smoothquant_matmul(x, w, scale), want.half())
 
 
+@pytest.mark.parametrize("m,n,k", [(65, 32, 512), (129, 8192 + 96, 768), (600, 4096 + 32, 512)])
+@pytest.mark.parametrize("quantised", [False, True])
+def test_int8_by_int8_with_the_activation(m, n, k, quantised):
+    """The bits of the product and of the activation's own launch over it."""
+    from lite_llama_amd import kernels as K
+    from lite_llama_amd import _lib as L
+    from lite_llama_amd.kernels.norm_act import Int8Rows
+    from lite_llama_amd.kernels.quantization import quantize_activations_int8, smoothquant_prefill_swiglu
+
+    g = gen(n)
+    w = torch.randint(-127, 128, (n, k), generator=g, device=DEV, dtype=torch.int8)
+    scale = torch.rand(n, 1, generator=g, device=DEV) * 0.001
+    x = torch.randn(m, k, generator=g, device=DEV).half()
+    both = K.smoothquant_matmul(x, w, scale)
+    want = torch.empty(m, n // 2, dtype=torch.float16, device=DEV)
+    L.check(L.lib().ll_silu_and_mul_pairs(want.data_ptr(), both.data_ptr(), m, n // 2, L.LL_F16, L.stream_ptr()), "pairs")
+    got = smoothquant_prefill_swiglu(Int8Rows(*quantize_activations_int8(x), x.shape) if quantised else x, w, scale)
+    assert torch.equal(got, want)
+    assert smoothquant_prefill_swiglu(x[:64], w, scale) is None
+
+
 @pytest.mark.parametrize("fmt", ["fp8", "int8"])
 @pytest.mark.parametrize("tokens,experts,top", [(1100, 4, 2), (2049, 5, 2), (1500, 3, 1)])
 @pytest.mark.parametrize("interleaved", [False, True])
