@@ -90,6 +90,15 @@ int ll_rope_kv_update(void* q, void* kv, const void* cos_t, const void* sin_t, v
                       int64_t sin_s_stride, int64_t pool_stride_t, int64_t pool_stride_h,
                       int qk_dtype, int cs_dtype, int idx_width, const int64_t* positions,
                       void* stream);
+/* ... behind the RMS norm of every q and k head (128 entries, 16-byte aligned rows): two ll_skip_rmsnorm launches and the above. */
+int ll_norm_rope_kv_update(void* q, void* kv, const void* cos_t, const void* sin_t, void* kv_buffer,
+                      const void* q_weight, const void* k_weight, float eps,
+                      const void* select_index, int64_t tokens, int n_qh, int n_kh, int hd,
+                      int64_t q_row_stride, int64_t kv_row_stride, int64_t seq_len,
+                      int64_t cos_b_stride, int64_t cos_s_stride, int64_t sin_b_stride,
+                      int64_t sin_s_stride, int64_t pool_stride_t, int64_t pool_stride_h,
+                      int qk_dtype, int cs_dtype, int idx_width, const int64_t* positions,
+                      void* stream);
 
 /* ---- a3: update_kv_buffer  (kernels/update_kv_buffer.py:54-89) ---------------
  * buf[idx[i], h, :] = vals[i, h, :]  (bit-exact copy; 2-byte elements). */

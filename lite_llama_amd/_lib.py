@@ -33,6 +33,7 @@ SIGNATURES = {
     "ll_activation": [P, P, L, I, I, P],
     "ll_rope": [P, P, P, P, L, I, I, I, L, L, L, L, L, L, L, I, I, P],
     "ll_rope_kv_update": [P, P, P, P, P, P, L, I, I, I, L, L, L, L, L, L, L, L, L, I, I, I, P, P],
+    "ll_norm_rope_kv_update": [P, P, P, P, P, P, P, F, P, L, I, I, I, L, L, L, L, L, L, L, L, L, I, I, I, P, P],
     "ll_update_kv_buffer": [P, P, P, L, I, I, L, L, L, L, I, P],
     "ll_update_kv_index": [P, P, P, P, L, L, L, I, I, I, P],
     "ll_flash_decoding_num_partitions": [L],

@@ -305,13 +305,23 @@ def rope_emb_forward(q, k, cos, sin, batch_size, seq_len):
 
 
 @torch.no_grad()
-def rope_and_cache(q, kv, cos, sin, batch_size, seq_len, select_index, kv_buffer, positions=None):
+def norm_rope_and_cache_supported(q, kv, kv_buffer, q_weight, k_weight) -> bool:
+    """Whether :func:`rope_and_cache` takes ``qk_norm`` for these rows: heads of 128 entries, one 16-bit dtype, 16-byte rows."""
+    return (q.is_cuda and q.shape[2] == 128 and q.dtype == kv.dtype == kv_buffer.dtype == q_weight.dtype == k_weight.dtype
+            and q.dtype in (torch.float16, torch.bfloat16) and q_weight.numel() == 128 and k_weight.numel() == 128
+            and q_weight.is_contiguous() and k_weight.is_contiguous()
+            and all(t.data_ptr() % 16 == 0 for t in (q, kv, kv_buffer, q_weight, k_weight))
+            and all(t.stride(0) % 8 == 0 and t.stride(1) % 8 == 0 and t.stride(2) == 1 for t in (q, kv, kv_buffer)))
+
+
+def rope_and_cache(q, kv, cos, sin, batch_size, seq_len, select_index, kv_buffer, positions=None, qk_norm=None):
     """Extension (one launch instead of two): ``rope_emb_forward(q, k)`` + ``update_kv_buffer(cat(k, v))``
     where ``kv [N, 2*Hkv, D]`` holds this step's K heads then V heads (typically a strided view of the
     fused qkv projection).  ``q`` and the K half of ``kv`` are rotated in place; rotated K and V of
     token ``i`` are written to ``kv_buffer[select_index[i]]``.  Bit-identical to the two-call form.
     With ``positions`` (int64 ``[N]``) ``cos``/``sin`` are position-indexed tables ``[max_pos, >= D/2]``
-    and token ``i`` reads row ``positions[i]`` (no per-step table producer)."""
+    and token ``i`` reads row ``positions[i]`` (no per-step table producer).  ``qk_norm = (q weight, k weight, eps)``: every q and k head
+    passes through its RMS norm first (:func:`norm_rope_and_cache_supported`; the values of ``skip_rmsnorm`` on the heads)."""
     L.require_cuda(q, kv, cos, sin, select_index, kv_buffer)
     N, n_qh, hd = q.shape
     n_kh = kv.shape[1] // 2
@@ -335,9 +345,14 @@ def rope_and_cache(q, kv, cos, sin, batch_size, seq_len, select_index, kv_buffer
         cos = cos.contiguous()
         sin = sin.contiguous()
         strides = (cos.stride(0), cos.stride(1), sin.stride(0), sin.stride(1))
+    fn, norm = L.lib().ll_rope_kv_update, ()
+    if qk_norm is not None:
+        if not norm_rope_and_cache_supported(q, kv, kv_buffer, qk_norm[0], qk_norm[1]):
+            raise ValueError("rope_and_cache: qk_norm needs heads of 128 entries in aligned 16-bit rows")
+        fn, norm = L.lib().ll_norm_rope_kv_update, (qk_norm[0].data_ptr(), qk_norm[1].data_ptr(), float(qk_norm[2]))
     L.check(
-        L.lib().ll_rope_kv_update(
-            q.data_ptr(), kv.data_ptr(), cos.data_ptr(), sin.data_ptr(), kv_buffer.data_ptr(),
+        fn(
+            q.data_ptr(), kv.data_ptr(), cos.data_ptr(), sin.data_ptr(), kv_buffer.data_ptr(), *norm,
             select_index.data_ptr(), N, n_qh, n_kh, hd, q.stride(0), kv.stride(0), seq_len, *strides,
             kv_buffer.stride(0), kv_buffer.stride(1), L.dtype_code(q.dtype), L.dtype_code(cos.dtype),
             L.index_width(select_index), L.ptr(positions), L.stream_ptr(),

@@ -25,7 +25,8 @@ import torch.nn.functional as F
 from .distributed.parallel_state import all_reduce_tp, divide, get_tp_rank, get_tp_world_size
 from .distributed.partition import ShardPlan, make_plan, scale_unit, set_active_plan
 from .kernels.attention import decode_attention, decode_attention_partials, decode_attention_partials_supported
-from .kernels.norm_act import Int8Rows, PartialSums, ScaledInt32Partials, rope_and_cache, skip_rmsnorm_partials, skip_rmsnorm_q8
+from .kernels.norm_act import (Int8Rows, PartialSums, ScaledInt32Partials, norm_rope_and_cache_supported, rope_and_cache,
+                               skip_rmsnorm_partials, skip_rmsnorm_q8)
 from .kernels import (
     flash_attention2_no_pad,
     flash_decoding,
@@ -316,23 +317,27 @@ class Attention(nn.Module):
                                    qk_norm=qk_norm)
             if out is not None:
                 return self.o_proj(out.view(batch, seq_len, self.q_size), partials_ok)
-        if self.use_qk_norm:
+        # heads of 128: the head norms ride in the rope + scatter launch, on the projection output in place
+        norm_rope = self.use_qk_norm and norm_fused and dense_rows and norm_rope_and_cache_supported(
+            xq, xkv, atten_info.kv_buffer[layer_index], self.q_norm_weight, self.k_norm_weight)
+        if self.use_qk_norm and not norm_rope:
             xq, _ = skip_rmsnorm(xq, None, self.q_norm_weight, self.eps)
             xk, _ = skip_rmsnorm(xk, None, self.k_norm_weight, self.eps)
-        fused = not self.use_qk_norm and dense_rows
+        fused = dense_rows and (norm_rope or not self.use_qk_norm)
+        head_norms = qk_norm if norm_rope else None
         if tables is not None and not fused:
             position_embeddings = tables.materialise()
         if fused and tables is not None:
             # rope (position-indexed tables) + KV scatter in one launch, in place
             rope_and_cache(xq, xkv, tables[0], tables[1], batch, seq_len, atten_info.cur_select_index,
-                           atten_info.kv_buffer[layer_index], positions=tables[2])
+                           atten_info.kv_buffer[layer_index], positions=tables[2], qk_norm=head_norms)
             out = self.attn(xq, xkv, atten_info, layer_index, is_prefill=seq_len > 1, cached=True)
             return self.o_proj(out.view(batch, seq_len, self.q_size))
         cos, sin = position_embeddings
         if fused:
             # rope + KV scatter in one launch, in place on the projection output
             rope_and_cache(xq, xkv, cos, sin, batch, seq_len, atten_info.cur_select_index,
-                           atten_info.kv_buffer[layer_index])
+                           atten_info.kv_buffer[layer_index], qk_norm=head_norms)
             out = self.attn(xq, xkv, atten_info, layer_index, is_prefill=seq_len > 1, cached=True)
         else:
             xq, xk = rope_emb_forward(xq, xk, cos, sin, batch, seq_len)
