@@ -554,6 +554,14 @@ int ll_slot_advance(void* b_seq_len, const void* b_req_idx, int32_t* cur_select_
                     const int32_t* table, int64_t table_stride_b, int64_t table_stride_s, int batch,
                     int idx_width, void* stream);
 
+/* Prompts on a padded grid [batch, longest] -> the tokens of all prompts one after the other (total = the sum of their lengths): ids,
+ * positions (element strides of the grid), scatter targets (grid order, int32 / int64), where every prompt starts, its length, and the
+ * packed place of the asked grid rows (negative: from the end; a pad position: the prompt's last token; outside the grid: total). */
+int ll_pack_prompts(const int64_t* ids, int64_t ids_stride_b, int64_t ids_stride_s, const int64_t* positions, int64_t pos_stride_b,
+                    int64_t pos_stride_s, const void* select_index, int sel_width, const void* b_seq_len, int len_width, int64_t batch,
+                    int64_t longest, int64_t total, const int64_t* rows, int64_t num_rows, int64_t* ids_out, int64_t* positions_out,
+                    void* select_out, int32_t* start_out, int64_t* len_out, int64_t* rows_out, void* stream);
+
 /* ---- a16: greedy argmax over logits [rows, n] (engine/sampler.py:227-228) ----- */
 int ll_argmax(int64_t* out, const void* logits, int64_t rows, int64_t n, int64_t stride_row,
               int dtype, void* stream);

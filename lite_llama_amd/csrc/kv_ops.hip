@@ -209,4 +209,83 @@ extern "C" int ll_slot_advance(void* b_seq_len, const void* b_req_idx, int32_t* 
   return LL_LAUNCH_CHECK();
 }
 
+// --------------------------------------------------------------------------- //
+// Prompts on a padded grid [batch, longest] -> the tokens of all prompts one after the other, in one launch: ids, positions and scatter
+// targets of the tokens that a prompt has, where every prompt starts, its length (cut so that it never reaches behind `total`), and
+// for the asked logits rows their place among the packed tokens.  What is bought: projections, norms and experts run on
+// sum(lens) rows instead of batch * longest (6001 of 8144: a 4-bit prefill 7.00 -> 5.61 ms).  Bound by its launch; a workgroup adds up the lengths in front of its prompt
+// itself, so nothing has to be scanned first.
+//   rows: an index of a pad position names the prompt's last token (pad positions have never had defined logits); one outside the
+//   grid becomes `total`, which the gather that uses it refuses.
+// --------------------------------------------------------------------------- //
+__global__ __launch_bounds__(256) void pack_prompts_kernel(
+    const int64_t* __restrict__ ids, int64_t ids_sb, int64_t ids_ss, const int64_t* __restrict__ pos, int64_t pos_sb, int64_t pos_ss,
+    const void* __restrict__ sel, int sel_w, const void* __restrict__ lens, int len_w, int batch, int64_t longest, int64_t total,
+    const int64_t* __restrict__ rows, int num_rows, int64_t* __restrict__ ids_out, int64_t* __restrict__ pos_out, void* __restrict__ sel_out,
+    int32_t* __restrict__ start_out, int64_t* __restrict__ len_out, int64_t* __restrict__ rows_out) {
+  const int tid = threadIdx.x;
+  auto length = [&](int i) -> int64_t {
+    const int64_t n = load_idx_rt(lens, i, len_w);
+    return n < 0 ? 0 : (n > longest ? longest : n);
+  };
+  if ((int)blockIdx.y == batch) {  // the asked rows
+    for (int r = blockIdx.x * 256 + tid; r < num_rows; r += gridDim.x * 256) {
+      int64_t at = rows[r];
+      if (at < 0) at += batch * longest;
+      int64_t to = total;
+      if (at >= 0 && at < batch * longest) {
+        const int i = (int)(at / longest);
+        int64_t j = at - i * longest, first = 0;
+        for (int o = 0; o < i; ++o) first += length(o);
+        const int64_t n = length(i);
+        j = j < n ? j : n - 1;
+        to = first + j;
+        to = to < 0 ? 0 : (to < total ? to : total - 1);
+      }
+      rows_out[r] = to;
+    }
+    return;
+  }
+  __shared__ int64_t part[4];
+  const int b = blockIdx.y;
+  int64_t first = 0;
+  for (int o = tid; o < b; o += 256) first += length(o);
+  for (int off = 32; off > 0; off >>= 1) first += __shfl_xor(first, off);
+  if ((tid & 63) == 0) part[tid >> 6] = first;
+  __syncthreads();
+  first = part[0] + part[1] + part[2] + part[3];
+  int64_t n = length(b);
+  if (first > total) first = total;
+  if (n > total - first) n = total - first;
+  if (blockIdx.x == 0 && tid == 0) {
+    start_out[b] = (int32_t)first;
+    len_out[b] = n;
+  }
+  const int64_t j = (int64_t)blockIdx.x * 256 + tid;
+  if (j >= n) return;
+  ids_out[first + j] = ids[b * ids_sb + j * ids_ss];
+  pos_out[first + j] = pos[b * pos_sb + j * pos_ss];
+  if (sel_w == LL_I32) ((int32_t*)sel_out)[first + j] = ((const int32_t*)sel)[b * longest + j];
+  else ((int64_t*)sel_out)[first + j] = ((const int64_t*)sel)[b * longest + j];
+}
+
+extern "C" int ll_pack_prompts(const int64_t* ids, int64_t ids_stride_b, int64_t ids_stride_s, const int64_t* positions,
+                               int64_t pos_stride_b, int64_t pos_stride_s, const void* select_index, int sel_width, const void* b_seq_len,
+                               int len_width, int64_t batch, int64_t longest, int64_t total, const int64_t* rows, int64_t num_rows,
+                               int64_t* ids_out, int64_t* positions_out, void* select_out, int32_t* start_out, int64_t* len_out,
+                               int64_t* rows_out, void* stream) {
+  if ((sel_width | len_width) & ~1) return LL_ERR_DTYPE;
+  if (batch < 1 || batch > 65534 || longest < 1 || total < 1 || total > batch * longest || batch * longest >= (1ll << 31) || num_rows < 0 ||
+      num_rows >= (1ll << 31))
+    return LL_ERR_SHAPE;
+  if (!ids || !positions || !select_index || !b_seq_len || !ids_out || !positions_out || !select_out || !start_out || !len_out ||
+      (num_rows > 0 && (!rows || !rows_out)))
+    return LL_ERR_ARG;
+  const dim3 grid((unsigned)((longest + 255) / 256), (unsigned)(batch + (num_rows > 0 ? 1 : 0)));
+  pack_prompts_kernel<<<grid, 256, 0, (hipStream_t)stream>>>(ids, ids_stride_b, ids_stride_s, positions, pos_stride_b, pos_stride_s,
+                                                             select_index, sel_width, b_seq_len, len_width, (int)batch, longest, total, rows,
+                                                             (int)num_rows, ids_out, positions_out, select_out, start_out, len_out, rows_out);
+  return LL_LAUNCH_CHECK();
+}
+
 extern "C" int ll_abi_version(void) { return 1; }

@@ -36,6 +36,7 @@ class AttentionMetadata:
     b_req_idx: torch.Tensor | None = None
     b_seq_len: torch.Tensor | None = None
     max_actual_seq_len: int = 0
+    prompt_grid: object = None                             # prefill only: what the host knows of the grid (slots.PromptGrid), or None
     kv_scales: tuple = (1.0, 1.0)                          # fp8 KV pool only (extension): stored value * scale = K / V
 
 

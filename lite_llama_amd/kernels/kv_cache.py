@@ -72,3 +72,31 @@ def update_kv_index(req_to_token_indexs, b_req_idx, b_seq_len, select_index):
         "update_kv_index",
     )
     return
+
+
+@torch.no_grad()
+def pack_prompts(input_ids, position_ids, select_index, b_seq_len, total: int, rows):
+    """Prompts on a padded grid ``[batch, longest]`` -> the tokens of all prompts one after the other (``total`` = the sum of their
+    lengths): ``(ids [1, total], positions [1, total], select_index [total], starts int32 [batch], lengths int64 [batch], rows)``, with
+    ``rows`` the packed places of the asked grid rows."""
+    L.require_cuda(input_ids, position_ids, select_index, b_seq_len, rows)
+    batch, longest = input_ids.shape
+    if input_ids.dtype != torch.int64 or position_ids.dtype != torch.int64 or rows.dtype != torch.int64 or rows.dim() != 1 \
+            or position_ids.shape != input_ids.shape or select_index.numel() != batch * longest or not select_index.is_contiguous() \
+            or b_seq_len.numel() != batch or not b_seq_len.is_contiguous() or not rows.is_contiguous():
+        raise ValueError("pack_prompts: int64 ids and positions [batch, longest], one scatter target per grid row, one length per prompt")
+    dev = input_ids.device
+    out = torch.empty(2 * total + batch + rows.numel(), dtype=torch.int64, device=dev)
+    ids, positions, lens, packed_rows = out.split([total, total, batch, rows.numel()])
+    select = torch.empty(total, dtype=select_index.dtype, device=dev)
+    starts = torch.empty(batch, dtype=torch.int32, device=dev)
+    L.check(
+        L.lib().ll_pack_prompts(
+            input_ids.data_ptr(), input_ids.stride(0), input_ids.stride(1), position_ids.data_ptr(), position_ids.stride(0),
+            position_ids.stride(1), select_index.data_ptr(), L.index_width(select_index), b_seq_len.data_ptr(), L.index_width(b_seq_len),
+            batch, longest, total, rows.data_ptr(), rows.numel(), ids.data_ptr(), positions.data_ptr(), select.data_ptr(),
+            starts.data_ptr(), lens.data_ptr(), packed_rows.data_ptr(), L.stream_ptr(),
+        ),
+        "pack_prompts",
+    )
+    return ids.view(1, total), positions.view(1, total), select, starts, lens, packed_rows

@@ -14,6 +14,7 @@ from the static table below and weights are synthetic (seeded).
 
 from __future__ import annotations
 
+import copy
 import math
 import os
 from dataclasses import dataclass, field
@@ -25,6 +26,7 @@ import torch.nn.functional as F
 from .distributed.parallel_state import all_reduce_tp, divide, get_tp_rank, get_tp_world_size
 from .distributed.partition import ShardPlan, make_plan, scale_unit, set_active_plan
 from .kernels.attention import decode_attention, decode_attention_partials, decode_attention_partials_supported
+from .kernels.kv_cache import pack_prompts
 from .kernels.norm_act import (Int8Rows, PartialSums, ScaledInt32Partials, norm_rope_and_cache_supported, rope_and_cache,
                                skip_rmsnorm_partials, skip_rmsnorm_q8)
 from .kernels import (
@@ -603,11 +605,28 @@ class CausalLM(nn.Module):
         self.rotary_emb = RotaryEmbedding(geo)
         self.eps = geo.rms_norm_eps
 
+    @staticmethod
+    def _packs(input_ids, position_ids, atten_info, logits_rows) -> bool:
+        """Whether a prefill whose host-side lengths are known runs on the prompts' tokens alone instead of the padded grid: pad
+        positions feed nothing but themselves (attention never reads their rows, their own logits are undefined)."""
+        grid = getattr(atten_info, "prompt_grid", None)
+        return (grid is not None and input_ids.is_cuda and tuple(input_ids.shape) == (grid.batch, grid.longest)
+                and 1 < grid.total < grid.batch * grid.longest and grid.describes(atten_info)
+                and position_ids.shape == input_ids.shape and input_ids.dtype == torch.int64 and position_ids.dtype == torch.int64
+                and torch.is_tensor(logits_rows) and logits_rows.is_cuda and logits_rows.dtype == torch.int64 and logits_rows.dim() == 1
+                and logits_rows.is_contiguous() and not torch.cuda.is_current_stream_capturing())
+
     @torch.no_grad()
     def forward(self, input_ids, position_ids, atten_info, logits_rows=None):
         """``[batch, seq]`` ids -> ``[batch, seq, vocab]`` fp16 logits.  ``logits_rows`` (extension:
         flat token indices) restricts the lm_head to those rows -- prefill only needs the last
         prompt position of every sequence, not ``batch*seq*vocab`` logits."""
+        if logits_rows is not None and self._packs(input_ids, position_ids, atten_info, logits_rows):
+            grid = atten_info.prompt_grid
+            input_ids, position_ids, select, starts, lens, logits_rows = pack_prompts(
+                input_ids, position_ids, atten_info.cur_select_index, atten_info.b_seq_len, grid.total, logits_rows)
+            atten_info = copy.copy(atten_info)   # (the caller's struct keeps describing the grid)
+            atten_info.cur_select_index, atten_info.b_start_loc, atten_info.b_seq_len = select, starts, lens
         hidden_states = self.embed_tokens(input_ids)
         position_embeddings = self.rotary_emb(hidden_states, position_ids)
         residual = None
