@@ -10,6 +10,11 @@
 //     weights non-temporal.  Four CONSUMERS, one per row group of the tile, run the chunk's 8 x MT MFMA 32x32x16 from LDS
 //     fragments and keep the tile's accumulators (16 x MT registers) for the whole K loop: no cross-wave exchange.  The loaders
 //     run ahead ACROSS tile boundaries, so a tile's epilogue overlaps the next tile's first chunks.
+//   * Long streams: workgroup b begins every tile at chunk b mod (K / 128) and wraps.  All of them beginning at column 0 ask the same few
+//     memory channels where a row is a power of two long (us for 600 MB, 1 row, all from column 0 -> staggered: K = 2048 113 -> 94,
+//     4096 127 -> 98, 8192 139 -> 124; 3584 90 -> 91.  Staggered within an XCD instead, b / 8: 98, 106, 124).  Sums of 16-bit products in
+//     another order round otherwise, so streams under 256 MB, which gain little or nothing (32 rows, K = 2048: 134 MB 31 -> 28 us, 46 MB
+//     13.9 -> 14.9), keep the ascending one; int8 sums are exact, and staggered from 64 MB.
 //   * one s_barrier per chunk; the loaders' operation count per chunk is static (8 + 2 MT pieces each).
 #include <stdlib.h>
 
@@ -37,6 +42,7 @@ struct R16Params {
   int64_t m, n, k, x_stride, w_stride;
   int chunks;        // K / 128
   int rbase, rrem;   // workgroup b owns row groups [b * rbase + min(b, rrem), + rbase + (b < rrem))
+  int stagger;       // workgroups begin a tile at different chunks
   int epi;           // 0: out[m, n] (+ bias);  1: rows are (gate_j, up_j) pairs -> out[m, n / 2] = silu(gate) * up
   const float* a_scale;  // R16_I8 only: per-token activation scales [m], per-channel weight scales [n] (smoothquant, w8a8.py:118-149)
   const float* w_scale;
@@ -83,7 +89,7 @@ __global__ __launch_bounds__(R16_THREADS) __attribute__((amdgpu_waves_per_eu(2, 
       if (r >= p.m) r = p.m - 1;  // rows >= M feed only unstored outputs
       xoff[j] = (uint32_t)(r * p.x_stride * 2 + slot * 16);
     }
-    int issued = 0, t = 0, c = 0;
+    int issued = 0, t = 0, done = 0, c = p.stagger ? b % p.chunks : 0;
     uint32_t dst = 0;
     auto issue = [&]() {
       const int rg = lo + 4 * t + L;
@@ -100,7 +106,8 @@ __global__ __launch_bounds__(R16_THREADS) __attribute__((amdgpu_waves_per_eu(2, 
 #pragma unroll
       for (int j = 0; j < XP; ++j) v3_dma16<false>(dst + LD::W_BYTES + (XP * L + j) * 1024, xb, xoff[j]);
       ++issued;
-      if (++c == p.chunks) { c = 0; ++t; }
+      if (++c == p.chunks) c = 0;
+      if (++done == p.chunks) { done = 0; ++t; }
       dst = dst + LD::SLOT == R * LD::SLOT ? 0 : dst + LD::SLOT;
     };
     const int pre = units < R - 1 ? units : R - 1;
@@ -281,6 +288,7 @@ extern "C" int ll_dense16_rows_matmul(void* out, const void* x, const void* w, c
   p.out = (uint16_t*)out; p.x = (const uint16_t*)x; p.w = (const uint16_t*)w; p.bias = (const uint16_t*)bias;
   p.m = m; p.n = n; p.k = k; p.x_stride = x_stride_m; p.w_stride = w_stride_n;
   p.chunks = (int)(k / 128);
+  p.stagger = n * k * 2 >= (1ll << 28);
   p.epi = epilogue;
   const int64_t rgs = n / 32;
   int grid = r16_num_cus();
@@ -331,6 +339,7 @@ extern "C" int ll_w8a8_rows_matmul(void* out, const int8_t* qa, const float* a_s
   p.m = m; p.n = n; p.k = k;
   p.x_stride = qa_stride_m / 2; p.w_stride = qw_stride_n / 2;  // the kernel addresses rows in 2-byte units
   p.chunks = (int)(k / 256);                                    // 256 bytes of a row per chunk
+  p.stagger = n * k >= (1ll << 26);
   p.epi = epilogue;
   const int64_t rgs = n / 32;
   int grid = r16_num_cus();

@@ -1,0 +1,36 @@
+"""Row-group products over weight streams long enough to be staggered (csrc/gemm_w16_rows.hip) against products of the same operands in fp32 / int64."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n,k", [(65536 + 32, 2048), (32768, 4224), (262144 * 4, 128)])   # (one chunk only: nothing to wrap)
+@pytest.mark.parametrize("m", [1, 33])
+def test_staggered_rows(dtype, n, k, m):
+    from lite_llama_amd.kernels.quantization import dense16_rows_linear
+
+    g = torch.Generator(device=DEV).manual_seed(n + k)
+    w = (torch.randn(n, k, generator=g, device=DEV, dtype=torch.float32) * k ** -0.5).to(dtype)
+    x = torch.randn(m, k, generator=g, device=DEV).to(dtype)
+    got = dense16_rows_linear(x, w)
+    want = torch.cat([x.float() @ part.float().T for part in w.split(65536)], dim=1)
+    # one rounding to the storage dtype; fp32 sums of k products of size ~ k^-1/2 in another order: far below 2^-14
+    unit = 2.0 ** (-11 if dtype == torch.float16 else -8)
+    assert ((got.float() - want).abs() <= unit * want.abs() + 2.0 ** -14).all()
+
+
+def test_staggered_int8_rows():
+    from lite_llama_amd.kernels.quantization import smoothquant_rows_matmul
+
+    n, k, m = 16384 + 32, 4096, 30
+    g = torch.Generator(device=DEV).manual_seed(7)
+    w = torch.randint(-127, 128, (n, k), generator=g, device=DEV, dtype=torch.int8)
+    scale = torch.rand(n, generator=g, device=DEV) * 1e-3
+    x = torch.randn(m, k, generator=g, device=DEV).half()
+    out = smoothquant_rows_matmul(x, w, scale)
+    head = smoothquant_rows_matmul(x, w[:8192], scale[:8192])   # (32 MB: not staggered; sums of whole numbers have one value)
+    assert torch.equal(out[:, :8192], head)
