@@ -13,6 +13,7 @@
 
 #include "common.h"
 #include "gemm_tile256.h"
+#include "moe_stream.h"
 
 struct alignas(16) Q4 {
   uint32_t x, y, z, w;
@@ -767,6 +768,19 @@ extern "C" int ll_moe_gemm(void* c, const void* a, const void* w, const float* w
     t.topk_w = mul_routed_weight & 1 ? (const uint16_t*)topk_w : nullptr;
     t.w_stride_e = w_stride_e; t.s_stride_e = s_stride_e; t.num_slots = (int)num_slots; t.top_k = top_k;
     return tile256_grouped_launch(t, wfmt, stream);
+  }
+  if (num_slots < (1ll << 30) && n <= (1 << 24) && k <= (1 << 24)) {   // few rows per expert: the weights as one stream per CU
+    const int eb = wfmt == LL_W_F16 ? 2 : 1, form = wfmt == LL_W_F16 ? MS_W16 : wfmt == LL_W_FP8E4M3 ? MS_FP8 : MS_INT8;
+    const int mode = mul_routed_weight & 2 ? MS_GLU_ROUNDED : MS_SCALED;
+    const int64_t experts = em / block_m + 1;   // (what the lists hold: at least as many runs as there are)
+    MoeStreamParams t{};
+    t.out = (uint16_t*)c; t.a = (const uint16_t*)a; t.w = (const unsigned char*)w; t.scales = w_scale;
+    t.weight16 = mul_routed_weight & 1 ? (const uint16_t*)topk_w : nullptr;
+    t.sorted = sorted_ids; t.block_expert = expert_ids; t.num_post = num_post;
+    t.a_ld = a_stride_m; t.out_ld = mul_routed_weight & 2 ? n / 2 : n; t.w_stride_e = w_stride_e * eb; t.w_stride_n = w_stride_n * eb;
+    t.s_stride_e = s_stride_e; t.s_stride_n = s_stride_n; t.s_stride_k = s_stride_k; t.group_n = group_n; t.group_k = group_k;
+    t.K = (int)k; t.N = (int)n; t.num_slots = (int)num_slots; t.a_div = top_k; t.block_m = block_m; t.safe = (int)em;
+    if (em < (1ll << 31) && moe_stream_wants(t, form, mode, LL_F16, experts)) return moe_stream_launch(t, form, mode, LL_F16, (hipStream_t)stream);
   }
   MoeParams p{};
   p.c = (uint16_t*)c; p.a = (const uint16_t*)a; p.w = w; p.w_scale = w_scale; p.topk_w = (const uint16_t*)topk_w;
