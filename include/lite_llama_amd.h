@@ -278,6 +278,20 @@ int ll_w4a16_mtiled_supported(int64_t m, int64_t n, int64_t k, int group_size); 
 int ll_w4a16_matmul_prepacked_mtiled(void* out, const void* x, const void* wpacked, const void* spacked, const void* bias,
                                      int64_t m, int64_t n, int64_t k, int group_size, int64_t x_stride_m, int epilogue,
                                      void* stream);
+/* ... and the products below whose many rows take 256 x 256 tiles, with scratch memory (device, 16-byte aligned, ll_tile256_split_bytes of it; wf 0
+ * int4, 1 fp8, 2 int8, 3 int8 x int8; 0 bytes: none is used) through which the tiles behind the last full round of the chip are shared by several
+ * workgroups each.  Without it, or with less, the forms without _split. */
+int64_t ll_tile256_split_bytes(int64_t m, int64_t n, int64_t k, int wf);
+int ll_w4a16_matmul_prepacked_mtiled_split(void* out, const void* x, const void* wpacked, const void* spacked, const void* bias,
+                                           int64_t m, int64_t n, int64_t k, int group_size, int64_t x_stride_m, int epilogue,
+                                           void* planes, int64_t plane_bytes, void* stream);
+int ll_w8a16_matmul_split(void* out, const void* x, const void* qweight, const float* scales, const void* bias, int64_t m, int64_t n,
+                          int64_t k, int group_n, int64_t group_k, int wfmt, int64_t x_stride_m, int64_t qw_stride_n, int64_t s_stride_n,
+                          int64_t s_stride_k, float* workspace, int32_t* counters, void* planes, int64_t plane_bytes, void* stream);
+int ll_w8a8_matmul_split(void* out, const int8_t* qa, const float* a_scale, const int8_t* qweight, const float* w_scale, const void* bias,
+                         int64_t m, int64_t n, int64_t k, int64_t qw_stride_n, int32_t* acc_out, int32_t* workspace, int32_t* counters,
+                         void* planes, int64_t plane_bytes, void* stream);
+
 /* Host-side introspection (tests, DESIGN_NOTEBOOK.md; no device work): the launch plan ll_w4a16_matmul_prepacked uses for (n, k,
  * epilogue) as 16 ints -- grid, 128-row blocks per tile, tiles, chunks, slab slots, tile-group split (gt, gbase, grem, lead,
  * xcd_shift), stream-K units per workgroup, four reserved zeros, compute units assumed.  tests/test_host_cpu.py restates the

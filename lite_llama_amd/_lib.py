@@ -62,6 +62,10 @@ SIGNATURES = {
     "ll_w4a16_v4_plan": [L, L, L, I, I, P],
     "ll_w4a16_mtiled_supported": [L, L, L, I],
     "ll_w4a16_matmul_prepacked_mtiled": [P, P, P, P, P, L, L, L, I, L, I, P],
+    "ll_tile256_split_bytes": [L, L, L, I],
+    "ll_w4a16_matmul_prepacked_mtiled_split": [P, P, P, P, P, L, L, L, I, L, I, P, L, P],
+    "ll_w8a16_matmul_split": [P, P, P, P, P, L, L, L, I, L, I, L, L, L, L, P, P, P, L, P],
+    "ll_w8a8_matmul_split": [P, P, P, P, P, P, L, L, L, L, P, P, P, P, L, P],
     "ll_w4a16_v3_plan": [L, L, L, I, I, P],
     "ll_w8a16_matmul": [P, P, P, P, P, L, L, L, I, L, I, L, L, L, L, P, P, P],
     "ll_quantize_activations_int8": [P, P, P, L, L, L, P],
@@ -159,7 +163,7 @@ SIGNATURES = {
     "ll_stream_norm": [P, L, L, P, P, L, P, P, P, P, P, P, P, F, F, P, L, L, L, I, P],
 }
 
-_RETURNS_I64 = {"ll_linear_scan_walk_floats", "ll_rglru_scan_scratch_floats", "ll_delta_scan_scratch_floats", "ll_ragged_attention_partition", "ll_mingru_scan_scratch_floats", "ll_moe_rows_block", "ll_kv_alloc_scratch_bytes", "ll_tp_oneshot_flag_words", "ll_moe_router_workspace_floats", "ll_moe_align_workspace_ints"}
+_RETURNS_I64 = {"ll_tile256_split_bytes", "ll_linear_scan_walk_floats", "ll_rglru_scan_scratch_floats", "ll_delta_scan_scratch_floats", "ll_ragged_attention_partition", "ll_mingru_scan_scratch_floats", "ll_moe_rows_block", "ll_kv_alloc_scratch_bytes", "ll_tp_oneshot_flag_words", "ll_moe_router_workspace_floats", "ll_moe_align_workspace_ints"}
 _lib = None
 
 

@@ -13,7 +13,9 @@ struct T2Params {
   int32_t* acc_out;         // int8 x int8: raw sums [M][N] or nullptr
   int64_t m, n, k, x_stride, w_stride, s_stride_n, s_stride_k, group_k;
   int group_n, chunks, gshift, epi;
-  int tiles_m, tiles_n;     // (filled by the launch)
+  int tiles_m, tiles_n;     // (filled by the launch, like the next ones)
+  int full, rest, slices, slice_steps;  // tiles that are multiplied whole, tiles behind them in `slices` parts of slice_steps steps
+  void* planes;             // their sums
   // expert products (8-bit weights): blocks of 256 sorted slots of one expert, num_post of them in all (a device value)
   const int32_t *sorted_ids, *expert_ids, *num_post;
   const uint16_t* topk_w;   // weight per slot, or nullptr
@@ -21,7 +23,8 @@ struct T2Params {
   int num_slots, top_k;
 };
 
-// Whether [m, k] x [n, k]^T should take the 256 x 256 tiles; wf as the kernel's (0 int4, 1 fp8, 2 int8, 3 int8 x int8).
-int tile256_wants(int64_t m, int64_t n, int64_t k, int wf);
-int tile256_launch(T2Params& p, int wf, void* stream);
+// Whether [m, k] x [n, k]^T should take the 256 x 256 tiles; wf as the kernel's (0 int4, 1 fp8, 2 int8, 3 int8 x int8); split: the caller
+// brings the ll_tile256_split_bytes() that the last round of tiles is shared through.
+int tile256_wants(int64_t m, int64_t n, int64_t k, int wf, bool split = false);
+int tile256_launch(T2Params& p, int wf, void* planes, int64_t plane_bytes, void* stream);
 int tile256_grouped_launch(T2Params& p, int wf, void* stream);

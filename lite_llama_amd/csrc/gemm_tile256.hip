@@ -14,6 +14,8 @@
 //     under its MFMAs.  At the barrier everything requested before it has to be there;
 //   * the steps of a workgroup's tiles are one sequence: the next tile's first steps are requested under this tile's last, its first weights
 //     parked before the epilogue (a tile per launch slot instead spent 13 - 27 thousand cycles of 100 - 150 on its ramp and epilogue);
+//   * the tiles behind the last full round of the chip are cut along the contraction, a slice per idle CU (SPLIT), and added up by a launch of
+//     their own (t2_plan has the rule and what it buys);
 //   * tiles are dealt to the 8 XCDs in contiguous ranges of an order that walks 8 row tiles x 4 column tiles together: the 32 CUs of an
 //     XCD share 8 + 4 operand tiles through their L2, whatever the number of tiles.
 // What bounds it: calls back to back on an otherwise idle card, silu(gate) * up in the epilogue.  8144 x 37888 x 3584 int4: 1.85 ms = 1.19 PFLOP/s
@@ -31,7 +33,8 @@
 // WF: 0 int4 (the decode engines' packed stream), 1 fp8 e4m3, 2 int8 (fp16 activations), 3 int8 x int8.
 // MF: 32-row token fragments of a wave: 4 on four waves, 2 on eight.
 // GROUPED: expert products over rows sorted by expert (moe.hip: blocks of 256 slots of one expert).
-template <int WF, int MF, bool GROUPED>
+// SPLIT: slices of the contraction of the tiles behind the full rounds, one per workgroup: raw sums -> planes (tile256_finish_kernel).
+template <int WF, int MF, bool GROUPED, bool SPLIT>
 __global__ __launch_bounds__(1024 / MF) __attribute__((amdgpu_waves_per_eu(4 / MF, 4 / MF))) void tile256_kernel(const T2Params p) {
   constexpr int NWV = 16 / MF;         // waves
   constexpr int XP = 32 / NWV;         // activation pieces per wave and step
@@ -45,12 +48,12 @@ __global__ __launch_bounds__(1024 / MF) __attribute__((amdgpu_waves_per_eu(4 / M
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nl = lane & 31, h = lane >> 5;
-  const int ksteps = (int)(p.k / BK);
+  int ksteps = (int)(p.k / BK), kfirst = 0;
   auto swz = [](int row, int slot) { return slot ^ ((row >> 1) & 7); };
 
   // ---- the workgroup's tiles: its XCD's range, every `stride`-th ----
   const int tiles_m = GROUPED ? p.num_post[0] >> 8 : p.tiles_m;
-  const int tiles = tiles_m * p.tiles_n, per = (tiles + 7) >> 3;
+  const int tiles = GROUPED ? tiles_m * p.tiles_n : SPLIT ? p.rest * p.slices : p.full, per = (tiles + 7) >> 3;
   const int stride = (int)gridDim.x >> 3;
   int t = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
   const int tend = ((int)blockIdx.x & 7) * per + per < tiles ? ((int)blockIdx.x & 7) * per + per : tiles;
@@ -63,6 +66,13 @@ __global__ __launch_bounds__(1024 / MF) __attribute__((amdgpu_waves_per_eu(4 / M
     m = (8 * g + (i - n * rows)) * 256;
     n *= 256;
   };
+  const int item = t;
+  if constexpr (SPLIT) {   // items of one slice stand together: the CUs of an XCD read the same columns of the contraction
+    const int slice = t / p.rest;
+    t = p.full + t - slice * p.rest;
+    kfirst = slice * p.slice_steps;
+    ksteps = ksteps - kfirst < p.slice_steps ? ksteps - kfirst : p.slice_steps;
+  }
   int m0, n0, m1, n1;  // first row / column of the tile that is multiplied, of the one whose steps are requested after it
   tile_of(t, m0, n0);
 
@@ -141,6 +151,11 @@ __global__ __launch_bounds__(1024 / MF) __attribute__((amdgpu_waves_per_eu(4 / M
   // are multiplied.  xk / wk: steps requested of the tile that is aimed at; kin / kg: the scale block of the step requested next.
   int xk = 0, wk = 0, kin = 0;
   int64_t kg = 0;
+  if constexpr (SPLIT && WF != 0 && !I8A) {
+    const int64_t from = (int64_t)kfirst * 64, block = from / p.group_k;
+    kin = (int)(from - block * p.group_k);
+    kg = block * p.s_stride_k;
+  }
   auto load_w = [&](WRegs& r) {
     if constexpr (I8A) return;
     if (wk == ksteps) {
@@ -149,7 +164,7 @@ __global__ __launch_bounds__(1024 / MF) __attribute__((amdgpu_waves_per_eu(4 / M
       aim_w(m1, n1);
     }
     if constexpr (WF == 0) {
-      const int c = wk >> 1, kh = wk & 1;
+      const int c = (SPLIT ? kfirst + wk : wk) >> 1, kh = wk & 1;   // (slices begin at even steps)
 #pragma unroll
       for (int j = 0; j < NL; ++j) {
         r.w[j] = *reinterpret_cast<const u32x4*>(wbase + (size_t)c * 8192 + kh * 4096 + woff[j]);
@@ -158,7 +173,7 @@ __global__ __launch_bounds__(1024 / MF) __attribute__((amdgpu_waves_per_eu(4 / M
     } else {
 #pragma unroll
       for (int j = 0; j < NL; ++j) {
-        r.w[j] = *reinterpret_cast<const u32x4*>(wbase + (size_t)wk * 64 + woff[j]);
+        r.w[j] = *reinterpret_cast<const u32x4*>(wbase + (size_t)(SPLIT ? kfirst + wk : wk) * 64 + woff[j]);
         r.s1[j] = *reinterpret_cast<const float*>(sbase + kg * 4 + soff[j]);
       }
       kin += 64;
@@ -177,8 +192,8 @@ __global__ __launch_bounds__(1024 / MF) __attribute__((amdgpu_waves_per_eu(4 / M
         aim_x(m1);
         if constexpr (I8A) aim_w(m1, n1);
       }
-      xb = p.x + (size_t)xk * 128;
-      if constexpr (I8A) wb = p.w + (size_t)xk * 128;
+      xb = p.x + (size_t)(SPLIT ? kfirst + xk : xk) * 128;
+      if constexpr (I8A) wb = p.w + (size_t)(SPLIT ? kfirst + xk : xk) * 128;
       ++xk;
     }
     if (j < XP) v3_dma16<false>((uint32_t)(buf * OPND + (wv * XP + j) * 1024), xb, xoff[j]);
@@ -295,7 +310,7 @@ __global__ __launch_bounds__(1024 / MF) __attribute__((amdgpu_waves_per_eu(4 / M
     __builtin_amdgcn_sched_barrier(0);                                                                   \
   }
   for (;;) {
-  const bool more = t + stride < tend;
+  const bool more = !SPLIT && t + stride < tend;
   if (more) tile_of(t + stride, m1, n1);  // (else: the same tile's first steps once more, never multiplied)
   fetch_slots(m1);
   int slot0[GROUPED ? MF : 1];
@@ -323,6 +338,28 @@ __global__ __launch_bounds__(1024 / MF) __attribute__((amdgpu_waves_per_eu(4 / M
       T2_STEP(rB, Q1, Q0, false)
       left -= 2;
     } while (left > 0);
+  }
+
+  if constexpr (SPLIT) {   // 1 KB per wave and store: the finishing launch reads them in the same order
+#pragma unroll
+    for (int ni = 0; ni < 4; ++ni)
+#pragma unroll
+      for (int mi = 0; mi < MF; ++mi) {
+        asm volatile("" : "+a"(acc[ni][mi]));
+        Acc a = acc[ni][mi];
+        char* to = (char*)p.planes + ((size_t)item * 64 + (wv * 4 + ni) * MF + mi) * 4096 + lane * 16;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          i32x4 v;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            if constexpr (I8A) v[e] = a[4 * g + e];
+            else v[e] = (int)__float_as_uint(a[4 * g + e]);
+          }
+          *reinterpret_cast<i32x4*>(to + g * 1024) = v;
+        }
+      }
+    break;
   }
 
   // ---- epilogue: a lane holds, for token row m = nl, the weight rows 8 g + 4 h .. + 3 of a 32-row group ----
@@ -446,6 +483,117 @@ __global__ __launch_bounds__(1024 / MF) __attribute__((amdgpu_waves_per_eu(4 / M
   __builtin_amdgcn_s_waitcnt(0x0070);  // (the requests past the last tile have landed before the LDS is given back)
 }
 
+// Sums of the slices of the tiles behind the full rounds, in slice order, through the epilogue above.  A wave per 32 x 32 results; bound by
+// reading the planes (4 TB/s).
+template <int WF, int MF>
+__global__ __launch_bounds__(256) void tile256_finish_kernel(const T2Params p) {
+  constexpr bool I8A = WF == 3;
+  const int lane = threadIdx.x & 63, nl = lane & 31, h = lane >> 5;
+  const int ti = (int)blockIdx.x >> 4, frag = ((int)blockIdx.x & 15) * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  constexpr int MP = 8 / MF;
+  const int mi = frag % MF, ni = frag / MF & 3, wv = frag / (4 * MF);
+  const int wn = wv / MP, wm = MF == 2 ? (wv + 2 * wn) % MP : wv % MP;
+  int i = p.full + ti;
+  const int gsz = 8 * p.tiles_n, g8 = i / gsz;
+  i -= g8 * gsz;
+  const int rows = p.tiles_m - 8 * g8 < 8 ? p.tiles_m - 8 * g8 : 8, tn = i / rows;
+  const int64_t mrow = (int64_t)(8 * g8 + (i - tn * rows)) * 256 + (wm * MF + mi) * 32 + nl;
+  const int64_t ncol = (int64_t)tn * 256 + wn * 128 + ni * 32;
+  if (ncol >= p.n || mrow - nl >= p.m) return;   // (wave-uniform)
+  const char* from = (const char*)p.planes + ((size_t)ti * 64 + frag) * 4096 + lane * 16;
+  const size_t plane = (size_t)p.rest * 64 * 4096;
+  i32x4 sum[4];
+#pragma unroll
+  for (int g = 0; g < 4; ++g) sum[g] = *reinterpret_cast<const i32x4*>(from + g * 1024);
+  for (int s = 1; s < p.slices; ++s) {
+    from += plane;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const i32x4 v = *reinterpret_cast<const i32x4*>(from + g * 1024);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if constexpr (I8A) sum[g][e] += v[e];
+        else sum[g][e] = (int)__float_as_uint(__uint_as_float((uint32_t)sum[g][e]) + __uint_as_float((uint32_t)v[e]));
+      }
+    }
+  }
+  const bool row_ok = mrow < p.m;
+  const float as = I8A ? p.a_scale[row_ok ? mrow : 0] : 1.f;
+  uint32_t lo[4], hi[4], sg[4];
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const int64_t col = ncol + 8 * g + 4 * h;
+    float v[4];
+    if constexpr (I8A) {
+      const f32x4 ws = *reinterpret_cast<const f32x4*>(p.scales + col);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = ((float)sum[g][e] * as) * ws[e];
+      if (p.acc_out && row_ok) *reinterpret_cast<i32x4*>(p.acc_out + mrow * p.n + col) = sum[g];
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = __uint_as_float((uint32_t)sum[g][e]);
+    }
+    if (p.bias) {
+      const uint2 b = *reinterpret_cast<const uint2*>(p.bias + col);
+      v[0] += f16_bits_to_f32((uint16_t)(b.x & 0xffffu));
+      v[1] += f16_bits_to_f32((uint16_t)(b.x >> 16));
+      v[2] += f16_bits_to_f32((uint16_t)(b.y & 0xffffu));
+      v[3] += f16_bits_to_f32((uint16_t)(b.y >> 16));
+    }
+    uint16_t o[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = f32_to_f16_bits(ll_pinned(v[e]));
+    lo[g] = (uint32_t)o[0] | ((uint32_t)o[1] << 16);
+    hi[g] = (uint32_t)o[2] | ((uint32_t)o[3] << 16);
+    if (p.epi)
+      sg[g] = (uint32_t)f32_to_f16_bits(ll_silu_mul_f32(f16_bits_to_f32(o[0]), f16_bits_to_f32(o[1]))) |
+              ((uint32_t)f32_to_f16_bits(ll_silu_mul_f32(f16_bits_to_f32(o[2]), f16_bits_to_f32(o[3]))) << 16);
+  }
+  if (!row_ok) return;
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const int64_t col = ncol + 8 * g + 4 * h;
+    if (p.epi) *reinterpret_cast<uint32_t*>(p.out + mrow * (p.n >> 1) + (col >> 1)) = sg[g];
+    else *reinterpret_cast<uint2*>(p.out + mrow * p.n + col) = uint2{lo[g], hi[g]};
+  }
+}
+
+// How the tiles behind the full rounds are shared: `slices` parts of the contraction each (1: not at all), of `steps` 64 (int8 x int8 128)
+// columns.  A few tiles alone cost a whole contraction on idle neighbours; shared, 1 / slices of it, the sums' way to memory and back (0.1 us a
+// plane) and a launch.  us, whole -> shared, int8 x int8 4096 x 14336: 16 tiles (100 rows) 114 -> 33, 64 121 -> 70, 128 128 -> 115, 272 (4280 rows)
+// 291 -> 216; 4096 x 4096, 32 tiles 42 -> 29, 272 96 -> 83; fp8 2048 x 4096, 16 tiles 86 -> 32, 64 89 -> 56; int4 37888 x 3584, 296
+// tiles 166 -> 142, but 888 (120 behind three rounds, halves) 366 -> 375: behind full rounds it has to promise more.
+struct T2Plan {
+  int full, rest, slices, steps;
+  double rounds;   // what all tiles cost, in full rounds
+};
+static T2Plan t2_plan(int64_t m, int64_t n, int64_t k, int wf) {
+  const int64_t tiles = ((m + 255) / 256) * ((n + 255) / 256);
+  T2Plan r{(int)(tiles / 256 * 256), (int)(tiles % 256), 1, 0, 0.0};
+  const int steps = (int)(k / (wf == 3 ? 128 : 64));
+  const double step = 1.45, whole = steps * step;   // us
+  double best = (r.full > 0 ? 0.8 : 0.95) * whole;
+  r.rounds = (double)((tiles + 255) / 256);
+  for (int s = 2; s <= 64 && s * r.rest <= 256 && r.rest > 0; ++s) {
+    const int each = (steps + 2 * s - 1) / (2 * s) * 2;
+    const int parts = (steps + each - 1) / each;
+    if (steps - (parts - 1) * each < 8) continue;
+    const double cost = each * step + 6.0 + 0.1 * r.rest * parts;
+    if (cost >= best) continue;
+    best = cost;
+    r.slices = parts;
+    r.steps = each;
+    r.rounds = r.full / 256 + cost / whole;
+  }
+  return r;
+}
+
+extern "C" int64_t ll_tile256_split_bytes(int64_t m, int64_t n, int64_t k, int wf) {
+  if (m < 1 || n < 1 || m >= (1ll << 30) || n >= (1ll << 30) || wf < 0 || wf > 3 || !tile256_wants(m, n, k, wf, true)) return 0;
+  const T2Plan r = t2_plan(m, n, k, wf);
+  return r.slices > 1 ? (int64_t)r.rest * r.slices * 64 * 4096 : 0;
+}
+
 // Whether the 256 x 256 tiles take [m, k] x [n, k]^T: an even number of steps, at least eight (the pipeline's reach is four), and shapes at
 // which they are the faster engine.  They pay about 3 us once (a ramp of three steps, one workgroup on a CU), and the CUs that the last round
 // of tiles leaves idle; the 128-row engines walk groups of 16 x 16 tiles, and pay for columns that end early in one.  us, 128-row engine ->
@@ -455,14 +603,20 @@ __global__ __launch_bounds__(1024 / MF) __attribute__((amdgpu_waves_per_eu(4 / M
 //          is below what the 128-row engine wastes on its 17th .. 32nd column (3584 columns, 10 700 rows = 2.3 rounds 1.12x, 9300 = 2.02 0.96x;
 //          4096 x 3584, 7168 rows = 1.75 rounds 1.07x, 6144 = 1.5 0.95x).  Short contractions pay the ramp per tile: k 512 4352 x 2048
 //          rows 0.91x, 8192 x 4096 0.86x, k 1024 4096 x 6144 0.87x, 12288 x 2048 0.91x.
+//          With their last round shared (t2_plan), few tiles of a long contraction are faster here too (3584 x 18944, 28 tiles 249 -> 80 us, 112 293
+//          -> 255; 3584 x 3584, 28 tiles 53 -> 36, 84 57 -> 61), and a sliver behind a full round loses nothing (4608 x 3584, 306 tiles 167 -> 151).
 //   8-bit  weights under fp16: any rows past 16 column tiles (5120 x 2048 fp8, 96 rows 1.4x, 8192 1.6x); up to 16 the 128-row engine's one round
 //          is as good until k or the rows outgrow it: k 2048, 256 rows 4096 columns 41.4 -> 44.9 (int8), k 3072 1.14x; k 1024, 1024 rows 1.06x (fp8).
 //   int8   x int8: 4096 x 512, 65 rows 13.0 -> 16.4; k 3072 1.0x, 4096 1.05x; 256 rows k 1536 1.01x; 28672 x 4096, 5000 rows 1.15x.
-int tile256_wants(int64_t m, int64_t n, int64_t k, int wf) {
+int tile256_wants(int64_t m, int64_t n, int64_t k, int wf, bool split) {
   if (k % (wf == 3 ? 256 : 128) != 0 || k < 512) return 0;
   if (m >= (1ll << 30) || n >= (1ll << 30)) return 0;
   const int64_t rows = (m + 255) / 256, cols = (n + 255) / 256, tiles = rows * cols, rounds = (tiles + 255) / 256;
-  if (wf == 0) {
+  const T2Plan plan = t2_plan(m, n, k, wf);
+  if (wf == 0 && split && plan.slices > 1) {
+    if (plan.full > 0) return cols > 16 || plan.rounds * 256 * cols * 20 <= tiles * 16 * 23;
+    return plan.rounds * 1.45 * (k / 64) < (cols > 16 ? 1.2 : 0.87) * (k / 64) + 4;   // (us; the 128-row engine's one round)
+  } else if (wf == 0) {
     if (cols <= 16) {
       if (tiles < 144 || (tiles > 256 && tiles < 368)) return 0;
       if (tiles > 256 && rounds * 256 * cols * 20 > tiles * 16 * 23) return 0;  // rounds / filled rounds <= 1.15 * 16 / cols
@@ -482,36 +636,53 @@ int tile256_wants(int64_t m, int64_t n, int64_t k, int wf) {
   return k >= (wf == 2 && least > 512 && rows <= 8 ? least + 512 : least);
 }
 
-template <int WF, int MF, bool GROUPED>
+template <int WF, int MF, bool GROUPED, bool SPLIT>
 static int t2_go(const T2Params& p, unsigned grid, hipStream_t st) {
   constexpr int bytes = 4 * 256 * 128;
   static bool attr[16] = {false};
   int dev = 0;
   (void)hipGetDevice(&dev);
   if (dev >= 0 && dev < 16 && !attr[dev]) {
-    (void)hipFuncSetAttribute((const void*)tile256_kernel<WF, MF, GROUPED>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    (void)hipFuncSetAttribute((const void*)tile256_kernel<WF, MF, GROUPED, SPLIT>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     attr[dev] = true;
   }
-  tile256_kernel<WF, MF, GROUPED><<<dim3(grid), 1024 / MF, bytes, st>>>(p);
+  tile256_kernel<WF, MF, GROUPED, SPLIT><<<dim3(grid), 1024 / MF, bytes, st>>>(p);
   return hipGetLastError() == hipSuccess ? LL_OK : LL_ERR_LAUNCH;
 }
 
-int tile256_launch(T2Params& p, int wf, void* stream) {
+template <int WF, int MF>
+static int t2_all(T2Params& p, hipStream_t st) {
+  auto grid = [](int64_t tiles) { return (unsigned)((tiles + 7) / 8 < 32 ? (tiles + 7) / 8 * 8 : 256); };  // at most one workgroup per CU
+  if (p.full > 0) {
+    const int r = t2_go<WF, MF, false, false>(p, grid(p.full), st);
+    if (r != LL_OK || p.slices <= 1) return r;
+  }
+  const int r = t2_go<WF, MF, false, true>(p, grid((int64_t)p.rest * p.slices), st);
+  if (r != LL_OK) return r;
+  tile256_finish_kernel<WF, MF><<<dim3((unsigned)p.rest * 16), 256, 0, st>>>(p);
+  return hipGetLastError() == hipSuccess ? LL_OK : LL_ERR_LAUNCH;
+}
+
+int tile256_launch(T2Params& p, int wf, void* planes, int64_t plane_bytes, void* stream) {
   p.tiles_m = (int)((p.m + 255) / 256);
   p.tiles_n = (int)((p.n + 255) / 256);
-  const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;
-  const unsigned grid = (unsigned)((tiles + 7) / 8 < 32 ? (tiles + 7) / 8 * 8 : 256);  // at most one workgroup per CU
+  const T2Plan r = t2_plan(p.m, p.n, p.k, wf);
+  p.slices = 1;
+  p.full = p.tiles_m * p.tiles_n;
+  if (r.slices > 1 && planes && plane_bytes >= (int64_t)r.rest * r.slices * 64 * 4096 && ll_aligned16(planes)) {
+    p.full = r.full; p.rest = r.rest; p.slices = r.slices; p.slice_steps = r.steps; p.planes = planes;
+  }
   hipStream_t st = (hipStream_t)stream;
   switch (wf) {
-    case 0: return t2_go<0, 2, false>(p, grid, st);
-    case 1: return t2_go<1, 2, false>(p, grid, st);
-    case 2: return t2_go<2, 2, false>(p, grid, st);
-    default: return t2_go<3, 4, false>(p, grid, st);
+    case 0: return t2_all<0, 2>(p, st);
+    case 1: return t2_all<1, 2>(p, st);
+    case 2: return t2_all<2, 2>(p, st);
+    default: return t2_all<3, 4>(p, st);
   }
 }
 
 int tile256_grouped_launch(T2Params& p, int wf, void* stream) {
   p.tiles_n = (int)((p.n + 255) / 256);
   hipStream_t st = (hipStream_t)stream;
-  return wf == 1 ? t2_go<1, 2, true>(p, 256, st) : t2_go<2, 2, true>(p, 256, st);
+  return wf == 1 ? t2_go<1, 2, true, false>(p, 256, st) : t2_go<2, 2, true, false>(p, 256, st);
 }

@@ -258,9 +258,9 @@ extern "C" int ll_w4a16_mtiled_supported(int64_t m, int64_t n, int64_t k, int gr
 
 // out [m][n] (epilogue 0, + bias) or [m][n / 2] (epilogue 1: fused gate|up rows interleaved) = x [m][k] @ dequant(W)^T over the
 // load-time layouts of the decode engine; any m >= 1 (meant for m > 64: the decode engines stream the weights once for fewer rows).
-extern "C" int ll_w4a16_matmul_prepacked_mtiled(void* out, const void* x, const void* wpacked, const void* spacked, const void* bias,
-                                                int64_t m, int64_t n, int64_t k, int group_size, int64_t x_stride_m, int epilogue,
-                                                void* stream) {
+extern "C" int ll_w4a16_matmul_prepacked_mtiled_split(void* out, const void* x, const void* wpacked, const void* spacked, const void* bias,
+                                                      int64_t m, int64_t n, int64_t k, int group_size, int64_t x_stride_m, int epilogue,
+                                                      void* planes, int64_t plane_bytes, void* stream) {
   if (m < 0 || n <= 0 || k <= 0 || group_size <= 0) return LL_ERR_SHAPE;
   if (m == 0) return LL_OK;
   if (!ll_w4a16_mtiled_supported(m, n, k, group_size) || x_stride_m % 8 != 0 || (epilogue != 0 && epilogue != 1)) return LL_ERR_SHAPE;
@@ -270,11 +270,11 @@ extern "C" int ll_w4a16_matmul_prepacked_mtiled(void* out, const void* x, const 
   int sh = 0;
   while ((128 << sh) < group_size) ++sh;
   static const int wmh_env = getenv("LL_PF_WMH") ? atoi(getenv("LL_PF_WMH")) : 0;  // A/B knob, read once (1 / 2: this engine, at that tile height)
-  if (!(wmh_env == 1 || wmh_env == 2) && tile256_wants(m, n, k, 0)) {  // (gemm_tile256.hip: both engines' figures beside the rule)
+  if (!(wmh_env == 1 || wmh_env == 2) && tile256_wants(m, n, k, 0, planes && plane_bytes >= ll_tile256_split_bytes(m, n, k, 0))) {  // (gemm_tile256.hip: both engines' figures beside the rule)
     T2Params t{};
     t.out = (uint16_t*)out; t.x = (const unsigned char*)x; t.w = (const unsigned char*)wpacked; t.sp = spacked; t.bias = (const uint16_t*)bias;
     t.m = m; t.n = n; t.k = k; t.x_stride = x_stride_m * 2; t.chunks = (int)(k / 128); t.gshift = sh; t.epi = epilogue;
-    return tile256_launch(t, 0, stream);
+    return tile256_launch(t, 0, planes, plane_bytes, stream);
   }
   PfParams p{};
   p.out = (uint16_t*)out; p.x = (const uint16_t*)x; p.wp = wpacked; p.sp = spacked; p.bias = (const uint16_t*)bias;
@@ -299,4 +299,10 @@ extern "C" int ll_w4a16_matmul_prepacked_mtiled(void* out, const void* x, const 
   if (wmh == 2) wgemm_prefill_kernel<2><<<dim3((unsigned)grid), 512, lds_bytes, (hipStream_t)stream>>>(p);
   else wgemm_prefill_kernel<1><<<dim3((unsigned)grid), 256, lds_bytes, (hipStream_t)stream>>>(p);
   return LL_LAUNCH_CHECK();
+}
+
+extern "C" int ll_w4a16_matmul_prepacked_mtiled(void* out, const void* x, const void* wpacked, const void* spacked, const void* bias,
+                                                int64_t m, int64_t n, int64_t k, int group_size, int64_t x_stride_m, int epilogue,
+                                                void* stream) {
+  return ll_w4a16_matmul_prepacked_mtiled_split(out, x, wpacked, spacked, bias, m, n, k, group_size, x_stride_m, epilogue, nullptr, 0, stream);
 }

@@ -296,7 +296,8 @@ extern "C" int ll_w8_mtiled_supported(int64_t m, int64_t n, int64_t k, int wfmt,
 // Returns 1 when the launch was issued, 0 when the shape / alignment is not served (nothing happened), < 0 on a launch error.
 extern "C" int ll_w8_mtiled_try(void* out, const void* x, const void* w, const float* scales, const float* a_scale, const void* bias,
                                 int32_t* acc_out, int64_t m, int64_t n, int64_t k, int group_n, int64_t group_k, int wfmt,
-                                int64_t x_stride, int64_t w_stride, int64_t s_stride_n, int64_t s_stride_k, void* stream) {
+                                int64_t x_stride, int64_t w_stride, int64_t s_stride_n, int64_t s_stride_k, void* planes, int64_t plane_bytes,
+                                void* stream) {
   if (group_k <= 0 || group_k > k) group_k = k;
   if (!ll_w8_mtiled_supported(m, n, k, wfmt, group_k)) return 0;
   const int eb = wfmt == 3 ? 1 : 2;  // bytes per activation element
@@ -306,13 +307,13 @@ extern "C" int ll_w8_mtiled_try(void* out, const void* x, const void* w, const f
   if (wfmt != 3 && !scales) return 0;
   if (bias && (reinterpret_cast<uintptr_t>(bias) & 7u)) return 0;
   static const int wmh_env = getenv("LL_P8_WMH") ? atoi(getenv("LL_P8_WMH")) : 0;  // A/B knob, read once (1 / 2: this engine, at that tile height)
-  if (!(wmh_env == 1 || wmh_env == 2) && tile256_wants(m, n, k, wfmt)) {  // (gemm_tile256.hip; the kernel below keeps k that is no multiple of 128, for int8 x int8 256)
+  if (!(wmh_env == 1 || wmh_env == 2) && tile256_wants(m, n, k, wfmt, planes && plane_bytes >= ll_tile256_split_bytes(m, n, k, wfmt))) {  // (gemm_tile256.hip; the kernel below keeps k that is no multiple of 128, for int8 x int8 256)
     T2Params t{};
     t.out = (uint16_t*)out; t.x = (const unsigned char*)x; t.w = (const unsigned char*)w; t.scales = scales; t.a_scale = a_scale;
     t.bias = (const uint16_t*)bias; t.acc_out = acc_out;
     t.m = m; t.n = n; t.k = k; t.x_stride = x_stride * eb; t.w_stride = w_stride;
     t.s_stride_n = s_stride_n; t.s_stride_k = s_stride_k; t.group_k = group_k; t.group_n = group_n > 0 ? group_n : 1;
-    return tile256_launch(t, wfmt, stream) == LL_OK ? 1 : LL_ERR_LAUNCH;
+    return tile256_launch(t, wfmt, planes, plane_bytes, stream) == LL_OK ? 1 : LL_ERR_LAUNCH;
   }
   P8Params p{};
   p.out = (uint16_t*)out; p.x = (const unsigned char*)x; p.w = (const unsigned char*)w; p.scales = scales; p.a_scale = a_scale;
@@ -369,5 +370,5 @@ extern "C" int ll_w8a8_mtiled_swiglu(void* out, const int8_t* qa, const float* a
   T2Params t{};
   t.out = (uint16_t*)out; t.x = (const unsigned char*)qa; t.w = (const unsigned char*)qweight; t.scales = w_scale; t.a_scale = a_scale;
   t.m = m; t.n = n; t.k = k; t.x_stride = k; t.w_stride = qw_stride_n; t.group_k = k; t.group_n = 1; t.epi = 1;
-  return tile256_launch(t, 3, stream);
+  return tile256_launch(t, 3, nullptr, 0, stream);
 }

@@ -650,7 +650,7 @@ extern "C" int64_t ll_dense8_partial_words(int64_t m, int64_t n, int64_t k);
 extern "C" int64_t ll_dense16_partial_words(int64_t m, int64_t n, int64_t k);
 extern "C" int ll_w8_mtiled_try(void* out, const void* x, const void* w, const float* scales, const float* a_scale, const void* bias,
                                 int32_t* acc_out, int64_t m, int64_t n, int64_t k, int group_n, int64_t group_k, int wfmt,
-                                int64_t x_stride, int64_t w_stride, int64_t s_stride_n, int64_t s_stride_k, void* stream);  // gemm_w8_prefill.hip
+                                int64_t x_stride, int64_t w_stride, int64_t s_stride_n, int64_t s_stride_k, void* planes, int64_t plane_bytes, void* stream);  // gemm_w8_prefill.hip
 extern "C" int ll_dense8_try(void* out, const void* x, const void* w, const float* scales, const float* a_scale,
                              const void* bias, int32_t* acc_out, int64_t m, int64_t n, int64_t k, int group_n,
                              int64_t group_k, int wfmt, int64_t x_stride, int64_t w_stride, int64_t s_stride_n,
@@ -717,11 +717,11 @@ extern "C" int ll_w4a16_matmul(void* out, const void* x, const int32_t* qweight,
   return LL_ERR_SHAPE;
 }
 
-extern "C" int ll_w8a16_matmul(void* out, const void* x, const void* qweight, const float* scales,
+extern "C" int ll_w8a16_matmul_split(void* out, const void* x, const void* qweight, const float* scales,
                                const void* bias, int64_t m, int64_t n, int64_t k, int group_n,
                                int64_t group_k, int wfmt, int64_t x_stride_m, int64_t qw_stride_n,
-                               int64_t s_stride_n, int64_t s_stride_k, float* workspace,
-                               int32_t* counters, void* stream) {
+                                     int64_t s_stride_n, int64_t s_stride_k, float* workspace,
+                                     int32_t* counters, void* planes, int64_t plane_bytes, void* stream) {
   if (wfmt != LL_W_FP8E4M3 && wfmt != LL_W_INT8) return LL_ERR_DTYPE;
   if (m < 0 || n <= 0 || k <= 0 || group_n <= 0 || group_k <= 0) return LL_ERR_SHAPE;
   if (group_k > k) group_k = k;
@@ -731,7 +731,7 @@ extern "C" int ll_w8a16_matmul(void* out, const void* x, const void* qweight, co
   if (m == 0) return LL_OK;
   if (m > 64) {  // prefill shapes (round 6): M x N tiled MFMA GEMM, the weight tile fetched once per 256 rows (gemm_w8_prefill.hip)
     const int r = ll_w8_mtiled_try(out, x, qweight, scales, nullptr, bias, nullptr, m, n, k, group_n, group_k,
-                                   wfmt == LL_W_FP8E4M3 ? 1 : 2, x_stride_m, qw_stride_n, s_stride_n, s_stride_k, stream);
+                                   wfmt == LL_W_FP8E4M3 ? 1 : 2, x_stride_m, qw_stride_n, s_stride_n, s_stride_k, planes, plane_bytes, stream);
     if (r != 0) return r > 0 ? LL_OK : r;
   }
   {  // decode shapes: full-line weight tiles, split-K partials in the workspace (gemm_w8_skinny.hip)
@@ -749,16 +749,16 @@ extern "C" int ll_w8a16_matmul(void* out, const void* x, const void* qweight, co
   return wfmt == LL_W_FP8E4M3 ? launch_wgemm<FMT_FP8, 1>(p, st) : launch_wgemm<FMT_I8, 1>(p, st);
 }
 
-extern "C" int ll_w8a8_matmul(void* out, const int8_t* qa, const float* a_scale, const int8_t* qweight,
+extern "C" int ll_w8a8_matmul_split(void* out, const int8_t* qa, const float* a_scale, const int8_t* qweight,
                               const float* w_scale, const void* bias, int64_t m, int64_t n, int64_t k,
-                              int64_t qw_stride_n, int32_t* acc_out, int32_t* workspace,
-                              int32_t* counters, void* stream) {
+                                    int64_t qw_stride_n, int32_t* acc_out, int32_t* workspace,
+                                    int32_t* counters, void* planes, int64_t plane_bytes, void* stream) {
   if (m < 0 || n <= 0 || k <= 0) return LL_ERR_SHAPE;
   if (k % 16 != 0 || qw_stride_n % 16 != 0) return LL_ERR_SHAPE;
   if (!ll_aligned16(qa) || !ll_aligned16(qweight)) return LL_ERR_ARG;
   if (m == 0) return LL_OK;
   if (m > 64) {  // prefill shapes (round 6): the M-tiled int8 x int8 engine (gemm_w8_prefill.hip)
-    const int r = ll_w8_mtiled_try(out, qa, qweight, w_scale, a_scale, bias, acc_out, m, n, k, 1, k, 3, k, qw_stride_n, 0, 0, stream);
+    const int r = ll_w8_mtiled_try(out, qa, qweight, w_scale, a_scale, bias, acc_out, m, n, k, 1, k, 3, k, qw_stride_n, 0, 0, planes, plane_bytes, stream);
     if (r != 0) return r > 0 ? LL_OK : r;
   }
   {
@@ -772,6 +772,22 @@ extern "C" int ll_w8a8_matmul(void* out, const int8_t* qa, const float* a_scale,
   p.m = m; p.n = n; p.k = k; p.x_stride = k; p.w_stride = qw_stride_n;
   p.group_n = 1; p.group_k = k;
   return launch_wgemm<FMT_I8I8, 1>(p, (hipStream_t)stream);
+}
+
+extern "C" int ll_w8a16_matmul(void* out, const void* x, const void* qweight, const float* scales,
+                               const void* bias, int64_t m, int64_t n, int64_t k, int group_n,
+                               int64_t group_k, int wfmt, int64_t x_stride_m, int64_t qw_stride_n,
+                               int64_t s_stride_n, int64_t s_stride_k, float* workspace,
+                               int32_t* counters, void* stream) {
+  return ll_w8a16_matmul_split(out, x, qweight, scales, bias, m, n, k, group_n, group_k, wfmt, x_stride_m, qw_stride_n, s_stride_n, s_stride_k,
+                               workspace, counters, nullptr, 0, stream);
+}
+
+extern "C" int ll_w8a8_matmul(void* out, const int8_t* qa, const float* a_scale, const int8_t* qweight,
+                              const float* w_scale, const void* bias, int64_t m, int64_t n, int64_t k,
+                              int64_t qw_stride_n, int32_t* acc_out, int32_t* workspace,
+                              int32_t* counters, void* stream) {
+  return ll_w8a8_matmul_split(out, qa, a_scale, qweight, w_scale, bias, m, n, k, qw_stride_n, acc_out, workspace, counters, nullptr, 0, stream);
 }
 
 // ---------------------------------------------------------------------------------- //

@@ -191,6 +191,12 @@ def w4a16_matmul_prepacked(x, packed_weight, packed_scales, *, group_size: int =
     return out.reshape(*leading, n_out)
 
 
+def _split_scratch(m: int, n: int, k: int, wf: int, device):
+    """Scratch memory through which a product of many rows shares the tiles behind its last full round: ``(tensor or None, bytes)``."""
+    size = L.lib().ll_tile256_split_bytes(m, n, k, wf) if m > 64 else 0
+    return (torch.empty(size, dtype=torch.uint8, device=device) if size else None), size
+
+
 def w4a16_mtiled_supported(m: int, n: int, k: int, group_size: int) -> bool:
     return bool(L.lib().ll_w4a16_mtiled_supported(m, n, k, int(group_size)))
 
@@ -217,9 +223,10 @@ def w4a16_matmul_prepacked_rows(x, packed_weight, packed_scales, *, group_size: 
         bias = bias.half()
     n_out = n // 2 if gate_up_swiglu else n
     out = torch.empty((m, n_out), dtype=x.dtype, device=x.device)
-    L.check(L.lib().ll_w4a16_matmul_prepacked_mtiled(out.data_ptr(), a.data_ptr(), packed_weight.data_ptr(), packed_scales.data_ptr(),
-                                                     L.ptr(bias), m, n, k, int(group_size), a.stride(0), 1 if gate_up_swiglu else 0,
-                                                     L.stream_ptr()), "w4a16_matmul_prepacked_rows")
+    planes, size = _split_scratch(m, n, k, 0, x.device)
+    L.check(L.lib().ll_w4a16_matmul_prepacked_mtiled_split(out.data_ptr(), a.data_ptr(), packed_weight.data_ptr(), packed_scales.data_ptr(),
+                                                           L.ptr(bias), m, n, k, int(group_size), a.stride(0), 1 if gate_up_swiglu else 0,
+                                                           L.ptr(planes), size, L.stream_ptr()), "w4a16_matmul_prepacked_rows")
     return out.reshape(*x.shape[:-1], n_out)
 
 
@@ -289,12 +296,13 @@ def w8a16_matmul(
         bias = bias.half()
     out = torch.empty((m, n), dtype=x.dtype, device=x.device)
     ws, cnt = L.gemm_workspace(x.device, m, n, k)
+    planes, size = _split_scratch(m, n, k, 1 if is_fp8 else 2, x.device)
     L.check(
-        L.lib().ll_w8a16_matmul(
+        L.lib().ll_w8a16_matmul_split(
             out.data_ptr(), a.data_ptr(), qweight.data_ptr(), scales.data_ptr(), L.ptr(bias), m, n, k,
             int(group_n), int(min(group_k, k)), L.LL_W_FP8E4M3 if is_fp8 else L.LL_W_INT8, a.stride(0),
             qweight.stride(0), scales.stride(0), scales.stride(1), ws.data_ptr(), cnt.data_ptr(),
-            L.stream_ptr(),
+            L.ptr(planes), size, L.stream_ptr(),
         ),
         "w8a16_matmul",
     )
@@ -357,11 +365,12 @@ def smoothquant_matmul(
     out = torch.empty((m, n), dtype=torch.float16, device=qa.device)
     acc = torch.empty((m, n), dtype=torch.int32, device=qa.device) if _return_int32 else None
     ws, cnt = L.gemm_workspace(qa.device, m, n, k)
+    planes, size = _split_scratch(m, n, k, 3, qa.device)
     L.check(
-        L.lib().ll_w8a8_matmul(
+        L.lib().ll_w8a8_matmul_split(
             out.data_ptr(), qa.data_ptr(), a_scale.data_ptr(), qweight.data_ptr(),
             weight_scales.data_ptr(), L.ptr(bias), m, n, k, qweight.stride(0), L.ptr(acc),
-            ws.data_ptr(), cnt.data_ptr(), L.stream_ptr(),
+            ws.data_ptr(), cnt.data_ptr(), L.ptr(planes), size, L.stream_ptr(),
         ),
         "smoothquant_matmul",
     )
