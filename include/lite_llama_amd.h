@@ -568,6 +568,20 @@ int ll_slot_advance(void* b_seq_len, const void* b_req_idx, int32_t* cur_select_
                     const int32_t* table, int64_t table_stride_b, int64_t table_stride_s, int batch,
                     int idx_width, void* stream);
 
+/* A decoder layer of an unquantised llama-shaped model (norm, q|k|v, rotation + scatter, attention, o, norm, gate|up + activation, down) over
+ * the tokens (<= 192) of `prompts` prompts, in one call.  residual [tokens][hidden]: updated in place; planes_in > 0: that many fp32 partial
+ * sums per part at `planes` are added to it first (the layer before left them).  Scratch: x [tokens][hidden], qkv [tokens][(heads + 2 kv_heads)
+ * head_dim], attn [tokens][heads head_dim], act [tokens][inter], planes fp32 [parts][max_splits][part][hidden]:
+ * the tokens go through in `parts` = ceil(tokens / 64) parts of `part` = ceil(tokens / parts) rows, with partial sums of their own.  Weights are contiguous [out][in],
+ * gate|up rows interleaved.  Returns the partial sums it left at `planes`, 0: not served (nothing was launched), < 0: an error. */
+int ll_prefill_layer16(void* residual, void* x, int planes_in, float* planes, void* qkv, void* attn, void* act, const void* norm1,
+                       const void* norm2, float eps, const void* w_qkv, const void* b_qkv, const void* w_o, const void* w_gate_up,
+                       const void* w_down, const void* cos_t, const void* sin_t, int64_t cos_b_stride, int64_t cos_s_stride,
+                       int64_t sin_b_stride, int64_t sin_s_stride, void* pool, int64_t pool_stride_t, int64_t pool_stride_h,
+                       const void* select_index, int select_width, const void* starts, int start_width, const void* lens, int len_width,
+                       int64_t prompts, int64_t max_len, int64_t tokens, int64_t seq_len, int64_t hidden, int heads, int kv_heads, int head_dim,
+                       int64_t inter, float sm_scale, int dtype, int cs_dtype, int max_splits, void* stream);
+
 /* Prompts on a padded grid [batch, longest] -> the tokens of all prompts one after the other (total = the sum of their lengths): ids,
  * positions (element strides of the grid), scatter targets (grid order, int32 / int64), where every prompt starts, its length, and the
  * packed place of the asked grid rows (negative: from the end; a pad position: the prompt's last token; outside the grid: total). */

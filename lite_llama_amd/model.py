@@ -40,6 +40,7 @@ from .kernels import (
     flash_decoding_fp8kv,
 )
 from .linear import ColumnParallelLinear, LinearBase, MergedColumnLinear, RowParallelLinear
+from .prefill_layers import ShortPrefill
 from .quantization import QuantConfig, get_moe_method
 
 _LOG2E = 1.4426950408889634  # prefill kernel evaluates exp2 (base.py:45-47)
@@ -630,8 +631,15 @@ class CausalLM(nn.Module):
         hidden_states = self.embed_tokens(input_ids)
         position_embeddings = self.rotary_emb(hidden_states, position_ids)
         residual = None
+        short = ShortPrefill.of(self, hidden_states, position_embeddings, atten_info)   # a host call per layer
         for i, layer in enumerate(self.layers):
-            hidden_states, residual = layer(hidden_states, atten_info, i, position_embeddings, residual)
+            done = short.layer(layer, i, hidden_states, residual) if short is not None else None
+            if done is None:
+                hidden_states = short.done(hidden_states) if short is not None else hidden_states
+                done = layer(hidden_states, atten_info, i, position_embeddings, residual)
+            hidden_states, residual = done
+        if short is not None:
+            hidden_states = short.done(hidden_states)
         hidden_states, _ = add_norm(hidden_states, residual, self.norm_weight, self.eps)
         if logits_rows is not None:
             hidden_states = hidden_states.view(-1, hidden_states.shape[-1])[logits_rows]
