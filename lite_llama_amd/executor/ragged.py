@@ -50,7 +50,6 @@ class _DecodeCell:
 
     graph = None
     packed = None
-    rows = None
     logits = None
 
 
@@ -209,7 +208,9 @@ class RaggedRunner:
         if (self.capture_decode and collect_layers is None and all(len(t) == 1 for _, t in entries)
                 and logits_rows == list(range(len(entries)))):
             return self._decode_step_captured(entries)
-        step, token_ids, rows = self._build(entries, logits_rows)
+        every = len(logits_rows) > 0 and logits_rows == list(range(sum(len(t) for _, t in entries)))
+        step, token_ids, rows = self._build(entries, [] if every else logits_rows)
+        rows = "all" if every else rows
         return self.model(token_ids, step, self.cache, self.token_table, logits_rows=rows, collect_layers=collect_layers)
 
     # ------------------------------------------------------------------ captured decode steps ---- #
@@ -230,8 +231,7 @@ class RaggedRunner:
             self._sightings[key] = self._sightings.get(key, 0) + 1
             if self._sightings[key] < 2:
                 step, token_ids = self._step_from(host.to(self.device), [len(p) for p in parts], len(entries), 1, longest_context)
-                rows = torch.arange(len(entries), device=self.device)
-                return self.model(token_ids, step, self.cache, self.token_table, logits_rows=rows)
+                return self.model(token_ids, step, self.cache, self.token_table, logits_rows="all")
             cell = self._capture_cell(key, host, [len(p) for p in parts], len(entries), key[1] * part)
         cell.packed.copy_(host, non_blocking=True)   # (behind the graph's previous replay; the next step is planned meanwhile)
         cell.graph.replay()
@@ -243,12 +243,11 @@ class RaggedRunner:
             self._cells.pop(next(iter(self._cells)))
         cell = _DecodeCell()
         cell.packed = host.to(self.device)
-        cell.rows = torch.arange(num_seqs, device=self.device)
         torch.cuda.synchronize()
         cell.graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(cell.graph):
             step, token_ids = self._step_from(cell.packed, sizes, num_seqs, 1, context_bound)
-            cell.logits = self.model(token_ids, step, self.cache, self.token_table, logits_rows=cell.rows)
+            cell.logits = self.model(token_ids, step, self.cache, self.token_table, logits_rows="all")
         self._cells[key] = cell
         self._sightings.pop(key, None)
         return cell

@@ -1508,8 +1508,8 @@ class LayeredLM(nn.Module):
 
     @torch.no_grad()
     def forward(self, token_ids, step, cache, token_table, logits_rows=None, collect_layers: list | None = None):
-        """``token_ids [n]`` int64 of the step's flat token array.  ``logits_rows``: int64 indices into it (``None``: no
-        logits, the step only fills cache and state).  ``collect_layers``: a list that receives the fp32 residual stream after
+        """``token_ids [n]`` int64 of the step's flat token array.  ``logits_rows``: int64 indices into it, ``"all"`` for every row in order
+        (decoded tokens: nothing has to be gathered), or ``None``: no logits, the step only fills cache and state.  ``collect_layers``: a list that receives the fp32 residual stream after
         every layer run (diagnostics; costs one add per run)."""
         if self.geo.pair_buckets or self.geo.embed_scale != 1.0:
             x0 = embed_pair(token_ids, self.embed_tokens.weight, self.geo.embed_scale, self.pair_table if self.geo.pair_buckets else None,
@@ -1536,18 +1536,19 @@ class LayeredLM(nn.Module):
                     collect_layers.append(x + delta.float() if delta is not None else x.clone())
         if logits_rows is None:
             return None
-        x = x[logits_rows].contiguous()
-        if self.geo.sandwich or self.geo.post_norm:
-            h = gated_group_norm(x, delta.rows(logits_rows) if delta is not None else None, self.norm_weight, self.geo.eps,
-                                 self.geo.norm_groups)
-        elif self.geo.streams:
-            h, _ = stream_norm(x, delta.rows(logits_rows) if delta is not None else None, self.geo.streams, None, self.norm_weight,
-                               self.geo.eps, self.geo.norm_base)
-        else:
-            if isinstance(delta, SummedUpdate):
+        if not isinstance(logits_rows, str):
+            x = x[logits_rows].contiguous()
+            if isinstance(delta, torch.Tensor):
+                delta = delta[logits_rows].contiguous()
+            elif delta is not None:
                 delta = delta.rows(logits_rows)
-            else:
-                delta = delta[logits_rows].contiguous() if delta is not None else None
+        elif logits_rows != "all":
+            raise ValueError(f"logits_rows: indices, 'all' or None, got {logits_rows!r}")
+        if self.geo.sandwich or self.geo.post_norm:
+            h = gated_group_norm(x, delta, self.norm_weight, self.geo.eps, self.geo.norm_groups)
+        elif self.geo.streams:
+            h, _ = stream_norm(x, delta, self.geo.streams, None, self.norm_weight, self.geo.eps, self.geo.norm_base)
+        else:
             h, _ = add_rmsnorm_shift(x, delta, self.norm_weight, self.geo.eps, x_out=x, out_scale=self.geo.logit_scale)
         logits = self.lm_head(h)
         return softcap_(logits, self.geo.logit_softcap) if self.geo.logit_softcap else logits
