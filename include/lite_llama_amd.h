@@ -371,6 +371,12 @@ int ll_dense16_matmul(void* out, const void* x, const void* w, const void* bias,
 int ll_dense16_rows_supported(int64_t m, int64_t n, int64_t k, int epilogue); /* 1 / 0 */
 int ll_dense16_rows_matmul(void* out, const void* x, const void* w, const void* bias, int64_t m, int64_t n, int64_t k,
                            int64_t x_stride_m, int64_t w_stride_n, int dtype, int epilogue, void* stream);
+/* F.linear of m <= 64 rows over a narrow unquantised weight: out [m][n] = x [m][k] @ w [n][k]^T (+ bias), finished outputs in one launch whatever n.
+ * k % 8 == 0; rows of x and w 16-byte aligned (strides in elements, multiples of 8), out and bias 8-byte aligned. */
+int ll_dense16_narrow_supported(int64_t m, int64_t n, int64_t k); /* 1 / 0 */
+int ll_dense16_narrow_wins(int64_t m, int64_t n, int64_t k); /* 1 where it measured faster than the other routes, else 0 */
+int ll_dense16_narrow_matmul(void* out, const void* x, const void* w, const void* bias, int64_t m, int64_t n, int64_t k, int64_t x_stride_m,
+                             int64_t w_stride_n, int dtype, void* stream);
 /* The same loop for a SmoothQuant (W8A8) projection whose rows arrive already quantised: exact int32 sums on mfma_i32_32x32x32_i8,
  * then ll_w8a8_matmul's epilogue fp16(((float)sum * a_scale[m]) * w_scale[n] (+ bias)) (kernels/quantization/w8a8.py:118-149);
  * epilogue 1: rows of qw interleaved (gate_j, up_j) -> out [m][n / 2] = silu(gate) * up (= ll_w8a8_finish_swiglu).  One launch,

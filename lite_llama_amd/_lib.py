@@ -96,6 +96,9 @@ SIGNATURES = {
     "ll_moe_router": [P, P, P, P, P, L, I, L, L, L, I, I, I, I, P, P, P, P, P],
     "ll_argmax": [P, P, L, L, L, I, P],
     "ll_decode_advance": [P, L, P, P, P, P, P, P, P, P, L, L, I, P],
+    "ll_dense16_narrow_supported": [L, L, L],
+    "ll_dense16_narrow_wins": [L, L, L],
+    "ll_dense16_narrow_matmul": [P, P, P, P, L, L, L, L, L, I, P],
     "ll_prefill_layer16": [P, P, I, P, P, P, P, P, P, F, P, P, P, P, P, P, P, L, L, L, L, P, L, L, P, I, P, I, P, I, L, L, L, L, L, I, I, I, L, F, I, I,
                            I, P],
     "ll_pack_prompts": [P, L, L, P, L, L, P, I, P, I, L, L, L, P, L, P, P, P, P, P, P, P],

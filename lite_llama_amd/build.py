@@ -30,7 +30,7 @@ FILE_FLAGS = {"gemm_short.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"]}
 
 
 # part libraries: the sources ONE model family needs (a fresh checkout serving only that family builds nothing else)
-PARTS = {"ragged": ["seq_mix.hip", "ragged_attn.hip", "ragged_attn_mfma.hip", "group_norm.hip", "latent_attn.hip", "moe_sparse.hip", "moe_stream.hip",
+PARTS = {"ragged": ["seq_mix.hip", "ragged_attn.hip", "ragged_attn_mfma.hip", "group_norm.hip", "latent_attn.hip", "moe_sparse.hip", "moe_stream.hip", "gemm_narrow.hip",
                     "linear_mix.hip", "delta_scan.hip", "stream_norm.hip", "retention.hip", "kv_paged.hip", "kv_ops.hip", "sampler.hip"]}
 
 

@@ -3,8 +3,8 @@
 // Bound by the host: the eight launches of such a layer take 35 - 60 us, and each of them cost 16 - 24 us of interpreter time to prepare (a prompt of
 // 37 tokens through 12 layers of 896: 2290 us, of which the GPU worked 670).  The launches are the eager route's own, in its order and with
 // its arithmetic: norm, q|k|v, rotation + cache scatter, attention, o as split-K partials that the next norm adds up, gate|up with the
-// activation in its epilogue, down as partials.  (The eager route asks the library for q|k|v and o; here both stay on the row-group loop and
-// the split-K engine: 8 us each against 8, without 24 us of the library's host side.)
+// activation in its epilogue, down as partials.  (The eager route asks the library for q|k|v and o; here they stay on the narrow kernel or
+// the row-group loop and on the split-K engine: 5 - 9 us each against 8, without 24 us of the library's host side.)
 // These engines take 64 rows: more go through them in parts of equal size, whose weights the Infinity Cache
 // holds between them, if the layer's are no more than 100 MB.  us, eager -> here: 12 layers of 896 / 4864, 37 tokens 2290 -> 790, 100 2850 -> 1090, 200
 // (four parts) 2790 -> 1530; 4 layers of 1536 / 8960 (94 MB each), 64 tokens 850 -> 374, 100 1020 -> 616, 180 1034 -> 858, 256 1025 -> 1096.
@@ -55,7 +55,9 @@ extern "C" int ll_prefill_layer16(void* residual, void* x, int planes_in, float*
     const int64_t m = i + 1 < parts ? part : last;
     if (planes_in > 0)
       LL_TRY(ll_skip_rmsnorm_partials(rows(x, at, hidden), sums(i), planes_in, rows(residual, at, hidden), norm1, m, hidden, eps, dtype, stream));
-    LL_TRY(ll_dense16_rows_matmul(rows(qkv, at, row), rows(x, at, hidden), w_qkv, b_qkv, m, row, hidden, hidden, hidden, dtype, 0, stream));
+    if (ll_dense16_narrow_wins(m, row, hidden))
+      LL_TRY(ll_dense16_narrow_matmul(rows(qkv, at, row), rows(x, at, hidden), w_qkv, b_qkv, m, row, hidden, hidden, hidden, dtype, stream));
+    else LL_TRY(ll_dense16_rows_matmul(rows(qkv, at, row), rows(x, at, hidden), w_qkv, b_qkv, m, row, hidden, hidden, hidden, dtype, 0, stream));
   }
   LL_TRY(ll_rope_kv_update(qkv, k, cos_t, sin_t, pool, select_index, tokens, heads, kv_heads, head_dim, row, row, seq_len, cos_b_stride,
                            cos_s_stride, sin_b_stride, sin_s_stride, pool_stride_t, pool_stride_h, dtype, cs_dtype, select_width, nullptr, stream));

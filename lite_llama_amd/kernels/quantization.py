@@ -603,6 +603,30 @@ def dense16_rows_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tenso
     return out.reshape(*x.shape[:-1], n_out)
 
 
+def dense16_narrow_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None):
+    """``F.linear(x, weight, bias)`` of up to 64 rows over a narrow unquantised fp16 / bf16 weight (csrc/gemm_narrow.hip); rows of ``x`` may
+    be a column range of wider ones.  ``None`` where the call is not served or another route measured faster
+    (``ll_dense16_narrow_wins``)."""
+    if x.dtype not in (torch.float16, torch.bfloat16) or weight.dtype != x.dtype or weight.dim() != 2 or not x.is_cuda:
+        return None
+    n, k = weight.shape
+    if x.shape[-1] != k or k == 0 or x.numel() > 64 * k or not L.has("ll_dense16_narrow_wins"):
+        return None
+    m = x.numel() // k
+    if not L.lib().ll_dense16_narrow_wins(m, n, k) or os.environ.get("LL_DENSE16_NARROW_OFF"):
+        return None
+    a = x if x.dim() == 2 and x.stride(1) == 1 and x.stride(0) >= k else _flatten(x, k)
+    if (a.stride(0) % 8 or a.data_ptr() % 16 or weight.stride(1) != 1 or weight.stride(0) % 8 or weight.stride(0) < k or weight.data_ptr() % 16
+            or (m > 1 and a.stride(0) < k)):
+        return None
+    if bias is not None and (bias.dtype != x.dtype or bias.numel() != n or not bias.is_contiguous() or bias.data_ptr() % 8):
+        return None
+    out = torch.empty((m, n), dtype=x.dtype, device=x.device)
+    L.check(L.lib().ll_dense16_narrow_matmul(out.data_ptr(), a.data_ptr(), weight.data_ptr(), L.ptr(bias), m, n, k, max(a.stride(0), k),
+                                             weight.stride(0), L.dtype_code(x.dtype), L.stream_ptr()), "dense16_narrow_linear")
+    return out.reshape(*x.shape[:-1], n)
+
+
 def dense16_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None, policy: str = "always"):
     """Extension: ``F.linear(x, weight, bias)`` for decode shapes (<= 64 rows) of an UNQUANTISED fp16 / bf16 weight
     ``[N, K]`` on the split-K weight-streaming kernel (csrc/gemm_w8_skinny.hip, 16-bit form) -- the reference's

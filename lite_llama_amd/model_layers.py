@@ -1096,7 +1096,8 @@ class GatedLinearAttention(nn.Module):
     def forward(self, h, step, cache, run: int, token_table):
         s, qk, v = self.spec, self.qk, self.v
         rows = self.in_proj(h)
-        logits = self.decay_proj(rows[:, 2 * qk + 2 * v:].contiguous())
+        low = rows[:, 2 * qk + 2 * v:]   # (a decoded token's kernel reads the columns where they are)
+        logits = self.decay_proj(low if low.shape[0] <= 64 and rows.shape[1] % 8 == 0 else low.contiguous())
         o = linear_scan(rows[:, :qk], rows[:, qk:2 * qk], rows[:, 2 * qk:2 * qk + v], s.heads, s.dim, s.vdim, step,
                         cache.recurrent[run], q_scale=s.dim ** -0.5, gate=logits, gate_bias=self.decay_bias, tau=s.tau)
         return self.o_proj(gated_out_norm(o, self.out_norm_weight, self.eps, parts=s.heads, gate=rows[:, 2 * qk + v:2 * qk + 2 * v],

@@ -17,7 +17,7 @@ import torch.nn.functional as F
 from ..kernels import fused_moe, smoothquant_matmul, w4a16_matmul, w8a16_matmul
 from ..kernels.quantization import (smoothquant_gate_up_swiglu, smoothquant_matmul_partials, smoothquant_prefill_swiglu,
                                      smoothquant_rows_matmul)
-from ..kernels.quantization import (dense16_linear, dense16_rows_linear, dense16_rows_wins, dense_matmul_partials, pack_w4a16_scales, pack_w4a16_weights, unpack_w4a16_weights, w4a16_matmul_partials,
+from ..kernels.quantization import (dense16_linear, dense16_narrow_linear, dense16_rows_linear, dense16_rows_wins, dense_matmul_partials, pack_w4a16_scales, pack_w4a16_weights, unpack_w4a16_weights, w4a16_matmul_partials,
                                     w4a16_matmul_prepacked_rows, w4a16_mtiled_supported,
                                     w4a16_matmul_prepacked, w4a16_prepacked_supported)
 from .config import FP8, INT4, INT8, SMOOTHQUANT, QuantConfig
@@ -64,6 +64,10 @@ class UnquantizedLinearMethod(LinearQuantMethod):
 
     def apply(self, layer, x):
         m = x.numel() // x.shape[-1] if x.shape[-1] else 0
+        if m <= 64:
+            out = dense16_narrow_linear(x, layer.weight, layer.bias)  # a few rows over a narrow output: one launch, whole sums
+            if out is not None:
+                return out
         if dense16_rows_wins(m, layer.weight.shape[0], layer.weight.shape[1]):  # wide outputs: the row-group loop (round 5)
             out = dense16_rows_linear(x, layer.weight, layer.bias)
             if out is not None:
