@@ -127,83 +127,108 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const void* __restri
     }
 }
 
-// router, second launch: one 64-thread workgroup per token over its logits.  LDS: scores [E], group score [G], group kept
-// [G], chosen scores [top].  SCORING 0: sigmoid scores, weights = chosen / sum; 1: the logits themselves rank the experts (no
-// groups) and the weights are the softmax over the chosen logits alone; 2: scores = softmax over ALL logits (no groups), the
-// experts are ranked by score + correction[e], the weights are the chosen scores themselves (not renormalised); the last
-// `identity` experts have no weights of their own -- a slot that chose one keeps its id (>= experts - identity, which the sort
-// by expert never places) and its score is added to extra_scale[t], the factor of the token's own input row; 3: sigmoid scores
-// as in 0, but the weights are the chosen scores themselves (not renormalised); 4: scores = softmax over ALL logits, a group's score is
-// its largest, weights = chosen / sum
-template <int SCORING, int DT = LL_F32>
-__global__ __launch_bounds__(64) void group_select_kernel(const float* __restrict__ logits, int rows, int experts, int top,
-                                                          int group_count, int group_keep, float route_scale,
-                                                          int32_t* __restrict__ ids, float* __restrict__ weights,
-                                                          float* __restrict__ extra_scale, const void* __restrict__ correction = nullptr,
-                                                          int identity = 0) {
-  extern __shared__ float lds[];
-  float* score = lds;                       // [experts]
-  float* gscore = score + experts;          // [group_count]
-  float* gkeep = gscore + group_count;      // [group_count]
-  float* chosen = gkeep + group_count;      // [top]
-  const int64_t t = blockIdx.x;
-  const int lane = threadIdx.x;
-  if constexpr (SCORING == 2) {
-    // softmax over all experts: every lane adds the exponentials in index order (one value for the whole wave); the ranking
-    // below sees score + correction, the weights the score alone
+// The choice of one token's experts from its logits, by one wave (`lane` of 64; LDS operations of a wave complete in order, so its lanes need no
+// barrier between them).  LDS per token: scores [E], plain scores [E], group score [G], group kept [G], chosen scores [top], chosen
+// experts [top].  SCORING 0: sigmoid scores, weights = chosen / sum; 1: the logits themselves rank the experts (no groups) and the weights are
+// the softmax over the chosen logits alone; 2: scores = softmax over ALL logits (no groups), the experts are ranked by score + correction[e],
+// the weights are the chosen scores themselves (not renormalised); the last `identity` experts have no weights of their own -- a slot that
+// chose one keeps its id (>= experts - identity, which the sort by expert never places) and its score is added to extra_scale[t], the factor
+// of the token's own input row; 3: sigmoid scores as in 0, but the weights are the chosen scores themselves (not renormalised); 4: scores =
+// softmax over ALL logits, a group's score is its largest, weights = chosen / sum
+struct SelectArgs {
+  int rows, experts, top, group_count, group_keep, identity;
+  float route_scale;
+  int32_t* ids;
+  float* weights;
+  float* extra_scale;
+  const void* correction;
+};
+static size_t select_floats(int experts, int group_count, int top) { return (size_t)2 * experts + 2 * group_count + 2 * top; }
+
+__device__ __forceinline__ void select_settle() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
+template <int SCORING, int DT>
+__device__ __forceinline__ void select_token(const SelectArgs& p, const float* z, int64_t t, float* lds, int lane) {
+  const int experts = p.experts, top = p.top;
+  float* score = lds;
+  float* plain = score + experts;
+  float* gscore = plain + experts;
+  float* gkeep = gscore + p.group_count;
+  float* chosen = gkeep + p.group_count;
+  int* chosen_id = reinterpret_cast<int*>(chosen + top);
+  if constexpr (SCORING == 2 || SCORING == 4) {
+    // softmax over all experts: every lane adds the exponentials in index order (one value for the whole wave)
     float top_z = -INFINITY;
-    for (int e = 0; e < experts; ++e) top_z = fmaxf(top_z, logits[t * rows + e]);
+    for (int e = lane; e < experts; e += 64) top_z = fmaxf(top_z, z[e]);
+    top_z = wave_max(top_z);
+    for (int e = lane; e < experts; e += 64) plain[e] = expf(z[e] - top_z);
+    float shift[2] = {0.f, 0.f};   // (the first 128 experts' corrections are requested before they are needed)
+    if (SCORING == 2 && p.correction)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) shift[i] = ldv<DT>(p.correction, lane + 64 * i < experts ? lane + 64 * i : 0);
+    select_settle();
     float total = 0.f;
-    for (int e = 0; e < experts; ++e) total += expf(logits[t * rows + e] - top_z);
-    float* plain = chosen + top;            // [experts] scores without the correction
+#pragma unroll 8
+    for (int e = 0; e < experts; ++e) total += plain[e];   // (eight LDS reads on their way at a time)
+    select_settle();
     for (int e = lane; e < experts; e += 64) {
-      const float sc = expf(logits[t * rows + e] - top_z) / total;
+      const float sc = plain[e] / total;
       plain[e] = sc;
-      score[e] = correction ? sc + ldv<DT>(correction, e) : sc;
+      score[e] = SCORING == 2 && p.correction ? sc + (e < 64 ? shift[0] : e < 128 ? shift[1] : ldv<DT>(p.correction, e)) : sc;
     }
-    __syncthreads();
-    for (int e = lane; e < experts; e += 64) {
-      const float mine = score[e];
-      int rank = 0;
+    if (SCORING == 4 && p.extra_scale)
+      for (int e = experts + lane; e < p.rows; e += 64) p.extra_scale[t] = sigmoid_exact(z[e]);
+  } else {
+    for (int e = lane; e < p.rows; e += 64) {
+      if (e < experts) score[e] = SCORING == 1 ? z[e] : sigmoid_exact(z[e]);
+      else p.extra_scale[t] = sigmoid_exact(z[e]);
+    }
+  }
+  select_settle();
+  if constexpr (SCORING == 2) {
+    auto place = [&](int e, int rank) {
+      if (e < experts && rank < top) {
+        p.ids[t * top + rank] = e;
+        chosen_id[rank] = e;
+        chosen[rank] = plain[e];
+        p.weights[t * top + rank] = plain[e] * p.route_scale;
+      }
+    };
+    int e0 = lane;
+    for (; e0 - lane + 64 < experts; e0 += 128) {   // two experts of a lane at a time
+      const int e1 = e0 + 64;
+      const float mine0 = score[e0], mine1 = score[e1 < experts ? e1 : 0];
+      int rank0 = 0, rank1 = 0;
+#pragma unroll 8
       for (int o = 0; o < experts; ++o) {
         const float sc = score[o];
-        rank += (sc > mine || (sc == mine && o < e)) ? 1 : 0;
+        rank0 += (sc > mine0 || (sc == mine0 && o < e0)) ? 1 : 0;
+        rank1 += (sc > mine1 || (sc == mine1 && o < e1)) ? 1 : 0;
       }
-      if (rank < top) {
-        ids[t * top + rank] = e;
-        chosen[rank] = plain[e];
-        weights[t * top + rank] = plain[e] * route_scale;
-      }
+      place(e0, rank0);
+      place(e1, rank1);
     }
-    __syncthreads();
-    if (extra_scale && lane == 0) {         // slots in rank order: the same sum whatever lane found which slot
+    if (e0 - lane < experts) {
+      const float mine = score[e0 < experts ? e0 : 0];
+      int rank = 0;
+#pragma unroll 8
+      for (int o = 0; o < experts; ++o) {
+        const float sc = score[o];
+        rank += (sc > mine || (sc == mine && o < e0)) ? 1 : 0;
+      }
+      place(e0, rank);
+    }
+    select_settle();
+    if (p.extra_scale) {                      // slots in rank order: the same sum whatever lane found which slot
       float own = 0.f;
-      for (int k = 0; k < top; ++k)
-        if (ids[t * top + k] >= experts - identity) own += chosen[k];
-      extra_scale[t] = own * route_scale;
+#pragma unroll 8
+      for (int k = 0; k < top; ++k) own += chosen_id[k] >= experts - p.identity ? chosen[k] : 0.f;
+      if (lane == 0) p.extra_scale[t] = own * p.route_scale;
     }
     return;
   }
-  for (int e = lane; e < rows; e += 64) {
-    const float z = logits[t * rows + e];
-    if (e < experts) score[e] = (SCORING == 1 || SCORING == 4) ? z : sigmoid_exact(z);
-    else extra_scale[t] = sigmoid_exact(z);
-  }
-  __syncthreads();
-  if constexpr (SCORING == 4) {   // the logits become softmax scores; every lane adds all exponentials in index order
-    float top_z = -INFINITY;
-    for (int e = 0; e < experts; ++e) top_z = fmaxf(top_z, score[e]);
-    __syncthreads();
-    for (int e = lane; e < experts; e += 64) score[e] = expf(score[e] - top_z);
-    __syncthreads();
-    float total = 0.f;
-    for (int e = 0; e < experts; ++e) total += score[e];
-    __syncthreads();
-    for (int e = lane; e < experts; e += 64) score[e] /= total;
-    __syncthreads();
-  }
-  const int per = experts / group_count;
-  for (int g = lane; g < group_count; g += 64) {
+  const int per = experts / p.group_count;
+  for (int g = lane; g < p.group_count; g += 64) {
     float b1 = -INFINITY, b2 = -INFINITY;   // the two largest of the group
     for (int j = 0; j < per; ++j) {
       const float s = score[g * per + j];
@@ -212,40 +237,131 @@ __global__ __launch_bounds__(64) void group_select_kernel(const float* __restric
     }
     gscore[g] = SCORING != 4 && per > 1 ? b1 + b2 : b1;
   }
-  __syncthreads();
-  for (int g = lane; g < group_count; g += 64) {
+  select_settle();
+  for (int g = lane; g < p.group_count; g += 64) {
     const float mine = gscore[g];
     int rank = 0;
-    for (int o = 0; o < group_count; ++o) {
+    for (int o = 0; o < p.group_count; ++o) {
       const float s = gscore[o];
       rank += (s > mine || (s == mine && o < g)) ? 1 : 0;
     }
-    gkeep[g] = rank < group_keep ? 1.0f : 0.0f;
+    gkeep[g] = rank < p.group_keep ? 1.0f : 0.0f;
   }
-  __syncthreads();
+  select_settle();
   for (int e = lane; e < experts; e += 64) {
     if (gkeep[e / per] == 0.0f) continue;
     const float mine = score[e];
     int rank = 0;
+#pragma unroll 8
     for (int o = 0; o < experts; ++o) {
       const float s = score[o];
       rank += (gkeep[o / per] != 0.0f && (s > mine || (s == mine && o < e))) ? 1 : 0;
     }
     if (rank < top) {
-      ids[t * top + rank] = e;
+      p.ids[t * top + rank] = e;
       chosen[rank] = mine;
     }
   }
-  __syncthreads();
+  select_settle();
   float sum = 0.f;
   if constexpr (SCORING == 1) {   // chosen[0] is the largest: exp(z - z_max) summed in slot order by every lane
     for (int k = 0; k < top; ++k) sum += expf(chosen[k] - chosen[0]);
-    for (int k = lane; k < top; k += 64) weights[t * top + k] = expf(chosen[k] - chosen[0]) / sum * route_scale;
+    for (int k = lane; k < top; k += 64) p.weights[t * top + k] = expf(chosen[k] - chosen[0]) / sum * p.route_scale;
   } else if constexpr (SCORING == 3) {
-    for (int k = lane; k < top; k += 64) weights[t * top + k] = chosen[k] * route_scale;
+    for (int k = lane; k < top; k += 64) p.weights[t * top + k] = chosen[k] * p.route_scale;
   } else {
     for (int k = 0; k < top; ++k) sum += chosen[k];
-    for (int k = lane; k < top; k += 64) weights[t * top + k] = chosen[k] / (sum + 1e-20f) * route_scale;
+    for (int k = lane; k < top; k += 64) p.weights[t * top + k] = chosen[k] / (sum + 1e-20f) * p.route_scale;
+  }
+}
+
+// router of many experts, second launch: a wave per token over its logits
+template <int SCORING, int DT>
+__global__ __launch_bounds__(64) void group_select_kernel(const float* __restrict__ logits, const SelectArgs p) {
+  extern __shared__ float lds[];
+  select_token<SCORING, DT>(p, logits + (int64_t)blockIdx.x * p.rows, blockIdx.x, lds, threadIdx.x);
+}
+
+// ------------------------------------------------------------------------------------------------------------------------
+// router in one launch (up to kRouterRows rows of weights): a workgroup of eight waves per TW tokens.  A wave owns an eighth of the rows, five at
+// a time, and sums as the form above does (lanes' pieces in order, then the lanes in a fixed order: the same bits; 16-bit products are
+// exact in fp32, so fused multiply-adds round where product and sum did); the logits meet in LDS and the first TW waves choose.
+// Bound by its launch, one trip for the weights (L2: 140 KB per workgroup) and the chain of the choice.  us, logits and choice in two launches ->
+// here, 34 rows of 2048, top 4: 1 token 12.9 -> 7.6, 262 14.4 -> 9.1, 512 24.5 -> 9.3, 3264
+// 44 -> 23; 68 rows of 3072, top 8: 32 tokens 22.9 -> 12.9, 512 37 -> 21, 3264 85 -> 54 (three pieces of the width at a time on sixteen waves spill: 20).
+// ------------------------------------------------------------------------------------------------------------------------
+constexpr int kRouterRows = 512;
+
+template <int SCORING, int DT, int VEC, int TW, int NW>
+__global__ __launch_bounds__(64 * NW) void router_kernel(const void* __restrict__ h, int64_t h_ld, const void* __restrict__ w_router,
+                                                     const void* __restrict__ w_extra, int width, int64_t n, const SelectArgs p) {
+  constexpr int EW = 5, PU = TW > 1 ? 1 : NW == 8 ? 4 : 2;   // rows of weights and pieces of the width that are requested together
+  extern __shared__ float lds[];                // [TW][rows] logits, then what select_token wants, TW times
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int64_t t0 = (int64_t)blockIdx.x * TW;
+  const int rows = p.rows, share = (rows + NW - 1) / NW, from = wave * share, to = from + share < rows ? from + share : rows;
+  int64_t hat[TW];
+#pragma unroll
+  for (int i = 0; i < TW; ++i) hat[i] = (t0 + i < n ? t0 + i : n - 1) * h_ld;
+  for (int e0 = from; e0 < to; e0 += EW) {
+    const void* wp[EW];
+    int64_t wat[EW];
+#pragma unroll
+    for (int j = 0; j < EW; ++j) {
+      const int e = e0 + j < to ? e0 + j : to - 1;
+      wp[j] = e < p.experts ? w_router : w_extra;
+      wat[j] = e < p.experts ? (int64_t)e * width : 0;
+    }
+    float acc[TW][EW];
+#pragma unroll
+    for (int i = 0; i < TW; ++i)
+#pragma unroll
+      for (int j = 0; j < EW; ++j) acc[i][j] = 0.f;
+    for (int p0 = lane * VEC; p0 < width; p0 += 64 * VEC * PU) {
+      float hv[PU][TW][VEC], wv[PU][EW][VEC];
+#pragma unroll
+      for (int u = 0; u < PU; ++u) {
+        const int at = p0 + u * 64 * VEC;
+        const bool in = at < width;
+#pragma unroll
+        for (int i = 0; i < TW; ++i) {
+          load_piece<DT, VEC>(h, hat[i] + (in ? at : p0), hv[u][i]);
+          if (!in)
+#pragma unroll
+            for (int k = 0; k < VEC; ++k) hv[u][i][k] = 0.f;
+        }
+#pragma unroll
+        for (int j = 0; j < EW; ++j) {
+          load_piece<DT, VEC>(wp[j], wat[j] + (in ? at : p0), wv[u][j]);
+          if (!in)
+#pragma unroll
+            for (int k = 0; k < VEC; ++k) wv[u][j][k] = 0.f;
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < PU; ++u)
+#pragma unroll
+        for (int j = 0; j < EW; ++j)
+#pragma unroll
+          for (int i = 0; i < TW; ++i)
+#pragma unroll
+            for (int k = 0; k < VEC; ++k) {
+              if constexpr (DT == LL_F32) acc[i][j] += hv[u][i][k] * wv[u][j][k];
+              else acc[i][j] = __builtin_fmaf(hv[u][i][k], wv[u][j][k], acc[i][j]);
+            }
+    }
+#pragma unroll
+    for (int i = 0; i < TW; ++i)
+#pragma unroll
+      for (int j = 0; j < EW; ++j) {
+        const float v = wave_sum(acc[i][j]);
+        if (lane == 0 && e0 + j < to) lds[i * rows + e0 + j] = v;
+      }
+  }
+  __syncthreads();
+  if (wave < TW && t0 + wave < n) {
+    const int64_t each = (int64_t)2 * p.experts + 2 * p.group_count + 2 * p.top;
+    select_token<SCORING, DT>(p, lds + wave * rows, t0 + wave, lds + TW * rows + wave * each, lane);
   }
 }
 
@@ -643,9 +759,30 @@ extern "C" int ll_group_router(const void* h, int64_t h_ld, const void* w_router
   const int rows = (int)experts + (w_extra ? 1 : 0);
   const int vec = dtype == LL_F32 ? 4 : 8;
   const bool aligned = width % vec == 0 && h_ld % vec == 0 && ll_aligned16(h) && ll_aligned16(w_router) && (!w_extra || ll_aligned16(w_extra));
+  hipStream_t st = (hipStream_t)stream;
+  const SelectArgs p{rows, (int)experts, (int)top, (int)group_count, (int)group_keep, (int)identity, route_scale, ids, weights, extra_scale, correction};
+  const size_t each = select_floats((int)experts, (int)group_count, (int)top);
+  if (rows <= kRouterRows) {
+    const int tw = n > 256 ? 4 : 1, nw = tw == 1 && rows > 40 ? 16 : 8;   // tokens per workgroup; waves
+    const dim3 grid((unsigned)((n + tw - 1) / tw));
+    const size_t lds = sizeof(float) * tw * (rows + each);
+#define LL_R(S, DT, V, T, W) router_kernel<S, DT, V, T, W><<<grid, 64 * W, lds, st>>>(h, h_ld, w_router, w_extra, (int)width, n, p)
+#define LL_RT(S, DT, V) do { if (tw == 4) LL_R(S, DT, V, 4, 8); else if (nw == 16) LL_R(S, DT, V, 1, 16); else LL_R(S, DT, V, 1, 8); } while (0)
+#define LL_RV(S, DT, V) do { if (aligned) LL_RT(S, DT, V); else LL_RT(S, DT, 1); } while (0)
+#define LL_RS(DT, V)                                                                                                                  \
+  do {                                                                                                                                \
+    if (scoring == 0) LL_RV(0, DT, V); else if (scoring == 1) LL_RV(1, DT, V); else if (scoring == 2) LL_RV(2, DT, V);                \
+    else if (scoring == 3) LL_RV(3, DT, V); else LL_RV(4, DT, V);                                                                     \
+  } while (0)
+    if (dtype == LL_F32) LL_RS(LL_F32, 4); else if (dtype == LL_F16) LL_RS(LL_F16, 8); else LL_RS(LL_BF16, 8);
+#undef LL_RS
+#undef LL_RV
+#undef LL_RT
+#undef LL_R
+    return LL_LAUNCH_CHECK();
+  }
   const int ew = n >= 512 ? 8 : 2;   // weight rows per wave
   const dim3 grid((unsigned)((n + 7) / 8), (unsigned)((rows + 4 * ew - 1) / (4 * ew)));
-  hipStream_t st = (hipStream_t)stream;
 #define LL_RL_ARGS h, h_ld, w_router, w_extra, (int)width, (int)experts, rows, logits, n
 #define LL_RL(DT, V)                                                                         \
   if (ew == 8) router_logits_kernel<DT, V, 8><<<grid, 256, 0, st>>>(LL_RL_ARGS);             \
@@ -663,25 +800,17 @@ extern "C" int ll_group_router(const void* h, int64_t h_ld, const void* w_router
   }
 #undef LL_RL
 #undef LL_RL_ARGS
-  const size_t lds = sizeof(float) * (size_t)(experts + 2 * group_count + top + (scoring == 2 ? experts : 0));
+  const size_t lds = sizeof(float) * each;
+#define LL_GS(S, DT) group_select_kernel<S, DT><<<dim3((unsigned)n), 64, lds, st>>>(logits, p)
   if (scoring == 2) {
-#define CALL(DT)                                                                                                                    \
-  group_select_kernel<2, DT><<<dim3((unsigned)n), 64, lds, st>>>(logits, rows, (int)experts, (int)top, 1, 1, route_scale, ids, weights, \
-                                                                 extra_scale, correction, (int)identity)
+#define CALL(DT) LL_GS(2, DT)
     LL_BY_DTYPE(dtype, CALL);
 #undef CALL
-  } else if (scoring == 1)
-    group_select_kernel<1><<<dim3((unsigned)n), 64, lds, st>>>(logits, rows, (int)experts, (int)top, (int)group_count, (int)group_keep,
-                                                               route_scale, ids, weights, extra_scale);
-  else if (scoring == 4)
-    group_select_kernel<4><<<dim3((unsigned)n), 64, lds, st>>>(logits, rows, (int)experts, (int)top, (int)group_count, (int)group_keep,
-                                                               route_scale, ids, weights, extra_scale);
-  else if (scoring == 3)
-    group_select_kernel<3><<<dim3((unsigned)n), 64, lds, st>>>(logits, rows, (int)experts, (int)top, (int)group_count, (int)group_keep,
-                                                               route_scale, ids, weights, extra_scale);
-  else
-    group_select_kernel<0><<<dim3((unsigned)n), 64, lds, st>>>(logits, rows, (int)experts, (int)top, (int)group_count, (int)group_keep,
-                                                               route_scale, ids, weights, extra_scale);
+  } else if (scoring == 1) LL_GS(1, LL_F32);
+  else if (scoring == 4) LL_GS(4, LL_F32);
+  else if (scoring == 3) LL_GS(3, LL_F32);
+  else LL_GS(0, LL_F32);
+#undef LL_GS
   return LL_LAUNCH_CHECK();
 }
 

@@ -1,0 +1,48 @@
+"""The router in one launch and the two-launch form of many experts (csrc/moe_sparse.hip) against 64-bit scores: one token and one past a workgroup's
+tokens, experts off the waves' shares and past one and two per lane, widths off the pieces, every scoring."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV, F64 = "cuda", torch.float64
+
+
+@pytest.mark.parametrize("n,width,experts", [(1, 40, 5), (3, 2048, 34), (256, 136, 40), (257, 72, 41), (33, 3080, 65), (9, 100, 130), (600, 264, 68),
+                                             (5, 520, 511), (7, 520, 513)])
+@pytest.mark.parametrize("scoring", ["sigmoid", "softmax_chosen", "softmax_all", "sigmoid_plain", "softmax_groups"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_choice(n, width, experts, scoring, dtype):
+    from lite_llama_amd.kernels.fused_moe import group_router
+
+    g = torch.Generator(device=DEV).manual_seed(n + width + experts)
+    top, route_scale, identity = min(4, experts), 1.5, 1
+    h = torch.randn(n, width, generator=g, device=DEV).to(dtype)
+    w = (torch.randn(experts, width, generator=g, device=DEV) * 2 * width ** -0.5).to(dtype)
+    z = h.to(F64) @ w.to(F64).T
+    kw, extra = {"scoring": scoring}, None
+    if scoring == "softmax_all":
+        kw.update(correction=(torch.randn(experts, generator=g, device=DEV) * 0.02).to(dtype), identity=identity)
+    else:
+        extra = torch.randn(width, generator=g, device=DEV).to(dtype) * width ** -0.5
+        kw.update(extra_weight=extra)
+    ids, weights, own = group_router(h, w, top, route_scale=route_scale, **kw)
+    score = z if scoring == "softmax_chosen" else torch.sigmoid(z) if scoring.startswith("sigmoid") else torch.softmax(z, -1)
+    rank = score + kw["correction"].to(F64) if scoring == "softmax_all" else score
+    best, want = rank.topk(min(top + 1, experts), -1)
+    # logits are fp32 sums of up to 3080 products of unit deviation (about 1e-6 off); a softmax's scores are off by that share of
+    # themselves, the correction's sum by an fp32 unit: scores closer than ten times as much may change places
+    close = 1e-5 * (best[:, :1].abs() if scoring.startswith("softmax_") and scoring != "softmax_chosen" else 1.0) + 1e-7
+    clear = (best[:, :-1] - best[:, 1:] > close).all(-1)
+    assert clear.float().mean() > 0.8
+    want = want[:, :top]
+    assert torch.equal(ids[clear].long(), want[clear])
+    chosen = score.gather(1, want)
+    weight = {"sigmoid": chosen / chosen.sum(-1, keepdim=True), "softmax_chosen": torch.softmax(chosen, -1), "softmax_all": chosen,
+              "sigmoid_plain": chosen, "softmax_groups": chosen / chosen.sum(-1, keepdim=True)}[scoring] * route_scale
+    assert (weights[clear].to(F64) - weight[clear]).abs().max() <= 2e-5
+    if extra is not None:
+        assert (own.to(F64) - torch.sigmoid(h.to(F64) @ extra.to(F64))).abs().max() <= 2e-5
+    else:
+        mine = torch.where(want >= experts - identity, chosen, torch.zeros_like(chosen)).sum(-1) * route_scale
+        assert (own[clear].to(F64) - mine[clear]).abs().max() <= 2e-5
