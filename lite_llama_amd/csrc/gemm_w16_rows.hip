@@ -2,20 +2,20 @@
 // a dequantiser.  Reference: lite_llama/models/quantization/methods/unquantized.py:21-22 and the lm_head of models/base.py:486-489
 // are torch's library GEMM; BASELINE config 2 (Qwen2.5-1.5B bf16, batch 32) has its fused gate|up and the lm_head there.
 //   * A workgroup owns a contiguous run of 32-row groups (N / 32 groups dealt over the CUs, sizes differing by at most one) and ALL
-//     of K; it walks its run in tiles of up to 4 groups.  Finished outputs only: no split-K planes, no finish launch, bias or the
-//     fused swiglu of a row-interleaved gate|up in the epilogue (the decode engines' epilogue, common.h::ll_silu_mul_f32).
-//   * 8 waves: four LOADERS stream, per 128-k chunk, the tile's 4 x [32 rows x 256 B] weight blocks and the [M x 256 B] activation
-//     block into an R-slot LDS ring by LDS-DMA -- row-major with the 16-byte slots of row r at slot ^ (r & 15), swizzled through the
-//     per-lane SOURCE address (the activation image of the int4 engines, now for both operands): fragment reads are conflict free;
-//     weights non-temporal.  Four CONSUMERS, one per row group of the tile, run the chunk's 8 x MT MFMA 32x32x16 from LDS
-//     fragments and keep the tile's accumulators (16 x MT registers) for the whole K loop: no cross-wave exchange.  The loaders
-//     run ahead ACROSS tile boundaries, so a tile's epilogue overlaps the next tile's first chunks.
-//   * Long streams: workgroup b begins every tile at chunk b mod (K / 128) and wraps.  All of them beginning at column 0 ask the same few
-//     memory channels where a row is a power of two long (us for 600 MB, 1 row, all from column 0 -> staggered: K = 2048 113 -> 94,
-//     4096 127 -> 98, 8192 139 -> 124; 3584 90 -> 91.  Staggered within an XCD instead, b / 8: 98, 106, 124).  Sums of 16-bit products in
+//     of K; it walks its run in tiles of up to 4 groups (WIDE: 8), of equal size to within one.  Finished outputs only: no
+//     split-K planes, no finish launch, bias or the fused swiglu of a row-interleaved gate|up in the epilogue (the decode engines'
+//     epilogue, common.h::ll_silu_mul_f32).
+//   * Four LOADERS stream, per unit of 256 (128) bytes of every row, the tile's weight blocks -- 32 KB -- and the activation block into a ring of
+//     LDS slots by LDS-DMA: row-major with the 16-byte slots of a row permuted by R16Lds::swizzle, through the per-lane SOURCE
+//     address: fragment reads are conflict free; weights non-temporal.  CONSUMERS, one per row group of the tile, run the unit's MFMA
+//     32x32x16 from LDS fragments and keep the tile's accumulators (16 x MT registers) for the whole K loop: no cross-wave exchange.
+//     The loaders run ahead ACROSS tile boundaries, so a tile's epilogue overlaps the next tile's first units.
+//   * Long streams of rows a multiple of 4 KB long: workgroup b begins every tile at unit b mod units and wraps.  All of them beginning at
+//     column 0 ask the same few memory channels (us for 600 MB, 1 row, all from column 0 -> staggered: K = 2048 113 -> 94, 4096 127 -> 98,
+//     8192 139 -> 124; staggered within an XCD instead, b / 8: 98, 106, 124.  K = 3584: 90 -> 91, 37888 rows of it 50 -> 52).  Sums of 16-bit products in
 //     another order round otherwise, so streams under 256 MB, which gain little or nothing (32 rows, K = 2048: 134 MB 31 -> 28 us, 46 MB
 //     13.9 -> 14.9), keep the ascending one; int8 sums are exact, and staggered from 64 MB.
-//   * one s_barrier per chunk; the loaders' operation count per chunk is static (8 + 2 MT pieces each).
+//   * one s_barrier per unit; the loaders' operation count per unit is static.
 #include <stdlib.h>
 
 #include "common.h"
@@ -23,15 +23,21 @@
 
 typedef __bf16 r16_bf16x8 __attribute__((ext_vector_type(8)));
 
-#define R16_THREADS 512
-template <int MT>
+// WIDE (more than 32 rows over more than four row groups per CU): tiles of eight groups in units of 128 bytes, so that a fifth of what a CU fetches
+// is activations, as with 32 rows, and not a third; 96 KB of weights on their way and not 64.  us, 64 rows, 16-bit: 128256 x 4096 184 -> 167, 152064 x
+// 3584 199 -> 192, 37888 x 3584 54 -> 46; int8 128256 x 4096 97 -> 89.  Where the groups are few a tile is not full: 11264 x 2048 15.1 -> 22.3.
+template <int MT, bool WIDE>
 struct R16Lds {
-  static constexpr int W_BYTES = 4 * 8192;        // four row groups x [32 rows][256 B]
-  static constexpr int X_BYTES = MT * 8192;       // [32 MT rows][256 B]
-  static constexpr int SLOT = W_BYTES + X_BYTES;  // 40 KB (M <= 32) / 48 KB
-  static constexpr int R = MT == 1 ? 4 : 3;
+  static constexpr int GROUPS = WIDE ? 8 : 4;     // row groups of a tile, a consumer each
+  static constexpr int THREADS = 64 * (GROUPS + 4);
+  static constexpr int KB = WIDE ? 128 : 256;     // bytes of a row per unit
+  static constexpr int W_BYTES = GROUPS * 32 * KB;
+  static constexpr int X_BYTES = 32 * MT * KB;
+  static constexpr int SLOT = W_BYTES + X_BYTES;  // 40 KB; 48 KB (more than 32 rows, four groups)
+  static constexpr int R = 160 * 1024 / SLOT;     // 4; 3
   static constexpr int BYTES = R * SLOT;
-  static_assert(BYTES <= 160 * 1024, "LDS");
+  // which 16-byte slot of its row a piece stands in: slot ^ swizzle(row), so that the lanes of a fragment read meet all banks
+  static __device__ __forceinline__ int swizzle(int row) { return WIDE ? (row >> 1) & 7 : row & 15; }
 };
 
 struct R16Params {
@@ -40,7 +46,7 @@ struct R16Params {
   const uint16_t* w;
   const uint16_t* bias;
   int64_t m, n, k, x_stride, w_stride;
-  int chunks;        // K / 128
+  int chunks;        // units of a row: its bytes / R16Lds::KB
   int rbase, rrem;   // workgroup b owns row groups [b * rbase + min(b, rrem), + rbase + (b < rrem))
   int stagger;       // workgroups begin a tile at different chunks
   int epi;           // 0: out[m, n] (+ bias);  1: rows are (gate_j, up_j) pairs -> out[m, n / 2] = silu(gate) * up
@@ -56,58 +62,65 @@ __device__ __forceinline__ void r16_wait_units(int k) {  // at most k units of N
   else v3_vmcnt<2 * N>();
 }
 
-template <int MT, int DT>
-__global__ __launch_bounds__(R16_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void wgemm16_rows_kernel(const R16Params p) {
+template <int MT, int DT, bool WIDE>
+__global__ __launch_bounds__((R16Lds<MT, WIDE>::THREADS)) __attribute__((amdgpu_waves_per_eu(WIDE ? 3 : 2, WIDE ? 3 : 2))) void wgemm16_rows_kernel(const R16Params p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  using LD = R16Lds<MT>;
-  constexpr int R = LD::R;
-  constexpr int XP = 2 * MT;   // activation pieces (4 rows x 256 B) per loader wave
-  constexpr int OPS = 8 + XP;  // LDS-DMA operations per loader wave and chunk
+  using LD = R16Lds<MT, WIDE>;
+  constexpr int R = LD::R, KB = LD::KB, GROUPS = LD::GROUPS;
+  constexpr int PER = 1024 / KB, SLOTS = KB / 16;   // rows of an LDS-DMA operation; 16-byte slots of a row
+  constexpr int GL = GROUPS / 4;                    // row groups of a loader wave
+  constexpr int XP = LD::X_BYTES / 4096;  // activation operations per loader wave and unit
+  constexpr int OPS = 8 + XP;  // LDS-DMA operations per loader wave and unit
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int b = (int)blockIdx.x;
   const int lo = b * p.rbase + (b < p.rrem ? b : p.rrem);
   const int cnt = p.rbase + (b < p.rrem ? 1 : 0);
   if (cnt <= 0) return;
-  const int hi = lo + cnt;
-  const int tiles = (cnt + 3) >> 2;
+  // (tiles of equal size to within one: a last tile of a group or two would walk the whole contraction with little on its way)
+  const int tiles = (cnt + GROUPS - 1) / GROUPS, tbase = cnt / tiles, trem = cnt - tbase * tiles;
   const int units = tiles * p.chunks;
 
-  if (wv >= 4) {
+  if (wv >= GROUPS) {
     // ======================================== loaders ======================================== //
-    const int L = wv - 4;  // weight block of row group L of every tile + activation pieces XP * L ..
+    const int L = wv - GROUPS;  // weight rows [L * 32 GL, + 32 GL) of every tile + activation operations XP * L ..
     uint32_t woff[8], xoff[XP];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const int r = j * 4 + (lane >> 4), slot = (lane & 15) ^ (r & 15);
+      const int r = j * PER + lane / SLOTS, slot = (lane % SLOTS) ^ LD::swizzle(r & 31);
       woff[j] = (uint32_t)((int64_t)r * p.w_stride * 2 + slot * 16);
     }
 #pragma unroll
     for (int j = 0; j < XP; ++j) {
-      int64_t r = (XP * L + j) * 4 + (lane >> 4);
-      const int slot = (lane & 15) ^ (int)(r & 15);
+      int64_t r = (XP * L + j) * PER + lane / SLOTS;
+      const int slot = (lane % SLOTS) ^ LD::swizzle((int)(r & 31));
       if (r >= p.m) r = p.m - 1;  // rows >= M feed only unstored outputs
       xoff[j] = (uint32_t)(r * p.x_stride * 2 + slot * 16);
     }
-    int issued = 0, t = 0, done = 0, c = p.stagger ? b % p.chunks : 0;
+    int issued = 0, t = 0, size = tbase + (trem > 0 ? 1 : 0), done = 0, c = 0;
+    if (p.stagger)
+      for (c = b; c >= p.chunks; c -= p.chunks) {}
+    const char* wt = (const char*)p.w + (size_t)(lo + L * GL) * 32 * (size_t)p.w_stride * 2;   // this wave's rows of the tile
     uint32_t dst = 0;
     auto issue = [&]() {
-      const int rg = lo + 4 * t + L;
-      // a short last tile: the idle loader keeps its eight operations (the counted waits stay static) but points them at ONE
-      // cached KB (the first of the matrix) -- no weight bytes are fetched twice; its LDS block is never read
-      const bool live = rg < hi;
-      const char* wb = live ? (const char*)p.w + (size_t)rg * 32 * (size_t)p.w_stride * 2 + (size_t)c * 256 : (const char*)p.w;
-      const char* xb = (const char*)p.x + (size_t)c * 256;
+      const char* wb = wt + (size_t)c * KB;
+      const char* xb = (const char*)p.x + (size_t)c * KB;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        if (live) v3_dma16<true>(dst + L * 8192 + j * 1024, wb, woff[j]);
-        else v3_dma16<false>(dst + L * 8192 + j * 1024, wb, (uint32_t)(lane * 16));
+        // a short tile: an idle loader keeps its operations (the counted waits stay static) but points them at ONE cached KB (the first of
+        // the matrix) -- no weight bytes are fetched twice; its LDS block is never read
+        if (L * GL + j * GL / 8 < size) v3_dma16<true>(dst + L * 8192 + j * 1024, wb, woff[j]);
+        else v3_dma16<false>(dst + L * 8192 + j * 1024, (const char*)p.w, (uint32_t)(lane * 16));
       }
 #pragma unroll
       for (int j = 0; j < XP; ++j) v3_dma16<false>(dst + LD::W_BYTES + (XP * L + j) * 1024, xb, xoff[j]);
       ++issued;
       if (++c == p.chunks) c = 0;
-      if (++done == p.chunks) { done = 0; ++t; }
+      if (++done == p.chunks) {
+        done = 0;
+        wt += (size_t)size * 32 * (size_t)p.w_stride * 2;
+        size = tbase + (++t < trem ? 1 : 0);
+      }
       dst = dst + LD::SLOT == R * LD::SLOT ? 0 : dst + LD::SLOT;
     };
     const int pre = units < R - 1 ? units : R - 1;
@@ -125,7 +138,7 @@ __global__ __launch_bounds__(R16_THREADS) __attribute__((amdgpu_waves_per_eu(2, 
 
   // ======================================= consumers ======================================= //
   const int nl = lane & 31, h = lane >> 5;
-  const int wrow = wv * 8192 + nl * 256;  // this wave's row group of the tile, weight row nl
+  const int wrow = (wv * 32 + nl) * KB;  // this wave's row group of the tile, weight row nl
   constexpr int ODT = DT == R16_I8 ? LL_F16 : DT;  // output / bias storage type
   f32x16 acc[MT];
   i32x16 iacc[MT];
@@ -139,22 +152,22 @@ __global__ __launch_bounds__(R16_THREADS) __attribute__((amdgpu_waves_per_eu(2, 
     bb = r[1];
   };
   const bool has_bias = p.bias != nullptr;
-  int t = 0, c = 0;
+  int t = 0, first = lo, size = tbase + (trem > 0 ? 1 : 0), c = 0;
   uint32_t slot = 0;
   asm volatile("s_barrier" ::: "memory");  // P0: unit 0 has landed
   for (int u = 0; u < units; ++u) {
-    const int rg = lo + 4 * t + wv;
-    const bool mine = rg < hi;
+    const int rg = first + wv;
+    const bool mine = wv < size;
     if (mine) {
       const unsigned char* wb = lds + slot + wrow;
-      const unsigned char* xb = lds + slot + LD::W_BYTES + nl * 256;
+      const unsigned char* xb = lds + slot + LD::W_BYTES + nl * KB;
 #pragma unroll
-      for (int s = 0; s < 8; ++s) {
-        const int off = ((2 * s + h) ^ (nl & 15)) * 16;
+      for (int s = 0; s < KB / 32; ++s) {
+        const int off = ((2 * s + h) ^ LD::swizzle(nl)) * 16;
         const u32x4 wf = *reinterpret_cast<const u32x4*>(wb + off);
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-          const u32x4 xf = *reinterpret_cast<const u32x4*>(xb + mt * 8192 + off);
+          const u32x4 xf = *reinterpret_cast<const u32x4*>(xb + mt * 32 * KB + off);
           if constexpr (DT == LL_F16)
             acc[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, wf), __builtin_bit_cast(f16x8, xf), acc[mt], 0, 0, 0);
           else if constexpr (DT == LL_BF16)
@@ -239,7 +252,8 @@ __global__ __launch_bounds__(R16_THREADS) __attribute__((amdgpu_waves_per_eu(2, 
           for (int e = 0; e < 16; ++e) { acc[mt][e] = 0.f; iacc[mt][e] = 0; }
         }
       }
-      ++t;
+      first += size;
+      size = tbase + (++t < trem ? 1 : 0);
     }
   }
 }
@@ -255,7 +269,7 @@ static int r16_num_cus() {
   return cus[dev];
 }
 
-// the row-group loop needs R16Lds<MT>::BYTES of LDS per workgroup (160 KB at MT = 1): callers fall back when the device's opt-in
+// the row-group loop needs R16Lds::BYTES of LDS per workgroup (160 KB at MT = 1): callers fall back when the device's opt-in
 // limit is smaller
 static bool r16_lds_fits(int64_t m) {
   static int optin[16] = {0};
@@ -265,7 +279,7 @@ static bool r16_lds_fits(int64_t m) {
     int v = 0;
     optin[dev] = hipDeviceGetAttribute(&v, hipDeviceAttributeSharedMemPerBlockOptin, dev) == hipSuccess && v > 0 ? v : 160 * 1024;
   }
-  return (m <= 32 ? R16Lds<1>::BYTES : R16Lds<2>::BYTES) <= optin[dev];
+  return (m <= 32 ? R16Lds<1, false>::BYTES : R16Lds<2, true>::BYTES) <= optin[dev];   // (the larger of the two for m > 32)
 }
 
 extern "C" int ll_dense16_rows_supported(int64_t m, int64_t n, int64_t k, int epilogue) {
@@ -287,29 +301,32 @@ extern "C" int ll_dense16_rows_matmul(void* out, const void* x, const void* w, c
   R16Params p{};
   p.out = (uint16_t*)out; p.x = (const uint16_t*)x; p.w = (const uint16_t*)w; p.bias = (const uint16_t*)bias;
   p.m = m; p.n = n; p.k = k; p.x_stride = x_stride_m; p.w_stride = w_stride_n;
-  p.chunks = (int)(k / 128);
-  p.stagger = n * k * 2 >= (1ll << 28);
+  p.stagger = n * k * 2 >= (1ll << 28) && w_stride_n % 2048 == 0;
   p.epi = epilogue;
   const int64_t rgs = n / 32;
   int grid = r16_num_cus();
   if (grid > rgs) grid = (int)rgs;
   p.rbase = (int)(rgs / grid); p.rrem = (int)(rgs % grid);
+  const bool wide = m > 32 && rgs > 4 * (int64_t)grid;
+  p.chunks = (int)(k * 2 / (wide ? 128 : 256));
   hipStream_t st = (hipStream_t)stream;
-#define R16_GO(MT, DT)                                                                                                   \
+#define R16_GO(MT, DT, WIDE)                                                                                                   \
   {                                                                                                                      \
     static bool attr_[16] = {false}; /* per device */                                                   \
     int dev_ = 0;                                                                                                        \
     (void)hipGetDevice(&dev_);                                                                                           \
     if (dev_ >= 0 && dev_ < 16 && !attr_[dev_]) {                                                                        \
-      (void)hipFuncSetAttribute((const void*)wgemm16_rows_kernel<MT, DT>, hipFuncAttributeMaxDynamicSharedMemorySize, R16Lds<MT>::BYTES); \
+      (void)hipFuncSetAttribute((const void*)wgemm16_rows_kernel<MT, DT, WIDE>, hipFuncAttributeMaxDynamicSharedMemorySize, R16Lds<MT, WIDE>::BYTES); \
       attr_[dev_] = true;                                                                                                \
     }                                                                                                                    \
-    wgemm16_rows_kernel<MT, DT><<<dim3((unsigned)grid), R16_THREADS, R16Lds<MT>::BYTES, st>>>(p);                          \
+    wgemm16_rows_kernel<MT, DT, WIDE><<<dim3((unsigned)grid), R16Lds<MT, WIDE>::THREADS, R16Lds<MT, WIDE>::BYTES, st>>>(p);                          \
   }
   if (m <= 32) {
-    if (dtype == LL_F16) R16_GO(1, LL_F16) else R16_GO(1, LL_BF16)
+    if (dtype == LL_F16) R16_GO(1, LL_F16, false) else R16_GO(1, LL_BF16, false)
+  } else if (wide) {
+    if (dtype == LL_F16) R16_GO(2, LL_F16, true) else R16_GO(2, LL_BF16, true)
   } else {
-    if (dtype == LL_F16) R16_GO(2, LL_F16) else R16_GO(2, LL_BF16)
+    if (dtype == LL_F16) R16_GO(2, LL_F16, false) else R16_GO(2, LL_BF16, false)
   }
 #undef R16_GO
   return LL_LAUNCH_CHECK();
@@ -338,26 +355,27 @@ extern "C" int ll_w8a8_rows_matmul(void* out, const int8_t* qa, const float* a_s
   p.a_scale = a_scale; p.w_scale = w_scale;
   p.m = m; p.n = n; p.k = k;
   p.x_stride = qa_stride_m / 2; p.w_stride = qw_stride_n / 2;  // the kernel addresses rows in 2-byte units
-  p.chunks = (int)(k / 256);                                    // 256 bytes of a row per chunk
-  p.stagger = n * k >= (1ll << 26);
+  p.stagger = n * k >= (1ll << 26) && qw_stride_n % 4096 == 0;
   p.epi = epilogue;
   const int64_t rgs = n / 32;
   int grid = r16_num_cus();
   if (grid > rgs) grid = (int)rgs;
   p.rbase = (int)(rgs / grid); p.rrem = (int)(rgs % grid);
+  const bool wide = m > 32 && rgs > 4 * (int64_t)grid;
+  p.chunks = (int)(k / (wide ? 128 : 256));
   hipStream_t st = (hipStream_t)stream;
-#define R16_GO8(MT)                                                                                                      \
+#define R16_GO8(MT, WIDE)                                                                                                      \
   {                                                                                                                      \
     static bool attr_[16] = {false}; /* per device */                                                   \
     int dev_ = 0;                                                                                                        \
     (void)hipGetDevice(&dev_);                                                                                           \
     if (dev_ >= 0 && dev_ < 16 && !attr_[dev_]) {                                                                        \
-      (void)hipFuncSetAttribute((const void*)wgemm16_rows_kernel<MT, R16_I8>, hipFuncAttributeMaxDynamicSharedMemorySize, R16Lds<MT>::BYTES); \
+      (void)hipFuncSetAttribute((const void*)wgemm16_rows_kernel<MT, R16_I8, WIDE>, hipFuncAttributeMaxDynamicSharedMemorySize, R16Lds<MT, WIDE>::BYTES); \
       attr_[dev_] = true;                                                                                                \
     }                                                                                                                    \
-    wgemm16_rows_kernel<MT, R16_I8><<<dim3((unsigned)grid), R16_THREADS, R16Lds<MT>::BYTES, st>>>(p);                      \
+    wgemm16_rows_kernel<MT, R16_I8, WIDE><<<dim3((unsigned)grid), R16Lds<MT, WIDE>::THREADS, R16Lds<MT, WIDE>::BYTES, st>>>(p);                      \
   }
-  if (m <= 32) R16_GO8(1) else R16_GO8(2)
+  if (m <= 32) R16_GO8(1, false) else if (wide) R16_GO8(2, true) else R16_GO8(2, false)
 #undef R16_GO8
   return LL_LAUNCH_CHECK();
 }

@@ -34,3 +34,32 @@ def test_staggered_int8_rows():
     out = smoothquant_rows_matmul(x, w, scale)
     head = smoothquant_rows_matmul(x, w[:8192], scale[:8192])   # (32 MB: not staggered; sums of whole numbers have one value)
     assert torch.equal(out[:, :8192], head)
+
+
+# more than four row groups per CU: tiles of eight for more than 32 rows; runs of 4 and 5, 8 and 9, 17 groups; one unit of the contraction
+@pytest.mark.parametrize("n", [32 * 1025, 32 * 2049, 32 * 4352])
+@pytest.mark.parametrize("k", [128, 512])
+@pytest.mark.parametrize("m", [32, 33, 64])
+@pytest.mark.parametrize("swiglu", [False, True])
+def test_row_group_runs(n, k, m, swiglu):
+    from lite_llama_amd.kernels.quantization import dense16_rows_linear, quantize_activations_int8, smoothquant_rows_matmul
+
+    g = torch.Generator(device=DEV).manual_seed(n + k)
+    w = (torch.randn(n, k, generator=g, device=DEV) * k ** -0.5).half()
+    x = torch.randn(m, k, generator=g, device=DEV).half()
+    want = x.float() @ w.float().T
+    got = dense16_rows_linear(x, w, gate_up_swiglu=swiglu)
+    if swiglu:
+        gate, up = want[:, 0::2].half().float(), want[:, 1::2].half().float()
+        want = torch.nn.functional.silu(gate) * up
+        # gate and up are rounded to fp16 first: a unit of each, times the other (and |silu'| <= 1.1)
+        bar = 2.0 ** -9 * (want.abs() + gate.abs() + up.abs() + 2.0 ** -4)
+    else:
+        bar = 2.0 ** -11 * want.abs() + 2.0 ** -14
+    assert ((got.float() - want).abs() <= bar).all()
+    if not swiglu and k % 256 == 0:
+        codes = torch.randint(-127, 128, (n, k), generator=g, device=DEV, dtype=torch.int8)
+        scale = torch.rand(n, generator=g, device=DEV) * 1e-3
+        qa, a = quantize_activations_int8(x)
+        sums = qa.float() @ codes.float().T                 # (whole numbers below 2^24: exact)
+        assert torch.equal(smoothquant_rows_matmul(x, codes, scale), ((sums * a.view(-1, 1)) * scale.view(1, -1)).half())
