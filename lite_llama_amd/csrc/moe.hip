@@ -780,7 +780,7 @@ extern "C" int ll_moe_gemm(void* c, const void* a, const void* w, const float* w
     t.a_ld = a_stride_m; t.out_ld = mul_routed_weight & 2 ? n / 2 : n; t.w_stride_e = w_stride_e * eb; t.w_stride_n = w_stride_n * eb;
     t.s_stride_e = s_stride_e; t.s_stride_n = s_stride_n; t.s_stride_k = s_stride_k; t.group_n = group_n; t.group_k = group_k;
     t.K = (int)k; t.N = (int)n; t.num_slots = (int)num_slots; t.a_div = top_k; t.block_m = block_m; t.safe = (int)em;
-    if (em < (1ll << 31) && moe_stream_wants(t, form, mode, LL_F16, experts)) return moe_stream_launch(t, form, mode, LL_F16, (hipStream_t)stream);
+    if (em < (1ll << 31) && moe_stream_wants(t, form, mode, LL_F16, experts)) return moe_stream_launch(t, form, mode, LL_F16, experts, (hipStream_t)stream);
   }
   MoeParams p{};
   p.c = (uint16_t*)c; p.a = (const uint16_t*)a; p.w = w; p.w_scale = w_scale; p.topk_w = (const uint16_t*)topk_w;

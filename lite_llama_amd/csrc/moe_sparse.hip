@@ -884,7 +884,7 @@ extern "C" int ll_moe_rows_gemm(const void* a, int64_t a_ld, int64_t a_div, cons
       t.a_ld = a_ld; t.out_ld = out_ld; t.w_stride_e = w_stride_e * 2; t.w_stride_n = K * 2; t.K = (int)K; t.N = (int)N;
       t.num_slots = (int)num_slots; t.a_div = (int)a_div; t.block_m = (int)block; t.limit = glu_limit;
       t.safe = (int)(num_slots + experts * (block - 1));
-      if (moe_stream_wants(t, MS_W16, form, dtype, experts)) return moe_stream_launch(t, MS_W16, form, dtype, st);
+      if (moe_stream_wants(t, MS_W16, form, dtype, experts)) return moe_stream_launch(t, MS_W16, form, dtype, experts, st);
     }
     const int64_t tiles_n = (N + (mode == 1 ? 63 : 127)) / (mode == 1 ? 64 : 128), max_tiles = most * tiles_n;
     if (max_tiles > 0x7ffffff0ll) return LL_ERR_SHAPE;

@@ -32,4 +32,4 @@ struct MoeStreamParams {
 
 // whether the streaming form takes this call
 bool moe_stream_wants(const MoeStreamParams& p, int wfmt, int mode, int dtype, int64_t experts);
-int moe_stream_launch(const MoeStreamParams& p, int wfmt, int mode, int dtype, hipStream_t stream);
+int moe_stream_launch(const MoeStreamParams& p, int wfmt, int mode, int dtype, int64_t experts, hipStream_t stream);

@@ -16,7 +16,8 @@
 //     workgroup per CU, 117 with two; 16-bit weights gain nothing by it).  Ring depths of 4 to 6 units are alike.
 //   us for both products, tiles -> here.  8-bit floats, 128 experts of 2048 / 768, top 8: 1 token 42 -> 24, 8 67 -> 54, 32 120 -> 102, 64
 //   137 -> 117 (604 MB: 5.2 TB/s).  bf16, 34 of 2048 / 704, top 4: 1 token 33 -> 17, 32 tokens 77 -> 58, 128 78 -> 65; 68 of 3072 / 512,
-//   top 8: 6 tokens 89 -> 74, 32 156 -> 111 (642 MB), 128 160 -> 126, 262 (31 rows per expert) 165 -> 185: the rule of moe_stream_wants.
+//   top 8: 6 tokens 89 -> 74, 32 156 -> 111 (642 MB), 128 160 -> 126; in pieces of 64 rows 160 tokens 161 -> 131, 262 (31 rows per expert) 165 ->
+//   150 (pieces of 32: 185), 34 experts 200 77 -> 73, 300 (35) 78.5 -> 77, 400 (47) 80 -> 85: the rule of moe_stream_wants.
 #include <stdlib.h>
 
 #include "gemm_w4_common.h"
@@ -29,11 +30,11 @@ typedef __bf16 ms_bf16x8 __attribute__((ext_vector_type(8)));
 constexpr int MS_LIST = 512, MS_OWN = 8;   // row blocks in all / of one workgroup
 constexpr int MS_W_BYTES = 64 * 256;
 
-template <int WF>
+template <int WF, int MT_>
 struct MsLds {
   static constexpr int THREADS = 512;                          // four consumers, four loaders
   static constexpr int PER_CU = WF == MS_W16 ? 1 : 2, RING = WF == MS_W16 ? 4 : 3;
-  static constexpr int MT = WF == MS_W16 ? 2 : 1, ROWS = 16 * MT;   // rows of a piece of a block
+  static constexpr int MT = MT_, ROWS = 16 * MT;               // rows of a piece of a block
   static constexpr int KU = WF == MS_W16 ? 128 : 256;          // contraction entries of a unit
   static constexpr int X_BYTES = ROWS * KU * 2;
   static constexpr int S_BYTES = WF == MS_W16 ? 0 : 64 * 4 * 4;   // scales: [loader][64-column step][16 rows]
@@ -45,7 +46,7 @@ struct MsLds {
   static constexpr int COUNTS = WEIGHTS + MS_OWN * ROWS * 4;   // int32 [8], [1]
   static constexpr int BYTES = COUNTS + 48;                    // (nothing static: the ring begins at LDS byte 0)
   static_assert(BYTES * PER_CU <= 160 * 1024, "LDS");
-  static_assert(X_BYTES == 8192, "two activation pieces per loader and unit");
+  static constexpr int XOPS = X_BYTES / 4096;                  // activation operations per loader and unit
 };
 
 __device__ const uint32_t ms_zeros[4] __attribute__((aligned(16))) = {0, 0, 0, 0};   // what pieces without an entry read
@@ -108,9 +109,9 @@ __device__ __forceinline__ float ms_glu(float g, float u, float limit) {
   return g * ll_sigmoidf(g) * u;
 }
 
-template <int WF, int MODE, int XOPS>
+template <int WF, int MT, int MODE, int XOPS>
 __device__ __forceinline__ void ms_load(const MoeStreamParams& p, unsigned char* lds, int L, int lane, int lo, int hi, int rgs, int i0, int units, int total) {
-  using LD = MsLds<WF>;
+  using LD = MsLds<WF, MT>;
   constexpr int KU = LD::KU, EB = WF == MS_W16 ? 2 : 1, ROWS = LD::ROWS;
   constexpr int OPS = 4 + XOPS + (WF == MS_W16 ? 0 : 1);
   const int32_t* experts = reinterpret_cast<const int32_t*>(lds + LD::OWN);
@@ -208,11 +209,11 @@ __device__ __forceinline__ void ms_load(const MoeStreamParams& p, unsigned char*
   }
 }
 
-template <int DT, int WF, int MODE>
-__global__ __launch_bounds__(MsLds<WF>::THREADS) __attribute__((amdgpu_waves_per_eu(2 * MsLds<WF>::PER_CU, 2 * MsLds<WF>::PER_CU))) void moe_stream_kernel(const MoeStreamParams p) {
+template <int DT, int WF, int MT, int MODE>
+__global__ __launch_bounds__((MsLds<WF, MT>::THREADS)) __attribute__((amdgpu_waves_per_eu(2 * (MsLds<WF, MT>::PER_CU), 2 * (MsLds<WF, MT>::PER_CU)))) void moe_stream_kernel(const MoeStreamParams p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  using LD = MsLds<WF>;
-  constexpr int KU = LD::KU, MT = LD::MT, ROWS = LD::ROWS, THREADS = LD::THREADS;
+  using LD = MsLds<WF, MT>;
+  constexpr int KU = LD::KU, ROWS = LD::ROWS, THREADS = LD::THREADS;
   constexpr bool PAIRS = MODE == MS_GLU || MODE == MS_GLU_ROUNDED;
   uint32_t* list = reinterpret_cast<uint32_t*>(lds + LD::LIST);
   int32_t* rows = reinterpret_cast<int32_t*>(lds + LD::SLOTS);
@@ -296,8 +297,8 @@ __global__ __launch_bounds__(MsLds<WF>::THREADS) __attribute__((amdgpu_waves_per
   const int full = __builtin_amdgcn_readfirstlane(*most_rows);
 
   if (wv >= 4) {
-    if (full > ROWS / 2) ms_load<WF, MODE, 2>(p, lds, wv - 4, lane, lo, hi, rgs, i0, units, total);
-    else ms_load<WF, MODE, 1>(p, lds, wv - 4, lane, lo, hi, rgs, i0, units, total);
+    if (full > ROWS / 2) ms_load<WF, MT, MODE, LD::XOPS>(p, lds, wv - 4, lane, lo, hi, rgs, i0, units, total);
+    else ms_load<WF, MT, MODE, LD::XOPS / 2>(p, lds, wv - 4, lane, lo, hi, rgs, i0, units, total);
     return;
   }
 
@@ -329,23 +330,20 @@ __global__ __launch_bounds__(MsLds<WF>::THREADS) __attribute__((amdgpu_waves_per
         const unsigned char* xb = lds + slot_at + MS_W_BYTES + r * (KU * 2);
         // (all fragments of the unit are requested before the first is used: one wave per matrix core waits for LDS once)
         if constexpr (WF == MS_W16) {
-          u32x4 wf[4], x0[4], x1[4];
+          u32x4 wf[4], x[MT][4];
 #pragma unroll
-          for (int s = 0; s < 4; ++s) {
-            const int at = ((4 * s + q) ^ r) * 16;
-            wf[s] = *reinterpret_cast<const u32x4*>(wb + at);
-            x0[s] = *reinterpret_cast<const u32x4*>(xb + at);
-          }
-          if (full > 16) {
+          for (int s = 0; s < 4; ++s) wf[s] = *reinterpret_cast<const u32x4*>(wb + ((4 * s + q) ^ r) * 16);
 #pragma unroll
-            for (int s = 0; s < 4; ++s) x1[s] = *reinterpret_cast<const u32x4*>(xb + 16 * KU * 2 + ((4 * s + q) ^ r) * 16);
-            __builtin_amdgcn_sched_barrier(0);
+          for (int m = 0; m < MT; ++m)
+            if (m == 0 || 16 * m < full)
 #pragma unroll
-            for (int s = 0; s < 4; ++s) acc[1] = ms_mfma<DT>(wf[s], x1[s], acc[1]);
-          } else
-            __builtin_amdgcn_sched_barrier(0);
+              for (int s = 0; s < 4; ++s) x[m][s] = *reinterpret_cast<const u32x4*>(xb + 16 * m * KU * 2 + ((4 * s + q) ^ r) * 16);
+          __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-          for (int s = 0; s < 4; ++s) acc[0] = ms_mfma<DT>(wf[s], x0[s], acc[0]);
+          for (int m = 0; m < MT; ++m)
+            if (m == 0 || 16 * m < full)
+#pragma unroll
+              for (int s = 0; s < 4; ++s) acc[m] = ms_mfma<DT>(wf[s], x[m][s], acc[m]);
         } else {
           // a lane's 16 weights of a 64-column step feed two products; the activations' columns are taken in the same order.  The step's
           // sums are multiplied by the scales of their weight rows: a weight enters exactly.
@@ -445,19 +443,22 @@ int ms_cus(int* lds) {
   return cus[dev];
 }
 
-int ms_lds(int wfmt) { return wfmt == MS_W16 ? MsLds<MS_W16>::BYTES : MsLds<MS_FP8>::BYTES; }
+int ms_lds(int wfmt, int rows) { return wfmt != MS_W16 ? MsLds<MS_FP8, 1>::BYTES : rows == 64 ? MsLds<MS_W16, 4>::BYTES : MsLds<MS_W16, 2>::BYTES; }
 
-template <int DT, int WF, int MODE>
+// rows of a piece: 16 with 8-bit weights, 32 with 16-bit ones, 64 where 16 and more meet an expert on average
+int ms_rows(const MoeStreamParams& p, int wfmt, int64_t experts) { return wfmt != MS_W16 ? 16 : p.num_slots > 16 * experts ? 64 : 32; }
+
+template <int DT, int WF, int MT, int MODE>
 int ms_go(const MoeStreamParams& p, int grid, hipStream_t stream) {
-  constexpr int bytes = MsLds<WF>::BYTES;
+  constexpr int bytes = MsLds<WF, MT>::BYTES;
   static bool attr[16] = {false};
   int dev = 0;
   (void)hipGetDevice(&dev);
   if (dev >= 0 && dev < 16 && !attr[dev]) {
-    (void)hipFuncSetAttribute((const void*)moe_stream_kernel<DT, WF, MODE>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    (void)hipFuncSetAttribute((const void*)moe_stream_kernel<DT, WF, MT, MODE>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     attr[dev] = true;
   }
-  moe_stream_kernel<DT, WF, MODE><<<dim3((unsigned)grid * MsLds<WF>::PER_CU), MsLds<WF>::THREADS, bytes, stream>>>(p);
+  moe_stream_kernel<DT, WF, MT, MODE><<<dim3((unsigned)grid * MsLds<WF, MT>::PER_CU), MsLds<WF, MT>::THREADS, bytes, stream>>>(p);
   return LL_LAUNCH_CHECK();
 }
 
@@ -466,7 +467,7 @@ int ms_go(const MoeStreamParams& p, int grid, hipStream_t stream) {
 bool moe_stream_wants(const MoeStreamParams& p, int wfmt, int mode, int dtype, int64_t experts) {
   static const bool off = getenv("LL_MOE_NO_STREAM") != nullptr;   // A/B knob, read once
   if (off || (dtype != LL_F16 && (dtype != LL_BF16 || wfmt != MS_W16)) || experts > 65535) return false;
-  const int eb = wfmt == MS_W16 ? 2 : 1, rows = wfmt == MS_W16 ? 32 : 16;
+  const int eb = wfmt == MS_W16 ? 2 : 1, rows = ms_rows(p, wfmt, experts);
   if (p.block_m % rows || p.K < 128 || (int64_t)p.K * eb % 16 || p.K > (1 << 24) || p.N < 16 || p.N > (1 << 24) || p.a_ld % 8 ||
       p.w_stride_n % 16 || p.w_stride_e % 16 || !ll_aligned16(p.a) || !ll_aligned16(p.w) || (mode == MS_GLU_ROUNDED && p.N % 2))
     return false;
@@ -477,17 +478,17 @@ bool moe_stream_wants(const MoeStreamParams& p, int wfmt, int mode, int dtype, i
         ((int64_t)p.N * p.s_stride_n + p.K / 64 * p.s_stride_k) * 4 >= (1ll << 32))
       return false;
   }
-  // few rows per expert (figures above): pieces of 32 rows, of 16 with 8-bit weights, whose rows beyond the first piece stream the weights again
-  if (p.num_slots > (wfmt == MS_W16 ? 16 : 12) * experts) return false;
+  // few rows per expert (figures above): pieces of 32 or 64 rows, of 16 with 8-bit weights; an expert's rows beyond its first piece stream the weights again
+  if (p.num_slots > (wfmt == MS_W16 ? 36 : 12) * experts) return false;
   int lds = 0;
   const int cus = ms_cus(&lds);
   const int64_t most = ((int64_t)p.num_slots + (experts + 1) * (p.block_m - 1)) / rows + 1;
   const int64_t filled = p.num_slots / rows + experts + 1;   // pieces with a slot
-  return cus > 0 && filled <= MS_LIST && filled / cus + 2 <= MS_OWN && most <= 65535 && ms_lds(wfmt) <= lds &&
+  return cus > 0 && filled <= MS_LIST && filled / cus + 2 <= MS_OWN && most <= 65535 && ms_lds(wfmt, rows) <= lds &&
          (filled + 1) * (((int64_t)p.N + 7) / 8) < (1ll << 30);
 }
 
-int moe_stream_launch(const MoeStreamParams& asked, int wfmt, int mode, int dtype, hipStream_t stream) {
+int moe_stream_launch(const MoeStreamParams& asked, int wfmt, int mode, int dtype, int64_t experts, hipStream_t stream) {
   MoeStreamParams p = asked;
   p.group_n = p.group_n < p.N ? p.group_n : p.N;
   p.k_shift = 31;
@@ -495,9 +496,10 @@ int moe_stream_launch(const MoeStreamParams& asked, int wfmt, int mode, int dtyp
     for (p.k_shift = 6; (1ll << p.k_shift) < p.group_k; ++p.k_shift) {}
   int lds = 0;
   const int cus = ms_cus(&lds);
-  if (wfmt == MS_FP8) return mode == MS_GLU_ROUNDED ? ms_go<LL_F16, MS_FP8, MS_GLU_ROUNDED>(p, cus, stream) : ms_go<LL_F16, MS_FP8, MS_SCALED>(p, cus, stream);
-  if (wfmt == MS_INT8) return mode == MS_GLU_ROUNDED ? ms_go<LL_F16, MS_INT8, MS_GLU_ROUNDED>(p, cus, stream) : ms_go<LL_F16, MS_INT8, MS_SCALED>(p, cus, stream);
-#define MS_W(DT, MODE) return ms_go<DT, MS_W16, MODE>(p, cus, stream)
+  if (wfmt == MS_FP8) return mode == MS_GLU_ROUNDED ? ms_go<LL_F16, MS_FP8, 1, MS_GLU_ROUNDED>(p, cus, stream) : ms_go<LL_F16, MS_FP8, 1, MS_SCALED>(p, cus, stream);
+  if (wfmt == MS_INT8) return mode == MS_GLU_ROUNDED ? ms_go<LL_F16, MS_INT8, 1, MS_GLU_ROUNDED>(p, cus, stream) : ms_go<LL_F16, MS_INT8, 1, MS_SCALED>(p, cus, stream);
+  const bool deep = ms_rows(p, wfmt, experts) == 64;
+#define MS_W(DT, MODE) return deep ? ms_go<DT, MS_W16, 4, MODE>(p, cus, stream) : ms_go<DT, MS_W16, 2, MODE>(p, cus, stream)
   if (dtype == LL_F16) {
     if (mode == MS_SCALED) MS_W(LL_F16, MS_SCALED);
     if (mode == MS_RELU2) MS_W(LL_F16, MS_RELU2);

@@ -20,7 +20,7 @@ def _ids(tokens, experts, top, g, hot):
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("width,ff,experts,tokens,top", [(128, 16, 5, 1, 1), (136, 200, 9, 40, 2), (264, 128, 40, 33, 4), (2048, 704, 34, 32, 4),
-                                                         (392, 1000, 300, 64, 8), (640, 136, 3, 20, 2)])
+                                                         (392, 1000, 300, 64, 8), (640, 136, 3, 20, 2), (264, 128, 3, 40, 2), (1032, 72, 5, 85, 2)])
 @pytest.mark.parametrize("form", ["silu", "clamped", "square"])
 def test_16_bit_experts(dtype, width, ff, experts, tokens, top, form):
     from lite_llama_amd.kernels.fused_moe import sparse_glu_experts, sparse_square_experts
