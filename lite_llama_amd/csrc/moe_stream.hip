@@ -15,7 +15,7 @@
 //     workgroup per CU fills those gaps (128 experts of 2048 / 768 in 8-bit floats, 64 tokens with 8 each, both products: 128 us with one
 //     workgroup per CU, 117 with two; 16-bit weights gain nothing by it).  Ring depths of 4 to 6 units are alike.
 //   us for both products, tiles -> here.  8-bit floats, 128 experts of 2048 / 768, top 8: 1 token 42 -> 24, 8 67 -> 54, 32 120 -> 102, 64
-//   137 -> 117 (604 MB: 5.2 TB/s).  bf16, 34 of 2048 / 704, top 4: 1 token 33 -> 17, 32 tokens 77 -> 58, 128 78 -> 65; 68 of 3072 / 512,
+//   137 -> 117 (604 MB: 5.2 TB/s); in pieces of 32 rows (of 16) 200 167 -> 155 (167), 256 178 -> 162 (209), 320 181 -> 168, 400 186 -> 191.  bf16, 34 of 2048 / 704, top 4: 1 token 33 -> 17, 32 tokens 77 -> 58, 128 78 -> 65; 68 of 3072 / 512,
 //   top 8: 6 tokens 89 -> 74, 32 156 -> 111 (642 MB), 128 160 -> 126; in pieces of 64 rows 160 tokens 161 -> 131, 262 (31 rows per expert) 165 ->
 //   150 (pieces of 32: 185), 34 experts 200 77 -> 73, 300 (35) 78.5 -> 77, 400 (47) 80 -> 85: the rule of moe_stream_wants.
 #include <stdlib.h>
@@ -33,7 +33,7 @@ constexpr int MS_W_BYTES = 64 * 256;
 template <int WF, int MT_>
 struct MsLds {
   static constexpr int THREADS = 512;                          // four consumers, four loaders
-  static constexpr int PER_CU = WF == MS_W16 ? 1 : 2, RING = WF == MS_W16 ? 4 : 3;
+  static constexpr int PER_CU = WF != MS_W16 && MT_ == 1 ? 2 : 1, RING = PER_CU == 2 ? 3 : 4;
   static constexpr int MT = MT_, ROWS = 16 * MT;               // rows of a piece of a block
   static constexpr int KU = WF == MS_W16 ? 128 : 256;          // contraction entries of a unit
   static constexpr int X_BYTES = ROWS * KU * 2;
@@ -348,25 +348,41 @@ __global__ __launch_bounds__((MsLds<WF, MT>::THREADS)) __attribute__((amdgpu_wav
           // a lane's 16 weights of a 64-column step feed two products; the activations' columns are taken in the same order.  The step's
           // sums are multiplied by the scales of their weight rows: a weight enters exactly.
           const float* sb = reinterpret_cast<const float*>(lds + slot_at + MS_W_BYTES + LD::X_BYTES) + wv * 64 + 4 * q;
-          u32x4 raw[4], x0[4], x1[4];
+          u32x4 raw[4], x0[MT][4], x1[MT][4];
           f32x4 sv[4], step[4];
 #pragma unroll
           for (int t = 0; t < 4; ++t) {
             raw[t] = *reinterpret_cast<const u32x4*>(wb + ((4 * t + q) ^ r) * 16);
-            x0[t] = *reinterpret_cast<const u32x4*>(xb + ((8 * t + 2 * q) ^ r) * 16);
-            x1[t] = *reinterpret_cast<const u32x4*>(xb + ((8 * t + 2 * q + 1) ^ r) * 16);
             sv[t] = *reinterpret_cast<const f32x4*>(sb + t * 16);
           }
+#pragma unroll
+          for (int m = 0; m < MT; ++m)
+            if (m == 0 || 16 * m < full)
+#pragma unroll
+              for (int t = 0; t < 4; ++t) {
+                x0[m][t] = *reinterpret_cast<const u32x4*>(xb + 16 * m * KU * 2 + ((8 * t + 2 * q) ^ r) * 16);
+                x1[m][t] = *reinterpret_cast<const u32x4*>(xb + 16 * m * KU * 2 + ((8 * t + 2 * q + 1) ^ r) * 16);
+              }
           __builtin_amdgcn_sched_barrier(0);
+          u32x4 w0[4], w1[4];
 #pragma unroll
           for (int t = 0; t < 4; ++t) {
-            step[t] = ms_mfma<LL_F16>(ms_widen<WF>(raw[t].x, raw[t].y), x0[t], f32x4{0.f, 0.f, 0.f, 0.f});
-            step[t] = ms_mfma<LL_F16>(ms_widen<WF>(raw[t].z, raw[t].w), x1[t], step[t]);
+            w0[t] = ms_widen<WF>(raw[t].x, raw[t].y);
+            w1[t] = ms_widen<WF>(raw[t].z, raw[t].w);
           }
 #pragma unroll
-          for (int t = 0; t < 4; ++t)
+          for (int m = 0; m < MT; ++m)
+            if (m == 0 || 16 * m < full) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) acc[0][i] = __builtin_fmaf(step[t][i], sv[t][i], acc[0][i]);
+              for (int t = 0; t < 4; ++t) {
+                step[t] = ms_mfma<LL_F16>(w0[t], x0[m][t], f32x4{0.f, 0.f, 0.f, 0.f});
+                step[t] = ms_mfma<LL_F16>(w1[t], x1[m][t], step[t]);
+              }
+#pragma unroll
+              for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[m][i] = __builtin_fmaf(step[t][i], sv[t][i], acc[m][i]);
+            }
         }
       }
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // B_u: this unit's slot may be refilled
@@ -375,7 +391,9 @@ __global__ __launch_bounds__((MsLds<WF, MT>::THREADS)) __attribute__((amdgpu_wav
     if (mine) {
       if constexpr (WF == MS_FP8) {
 #pragma unroll
-        for (int t = 0; t < 4; ++t) acc[0][t] *= 256.0f;   // (exact: what ms_widen left out)
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+          for (int t = 0; t < 4; ++t) acc[m][t] *= 256.0f;   // (exact: what ms_widen left out)
       }
       // a lane holds weight rows 4 q .. 4 q + 3 of the group for row r (+ 16 m)
 #pragma unroll
@@ -443,10 +461,10 @@ int ms_cus(int* lds) {
   return cus[dev];
 }
 
-int ms_lds(int wfmt, int rows) { return wfmt != MS_W16 ? MsLds<MS_FP8, 1>::BYTES : rows == 64 ? MsLds<MS_W16, 4>::BYTES : MsLds<MS_W16, 2>::BYTES; }
+int ms_lds(int wfmt, int rows) { return wfmt != MS_W16 ? (rows == 32 ? MsLds<MS_FP8, 2>::BYTES : MsLds<MS_FP8, 1>::BYTES) : rows == 64 ? MsLds<MS_W16, 4>::BYTES : MsLds<MS_W16, 2>::BYTES; }
 
-// rows of a piece: 16 with 8-bit weights, 32 with 16-bit ones, 64 where 16 and more meet an expert on average
-int ms_rows(const MoeStreamParams& p, int wfmt, int64_t experts) { return wfmt != MS_W16 ? 16 : p.num_slots > 16 * experts ? 64 : 32; }
+// rows of a piece: with 8-bit weights 16, or 32 where 8 and more meet an expert on average; with 16-bit ones 32, or 64 from 16 on
+int ms_rows(const MoeStreamParams& p, int wfmt, int64_t experts) { return wfmt != MS_W16 ? (p.num_slots > 8 * experts && p.block_m % 32 == 0 ? 32 : 16) : p.num_slots > 16 * experts ? 64 : 32; }
 
 template <int DT, int WF, int MT, int MODE>
 int ms_go(const MoeStreamParams& p, int grid, hipStream_t stream) {
@@ -478,8 +496,8 @@ bool moe_stream_wants(const MoeStreamParams& p, int wfmt, int mode, int dtype, i
         ((int64_t)p.N * p.s_stride_n + p.K / 64 * p.s_stride_k) * 4 >= (1ll << 32))
       return false;
   }
-  // few rows per expert (figures above): pieces of 32 or 64 rows, of 16 with 8-bit weights; an expert's rows beyond its first piece stream the weights again
-  if (p.num_slots > (wfmt == MS_W16 ? 36 : 12) * experts) return false;
+  // few rows per expert (figures above): pieces of 32 or 64 rows, of 16 or 32 with 8-bit weights; an expert's rows beyond its first piece stream the weights again
+  if (p.num_slots > (wfmt == MS_W16 ? 36 : rows == 32 ? 16 : 12) * experts) return false;
   int lds = 0;
   const int cus = ms_cus(&lds);
   const int64_t most = ((int64_t)p.num_slots + (experts + 1) * (p.block_m - 1)) / rows + 1;
@@ -496,8 +514,16 @@ int moe_stream_launch(const MoeStreamParams& asked, int wfmt, int mode, int dtyp
     for (p.k_shift = 6; (1ll << p.k_shift) < p.group_k; ++p.k_shift) {}
   int lds = 0;
   const int cus = ms_cus(&lds);
-  if (wfmt == MS_FP8) return mode == MS_GLU_ROUNDED ? ms_go<LL_F16, MS_FP8, 1, MS_GLU_ROUNDED>(p, cus, stream) : ms_go<LL_F16, MS_FP8, 1, MS_SCALED>(p, cus, stream);
-  if (wfmt == MS_INT8) return mode == MS_GLU_ROUNDED ? ms_go<LL_F16, MS_INT8, 1, MS_GLU_ROUNDED>(p, cus, stream) : ms_go<LL_F16, MS_INT8, 1, MS_SCALED>(p, cus, stream);
+#define MS_8(WF, MODE) return ms_rows(p, wfmt, experts) == 32 ? ms_go<LL_F16, WF, 2, MODE>(p, cus, stream) : ms_go<LL_F16, WF, 1, MODE>(p, cus, stream)
+  if (wfmt == MS_FP8) {
+    if (mode == MS_GLU_ROUNDED) MS_8(MS_FP8, MS_GLU_ROUNDED);
+    MS_8(MS_FP8, MS_SCALED);
+  }
+  if (wfmt == MS_INT8) {
+    if (mode == MS_GLU_ROUNDED) MS_8(MS_INT8, MS_GLU_ROUNDED);
+    MS_8(MS_INT8, MS_SCALED);
+  }
+#undef MS_8
   const bool deep = ms_rows(p, wfmt, experts) == 64;
 #define MS_W(DT, MODE) return deep ? ms_go<DT, MS_W16, 4, MODE>(p, cus, stream) : ms_go<DT, MS_W16, 2, MODE>(p, cus, stream)
   if (dtype == LL_F16) {

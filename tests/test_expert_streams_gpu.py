@@ -64,7 +64,8 @@ def test_16_bit_experts(dtype, width, ff, experts, tokens, top, form):
 
 @pytest.mark.parametrize("fmt", ["fp8", "int8"])
 @pytest.mark.parametrize("width,ff,experts,tokens,top,group", [(128, 128, 4, 1, 2, 128), (144, 160, 6, 9, 2, 64), (384, 272, 30, 17, 3, 128),
-                                                               (2048, 768, 128, 64, 8, 128), (512, 256, 20, 100, 2, 4096)])
+                                                               (2048, 768, 128, 64, 8, 128), (512, 256, 20, 100, 2, 4096),
+                                                               (400, 144, 8, 60, 2, 4096), (256, 272, 9, 130, 1, 64)])
 @pytest.mark.parametrize("interleaved", [False, True])
 def test_8_bit_experts(fmt, width, ff, experts, tokens, top, group, interleaved):
     from lite_llama_amd.kernels.fused_moe import fused_moe
