@@ -219,61 +219,115 @@ __global__ __launch_bounds__(256) void linear_scan_kernel(const ScanArgs a) {
 // runs of many tokens: the walk above, with the same bits, in two kernels.  Token by token it is three fp32 operations per state entry; what
 // it spent its time on was everything around them -- per 16 columns of a head the rows were loaded, activated and written to LDS again,
 // eight 16-byte records were read for 24 operations, and every 16 tokens waited for their rows from memory.
-//   scan_terms_kernel    per token, once: (key, query) pairs behind activation and scale, decays per key entry, (decay, step size) pairs
+//   scan_terms_kernel    per token, once: (key, query) pairs and values behind activation and scale, decays per key entry, (decay, step size)
 //   linear_walk_kernel   a workgroup per (sequence, head, 16 CV columns): thread (kg, piece) owns CV neighbouring columns of the state rows kg,
 //                        kg + 16, ...; eight tokens at a time come to LDS by DMA under the walk over the eight in front of them, a token's
-//                        records are read under the products of the one in front of it, and the partial read-outs of eight tokens are
-//                        added at once (row groups in order, as in the walk above): only the walk's own instructions stand between its tokens
-// us, before -> both kernels, 8 runs of 256 - 512 tokens | one of 1024: per entry, 8 heads of 128 x 256: 536 -> 182 | 417 -> 196; fixed, 16 of
-// 128 x 128: 439 -> 153 | 340 -> 166; per token, 32 of 128 x 64: 443 -> 147 | 344 -> 164 (the terms take 10 - 21 of each).  The longest run's
-// own operations need 70 (two columns per thread).  Sums over chunks of 16 tokens as matrix products took 95 | 130, but round in another order.
+//                        numbers are read in pieces of 16 bytes under the products of the one in front of it, and the partial read-outs of
+//                        eight tokens are added at once (row groups in order, as in the walk above)
+// Per stage of eight tokens the walk asks for one or two barriers and a handful of scalar additions beside its tokens: values too come behind
+// their activation and by DMA, addresses advance by constants, a stage's sums are added up under the next one.  us of both kernels, values
+// activated in the walk and pairs read in eight bytes -> now, 8 runs of 256 - 512 tokens | one of 1024: per entry, 8 heads of 128 x 256:
+// 171 -> 129 | 192 -> 131; fixed, 16 of 128 x 128: 143 -> 117 | 162 -> 127; per token, 32 of 128 x 64: 134 -> 117 | 157 -> 138 (the terms take
+// 9 - 25 of each).  The longest run's own operations need 41 (one column per thread, one wave per SIMD: what is left is the latency of its
+// reads); many runs are bound by those operations and the reads from LDS together.  Keys, queries and decays taken from another lane of 16
+// on the way (row_newbcast: one LDS read of four bytes instead of six of sixteen) came to 130 - 143 | 147 - 186: such an operand halves the rate.
+// Sums over chunks of 16 tokens as matrix products take fewer operations, but round in another order.
 // ------------------------------------------------------------------------------------------------------------------------
-constexpr int kTB = 8;   // tokens per stage of the walk
+constexpr int kTB = 8;          // tokens per stage of the walk
+constexpr int kTermPieces = 1;  // pieces of 16 bytes per thread of scan_terms_kernel
 
+// A token's terms: columns of its (key, query) pairs, then of its decays (kind 1), then of its values (heads of dvp columns, zeros behind dv),
+// then its (decay, step size) pairs (kind 2).  Rows of a head are kept in the order the walk reads them in: rows 16 r + kg of two r (decays:
+// four) lie side by side for every kg, so that a row group's numbers come in pieces of 16 bytes and the pieces of all groups are neighbours.
 template <int DT>
 __global__ __launch_bounds__(256) void scan_terms_kernel(const ScanArgs a, float2* __restrict__ kq, float* __restrict__ decay,
-                                                         float2* __restrict__ td, int64_t n, int64_t total) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= total) return;
-  const int heads = a.heads, qk_heads = heads / a.qk_rep, dk = a.dk;
-  const int cols = (a.kind == 1 ? heads : qk_heads) * dk;
-  const int64_t row = i / cols;
-  const int c = (int)(i - row * cols);
-  if (a.kind == 1)
-    decay[i] = entry_decay(ldv<DT>(a.gate, row * a.gate_ld + c) + ldv<DT>(a.gate_bias, c), a.inv_tau);
-  if (row < n && c < qk_heads * dk) {
-    float qv = ldv<DT>(a.q, row * a.q_ld + c), kv = ldv<DT>(a.k, row * a.k_ld + c);
-    if (a.act) {
-      qv *= act_sigmoid<DT>(qv);
-      kv *= act_sigmoid<DT>(kv);
+                                                         float2* __restrict__ td, float* __restrict__ values, int dvp) {
+  const int64_t row = blockIdx.x;
+  const int heads = a.heads, dk = a.dk, dv = a.dv;
+  const int pairs = heads / a.qk_rep * dk, decays = a.kind == 1 ? heads * dk : 0, vals = heads * dvp, steps = a.kind == 2 ? heads : 0;
+#pragma unroll
+  for (int j = 0; j < kTermPieces; ++j) {   // pieces of 16 bytes
+    int c = ((int)blockIdx.y * kTermPieces + j) * 256 + (int)threadIdx.x;
+    if (c < pairs / 2) {
+      const int at = (c & ~15) * 2 + (c & 15);
+      float qv[2], kv[2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        qv[e] = ldv<DT>(a.q, row * a.q_ld + at + 16 * e);
+        kv[e] = ldv<DT>(a.k, row * a.k_ld + at + 16 * e);
+      }
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        if (a.act) {
+          qv[e] *= act_sigmoid<DT>(qv[e]);
+          kv[e] *= act_sigmoid<DT>(kv[e]);
+        }
+        qv[e] *= a.q_scale;
+      }
+      *reinterpret_cast<f32x4*>(kq + row * pairs + 2 * c) = f32x4{kv[0], qv[0], kv[1], qv[1]};
+      continue;
     }
-    kq[row * qk_heads * dk + c] = float2{kv, qv * a.q_scale};
-  }
-  if (a.kind == 2 && i < n * heads) {
-    const int64_t t = i / heads;
-    const int h = (int)(i - t * heads);
-    const float step = softplus(ldv<DT>(a.dt, t * a.dt_ld + h) + ldv<DT>(a.dt_bias, h));
-    td[i] = float2{expf(-expf(ldv<DT>(a.a_log, h)) * step), step};
+    c -= pairs / 2;
+    if (c < decays / 4) {
+      const int at = (c & ~15) * 4 + (c & 15);
+      f32x4 d;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) d[e] = ldv<DT>(a.gate, row * a.gate_ld + at + 16 * e) + ldv<DT>(a.gate_bias, at + 16 * e);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) d[e] = entry_decay(d[e], a.inv_tau);
+      *reinterpret_cast<f32x4*>(decay + row * decays + 4 * c) = d;
+      continue;
+    }
+    c -= decays / 4;
+    if (c < vals / 4) {
+      const int h = 4 * c / dvp, cc = 4 * c - h * dvp;
+      f32x4 x;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = cc + e < dv ? ldv<DT>(a.v, row * a.v_ld + (int64_t)h * dv + cc + e) : 0.f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (a.act) x[e] *= act_sigmoid<DT>(x[e]);
+      *reinterpret_cast<f32x4*>(values + row * vals + 4 * c) = x;
+      continue;
+    }
+    c -= vals / 4;
+    if (c < steps) {
+      const float step = softplus(ldv<DT>(a.dt, row * a.dt_ld + c) + ldv<DT>(a.dt_bias, c));
+      td[row * heads + c] = float2{expf(-expf(ldv<DT>(a.a_log, c)) * step), step};
+    }
   }
 }
 
-// 64 lanes x 16 bytes from per-lane addresses to 1 KB of LDS at byte `dst` (counted by vmcnt, which the compiler does not see)
-__device__ __forceinline__ void dma16(uint32_t dst, const void* src) {
-  dst = __builtin_amdgcn_readfirstlane(dst);
+// 64 lanes x 16 (4) bytes from base + per-lane offsets to 1 KB (256 bytes) of LDS at byte `dst` (counted by vmcnt, which the compiler does not see)
+__device__ __forceinline__ void dma16(uint32_t dst, const void* base, uint32_t off) {
   uint32_t keep;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\ts_mov_b32 m0, %0"
-               : "=&s"(keep) : "s"(dst), "v"(src) : "memory");
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep) : "s"(dst), "v"(off), "s"(base) : "memory");
+}
+__device__ __forceinline__ void dma4(uint32_t dst, const void* base, uint32_t off) {
+  uint32_t keep;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %2, %3\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep) : "s"(dst), "v"(off), "s"(base) : "memory");
 }
 
-// dk == 16 RMAX.  dt: the values' storage dtype (a few conversions per eight tokens: no form of its own)
+// LDS of a workgroup, in floats: two stages of the pairs, the decays (kind 1), four of the values and (decay, step size) pairs (kind 2);
+// partial read-outs of a token: 16 row groups of the columns, and 16 more so that the reads of several tokens meet no bank twice.  One column per
+// thread: two stages of sums, which saves a barrier per stage (1024 tokens: 140 -> 131 us); two columns: one, for a third and fourth workgroup
+// per CU (32 runs of 60 - 120: 119 -> 107)
 template <int RMAX, int CV, int KIND>
-__global__ __launch_bounds__(256) void linear_walk_kernel(const ScanArgs a, const float2* __restrict__ kq, const float2* __restrict__ td, int dt) {
-  constexpr int dk = 16 * RMAX, CW = 16 * CV, NV = (kTB * CW + 255) / 256, NB = kTB * dk * 2;
+struct WalkLds {
+  static constexpr int dk = 16 * RMAX, CW = 16 * CV, KQ = kTB * dk * 2, DEC = KIND == 1 ? kTB * dk : 0, V = kTB * CW + (KIND == 2 ? 64 : 0);
+  static constexpr int SUM = 16 * CW + 16, SUMS = CV == 1 ? 2 : 1;
+  static constexpr int dec = 2 * KQ, values = dec + 2 * DEC, sums = values + 4 * V, total = sums + SUMS * kTB * SUM;
+};
+
+// dk == 16 RMAX.  dt: storage dtype of the skip weights
+template <int RMAX, int CV, int KIND>
+__global__ __launch_bounds__(256) void linear_walk_kernel(const ScanArgs a, const float2* __restrict__ kq, const float2* __restrict__ td,
+                                                          const float* __restrict__ values, int dvp, int dt) {
+  using L = WalkLds<RMAX, CV, KIND>;
+  constexpr int dk = L::dk, CW = L::CW;
   extern __shared__ __attribute__((aligned(16))) float lds[];
-  float* skq = lds;                                    // [2][kTB][dk] (key, query)
-  float* sdec = skq + 2 * NB;                          // KIND 1: [2][kTB][dk] decays; 2: [2][kTB]
-  float* sv = sdec + 2 * kTB * (KIND == 1 ? dk : 1);   // [2][kTB][CW] what enters the state
-  float* sp = sv + 2 * kTB * CW;                       // [kTB][16 groups][CW] partial read-outs
   const int b = blockIdx.y, head = blockIdx.x, c0 = blockIdx.z * CW;   // (heads over the XCDs: sequences differ in length)
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), col = (tid & 15) * CV, kg = tid >> 4;
   const int dv = a.dv, heads = a.heads, qh = head / a.qk_rep, qk_heads = heads / a.qk_rep;
@@ -303,72 +357,65 @@ __global__ __launch_bounds__(256) void linear_walk_kernel(const ScanArgs a, cons
   const float fixed = KIND == 0 ? a.head_decay[head] : 0.f;
   const bool skips = KIND == 2 && a.skip;
   const float skip = !skips ? 0.f : dt == LL_F32 ? ldv<LL_F32>(a.skip, head) : dt == LL_F16 ? ldv<LL_F16>(a.skip, head) : ldv<LL_BF16>(a.skip, head);
-  // eight tokens' pairs (and decays) to LDS: 16-byte pieces in token order; a token behind the run repeats its last row
-  auto request = [&](int base, int buf) {
+  // Eight tokens' numbers to LDS.  Where a wave has no piece of its own it repeats another one's (the same bytes to the same place).  Tokens behind the run are other runs' or the scratch's spare rows, and nobody's to read.
+  const char* kq_at = (const char*)(kq + ((int64_t)t0 * qk_heads + qh) * dk);
+  const char* dec_at = (const char*)(a.decay_pre + ((int64_t)t0 * heads + head) * dk);
+  const char* td_at = (const char*)(td + (int64_t)t0 * heads + head);
+  const char* v_at = (const char*)(values + ((int64_t)t0 * heads + head) * dvp + c0);
+  uint32_t kq_off[RMAX / 4], dec_off[(RMAX + 7) / 8];
 #pragma unroll
-    for (int j = 0; j < RMAX; j += 4) {
-      const int p = (wave + j) * 64 + lane, tt = p / (dk / 2), at = p - tt * (dk / 2);
-      const int row = base + tt < t1 ? base + tt : t1 - 1;
-      dma16((uint32_t)((buf * NB) * 4 + (wave + j) * 1024), kq + ((int64_t)row * qk_heads + qh) * dk + 2 * at);
-    }
+  for (int j = 0; j < RMAX / 4; ++j) {
+    const int p = (wave + 4 * j) * 64 + lane;
+    kq_off[j] = (uint32_t)(p / (dk / 2)) * (uint32_t)(qk_heads * dk * 8) + (uint32_t)(p % (dk / 2)) * 16u;
+  }
+#pragma unroll
+  for (int j = 0; j < (RMAX + 7) / 8; ++j) {
+    const int p = ((RMAX == 4 ? wave & 1 : wave) + 4 * j) * 64 + lane;
+    dec_off[j] = (uint32_t)(p / (dk / 4)) * (uint32_t)(heads * dk * 4) + (uint32_t)(p % (dk / 4)) * 16u;
+  }
+  const int vw = CV == 1 ? wave & 1 : wave;
+  const uint32_t v_off = (uint32_t)((vw * 64 + lane) / CW) * (uint32_t)(heads * dvp * 4) + (uint32_t)(lane % CW) * 4u;
+  const uint32_t td_off = (uint32_t)(lane / 2 % kTB) * (uint32_t)(heads * 8) + (uint32_t)(lane & 1) * 4u;
+  auto request = [&](int slot, int vslot) {
+#pragma unroll
+    for (int j = 0; j < RMAX / 4; ++j) dma16((uint32_t)(slot * L::KQ * 4 + (wave + 4 * j) * 1024), kq_at, kq_off[j]);
     if constexpr (KIND == 1) {
 #pragma unroll
-      for (int j = 0; j < RMAX / 2; j += 4) {
-        if (wave + j >= RMAX / 2) break;
-        const int p = (wave + j) * 64 + lane, tt = p / (dk / 4), at = p - tt * (dk / 4);
-        const int row = base + tt < t1 ? base + tt : t1 - 1;
-        dma16((uint32_t)((2 * NB + buf * kTB * dk) * 4 + (wave + j) * 1024), a.decay_pre + ((int64_t)row * heads + head) * dk + 4 * at);
-      }
+      for (int j = 0; j < (RMAX + 7) / 8; ++j)
+        dma16((uint32_t)((L::dec + slot * L::DEC) * 4 + ((RMAX == 4 ? wave & 1 : wave) + 4 * j) * 1024), dec_at, dec_off[j]);
     }
-  };
-  // values of a stage: entries tid + 256 j of [kTB][CW], bits first
-  uint32_t raw[NV];
-  float2 rt[NV];
-  float sx[NV];
-  auto fetch = [&](int base) {
-#pragma unroll
-    for (int j = 0; j < NV; ++j) {
-      const int i = tid + 256 * j, tt = i / CW, cc = i % CW;
-      const int row = base + tt < t1 ? base + tt : t1 - 1;
-      const int64_t at = (int64_t)row * a.v_ld + (int64_t)head * dv + (c0 + cc < dv ? c0 + cc : 0);
-      raw[j] = dt == LL_F32 ? ((const uint32_t*)a.v)[at] : ((const uint16_t*)a.v)[at];
-      if constexpr (KIND == 2) rt[j] = td[(int64_t)row * heads + head];
-    }
-  };
-  auto stage = [&](int buf) {
-#pragma unroll
-    for (int j = 0; j < NV; ++j) {
-      const int i = tid + 256 * j, tt = i / CW, cc = i % CW;
-      float x = dt == LL_F32 ? __uint_as_float(raw[j]) : dt == LL_F16 ? to_f32<LL_F16>((uint16_t)raw[j]) : to_f32<LL_BF16>((uint16_t)raw[j]);
-      if (c0 + cc >= dv) x = 0.f;
-      if (a.act) x *= dt == LL_F32 ? act_sigmoid<LL_F32>(x) : act_sigmoid<LL_BF16>(x);
-      sx[j] = skips ? skip * x : 0.f;
-      if (i >= kTB * CW) continue;
-      sv[buf * kTB * CW + i] = KIND == 2 ? rt[j].y * x : x;
-      if (KIND == 2 && cc == 0) sdec[buf * kTB + tt] = rt[j].x;
-    }
+    dma4((uint32_t)((L::values + vslot * L::V) * 4 + vw * 256), v_at, v_off);
+    if constexpr (KIND == 2) dma4((uint32_t)((L::values + vslot * L::V + kTB * CW) * 4), td_at, td_off);
+    kq_at += (int64_t)kTB * qk_heads * dk * 8;
+    dec_at += (int64_t)kTB * heads * dk * 4;
+    td_at += (int64_t)kTB * heads * 8;
+    v_at += (int64_t)kTB * heads * dvp * 4;
   };
   struct Token {   // what a thread reads of a token
-    float2 g[RMAX];
-    float dec[KIND == 1 ? RMAX : 1], v[CV];
+    f32x4 kq[RMAX / 2], dec[KIND == 1 ? RMAX / 4 : 1];
+    float v[CV];
   };
-  auto read = [&](int buf, int tt, Token& k) {
-    const float* val = sv + (buf * kTB + tt) * CW + col;
-    const float* kp = skq + buf * NB + (tt * dk + kg) * 2;
-    const float* dp = sdec + (KIND == 1 ? (buf * kTB + tt) * dk + kg : buf * kTB + tt);
+  auto read = [&](int slot, int vslot, int tt, Token& k) {
+    const float* val = lds + L::values + vslot * L::V;
     if constexpr (CV == 2) {
-      const float2 w = *reinterpret_cast<const float2*>(val);
+      const float2 w = *reinterpret_cast<const float2*>(val + tt * CW + col);
       k.v[0] = w.x;
       k.v[1] = w.y;
     } else {
-      k.v[0] = val[0];
+      k.v[0] = val[tt * CW + col];
     }
-    if constexpr (KIND == 0) k.dec[0] = fixed;
-    if constexpr (KIND == 2) k.dec[0] = dp[0];
 #pragma unroll
-    for (int r = 0; r < RMAX; ++r) {
-      k.g[r] = *reinterpret_cast<const float2*>(kp + 32 * r);
-      if constexpr (KIND == 1) k.dec[r] = dp[16 * r];
+    for (int j = 0; j < RMAX / 2; ++j) k.kq[j] = *reinterpret_cast<const f32x4*>(lds + slot * L::KQ + tt * dk * 2 + j * 64 + kg * 4);
+    if constexpr (KIND == 0) k.dec[0][0] = fixed;
+    if constexpr (KIND == 1) {
+#pragma unroll
+      for (int j = 0; j < RMAX / 4; ++j) k.dec[j] = *reinterpret_cast<const f32x4*>(lds + L::dec + slot * L::DEC + tt * dk + j * 64 + kg * 4);
+    }
+    if constexpr (KIND == 2) {
+      const float2 w = *reinterpret_cast<const float2*>(val + kTB * CW + 2 * tt);
+      k.dec[0][0] = w.x;
+#pragma unroll
+      for (int e = 0; e < CV; ++e) k.v[e] = w.y * k.v[e];
     }
   };
   auto walk = [&](const Token& k, float (&acc)[CV]) {
@@ -378,73 +425,72 @@ __global__ __launch_bounds__(256) void linear_walk_kernel(const ScanArgs a, cons
     for (int r = 0; r < RMAX; ++r)
 #pragma unroll
       for (int e = 0; e < CV; ++e) {
-        S[r][e] = __builtin_fmaf(k.dec[KIND == 1 ? r : 0], S[r][e], k.g[r].x * k.v[e]);
-        acc[e] = __builtin_fmaf(S[r][e], k.g[r].y, acc[e]);
+        S[r][e] = __builtin_fmaf(KIND == 1 ? k.dec[r / 4][r % 4] : k.dec[0][0], S[r][e], k.kq[r / 2][2 * r % 4] * k.v[e]);
+        acc[e] = __builtin_fmaf(S[r][e], k.kq[r / 2][2 * r % 4 + 1], acc[e]);
       }
   };
-  auto leave = [&](int tt, const float (&acc)[CV]) {
-    float* at = sp + (tt * 16 + kg) * CW + col;
+  float* sums = lds + L::sums;
+  auto leave = [&](int half, int tt, const float (&acc)[CV]) {
+    float* at = sums + (half * kTB + tt) * L::SUM + kg * CW + col;
     if constexpr (CV == 2) *reinterpret_cast<float2*>(at) = float2{acc[0], acc[1]};
     else at[0] = acc[0];
   };
-  auto add_up = [&](int base, const float (&x)[NV]) {
-#pragma unroll
-    for (int j = 0; j < NV; ++j) {
-      const int i = tid + 256 * j, tt = i / CW, cc = i % CW;
-      if (i >= kTB * CW || base + tt >= t1) continue;
+  // the stage in front: its partial sums in the order of the row groups
+  const int st_tt = tid / CW, st_cc = tid % CW;
+  const bool adds = tid < kTB * CW && c0 + st_cc < dv;
+  float* out = a.o + ((int64_t)(t0 + st_tt) * heads + head) * dv + c0 + st_cc;
+  auto add_up = [&](int tokens, int half, int vslot) {
+    if (adds && st_tt < tokens) {
       float o = 0.f;
 #pragma unroll
-      for (int g2 = 0; g2 < 16; ++g2) o += sp[(tt * 16 + g2) * CW + cc];
-      if (c0 + cc < dv) a.o[((int64_t)(base + tt) * heads + head) * dv + c0 + cc] = o + x[j];
+      for (int g2 = 0; g2 < 16; ++g2) o += sums[(half * kTB + st_tt) * L::SUM + g2 * CW + st_cc];
+      *out = o + (skips ? skip * lds[L::values + vslot * L::V + st_tt * CW + st_cc] : 0.f);
     }
+    out += (int64_t)kTB * heads * dv;
   };
-  fetch(t0);
-  request(t0, 0);
-  stage(0);
-  int buf = 0;
+  request(0, 0);
+  int stage = 0;
   for (int base = t0; base < t1; base += kTB) {
-    const int nt = t1 - base < kTB ? t1 - base : kTB;
+    const int nt = t1 - base < kTB ? t1 - base : kTB, slot = stage & 1, half = L::SUMS == 2 ? stage & 1 : 0;
     asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(0x0070);   // this stage's pairs and values are there; the partial sums have been read
+    __builtin_amdgcn_s_waitcnt(0x0070);   // this stage is there, and every wave is through with the stage in front
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    float x_now[NV];
-#pragma unroll
-    for (int j = 0; j < NV; ++j) x_now[j] = sx[j];
-    const bool more = base + kTB < t1;
-    if (more) {
-      request(base + kTB, buf ^ 1);
-      fetch(base + kTB);
-    }
+    if (base + kTB < t1) request(slot ^ 1, (stage + 1) & 3);
     if (nt == kTB) {
       float acc[kTB][CV];   // (written behind the last token: a write to LDS between them would hold the reads of the next)
       Token k[2];
-      read(buf, 0, k[0]);
+      read(slot, stage & 3, 0, k[0]);
+      if (stage) add_up(kTB, L::SUMS == 2 ? half ^ 1 : 0, (stage - 1) & 3);
 #pragma unroll
       for (int tt = 0; tt < kTB; ++tt) {
-        if (tt + 1 < kTB) read(buf, tt + 1, k[(tt + 1) & 1]);
+        if (tt + 1 < kTB) read(slot, stage & 3, tt + 1, k[(tt + 1) & 1]);
         __builtin_amdgcn_sched_barrier(0);   // (the next token's reads stay in front of this one's products)
         walk(k[tt & 1], acc[tt]);
       }
+      if constexpr (L::SUMS == 1) {   // (every wave has read the sums in front; the next stage may still be on its way)
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0xc07f);
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+      }
 #pragma unroll
-      for (int tt = 0; tt < kTB; ++tt) leave(tt, acc[tt]);
+      for (int tt = 0; tt < kTB; ++tt) leave(half, tt, acc[tt]);
     } else {
+      if (stage) add_up(kTB, L::SUMS == 2 ? half ^ 1 : 0, (stage - 1) & 3);
+      if constexpr (L::SUMS == 1) __syncthreads();
       for (int tt = 0; tt < nt; ++tt) {
         float acc[CV];
         Token k;
-        read(buf, tt, k);
+        read(slot, stage & 3, tt, k);
         walk(k, acc);
-        leave(tt, acc);
+        leave(half, tt, acc);
       }
     }
-    if (more) stage(buf ^ 1);
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(0xc07f);   // (LDS only: the next stage may still be on its way)
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    add_up(base, x_now);
-    buf ^= 1;
+    ++stage;
   }
+  __syncthreads();
+  add_up(t1 - t0 - (stage - 1) * kTB, L::SUMS == 2 ? (stage - 1) & 1 : 0, (stage - 1) & 3);
 #pragma unroll
   for (int r = 0; r < RMAX; ++r) {
     if (!active) continue;
@@ -863,6 +909,8 @@ constexpr int64_t kWalkFloats = 1ll << 28;   // largest scratch of the two-kerne
 
 extern "C" int ll_linear_scan_supported(int64_t dk, int64_t dv) { return dk >= 1 && dk <= 256 && dv >= 1 ? 1 : 0; }
 
+static int64_t walk_columns(int64_t dv) { return (dv + 31) / 32 * 32; }   // whole slices of columns, of either width
+
 // Floats of scratch for the two-kernel walk, 0 where the one above serves: heads of 64, 128 or 256 entries (whole 16-byte pieces and DMA
 // rounds) and a longest run of 24 tokens.  One run, us, one kernel / two: of 24 16 / 10 (per entry), 12 / 9 (fixed and per token), 8.1 / 7.6 (fixed,
 // 24 heads of 64 x 128); of 16 12 / 8, 9.0 / 7.4, 9.2 / 8.3, but 6.5 / 6.8, and 6.8 / 7.5 for 48 heads of 64 x 64.
@@ -871,8 +919,9 @@ extern "C" int64_t ll_linear_scan_walk_floats(int64_t n, int64_t batch, int64_t 
   if (n < 1 || batch < 1 || batch > 65535 || heads < 1 || heads > 65535 || (dk != 64 && dk != 128 && dk != 256) || dv < 1 || qk_rep < 1 || heads % qk_rep ||
       longest_run < 24)
     return 0;
-  const int64_t per = heads / qk_rep * dk * 2 + (kind == 1 ? heads * dk : 0) + (kind == 2 ? heads * 2 : 0);
-  return per > kWalkFloats / n ? 0 : n * per;
+  // (a token's columns: at most 65535 workgroups of 1024 for its terms)
+  const int64_t per = heads / qk_rep * dk * 2 + (kind == 1 ? heads * dk : 0) + (kind == 2 ? heads * 2 : 0) + heads * walk_columns(dv);
+  return per > kWalkFloats / (n + kTB) || per > 65535ll * 1024 ? 0 : (n + kTB) * per;   // (a last stage is read whole: spare rows)
 }
 
 static int linear_scan(const void* q, int64_t q_ld, const void* k, int64_t k_ld, const void* v, int64_t v_ld, int64_t heads,
@@ -904,47 +953,46 @@ static int linear_scan(const void* q, int64_t q_ld, const void* k, int64_t k_ld,
   if (walk_scratch) {
     const int64_t floats = ll_linear_scan_walk_floats(n, batch, heads, dk, dv, qk_rep, kind, longest_run);
     if (floats <= 0 || !ll_aligned16(walk_scratch)) return LL_ERR_SHAPE;
+    const int dvp = (int)walk_columns(dv);
     const int64_t pairs = n * (heads / qk_rep) * dk;
     float2* kq = reinterpret_cast<float2*>(walk_scratch);
     float* decay = walk_scratch + 2 * pairs;
     float2* td = reinterpret_cast<float2*>(decay);
-    int64_t total = kind == 1 ? n * heads * dk : pairs;
-    if (kind == 2 && total < n * heads) total = n * heads;
-    if ((total + 255) / 256 > 0x7fffffffll || n >= (1ll << 31)) return LL_ERR_SHAPE;
+    float* values = decay + (kind == 1 ? n * heads * dk : 0) + (kind == 2 ? (n * heads + 1) / 2 * 4 : 0);
+    const int64_t pieces = heads / qk_rep * dk / 2 + (kind == 1 ? heads * dk / 4 : 0) + (kind == 2 ? heads : 0) + heads * dvp / 4;
     hipStream_t wst = (hipStream_t)stream;
-#define CALL(DT) scan_terms_kernel<DT><<<dim3((unsigned)((total + 255) / 256)), 256, 0, wst>>>(a, kq, decay, td, n, total)
+    const dim3 tgrid((unsigned)n, (unsigned)((pieces + 256 * kTermPieces - 1) / (256 * kTermPieces)));
+#define CALL(DT) scan_terms_kernel<DT><<<tgrid, 256, 0, wst>>>(a, kq, decay, td, values, dvp)
     LL_BY_DTYPE(dtype, CALL);
 #undef CALL
     a.decay_pre = decay;
-    // two columns per thread once there is more than a workgroup of one column per CU (sequences counted by the longest run's length: decoded
-    // tokens beside a portion weigh nothing): a record read serves twice the products.  us, one / two: runs of 64, per entry, 8 heads of
-    // 128 x 256: one sequence 17 / 20, two (256 workgroups) 19 / 21, four 25 / 23, eight 44 / 32; 12 heads: two (384) 24 / 22
+    // two columns per thread from three workgroups of one column per CU on (sequences counted by the longest run's length: decoded tokens beside
+    // a portion weigh nothing): a number read serves twice the products.  us, one / two: runs of 64, per entry, 8 heads of 128 x 256: one sequence
+    // 14 / 18, four (512 workgroups) 19 / 20, eight 33 / 27; runs of 300, six (768): 91 / 86, fixed 75 / 77; 32 runs of 60 - 120: 139 / 107
     const int cv = dv % 2 == 0 && (reinterpret_cast<uintptr_t>(state) & 7u) == 0 &&
-                           (n + longest_run - 1) / longest_run * heads * ((dv + 15) / 16) > 320 ? 2 : 1;
-    const int cw = 16 * cv;
-    const size_t wlds = sizeof(float) * (size_t)(2 * kTB * (2 * dk + (kind == 1 ? dk : 1) + 9 * cw));
-    const dim3 wgrid((unsigned)heads, (unsigned)batch, (unsigned)((dv + cw - 1) / cw));
+                           (n + longest_run - 1) / longest_run * heads * ((dv + 15) / 16) >= 768 ? 2 : 1;
+    const dim3 wgrid((unsigned)heads, (unsigned)batch, (unsigned)((dv + 16 * cv - 1) / (16 * cv)));
     int dev = 0;
     (void)hipGetDevice(&dev);
-#define CALL_W(R, C, KD)                                                                                                               \
-  do {                                                                                                                                 \
-    static bool attr[16] = {false};                                                                                                    \
-    if (dev >= 0 && dev < 16 && !attr[dev]) {                                                                                          \
-      (void)hipFuncSetAttribute((const void*)linear_walk_kernel<R, C, KD>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);    \
-      attr[dev] = true;                                                                                                                \
-    }                                                                                                                                  \
-    linear_walk_kernel<R, C, KD><<<wgrid, 256, wlds, wst>>>(a, kq, td, dtype);                                                         \
+#define CALL_W(R, C, KD)                                                                                                            \
+  do {                                                                                                                              \
+    static bool attr[16] = {false};                                                                                                 \
+    if (dev >= 0 && dev < 16 && !attr[dev]) {                                                                                       \
+      (void)hipFuncSetAttribute((const void*)linear_walk_kernel<R, C, KD>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); \
+      attr[dev] = true;                                                                                                             \
+    }                                                                                                                               \
+    linear_walk_kernel<R, C, KD><<<wgrid, 256, sizeof(float) * WalkLds<R, C, KD>::total, wst>>>(a, kq, td, values, dvp, dtype);      \
   } while (0)
-#define CALL_C(R, KD)                 \
-  if (cv == 2) CALL_W(R, 2, KD); \
+#define CALL_C(R, KD)              \
+  if (cv == 2) CALL_W(R, 2, KD);   \
   else CALL_W(R, 1, KD)
-#define CALL_K(R)                     \
-  if (kind == 0) { CALL_C(R, 0); }    \
+#define CALL_K(R)                    \
+  if (kind == 0) { CALL_C(R, 0); }   \
   else if (kind == 1) { CALL_C(R, 1); } \
   else { CALL_C(R, 2); }
-    if (dk == 64) { CALL_K(4) }
-    else if (dk == 128) { CALL_K(8) }
-    else { CALL_K(16) }
+    if (dk == 64) { CALL_K(4); }
+    else if (dk == 128) { CALL_K(8); }
+    else { CALL_K(16); }
 #undef CALL_K
 #undef CALL_C
 #undef CALL_W

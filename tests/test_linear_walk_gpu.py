@@ -81,6 +81,13 @@ def test_runs_of_many_tokens(dtype, kind, heads, qk_heads, dk, dv, runs):
     assert torch.equal(outs[0], outs[1]) and torch.equal(states[0], states[1])
 
 
+@pytest.mark.parametrize("kind,heads,qk_heads,dk,dv", [("fixed", 64, 64, 64, 200), ("entry", 48, 24, 128, 258), ("token", 112, 7, 256, 98)])
+@pytest.mark.parametrize("runs", [[(0, 24)], [(5, 1), (9, 79), (0, 16), (3, 17), (0, 1)]])
+def test_runs_of_many_tokens_in_two_columns_per_thread(kind, heads, qk_heads, dk, dv, runs):
+    """Three workgroups of 16 columns per CU and more; a last slice of 2, 8 and 32 columns."""
+    test_runs_of_many_tokens(torch.bfloat16, kind, heads, qk_heads, dk, dv, runs)
+
+
 @pytest.mark.parametrize("dv", [16, 320])   # one state column per thread, two
 def test_a_run_without_tokens_leaves_the_state_it_started_from(dv):
     """Zeros where it starts at position 0, whatever an earlier owner of the slot left; as in the walk in one kernel."""
