@@ -651,7 +651,8 @@ __device__ __forceinline__ void st8(void* p, int64_t i, const float (&o)[8]) {
   }
 }
 
-// The read-out norm for long parts: one workgroup per (token, part), same arithmetic per element as the wave form.
+// The read-out norm for long parts off 16-byte borders or beyond 8192 channels: one workgroup per (token, part), same arithmetic per element as
+// the wave form.
 template <int DT>
 __global__ __launch_bounds__(256) void gated_out_norm_block_kernel(void* __restrict__ out, int64_t out_ld, const float* __restrict__ o,
                                                                    const void* __restrict__ gate, int64_t gate_ld, int gate_kind,
@@ -696,31 +697,37 @@ __device__ __forceinline__ float row16_sum(float v) {
   return v;
 }
 
-// The read-out norm of short parts (a head: up to 128 NP channels, a multiple of 8) in 16-byte pieces: one 16-lane row per (token,
-// part), lane r owns the eight channels at 8 (r + 16 j).  Every value is read once; same arithmetic per element as the wave form.
-template <int DT, int NP>
+// The read-out norm in 16-byte pieces: TP threads per (token, part), thread r owns the eight channels at 8 (r + TP j).  TP 16: short parts (a
+// head: up to 128 NP channels, a multiple of 8), one 16-lane row each; TP 256: long parts (up to 2048 NP), a workgroup each.  Every value is
+// read once; same arithmetic per element as the wave form.  Bound by the chain load -> sum -> store for few tokens, by memory for many: one
+// gated part of 2048, us, the block form (reads twice, two or four bytes at a time) -> now: 32
+// tokens 6.9 -> 3.6, 3000 tokens 19.1 -> 12.1 (4.1 TB/s); of 4096, 11.6 -> 4.7, 38.7 -> 20.4.
+template <int DT, int NP, int TP>
 __global__ __launch_bounds__(256) void gated_out_norm_vec_kernel(void* __restrict__ out, int64_t out_ld, const float* __restrict__ o,
                                                                  const void* __restrict__ gate, int64_t gate_ld, int gate_kind,
                                                                  int gate_first, const void* __restrict__ w, int w_len, float eps,
                                                                  float out_scale, int64_t items, int parts, int ps) {
-  const int64_t item = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
-  if (item >= items) return;   // (whole 16-lane rows leave; nothing below crosses rows)
-  const int r = threadIdx.x & 15;
+  const int64_t item = TP == 16 ? (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4) : (int64_t)blockIdx.x;
+  if (TP == 16 && item >= items) return;   // (whole 16-lane rows leave; nothing below crosses rows)
+  const int r = threadIdx.x & (TP - 1);
   const int64_t t = item / parts;
   const int c0 = (int)(item - t * parts) * ps;
-  float v[NP][8], g[NP][8];
+  __shared__ __attribute__((aligned(16))) float all[TP == 16 ? 4 : 2048 * NP];
+  float v[NP][8], g[NP][8], wv[NP][8];
   float ss = 0.f;
 #pragma unroll
   for (int j = 0; j < NP; ++j) {
-    const int cc = 8 * (r + 16 * j);
+    const int cc = 8 * (r + TP * j);
     const bool in = cc < ps;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       v[j][e] = 0.f;
       g[j][e] = 1.f;
+      wv[j][e] = 1.f;
     }
     if (in) {
       ld8<LL_F32>(o, t * (int64_t)parts * ps + c0 + cc, v[j]);
+      if (w) ld8<DT>(w, (c0 + cc) % w_len, wv[j]);
       if (gate_kind) {
         ld8<DT>(gate, t * gate_ld + c0 + cc, g[j]);
 #pragma unroll
@@ -734,20 +741,30 @@ __global__ __launch_bounds__(256) void gated_out_norm_vec_kernel(void* __restric
         for (int e = 0; e < 8; ++e) v[j][e] *= g[j][e];
       }
     }
+    if constexpr (TP == 16) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) ss += v[j][e] * v[j][e];
+      for (int e = 0; e < 8; ++e) ss += v[j][e] * v[j][e];
+    } else if (in) {
+      *reinterpret_cast<f32x4*>(all + cc) = f32x4{v[j][0], v[j][1], v[j][2], v[j][3]};
+      *reinterpret_cast<f32x4*>(all + cc + 4) = f32x4{v[j][4], v[j][5], v[j][6], v[j][7]};
+    }
   }
-  ss = row16_sum(ss);
+  if constexpr (TP == 16) {
+    ss = row16_sum(ss);
+  } else {   // (the block form's order: the same sum on and off 16-byte borders)
+    __shared__ float red[4];
+    __syncthreads();
+    for (int cc = threadIdx.x; cc < ps; cc += 256) ss += all[cc] * all[cc];
+    ss = block_sum256(ss, red);
+  }
   const float inv = 1.0f / sqrtf(ss / (float)ps + eps);
 #pragma unroll
   for (int j = 0; j < NP; ++j) {
-    const int cc = 8 * (r + 16 * j);
+    const int cc = 8 * (r + TP * j);
     if (cc < ps) {
-      float wv[8];
-      if (w) ld8<DT>(w, (c0 + cc) % w_len, wv);
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        float y = v[j][e] * inv * (w ? wv[e] : 1.0f);
+        float y = v[j][e] * inv * wv[j][e];
         if (!gate_first) y *= g[j][e];
         v[j][e] = y * out_scale;
       }
@@ -1067,7 +1084,23 @@ extern "C" int ll_gated_out_norm(void* out, int64_t out_ld, const float* o, cons
   if (!out || !o || (gate_kind && (!gate || gate_ld < width))) return LL_ERR_ARG;
   const int64_t items = n * parts;
   if (items > 0x7fffffffll) return LL_ERR_SHAPE;
-  if (width / parts >= 512) {   // long parts: a workgroup each (the form depends on the part's length only)
+  const int al = dtype == LL_F32 ? 4 : 8, ps = (int)(width / parts);
+  const bool pieces = ps % 8 == 0 && out_ld % al == 0 && ll_aligned16(out) && ll_aligned16(o) &&
+                      (!gate_kind || (gate_ld % al == 0 && ll_aligned16(gate))) && (!w || (w_len % 8 == 0 && ll_aligned16(w)));
+  if (ps >= 512 && ps <= 8192 && pieces) {   // long parts in 16-byte pieces
+#define CALL_N(DT, NP)                                                                                                           \
+  gated_out_norm_vec_kernel<DT, NP, 256><<<dim3((unsigned)items), 256, 0, (hipStream_t)stream>>>(                                \
+      out, out_ld, o, gate, gate_ld, gate_kind, gate_first ? 1 : 0, w, (int)(w ? w_len : 8), eps, out_scale, items, (int)parts, ps)
+#define CALL(DT)                       \
+  if (ps <= 2048) CALL_N(DT, 1);       \
+  else if (ps <= 4096) CALL_N(DT, 2);  \
+  else CALL_N(DT, 4)
+    LL_BY_DTYPE(dtype, CALL);
+#undef CALL
+#undef CALL_N
+    return LL_LAUNCH_CHECK();
+  }
+  if (ps >= 512) {   // long parts off those borders: a workgroup each
 #define CALL(DT)                                                                                                                   \
   gated_out_norm_block_kernel<DT><<<dim3((unsigned)items), 256, 0, (hipStream_t)stream>>>(                                         \
       out, out_ld, o, gate, gate_ld, gate_kind, gate_first ? 1 : 0, w, (int)(w ? w_len : 1), eps, out_scale, (int)parts, (int)(width / parts))
@@ -1075,12 +1108,10 @@ extern "C" int ll_gated_out_norm(void* out, int64_t out_ld, const float* o, cons
 #undef CALL
     return LL_LAUNCH_CHECK();
   }
-  const int al = dtype == LL_F32 ? 4 : 8, ps = (int)(width / parts);
-  if (ps % 8 == 0 && ps <= 512 && out_ld % al == 0 && ll_aligned16(out) && ll_aligned16(o) &&
-      (!gate_kind || (gate_ld % al == 0 && ll_aligned16(gate))) && (!w || (w_len % 8 == 0 && ll_aligned16(w)))) {
+  if (pieces) {
     const dim3 vgrid((unsigned)((items + 15) / 16));
 #define CALL_N(DT, NP)                                                                                                           \
-  gated_out_norm_vec_kernel<DT, NP><<<vgrid, 256, 0, (hipStream_t)stream>>>(                                                     \
+  gated_out_norm_vec_kernel<DT, NP, 16><<<vgrid, 256, 0, (hipStream_t)stream>>>(                                                     \
       out, out_ld, o, gate, gate_ld, gate_kind, gate_first ? 1 : 0, w, (int)(w ? w_len : 8), eps, out_scale, items, (int)parts, ps)
 #define CALL(DT)                      \
   if (ps <= 128) CALL_N(DT, 1);       \

@@ -5,8 +5,9 @@
 //                     neighbours, a group's score is the sum of its two best scores, only the best `group_keep` groups stay
 //                     eligible; the `top` best eligible experts are chosen, their scores divided by their sum (+ 1e-20) and
 //                     multiplied by `route_scale`.  One more row of weights may give a per-token sigmoid scale (for a shared
-//                     expert).  Two launches: the logits as an 8 x 8 register-tiled product per wave, then one wave per token
-//                     that selects by ranks (ties: the lower index first), so slot k of a token holds its k-th best expert.
+//                     expert).  Up to 512 tokens in one launch (a workgroup forms its tokens' logits and selects), beyond in two:
+//                     the logits as an 8 x 8 register-tiled product per wave, then one wave per token.  Selection by ranks (ties:
+//                     the lower index first), so slot k of a token holds its k-th best expert.
 //   ll_moe_sort       slots (token, k) sorted by expert, every expert's run padded to the row-block size with a sentinel:
 //                     sorted_ids / block_expert / num_post as in moe_align_block_size.  Deterministic: no atomics.
 //   ll_moe_rows_gemm  the grouped products over sorted row blocks: act = silu(a Wg_e^T) * (a Wu_e^T) (gate and up rows
