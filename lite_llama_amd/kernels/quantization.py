@@ -579,6 +579,11 @@ def dense16_rows_wins(m: int, n: int, k: int) -> bool:
     return 1 <= m <= 64 and n >= 8192 and n % 32 == 0 and k % 128 == 0
 
 
+def _on_one_device(x: torch.Tensor, *operands) -> bool:
+    """Whether all operands are where ``x`` is: a kernel is handed their addresses, whatever they point at."""
+    return all(t is None or t.device == x.device for t in operands)
+
+
 def dense16_rows_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None, *, gate_up_swiglu: bool = False):
     """Extension (round 5): ``F.linear(x, weight, bias)`` -- or, with ``gate_up_swiglu``, ``silu(gate) * up`` of a fused gate|up
     weight whose rows are interleaved ``(gate_j, up_j)`` -- for decode shapes (<= 64 rows) of an UNQUANTISED fp16 / bf16 weight
@@ -588,7 +593,8 @@ def dense16_rows_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tenso
             or os.environ.get("LL_DENSE16_ROWS_OFF") or not L.has("ll_dense16_rows_matmul")):
         return None
     n, k = weight.shape
-    if x.shape[-1] != k or (bias is not None and (bias.dtype != x.dtype or bias.numel() != n or gate_up_swiglu)):
+    if (x.shape[-1] != k or (bias is not None and (bias.dtype != x.dtype or bias.numel() != n or gate_up_swiglu))
+            or not _on_one_device(x, weight, bias)):
         return None
     a = _flatten(x, k)
     m = a.shape[0]
@@ -610,7 +616,7 @@ def dense16_narrow_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Ten
     if x.dtype not in (torch.float16, torch.bfloat16) or weight.dtype != x.dtype or weight.dim() != 2 or not x.is_cuda:
         return None
     n, k = weight.shape
-    if x.shape[-1] != k or k == 0 or x.numel() > 64 * k or not L.has("ll_dense16_narrow_wins"):
+    if x.shape[-1] != k or k == 0 or x.numel() > 64 * k or not _on_one_device(x, weight, bias) or not L.has("ll_dense16_narrow_wins"):
         return None
     m = x.numel() // k
     if not L.lib().ll_dense16_narrow_wins(m, n, k) or os.environ.get("LL_DENSE16_NARROW_OFF"):
@@ -639,7 +645,7 @@ def dense16_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | N
             or os.environ.get("LL_DENSE16_OFF") or not L.has("ll_dense16_matmul")):
         return None
     n, k = weight.shape
-    if x.shape[-1] != k or (bias is not None and (bias.dtype != x.dtype or bias.numel() != n)):
+    if x.shape[-1] != k or (bias is not None and (bias.dtype != x.dtype or bias.numel() != n)) or not _on_one_device(x, weight, bias):
         return None
     a = _flatten(x, k)
     m = a.shape[0]
