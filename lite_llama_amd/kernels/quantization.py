@@ -10,6 +10,7 @@ import math
 import os
 
 import torch
+from torch.autograd import forward_ad
 
 from .. import _lib as L
 
@@ -584,6 +585,23 @@ def _on_one_device(x: torch.Tensor, *operands) -> bool:
     return all(t is None or t.device == x.device for t in operands)
 
 
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def _is_followed(x: torch.Tensor, weight: torch.Tensor, bias) -> bool:
+    """Whether something wants to see the operation itself on these and not only its result: a tensor type or a dispatch mode of its own,
+    autograd, a function transform, a forward-mode tangent, autocast, a trace."""
+    if type(x) not in _PLAIN or type(weight) not in _PLAIN or (bias is not None and type(bias) not in _PLAIN):
+        return True
+    if torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad or (bias is not None and bias.requires_grad)):
+        return True
+    if torch._C._functorch.maybe_current_level() is not None or torch._C._len_torch_dispatch_stack() > 0:
+        return True
+    if any(t is not None and forward_ad.unpack_dual(t).tangent is not None for t in (x, weight, bias)):
+        return True
+    return torch.is_autocast_enabled("cuda") or torch._C._get_tracing_state() is not None
+
+
 def dense16_rows_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None, *, gate_up_swiglu: bool = False):
     """Extension (round 5): ``F.linear(x, weight, bias)`` -- or, with ``gate_up_swiglu``, ``silu(gate) * up`` of a fused gate|up
     weight whose rows are interleaved ``(gate_j, up_j)`` -- for decode shapes (<= 64 rows) of an UNQUANTISED fp16 / bf16 weight
@@ -611,15 +629,15 @@ def dense16_rows_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tenso
 
 def dense16_narrow_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None):
     """``F.linear(x, weight, bias)`` of up to 64 rows over a narrow unquantised fp16 / bf16 weight (csrc/gemm_narrow.hip); rows of ``x`` may
-    be a column range of wider ones.  ``None`` where the call is not served or another route measured faster
-    (``ll_dense16_narrow_wins``)."""
+    be a column range of wider ones.  ``None`` where the call is not served, another route measured faster
+    (``ll_dense16_narrow_wins``), or the result has to carry more than its values (:func:`_is_followed`)."""
     if x.dtype not in (torch.float16, torch.bfloat16) or weight.dtype != x.dtype or weight.dim() != 2 or not x.is_cuda:
         return None
     n, k = weight.shape
     if x.shape[-1] != k or k == 0 or x.numel() > 64 * k or not _on_one_device(x, weight, bias) or not L.has("ll_dense16_narrow_wins"):
         return None
     m = x.numel() // k
-    if not L.lib().ll_dense16_narrow_wins(m, n, k) or os.environ.get("LL_DENSE16_NARROW_OFF"):
+    if not L.lib().ll_dense16_narrow_wins(m, n, k) or os.environ.get("LL_DENSE16_NARROW_OFF") or _is_followed(x, weight, bias):
         return None
     a = x if x.dim() == 2 and x.stride(1) == 1 and x.stride(0) >= k else _flatten(x, k)
     if (a.stride(0) % 8 or a.data_ptr() % 16 or weight.stride(1) != 1 or weight.stride(0) % 8 or weight.stride(0) < k or weight.data_ptr() % 16

@@ -1,10 +1,9 @@
 """Which projections go to a kernel by address (kernels/quantization.py), without a GPU: tensors that call themselves GPU tensors, and a library
 that notes what it is asked for."""
 
-import types
-
 import pytest
 import torch
+import torch.utils._python_dispatch
 from torch import nn
 
 from lite_llama_amd.kernels import quantization as Q
@@ -48,5 +47,46 @@ def test_operands_on_another_device_are_left_to_the_library(launches, linear, wh
     else:
         bias = torch.empty(896, dtype=torch.float16, device="meta")
     assert linear(x, weight, bias) is None and launches() == []
-    linear(x, _gpu(896, 896), _gpu(896))
-    assert len(launches()) == 1   # (where all of them are, the kernel runs)
+    if linear is not Q.dense16_narrow_linear:   # (where all of them are, the kernel runs; the narrow one takes no tensor types of others)
+        linear(x, _gpu(896, 896), _gpu(896))
+        assert len(launches()) == 1
+
+
+def _plain(*shape, dtype=torch.float16):
+    return torch.zeros(*shape, dtype=dtype)
+
+
+@pytest.mark.parametrize("bias", [True, False])
+def test_results_that_carry_more_than_values_are_left_to_the_library(launches, monkeypatch, bias):
+    """The narrow projections replaced ``F.linear`` calls, which gradients, tangents, transforms, modes and autocast pass through."""
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    x, weight, b = _plain(4, 896), _plain(896, 896), _plain(896) if bias else None
+    ask = Q.dense16_narrow_linear
+
+    def left(x=x, weight=weight, b=b):
+        at = len(launches())
+        out = ask(x, weight, b)
+        assert (out is None) == (len(launches()) == at)
+        return out is None
+
+    assert not left() and not left(weight=nn.Parameter(weight, requires_grad=False))
+    assert left(x=x.clone().requires_grad_()) and left(weight=nn.Parameter(weight))
+    with torch.no_grad():
+        assert not left(x=x.clone().requires_grad_()) and not left(weight=nn.Parameter(weight))
+    if bias:
+        assert left(b=nn.Parameter(b))
+    assert left(weight=weight.as_subclass(OnGpu))
+    with torch.autograd.forward_ad.dual_level():
+        assert left(x=torch.autograd.forward_ad.make_dual(x, x)) and not left()
+    seen = []
+    torch.func.vmap(lambda row: (seen.append(left(x=row)), row)[1])(_plain(2, 4, 896))
+    assert seen == [True]
+
+    class Mode(torch.utils._python_dispatch.TorchDispatchMode):
+        def __torch_dispatch__(self, func, kinds, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    with Mode():
+        assert left()
+    monkeypatch.setattr(torch, "is_autocast_enabled", lambda kind: True)
+    assert left()
