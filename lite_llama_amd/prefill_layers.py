@@ -58,7 +58,7 @@ class ShortPrefill:
             return None
         cos, sin = position_embeddings
         select, starts, lens = info.cur_select_index, info.b_start_loc, info.b_seq_len
-        if not all(torch.is_tensor(t) and t.is_cuda for t in (cos, sin, select, starts, lens)):
+        if not all(torch.is_tensor(t) and t.device == hidden.device for t in (cos, sin, select, starts, lens)):
             return None
         if (cos.dim() != 3 or cos.shape != sin.shape or cos.dtype != sin.dtype or not cos.is_contiguous() or not sin.is_contiguous()
                 or cos.dtype not in (torch.float16, torch.bfloat16, torch.float32)
@@ -119,15 +119,15 @@ class ShortPrefill:
         norm1, norm2 = layer.input_layernorm_weight, layer.post_attention_layernorm_weight
         weights = ((qkv.weight, row, width), (o.weight, width, q_size), (gate_up.weight, 2 * inter, width), (down.weight, width, inter))
         for w, n, k in weights:
-            if w.dtype != dt or not w.is_cuda or tuple(w.shape) != (n, k) or not w.is_contiguous():
+            if w.dtype != dt or w.device != self.device or tuple(w.shape) != (n, k) or not w.is_contiguous():
                 return None
         bias = qkv.bias
-        if bias is not None and (bias.dtype != dt or bias.numel() != row or not bias.is_contiguous()):
+        if bias is not None and (bias.dtype != dt or bias.device != self.device or bias.numel() != row or not bias.is_contiguous()):
             return None
         for w in (norm1, norm2):
-            if w.dtype != dt or w.numel() != width or not w.is_contiguous():
+            if w.dtype != dt or w.device != self.device or w.numel() != width or not w.is_contiguous():
                 return None
-        if (pool.dtype != dt or not pool.is_cuda or pool.dim() != 3 or pool.shape[1] != 2 * kv_heads or pool.shape[2] != dim or pool.stride(2) != 1
+        if (pool.dtype != dt or pool.device != self.device or pool.dim() != 3 or pool.shape[1] != 2 * kv_heads or pool.shape[2] != dim or pool.stride(2) != 1
                 or self.cos.shape[2] < dim // 2 or info.cur_select_index.numel() < self.tokens):
             return None
         _, buf, (x, qkv_rows, attn_rows, act_rows), planes, plane_view = self._scratch(row, q_size, inter)

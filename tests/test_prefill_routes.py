@@ -1,0 +1,61 @@
+"""Which layers of a short prefill go out in one host call (prefill_layers.py) and which prefills run on the prompts' tokens alone
+(model.py::CausalLM._packs), without a GPU: tensors that call themselves GPU tensors, and a library that notes what it is asked for."""
+
+import types
+
+import pytest
+import torch
+from torch import nn
+
+import lite_llama_amd.prefill_layers as P
+from lite_llama_amd.model import CausalLM, RotaryEmbedding, tiny_geometry
+
+
+@pytest.fixture
+def plain(monkeypatch):
+    """A two-layer model with merged projections, a pass over 5 tokens of it, and the layer calls that reached the library."""
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    calls = []
+    monkeypatch.setattr(P.L, "lib", lambda: types.SimpleNamespace(ll_prefill_layer16=lambda *a: (calls.append(a), 0)[1]))
+    monkeypatch.setattr(P.L, "has", lambda name: True)
+    monkeypatch.setattr(P.L, "stream_ptr", lambda: 0)
+    model = CausalLM(tiny_geometry())
+    info = types.SimpleNamespace(cur_select_index=torch.arange(5), b_start_loc=torch.zeros(1, dtype=torch.int32), b_seq_len=torch.tensor([5]),
+                                 max_actual_seq_len=5, kv_buffer=[torch.zeros(8, 4, 64, dtype=torch.float16)] * 2)
+    hidden = torch.zeros(1, 5, 256, dtype=torch.float16)
+    position = RotaryEmbedding(model.geo)(hidden, torch.arange(5)[None])
+
+    def issued():
+        """Whether layer 0 goes out in one call."""
+        del calls[:]
+        short = P.ShortPrefill.of(model, hidden, position, info)
+        if short is not None:
+            assert short.layer(model.layers[0], 0, hidden.clone(), None) is None   # (the library declines)
+        return len(calls) == 1
+
+    assert issued()
+    return types.SimpleNamespace(model=model, info=info, issued=issued)
+
+
+def _meta(t):
+    return torch.empty_like(t, device="meta")
+
+
+@pytest.mark.parametrize("what", ["input_layernorm_weight", "post_attention_layernorm_weight", "o_proj", "down_proj", "bias", "pool", "lens", "starts",
+                                  "select"])
+def test_tensors_on_another_device_keep_the_layers_own_forward(plain, what):
+    layer, info = plain.model.layers[0], plain.info
+    if "layernorm" in what:
+        setattr(layer, what, nn.Parameter(_meta(getattr(layer, what)), requires_grad=False))
+    elif what in ("o_proj", "down_proj"):
+        module = layer.self_attn.o_proj if what == "o_proj" else layer.mlp.down_proj
+        module.weight = nn.Parameter(_meta(module.weight), requires_grad=False)
+    elif what == "bias":
+        layer.self_attn._qkv._holder.bias = _meta(layer.self_attn._qkv._holder.bias)
+    elif what == "pool":
+        info.kv_buffer = [_meta(t) for t in info.kv_buffer]
+    else:
+        name = {"lens": "b_seq_len", "starts": "b_start_loc", "select": "cur_select_index"}[what]
+        setattr(info, name, _meta(getattr(info, name)))
+    assert not plain.issued()
