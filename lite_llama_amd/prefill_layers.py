@@ -103,7 +103,8 @@ class ShortPrefill:
         o, down, paged = attn.o_proj, mlp.down_proj, attn.attn
         if not _plain(o, RowParallelLinear) or not _plain(down, RowParallelLinear) or not _plain(paged, PagedAttention):
             return None
-        if type(o.quant_method) is not UnquantizedLinearMethod or type(down.quant_method) is not UnquantizedLinearMethod:
+        if (type(o.quant_method) is not UnquantizedLinearMethod or type(down.quant_method) is not UnquantizedLinearMethod
+                or o.bias is not None or down.bias is not None):
             return None
         qkv, gate_up = attn._qkv, mlp._gate_up
         if not qkv.refresh() or not gate_up.refresh():

@@ -59,3 +59,11 @@ def test_tensors_on_another_device_keep_the_layers_own_forward(plain, what):
         name = {"lens": "b_seq_len", "starts": "b_start_loc", "select": "cur_select_index"}[what]
         setattr(info, name, _meta(getattr(info, name)))
     assert not plain.issued()
+
+
+@pytest.mark.parametrize("what", ["o_proj", "down_proj"])
+def test_a_bias_behind_a_row_parallel_projection_is_added_by_the_layer(plain, what):
+    layer = plain.model.layers[0]
+    module = layer.self_attn.o_proj if what == "o_proj" else layer.mlp.down_proj
+    module.bias = nn.Parameter(torch.ones(256, dtype=torch.float16), requires_grad=False)
+    assert not plain.issued()
