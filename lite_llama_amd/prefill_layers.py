@@ -18,7 +18,7 @@ from .kernels.norm_act import PartialSums
 
 _LOG2E = 1.4426950408889634
 _MAX_PLANES = 12
-_KNOBS = ("LL_DENSE16_ROWS_OFF", "LL_DENSE_NO_PARTIALS", "LL_DENSE16_OFF", "LL_NO_LAYER_CALLS")
+_KNOBS = ("LL_DENSE16_ROWS_OFF", "LL_DENSE_NO_PARTIALS", "LL_DENSE16_OFF", "LL_DENSE16_NARROW_OFF", "LL_NO_LAYER_CALLS")
 
 
 def _plain(module, kind) -> bool:

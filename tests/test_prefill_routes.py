@@ -67,3 +67,9 @@ def test_a_bias_behind_a_row_parallel_projection_is_added_by_the_layer(plain, wh
     module = layer.self_attn.o_proj if what == "o_proj" else layer.mlp.down_proj
     module.bias = nn.Parameter(torch.ones(256, dtype=torch.float16), requires_grad=False)
     assert not plain.issued()
+
+
+@pytest.mark.parametrize("switch", ["LL_DENSE16_ROWS_OFF", "LL_DENSE_NO_PARTIALS", "LL_DENSE16_OFF", "LL_DENSE16_NARROW_OFF", "LL_NO_LAYER_CALLS"])
+def test_switches_of_the_routes_that_a_call_contains(plain, monkeypatch, switch):
+    monkeypatch.setenv(switch, "1")
+    assert not plain.issued()
