@@ -22,6 +22,7 @@ from dataclasses import dataclass, field
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.nn.modules import module as _nn
 
 from .distributed.parallel_state import all_reduce_tp, divide, get_tp_rank, get_tp_world_size
 from .distributed.partition import ShardPlan, make_plan, scale_unit, set_active_plan
@@ -43,6 +44,7 @@ from .linear import ColumnParallelLinear, LinearBase, MergedColumnLinear, RowPar
 from .prefill_layers import ShortPrefill
 from .quantization import QuantConfig, get_moe_method
 
+_OWN = __name__.partition(".")[0] + "."   # modules of this package
 _LOG2E = 1.4426950408889634  # prefill kernel evaluates exp2 (base.py:45-47)
 
 
@@ -606,22 +608,42 @@ class CausalLM(nn.Module):
         self.rotary_emb = RotaryEmbedding(geo)
         self.eps = geo.rms_norm_eps
 
-    @staticmethod
-    def _packs(input_ids, position_ids, atten_info, logits_rows) -> bool:
+    def _packs(self, input_ids, position_ids, atten_info, logits_rows) -> bool:
         """Whether a prefill whose host-side lengths are known runs on the prompts' tokens alone instead of the padded grid: pad
-        positions feed nothing but themselves (attention never reads their rows, their own logits are undefined)."""
+        positions feed nothing but themselves (attention never reads their rows, their own logits are undefined), and no hook or
+        module from elsewhere is there to see them."""
         grid = getattr(atten_info, "prompt_grid", None)
         return (grid is not None and input_ids.is_cuda and tuple(input_ids.shape) == (grid.batch, grid.longest)
                 and 1 < grid.total < grid.batch * grid.longest and grid.describes(atten_info)
                 and position_ids.shape == input_ids.shape and input_ids.dtype == torch.int64 and position_ids.dtype == torch.int64
                 and torch.is_tensor(logits_rows) and logits_rows.is_cuda and logits_rows.dtype == torch.int64 and logits_rows.dim() == 1
-                and logits_rows.is_contiguous() and not torch.cuda.is_current_stream_capturing())
+                and logits_rows.is_contiguous() and not torch.cuda.is_current_stream_capturing() and self._only_own_modules())
+
+    def _only_own_modules(self) -> bool:
+        """Whether nothing below this module but the framework's own code is run: no hook (0.4 us a module to look), no foreign class, no
+        ``forward`` of an instance's own."""
+        if (_nn._global_forward_hooks or _nn._global_forward_pre_hooks or _nn._global_backward_hooks or _nn._global_backward_pre_hooks):
+            return False
+        todo = list(self._modules.values())
+        while todo:
+            module = todo.pop()
+            if module is None:
+                continue
+            state, kind = module.__dict__, type(module)
+            if (state["_forward_hooks"] or state["_forward_pre_hooks"] or state["_backward_hooks"] or state["_backward_pre_hooks"]
+                    or "forward" in state or (kind is not nn.ModuleList and kind is not nn.Embedding and not kind.__module__.startswith(_OWN))):
+                return False
+            todo.extend(state["_modules"].values())
+        return True
 
     @torch.no_grad()
     def forward(self, input_ids, position_ids, atten_info, logits_rows=None):
         """``[batch, seq]`` ids -> ``[batch, seq, vocab]`` fp16 logits.  ``logits_rows`` (extension:
         flat token indices) restricts the lm_head to those rows -- prefill only needs the last
-        prompt position of every sequence, not ``batch*seq*vocab`` logits."""
+        prompt position of every sequence, not ``batch*seq*vocab`` logits.
+
+        A prefill of prompts of different lengths may run on their tokens alone, as one row ``[1, tokens]`` with metadata to match
+        (:meth:`_packs`): not where a hook or a module of another origin would see it."""
         if logits_rows is not None and self._packs(input_ids, position_ids, atten_info, logits_rows):
             grid = atten_info.prompt_grid
             input_ids, position_ids, select, starts, lens, logits_rows = pack_prompts(

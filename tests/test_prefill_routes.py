@@ -73,3 +73,47 @@ def test_a_bias_behind_a_row_parallel_projection_is_added_by_the_layer(plain, wh
 def test_switches_of_the_routes_that_a_call_contains(plain, monkeypatch, switch):
     monkeypatch.setenv(switch, "1")
     assert not plain.issued()
+
+
+@pytest.fixture
+def grid(plain):
+    """Whether two prompts of 2 and 5 tokens on a grid of 10 run packed through the model."""
+    from lite_llama_amd.executor.slots import PromptGrid
+
+    info = types.SimpleNamespace(b_seq_len=torch.tensor([2, 5]), b_start_loc=torch.arange(2, dtype=torch.int32) * 5,
+                                 cur_select_index=torch.arange(10, dtype=torch.int32), max_actual_seq_len=5)
+    info.prompt_grid = PromptGrid(info, [2, 5])
+    ids, positions, last = torch.zeros(2, 5, dtype=torch.int64), torch.arange(5).expand(2, 5), torch.tensor([1, 9])
+    assert plain.model._packs(ids, positions, info, last)
+    return types.SimpleNamespace(model=plain.model, packs=lambda: plain.model._packs(ids, positions, info, last))
+
+
+@pytest.mark.parametrize("at", ["embed_tokens", "layers.1", "layers.0.self_attn.attn", "layers.1.mlp.down_proj"])
+@pytest.mark.parametrize("hook", ["register_forward_hook", "register_forward_pre_hook", "register_full_backward_hook"])
+def test_hooks_see_the_grid(grid, at, hook):
+    handle = getattr(grid.model.get_submodule(at), hook)(lambda *a: None)
+    assert not grid.packs()
+    handle.remove()
+    assert grid.packs()
+
+
+def test_modules_of_other_origin_see_the_grid(grid):
+    model, attention = grid.model, grid.model.layers[0].self_attn
+
+    class Other(type(attention)):
+        pass
+
+    handle = torch.nn.modules.module.register_module_forward_hook(lambda *a: None)
+    assert not grid.packs()
+    handle.remove()
+    model.layers[0].self_attn = nn.Identity()
+    assert not grid.packs()
+    model.layers[0].self_attn = attention
+    attention.__class__ = Other
+    assert not grid.packs()
+    attention.__class__ = Other.__bases__[0]
+    model.layers[1].forward = types.MethodType(type(model.layers[1]).forward, model.layers[1])
+    assert not grid.packs()
+    del model.layers[1].forward
+    model.register_forward_hook(lambda *a: None)   # (the model's own inputs and logits are the same either way)
+    assert grid.packs()
