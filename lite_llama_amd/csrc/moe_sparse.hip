@@ -129,8 +129,8 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const void* __restri
 }
 
 // The choice of one token's experts from its logits, by one wave (`lane` of 64; LDS operations of a wave complete in order, so its lanes need no
-// barrier between them).  LDS per token: scores [E], plain scores [E], group score [G], group kept [G], chosen scores [top], chosen
-// experts [top].  SCORING 0: sigmoid scores, weights = chosen / sum; 1: the logits themselves rank the experts (no groups) and the weights are
+// barrier between them).  LDS per token: scores [E], group score [G], group kept [G], chosen scores [top], and for SCORING 2 plain scores [E]
+// (4096 experts, 4096 groups and 64 slots stay below the 64 KB of a launch).  SCORING 0: sigmoid scores, weights = chosen / sum; 1: the logits themselves rank the experts (no groups) and the weights are
 // the softmax over the chosen logits alone; 2: scores = softmax over ALL logits (no groups), the experts are ranked by score + correction[e],
 // the weights are the chosen scores themselves (not renormalised); the last `identity` experts have no weights of their own -- a slot that
 // chose one keeps its id (>= experts - identity, which the sort by expert never places) and its score is added to extra_scale[t], the factor
@@ -144,7 +144,9 @@ struct SelectArgs {
   float* extra_scale;
   const void* correction;
 };
-static size_t select_floats(int experts, int group_count, int top) { return (size_t)2 * experts + 2 * group_count + 2 * top; }
+__host__ __device__ static inline size_t select_floats(int scoring, int experts, int group_count, int top) {
+  return (size_t)(scoring == 2 ? 2 : 1) * experts + 2 * group_count + top;
+}
 
 __device__ __forceinline__ void select_settle() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
@@ -152,11 +154,10 @@ template <int SCORING, int DT>
 __device__ __forceinline__ void select_token(const SelectArgs& p, const float* z, int64_t t, float* lds, int lane) {
   const int experts = p.experts, top = p.top;
   float* score = lds;
-  float* plain = score + experts;
-  float* gscore = plain + experts;
+  float* gscore = score + experts;
   float* gkeep = gscore + p.group_count;
   float* chosen = gkeep + p.group_count;
-  int* chosen_id = reinterpret_cast<int*>(chosen + top);
+  float* plain = SCORING == 2 ? chosen + top : score;
   if constexpr (SCORING == 2 || SCORING == 4) {
     // softmax over all experts: every lane adds the exponentials in index order (one value for the whole wave)
     float top_z = -INFINITY;
@@ -190,8 +191,7 @@ __device__ __forceinline__ void select_token(const SelectArgs& p, const float* z
     auto place = [&](int e, int rank) {
       if (e < experts && rank < top) {
         p.ids[t * top + rank] = e;
-        chosen_id[rank] = e;
-        chosen[rank] = plain[e];
+        chosen[rank] = e >= experts - p.identity ? plain[e] : 0.f;   // (what the token's own row is scaled by)
         p.weights[t * top + rank] = plain[e] * p.route_scale;
       }
     };
@@ -223,7 +223,7 @@ __device__ __forceinline__ void select_token(const SelectArgs& p, const float* z
     if (p.extra_scale) {                      // slots in rank order: the same sum whatever lane found which slot
       float own = 0.f;
 #pragma unroll 8
-      for (int k = 0; k < top; ++k) own += chosen_id[k] >= experts - p.identity ? chosen[k] : 0.f;
+      for (int k = 0; k < top; ++k) own += chosen[k];
       if (lane == 0) p.extra_scale[t] = own * p.route_scale;
     }
     return;
@@ -361,7 +361,7 @@ __global__ __launch_bounds__(64 * NW) void router_kernel(const void* __restrict_
   }
   __syncthreads();
   if (wave < TW && t0 + wave < n) {
-    const int64_t each = (int64_t)2 * p.experts + 2 * p.group_count + 2 * p.top;
+    const int64_t each = (int64_t)select_floats(SCORING, p.experts, p.group_count, p.top);
     select_token<SCORING, DT>(p, lds + wave * rows, t0 + wave, lds + TW * rows + wave * each, lane);
   }
 }
@@ -762,7 +762,7 @@ extern "C" int ll_group_router(const void* h, int64_t h_ld, const void* w_router
   const bool aligned = width % vec == 0 && h_ld % vec == 0 && ll_aligned16(h) && ll_aligned16(w_router) && (!w_extra || ll_aligned16(w_extra));
   hipStream_t st = (hipStream_t)stream;
   const SelectArgs p{rows, (int)experts, (int)top, (int)group_count, (int)group_keep, (int)identity, route_scale, ids, weights, extra_scale, correction};
-  const size_t each = select_floats((int)experts, (int)group_count, (int)top);
+  const size_t each = select_floats(scoring, (int)experts, (int)group_count, (int)top);
   if (rows <= kRouterRows) {
     const int tw = n > 256 ? 4 : 1, nw = tw == 1 && rows > 40 ? 16 : 8;   // tokens per workgroup; waves
     const dim3 grid((unsigned)((n + tw - 1) / tw));

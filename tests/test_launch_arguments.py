@@ -15,14 +15,15 @@ RUNTIME = r"""
 #include <string.h>
 static int launches = 0;
 static dim3 cfg_grid, cfg_block;
+static size_t cfg_lds = 0;
 extern "C" {
 void** __hipRegisterFatBinary(void*) { static void* h; return &h; }
 void __hipRegisterFunction(void**, const void*, char*, const char*, unsigned, void*, void*, void*, void*, int*) {}
 void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
 void __hipUnregisterFatBinary(void**) {}
-hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t, hipStream_t) { cfg_grid = g; cfg_block = b; return hipSuccess; }
+hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t s, hipStream_t) { cfg_grid = g; cfg_block = b; cfg_lds = s; return hipSuccess; }
 hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* s, hipStream_t* st) {
-  *g = cfg_grid; *b = cfg_block; *s = 0; *st = nullptr;
+  *g = cfg_grid; *b = cfg_block; *s = cfg_lds; *st = nullptr;
   return hipSuccess;
 }
 hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
@@ -232,3 +233,29 @@ def test_expert_blocks_of_256_are_taken_where_they_fill_the_chip(experts, top, h
 
     w1, w2 = (torch.empty(experts, *s, dtype=torch.int8, device="meta") for s in ((2 * inter, hidden), (hidden, inter)))
     assert _tiles_256_pay(tokens * top, experts, w1, w2, int8) == pays
+
+
+ROUTER = r"""
+static unsigned most_lds = 0;
+bool moe_stream_wants(const MoeStreamParams&, int, int, int, int64_t) { return false; }
+int moe_stream_launch(const MoeStreamParams&, int, int, int, int64_t, hipStream_t) { return LL_OK; }
+extern "C" {
+hipError_t hipLaunchKernel(const void*, dim3, dim3, void**, size_t lds, hipStream_t) {
+  if (lds > most_lds) most_lds = lds;
+  return hipSuccess;
+}
+unsigned router_lds() { const unsigned n = most_lds; most_lds = 0; return n; }
+}
+"""
+
+
+def test_every_router_that_is_accepted_fits_the_lds_of_a_launch(tmp_path):
+    lib = _host_library(tmp_path, "moe_sparse.hip", ROUTER)
+    P, L, I, F = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_float
+    lib.ll_group_router.argtypes = [P, L, P, P, L, L, L, L, L, L, F, I, P, P, P, P, P, L, I, P]
+    for scoring in range(5):
+        for experts, groups, top in [(4096, 4096, 64), (4096, 1, 64), (4096, 2048, 64), (513, 513, 64), (512, 512, 64), (511, 511, 64), (64, 64, 64)]:
+            groups = 1 if scoring in (1, 2) else groups
+            for tokens in (1, 300):
+                assert lib.ll_group_router(4096, 64, 4096, None, tokens, 64, experts, top, groups, groups, 1.0, scoring, *[4096] * 4, None, 0, 1, None) == 0
+                assert 0 < lib.router_lds() <= 64 * 1024, (scoring, experts, groups, tokens)

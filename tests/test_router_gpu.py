@@ -46,3 +46,27 @@ def test_choice(n, width, experts, scoring, dtype):
     else:
         mine = torch.where(want >= experts - identity, chosen, torch.zeros_like(chosen)).sum(-1) * route_scale
         assert (own[clear].to(F64) - mine[clear]).abs().max() <= 2e-5
+
+
+@pytest.mark.parametrize("scoring", ["sigmoid", "softmax_chosen", "softmax_all", "sigmoid_plain", "softmax_groups"])
+@pytest.mark.parametrize("experts,top", [(4096, 64), (513, 4)])
+def test_the_largest_choices(scoring, experts, top):
+    """As many experts, groups of one and slots as are accepted: their tables are as large as a launch's LDS allows."""
+    from lite_llama_amd.kernels.fused_moe import group_router
+
+    g = torch.Generator(device=DEV).manual_seed(experts)
+    h = torch.randn(3, 64, generator=g, device=DEV)
+    w = torch.randn(experts, 64, generator=g, device=DEV) * 0.25
+    groups = 1 if scoring in ("softmax_chosen", "softmax_all") else experts
+    ids, weights, own = group_router(h, w, top, groups, groups, scoring=scoring, **({"identity": 1000 if experts > 1000 else 5} if scoring == "softmax_all" else {}))
+    z = h.to(F64) @ w.to(F64).T
+    score = z if scoring == "softmax_chosen" else torch.sigmoid(z) if scoring.startswith("sigmoid") else torch.softmax(z, -1)
+    best, want = z.topk(top, -1)                 # (every score rises with its logit)
+    clear = (z.topk(top + 1, -1).values.diff(dim=-1).abs() > 1e-5).all(-1)
+    assert clear.any() and torch.equal(ids[clear].long(), want[clear])
+    chosen = score.gather(1, want)
+    weight = {"softmax_chosen": torch.softmax(best, -1), "softmax_all": chosen, "sigmoid_plain": chosen}.get(scoring, chosen / chosen.sum(-1, keepdim=True))
+    assert (weights[clear].to(F64) - weight[clear]).abs().max() <= 2e-5
+    if scoring == "softmax_all":
+        mine = torch.where(want >= experts - (1000 if experts > 1000 else 5), chosen, torch.zeros_like(chosen)).sum(-1)
+        assert (own[clear].to(F64) - mine[clear]).abs().max() <= 2e-5
