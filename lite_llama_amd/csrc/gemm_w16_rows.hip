@@ -10,7 +10,7 @@
 //     address: fragment reads are conflict free; weights non-temporal.  CONSUMERS, one per row group of the tile, run the unit's MFMA
 //     32x32x16 from LDS fragments and keep the tile's accumulators (16 x MT registers) for the whole K loop: no cross-wave exchange.
 //     The loaders run ahead ACROSS tile boundaries, so a tile's epilogue overlaps the next tile's first units.
-//   * Long streams of rows a multiple of 4 KB long: workgroup b begins every tile at unit b mod units and wraps.  All of them beginning at
+//   * Long streams of rows a multiple of 4 KB long: workgroup b begins every tile b steps of 256 bytes into its rows and wraps.  All of them beginning at
 //     column 0 ask the same few memory channels (us for 600 MB, 1 row, all from column 0 -> staggered: K = 2048 113 -> 94, 4096 127 -> 98,
 //     8192 139 -> 124; staggered within an XCD instead, b / 8: 98, 106, 124.  K = 3584: 90 -> 91, 37888 rows of it 50 -> 52).  Sums of 16-bit products in
 //     another order round otherwise, so streams under 256 MB, which gain little or nothing (32 rows, K = 2048: 134 MB 31 -> 28 us, 46 MB
@@ -98,8 +98,10 @@ __global__ __launch_bounds__((R16Lds<MT, WIDE>::THREADS)) __attribute__((amdgpu_
       xoff[j] = (uint32_t)(r * p.x_stride * 2 + slot * 16);
     }
     int issued = 0, t = 0, size = tbase + (trem > 0 ? 1 : 0), done = 0, c = 0;
-    if (p.stagger)
-      for (c = b; c >= p.chunks; c -= p.chunks) {}
+    if (p.stagger) {   // (WIDE units are half as long: two of them per step, so that a row's sum begins at the same column in either form)
+      for (c = b; c >= p.chunks * KB / 256; c -= p.chunks * KB / 256) {}
+      c *= 256 / KB;
+    }
     const char* wt = (const char*)p.w + (size_t)(lo + L * GL) * 32 * (size_t)p.w_stride * 2;   // this wave's rows of the tile
     uint32_t dst = 0;
     auto issue = [&]() {

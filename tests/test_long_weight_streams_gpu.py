@@ -8,7 +8,8 @@ DEV = "cuda"
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("n,k", [(65536 + 32, 2048), (32768, 4224), (262144 * 4, 128)])   # (one chunk only: nothing to wrap)
+# (rows a multiple of 4 KB: every workgroup of its own column; the last two, 256 MB as well, are of other rows: all from column 0)
+@pytest.mark.parametrize("n,k", [(65536 + 32, 2048), (32768 + 96, 4096), (8192, 16384), (32768, 4224), (262144 * 4, 128)])
 @pytest.mark.parametrize("m", [1, 33])
 def test_staggered_rows(dtype, n, k, m):
     from lite_llama_amd.kernels.quantization import dense16_rows_linear
@@ -21,6 +22,20 @@ def test_staggered_rows(dtype, n, k, m):
     # one rounding to the storage dtype; fp32 sums of k products of size ~ k^-1/2 in another order: far below 2^-14
     unit = 2.0 ** (-11 if dtype == torch.float16 else -8)
     assert ((got.float() - want).abs() <= unit * want.abs() + 2.0 ** -14).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n,k", [(65536 + 32, 2048), (33792 + 32, 4096)])
+def test_a_rows_sums_do_not_depend_on_how_many_rows_there_are(dtype, n, k):
+    """Tiles of four and of eight row groups (up to 32 rows, more) begin a staggered weight's rows at the same column."""
+    from lite_llama_amd.kernels.quantization import dense16_rows_linear
+
+    g = torch.Generator(device=DEV).manual_seed(n)
+    w = (torch.randn(n, k, generator=g, device=DEV) * k ** -0.5).to(dtype)
+    x = torch.randn(64, k, generator=g, device=DEV).to(dtype)
+    every = dense16_rows_linear(x, w)
+    for m in (1, 32, 33):
+        assert torch.equal(dense16_rows_linear(x[:m], w), every[:m])
 
 
 def test_staggered_int8_rows():
