@@ -651,6 +651,19 @@ __device__ __forceinline__ void st8(void* p, int64_t i, const float (&o)[8]) {
   }
 }
 
+// v * scale -> storage bits, the last step of a long part's norm: for fp16 one rounding of the exact product, in one instruction that both forms
+// below name (left to the compiler, the form of two values at a time rounded to fp32 first, and the bits hung on the rows' alignment)
+template <int DT>
+__device__ __forceinline__ uint16_t scaled_bits(float v, float scale) {
+  if constexpr (DT == LL_F16) {
+    uint32_t r;
+    asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(r) : "v"(scale), "v"(v));
+    return (uint16_t)r;
+  } else {
+    return from_f32<DT>(v * scale);
+  }
+}
+
 // The read-out norm for long parts off 16-byte borders or beyond 8192 channels: one workgroup per (token, part), same arithmetic per element as
 // the wave form.
 template <int DT>
@@ -683,7 +696,8 @@ __global__ __launch_bounds__(256) void gated_out_norm_block_kernel(void* __restr
     if (gate_first) v *= g;
     v = v * inv * (w ? ldv<DT>(w, (c0 + cc) % w_len) : 1.0f);
     if (!gate_first) v *= g;
-    stv<DT>(out, t * out_ld + c0 + cc, v * out_scale);
+    if constexpr (DT == LL_F32) ((float*)out)[t * out_ld + c0 + cc] = v * out_scale;
+    else ((uint16_t*)out)[t * out_ld + c0 + cc] = scaled_bits<DT>(v, out_scale);
   }
 }
 
@@ -766,9 +780,18 @@ __global__ __launch_bounds__(256) void gated_out_norm_vec_kernel(void* __restric
       for (int e = 0; e < 8; ++e) {
         float y = v[j][e] * inv * wv[j][e];
         if (!gate_first) y *= g[j][e];
-        v[j][e] = y * out_scale;
+        v[j][e] = y;
       }
-      st8<DT>(out, t * out_ld + c0 + cc, v[j]);
+      if constexpr (TP == 256 && DT != LL_F32) {
+        U16x8 u;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) u.v[e] = scaled_bits<DT>(v[j][e], out_scale);
+        *reinterpret_cast<U16x8*>((uint16_t*)out + t * out_ld + c0 + cc) = u;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[j][e] *= out_scale;
+        st8<DT>(out, t * out_ld + c0 + cc, v[j]);
+      }
     }
   }
 }

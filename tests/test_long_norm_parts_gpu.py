@@ -33,11 +33,7 @@ def test_long_parts(dtype, parts, ps, w_len, gate, first):
     unit = {torch.float32: 0.0, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dtype]
     assert ((out[:, 8:].to(F64) - y).abs() <= (32 * 2.0 ** -24 + unit) * y.abs() + 2.0 ** -24).all()
     assert out[:, :8].abs().max() == 0
-    # one element off the 16-byte borders: the plain form, the same bits -- but for fp16, where the compiler makes one instruction of the last product
-    # and its rounding in one of the forms (one rounding instead of two): a unit in the last place
+    # one element off the 16-byte borders: the plain form, the same bits
     off = torch.zeros(n, width + 9, device=DEV, dtype=dtype)
     gated_out_norm(o, w, eps, parts=parts, gate=wide[:, 8:] if gate else None, gate_kind=gate, gate_first=first, scale=scale, out=off[:, 9:])
-    if dtype == torch.float16:
-        assert ((off[:, 9:].to(F64) - out[:, 8:].to(F64)).abs() <= 2.0 ** -10 * y.abs() + 2.0 ** -24).all()
-    else:
-        assert torch.equal(off[:, 9:], out[:, 8:])
+    assert torch.equal(off[:, 9:], out[:, 8:])
