@@ -817,7 +817,7 @@ int ll_moe_rows_gemm(const void* a, int64_t a_ld, int64_t a_div, const void* w, 
  * of the step brings (0: unknown); sizes the staging buffers, and 1 selects the form for decoded tokens.
  * ll_linear_scan_walk: the same bits over runs of many tokens, in two kernels.  walk_scratch: ll_linear_scan_walk_floats(...) fp32,
  * 16-byte aligned (0: not served, use ll_linear_scan): up to 2^28 of them -- 8 bytes per token and key entry, 4 more per token, head and
- * key entry for kind 1, 4 per token and value column (a head's rounded up to 32), for eight tokens more than there are.
+ * key entry for kind 1 -- and 4 bytes per token and value column (a head's rounded up to 32), for eight tokens more than there are.
  * ll_gated_out_norm: o fp32 [n, width] -> RMS norm over `parts` equal consecutive parts, times w[(channel) mod w_len] (NULL:
  * none), times act(gate) (gate_kind 0 none, 1 silu, 2 sigmoid; gate_first: before the norm), times out_scale -> out rows of
  * stride out_ld.

@@ -938,7 +938,7 @@ __global__ __launch_bounds__(256) void rownorm_rope_cache_vec_kernel(
 
 }  // namespace
 
-constexpr int64_t kWalkFloats = 1ll << 28;   // largest scratch of the two-kernel walk (1 GiB)
+constexpr int64_t kWalkFloats = 1ll << 28;   // most pairs, decays and steps in the scratch of the two-kernel walk (1 GiB)
 
 #define LL_BY_DTYPE(dtype, CALL)                  \
   do {                                            \
@@ -959,9 +959,12 @@ extern "C" int64_t ll_linear_scan_walk_floats(int64_t n, int64_t batch, int64_t 
   if (n < 1 || batch < 1 || batch > 65535 || heads < 1 || heads > 65535 || (dk != 64 && dk != 128 && dk != 256) || dv < 1 || qk_rep < 1 || heads % qk_rep ||
       longest_run < 24)
     return 0;
-  // (a token's columns: at most 65535 workgroups of 1024 for its terms)
-  const int64_t per = heads / qk_rep * dk * 2 + (kind == 1 ? heads * dk : 0) + (kind == 2 ? heads * 2 : 0) + heads * walk_columns(dv);
-  return per > kWalkFloats / (n + kTB) || per > 65535ll * 1024 ? 0 : (n + kTB) * per;   // (a last stage is read whole: spare rows)
+  const int64_t terms = heads / qk_rep * dk * 2 + (kind == 1 ? heads * dk : 0) + (kind == 2 ? heads * 2 : 0);
+  const int64_t values = heads * walk_columns(dv), per = terms + values;
+  // The values take no more than twice the step's fp32 results, so only short heads' are bounded by themselves.  (A token's columns: at
+  // most 65535 workgroups of 1024 for its terms)
+  if (terms > kWalkFloats / n || (walk_columns(dv) > 2 * dv && values > kWalkFloats / n) || per > 65535ll * 1024) return 0;
+  return (n + kTB) * per;   // (a last stage is read whole: spare rows)
 }
 
 static int linear_scan(const void* q, int64_t q_ld, const void* k, int64_t k_ld, const void* v, int64_t v_ld, int64_t heads,

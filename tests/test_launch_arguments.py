@@ -259,3 +259,16 @@ def test_every_router_that_is_accepted_fits_the_lds_of_a_launch(tmp_path):
             for tokens in (1, 300):
                 assert lib.ll_group_router(4096, 64, 4096, None, tokens, 64, experts, top, groups, groups, 1.0, scoring, *[4096] * 4, None, 0, 1, None) == 0
                 assert 0 < lib.router_lds() <= 64 * 1024, (scoring, experts, groups, tokens)
+
+
+# (tokens, heads, key heads, key width, value width, kind): the longest steps, a little below 2^28 floats of pairs, decays and steps
+@pytest.mark.parametrize("n,heads,qk_heads,dk,dv,kind", [(65000, 16, 16, 128, 128, 0), (43000, 8, 8, 256, 256, 1), (130000, 8, 8, 128, 256, 0),
+                                                         (64000, 32, 16, 128, 64, 2), (500000, 8, 4, 64, 64, 2), (24, 4096, 4096, 256, 512, 1)])
+def test_long_steps_keep_the_walk_in_two_kernels(linear_mix, n, heads, qk_heads, dk, dv, kind):
+    fn = linear_mix.ll_linear_scan_walk_floats
+    fn.argtypes, fn.restype = [ctypes.c_int64] * 6 + [ctypes.c_int, ctypes.c_int64], ctypes.c_int64
+    terms = qk_heads * dk * 2 + (heads * dk if kind == 1 else 0) + (heads * 2 if kind == 2 else 0)
+    assert 0.7 * 2 ** 28 < n * terms <= 2 ** 28 or n == 24
+    assert fn(n, 4, heads, dk, dv, heads // qk_heads, kind, n // 4 + 24) == (n + 8) * (terms + heads * -(-dv // 32) * 32)
+    assert fn(2 ** 28 // terms + 1, 4, heads, dk, dv, heads // qk_heads, kind, 1000) == 0
+    assert fn(n, 4, heads, dk, dv, heads // qk_heads, kind, 23) == 0

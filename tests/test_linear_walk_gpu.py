@@ -88,6 +88,22 @@ def test_runs_of_many_tokens_in_two_columns_per_thread(kind, heads, qk_heads, dk
     test_runs_of_many_tokens(torch.bfloat16, kind, heads, qk_heads, dk, dv, runs)
 
 
+def test_a_step_whose_scratch_passes_a_gigabyte():
+    """Terms below 2^28 floats, terms and values above: the same bits as the walk in one kernel, at the far end of the scratch too."""
+    from lite_llama_amd import _lib
+    from lite_llama_amd.kernels.recurrent import linear_scan
+
+    heads, dk, dv, runs = 16, 128, 128, [(0, 47000), (3, 24), (9, 1), (0, 975)]
+    n = sum(c for _, c in runs)
+    q, k, v, kw = _inputs("fixed", heads, heads, dk, dv, n, torch.bfloat16, 3)
+    step = _step([(i, f, c, 0) for i, (f, c) in enumerate(runs)], None)
+    assert _lib.lib().ll_linear_scan_walk_floats(n, len(runs), heads, dk, dv, 1, 0, step.longest_run) > 2 ** 28
+    start = torch.randn(len(runs), heads, dk, dv, device=DEV)
+    states = [start.clone(), start.clone()]
+    outs = [linear_scan(q, k, v, heads, dk, dv, dataclasses.replace(step, longest_run=m), s, **kw) for m, s in zip((step.longest_run, 0), states)]
+    assert torch.equal(outs[0], outs[1]) and torch.equal(states[0], states[1])
+
+
 @pytest.mark.parametrize("dv", [16, 320])   # one state column per thread, two
 def test_a_run_without_tokens_leaves_the_state_it_started_from(dv):
     """Zeros where it starts at position 0, whatever an earlier owner of the slot left; as in the walk in one kernel."""
