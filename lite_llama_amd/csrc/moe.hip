@@ -737,6 +737,22 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel2(const MoeParams p) {
   }
 }
 
+// Rows per expert up to which the weights as one stream per CU (moe_stream.hip) are the faster form here: rows of an expert beyond its first piece
+// stream its weights again, and the tiles are the better the more of them there are.  us, tiles / stream, both products, random choices:
+//   16 bits 128 experts of 2048 / 768, 16 rows 258 / 239, 22 260 / 260, 28 268 / 278, 64 403 / 451; 200 of 2048 / 512, 22 289 / 285, 28 299 / 307; 96 of 2048 / 768, 32
+//           222 / 219, 40 230 / 235; 64 of 2048 / 1024, 32 201 / 183, 48 208 / 206, 64 271 / 315; 48 of 2048 / 1408, 32 198 / 200, 40 206 / 213; fewer:
+//           16 of 2048 / 1024, 56 81 / 72, 64 85 / 88; 8 of 4096 / 14336, 40 599 / 563, 56 611 / 582 and 651 / 693, 64 769 / 846
+//   8 bits  128 of 2048 / 768, 18 175 / 164, 20 177 / 183; 128 of 4096 / 1536, 18 590 / 542; 200 of 2048 / 512, 18 195 / 191, 24 202 / 206;
+//           128 of 1024 / 512, 12 80 / 77, 14 81 / 84, 18 83 / 85; up to 96: 96 of 2048 / 768, 24 152 / 150, 28 157 / 162; 64, 22 105 / 104, 28 108 / 124;
+//           32, 24 67 / 57, 28 69 / 66, 32 75 / 78; 16 of 2048 / 1024, 24 59 / 46, 36 61 / 65; 8 of 4096 / 14336, 24 422 / 344, 32 431 / 449
+//   where the tiles leave half the CUs idle: 4 of 1024 / 512, 32 rows, 16 bits 30 / 27, 8 bits 31 / 27, 80 36 / 27, 38 / 31; 8 of 2048 / 768, 80 59 / 52, 59 / 50
+//   where they cannot read whole lines: 34 of 2048 / 704, 16 bits, 64 178 / 129, 100 225 / 169
+static int64_t moe_stream_most_rows(int64_t experts, int64_t n, int64_t k, int wfmt, bool lines) {
+  const bool few = (n + 127) / 128 * experts <= 128;   // (tiles)
+  if (wfmt == LL_W_F16) return few || !lines ? 80 : experts > 96 ? 22 : experts > 40 ? 32 : 56;
+  return few ? 32 : experts <= 96 ? 24 : n * k > (1 << 20) ? 18 : 12;
+}
+
 extern "C" int ll_moe_gemm(void* c, const void* a, const void* w, const float* w_scale, const void* topk_w,
                            const int32_t* sorted_ids, const int32_t* expert_ids, const int32_t* num_post,
                            int64_t num_slots, int64_t em, int block_m, int64_t n, int64_t k, int top_k,
@@ -769,10 +785,15 @@ extern "C" int ll_moe_gemm(void* c, const void* a, const void* w, const float* w
     t.w_stride_e = w_stride_e; t.s_stride_e = s_stride_e; t.num_slots = (int)num_slots; t.top_k = top_k;
     return tile256_grouped_launch(t, wfmt, stream);
   }
-  if (num_slots < (1ll << 30) && n <= (1 << 24) && k <= (1 << 24)) {   // few rows per expert: the weights as one stream per CU
+  static const bool v1_forced = getenv("LL_MOE_V1") != nullptr;  // A/B knob, read once
+  const bool lines = !v1_forced && k % 128 == 0 && (w_stride_n * (wfmt == LL_W_F16 ? 2 : 1)) % 16 == 0 &&
+                     (w_stride_e * (wfmt == LL_W_F16 ? 2 : 1)) % 16 == 0 && ll_aligned16(w) && ll_aligned16(a) &&
+                     (wfmt == LL_W_F16 || group_k % 64 == 0);
+  const int64_t spare = (em - num_slots) / (block_m - 1), experts = spare > 1 ? spare : 1;   // (em: the slots and block_m - 1 entries per expert)
+  if (num_slots <= moe_stream_most_rows(experts, n, k, wfmt, lines) * experts && num_slots < (1ll << 30) && n <= (1 << 24) && k <= (1 << 24)) {
     const int eb = wfmt == LL_W_F16 ? 2 : 1, form = wfmt == LL_W_F16 ? MS_W16 : wfmt == LL_W_FP8E4M3 ? MS_FP8 : MS_INT8;
     const int mode = mul_routed_weight & 2 ? MS_GLU_ROUNDED : MS_SCALED;
-    const int64_t experts = em / block_m + 1;   // (what the lists hold: at least as many runs as there are)
+    const int64_t runs = em / block_m + 1;   // (whatever em is: the lists hold no more blocks)
     MoeStreamParams t{};
     t.out = (uint16_t*)c; t.a = (const uint16_t*)a; t.w = (const unsigned char*)w; t.scales = w_scale;
     t.weight16 = mul_routed_weight & 1 ? (const uint16_t*)topk_w : nullptr;
@@ -780,7 +801,7 @@ extern "C" int ll_moe_gemm(void* c, const void* a, const void* w, const float* w
     t.a_ld = a_stride_m; t.out_ld = mul_routed_weight & 2 ? n / 2 : n; t.w_stride_e = w_stride_e * eb; t.w_stride_n = w_stride_n * eb;
     t.s_stride_e = s_stride_e; t.s_stride_n = s_stride_n; t.s_stride_k = s_stride_k; t.group_n = group_n; t.group_k = group_k;
     t.K = (int)k; t.N = (int)n; t.num_slots = (int)num_slots; t.a_div = top_k; t.block_m = block_m; t.safe = (int)em;
-    if (em < (1ll << 31) && moe_stream_wants(t, form, mode, LL_F16, experts)) return moe_stream_launch(t, form, mode, LL_F16, experts, (hipStream_t)stream);
+    if (em < (1ll << 31) && moe_stream_wants(t, form, mode, LL_F16, experts, runs)) return moe_stream_launch(t, form, mode, LL_F16, experts, (hipStream_t)stream);
   }
   MoeParams p{};
   p.c = (uint16_t*)c; p.a = (const uint16_t*)a; p.w = w; p.w_scale = w_scale; p.topk_w = (const uint16_t*)topk_w;
@@ -791,10 +812,6 @@ extern "C" int ll_moe_gemm(void* c, const void* a, const void* w, const float* w
   p.s_stride_e = s_stride_e; p.s_stride_n = s_stride_n; p.s_stride_k = s_stride_k;
   dim3 grid((unsigned)((n + 127) / 128), (unsigned)((em + block_m - 1) / block_m));
   hipStream_t st = (hipStream_t)stream;
-  static const bool v1_forced = getenv("LL_MOE_V1") != nullptr;  // A/B knob, read once
-  const bool lines = !v1_forced && k % 128 == 0 && (w_stride_n * (wfmt == LL_W_F16 ? 2 : 1)) % 16 == 0 &&
-                     (w_stride_e * (wfmt == LL_W_F16 ? 2 : 1)) % 16 == 0 && ll_aligned16(w) && ll_aligned16(a) &&
-                     (wfmt == LL_W_F16 || group_k % 64 == 0);
   // 128-row blocks (round 6: prefill-sized inputs, hundreds of rows per expert): the full-line form only -- a weight tile is
   // dequantised once for four MFMA row tiles and re-read from L2 half as often as with 64-row blocks
   if (block_m == 128 && !lines) return LL_ERR_SHAPE;

@@ -877,7 +877,7 @@ extern "C" int ll_moe_rows_gemm(const void* a, int64_t a_ld, int64_t a_div, cons
   static const bool no_mfma = getenv("LL_MOE_ROWS_VALU") != nullptr;   // A/B knob, read once
   const bool mfma = !no_mfma && dtype != LL_F32 && K % 8 == 0 && a_ld % 8 == 0 && w_stride_e % 8 == 0 && ll_aligned16(a) && ll_aligned16(w);
   if (block == 128 && mfma) {
-    if (num_slots < (1ll << 30) && N <= (1 << 24) && K <= (1 << 24)) {   // few rows per expert: the weights as one stream per CU
+    if (num_slots <= 36 * experts && num_slots < (1ll << 30) && N <= (1 << 24) && K <= (1 << 24)) {   // few rows per expert: the weights as one stream per CU (moe_stream.hip: figures)
       const int form = mode == 1 ? MS_GLU : mode == 2 ? MS_RELU2 : MS_SCALED;
       MoeStreamParams t{};
       t.out = (uint16_t*)out; t.a = (const uint16_t*)a; t.w = (const unsigned char*)w; t.weight32 = mode == 1 ? nullptr : slot_weight;
@@ -885,7 +885,7 @@ extern "C" int ll_moe_rows_gemm(const void* a, int64_t a_ld, int64_t a_div, cons
       t.a_ld = a_ld; t.out_ld = out_ld; t.w_stride_e = w_stride_e * 2; t.w_stride_n = K * 2; t.K = (int)K; t.N = (int)N;
       t.num_slots = (int)num_slots; t.a_div = (int)a_div; t.block_m = (int)block; t.limit = glu_limit;
       t.safe = (int)(num_slots + experts * (block - 1));
-      if (moe_stream_wants(t, MS_W16, form, dtype, experts)) return moe_stream_launch(t, MS_W16, form, dtype, experts, st);
+      if (moe_stream_wants(t, MS_W16, form, dtype, experts, experts)) return moe_stream_launch(t, MS_W16, form, dtype, experts, st);
     }
     const int64_t tiles_n = (N + (mode == 1 ? 63 : 127)) / (mode == 1 ? 64 : 128), max_tiles = most * tiles_n;
     if (max_tiles > 0x7ffffff0ll) return LL_ERR_SHAPE;

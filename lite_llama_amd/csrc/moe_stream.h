@@ -30,6 +30,7 @@ struct MoeStreamParams {
   int k_shift;                  // set by the launch
 };
 
-// whether the streaming form takes this call
-bool moe_stream_wants(const MoeStreamParams& p, int wfmt, int mode, int dtype, int64_t experts);
+// whether the streaming form can take this call (how many rows per expert it pays for depends on the caller's other form); runs: of row blocks with the
+// same expert there are no more than this many (the experts, or what is known of them)
+bool moe_stream_wants(const MoeStreamParams& p, int wfmt, int mode, int dtype, int64_t experts, int64_t runs);
 int moe_stream_launch(const MoeStreamParams& p, int wfmt, int mode, int dtype, int64_t experts, hipStream_t stream);

@@ -17,7 +17,8 @@
 //   us for both products, tiles -> here.  8-bit floats, 128 experts of 2048 / 768, top 8: 1 token 42 -> 24, 8 67 -> 54, 32 120 -> 102, 64
 //   137 -> 117 (604 MB: 5.2 TB/s); in pieces of 32 rows (of 16) 200 167 -> 155 (167), 256 178 -> 162 (209), 320 181 -> 168, 400 186 -> 191.  bf16, 34 of 2048 / 704, top 4: 1 token 33 -> 17, 32 tokens 77 -> 58, 128 78 -> 65; 68 of 3072 / 512,
 //   top 8: 6 tokens 89 -> 74, 32 156 -> 111 (642 MB), 128 160 -> 126; in pieces of 64 rows 160 tokens 161 -> 131, 262 (31 rows per expert) 165 ->
-//   150 (pieces of 32: 185), 34 experts 200 77 -> 73, 300 (35) 78.5 -> 77, 400 (47) 80 -> 85: the rule of moe_stream_wants.
+//   150 (pieces of 32: 185), 34 experts 200 77 -> 73, 300 (35) 78.5 -> 77, 400 (47) 80 -> 85: up to 36 rows per expert in ll_moe_rows_gemm.  ll_moe_gemm has other
+//   tiles and lines of its own (moe.hip).
 #include <stdlib.h>
 
 #include "gemm_w4_common.h"
@@ -463,8 +464,13 @@ int ms_cus(int* lds) {
 
 int ms_lds(int wfmt, int rows) { return wfmt != MS_W16 ? (rows == 32 ? MsLds<MS_FP8, 2>::BYTES : MsLds<MS_FP8, 1>::BYTES) : rows == 64 ? MsLds<MS_W16, 4>::BYTES : MsLds<MS_W16, 2>::BYTES; }
 
-// rows of a piece: with 8-bit weights 16, or 32 where 8 and more meet an expert on average; with 16-bit ones 32, or 64 from 16 on
-int ms_rows(const MoeStreamParams& p, int wfmt, int64_t experts) { return wfmt != MS_W16 ? (p.num_slots > 8 * experts && p.block_m % 32 == 0 ? 32 : 16) : p.num_slots > 16 * experts ? 64 : 32; }
+// rows of a piece.  8-bit weights: 16, or 32 from 9 rows per expert on, beside many experts from 12 on (us, pieces of 16 / 32: 128 experts of 2048 / 768, 10 rows
+// 147 / 153, 12 160 / 156, 16 204 / 162; 200 of 2048 / 512, 12 170 / 181, 14 192 / 184; 64 of 2048 / 768, 10 76 / 77, 12 83 / 81; 32, 10 44 / 43, 12 52 / 49; 8,
+// 10 28 / 24).  16-bit ones: 32, or 64 from 16 on (128, 16 239 / 240, 24 271 / 265, 32 375 / 282)
+int ms_rows(const MoeStreamParams& p, int wfmt, int64_t experts) {
+  if (wfmt != MS_W16) return p.num_slots > (experts > 40 ? 12 : 9) * experts && p.block_m % 32 == 0 ? 32 : 16;
+  return p.num_slots > 16 * experts && p.block_m % 64 == 0 ? 64 : 32;
+}
 
 template <int DT, int WF, int MT, int MODE>
 int ms_go(const MoeStreamParams& p, int grid, hipStream_t stream) {
@@ -482,9 +488,9 @@ int ms_go(const MoeStreamParams& p, int grid, hipStream_t stream) {
 
 }  // namespace
 
-bool moe_stream_wants(const MoeStreamParams& p, int wfmt, int mode, int dtype, int64_t experts) {
+bool moe_stream_wants(const MoeStreamParams& p, int wfmt, int mode, int dtype, int64_t experts, int64_t runs) {
   static const bool off = getenv("LL_MOE_NO_STREAM") != nullptr;   // A/B knob, read once
-  if (off || (dtype != LL_F16 && (dtype != LL_BF16 || wfmt != MS_W16)) || experts > 65535) return false;
+  if (off || (dtype != LL_F16 && (dtype != LL_BF16 || wfmt != MS_W16)) || experts > 65535 || runs > 65535) return false;
   const int eb = wfmt == MS_W16 ? 2 : 1, rows = ms_rows(p, wfmt, experts);
   if (p.block_m % rows || p.K < 128 || (int64_t)p.K * eb % 16 || p.K > (1 << 24) || p.N < 16 || p.N > (1 << 24) || p.a_ld % 8 ||
       p.w_stride_n % 16 || p.w_stride_e % 16 || !ll_aligned16(p.a) || !ll_aligned16(p.w) || (mode == MS_GLU_ROUNDED && p.N % 2))
@@ -496,12 +502,10 @@ bool moe_stream_wants(const MoeStreamParams& p, int wfmt, int mode, int dtype, i
         ((int64_t)p.N * p.s_stride_n + p.K / 64 * p.s_stride_k) * 4 >= (1ll << 32))
       return false;
   }
-  // few rows per expert (figures above): pieces of 32 or 64 rows, of 16 or 32 with 8-bit weights; an expert's rows beyond its first piece stream the weights again
-  if (p.num_slots > (wfmt == MS_W16 ? 36 : rows == 32 ? 16 : 12) * experts) return false;
   int lds = 0;
   const int cus = ms_cus(&lds);
-  const int64_t most = ((int64_t)p.num_slots + (experts + 1) * (p.block_m - 1)) / rows + 1;
-  const int64_t filled = p.num_slots / rows + experts + 1;   // pieces with a slot
+  const int64_t most = ((int64_t)p.num_slots + (runs + 1) * (p.block_m - 1)) / rows + 1;
+  const int64_t filled = p.num_slots / rows + runs + 1;   // pieces with a slot
   return cus > 0 && filled <= MS_LIST && filled / cus + 2 <= MS_OWN && most <= 65535 && ms_lds(wfmt, rows) <= lds &&
          (filled + 1) * (((int64_t)p.N + 7) / 8) < (1ll << 30);
 }

@@ -105,3 +105,26 @@ def test_8_bit_experts(fmt, width, ff, experts, tokens, top, group, interleaved)
             # gate, up and their product are each rounded to fp16 (three half units, |silu'| <= 1.1), and so is the slot's result
             bound[t] += 2.0 ** -11 * (one.abs() + 6 * 3.3 * wt * ((d2[e] ** 2) @ act.abs().clamp(min=0.05) ** 2).sqrt())
     assert ((got.to(F64) - want).abs() <= bound + 2.0 ** -11 * want.abs() + 1e-6).all()
+
+
+@pytest.mark.parametrize("width,ff,experts,tokens,top", [(128, 144, 4, 48, 2), (264, 200, 4, 100, 2), (392, 128, 20, 130, 4), (256, 72, 2, 64, 1)])
+@pytest.mark.parametrize("interleaved", [False, True])
+def test_fp16_experts(width, ff, experts, tokens, top, interleaved):
+    """Blocks of 32 and 64 slots in pieces of 32 and 64 rows, experts of one piece and of two."""
+    from lite_llama_amd.kernels.fused_moe import fused_moe
+
+    g = torch.Generator(device=DEV).manual_seed(width + ff)
+    w1, w2 = ((torch.randn(experts, *s, generator=g, device=DEV) * s[1] ** -0.5).half() for s in ((2 * ff, width), (width, ff)))
+    x = torch.randn(tokens, width, generator=g, device=DEV).half()
+    ids, weights = _ids(tokens, experts, top, g, False), torch.rand(tokens, top, generator=g, device=DEV).half()
+    got = fused_moe(x, w1, w2, weights, ids, w1_interleaved=interleaved)
+    y = torch.einsum("enk,tk->ten", w1.double().cpu(), x.double().cpu()).to(DEV)   # (every expert of every token)
+    gate, u = (y[..., 0::2], y[..., 1::2]) if interleaved else (y[..., :ff], y[..., ff:])
+    act = torch.nn.functional.silu(gate) * u
+    out = torch.einsum("enk,tek->ten", w2.double().cpu(), act.cpu()).to(DEV)
+    spread = torch.einsum("enk,tek->ten", w2.double().cpu() ** 2, act.cpu().abs().clamp(min=0.05) ** 2).to(DEV).sqrt()
+    slot = torch.zeros(tokens, experts, dtype=F64, device=DEV).scatter_(1, ids.long(), weights.to(F64)).unsqueeze(-1)
+    want = (out * slot).sum(1)
+    # gate, up and their product are each rounded to fp16 (three half units, |silu'| <= 1.1), and so are a slot's result and the sum
+    bound = 2.0 ** -11 * ((out.abs() + 6 * 3.3 * spread) * slot).sum(1)
+    assert ((got.to(F64) - want).abs() <= bound + 2.0 ** -11 * want.abs() + 1e-6).all()

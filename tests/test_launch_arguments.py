@@ -237,7 +237,7 @@ def test_expert_blocks_of_256_are_taken_where_they_fill_the_chip(experts, top, h
 
 ROUTER = r"""
 static unsigned most_lds = 0;
-bool moe_stream_wants(const MoeStreamParams&, int, int, int, int64_t) { return false; }
+bool moe_stream_wants(const MoeStreamParams&, int, int, int, int64_t, int64_t) { return false; }
 int moe_stream_launch(const MoeStreamParams&, int, int, int, int64_t, hipStream_t) { return LL_OK; }
 extern "C" {
 hipError_t hipLaunchKernel(const void*, dim3, dim3, void**, size_t lds, hipStream_t) {
@@ -272,3 +272,61 @@ def test_long_steps_keep_the_walk_in_two_kernels(linear_mix, n, heads, qk_heads,
     assert fn(n, 4, heads, dk, dv, heads // qk_heads, kind, n // 4 + 24) == (n + 8) * (terms + heads * -(-dv // 32) * 32)
     assert fn(2 ** 28 // terms + 1, 4, heads, dk, dv, heads // qk_heads, kind, 1000) == 0
     assert fn(n, 4, heads, dk, dv, heads // qk_heads, kind, 23) == 0
+
+
+MOE = r"""
+#include "gemm_tile256.h"
+static int64_t asked[2];
+int tile256_grouped_launch(T2Params&, int, void*) { return LL_OK; }
+bool moe_stream_wants(const MoeStreamParams&, int, int, int, int64_t experts, int64_t runs) { asked[0] = experts; asked[1] = runs; return false; }
+int moe_stream_launch(const MoeStreamParams&, int, int, int, int64_t, hipStream_t) { return LL_OK; }
+extern "C" {
+hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { *v = 256; return hipSuccess; }
+hipError_t hipLaunchKernel(const void*, dim3, dim3, void**, size_t, hipStream_t) { return hipSuccess; }
+void stream_asked(int64_t* out) { out[0] = asked[0]; out[1] = asked[1]; asked[0] = asked[1] = 0; }
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def moe_gemm(tmp_path_factory):
+    """Experts and runs that a call of ll_moe_gemm names to the streaming form, or ``(0, 0)`` where it does not ask."""
+    lib = _host_library(tmp_path_factory.mktemp("host_moe"), "moe.hip", MOE)
+    P, L, I = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int
+    lib.ll_moe_gemm.argtypes = [P] * 8 + [L, L, I, L, L, I, I, I, I, L, L, L, L, L, L, L, I, P]
+
+    def call(fmt, experts, slots, block, n, k, spare=0):
+        em = slots + experts * (block - 1) + spare
+        wf = {"f16": 0, "fp8": 1, "int8": 2}[fmt]
+        assert lib.ll_moe_gemm(*[4096] * 8, slots, em, block, n, k, 1, 0, wf, 128, 128, k, n * k, k, 1, 1, 1, 0, None) == 0
+        out = (ctypes.c_int64 * 2)()
+        lib.stream_asked(out)
+        return tuple(out)
+
+    return call
+
+
+@pytest.mark.parametrize("experts", [1, 2, 4, 8, 34, 128, 300])
+@pytest.mark.parametrize("block", [16, 32, 64])
+@pytest.mark.parametrize("fmt", ["f16", "fp8"])
+def test_the_streaming_form_counts_the_experts(moe_gemm, experts, block, fmt):
+    """Not the blocks of their lists, which grow with the slots: the rows per expert from which tiles are faster are rows per expert."""
+    for rows in (1, 5, 10):
+        slots = rows * experts
+        asked, runs = moe_gemm(fmt, experts, slots, block, 1536, 2048)
+        assert asked == experts
+        assert runs >= min(experts, slots) and runs * block >= slots + experts * (block - 1)   # (blocks that the lists can hold)
+
+
+# (format, experts, n, k, rows per expert): which form was faster, both products of fused_moe on the GPU
+@pytest.mark.parametrize("fmt,experts,n,k,rows,stream", [
+    ("fp8", 128, 1536, 2048, 18, True), ("fp8", 128, 1536, 2048, 20, False), ("int8", 128, 1536, 2048, 28, False), ("fp8", 128, 3072, 4096, 18, True),
+    ("fp8", 128, 1024, 1024, 12, True), ("fp8", 128, 1024, 1024, 14, False), ("fp8", 200, 1024, 2048, 18, True), ("fp8", 64, 1536, 2048, 22, True),
+    ("fp8", 64, 1536, 2048, 28, False), ("fp8", 32, 1536, 2048, 24, True), ("fp8", 32, 1536, 2048, 32, False), ("int8", 8, 28672, 4096, 24, True),
+    ("int8", 8, 28672, 4096, 40, False), ("f16", 128, 1536, 2048, 20, True), ("f16", 128, 1536, 2048, 28, False),
+    ("f16", 64, 2048, 2048, 32, True), ("f16", 64, 2048, 2048, 64, False), ("f16", 4, 1024, 1024, 80, True), ("f16", 34, 2048, 704, 80, True),
+    ("fp8", 4, 1024, 1024, 32, True), ("fp8", 4, 1024, 1024, 100, False), ("f16", 48, 2816, 2048, 24, True),
+    ("f16", 48, 2816, 2048, 40, False), ("f16", 34, 1408, 2048, 56, True), ("f16", 16, 2048, 2048, 56, True), ("f16", 16, 2048, 2048, 64, False),
+    ("f16", 8, 28672, 4096, 56, True), ("f16", 8, 28672, 4096, 64, False)])
+def test_the_streaming_form_is_asked_where_it_is_faster(moe_gemm, fmt, experts, n, k, rows, stream):
+    assert (moe_gemm(fmt, experts, rows * experts, 64, n, k)[0] == experts) == stream
