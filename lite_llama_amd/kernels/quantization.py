@@ -580,9 +580,10 @@ def dense16_rows_wins(m: int, n: int, k: int) -> bool:
     return 1 <= m <= 64 and n >= 8192 and n % 32 == 0 and k % 128 == 0
 
 
-def _on_one_device(x: torch.Tensor, *operands) -> bool:
+def _on_one_device(x: torch.Tensor, weight: torch.Tensor, bias) -> bool:
     """Whether all operands are where ``x`` is: a kernel is handed their addresses, whatever they point at."""
-    return all(t is None or t.device == x.device for t in operands)
+    here = x.device
+    return weight.device == here and (bias is None or bias.device == here)
 
 
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
@@ -595,11 +596,10 @@ def _is_followed(x: torch.Tensor, weight: torch.Tensor, bias) -> bool:
         return True
     if torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad or (bias is not None and bias.requires_grad)):
         return True
-    if torch._C._functorch.maybe_current_level() is not None or torch._C._len_torch_dispatch_stack() > 0:
+    if forward_ad._current_level >= 0 and any(t is not None and forward_ad.unpack_dual(t).tangent is not None for t in (x, weight, bias)):
         return True
-    if any(t is not None and forward_ad.unpack_dual(t).tangent is not None for t in (x, weight, bias)):
-        return True
-    return torch.is_autocast_enabled("cuda") or torch._C._get_tracing_state() is not None
+    return (torch._C._functorch.maybe_current_level() is not None or torch._C._len_torch_dispatch_stack() > 0
+            or torch.is_autocast_enabled("cuda") or torch._C._get_tracing_state() is not None)
 
 
 def dense16_rows_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None, *, gate_up_swiglu: bool = False):

@@ -44,7 +44,8 @@ from .linear import ColumnParallelLinear, LinearBase, MergedColumnLinear, RowPar
 from .prefill_layers import ShortPrefill
 from .quantization import QuantConfig, get_moe_method
 
-_OWN = __name__.partition(".")[0] + "."   # modules of this package
+_OWN = __name__.partition(".")[0] + "."   # modules of this package ...
+_BARE = (nn.ModuleList, nn.ParameterDict, nn.Embedding)   # ... and what they are put together from
 _LOG2E = 1.4426950408889634  # prefill kernel evaluates exp2 (base.py:45-47)
 
 
@@ -631,7 +632,7 @@ class CausalLM(nn.Module):
                 continue
             state, kind = module.__dict__, type(module)
             if (state["_forward_hooks"] or state["_forward_pre_hooks"] or state["_backward_hooks"] or state["_backward_pre_hooks"]
-                    or "forward" in state or (kind is not nn.ModuleList and kind is not nn.Embedding and not kind.__module__.startswith(_OWN))):
+                    or "forward" in state or (kind not in _BARE and not kind.__module__.startswith(_OWN))):
                 return False
             todo.extend(state["_modules"].values())
         return True

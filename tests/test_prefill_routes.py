@@ -85,6 +85,8 @@ def grid(plain):
     info.prompt_grid = PromptGrid(info, [2, 5])
     ids, positions, last = torch.zeros(2, 5, dtype=torch.int64), torch.arange(5).expand(2, 5), torch.tensor([1, 9])
     assert plain.model._packs(ids, positions, info, last)
+    experts = CausalLM(tiny_geometry(num_experts=8, num_experts_per_tok=2, moe_intermediate_size=64, use_qk_norm=True))
+    assert experts._packs(ids, positions, info, last)
     return types.SimpleNamespace(model=plain.model, packs=lambda: plain.model._packs(ids, positions, info, last))
 
 
