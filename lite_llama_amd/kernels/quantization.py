@@ -587,6 +587,8 @@ def _on_one_device(x: torch.Tensor, weight: torch.Tensor, bias) -> bool:
 
 
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
+_transform_level, _dispatch_modes, _tracing_state = (torch._C._functorch.maybe_current_level, torch._C._len_torch_dispatch_stack,
+                                                     torch._C._get_tracing_state)
 
 
 def _is_followed(x: torch.Tensor, weight: torch.Tensor, bias) -> bool:
@@ -598,8 +600,7 @@ def _is_followed(x: torch.Tensor, weight: torch.Tensor, bias) -> bool:
         return True
     if forward_ad._current_level >= 0 and any(t is not None and forward_ad.unpack_dual(t).tangent is not None for t in (x, weight, bias)):
         return True
-    return (torch._C._functorch.maybe_current_level() is not None or torch._C._len_torch_dispatch_stack() > 0
-            or torch.is_autocast_enabled("cuda") or torch._C._get_tracing_state() is not None)
+    return (_transform_level() is not None or _dispatch_modes() > 0 or torch.is_autocast_enabled() or _tracing_state() is not None)
 
 
 def dense16_rows_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None, *, gate_up_swiglu: bool = False):
@@ -634,10 +635,12 @@ def dense16_narrow_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Ten
     if x.dtype not in (torch.float16, torch.bfloat16) or weight.dtype != x.dtype or weight.dim() != 2 or not x.is_cuda:
         return None
     n, k = weight.shape
-    if x.shape[-1] != k or k == 0 or x.numel() > 64 * k or not _on_one_device(x, weight, bias) or not L.has("ll_dense16_narrow_wins"):
+    if x.shape[-1] != k or k == 0 or x.numel() > 64 * k or not L.has("ll_dense16_narrow_wins"):
         return None
     m = x.numel() // k
-    if not L.lib().ll_dense16_narrow_wins(m, n, k) or os.environ.get("LL_DENSE16_NARROW_OFF") or _is_followed(x, weight, bias):
+    if not L.lib().ll_dense16_narrow_wins(m, n, k) or os.environ.get("LL_DENSE16_NARROW_OFF"):
+        return None
+    if not _on_one_device(x, weight, bias) or _is_followed(x, weight, bias):
         return None
     a = x if x.dim() == 2 and x.stride(1) == 1 and x.stride(0) >= k else _flatten(x, k)
     if (a.stride(0) % 8 or a.data_ptr() % 16 or weight.stride(1) != 1 or weight.stride(0) % 8 or weight.stride(0) < k or weight.data_ptr() % 16

@@ -88,5 +88,5 @@ def test_results_that_carry_more_than_values_are_left_to_the_library(launches, m
 
     with Mode():
         assert left()
-    monkeypatch.setattr(torch, "is_autocast_enabled", lambda kind: True)
+    monkeypatch.setattr(torch, "is_autocast_enabled", lambda *kind: True)
     assert left()
