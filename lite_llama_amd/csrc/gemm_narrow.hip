@@ -2,7 +2,8 @@
 // weights (up to about 25 MB) are too short a stream for a persistent loop (gemm_w16_rows.hip wants a 32-row group per CU) and too short to pay
 // a finishing launch for split-K planes.
 //   * A workgroup owns 16 (or 32) weight rows and ALL of K; its waves deal the contraction out in units of 128 entries and add their sums up
-//     in LDS, in wave order: finished outputs in one launch, a row's sums in an order that depends on nothing but K.
+//     in LDS, in wave order: finished outputs in one launch, a row's sums in an order that depends on K alone -- and for K > 1024 on whether
+//     there are more than 32 rows, which ll_dense16_narrow_wins leaves to other routes.
 //   * Fragments come straight from memory, 64 bytes of 16 rows per load (256 bytes of them, a whole row's unit per quarter wave, took 9 - 25 %
 //     longer); the next unit's weights are requested before this one is multiplied.
 // Bound by its launch, two trips to memory and the activations, which every workgroup reads from L2: bf16 2048 x 2048 1 row 5.6 us, 32 rows 8.9 (the

@@ -5,8 +5,8 @@
 //                     neighbours, a group's score is the sum of its two best scores, only the best `group_keep` groups stay
 //                     eligible; the `top` best eligible experts are chosen, their scores divided by their sum (+ 1e-20) and
 //                     multiplied by `route_scale`.  One more row of weights may give a per-token sigmoid scale (for a shared
-//                     expert).  Up to 512 tokens in one launch (a workgroup forms its tokens' logits and selects), beyond in two:
-//                     the logits as an 8 x 8 register-tiled product per wave, then one wave per token.  Selection by ranks (ties:
+//                     expert).  Up to 512 rows of router weights in one launch (a workgroup forms its tokens' logits and selects), more
+//                     in two: the logits as an 8 x 8 register-tiled product per wave, then one wave per token.  Selection by ranks (ties:
 //                     the lower index first), so slot k of a token holds its k-th best expert.
 //   ll_moe_sort       slots (token, k) sorted by expert, every expert's run padded to the row-block size with a sentinel:
 //                     sorted_ids / block_expert / num_post as in moe_align_block_size.  Deterministic: no atomics.
@@ -742,7 +742,7 @@ __global__ __launch_bounds__(256, 2) void moe_rows_gemm_tiled_kernel(const uint1
     else { CALL(LL_F32); }                   \
   } while (0)
 
-// logits: fp32 scratch [n][experts + (w_extra ? 1 : 0)]
+// logits: fp32 scratch [n][experts + (w_extra ? 1 : 0)], written where the router takes two launches (more than kRouterRows rows)
 extern "C" int ll_group_router(const void* h, int64_t h_ld, const void* w_router, const void* w_extra, int64_t n, int64_t width,
                                int64_t experts, int64_t top, int64_t group_count, int64_t group_keep, float route_scale, int scoring,
                                int32_t* ids, float* weights, float* extra_scale, float* logits, const void* correction, int64_t identity,

@@ -201,8 +201,8 @@ def test_a_forced_tile_height_is_the_128_row_engines(tmp_path, monkeypatch, sour
         lib.ll_w4a16_matmul_prepacked_mtiled.argtypes = [P] * 5 + [L, L, L, I, L, I, P]
         assert lib.ll_w4a16_matmul_prepacked_mtiled(*[4096] * 4, None, m, n, k, 128, k, 0, None) == 0
     else:
-        lib.ll_w8_mtiled_try.argtypes = [P] * 7 + [L, L, L, I, L, I, L, L, L, L, P]
-        assert lib.ll_w8_mtiled_try(*[4096] * 4, None, None, None, m, n, k, n, k, 1, k, k, 1, 1, None) == 1
+        lib.ll_w8_mtiled_try.argtypes = [P] * 7 + [L, L, L, I, L, I, L, L, L, L, P, L, P]
+        assert lib.ll_w8_mtiled_try(*[4096] * 4, None, None, None, m, n, k, n, k, 1, k, k, 1, 1, None, 0, None) == 1
     assert lib.launched_threads() == 256
 
 

@@ -62,7 +62,7 @@ def _exact(q, k, v, heads, dk, dv, runs, state, kw):
 @pytest.mark.parametrize("runs", [[(0, 24)], [(5, 1), (9, 79), (0, 16), (3, 17), (0, 1)], [(2, 95), (0, 33)]])
 def test_runs_of_many_tokens(dtype, kind, heads, qk_heads, dk, dv, runs):
     """Runs that end on and off eight tokens, beside single tokens; carried and fresh states; values off every tile of columns; one column
-    per thread and two."""
+    per thread (two below)."""
     from lite_llama_amd import _lib
     from lite_llama_amd.kernels.recurrent import linear_scan
 
@@ -81,11 +81,14 @@ def test_runs_of_many_tokens(dtype, kind, heads, qk_heads, dk, dv, runs):
     assert torch.equal(outs[0], outs[1]) and torch.equal(states[0], states[1])
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("kind,heads,qk_heads,dk,dv", [("fixed", 64, 64, 64, 200), ("entry", 48, 24, 128, 258), ("token", 112, 7, 256, 98)])
 @pytest.mark.parametrize("runs", [[(0, 24)], [(5, 1), (9, 79), (0, 16), (3, 17), (0, 1)]])
-def test_runs_of_many_tokens_in_two_columns_per_thread(kind, heads, qk_heads, dk, dv, runs):
+def test_runs_of_many_tokens_in_two_columns_per_thread(dtype, kind, heads, qk_heads, dk, dv, runs):
     """Three workgroups of 16 columns per CU and more; a last slice of 2, 8 and 32 columns."""
-    test_runs_of_many_tokens(torch.bfloat16, kind, heads, qk_heads, dk, dv, runs)
+    n, longest = sum(c for _, c in runs), max(c for _, c in runs)
+    assert -(-n // longest) * heads * -(-dv // 16) >= 768   # (where the walk takes two)
+    test_runs_of_many_tokens(dtype, kind, heads, qk_heads, dk, dv, runs)
 
 
 def test_a_step_whose_scratch_passes_a_gigabyte():
@@ -104,13 +107,14 @@ def test_a_step_whose_scratch_passes_a_gigabyte():
     assert torch.equal(outs[0], outs[1]) and torch.equal(states[0], states[1])
 
 
-@pytest.mark.parametrize("dv", [16, 320])   # one state column per thread, two
-def test_a_run_without_tokens_leaves_the_state_it_started_from(dv):
+@pytest.mark.parametrize("heads,dv,columns", [(8, 16, 1), (8, 320, 1), (24, 320, 2)])   # state columns per thread
+def test_a_run_without_tokens_leaves_the_state_it_started_from(heads, dv, columns):
     """Zeros where it starts at position 0, whatever an earlier owner of the slot left; as in the walk in one kernel."""
     from lite_llama_amd.kernels.recurrent import linear_scan
 
-    runs, heads, dk = [(0, 30), (0, 0), (7, 0), (3, 24)], 8, 64
+    runs, dk = [(0, 30), (0, 0), (7, 0), (3, 24)], 64
     n = sum(c for _, c in runs)
+    assert (-(-n // 30) * heads * -(-dv // 16) >= 768) == (columns == 2)
     q, k, v, kw = _inputs("fixed", heads, heads, dk, dv, n, torch.bfloat16, 5)
     step = _step([(i, f, c, 0) for i, (f, c) in enumerate(runs)], None)
     start = torch.randn(len(runs), heads, dk, dv, device=DEV)
