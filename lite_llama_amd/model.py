@@ -614,7 +614,7 @@ class CausalLM(nn.Module):
         positions feed nothing but themselves (attention never reads their rows, their own logits are undefined), and no hook or
         module from elsewhere is there to see them."""
         grid = getattr(atten_info, "prompt_grid", None)
-        return (grid is not None and input_ids.is_cuda and tuple(input_ids.shape) == (grid.batch, grid.longest)
+        return (grid is not None and input_ids.is_cuda and tuple(input_ids.shape) == (grid.batch, grid.longest) and grid.batch < 65535
                 and 1 < grid.total < grid.batch * grid.longest and grid.describes(atten_info)
                 and position_ids.shape == input_ids.shape and input_ids.dtype == torch.int64 and position_ids.dtype == torch.int64
                 and torch.is_tensor(logits_rows) and logits_rows.is_cuda and logits_rows.dtype == torch.int64 and logits_rows.dim() == 1

@@ -119,3 +119,13 @@ def test_modules_of_other_origin_see_the_grid(grid):
     del model.layers[1].forward
     model.register_forward_hook(lambda *a: None)   # (the model's own inputs and logits are the same either way)
     assert grid.packs()
+
+
+def test_more_prompts_than_the_packing_launch_takes_run_on_the_grid(grid):
+    from lite_llama_amd.executor.slots import PromptGrid
+
+    for n in (65534, 65535):
+        info = types.SimpleNamespace(b_seq_len=torch.ones(n), b_start_loc=torch.zeros(n), cur_select_index=torch.zeros(2 * n), max_actual_seq_len=2)
+        info.prompt_grid = PromptGrid(info, [1] * (n - 1) + [2])
+        ids = torch.zeros(n, 2, dtype=torch.int64)
+        assert grid.model._packs(ids, ids, info, torch.tensor([0])) == (n == 65534)
