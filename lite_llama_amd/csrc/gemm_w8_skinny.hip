@@ -16,6 +16,11 @@
 #include "common.h"
 #include "gemm_w8_common.h"
 
+// the form that streams a CU's whole share through LDS (gemm_split.hip): rows of whole 128-byte lines, n % 32 == 0
+int sk_partials_slices(int64_t m, int64_t n, int64_t k, int wfmt, int max_splits);
+int sk_launch(void* out, const void* x, const void* w, const float* scales, int64_t m, int64_t n, int64_t k, int group_n, int64_t group_k,
+              int wfmt, int64_t x_stride, int64_t w_stride, int64_t s_stride_n, int64_t s_stride_k, int max_splits, void* stream);
+
 namespace {
 
 struct alignas(16) Q4 {
@@ -298,16 +303,20 @@ extern "C" int ll_dense8_try(void* out, const void* x, const void* w, const floa
   p.nt_w = d8_nt(n * k);
   const int splits = d8_splits(n, k);
   p.cps = (p.chunks + splits - 1) / splits;
-  const int used = (p.chunks + p.cps - 1) / p.cps;  // every launched split has at least one chunk
+  int used = (p.chunks + p.cps - 1) / p.cps;  // every launched split has at least one chunk
   dim3 grid((unsigned)((n + 127) / 128), (unsigned)used);
   hipStream_t st = (hipStream_t)stream;
+  if (wfmt < D8_FP8 || wfmt > D8_I8I8) return 0;
+  const int planes = sk_launch(partials, x, w, scales, m, n, k, group_n, group_k, wfmt, x_stride * (wfmt == D8_I8I8 ? 1 : 2), w_stride, s_stride_n,
+                               s_stride_k, splits, stream);
+  if (planes < 0) return planes;
+  if (planes > 0) used = planes;
 #define LL_D8(WF)                                                        \
   if (m > 32) dense8_kernel<WF, 2><<<grid, 256, 0, st>>>(p);             \
   else dense8_kernel<WF, 1><<<grid, 256, 0, st>>>(p)
-  if (wfmt == D8_FP8) { LL_D8(D8_FP8); }
+  else if (wfmt == D8_FP8) { LL_D8(D8_FP8); }
   else if (wfmt == D8_I8) { LL_D8(D8_I8); }
-  else if (wfmt == D8_I8I8) { LL_D8(D8_I8I8); }
-  else return 0;
+  else { LL_D8(D8_I8I8); }
 #undef LL_D8
   const int64_t quads = m * n / 4;
   const dim3 fgrid((unsigned)((quads + 255) / 256));
@@ -350,21 +359,25 @@ extern "C" int ll_dense16_matmul(void* out, const void* x, const void* w, const 
   p.nt_w = d8_nt(n * k * 2);
   const int splits = d8_splits(n, k, 64);
   p.cps = (p.chunks + splits - 1) / splits;
-  const int used = (p.chunks + p.cps - 1) / p.cps;
+  int used = (p.chunks + p.cps - 1) / p.cps;
   dim3 grid((unsigned)((n + 127) / 128), (unsigned)used);
   hipStream_t st = (hipStream_t)stream;
   if (used == 1) {
     p.direct_out = (uint16_t*)out;
     p.direct_bias = (const uint16_t*)bias;
   }
-  if (dtype == LL_F16) {
+  const int planes = used == 1 ? 0 : sk_launch(partials, x, w, nullptr, m, n, k, 1, k, dtype == LL_F16 ? D8_F16 : D8_BF16, x_stride * 2,
+                                               w_stride * 2, 0, 0, splits, stream);
+  if (planes < 0) return planes;
+  if (planes > 0) used = planes;
+  else if (dtype == LL_F16) {
     if (m > 32) dense8_kernel<D8_F16, 2><<<grid, 256, 0, st>>>(p);
     else dense8_kernel<D8_F16, 1><<<grid, 256, 0, st>>>(p);
   } else {
     if (m > 32) dense8_kernel<D8_BF16, 2><<<grid, 256, 0, st>>>(p);
     else dense8_kernel<D8_BF16, 1><<<grid, 256, 0, st>>>(p);
   }
-  if (used == 1) return hipGetLastError() == hipSuccess ? 1 : LL_ERR_LAUNCH;
+  if (used == 1 && planes == 0) return hipGetLastError() == hipSuccess ? 1 : LL_ERR_LAUNCH;
   const int64_t quads = m * n / 4;
   const dim3 fgrid((unsigned)((quads + 255) / 256));
   if (dtype == LL_F16)
@@ -387,16 +400,10 @@ extern "C" int ll_dense16_matmul(void* out, const void* x, const void* w, const 
 // ll_skip_rmsnorm_q8, ll_w8a8_finish_swiglu (w8a8_fused.hip).  Returns the number of planes written (>= 1), 0 when the
 // shape is not served, < 0 on error.
 // ---------------------------------------------------------------------------------------------------------------- //
-// the short-stream form of this mode (gemm_short_dense.hip): launches of a few tens of KB per CU
-int sd_partials_slices(int64_t m, int64_t n, int64_t k, int wfmt, int max_splits);
-int sd_launch(float* out, const void* x, const void* w, const float* scales, int64_t m, int64_t n, int64_t k, int group_n,
-              int64_t group_k, int wfmt, int64_t x_stride, int64_t w_stride_bytes, int64_t s_stride_n, int64_t s_stride_k,
-              int max_splits, void* stream);
-
 extern "C" int ll_dense_partials_count(int64_t m, int64_t n, int64_t k, int wfmt, int max_splits) {
   const bool w16 = wfmt == D8_F16 || wfmt == D8_BF16;
   if (wfmt != D8_FP8 && wfmt != D8_I8 && wfmt != D8_I8I8 && !w16) return 0;
-  if (const int s = sd_partials_slices(m, n, k, wfmt, max_splits)) return s;
+  if (const int s = sk_partials_slices(m, n, k, wfmt, max_splits)) return s;
   const int kch = w16 ? 64 : 128;
   if (m < 1 || m > 64 || n < 4 || n % 4 != 0 || k < kch || k % kch != 0 || max_splits < 1) return 0;
   const int chunks = (int)(k / kch);
@@ -414,12 +421,12 @@ extern "C" int ll_dense_partials(float* partials, const void* x, const void* w, 
   const bool i8a = wfmt == D8_I8I8;
   if (!partials || !x || !w || (!w16 && !i8a && !scales)) return LL_ERR_ARG;
   const int eb = w16 ? 2 : 1;
-  if (sd_partials_slices(m, n, k, wfmt, max_splits))  // (declines -- 0 -- exactly where the streaming engine below would)
-    return sd_launch(partials, x, w, scales, m, n, k, group_n, group_k, wfmt, x_stride, w_stride * eb, s_stride_n, s_stride_k,
-                     max_splits, stream);
   if ((w_stride * eb) % 16 != 0 || x_stride % (i8a ? 16 : 8) != 0 || !ll_aligned16(w) || !ll_aligned16(x) || !ll_aligned16(partials))
     return 0;
   if (!w16 && !i8a && group_k < k && group_k % 64 != 0) return 0;
+  if (sk_partials_slices(m, n, k, wfmt, max_splits))
+    return sk_launch(partials, x, w, scales, m, n, k, group_n, group_k, wfmt, x_stride * (i8a ? 1 : 2), w_stride * eb, s_stride_n, s_stride_k,
+                     max_splits, stream);
   D8Params p{};
   p.part = partials; p.x = x; p.w = (const unsigned char*)w; p.scales = scales;
   p.m = m; p.n = n; p.k = k; p.x_stride = x_stride; p.w_stride = w_stride * eb;

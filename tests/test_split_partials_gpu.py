@@ -1,0 +1,64 @@
+"""Split-K planes of narrow projections (csrc/gemm_split.hip): every tile width, more slices than units, shares of unequal length, rows
+that end inside a 32-row block, rows of a wider tensor."""
+
+import pytest
+import torch
+
+from lite_llama_amd import _lib as L
+
+DEV = "cuda"
+FP8, I8, I8I8, F16, BF16 = 1, 2, 3, 4, 5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", [FP8, I8, I8I8, F16, BF16])
+@pytest.mark.parametrize("m,n,k,cap", [(1, 32, 128, 12), (64, 96, 128, 12), (33, 64, 384, 2), (32, 1120, 1152, 12), (31, 4096, 640, 8),
+                                       (64, 5120, 2048, 8), (7, 8192, 256, 3), (45, 896, 4864, 12)])
+def test_planes_add_up_to_the_product(fmt, m, n, k, cap):
+    g = torch.Generator().manual_seed(n + k + fmt)
+    pad = 64   # rows of x and w are column ranges of wider tensors
+    if fmt in (F16, BF16):
+        dt = torch.float16 if fmt == F16 else torch.bfloat16
+        w = torch.randn(n, k + pad, generator=g).to(dt)
+        x = torch.randn(m, k + pad, generator=g).to(dt)
+        wide, scales, gk = w[:, :k].double(), None, k
+    else:
+        w = torch.randint(-127, 128, (n, k + pad), generator=g, dtype=torch.int8)
+        x = torch.randint(-127, 128, (m, k + pad), generator=g, dtype=torch.int8) if fmt == I8I8 else torch.randn(m, k + pad, generator=g).half()
+        gk = 64 if k % 128 else 128
+        # (powers of two: a widened weight is exact in fp16, what remains is the sums)
+        scales = None if fmt == I8I8 else 2.0 ** torch.randint(-4, 3, ((n + 31) // 32, (k + gk - 1) // gk), generator=g).float()
+        wide = w[:, :k].double()
+        if fmt == FP8:
+            w = torch.randn(n, k + pad, generator=g).to(torch.float8_e4m3fn)
+            wide, w = w[:, :k].double(), w.view(torch.uint8)
+        if scales is not None:
+            wide = wide * scales.double().repeat_interleave(32, 0)[:n].repeat_interleave(gk, 1)[:, :k]
+    ref = x[:, :k].double() @ wide.T
+    size = x[:, :k].double().abs() @ wide.abs().T
+    x, w, scales = x.to(DEV), w.to(DEV), None if scales is None else scales.to(DEV)
+    count = L.lib().ll_dense_partials_count(m, n, k, fmt, cap)
+    assert 1 <= count <= cap
+    guard = 64
+    planes = torch.full((count * m * n + guard,), 7777, dtype=torch.int32, device=DEV)
+    got = L.lib().ll_dense_partials(planes.data_ptr(), x.data_ptr(), w.data_ptr(), L.ptr(scales), m, n, k, 32, gk, fmt, x.stride(0), w.stride(0),
+                                    scales.stride(0) if scales is not None else 0, scales.stride(1) if scales is not None else 0, cap,
+                                    L.stream_ptr())
+    assert got == count
+    assert (planes[count * m * n:] == 7777).all()   # nothing past the last plane
+    body = planes[:count * m * n].view(count, m, n)
+    if fmt == I8I8:
+        assert torch.equal(body.sum(0, dtype=torch.int64).cpu(), ref.long())
+        return
+    total = body.view(torch.float32).double().sum(0).cpu()
+    # fp32 sums of k exact products, in whatever order: k * 2^-24 of the sum of their sizes bounds them from far above
+    assert ((total - ref).abs() <= k * 2.0 ** -24 * size + 1e-30).all()
+
+
+@pytest.mark.parametrize("fmt", [FP8, I8, I8I8, F16, BF16])
+@pytest.mark.parametrize("n,k", [(1536, 8960), (4096, 14336), (5120, 2048), (896, 896), (36, 128), (32, 64)])
+def test_plane_count_does_not_depend_on_the_rows(fmt, n, k):
+    for cap in (1, 3, 12):
+        counts = {L.lib().ll_dense_partials_count(m, n, k, fmt, cap) for m in (1, 31, 32, 33, 64)}
+        assert len(counts) == 1 and max(counts) <= cap
+    assert L.lib().ll_dense_partials_count(65, n, k, fmt, 12) == 0
