@@ -574,6 +574,16 @@ int ll_slot_advance(void* b_seq_len, const void* b_req_idx, int32_t* cur_select_
                     const int32_t* table, int64_t table_stride_b, int64_t table_stride_s, int batch,
                     int idx_width, void* stream);
 
+/* dst[i][0 .. words[i]) = src[i][..] in 4-byte words for up to five vectors, in one launch. */
+int ll_copy_words(void* const* dst, const void* const* src, const int64_t* words, int count, void* stream);
+
+/* residual = table[ids] (rows of n 16-bit values; an id outside [0, table_rows): NaN) and y = rmsnorm(residual) * weight; ll_embed_rmsnorm_q8:
+ * y (fp16) and its int8 rows with their scales, each optional.  n % 8 == 0, n <= 8192. */
+int ll_embed_rmsnorm(void* y, void* residual, const void* table, const int64_t* ids, const void* weight, int64_t rows, int64_t n,
+                     int64_t table_rows, float eps, int dtype, void* stream);
+int ll_embed_rmsnorm_q8(void* y, int8_t* q, float* q_scale, void* residual, const void* table, const int64_t* ids, const void* weight,
+                        int64_t rows, int64_t n, int64_t table_rows, float eps, void* stream);
+
 /* A decoder layer of an unquantised llama-shaped model (norm, q|k|v, rotation + scatter, attention, o, norm, gate|up + activation, down) over
  * the tokens (<= 192) of `prompts` prompts, in one call.  residual [tokens][hidden]: updated in place; planes_in > 0: that many fp32 partial
  * sums per part at `planes` are added to it first (the layer before left them).  Scratch: x [tokens][hidden], qkv [tokens][(heads + 2 kv_heads)

@@ -289,3 +289,30 @@ extern "C" int ll_pack_prompts(const int64_t* ids, int64_t ids_stride_b, int64_t
 }
 
 extern "C" int ll_abi_version(void) { return 1; }
+
+// Up to five vectors of 4-byte words (a captured step's inputs) in one launch: a copy each costs a launch of 4.4 us.
+struct CopyWordsParams {
+  uint32_t* dst[5];
+  const uint32_t* src[5];
+  int64_t words[5];
+};
+__global__ __launch_bounds__(256) void copy_words_kernel(const CopyWordsParams p) {
+  const int v = blockIdx.x;
+  for (int64_t i = threadIdx.x; i < p.words[v]; i += 256) p.dst[v][i] = p.src[v][i];
+}
+
+extern "C" int ll_copy_words(void* const* dst, const void* const* src, const int64_t* words, int count, void* stream) {
+  if (count < 0 || count > 5) return LL_ERR_SHAPE;
+  if (count == 0) return LL_OK;
+  if (!dst || !src || !words) return LL_ERR_ARG;
+  CopyWordsParams p{};
+  for (int i = 0; i < count; ++i) {
+    if (words[i] < 0) return LL_ERR_SHAPE;
+    if (!dst[i] || !src[i] || (((uintptr_t)dst[i] | (uintptr_t)src[i]) & 3)) return LL_ERR_ARG;
+    p.dst[i] = (uint32_t*)dst[i];
+    p.src[i] = (const uint32_t*)src[i];
+    p.words[i] = words[i];
+  }
+  copy_words_kernel<<<dim3((unsigned)count), 256, 0, (hipStream_t)stream>>>(p);
+  return LL_LAUNCH_CHECK();
+}

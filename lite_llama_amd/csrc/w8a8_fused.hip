@@ -32,13 +32,16 @@ __device__ __forceinline__ float q8_row_sum(float v, float* lds) {
 
 // SMAX == 0: the input is a finished fp16 tensor x [rows][n];  SMAX > 0: int32 planes [S][rows][n] + scales (+ bias).
 // HAS_RES as skip_rmsnorm (residual updated in place).  y (fp16) and q / q_scale (int8 rows + per-token scale) are each optional.
-template <int VPT, int SMAX, bool HAS_RES>
+// GATHER: x is a table of `table_rows` rows, row i of the input its row ids[i], which goes to r as it is (the first norm of a step).
+template <int VPT, int SMAX, bool HAS_RES, bool GATHER = false>
 __global__ __launch_bounds__(256) void skip_rmsnorm_q8_kernel(uint16_t* __restrict__ y, int8_t* __restrict__ q,
                                                               float* __restrict__ q_scale, const uint16_t* __restrict__ x,
                                                               const int32_t* __restrict__ part, int s_count,
                                                               const float* __restrict__ a_scale, const float* __restrict__ w_scale,
                                                               const uint16_t* __restrict__ bias, uint16_t* __restrict__ r,
-                                                              const uint16_t* __restrict__ w, int64_t rows, int n, float eps) {
+                                                              const uint16_t* __restrict__ w, int64_t rows, int n, float eps,
+                                                              const int64_t* __restrict__ ids = nullptr, int64_t table_rows = 0) {
+  static_assert(!GATHER || (SMAX == 0 && !HAS_RES), "a gathered row is the residual");
   constexpr int DT = LL_F16;
   constexpr int SL = SMAX > 0 ? SMAX : 1;
   __shared__ float lds[4];
@@ -53,6 +56,13 @@ __global__ __launch_bounds__(256) void skip_rmsnorm_q8_kernel(uint16_t* __restri
   f32x4 ws[VPT][2];
   bool ok[VPT];
   const float as = SMAX > 0 ? a_scale[row] : 0.f;
+  int64_t from = row;
+  bool known = true;
+  if constexpr (GATHER) {
+    from = ids[row];
+    known = from >= 0 && from < table_rows;   // (no such row: the results are NaN)
+    if (!known) from = 0;
+  }
 #pragma unroll
   for (int v = 0; v < VPT; ++v) {
     const int col = (v * 256 + tr) * 8;
@@ -72,7 +82,7 @@ __global__ __launch_bounds__(256) void skip_rmsnorm_q8_kernel(uint16_t* __restri
       ws[v][1] = *reinterpret_cast<const f32x4*>(w_scale + c0 + 4);
       bv[v] = *reinterpret_cast<const U16x8*>(bias ? bias + c0 : w + c0);  // (a pointer select: no load inside a branch)
     } else {
-      xv[v] = *reinterpret_cast<const U16x8*>(x + off);
+      xv[v] = *reinterpret_cast<const U16x8*>(x + (GATHER ? (ok[v] ? from * n + col : 0) : off));
     }
   }
   float sv[VPT][8];
@@ -89,6 +99,7 @@ __global__ __launch_bounds__(256) void skip_rmsnorm_q8_kernel(uint16_t* __restri
         const float f = q8_f32(((float)a * as) * ws[v][i >> 2][i & 3]);  // (acc.f32 * a_scale[m]) * w_scale[n], w8a8.py:118-120
         xin = to_f32<DT>(from_f32<DT>(q8_f32(bias ? f + to_f32<DT>(bv[v].v[i]) : f)));
       } else {
+        if constexpr (GATHER) xv[v].v[i] = known ? xv[v].v[i] : (uint16_t)0x7fff;
         xin = to_f32<DT>(xv[v].v[i]);
       }
       float s = xin;
@@ -98,8 +109,8 @@ __global__ __launch_bounds__(256) void skip_rmsnorm_q8_kernel(uint16_t* __restri
       }
       sv[v][i] = ok[v] ? s : 0.f;
     }
-    if constexpr (HAS_RES) {
-      if (ok[v]) *reinterpret_cast<U16x8*>(r + row * n + (v * 256 + tr) * 8) = rv[v];
+    if constexpr (HAS_RES || GATHER) {
+      if (ok[v]) *reinterpret_cast<U16x8*>(r + row * n + (v * 256 + tr) * 8) = GATHER ? xv[v] : rv[v];
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) ssq += sv[v][i] * sv[v][i] / nf;
@@ -265,6 +276,24 @@ extern "C" int ll_skip_rmsnorm_q8(void* y, int8_t* q, float* q_scale, const void
 #undef LL_Q8_S
 #undef LL_Q8_RES
 #undef LL_Q8_CASE
+  return LL_LAUNCH_CHECK();
+}
+
+// ll_skip_rmsnorm_q8 of residual = table[ids] (q / q_scale, or y, or both): embedding lookup, first norm and quantiser in one launch.
+extern "C" int ll_embed_rmsnorm_q8(void* y, int8_t* q, float* q_scale, void* residual, const void* table, const int64_t* ids, const void* weight,
+                                   int64_t rows, int64_t n, int64_t table_rows, float eps, void* stream) {
+  if (rows < 0 || n <= 0 || n % 8 != 0 || n > 8192 || table_rows < 1) return LL_ERR_SHAPE;
+  if (!residual || !table || !ids || !weight || (!y && !q) || (q && !q_scale)) return LL_ERR_ARG;
+  if (!ll_aligned16(y) || !ll_aligned16(residual) || !ll_aligned16(table) || !ll_aligned16(weight) || ((uintptr_t)q & 7) != 0) return LL_ERR_ARG;
+  if (rows == 0) return LL_OK;
+  hipStream_t st = (hipStream_t)stream;
+  const int nv = (int)(n / 8);
+#define LL_Q8_EMBED(VPT)                                                                                                              \
+  skip_rmsnorm_q8_kernel<VPT, 0, false, true><<<dim3((unsigned)rows), 256, 0, st>>>((uint16_t*)y, q, q_scale, (const uint16_t*)table, nullptr, 0, \
+                                                                                   nullptr, nullptr, nullptr, (uint16_t*)residual,     \
+                                                                                   (const uint16_t*)weight, rows, (int)n, eps, ids, table_rows)
+  if (nv <= 256) LL_Q8_EMBED(1); else if (nv <= 512) LL_Q8_EMBED(2); else LL_Q8_EMBED(4);
+#undef LL_Q8_EMBED
   return LL_LAUNCH_CHECK();
 }
 

@@ -70,6 +70,45 @@ class PartialSums:
         return out
 
 
+class EmbeddedRows:
+    """Rows ``ids`` of an embedding table that are not looked up yet: the first norm of a step reads them from the table and leaves
+    them as the residual (:func:`embed_rmsnorm`)."""
+
+    __slots__ = ("ids", "table", "shape", "dtype", "device")
+    is_cuda = True
+
+    def __init__(self, ids: torch.Tensor, table: torch.Tensor):
+        self.ids, self.table, self.shape = ids, table, (*ids.shape, table.shape[1])
+        self.dtype, self.device = table.dtype, table.device
+
+    @staticmethod
+    def served(ids: torch.Tensor, table: torch.Tensor) -> bool:
+        return (type(ids) is torch.Tensor and ids.is_cuda and ids.dtype == torch.int64 and ids.is_contiguous() and table.device == ids.device
+                and table.dtype in (torch.float16, torch.bfloat16) and table.dim() == 2 and table.is_contiguous() and table.shape[0] > 0
+                and table.shape[1] % 8 == 0 and 0 < table.shape[1] <= 8192 and table.data_ptr() % 16 == 0 and L.has("ll_embed_rmsnorm_q8"))
+
+
+@torch.no_grad()
+def embed_rmsnorm(X: EmbeddedRows, weight, eps=1e-5, *, q8: bool = False):
+    """``skip_rmsnorm(table[ids], None, weight)`` -- with ``q8`` ``skip_rmsnorm_q8`` -- in one launch: ``(Y | Int8Rows, residual)``."""
+    n, rows = X.table.shape[1], X.ids.numel()
+    residual = torch.empty((rows, n), dtype=X.dtype, device=X.device)
+    if weight.dtype != X.dtype:
+        weight = weight.to(X.dtype)
+    weight = weight.contiguous()
+    L.require_cuda(weight)
+    if q8:
+        q = torch.empty((rows, n), dtype=torch.int8, device=X.device)
+        scale = torch.empty((rows,), dtype=torch.float32, device=X.device)
+        L.check(L.lib().ll_embed_rmsnorm_q8(0, q.data_ptr(), scale.data_ptr(), residual.data_ptr(), X.table.data_ptr(), X.ids.data_ptr(),
+                                            weight.data_ptr(), rows, n, X.table.shape[0], float(eps), L.stream_ptr()), "embed_rmsnorm_q8")
+        return Int8Rows(q, scale, X.shape), residual.view(X.shape)
+    Y = torch.empty_like(residual)
+    L.check(L.lib().ll_embed_rmsnorm(Y.data_ptr(), residual.data_ptr(), X.table.data_ptr(), X.ids.data_ptr(), weight.data_ptr(), rows, n,
+                                     X.table.shape[0], float(eps), L.dtype_code(X.dtype), L.stream_ptr()), "embed_rmsnorm")
+    return Y.view(X.shape), residual.view(X.shape)
+
+
 class SlotSums(PartialSums):
     """:class:`PartialSums` of a fused-MoE block: ``parts`` are the down projection's per-slot rows ``[rows, k, n]`` in the
     activation dtype (router weights folded in); their fp32 sum over ``k``, rounded once, is the block's output (``moe_sum``).
@@ -147,7 +186,9 @@ def skip_rmsnorm_q8(X, residual, weight, eps=1e-5, *, quantize: bool = True, kee
     :class:`ScaledInt32Partials` of the previous W8A8 projection (its scale epilogue runs here); with ``quantize`` the
     normalised rows leave as :class:`Int8Rows` for the next W8A8 projection -- the values of ``dense8_finish`` ->
     ``skip_rmsnorm`` -> ``quantize_activations_int8``, bit for bit.  Returns ``(Int8Rows | Y, residual)``; ``keep_y`` also
-    stores the fp16 ``Y`` and returns ``((Int8Rows, Y), residual)``."""
+    stores the fp16 ``Y`` and returns ``((Int8Rows, Y), residual)``.  ``X`` may be :class:`EmbeddedRows` (the first norm of a step)."""
+    if isinstance(X, EmbeddedRows):
+        return embed_rmsnorm(X, weight, eps, q8=True)
     planes = X if isinstance(X, ScaledInt32Partials) else None
     if planes is not None:
         s, m, n = X.parts.shape

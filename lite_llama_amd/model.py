@@ -28,8 +28,8 @@ from .distributed.parallel_state import all_reduce_tp, divide, get_tp_rank, get_
 from .distributed.partition import ShardPlan, make_plan, scale_unit, set_active_plan
 from .kernels.attention import decode_attention, decode_attention_partials, decode_attention_partials_supported
 from .kernels.kv_cache import pack_prompts
-from .kernels.norm_act import (Int8Rows, PartialSums, ScaledInt32Partials, norm_rope_and_cache_supported, rope_and_cache,
-                               skip_rmsnorm_partials, skip_rmsnorm_q8)
+from .kernels.norm_act import (EmbeddedRows, Int8Rows, PartialSums, ScaledInt32Partials, embed_rmsnorm, norm_rope_and_cache_supported,
+                               rope_and_cache, skip_rmsnorm_partials, skip_rmsnorm_q8)
 from .kernels import (
     flash_attention2_no_pad,
     flash_decoding,
@@ -41,7 +41,7 @@ from .kernels import (
     flash_decoding_fp8kv,
 )
 from .linear import ColumnParallelLinear, LinearBase, MergedColumnLinear, RowParallelLinear
-from .prefill_layers import ShortPrefill
+from .prefill_layers import ShortPrefill, _plain
 from .quantization import QuantConfig, get_moe_method
 
 _OWN = __name__.partition(".")[0] + "."   # modules of this package ...
@@ -363,6 +363,10 @@ def add_norm(hidden_states, residual, weight, eps, q8: bool = False):
     """``skip_rmsnorm`` that also accepts a projection left as split-K partials (kernels/norm_act.py::PartialSums).
     ``q8`` (smoothquant blocks): the consumer reads per-token int8 rows -- the quantiser runs inside the norm launch and the
     result is an ``Int8Rows``."""
+    if isinstance(hidden_states, EmbeddedRows):
+        if q8 and hidden_states.dtype == torch.float16:
+            return skip_rmsnorm_q8(hidden_states, residual, weight, eps)
+        return embed_rmsnorm(hidden_states, weight, eps)
     if isinstance(hidden_states, ScaledInt32Partials):
         s_count, _, width = hidden_states.parts.shape
         # rows wider than 4096 keep four 8-value vectors per thread: more than 4 planes of them do not fit the register
@@ -637,6 +641,17 @@ class CausalLM(nn.Module):
             todo.extend(state["_modules"].values())
         return True
 
+    def _embed(self, input_ids):
+        """The embedding -- left to the first layer's norm where nothing but that would see it, and the pass is not one of the short prefills
+        that run their layers by a host call each."""
+        embed = self.embed_tokens
+        if (not self.layers or not (input_ids.dim() == 2 and (input_ids.shape[1] == 1 or input_ids.numel() > ShortPrefill.MAX_TOKENS))
+                or not _plain(embed, nn.Embedding) or embed.max_norm is not None or not _plain(self.layers[0], DecoderLayer)
+                or not _plain(self.rotary_emb, RotaryEmbedding) or _nn._global_forward_hooks or _nn._global_forward_pre_hooks
+                or _nn._global_backward_hooks or _nn._global_backward_pre_hooks or not EmbeddedRows.served(input_ids, embed.weight)):
+            return embed(input_ids)
+        return EmbeddedRows(input_ids, embed.weight)
+
     @torch.no_grad()
     def forward(self, input_ids, position_ids, atten_info, logits_rows=None):
         """``[batch, seq]`` ids -> ``[batch, seq, vocab]`` fp16 logits.  ``logits_rows`` (extension:
@@ -651,10 +666,10 @@ class CausalLM(nn.Module):
                 input_ids, position_ids, atten_info.cur_select_index, atten_info.b_seq_len, grid.total, logits_rows)
             atten_info = copy.copy(atten_info)   # (the caller's struct keeps describing the grid)
             atten_info.cur_select_index, atten_info.b_start_loc, atten_info.b_seq_len = select, starts, lens
-        hidden_states = self.embed_tokens(input_ids)
+        hidden_states = self._embed(input_ids)
         position_embeddings = self.rotary_emb(hidden_states, position_ids)
         residual = None
-        short = ShortPrefill.of(self, hidden_states, position_embeddings, atten_info)   # a host call per layer
+        short = None if isinstance(hidden_states, EmbeddedRows) else ShortPrefill.of(self, hidden_states, position_embeddings, atten_info)
         for i, layer in enumerate(self.layers):
             done = short.layer(layer, i, hidden_states, residual) if short is not None else None
             if done is None:
