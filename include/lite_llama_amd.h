@@ -574,6 +574,10 @@ int ll_slot_advance(void* b_seq_len, const void* b_req_idx, int32_t* cur_select_
                     const int32_t* table, int64_t table_stride_b, int64_t table_stride_s, int batch,
                     int idx_width, void* stream);
 
+/* cos / sin [batch * seq][2 half] of position * freq[j] in entries j and half + j; positions [batch][seq] with their strides (entries). */
+int ll_rotary_rows(void* cos_out, void* sin_out, const void* positions, int pos_width, int64_t stride_b, int64_t stride_s, const float* freq,
+                   int64_t batch, int64_t seq, int64_t half, int dtype, void* stream);
+
 /* dst[i][0 .. words[i]) = src[i][..] in 4-byte words for up to five vectors, in one launch. */
 int ll_copy_words(void* const* dst, const void* const* src, const int64_t* words, int count, void* stream);
 

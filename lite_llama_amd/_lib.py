@@ -102,6 +102,7 @@ SIGNATURES = {
     "ll_prefill_layer16": [P, P, I, P, P, P, P, P, P, F, P, P, P, P, P, P, P, L, L, L, L, P, L, L, P, I, P, I, P, I, L, L, L, L, L, I, I, I, L, F, I, I,
                            I, P],
     "ll_pack_prompts": [P, L, L, P, L, L, P, I, P, I, L, L, L, P, L, P, P, P, P, P, P, P],
+    "ll_rotary_rows": [P, P, P, I, L, L, P, L, L, L, I, P],
     "ll_copy_words": [P, P, P, I, P],
     "ll_embed_rmsnorm": [P, P, P, P, P, L, L, L, F, I, P],
     "ll_embed_rmsnorm_q8": [P, P, P, P, P, P, P, L, L, L, F, P],

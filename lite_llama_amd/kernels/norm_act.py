@@ -109,6 +109,24 @@ def embed_rmsnorm(X: EmbeddedRows, weight, eps=1e-5, *, q8: bool = False):
     return Y.view(X.shape), residual.view(X.shape)
 
 
+def rotary_rows(positions: torch.Tensor, freq: torch.Tensor, dtype):
+    """``(cos, sin)`` ``[batch, seq, 2 * len(freq)]`` of ``positions [batch, seq] * freq`` in ``dtype`` (angles in fp32), in one launch; ``None``
+    where the call is not served."""
+    if (type(positions) is not torch.Tensor or type(freq) not in (torch.Tensor, torch.nn.Parameter) or positions.device.type != "cuda" or positions.dim() != 2
+            or positions.dtype not in (torch.int32, torch.int64) or freq.device != positions.device or freq.dtype != torch.float32 or freq.dim() != 1
+            or not freq.is_contiguous() or dtype not in (torch.float16, torch.bfloat16) or not 0 < freq.numel() <= 4096 or not L.has("ll_rotary_rows")):
+        return None
+    batch, seq = positions.shape
+    if batch * seq * freq.numel() >= 1 << 38:
+        return None
+    out = torch.empty((2, batch, seq, 2 * freq.numel()), dtype=dtype, device=positions.device)
+    cos, sin = out.unbind(0)
+    L.check(L.lib().ll_rotary_rows(cos.data_ptr(), sin.data_ptr(), positions.data_ptr(), L.index_width(positions), positions.stride(0),
+                                   positions.stride(1), freq.data_ptr(), batch, seq, freq.numel(), L.dtype_code(dtype), L.stream_ptr()),
+            "rotary_rows")
+    return cos, sin
+
+
 class SlotSums(PartialSums):
     """:class:`PartialSums` of a fused-MoE block: ``parts`` are the down projection's per-slot rows ``[rows, k, n]`` in the
     activation dtype (router weights folded in); their fp32 sum over ``k``, rounded once, is the block's output (``moe_sum``).

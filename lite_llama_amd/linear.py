@@ -183,16 +183,26 @@ class MergedColumnLinear:
         self._holder = None
 
     def _snapshot(self):
-        return tuple((n, t.data_ptr(), t._version) for l in self.layers for n, t in l._parameters.items()
-                     if t is not None) + tuple((id(l.quant_method), id(getattr(l, "act_perm", None))) for l in self.layers)
+        key = []
+        for l in self.layers:
+            state = l.__dict__
+            for n, t in state["_parameters"].items():
+                if t is not None:
+                    key += (n, t.data_ptr(), t._version)
+            perm = state.get("act_perm")
+            key += (id(state.get("quant_method")), id(perm if perm is not None else state["_buffers"].get("act_perm")))
+        return tuple(key)
 
-    @torch.no_grad()
     def refresh(self) -> bool:
         """(Re)build the merged storage if a member's parameters were replaced; returns whether the
         merged path can be used.  Never allocates inside a graph capture."""
         key = self._snapshot()
         if key == self._key:
             return self._holder is not None
+        return self._rebuild()
+
+    @torch.no_grad()
+    def _rebuild(self) -> bool:
         first = self.layers[0]
         if not first.weight.is_cuda or torch.cuda.is_current_stream_capturing():
             return False

@@ -28,8 +28,8 @@ from .distributed.parallel_state import all_reduce_tp, divide, get_tp_rank, get_
 from .distributed.partition import ShardPlan, make_plan, scale_unit, set_active_plan
 from .kernels.attention import decode_attention, decode_attention_partials, decode_attention_partials_supported
 from .kernels.kv_cache import pack_prompts
-from .kernels.norm_act import (EmbeddedRows, Int8Rows, PartialSums, ScaledInt32Partials, embed_rmsnorm, norm_rope_and_cache_supported,
-                               rope_and_cache, skip_rmsnorm_partials, skip_rmsnorm_q8)
+from .kernels.norm_act import (EmbeddedRows, Int8Rows, PartialSums, ScaledInt32Partials, SlotSums, embed_rmsnorm, norm_rope_and_cache_supported,
+                               rope_and_cache, rotary_rows, skip_rmsnorm_partials, skip_rmsnorm_q8)
 from .kernels import (
     flash_attention2_no_pad,
     flash_decoding,
@@ -185,7 +185,8 @@ class RotaryEmbedding(nn.Module):
             # decode: hand out the position-indexed tables themselves; the fused rope kernel reads row
             # positions[i] (callers guarantee positions < the size given to ``ensure``)
             return RopeTables(c[0], c[1], position_ids.reshape(-1))
-        return self._tables(position_ids, x.dtype)
+        rows = rotary_rows(position_ids, self.inv_freq, x.dtype)   # (the same values)
+        return rows if rows is not None else self._tables(position_ids, x.dtype)
 
 
 # ------------------------------------------------------------------------------------- #
@@ -380,6 +381,18 @@ def add_norm(hidden_states, residual, weight, eps, q8: bool = False):
     if isinstance(hidden_states, PartialSums):
         return skip_rmsnorm_partials(hidden_states, residual, weight, eps)
     return skip_rmsnorm(hidden_states, residual, weight, eps)
+
+
+def _rows_of(hidden_states, residual, rows):
+    """``(whether it could be done, update, residual)`` of the listed rows alone."""
+    width = residual.shape[-1]
+    if torch.is_tensor(hidden_states):
+        hidden_states = hidden_states.view(-1, width)[rows]
+    elif type(hidden_states) is SlotSums:
+        hidden_states = SlotSums(hidden_states.parts[rows], (rows.numel(), width))
+    else:
+        return False, hidden_states, residual
+    return True, hidden_states, residual.view(-1, width)[rows]
 
 
 class FusedMLP(nn.Module):
@@ -678,8 +691,11 @@ class CausalLM(nn.Module):
             hidden_states, residual = done
         if short is not None:
             hidden_states = short.done(hidden_states)
+        picked = logits_rows is not None and residual is not None and input_ids.numel() > ShortPrefill.MAX_TOKENS
+        if picked:   # many rows, few of them asked for: the last norm runs on those (a row does not depend on its neighbours)
+            picked, hidden_states, residual = _rows_of(hidden_states, residual, logits_rows)
         hidden_states, _ = add_norm(hidden_states, residual, self.norm_weight, self.eps)
-        if logits_rows is not None:
+        if logits_rows is not None and not picked:
             hidden_states = hidden_states.view(-1, hidden_states.shape[-1])[logits_rows]
         if hidden_states.is_cuda and not os.environ.get("LL_LM_HEAD_LIBRARY"):
             from .kernels.quantization import dense16_linear, dense16_rows_linear, dense16_rows_wins

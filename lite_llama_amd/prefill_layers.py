@@ -28,12 +28,21 @@ def _plain(module, kind) -> bool:
 
 
 class RowParts:
-    """A projection's output left as :class:`PartialSums` of consecutive parts of its rows."""
+    """A projection's output left as the split-K planes of consecutive parts of its rows, in ``view`` (fp32)."""
 
-    __slots__ = ("parts", "shape", "dtype")
+    __slots__ = ("view", "planes", "rows", "part", "shape", "dtype")
 
-    def __init__(self, parts, shape, dtype):
-        self.parts, self.shape, self.dtype = parts, tuple(shape), dtype
+    def __init__(self, view, planes, rows, part, shape, dtype):
+        self.view, self.planes, self.rows, self.part, self.shape, self.dtype = view, planes, rows, part, tuple(shape), dtype
+
+    @property
+    def parts(self):
+        """``[planes, rows, width]`` of every part."""
+        out, width = [], self.shape[-1]
+        for i in range(-(-self.rows // self.part)):
+            rows, at = min(self.part, self.rows - i * self.part), i * _MAX_PLANES * self.part * width
+            out.append(self.view[at:at + self.planes * rows * width].view(self.planes, rows, width))
+        return out
 
     def materialise(self) -> torch.Tensor:
         return torch.cat([p.sum(0) for p in self.parts]).to(self.dtype).view(self.shape)
@@ -75,6 +84,19 @@ class ShortPrefill:
         self.parts = -(-self.tokens // 64)
         self.part = -(-self.tokens // self.parts)
         self._space = None
+        # what every layer of the pass is handed alike (the pass holds the tensors)
+        from .linear import ColumnParallelLinear, RowParallelLinear
+        from .model import Attention, DecoderLayer, FusedMLP, PagedAttention
+        from .quantization.methods import UnquantizedLinearMethod
+
+        self.kinds = (ColumnParallelLinear, RowParallelLinear, Attention, DecoderLayer, FusedMLP, PagedAttention, UnquantizedLinearMethod)
+        select, starts, lens = info.cur_select_index, info.b_start_loc, info.b_seq_len
+        self._held, self._longest = (select, starts, lens), info.max_actual_seq_len
+        self.tables = (cos.data_ptr(), sin.data_ptr(), cos.stride(0), cos.stride(1), sin.stride(0), sin.stride(1))
+        self.metadata = (select.data_ptr(), L.index_width(select), starts.data_ptr(), L.index_width(starts), lens.data_ptr(), L.index_width(lens),
+                         lens.shape[0], int(info.max_actual_seq_len))
+        self.codes = (L.dtype_code(self.dtype), L.dtype_code(cos.dtype))
+        self.run, self.stream = L.lib().ll_prefill_layer16, L.stream_ptr()
 
     def _scratch(self, row, q_size, inter):
         """Rows of 16 bits and the planes behind them, in one allocation for the pass."""
@@ -91,44 +113,48 @@ class ShortPrefill:
 
     def layer(self, layer, index: int, hidden, residual):
         """``(hidden, residual)`` as ``DecoderLayer.forward`` returns them, or ``None``: not served, nothing has run."""
-        from .linear import ColumnParallelLinear, RowParallelLinear
-        from .model import Attention, DecoderLayer, FusedMLP, PagedAttention
-        from .quantization.methods import UnquantizedLinearMethod
-
+        # (the tables of modules and parameters straight: a module's attribute lookup costs 0.3 us, and the pass looks at sixteen a layer)
+        ColumnParallelLinear, RowParallelLinear, Attention, DecoderLayer, FusedMLP, PagedAttention, Plain = self.kinds
         if not _plain(layer, DecoderLayer):
             return None
-        attn, mlp = layer.self_attn, layer.mlp
+        mods, params = layer._modules, layer._parameters
+        attn, mlp = mods.get("self_attn"), mods.get("mlp")
         if not _plain(attn, Attention) or not _plain(mlp, FusedMLP) or attn.use_qk_norm:
             return None
-        o, down, paged = attn.o_proj, mlp.down_proj, attn.attn
+        mods = attn._modules
+        o, down, paged = mods.get("o_proj"), mlp._modules.get("down_proj"), mods.get("attn")
         if not _plain(o, RowParallelLinear) or not _plain(down, RowParallelLinear) or not _plain(paged, PagedAttention):
             return None
-        if (type(o.quant_method) is not UnquantizedLinearMethod or type(down.quant_method) is not UnquantizedLinearMethod
-                or o.bias is not None or down.bias is not None):
+        # (``bias=None`` is an ordinary attribute, a bias set later is not)
+        if type(o.quant_method) is not Plain or type(down.quant_method) is not Plain or o.bias is not None or down.bias is not None:
             return None
         qkv, gate_up = attn._qkv, mlp._gate_up
         if not qkv.refresh() or not gate_up.refresh():
             return None
         qkv, gate_up = qkv._holder, gate_up._holder
-        if (qkv.interleaved or not gate_up.interleaved or type(qkv.quant_method) is not UnquantizedLinearMethod
-                or type(gate_up.quant_method) is not UnquantizedLinearMethod or gate_up.bias is not None):
+        if (qkv.interleaved or not gate_up.interleaved or type(qkv.quant_method) is not Plain or type(gate_up.quant_method) is not Plain
+                or gate_up.bias is not None):
             return None
-        heads, kv_heads, dim, width, dt = attn.num_heads, attn.num_kv_heads, attn.head_dim, self.width, self.dtype
+        heads, kv_heads, dim, width, dt, device = attn.num_heads, attn.num_kv_heads, attn.head_dim, self.width, self.dtype, self.device
         q_size, inter = heads * dim, down.input_size
         row = q_size + 2 * kv_heads * dim
         pool, info = self.info.kv_buffer[index], self.info
-        norm1, norm2 = layer.input_layernorm_weight, layer.post_attention_layernorm_weight
-        weights = ((qkv.weight, row, width), (o.weight, width, q_size), (gate_up.weight, 2 * inter, width), (down.weight, width, inter))
-        for w, n, k in weights:
-            if w.dtype != dt or w.device != self.device or tuple(w.shape) != (n, k) or not w.is_contiguous():
+        if (info.cur_select_index is not self._held[0] or info.b_start_loc is not self._held[1] or info.b_seq_len is not self._held[2]
+                or info.max_actual_seq_len != self._longest):   # (something between the layers gave the pass other metadata)
+            return None
+        norm1, norm2 = params.get("input_layernorm_weight"), params.get("post_attention_layernorm_weight")
+        w_qkv, w_o, w_gate_up, w_down, bias = qkv.weight, o._parameters.get("weight"), gate_up.weight, down._parameters.get("weight"), qkv.bias
+        if norm1 is None or norm2 is None or w_o is None or w_down is None:
+            return None
+        for w, shape in ((w_qkv, (row, width)), (w_o, (width, q_size)), (w_gate_up, (2 * inter, width)), (w_down, (width, inter))):
+            if w.dtype != dt or w.device != device or w.shape != shape or not w.is_contiguous():
                 return None
-        bias = qkv.bias
-        if bias is not None and (bias.dtype != dt or bias.device != self.device or bias.numel() != row or not bias.is_contiguous()):
+        if bias is not None and (bias.dtype != dt or bias.device != device or bias.numel() != row or not bias.is_contiguous()):
             return None
         for w in (norm1, norm2):
-            if w.dtype != dt or w.device != self.device or w.numel() != width or not w.is_contiguous():
+            if w.dtype != dt or w.device != device or w.numel() != width or not w.is_contiguous():
                 return None
-        if (pool.dtype != dt or pool.device != self.device or pool.dim() != 3 or pool.shape[1] != 2 * kv_heads or pool.shape[2] != dim or pool.stride(2) != 1
+        if (pool.dtype != dt or pool.device != device or pool.dim() != 3 or pool.shape[1] != 2 * kv_heads or pool.shape[2] != dim or pool.stride(2) != 1
                 or self.cos.shape[2] < dim // 2 or info.cur_select_index.numel() < self.tokens):
             return None
         _, buf, (x, qkv_rows, attn_rows, act_rows), planes, plane_view = self._scratch(row, q_size, inter)
@@ -136,31 +162,23 @@ class ShortPrefill:
             if not torch.is_tensor(hidden):
                 return None
             residual, planes_in = hidden, 0
-        elif type(hidden) is RowParts and hidden.parts[0].data_ptr() == planes:
-            planes_in = hidden.parts[0].shape[0]
+        elif type(hidden) is RowParts and hidden.view is plane_view:
+            planes_in = hidden.planes
         else:
             return None
-        cos, sin = self.cos, self.sin
-        left = L.lib().ll_prefill_layer16(
+        left = self.run(
             residual.data_ptr(), x, planes_in, planes, qkv_rows, attn_rows, act_rows, norm1.data_ptr(), norm2.data_ptr(), float(layer.eps),
-            qkv.weight.data_ptr(), L.ptr(bias), o.weight.data_ptr(), gate_up.weight.data_ptr(), down.weight.data_ptr(), cos.data_ptr(),
-            sin.data_ptr(), cos.stride(0), cos.stride(1), sin.stride(0), sin.stride(1), pool.data_ptr(), pool.stride(0), pool.stride(1),
-            info.cur_select_index.data_ptr(), L.index_width(info.cur_select_index), info.b_start_loc.data_ptr(),
-            L.index_width(info.b_start_loc), info.b_seq_len.data_ptr(), L.index_width(info.b_seq_len), info.b_seq_len.shape[0],
-            int(info.max_actual_seq_len), self.tokens, self.seq, width, heads, kv_heads, dim, inter, float(paged.scale * _LOG2E),
-            L.dtype_code(dt), L.dtype_code(cos.dtype), _MAX_PLANES, L.stream_ptr())
+            w_qkv.data_ptr(), 0 if bias is None else bias.data_ptr(), w_o.data_ptr(), w_gate_up.data_ptr(), w_down.data_ptr(), *self.tables,
+            pool.data_ptr(), pool.stride(0), pool.stride(1), *self.metadata, self.tokens, self.seq, width, heads, kv_heads, dim, inter,
+            float(paged.scale * _LOG2E), *self.codes, _MAX_PLANES, self.stream)
         if left == 0:
             return None
         if left < 0:
             L.check(left, "prefill_layer16")
-        sums, each = [], _MAX_PLANES * self.part * width
-        for i in range(self.parts):
-            rows = min(self.part, self.tokens - i * self.part)
-            sums.append(plane_view[i * each:i * each + left * rows * width].view(left, rows, width))
-        return RowParts(sums, (self.batch, self.seq, width), dt), residual
+        return RowParts(plane_view, left, self.tokens, self.part, (self.batch, self.seq, width), dt), residual
 
     def done(self, hidden):
         """What the layers left, as the model's other code takes it."""
         if type(hidden) is not RowParts:
             return hidden
-        return PartialSums(hidden.parts[0], hidden.shape, hidden.dtype) if len(hidden.parts) == 1 else hidden.materialise()
+        return PartialSums(hidden.parts[0], hidden.shape, hidden.dtype) if hidden.rows <= hidden.part else hidden.materialise()
