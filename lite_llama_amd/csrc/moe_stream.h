@@ -27,7 +27,9 @@ struct MoeStreamParams {
   int num_slots, a_div, block_m;
   int safe;                     // entries of `sorted` that exist whatever num_post says
   float limit;
-  int k_shift;                  // set by the launch
+  // set by the launch.  rows16: the scales of 16 rows are alike; grid_log2: 1 << that is no more than the workgroups
+  int k_shift, n_shift, rows16, grid_log2;
+  double per_workgroup, per_block, per_unit;   // 1 / workgroups, 1 / row groups of a block, 1 / units of a row
 };
 
 // whether the streaming form can take this call (how many rows per expert it pays for depends on the caller's other form); runs: of row blocks with the

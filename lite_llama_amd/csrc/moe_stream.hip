@@ -1,24 +1,30 @@
 // Grouped expert products of a few rows per expert: weights are streamed once, at the rate of memory.
 //
-//   * Persistent workgroups (one per CU; two where 8-bit weights have to be widened) own contiguous runs of 16-row groups of the weights that
-//     the step touches (row groups of all row blocks in order, dealt out to within one) and walk them in tiles of four groups, ALL of the
-//     contraction each.  Workgroups of one tile each, which this replaces where few rows meet an expert, come and go six times per CU and pay
-//     their chain of dependent loads (block -> expert and slots -> addresses -> weights) every time; here the row lists are read once, and
-//     the loads run ahead ACROSS tiles.
-//   * Four LOADER waves fill a ring of units by LDS-DMA -- 64 weight rows x 256 bytes, the block's activation rows of the same contraction
-//     range (half of their places are skipped where no block of the run fills them), 8-bit weights also their scales.  Four CONSUMER waves,
-//     one per row group, multiply from LDS (MFMA 16 x 16 x 32).  16-byte pieces of row r stand at slot ^ (r & 15): fragment reads are free of
-//     bank conflicts.  One barrier per unit.
+//   * Persistent workgroups, one per CU, own contiguous runs of 16-row groups of the weights that the step touches (row groups of all row blocks in
+//     order, dealt out to within one) and walk them in tiles of up to eight groups, ALL of the contraction each.  Workgroups of one tile each,
+//     which this replaces where few rows meet an expert, come and go six times per CU and pay their chain of dependent loads (block -> expert
+//     and slots -> addresses -> weights) every time; here the row lists are read once, and the loads run ahead ACROSS tiles.
+//   * Four LOADER waves fill a ring of units by LDS-DMA -- up to 128 weight rows x 256 bytes, the block's activation rows of the same contraction
+//     range, 8-bit weights also their scales (one request of a unit where 16 rows share them, eight where not).  Eight CONSUMER waves, one per
+//     row group, multiply from LDS (MFMA 16 x 16 x 32).  16-byte pieces of row r stand at slot ^ (r & 15): fragment reads are free of bank
+//     conflicts.  One barrier per unit.
+//   * The loaders are bound by issuing, so nothing is requested that no one reads -- neither row groups that a tile lacks nor places behind the
+//     fullest block's rows: a request of 64 zeros costs what one of weights does -- and a loader's wave goes first (s_setprio: 73.5 / 44.6 us
+//     for the two products of 64 tokens below, 71.8 / 42.0 with it).  The waits count what was really requested.
+//   * In front of the first unit stand the launch, the lists, their order, the addresses: 5 us, half of it instructions that are met for the first
+//     time.  Every loader finds the row blocks by itself, the weights of the first units are requested before any slot is known, and there is no
+//     integer division on the way (with them: 1 us more for both products).
 //   * An expert's contraction begins at unit e mod units and wraps: experts whose rows are a power of two long do not all ask the same
 //     memory channels, and the order of a sum depends on the expert alone, not on what else rides along.
-//   * Bound by memory, the chain in front of the first unit (about 5 us) and, for 8-bit weights, the widening between two barriers: a second
-//     workgroup per CU fills those gaps (128 experts of 2048 / 768 in 8-bit floats, 64 tokens with 8 each, both products: 128 us with one
-//     workgroup per CU, 117 with two; 16-bit weights gain nothing by it).  Ring depths of 4 to 6 units are alike.
-//   us for both products, tiles -> here.  8-bit floats, 128 experts of 2048 / 768, top 8: 1 token 42 -> 24, 8 67 -> 54, 32 120 -> 102, 64
-//   137 -> 117 (604 MB: 5.2 TB/s); in pieces of 32 rows (of 16) 200 167 -> 155 (167), 256 178 -> 162 (209), 320 181 -> 168, 400 186 -> 191.  bf16, 34 of 2048 / 704, top 4: 1 token 33 -> 17, 32 tokens 77 -> 58, 128 78 -> 65; 68 of 3072 / 512,
-//   top 8: 6 tokens 89 -> 74, 32 156 -> 111 (642 MB), 128 160 -> 126; in pieces of 64 rows 160 tokens 161 -> 131, 262 (31 rows per expert) 165 ->
-//   150 (pieces of 32: 185), 34 experts 200 77 -> 73, 300 (35) 78.5 -> 77, 400 (47) 80 -> 85: up to 36 rows per expert in ll_moe_rows_gemm.  ll_moe_gemm has other
-//   tiles and lines of its own (moe.hip).
+//   * Rows of 128 bytes in units twice as many: 80 / 46 us where these take 72 / 42 (memory answers half lines of 256 bytes worse).  Tiles of four
+//     groups, two workgroups per CU for 8-bit weights, which this replaces: the second one of a CU came 10 us late, and a tile of one group
+//     took as long as one of four.  us for both products, that -> here: 8-bit floats, 128 experts of 2048 / 768, top 8: 1 token 34 -> 29.9,
+//     8 70 -> 65, 32 108 -> 102, 64 124 -> 119 (604 MB: 5.1 TB/s), 128 140 -> 136, 200 169 -> 151, 256 174 -> 155, 320 191 -> 192; bf16, 34 of
+//     2048 / 704, top 4: 1 21.2 -> 21.1, 4 42 -> 33, 32 63 -> 59, 128 68 -> 62, 262 81 -> 67; 68 of 3072 / 512, top 8: 1 27.8 -> 29.1 (24 units
+//     of two groups in a row: latency), 6 69 -> 67, 32 119 -> 114, 128 133 -> 124, 262 159 -> 135.
+//   Lines against the tiles (before that change; us, tiles -> streams): 8-bit floats, 128 of 2048 / 768: 1 token 42 -> 24, 64 137 -> 117, 320 181 ->
+//   168, 400 186 -> 191; bf16, 34 of 2048 / 704, top 4: 1 token 33 -> 17, 128 78 -> 65, 300 (35 rows per expert) 78.5 -> 77, 400 (47) 80 -> 85; 68 of
+//   3072 / 512: 262 (31) 165 -> 150: up to 36 rows per expert in ll_moe_rows_gemm.  ll_moe_gemm has other tiles and lines of its own (moe.hip).
 #include <stdlib.h>
 
 #include "gemm_w4_common.h"
@@ -29,25 +35,27 @@ namespace {
 typedef __bf16 ms_bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int MS_LIST = 512, MS_OWN = 8;   // row blocks in all / of one workgroup
-constexpr int MS_W_BYTES = 64 * 256;
+constexpr int MS_WAVES = 12;               // eight consumers, four loaders
+constexpr int MS_KB = 256;                 // bytes of a weight row in a unit
 
 template <int WF, int MT_>
 struct MsLds {
-  static constexpr int THREADS = 512;                          // four consumers, four loaders
-  static constexpr int PER_CU = WF != MS_W16 && MT_ == 1 ? 2 : 1, RING = PER_CU == 2 ? 3 : 4;
+  static constexpr int THREADS = MS_WAVES * 64;
   static constexpr int MT = MT_, ROWS = 16 * MT;               // rows of a piece of a block
   static constexpr int KU = WF == MS_W16 ? 128 : 256;          // contraction entries of a unit
-  static constexpr int X_BYTES = ROWS * KU * 2;
-  static constexpr int S_BYTES = WF == MS_W16 ? 0 : 64 * 4 * 4;   // scales: [loader][64-column step][16 rows]
-  static constexpr int SLOT = MS_W_BYTES + X_BYTES + S_BYTES;
-  static constexpr int LIST = RING * SLOT;                  // int32 [MS_LIST]: row block | expert << 16
-  static constexpr int OWN = LIST + MS_LIST * 4;   // int32 [MS_OWN]: expert
-  static constexpr int SLOTS = OWN + MS_OWN * 4;               // int32 [MS_OWN][ROWS]
-  static constexpr int WEIGHTS = SLOTS + MS_OWN * ROWS * 4;    // float [MS_OWN][ROWS]
-  static constexpr int COUNTS = WEIGHTS + MS_OWN * ROWS * 4;   // int32 [8], [1]
-  static constexpr int BYTES = COUNTS + 48;                    // (nothing static: the ring begins at LDS byte 0)
-  static_assert(BYTES * PER_CU <= 160 * 1024, "LDS");
-  static constexpr int XOPS = X_BYTES / 4096;                  // activation operations per loader and unit
+  static constexpr int XB = KU * 2;                            // bytes of an activation row per unit
+  static constexpr int X_BYTES = ROWS * XB;
+  static constexpr int S_BYTES = WF == MS_W16 ? 0 : 8 * 4 * 16 * 4;   // scales: [row group][64-column step][16 rows], or, alike in 16 rows, [row group][step]
+  static constexpr int slot(int groups) { return groups * 16 * MS_KB + X_BYTES + S_BYTES; }   // of the ring: three units of eight row groups, four of four
+  static constexpr int LIST = 3 * slot(8);                  // int32 [MS_LIST]: row block | expert << 16
+  static constexpr int SLOTS = LIST + MS_LIST * 4;             // int32 [MS_OWN][ROWS]
+  static constexpr int FROM = SLOTS + MS_OWN * ROWS * 4;       // uint32 [MS_OWN][ROWS]: where the slot's activations begin, bytes
+  static constexpr int WEIGHTS = FROM + MS_OWN * ROWS * 4;     // float [MS_OWN][ROWS]
+  static constexpr int COUNTS = WEIGHTS + MS_OWN * ROWS * 4;   // int32: pieces, skipped, most rows
+  static constexpr int BYTES = COUNTS + 16;                    // (nothing static: the ring begins at LDS byte 0)
+  static_assert(BYTES <= 160 * 1024, "LDS");
+  static constexpr int XOPS = X_BYTES / 4096;                  // activation operations per loader and unit, at most
+  static_assert(4 * slot(4) <= LIST && 8 + 2 + XOPS <= 18 && 2 * (4 + 1 + XOPS) <= 18, "the ring, the waits");
 };
 
 __device__ const uint32_t ms_zeros[4] __attribute__((aligned(16))) = {0, 0, 0, 0};   // what pieces without an entry read
@@ -60,12 +68,30 @@ __device__ __forceinline__ void ms_dma16(uint32_t dst, const void* src) {
                : "=&s"(keep) : "s"(dst), "v"(src) : "memory");
 }
 
-template <int OPS>
-__device__ __forceinline__ void ms_wait_units(int k) {   // at most k units of OPS operations each may still be in flight
-  if (k <= 0) v3_vmcnt<0>();
-  else if (k == 1) v3_vmcnt<OPS>();
-  else v3_vmcnt<2 * OPS>();
+__device__ __forceinline__ void ms_wait(int k) {   // at most k operations may still be in flight
+#define MS_C(K) case K: v3_vmcnt<K>(); break;
+  switch (k) {
+    MS_C(1) MS_C(2) MS_C(3) MS_C(4) MS_C(5) MS_C(6) MS_C(7) MS_C(8) MS_C(9) MS_C(10) MS_C(11) MS_C(12) MS_C(13) MS_C(14) MS_C(15) MS_C(16) MS_C(17) MS_C(18)
+    default: v3_vmcnt<0>(); break;
+  }
+#undef MS_C
 }
+
+// A run of row groups in tiles of at most eight groups of one row block, the last two of a segment alike.
+struct MsWalk {
+  int i, r0, left;   // row block and group in it of the next tile, groups of the run not yet in a tile
+  __device__ __forceinline__ int open(int rgs) {   // the next tile's groups: r0 - its groups .. r0 of row block i
+    if (r0 == rgs) {
+      ++i;
+      r0 = 0;
+    }
+    const int s = rgs - r0 < left ? rgs - r0 : left;
+    const int h = s <= 8 ? s : s <= 16 ? (s + 1) >> 1 : 8;
+    r0 += h;
+    left -= h;
+    return h;
+  }
+};
 
 // eight 8-bit weights -> fp16, exactly (8-bit floats: times 2^-8; the codes 0x7f and 0xff as 480, as in moe.hip)
 template <int WF>
@@ -110,108 +136,137 @@ __device__ __forceinline__ float ms_glu(float g, float u, float limit) {
   return g * ll_sigmoidf(g) * u;
 }
 
-template <int WF, int MT, int MODE, int XOPS>
-__device__ __forceinline__ void ms_load(const MoeStreamParams& p, unsigned char* lds, int L, int lane, int lo, int hi, int rgs, int i0, int units, int total) {
+__device__ __forceinline__ int ms_over(int n, double inverse) {   // n / d, exactly: 0 <= n < 2^31, inverse = 1 / d, d < 2^20
+  return __builtin_amdgcn_readfirstlane((int)(((double)n + 0.5) * inverse));
+}
+
+// GROUPS: the run's tiles have no more row groups than that
+template <int WF, int MT, int MODE, int GROUPS>
+__device__ __forceinline__ void ms_load(const MoeStreamParams& p, unsigned char* lds, int L, int lane, MsWalk run, int rgs, int i0, int units, int total) {
   using LD = MsLds<WF, MT>;
-  constexpr int KU = LD::KU, EB = WF == MS_W16 ? 2 : 1, ROWS = LD::ROWS;
-  constexpr int OPS = 4 + XOPS + (WF == MS_W16 ? 0 : 1);
-  const int32_t* experts = reinterpret_cast<const int32_t*>(lds + LD::OWN);
-  const int32_t* rows = reinterpret_cast<const int32_t*>(lds + LD::SLOTS);
+  constexpr int KU = LD::KU, EB = WF == MS_W16 ? 2 : 1, ROWS = LD::ROWS, XOPS = LD::XOPS, XL = LD::XB / 16;   // lanes of an activation row
+  constexpr int RING = GROUPS == 4 ? 4 : 3, W_BYTES = GROUPS * 16 * MS_KB, SLOT = LD::slot(GROUPS);
+  const uint32_t* list = reinterpret_cast<const uint32_t*>(lds + LD::LIST);
+  const int32_t* rows = reinterpret_cast<const int32_t*>(lds + LD::FROM);
   const int row_bytes = p.K * EB;
+  // ---- weights (and scales) of the next unit.  (piece `at` of row r stands at at ^ (r & 15))
+  MsWalk wrun = run;
   const char *wbase = nullptr, *sbase = nullptr;   // the expert's matrix and scales
-  uint32_t woff[4], xoff[XOPS], soff = 0;          // where this lane's pieces of unit 0 begin
-  bool live = false;
-  int rg = lo, unit = 0, left = 0, issued = 0;
-  uint32_t dst = 0;
-  // (piece `at` of row r comes from byte 16 (at ^ (r & 15)) of it)
-  auto open = [&]() {   // the tile at row group rg
-    const int i = rg / rgs, r0 = rg - i * rgs;
-    const int e = __builtin_amdgcn_readfirstlane(experts[i - i0]);
-    int groups = rgs - r0 < 4 ? rgs - r0 : 4;
-    groups = hi - rg < groups ? hi - rg : groups;
-    live = L < groups;
-    const int g = r0 + L;
-    wbase = (const char*)p.w + (int64_t)e * p.w_stride_e;
+  uint32_t woff[GROUPS], soff[2] = {0, 0};                      // where this lane's pieces of unit 0 begin
+  int wunit = 0, wleft = 0, groups = 0;
+  uint32_t wdst = 0;
+  auto weights = [&]() {
+    if (wleft == 0) {
+      groups = wrun.open(rgs);
+      const int e = __builtin_amdgcn_readfirstlane((int)(list[wrun.i] >> 16)), r0 = wrun.r0 - groups;
+      wbase = (const char*)p.w + (int64_t)e * p.w_stride_e;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int r = 4 * j + (lane >> 4);
-      int row;
-      if constexpr (MODE == MS_GLU) {
-        row = 8 * g + (r >> 1);
-        row = (row < p.N ? row : p.N - 1) + (r & 1 ? p.N : 0);
-      } else {
-        row = 16 * g + r;
-        row = row < p.N ? row : p.N - 1;   // rows behind N feed results that are not stored
+      for (int j = 0; j < GROUPS; ++j) {
+        const int r = 4 * L + (lane >> 4), g = r0 + j;
+        int row;
+        if constexpr (MODE == MS_GLU) {
+          row = 8 * g + (r >> 1);
+          row = (row < p.N ? row : p.N - 1) + (r & 1 ? p.N : 0);
+        } else {
+          row = 16 * g + r;
+          row = row < p.N ? row : p.N - 1;   // rows behind N feed results that are not stored
+        }
+        woff[j] = (uint32_t)row * (uint32_t)p.w_stride_n + ((lane & 15) ^ r) * 16;
       }
-      woff[j] = (uint32_t)row * (uint32_t)p.w_stride_n + ((lane & 15) ^ r) * 16;
-    }
-    const int32_t* own = rows + (i - i0) * ROWS;
+      if constexpr (WF != MS_W16) {
+        sbase = (const char*)(p.scales + (int64_t)e * p.s_stride_e);
 #pragma unroll
-    for (int j = 0; j < XOPS; ++j) {
-      const int at = L + 4 * j;
-      const int r = WF == MS_W16 ? 4 * at + (lane >> 4) : 2 * at + (lane >> 5);
-      const int slot = own[r];   // (places without a slot read row 0: they feed results that are not stored)
-      xoff[j] = (slot < p.num_slots ? (uint32_t)(slot / p.a_div) * (uint32_t)(p.a_ld * 2) : 0u) +
-                ((WF == MS_W16 ? (lane & 15) : (lane & 31)) ^ (r & 15)) * 16;
+        for (int j = 0; j < GROUPS / 4; ++j) {
+          int row = p.rows16 ? 16 * (r0 + (lane >> 2)) : 16 * (r0 + 4 * j + L) + (lane & 15);
+          row = row < p.N ? row : p.N - 1;
+          soff[j] = (uint32_t)(p.n_shift >= 0 ? row >> p.n_shift : row / (int)p.group_n) * (uint32_t)(p.s_stride_n * 4);
+        }
+      }
+      wunit = e - ms_over(e, p.per_unit) * units;
+      wleft = units;
+    }
+    const int at = wunit * MS_KB;
+    const bool whole = at + MS_KB <= row_bytes;
+    const int piece = ((lane & 15) ^ (4 * L + (lane >> 4))) * 16;
+#pragma unroll
+    for (int j = 0; j < GROUPS; ++j) {
+      const uint32_t dst = wdst + (4 * j + L) * 1024;
+      if (j >= groups) break;
+      if (whole) v3_dma16<true>(dst, wbase + at, woff[j]);
+      else ms_dma16(dst, at + piece < row_bytes ? wbase + at + woff[j] : (const char*)ms_zeros);   // the contraction ends inside the unit: zeros behind it, on both sides
     }
     if constexpr (WF != MS_W16) {
-      int row = 16 * g + (lane & 15);
-      row = row < p.N ? row : p.N - 1;
-      sbase = (const char*)(p.scales + (int64_t)e * p.s_stride_e);
-      soff = (uint32_t)(row / (int)p.group_n) * (uint32_t)(p.s_stride_n * 4);
+      int k = wunit * KU + (p.rows16 ? lane & 3 : lane >> 4) * 64;
+      k = k < p.K ? k : p.K - 1;
+#pragma unroll
+      for (int j = 0; j < GROUPS / 4; ++j)
+        if (p.rows16 ? j == 0 && L == 3 : 4 * j + L < groups) v3_dma4<false>(wdst + W_BYTES + LD::X_BYTES + (p.rows16 ? 0 : (4 * j + L) * 256), sbase, soff[j] + (uint32_t)(k >> p.k_shift) * (uint32_t)(p.s_stride_k * 4));
     }
-    unit = e % units;
-    left = units;
-    rg += groups;
+    if (++wunit == units) wunit = 0;
+    --wleft;
+    wdst = wdst + SLOT == RING * SLOT ? 0 : wdst + SLOT;
   };
-  auto issue = [&]() {
-    if (left == 0) open();
-    const int at = unit * 256, xat = unit * (KU * 2);
-    if (at + 256 <= row_bytes) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if (live) v3_dma16<true>(dst + (4 * L + j) * 1024, wbase + at, woff[j]);
-        else v3_dma16<false>(dst + (4 * L + j) * 1024, ms_zeros, 0u);
-      }
-#pragma unroll
-      for (int j = 0; j < XOPS; ++j) v3_dma16<false>(dst + MS_W_BYTES + (L + 4 * j) * 1024, (const char*)p.a + xat, xoff[j]);
-    } else {   // the contraction ends inside the unit: zeros behind it, on both sides
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int piece = ((lane & 15) ^ (4 * j + (lane >> 4))) * 16;
-        ms_dma16(dst + (4 * L + j) * 1024, live && at + piece < row_bytes ? wbase + at + woff[j] : (const char*)ms_zeros);
-      }
+  // ---- its activations
+  MsWalk xrun = run;
+  uint32_t xoff[XOPS];
+  int xunit = 0, xleft = 0, xops = 0;
+  uint32_t xdst = W_BYTES;
+  auto xrow = [&](int j) { return (L + 4 * j) * (64 / XL) + lane / XL; };   // (pieces stand at at ^ (r & 15))
+  auto xpiece = [&](int j) { return (uint32_t)(lane % XL ^ (xrow(j) & 15)) * 16; };
+  auto activations = [&]() {
+    if (xleft == 0) {
+      (void)xrun.open(rgs);
+      const int32_t* own = rows + (xrun.i - i0) * ROWS;
 #pragma unroll
       for (int j = 0; j < XOPS; ++j) {
-        const int r = WF == MS_W16 ? 4 * (L + 4 * j) + (lane >> 4) : 2 * (L + 4 * j) + (lane >> 5);
-        const int piece = ((WF == MS_W16 ? (lane & 15) : (lane & 31)) ^ (r & 15)) * 16;
-        ms_dma16(dst + MS_W_BYTES + (L + 4 * j) * 1024, xat + piece < p.K * 2 ? (const char*)p.a + xat + xoff[j] : (const char*)ms_zeros);
+        xoff[j] = (uint32_t)own[xrow(j)] + xpiece(j);   // (places without a slot read row 0: they feed results that are not stored)
       }
+      const int e = __builtin_amdgcn_readfirstlane((int)(list[xrun.i] >> 16));
+      xunit = e - ms_over(e, p.per_unit) * units;
+      xleft = units;
     }
-    if constexpr (WF != MS_W16) {
-      int k = unit * KU + (lane >> 4) * 64;
-      k = k < p.K ? k : p.K - 1;
-      v3_dma4<false>(dst + MS_W_BYTES + LD::X_BYTES + L * 256, sbase, soff + (uint32_t)(k >> p.k_shift) * (uint32_t)(p.s_stride_k * 4));
+    const int xat = xunit * LD::XB;
+    const bool whole = xat + LD::XB <= p.K * 2;
+#pragma unroll
+    for (int j = 0; j < XOPS; ++j) {
+      const uint32_t dst = xdst + (L + 4 * j) * 1024;
+      if (j >= xops) break;
+      if (whole) v3_dma16<false>(dst, (const char*)p.a + xat, xoff[j]);
+      else ms_dma16(dst, xat + (int)xpiece(j) < p.K * 2 ? (const char*)p.a + xat + xoff[j] : (const char*)ms_zeros);
     }
-    if (++unit == units) unit = 0;
-    --left;
-    ++issued;
-    dst = dst + LD::SLOT == LD::RING * LD::SLOT ? 0 : dst + LD::SLOT;
+    if (++xunit == units) xunit = 0;
+    --xleft;
+    xdst = xdst + SLOT == RING * SLOT + W_BYTES ? W_BYTES : xdst + SLOT;
   };
-  const int pre = total < LD::RING - 1 ? total : LD::RING - 1;
-  for (int i = 0; i < pre; ++i) issue();
-  ms_wait_units<OPS>(issued - 1);
+  __builtin_amdgcn_s_setprio(3);   // (a consumer's arithmetic does not keep a request waiting)
+  // the weights of the whole ring are on their way before the slots are known
+  const int pre = total < RING - 1 ? total : RING - 1;
+  for (int i = 0; i < pre; ++i) weights();
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // slots
+  const int full = __builtin_amdgcn_readfirstlane(reinterpret_cast<const int*>(lds + LD::COUNTS)[2]);   // rows of the fullest block of the run
+  xops = (full - L * (64 / XL) + 256 / XL - 1) / (256 / XL);   // this wave's requests of a unit that hold any of them
+  xops = xops < 0 ? 0 : xops < XOPS ? xops : XOPS;
+  for (int i = 0; i < pre; ++i) activations();
+  ms_wait((pre - 1) * xops);   // (the activations of the first ring follow all its weights)
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // P0: unit 0 has landed
+  int ops = 0, before = 0;   // requests of the last unit and the one before it
   for (int u = 0; u < total; ++u) {
-    if (issued < total) issue();   // into the slot of unit u - 1, free since the barrier that ended it
-    const int need = total < u + 2 ? total : u + 2;
-    ms_wait_units<OPS>(issued - need);   // unit u + 1 has landed before the consumers are released into it
+    const bool more = u + RING - 1 < total;
+    if (more) {   // into the slot of unit u - 1, free since the barrier that ended it
+      weights();
+      activations();
+      before = ops;
+      ops = groups + xops + (WF == MS_W16 ? 0 : p.rows16 ? L == 3 : (groups > L) + (groups > 4 + L));
+    }
+    // unit u + 1 has landed before the consumers are released into it: behind it are the last RING - 2
+    if constexpr (RING == 3) ms_wait(more ? ops : 0);
+    else ms_wait(more ? ops + (u > 0 ? before : 0) : u + 3 == total && u > 0 ? ops : 0);
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // B_u
   }
 }
 
 template <int DT, int WF, int MT, int MODE>
-__global__ __launch_bounds__((MsLds<WF, MT>::THREADS)) __attribute__((amdgpu_waves_per_eu(2 * (MsLds<WF, MT>::PER_CU), 2 * (MsLds<WF, MT>::PER_CU)))) void moe_stream_kernel(const MoeStreamParams p) {
+__global__ __launch_bounds__((MsLds<WF, MT>::THREADS)) __attribute__((amdgpu_waves_per_eu(3, 3))) void moe_stream_kernel(const MoeStreamParams p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   using LD = MsLds<WF, MT>;
   constexpr int KU = LD::KU, ROWS = LD::ROWS, THREADS = LD::THREADS;
@@ -219,100 +274,120 @@ __global__ __launch_bounds__((MsLds<WF, MT>::THREADS)) __attribute__((amdgpu_wav
   uint32_t* list = reinterpret_cast<uint32_t*>(lds + LD::LIST);
   int32_t* rows = reinterpret_cast<int32_t*>(lds + LD::SLOTS);
   float* weights = reinterpret_cast<float*>(lds + LD::WEIGHTS);
-  int* part = reinterpret_cast<int*>(lds + LD::COUNTS);
-  int* most_rows = part + 8;
+  int* counts = reinterpret_cast<int*>(lds + LD::COUNTS);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int sub = p.block_m / ROWS;                       // pieces of ROWS rows per block
   const int rgs = MODE == MS_GLU ? (p.N + 7) / 8 : (p.N + 15) / 16;
   const int nout = MODE == MS_GLU_ROUNDED ? p.N / 2 : p.N;
-  if (tid == 0) *most_rows = 0;
-
-  // the pieces with a slot, in order (a block's slots stand in front).  Lists are requested before num_post is known, as far as they exist.
-  const int cap = (p.safe + ROWS - 1) / ROWS;
-  int first = p.num_slots, expert = 0;
-  if (tid < cap) {
-    first = p.sorted[tid * ROWS];
-    expert = p.block_expert[tid / sub];
-  }
-  int post = p.num_post[0];
-  asm volatile("" : "+v"(first), "+v"(expert), "+s"(post));   // (requested together)
-  const int pieces = post / ROWS;
+  const int units = (p.K + KU - 1) / KU;
+  const int b = (int)blockIdx.x, grid = (int)gridDim.x;
   int count = 0, skipped = 0;
-  for (int j0 = 0; j0 < pieces; j0 += THREADS) {
-    const int j = j0 + tid;
-    if ((j0 > 0 || tid >= cap) && j < pieces) {
-      first = p.sorted[j * ROWS];
-      expert = p.block_expert[j / sub];
-    }
-    const bool has = j < pieces && first < p.num_slots, in = has && expert >= 0;
-    const unsigned long long mask = __ballot(in), none = __ballot(has && expert < 0);
-    if (lane == 0) part[wv] = __popcll(mask) | __popcll(none) << 16;
-    __syncthreads();
-    int at = count, behind = skipped;
-    for (int w = 0; w < THREADS / 64; ++w) {
-      const int n = part[w];
-      if (w < wv) {
-        at += n & 0xffff;
-        behind += n >> 16;
+
+  // The pieces with a slot, in order (a block's slots stand in front).  Every loader wave finds them for itself -- the same values to the same
+  // places -- so that its first request waits for no barrier; lists are requested before num_post is known, as far as they exist.
+  if (wv >= 8) {
+    constexpr int AHEAD = 4;
+    const int cap = (p.safe + ROWS - 1) / ROWS;
+    int first[AHEAD], expert[AHEAD];
+#pragma unroll
+    for (int c = 0; c < AHEAD; ++c) {
+      const int j = 64 * c + lane;
+      first[c] = p.num_slots;
+      expert[c] = 0;
+      if (j < cap) {
+        first[c] = p.sorted[j * ROWS];
+        expert[c] = p.block_expert[sub == 1 ? j : j / sub];
       }
-      count += n & 0xffff;
-      skipped += n >> 16;
     }
-    const unsigned long long below = (1ull << lane) - 1ull;
-    at += __popcll(mask & below);
-    behind = MS_LIST - 1 - (behind + __popcll(none & below));
-    if (in && at < MS_LIST) list[at] = (uint32_t)j | (uint32_t)expert << 16;
-    if (has && expert < 0 && behind >= 0) list[behind] = (uint32_t)j;
-    __syncthreads();
+    int post = p.num_post[0];
+    asm volatile("" : "+v"(first[0]), "+v"(first[1]), "+v"(first[2]), "+v"(first[3]), "+v"(expert[0]), "+v"(expert[1]), "+v"(expert[2]), "+v"(expert[3]), "+s"(post));   // (requested together)
+    const int pieces = post / ROWS;
+    auto take = [&](int j, int slot, int e) {
+      const bool has = j < pieces && slot < p.num_slots, in = has && e >= 0;
+      const unsigned long long mask = __ballot(in), none = __ballot(has && e < 0), below = (1ull << lane) - 1ull;
+      const int at = count + __popcll(mask & below), behind = MS_LIST - 1 - (skipped + __popcll(none & below));
+      if (in && at < MS_LIST) list[at] = (uint32_t)j | (uint32_t)e << 16;
+      if (has && e < 0 && behind >= 0) list[behind] = (uint32_t)j;
+      count += __popcll(mask);
+      skipped += __popcll(none);
+    };
+#pragma unroll
+    for (int c = 0; c < AHEAD; ++c)
+      if (64 * c < pieces) take(64 * c + lane, first[c], expert[c]);
+    for (int j = 64 * AHEAD + lane; j - lane < pieces; j += 64) {
+      int slot = p.num_slots, e = 0;
+      if (j < pieces) {
+        slot = p.sorted[j * ROWS];
+        e = p.block_expert[sub == 1 ? j : j / sub];
+      }
+      take(j, slot, e);
+    }
+    counts[0] = count;
+    counts[1] = skipped;
+    counts[2] = 0;
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // lists
+  if (wv < 8) {
+    count = counts[0];
+    skipped = counts[1];
   }
   count = __builtin_amdgcn_readfirstlane(count);
   skipped = __builtin_amdgcn_readfirstlane(skipped);
-  if constexpr (!PAIRS) {   // slots that no expert serves: zeros (of the last product; nothing reads the first one's)
-    for (int t = (int)blockIdx.x; t < skipped * ROWS; t += (int)gridDim.x) {
-      const int slot = p.sorted[(int)list[MS_LIST - 1 - t / ROWS] * ROWS + t % ROWS];
-      if (slot < p.num_slots)
-        for (int c = tid; c < p.N; c += THREADS) p.out[(int64_t)slot * p.out_ld + c] = 0;
-    }
+  // Runs to within one row group.  (Divisions by multiplication with what the host hands over: nothing is requested before this is through.)
+  const int total_rg = count * rgs, each = ms_over(total_rg, p.per_workgroup), more = total_rg - each * grid;
+  int lo = each * b + (b < more ? b : more), hi = lo + each + (b < more ? 1 : 0), i0, own;   // own: row blocks of this run
+  const int lg = count > 1 ? 32 - __builtin_clz(count - 1) : 0, per = p.grid_log2 - lg;   // (1 << per workgroups per row block)
+  if (each < 8 && count > 0 && per >= 4 && rgs <= (each + 2) << per) {
+    // few blocks: runs within one, hardly longer ones -- a run across an end is two tiles, which is twice the time (one token, 4 of 40 experts of
+    // 2048 / 712: 25.9 -> 21.9 us for both products; 4 tokens, 16 of 34 of 2048 / 704: 38.3 -> 33.2)
+    i0 = b >> per;
+    own = i0 < count ? 1 : 0;
+    const int w = b & ((1 << per) - 1), part = rgs >> per, rest = rgs & ((1 << per) - 1);
+    lo = i0 * rgs + part * w + (w < rest ? w : rest);
+    hi = own ? lo + part + (w < rest ? 1 : 0) : lo;
+    own = lo < hi ? 1 : 0;
+  } else {
+    i0 = ms_over(lo, p.per_block);
+    own = lo < hi ? ms_over(hi - 1, p.per_block) - i0 + 1 : 0;
   }
-  const int64_t total_rg = (int64_t)count * rgs;
-  const int b = (int)blockIdx.x, grid = (int)gridDim.x;
-  const int lo = (int)(total_rg * b / grid), hi = (int)(total_rg * (b + 1) / grid);
-  if (lo >= hi) return;
-  const int i0 = lo / rgs, own = (hi - 1) / rgs - i0 + 1;   // row blocks of this run
-  if (tid < own) reinterpret_cast<int32_t*>(lds + LD::OWN)[tid] = (int)(list[i0 + tid] >> 16);
-  if (tid < own * ROWS) {
-    const int slot = p.sorted[(int)(list[i0 + tid / ROWS] & 0xffffu) * ROWS + tid % ROWS];
-    rows[tid] = slot;
-    if (slot < p.num_slots) atomicMax(most_rows, tid % ROWS + 1);
-  }
-  __syncthreads();
-  const int units = (p.K + KU - 1) / KU;
-  int tiles = 0;
-  for (int rg = lo; rg < hi; ++tiles) {
-    const int r0 = rg % rgs;
-    int groups = rgs - r0 < 4 ? rgs - r0 : 4;
-    rg += hi - rg < groups ? hi - rg : groups;
-  }
-  const int total = tiles * units;
-  const int full = __builtin_amdgcn_readfirstlane(*most_rows);
-
-  if (wv >= 4) {
-    if (full > ROWS / 2) ms_load<WF, MT, MODE, LD::XOPS>(p, lds, wv - 4, lane, lo, hi, rgs, i0, units, total);
-    else ms_load<WF, MT, MODE, LD::XOPS / 2>(p, lds, wv - 4, lane, lo, hi, rgs, i0, units, total);
+  MsWalk run{i0, lo - i0 * rgs, hi - lo};
+  const bool small = run.left <= 4;
+  const int slot_bytes = small ? LD::slot(4) : LD::slot(8), w_bytes = slot_bytes - LD::X_BYTES - LD::S_BYTES, ring = small ? 4 : 3;
+  if (wv >= 8) {
+    if (lo >= hi) return;   // (as a whole: the consumers behind their zeros)
+    __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0), for the compiler: it would wait for the lists' registers between the requests
+    const int head = rgs - run.r0 < run.left ? rgs - run.r0 : run.left, tail = run.left - head - (own - 2) * rgs;
+    const int total = units * ((head + 7) / 8 + (own > 1 ? (own - 2) * ((rgs + 7) / 8) + (tail + 7) / 8 : 0));
+    if (small) ms_load<WF, MT, MODE, 4>(p, lds, wv - 8, lane, run, rgs, i0, units, total);
+    else ms_load<WF, MT, MODE, 8>(p, lds, wv - 8, lane, run, rgs, i0, units, total);
     return;
   }
 
   // consumers: row group wv of every tile
-  for (int i = tid; i < own * ROWS; i += 256) {
-    const int slot = rows[i];
-    float v = 1.f;
-    if (slot < p.num_slots) {
-      if (p.weight32) v = p.weight32[slot];
-      else if (p.weight16) v = f16_bits_to_f32(p.weight16[slot]);
-    }
-    weights[i] = v;
+  static_assert(MS_OWN * ROWS <= 512, "a thread per slot");
+  int slot = p.num_slots;
+  if (tid < own * ROWS) {
+    slot = p.sorted[(int)(list[i0 + tid / ROWS] & 0xffffu) * ROWS + tid % ROWS];
+    rows[tid] = slot;
+    reinterpret_cast<uint32_t*>(lds + LD::FROM)[tid] = slot < p.num_slots ? (uint32_t)(p.a_div == 1 ? slot : slot / p.a_div) * (uint32_t)(p.a_ld * 2) : 0u;
+    if (slot < p.num_slots) atomicMax(counts + 2, tid % ROWS + 1);
   }
+  if (lo < hi) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // slots
+  uint32_t weight_bits = 0;   // (on its way until the first unit has landed)
+  if (slot < p.num_slots) {
+    if (p.weight32) weight_bits = reinterpret_cast<const uint32_t*>(p.weight32)[slot];
+    else if (p.weight16) weight_bits = p.weight16[slot];
+  }
+  if constexpr (!PAIRS) {   // slots that no expert serves: zeros (of the last product; nothing reads the first one's)
+    for (int t = b; t < skipped * ROWS; t += grid) {
+      const int slot = p.sorted[(int)list[MS_LIST - 1 - t / ROWS] * ROWS + t % ROWS];
+      if (slot < p.num_slots)
+        for (int c = tid; c < p.N; c += 512) p.out[(int64_t)slot * p.out_ld + c] = 0;
+    }
+  }
+  if (lo >= hi) return;
+  const int full = __builtin_amdgcn_readfirstlane(counts[2]);
   const int r = lane & 15, q = lane >> 4;
   f32x4 acc[MT];
 #pragma unroll
@@ -320,15 +395,14 @@ __global__ __launch_bounds__((MsLds<WF, MT>::THREADS)) __attribute__((amdgpu_wav
   const bool wide = ((PAIRS ? 2 : 4) * 2 - 1 & (int)(reinterpret_cast<uintptr_t>(p.out) | (uintptr_t)(p.out_ld * 2))) == 0;
   uint32_t slot_at = 0;
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // P0
-  for (int rg = lo; rg < hi;) {
-    const int i = rg / rgs, r0 = rg - i * rgs;
-    int groups = rgs - r0 < 4 ? rgs - r0 : 4;
-    groups = hi - rg < groups ? hi - rg : groups;
+  if (tid < own * ROWS) weights[tid] = slot >= p.num_slots ? 1.f : p.weight32 ? __uint_as_float(weight_bits) : p.weight16 ? f16_bits_to_f32((uint16_t)weight_bits) : 1.f;
+  while (run.left > 0) {
+    const int groups = run.open(rgs), i = run.i, r0 = run.r0 - groups;
     const bool mine = wv < groups;
     for (int u = 0; u < units; ++u) {
       if (mine) {
-        const unsigned char* wb = lds + slot_at + wv * 4096 + r * 256;
-        const unsigned char* xb = lds + slot_at + MS_W_BYTES + r * (KU * 2);
+        const unsigned char* wb = lds + slot_at + wv * 4096 + r * MS_KB;
+        const unsigned char* xb = lds + slot_at + w_bytes + r * LD::XB;
         // (all fragments of the unit are requested before the first is used: one wave per matrix core waits for LDS once)
         if constexpr (WF == MS_W16) {
           u32x4 wf[4], x[MT][4];
@@ -338,7 +412,7 @@ __global__ __launch_bounds__((MsLds<WF, MT>::THREADS)) __attribute__((amdgpu_wav
           for (int m = 0; m < MT; ++m)
             if (m == 0 || 16 * m < full)
 #pragma unroll
-              for (int s = 0; s < 4; ++s) x[m][s] = *reinterpret_cast<const u32x4*>(xb + 16 * m * KU * 2 + ((4 * s + q) ^ r) * 16);
+              for (int s = 0; s < 4; ++s) x[m][s] = *reinterpret_cast<const u32x4*>(xb + 16 * m * LD::XB + ((4 * s + q) ^ r) * 16);
           __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
           for (int m = 0; m < MT; ++m)
@@ -348,21 +422,28 @@ __global__ __launch_bounds__((MsLds<WF, MT>::THREADS)) __attribute__((amdgpu_wav
         } else {
           // a lane's 16 weights of a 64-column step feed two products; the activations' columns are taken in the same order.  The step's
           // sums are multiplied by the scales of their weight rows: a weight enters exactly.
-          const float* sb = reinterpret_cast<const float*>(lds + slot_at + MS_W_BYTES + LD::X_BYTES) + wv * 64 + 4 * q;
+          const float* sb = reinterpret_cast<const float*>(lds + slot_at + w_bytes + LD::X_BYTES) + wv * 64 + 4 * q;
           u32x4 raw[4], x0[MT][4], x1[MT][4];
           f32x4 sv[4], step[4];
 #pragma unroll
           for (int t = 0; t < 4; ++t) {
             raw[t] = *reinterpret_cast<const u32x4*>(wb + ((4 * t + q) ^ r) * 16);
-            sv[t] = *reinterpret_cast<const f32x4*>(sb + t * 16);
+          }
+          if (p.rows16) {
+            const f32x4 alike = *reinterpret_cast<const f32x4*>(lds + slot_at + w_bytes + LD::X_BYTES + wv * 16);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) sv[t] = f32x4{alike[t], alike[t], alike[t], alike[t]};
+          } else {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) sv[t] = *reinterpret_cast<const f32x4*>(sb + t * 16);
           }
 #pragma unroll
           for (int m = 0; m < MT; ++m)
             if (m == 0 || 16 * m < full)
 #pragma unroll
               for (int t = 0; t < 4; ++t) {
-                x0[m][t] = *reinterpret_cast<const u32x4*>(xb + 16 * m * KU * 2 + ((8 * t + 2 * q) ^ r) * 16);
-                x1[m][t] = *reinterpret_cast<const u32x4*>(xb + 16 * m * KU * 2 + ((8 * t + 2 * q + 1) ^ r) * 16);
+                x0[m][t] = *reinterpret_cast<const u32x4*>(xb + 16 * m * LD::XB + ((8 * t + 2 * q) ^ r) * 16);
+                x1[m][t] = *reinterpret_cast<const u32x4*>(xb + 16 * m * LD::XB + ((8 * t + 2 * q + 1) ^ r) * 16);
               }
           __builtin_amdgcn_sched_barrier(0);
           u32x4 w0[4], w1[4];
@@ -387,7 +468,7 @@ __global__ __launch_bounds__((MsLds<WF, MT>::THREADS)) __attribute__((amdgpu_wav
         }
       }
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // B_u: this unit's slot may be refilled
-      slot_at = slot_at + LD::SLOT == LD::RING * LD::SLOT ? 0 : slot_at + LD::SLOT;
+      slot_at = slot_at + slot_bytes == ring * slot_bytes ? 0 : slot_at + slot_bytes;
     }
     if (mine) {
       if constexpr (WF == MS_FP8) {
@@ -443,7 +524,6 @@ __global__ __launch_bounds__((MsLds<WF, MT>::THREADS)) __attribute__((amdgpu_wav
     }
 #pragma unroll
     for (int m = 0; m < MT; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
-    rg += groups;
   }
 }
 
@@ -482,7 +562,7 @@ int ms_go(const MoeStreamParams& p, int grid, hipStream_t stream) {
     (void)hipFuncSetAttribute((const void*)moe_stream_kernel<DT, WF, MT, MODE>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     attr[dev] = true;
   }
-  moe_stream_kernel<DT, WF, MT, MODE><<<dim3((unsigned)grid * MsLds<WF, MT>::PER_CU), MsLds<WF, MT>::THREADS, bytes, stream>>>(p);
+  moe_stream_kernel<DT, WF, MT, MODE><<<dim3((unsigned)grid), MsLds<WF, MT>::THREADS, bytes, stream>>>(p);
   return LL_LAUNCH_CHECK();
 }
 
@@ -513,11 +593,19 @@ bool moe_stream_wants(const MoeStreamParams& p, int wfmt, int mode, int dtype, i
 int moe_stream_launch(const MoeStreamParams& asked, int wfmt, int mode, int dtype, int64_t experts, hipStream_t stream) {
   MoeStreamParams p = asked;
   p.group_n = p.group_n < p.N ? p.group_n : p.N;
+  p.rows16 = p.group_n % 16 == 0 || p.group_n >= p.N;
+  int lds = 0;
+  const int cus = ms_cus(&lds);
+  p.n_shift = -1;
+  for (int i = 0; i < 31; ++i)
+    if (p.group_n == (1ll << i)) p.n_shift = i;
+  p.per_workgroup = 1.0 / cus;
+  p.per_unit = 1.0 / ((p.K * (wfmt == MS_W16 ? 2 : 1) + MS_KB - 1) / MS_KB);
+  for (p.grid_log2 = 0; (2 << p.grid_log2) <= cus; ++p.grid_log2) {}
+  p.per_block = 1.0 / (mode == MS_GLU ? (p.N + 7) / 8 : (p.N + 15) / 16);
   p.k_shift = 31;
   if (wfmt != MS_W16 && p.group_k < p.K)
     for (p.k_shift = 6; (1ll << p.k_shift) < p.group_k; ++p.k_shift) {}
-  int lds = 0;
-  const int cus = ms_cus(&lds);
 #define MS_8(WF, MODE) return ms_rows(p, wfmt, experts) == 32 ? ms_go<LL_F16, WF, 2, MODE>(p, cus, stream) : ms_go<LL_F16, WF, 1, MODE>(p, cus, stream)
   if (wfmt == MS_FP8) {
     if (mode == MS_GLU_ROUNDED) MS_8(MS_FP8, MS_GLU_ROUNDED);

@@ -128,3 +128,22 @@ def test_fp16_experts(width, ff, experts, tokens, top, interleaved):
     # gate, up and their product are each rounded to fp16 (three half units, |silu'| <= 1.1), and so are a slot's result and the sum
     bound = 2.0 ** -11 * ((out.abs() + 6 * 3.3 * spread) * slot).sum(1)
     assert ((got.to(F64) - want).abs() <= bound + 2.0 ** -11 * want.abs() + 1e-6).all()
+
+
+@pytest.mark.parametrize("experts", [16, 17])          # runs within one expert / across them
+@pytest.mark.parametrize("groups", [3, 4, 5, 8, 9, 16, 17, 25])
+def test_runs_of_row_groups(experts, groups):
+    """A row per expert; a workgroup's run is ``groups`` row groups long: one more than the small units hold, than a tile, than two."""
+    from lite_llama_amd.kernels.fused_moe import sparse_square_experts
+
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    width, ff = 136, 16 * (cus * groups // experts)
+    g = torch.Generator(device=DEV).manual_seed(groups)
+    up, down = ((torch.randn(experts, *s, generator=g, device=DEV) * s[1] ** -0.5).bfloat16() for s in ((ff, width), (width, ff)))
+    h, ids = torch.randn(experts, width, generator=g, device=DEV).bfloat16(), torch.randperm(experts, generator=g, device=DEV).to(torch.int32)[:, None]
+    weights = torch.rand(experts, 1, generator=g, device=DEV) + 0.1
+    got = sparse_square_experts(h, up, down, ids, weights)[:, 0].double()
+    act = torch.stack([torch.relu(up[e].double() @ h[t].double() * weights[t].double()) ** 2 for t, e in enumerate(ids[:, 0].tolist())])
+    want = torch.stack([down[e].double() @ act[t] for t, e in enumerate(ids[:, 0].tolist())])
+    # the activations' rounding, met by weights of deviation ff^-1/2 (6 deviations), and the result's own
+    assert ((got - want).abs() <= 2.0 ** -8 * (want.abs() + 6 * act.norm(dim=1, keepdim=True) * ff ** -0.5)).all()
