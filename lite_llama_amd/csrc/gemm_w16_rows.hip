@@ -15,7 +15,12 @@
 //     8192 139 -> 124; staggered within an XCD instead, b / 8: 98, 106, 124.  K = 3584: 90 -> 91, 37888 rows of it 50 -> 52).  Sums of 16-bit products in
 //     another order round otherwise, so streams under 256 MB, which gain little or nothing (32 rows, K = 2048: 134 MB 31 -> 28 us, 46 MB
 //     13.9 -> 14.9), keep the ascending one; int8 sums are exact, and staggered from 64 MB.
-//   * one s_barrier per unit; the loaders' operation count per unit is static.
+//   * one s_barrier per unit.  Of every row group each loader requests a quarter, and nothing is requested that no one reads: neither groups that a
+//     tile lacks nor activations behind the last row; the waits count what was.  (Loaders of one group each, which pointed the requests of
+//     groups that were not there at one cached KB so that the count stayed the same, took as long for a tile of one group as for four.  us,
+//     then -> here: 32 rows 6144 x 2048 11.6 -> 9.8, 8192 x 2048 11.8 -> 10.0, 11264 x 2048 14.2 -> 12.7, 6 rows 9216 x 3072 18.2 -> 14.1, 64 rows
+//     8192 x 2048 14.1 -> 12.7; tiles that are full, as before: 17920 x 1536 13.9, 128256 x 4096 160 (6.6 TB/s).  A higher priority for the
+//     loaders' waves gains nothing here.)
 #include <stdlib.h>
 
 #include "common.h"
@@ -55,11 +60,14 @@ struct R16Params {
 };
 #define R16_I8 2  // DT code of the int8 x int8 form: x / w are int8 rows of 256 k per chunk, out is fp16
 
-template <int N>
-__device__ __forceinline__ void r16_wait_units(int k) {  // at most k units of N operations each may still be in flight
-  if (k <= 0) v3_vmcnt<0>();
-  else if (k == 1) v3_vmcnt<N>();
-  else v3_vmcnt<2 * N>();
+__device__ __forceinline__ void r16_wait(int k) {  // at most k operations may still be in flight
+#define R16_C(K) case K: v3_vmcnt<K>(); break;
+  switch (k) {
+    R16_C(1) R16_C(2) R16_C(3) R16_C(4) R16_C(5) R16_C(6) R16_C(7) R16_C(8) R16_C(9) R16_C(10) R16_C(11) R16_C(12) R16_C(13) R16_C(14) R16_C(15)
+    R16_C(16) R16_C(17) R16_C(18) R16_C(19) R16_C(20)
+    default: v3_vmcnt<0>(); break;
+  }
+#undef R16_C
 }
 
 template <int MT, int DT, bool WIDE>
@@ -68,9 +76,9 @@ __global__ __launch_bounds__((R16Lds<MT, WIDE>::THREADS)) __attribute__((amdgpu_
   using LD = R16Lds<MT, WIDE>;
   constexpr int R = LD::R, KB = LD::KB, GROUPS = LD::GROUPS;
   constexpr int PER = 1024 / KB, SLOTS = KB / 16;   // rows of an LDS-DMA operation; 16-byte slots of a row
-  constexpr int GL = GROUPS / 4;                    // row groups of a loader wave
-  constexpr int XP = LD::X_BYTES / 4096;  // activation operations per loader wave and unit
-  constexpr int OPS = 8 + XP;  // LDS-DMA operations per loader wave and unit
+  constexpr int PG = 8 / GROUPS;                    // weight operations per loader wave, unit and row group
+  constexpr int XP = LD::X_BYTES / 4096;  // activation operations per loader wave and unit, at most
+  static_assert((R - 2) * (8 + XP) <= 20, "the waits");
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int b = (int)blockIdx.x;
@@ -83,56 +91,66 @@ __global__ __launch_bounds__((R16Lds<MT, WIDE>::THREADS)) __attribute__((amdgpu_
 
   if (wv >= GROUPS) {
     // ======================================== loaders ======================================== //
-    const int L = wv - GROUPS;  // weight rows [L * 32 GL, + 32 GL) of every tile + activation operations XP * L ..
-    uint32_t woff[8], xoff[XP];
+    // Of every group each takes a quarter; nothing is requested that no one reads.
+    const int L = wv - GROUPS;
+    uint32_t woff[PG], xoff[XP];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int r = j * PER + lane / SLOTS, slot = (lane % SLOTS) ^ LD::swizzle(r & 31);
-      woff[j] = (uint32_t)((int64_t)r * p.w_stride * 2 + slot * 16);
+    for (int q = 0; q < PG; ++q) {
+      const int r = (4 * q + L) * PER + lane / SLOTS, slot = (lane % SLOTS) ^ LD::swizzle(r);
+      woff[q] = (uint32_t)((int64_t)r * p.w_stride * 2 + slot * 16);
     }
 #pragma unroll
     for (int j = 0; j < XP; ++j) {
-      int64_t r = (XP * L + j) * PER + lane / SLOTS;
+      int64_t r = (4 * j + L) * PER + lane / SLOTS;
       const int slot = (lane % SLOTS) ^ LD::swizzle((int)(r & 31));
       if (r >= p.m) r = p.m - 1;  // rows >= M feed only unstored outputs
       xoff[j] = (uint32_t)(r * p.x_stride * 2 + slot * 16);
     }
-    int issued = 0, t = 0, size = tbase + (trem > 0 ? 1 : 0), done = 0, c = 0;
+    int xops = ((int)p.m - L * PER + 4 * PER - 1) / (4 * PER);   // this wave's activation operations that hold a row
+    xops = xops < 0 ? 0 : xops;
+    int issued = 0, t = 0, size = tbase + (trem > 0 ? 1 : 0), done = 0, c = 0, ops = 0, before = 0;   // operations of the last unit and the one before it
     if (p.stagger) {   // (WIDE units are half as long: two of them per step, so that a row's sum begins at the same column in either form)
       for (c = b; c >= p.chunks * KB / 256; c -= p.chunks * KB / 256) {}
       c *= 256 / KB;
     }
-    const char* wt = (const char*)p.w + (size_t)(lo + L * GL) * 32 * (size_t)p.w_stride * 2;   // this wave's rows of the tile
+    const size_t group = 32 * (size_t)p.w_stride * 2;
+    const char* wt = (const char*)p.w + (size_t)lo * group;   // the tile's rows
     uint32_t dst = 0;
     auto issue = [&]() {
       const char* wb = wt + (size_t)c * KB;
       const char* xb = (const char*)p.x + (size_t)c * KB;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        // a short tile: an idle loader keeps its operations (the counted waits stay static) but points them at ONE cached KB (the first of
-        // the matrix) -- no weight bytes are fetched twice; its LDS block is never read
-        if (L * GL + j * GL / 8 < size) v3_dma16<true>(dst + L * 8192 + j * 1024, wb, woff[j]);
-        else v3_dma16<false>(dst + L * 8192 + j * 1024, (const char*)p.w, (uint32_t)(lane * 16));
+      for (int g = 0; g < GROUPS; ++g) {
+        if (g >= size) break;
+#pragma unroll
+        for (int q = 0; q < PG; ++q) v3_dma16<true>(dst + g * 32 * KB + (4 * q + L) * 1024, wb, woff[q]);
+        wb += group;
       }
 #pragma unroll
-      for (int j = 0; j < XP; ++j) v3_dma16<false>(dst + LD::W_BYTES + (XP * L + j) * 1024, xb, xoff[j]);
+      for (int j = 0; j < XP; ++j) {
+        if (j >= xops) break;
+        v3_dma16<false>(dst + LD::W_BYTES + (4 * j + L) * 1024, xb, xoff[j]);
+      }
       ++issued;
+      before = ops;
+      ops = size * PG + xops;
       if (++c == p.chunks) c = 0;
       if (++done == p.chunks) {
         done = 0;
-        wt += (size_t)size * 32 * (size_t)p.w_stride * 2;
+        wt += (size_t)size * group;
         size = tbase + (++t < trem ? 1 : 0);
       }
       dst = dst + LD::SLOT == R * LD::SLOT ? 0 : dst + LD::SLOT;
     };
+    auto wait = [&](int later) { r16_wait(later <= 0 ? 0 : later == 1 ? ops : ops + before); };   // but for the last `later` units (at most R - 2), all have landed
     const int pre = units < R - 1 ? units : R - 1;
     for (int i = 0; i < pre; ++i) issue();
-    r16_wait_units<OPS>(issued - 1);  // unit 0 has landed
+    wait(issued - 1);  // unit 0 has landed
     asm volatile("s_barrier" ::: "memory");  // P0
     for (int u = 0; u < units; ++u) {
       if (issued < units) issue();  // into the slot of unit u - 1, free since the barrier that ended it
       const int need = units < u + 2 ? units : u + 2;
-      r16_wait_units<OPS>(issued - need);  // unit u + 1 has landed before the consumers are released into it
+      wait(issued - need);  // unit u + 1 has landed before the consumers are released into it
       asm volatile("s_barrier" ::: "memory");  // B_u
     }
     return;
