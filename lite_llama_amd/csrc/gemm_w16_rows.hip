@@ -10,11 +10,14 @@
 //     address: fragment reads are conflict free; weights non-temporal.  CONSUMERS, one per row group of the tile, run the unit's MFMA
 //     32x32x16 from LDS fragments and keep the tile's accumulators (16 x MT registers) for the whole K loop: no cross-wave exchange.
 //     The loaders run ahead ACROSS tile boundaries, so a tile's epilogue overlaps the next tile's first units.
-//   * Long streams of rows a multiple of 4 KB long: workgroup b begins every tile b steps of 256 bytes into its rows and wraps.  All of them beginning at
-//     column 0 ask the same few memory channels (us for 600 MB, 1 row, all from column 0 -> staggered: K = 2048 113 -> 94, 4096 127 -> 98,
-//     8192 139 -> 124; staggered within an XCD instead, b / 8: 98, 106, 124.  K = 3584: 90 -> 91, 37888 rows of it 50 -> 52).  Sums of 16-bit products in
-//     another order round otherwise, so streams under 256 MB, which gain little or nothing (32 rows, K = 2048: 134 MB 31 -> 28 us, 46 MB
-//     13.9 -> 14.9), keep the ascending one; int8 sums are exact, and staggered from 64 MB.
+//   * Long streams of rows a multiple of 4 KB long: workgroup b begins every tile b steps of 256 bytes into its rows and wraps; streams under 256 MB
+//     5 b steps.  All of them beginning at column 0 ask the same few memory channels, and so do runs of a power of two rows whose steps of b keep
+//     pace with them.  us for 600 MB, 1 row, all from column 0 -> staggered: K = 2048 113 -> 94, 4096 127 -> 98, 8192 139 -> 124; staggered within
+//     an XCD instead, b / 8: 98, 106, 124; K = 3584: 90 -> 91, 37888 rows of it 50 -> 52.  32 rows, column 0 / b / 5 b: 16384 x 2048 16.3 / 14.6 / 14.6,
+//     32768 x 2048 32.7 / 29.5 / 25.6, 49152 x 2048 45 / 36 / 36, 14336 x 4096 25.6 / 30.9 / 24.5, 16384 x 4096 29.6 / 36.6 / 26.2, 28672 x 4096
+//     50 / 42 / 43, 8192 x 8192 37 / 32 / 28, int8 28672 x 4096 - / 23.8 / 23.1, 16384 x 8192 - / 36.3 / 25.7; 7 b: 28672 x 4096 47; 11 b: 16384 x
+//     4096 29.4; b's bits reversed: 32000 x 4096 57 (b 46).  From 256 MB on b and 5 b are within 2 % of each other, either way.  Sums of 16-bit products
+//     in another order round otherwise, so streams under 64 MB, which gain less (8192 x 2048 10.7 -> 9.9), keep the ascending one; int8 sums are exact.
 //   * one s_barrier per unit.  Of every row group each loader requests a quarter, and nothing is requested that no one reads: neither groups that a
 //     tile lacks nor activations behind the last row; the waits count what was.  (Loaders of one group each, which pointed the requests of
 //     groups that were not there at one cached KB so that the count stayed the same, took as long for a tile of one group as for four.  us,
@@ -53,7 +56,7 @@ struct R16Params {
   int64_t m, n, k, x_stride, w_stride;
   int chunks;        // units of a row: its bytes / R16Lds::KB
   int rbase, rrem;   // workgroup b owns row groups [b * rbase + min(b, rrem), + rbase + (b < rrem))
-  int stagger;       // workgroups begin a tile at different chunks
+  int stagger;       // workgroup b begins a tile that many times b steps of 256 bytes into its rows
   int epi;           // 0: out[m, n] (+ bias);  1: rows are (gate_j, up_j) pairs -> out[m, n / 2] = silu(gate) * up
   const float* a_scale;  // R16_I8 only: per-token activation scales [m], per-channel weight scales [n] (smoothquant, w8a8.py:118-149)
   const float* w_scale;
@@ -110,8 +113,7 @@ __global__ __launch_bounds__((R16Lds<MT, WIDE>::THREADS)) __attribute__((amdgpu_
     xops = xops < 0 ? 0 : xops;
     int issued = 0, t = 0, size = tbase + (trem > 0 ? 1 : 0), done = 0, c = 0, ops = 0, before = 0;   // operations of the last unit and the one before it
     if (p.stagger) {   // (WIDE units are half as long: two of them per step, so that a row's sum begins at the same column in either form)
-      for (c = b; c >= p.chunks * KB / 256; c -= p.chunks * KB / 256) {}
-      c *= 256 / KB;
+      c = b * p.stagger % (p.chunks * KB / 256) * (256 / KB);
     }
     const size_t group = 32 * (size_t)p.w_stride * 2;
     const char* wt = (const char*)p.w + (size_t)lo * group;   // the tile's rows
@@ -321,7 +323,7 @@ extern "C" int ll_dense16_rows_matmul(void* out, const void* x, const void* w, c
   R16Params p{};
   p.out = (uint16_t*)out; p.x = (const uint16_t*)x; p.w = (const uint16_t*)w; p.bias = (const uint16_t*)bias;
   p.m = m; p.n = n; p.k = k; p.x_stride = x_stride_m; p.w_stride = w_stride_n;
-  p.stagger = n * k * 2 >= (1ll << 28) && w_stride_n % 2048 == 0;
+  p.stagger = w_stride_n % 2048 || n * k * 2 < (1ll << 26) ? 0 : n * k * 2 < (1ll << 28) ? 5 : 1;
   p.epi = epilogue;
   const int64_t rgs = n / 32;
   int grid = r16_num_cus();
@@ -375,7 +377,7 @@ extern "C" int ll_w8a8_rows_matmul(void* out, const int8_t* qa, const float* a_s
   p.a_scale = a_scale; p.w_scale = w_scale;
   p.m = m; p.n = n; p.k = k;
   p.x_stride = qa_stride_m / 2; p.w_stride = qw_stride_n / 2;  // the kernel addresses rows in 2-byte units
-  p.stagger = n * k >= (1ll << 26) && qw_stride_n % 4096 == 0;
+  p.stagger = qw_stride_n % 4096 || n * k < (1ll << 26) ? 0 : n * k < (1ll << 28) ? 5 : 1;
   p.epi = epilogue;
   const int64_t rgs = n / 32;
   int grid = r16_num_cus();
