@@ -171,13 +171,38 @@ __global__ __launch_bounds__(64) void fa_prefill(
 // L2 traffic at batch 64 x 512).  Each wave keeps 16 * QB query columns: K fragments are read from LDS once per tile
 // and used for QB query blocks, V^T fragments come from transposing LDS reads (ds_read_b64_tr_b16), the online softmax
 // runs once per 64 keys (one rescale of O per tile, skipped when no running maximum moved).
-template <int DT, int D, int QB>
+// ROPE (the type of the rotary tables' entries; -1: none): q and k come as the projection left them and are rotated on the way in, rounded as
+// rope_cache_kernel rounds them; what that kernel writes to the cache is written by workgroups of their own beside these (blockIdx.z past
+// the sequences), for every token and whatever the sequences cover.  A launch less per layer of a short prefill, whose launches are
+// what it costs: 37 tokens of 14 + 2 heads of 64, 3.1 + 4.4 -> 5.6 us, 12 layers 571 -> 534.
+struct FaRope {
+  const uint16_t *cos_t, *sin_t;         // [batch][position][at least D / 2]
+  int64_t cbs, css, sbs, sss;
+  uint16_t* pool;                        // [token][k heads, then v heads][D]
+  int64_t pst, psh;
+  const void* sel;
+  int sel_w, seq_len, tokens;
+};
+template <int DT, int CS>
+__device__ __forceinline__ i32x4 fa_rotated(const i32x4& own, const i32x4& other, const i32x4& c, const i32x4& s, bool low) {
+  const U16x8 x = __builtin_bit_cast(U16x8, own), y = __builtin_bit_cast(U16x8, other), cv = __builtin_bit_cast(U16x8, c), sv = __builtin_bit_cast(U16x8, s);
+  U16x8 o;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float a = to_f32<DT>(x.v[e]), b = to_f32<DT>(y.v[e]), cs = to_f32<CS>(cv.v[e]), sn = to_f32<CS>(sv.v[e]);
+    o.v[e] = from_f32<DT>(low ? a * cs - b * sn : a * cs + b * sn);
+  }
+  return __builtin_bit_cast(i32x4, o);
+}
+
+template <int DT, int D, int QB, int ROPE = -1>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void fa_prefill2(
     uint16_t* __restrict__ out, const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
     const uint16_t* __restrict__ v, const void* __restrict__ b_start_loc, const void* __restrict__ b_seq_len,
     int hq, int hkv, float sm_scale, int64_t q_st, int64_t q_sh, int64_t k_st, int64_t k_sh, int64_t v_st,
-    int64_t v_sh, int64_t o_st, int64_t o_sh, int start_w, int seq_w) {
+    int64_t v_sh, int64_t o_st, int64_t o_sh, int start_w, int seq_w, const FaRope rp) {
   constexpr int NS = D / 32, NT = D / 16, STR = D + 8, TK = 64;
+  constexpr int CS = ROPE < 0 ? LL_F16 : ROPE;
   constexpr int TPR = D / 8, RPP = 256 / TPR, PASSES = TK / RPP;  // 16-byte pieces per row, rows per pass
   __shared__ __attribute__((aligned(16))) uint16_t lds_k[TK * STR];
   __shared__ __attribute__((aligned(16))) uint16_t lds_v[TK * STR];
@@ -186,6 +211,35 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
   const int t = lane & 15, c = lane >> 4;
   const int head = blockIdx.y, b = blockIdx.z;
   const int kvh = head / (hq / hkv);
+  auto tables = [&](int tok, int64_t& cb, int64_t& sb) {   // where a token's row of the rotary tables begins
+    const int bi = (int)((uint32_t)tok / (uint32_t)rp.seq_len), si = tok - bi * rp.seq_len;
+    cb = bi * rp.cbs + si * rp.css;
+    sb = bi * rp.sbs + si * rp.sss;
+  };
+  auto at = [](const uint16_t* p) { return *reinterpret_cast<const i32x4*>(p); };
+  if constexpr (ROPE >= 0) {
+    if (b == (int)gridDim.z - 1) {   // the cache's rows, pieces of eight entries
+      constexpr int PIECES = D / 8;
+      const int items = rp.tokens * 2 * hkv * PIECES;
+      for (int i = (int)(blockIdx.y * gridDim.x + blockIdx.x) * 256 + tid; i < items; i += (int)(gridDim.x * gridDim.y) * 256) {
+        const int piece = i % PIECES, h = i / PIECES % (2 * hkv), tok = i / (PIECES * 2 * hkv), col = piece * 8;
+        const int64_t dst = rp.sel_w == LL_I32 ? (int64_t)((const int32_t*)rp.sel)[tok] : ((const int64_t*)rp.sel)[tok];
+        i32x4 x;
+        if (h >= hkv) {
+          x = at(v + tok * v_st + (h - hkv) * v_sh + col);
+        } else {
+          int64_t cb, sb;
+          tables(tok, cb, sb);
+          const bool low = col < D / 2;
+          const int j = low ? col : col - D / 2;
+          const uint16_t* row = k + tok * k_st + h * k_sh;
+          x = fa_rotated<DT, CS>(at(row + col), at(row + (low ? col + D / 2 : j)), at(rp.cos_t + cb + j), at(rp.sin_t + sb + j), low);
+        }
+        *reinterpret_cast<i32x4*>(rp.pool + dst * rp.pst + h * rp.psh + col) = x;
+      }
+      return;
+    }
+  }
   const int64_t seq_len = pa_load_idx(b_seq_len, b, seq_w);
   const int64_t start = pa_load_idx(b_start_loc, b, start_w);
   const int64_t q0 = (int64_t)(gridDim.x - 1 - blockIdx.x) * (64 * QB);  // the longest key ranges are dispatched first
@@ -200,6 +254,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
 #pragma unroll
     for (int s = 0; s < NS; ++s)
       qf[qb][s] = *reinterpret_cast<const Q4*>(q + (start + qrow) * q_st + (int64_t)head * q_sh + s * 32 + c * 8);
+    if constexpr (ROPE >= 0) {
+      int64_t cb, sb;
+      tables((int)(start + qrow), cb, sb);
+#pragma unroll
+      for (int s = 0; s < NS / 2; ++s) {
+        const i32x4 cv = at(rp.cos_t + cb + s * 32 + c * 8), sv = at(rp.sin_t + sb + s * 32 + c * 8);
+        const i32x4 x = __builtin_bit_cast(i32x4, qf[qb][s]), y = __builtin_bit_cast(i32x4, qf[qb][s + NS / 2]);
+        qf[qb][s] = __builtin_bit_cast(Q4, fa_rotated<DT, CS>(x, y, cv, sv, true));
+        qf[qb][s + NS / 2] = __builtin_bit_cast(Q4, fa_rotated<DT, CS>(y, x, cv, sv, false));
+      }
+    }
   }
   float m_i[QB], d_i[QB];
   f32x4 ot[QB][NT];
@@ -213,6 +278,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
 
   const int64_t kend = q0 + 64 * QB < seq_len ? q0 + 64 * QB : seq_len;  // causal: the workgroup needs keys < kend
   const int lrow = tid / TPR, lcol = (tid % TPR) * 8;
+  constexpr int ROT = ROPE < 0 ? 1 : PASSES;
+  [[maybe_unused]] const bool low = lcol < D / 2;
+  [[maybe_unused]] const int lj = low ? lcol : lcol - D / 2;
+  [[maybe_unused]] i32x4 ko[ROT], kc[ROT], ks[ROT];   // the other half's entries, the tables' entries
   i32x4 kr[PASSES], vr[PASSES];  // (vector type, not the Q4 struct: the struct copy into LDS kept the array in scratch)
   auto fetch = [&](int64_t p0) {
 #pragma unroll
@@ -221,12 +290,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
       if (key >= seq_len) key = seq_len - 1;
       kr[ps] = *reinterpret_cast<const i32x4*>(k + (start + key) * k_st + (int64_t)kvh * k_sh + lcol);
       vr[ps] = *reinterpret_cast<const i32x4*>(v + (start + key) * v_st + (int64_t)kvh * v_sh + lcol);
+      if constexpr (ROPE >= 0) {
+        int64_t cb, sb;
+        tables((int)(start + key), cb, sb);
+        ko[ps] = at(k + (start + key) * k_st + (int64_t)kvh * k_sh + (low ? lcol + D / 2 : lj));
+        kc[ps] = at(rp.cos_t + cb + lj);
+        ks[ps] = at(rp.sin_t + sb + lj);
+      }
     }
   };
   auto stage = [&](int64_t p0) {
 #pragma unroll
     for (int ps = 0; ps < PASSES; ++ps) {
       const int row = ps * RPP + lrow;
+      if constexpr (ROPE >= 0) kr[ps] = fa_rotated<DT, CS>(kr[ps], ko[ps], kc[ps], ks[ps], low);
       *reinterpret_cast<i32x4*>(&lds_k[row * STR + lcol]) = kr[ps];
       // rows past the sequence end are multiplied by p = 0: they must not hold NaN / Inf bit patterns
       *reinterpret_cast<i32x4*>(&lds_v[row * STR + lcol]) = p0 + row < seq_len ? vr[ps] : i32x4{0, 0, 0, 0};
@@ -356,7 +433,7 @@ static int launch_fa(void* out, const void* q, const void* k, const void* v, con
 #define LL_FA2(DD, QQ)                                                                                          \
   fa_prefill2<DT, DD, QQ><<<grid2, 256, 0, st>>>((uint16_t*)out, (const uint16_t*)q, (const uint16_t*)k,        \
                                                  (const uint16_t*)v, start, seq, hq, hkv, sm_scale, q_st, q_sh, \
-                                                 k_st, k_sh, v_st, v_sh, o_st, o_sh, start_w, seq_w)
+                                                 k_st, k_sh, v_st, v_sh, o_st, o_sh, start_w, seq_w, FaRope{})
     if (d == 64) {
       if (qb == 2) LL_FA2(64, 2); else LL_FA2(64, 1);
     } else {
@@ -403,4 +480,37 @@ extern "C" int ll_flash_attention_nopad(void* out, const void* q, const void* k,
   return launch_fa<LL_BF16>(out, q, k, v, b_start_loc, b_seq_len, batch, hq, hkv, d, max_seq_len, sm_scale,
                             q_stride_t, q_stride_h, k_stride_t, k_stride_h, v_stride_t, v_stride_h, o_stride_t,
                             o_stride_h, start_width, seq_width, st);
+}
+
+// The rotation and the cache's rows (ll_rope_kv_update, whose arguments these are) and the attention over them (ll_flash_attention_nopad) of tokens
+// packed as rows [q | k | v], in one launch.  1: done; 0: not its shape (heads of 64 or 128, 16-bit tables, everything in whole 16 bytes), nothing
+// was launched; below 0: an error.  The rows stay as they are.
+int fa_rope_launch(void* out, const void* qkv, int64_t row, const void* cos_t, const void* sin_t, int64_t cos_b_stride, int64_t cos_s_stride,
+                   int64_t sin_b_stride, int64_t sin_s_stride, void* pool, int64_t pool_stride_t, int64_t pool_stride_h, const void* select_index,
+                   int select_width, const void* starts, int start_width, const void* lens, int len_width, int64_t prompts, int64_t max_len,
+                   int64_t tokens, int64_t seq_len, int heads, int kv_heads, int d, float sm_scale, int dtype, int cs_dtype, hipStream_t st) {
+  if ((d != 64 && d != 128) || (cs_dtype != LL_F16 && cs_dtype != LL_BF16) || (dtype != LL_F16 && dtype != LL_BF16) || heads % kv_heads || max_len < 1 ||
+      prompts >= 65535 || tokens >= (1 << 20) || seq_len < 1 || seq_len >= (1 << 30) || ((select_width | start_width | len_width) & ~1) ||
+      (row | pool_stride_t | pool_stride_h | cos_b_stride | cos_s_stride | sin_b_stride | sin_s_stride) % 8 || !ll_aligned16(qkv) || !ll_aligned16(out) ||
+      !ll_aligned16(pool) || !ll_aligned16(cos_t) || !ll_aligned16(sin_t))
+    return 0;
+  const FaRope rp{(const uint16_t*)cos_t, (const uint16_t*)sin_t, cos_b_stride, cos_s_stride, sin_b_stride, sin_s_stride, (uint16_t*)pool, pool_stride_t,
+                  pool_stride_h, select_index, select_width, (int)seq_len, (int)tokens};
+  const int qb = max_len > 64 && d == 64 ? 2 : 1;   // (128 query entries and the tables' beside them do not fit the registers twice)
+  const uint16_t *q = (const uint16_t*)qkv, *k = q + (int64_t)heads * d, *v = k + (int64_t)kv_heads * d;
+  const dim3 grid((unsigned)((max_len + 64 * qb - 1) / (64 * qb)), (unsigned)heads, (unsigned)prompts + 1);
+#define LL_FAR(DT, DD, QQ, CS)                                                                                                               \
+  fa_prefill2<DT, DD, QQ, CS><<<grid, 256, 0, st>>>((uint16_t*)out, q, k, v, starts, lens, heads, kv_heads, sm_scale, row, d, row, d, row, d, \
+                                                    (int64_t)heads * d, d, start_width, len_width, rp)
+#define LL_FAR_Q(DT, DD, CS) do { if (qb == 2) LL_FAR(DT, DD, 2, CS); else LL_FAR(DT, DD, 1, CS); } while (0)
+#define LL_FAR_D(DT, CS) do { if (d == 64) LL_FAR_Q(DT, 64, CS); else LL_FAR(DT, 128, 1, CS); } while (0)
+#define LL_FAR_C(DT) do { if (cs_dtype == LL_F16) LL_FAR_D(DT, LL_F16); else LL_FAR_D(DT, LL_BF16); } while (0)
+  if (dtype == LL_F16) LL_FAR_C(LL_F16);
+  else LL_FAR_C(LL_BF16);
+#undef LL_FAR_C
+#undef LL_FAR_D
+#undef LL_FAR_Q
+#undef LL_FAR
+  const int rc = LL_LAUNCH_CHECK();
+  return rc == LL_OK ? 1 : rc;
 }

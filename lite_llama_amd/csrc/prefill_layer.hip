@@ -1,14 +1,19 @@
 // A decoder layer of an unquantised llama-shaped model over the tokens of a short prefill (at most 192), issued by ONE host call.
 //
-// Bound by the host: the eight launches of such a layer take 35 - 60 us, and each of them cost 16 - 24 us of interpreter time to prepare (a prompt of
+// Bound by the host: the launches of such a layer (seven; eight where the rotation has one of its own) take 28 - 60 us, and each of them cost 16 - 24 us of interpreter time to prepare (a prompt of
 // 37 tokens through 12 layers of 896: 2290 us, of which the GPU worked 670).  The launches are the eager route's own, in its order and with
-// its arithmetic: norm, q|k|v, rotation + cache scatter, attention, o as split-K partials that the next norm adds up, gate|up with the
+// its arithmetic: norm, q|k|v, rotation + cache scatter + attention, o as split-K partials that the next norm adds up, gate|up with the
 // activation in its epilogue, down as partials.  (The eager route asks the library for q|k|v and o; here they stay on the narrow kernel or
 // the row-group loop and on the split-K engine: 5 - 9 us each against 8, without 24 us of the library's host side.)
 // These engines take 64 rows: more go through them in parts of equal size, whose weights the Infinity Cache
-// holds between them, if the layer's are no more than 100 MB.  us, eager -> here: 12 layers of 896 / 4864, 37 tokens 2290 -> 790, 100 2850 -> 1090, 200
+// holds between them, if the layer's are no more than 100 MB.  us, eager -> here: 12 layers of 896 / 4864, 37 tokens 2290 -> 790 (534 since: fewer checks, the rotation in the attention's launch), 100 2850 -> 1090, 200
 // (four parts) 2790 -> 1530; 4 layers of 1536 / 8960 (94 MB each), 64 tokens 850 -> 374, 100 1020 -> 616, 180 1034 -> 858, 256 1025 -> 1096.
 #include "common.h"
+
+int fa_rope_launch(void* out, const void* qkv, int64_t row, const void* cos_t, const void* sin_t, int64_t cos_b_stride, int64_t cos_s_stride,
+                   int64_t sin_b_stride, int64_t sin_s_stride, void* pool, int64_t pool_stride_t, int64_t pool_stride_h, const void* select_index,
+                   int select_width, const void* starts, int start_width, const void* lens, int len_width, int64_t prompts, int64_t max_len,
+                   int64_t tokens, int64_t seq_len, int heads, int kv_heads, int d, float sm_scale, int dtype, int cs_dtype, hipStream_t st);
 
 extern "C" int ll_prefill_layer16(void* residual, void* x, int planes_in, float* planes, void* qkv, void* attn, void* act, const void* norm1,
                                   const void* norm2, float eps, const void* w_qkv, const void* b_qkv, const void* w_o, const void* w_gate_up,
@@ -59,10 +64,16 @@ extern "C" int ll_prefill_layer16(void* residual, void* x, int planes_in, float*
       LL_TRY(ll_dense16_narrow_matmul(rows(qkv, at, row), rows(x, at, hidden), w_qkv, b_qkv, m, row, hidden, hidden, hidden, dtype, stream));
     else LL_TRY(ll_dense16_rows_matmul(rows(qkv, at, row), rows(x, at, hidden), w_qkv, b_qkv, m, row, hidden, hidden, hidden, dtype, 0, stream));
   }
-  LL_TRY(ll_rope_kv_update(qkv, k, cos_t, sin_t, pool, select_index, tokens, heads, kv_heads, head_dim, row, row, seq_len, cos_b_stride,
-                           cos_s_stride, sin_b_stride, sin_s_stride, pool_stride_t, pool_stride_h, dtype, cs_dtype, select_width, nullptr, stream));
-  LL_TRY(ll_flash_attention_nopad(attn, qkv, k, v, starts, lens, (int)prompts, heads, kv_heads, head_dim, max_len, sm_scale, row, head_dim, row,
-                                  head_dim, row, head_dim, q_size, head_dim, dtype, start_width, len_width, stream));
+  r = fa_rope_launch(attn, qkv, row, cos_t, sin_t, cos_b_stride, cos_s_stride, sin_b_stride, sin_s_stride, pool, pool_stride_t, pool_stride_h, select_index,
+                     select_width, starts, start_width, lens, len_width, prompts, max_len, tokens, seq_len, heads, kv_heads, head_dim, sm_scale, dtype,
+                     cs_dtype, (hipStream_t)stream);
+  if (r < 0) return r;
+  if (r == 0) {
+    LL_TRY(ll_rope_kv_update(qkv, k, cos_t, sin_t, pool, select_index, tokens, heads, kv_heads, head_dim, row, row, seq_len, cos_b_stride,
+                             cos_s_stride, sin_b_stride, sin_s_stride, pool_stride_t, pool_stride_h, dtype, cs_dtype, select_width, nullptr, stream));
+    LL_TRY(ll_flash_attention_nopad(attn, qkv, k, v, starts, lens, (int)prompts, heads, kv_heads, head_dim, max_len, sm_scale, row, head_dim, row,
+                                    head_dim, row, head_dim, q_size, head_dim, dtype, start_width, len_width, stream));
+  }
   for (int64_t i = 0, at = 0; i < parts; ++i, at += part) {
     const int64_t m = i + 1 < parts ? part : last;
     r = ll_dense_partials(sums(i), rows(attn, at, q_size), w_o, nullptr, m, hidden, q_size, 1, q_size, wfmt, q_size, q_size, 0, 0, max_splits, stream);

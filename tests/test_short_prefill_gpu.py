@@ -91,3 +91,18 @@ def test_what_keeps_the_layers_own_forward(monkeypatch):
     assert _prefill(odd, dtype, [20], True, monkeypatch)[2] == 0
     normed = _model(dtype, use_qk_norm=True)
     assert _prefill(normed, dtype, [20], True, monkeypatch)[2] == 0
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("lens", [[1, 2], [37], [65], [31, 17, 40], [70, 90], [192]])
+@pytest.mark.parametrize("heads,kv_heads,dim", [(4, 2, 64), (2, 1, 128), (6, 2, 64), (8, 4, 32)])
+def test_rotation_and_attention_in_one_launch(dtype, lens, heads, kv_heads, dim, monkeypatch):
+    """Heads of 64 and 128 (heads of 32 keep two launches): a tile of queries and more, prompts of one length and of several, whose places
+    behind a prompt's end are written to the cache as well."""
+    model = _model(dtype, layers=2, hidden_size=256, num_heads=heads, num_kv_heads=kv_heads, head_dim=dim)
+    want, rows, none = _prefill(model, dtype, lens, False, monkeypatch)
+    got, mine, calls = _prefill(model, dtype, lens, True, monkeypatch)
+    assert none == 0 and calls == 2
+    _near(got, want, dtype, 2)
+    for a, b in zip(mine, rows):
+        _near(a, b, dtype, 2)
