@@ -742,8 +742,7 @@ int ll_gated_group_norm(const float* x_in, float* x_out, void* h_out, const void
                         const float* shared_scale, const void* gate, int64_t gate_ld, const void* gate_bias,
                         const void* post_w, const void* next_w, int64_t n, int64_t width, int64_t groups, float eps,
                         const void* y_bias, int dtype, void* stream);
-/* ... with y the fp32 planes [parts][n][width] that a split-K projection left, added up and rounded to dtype (16-bit weights, rows and
- * groups in pieces of four channels). */
+/* ... with y the fp32 planes [parts][n][width] that a split-K projection left (16-bit weights, rows and groups in pieces of four channels). */
 int ll_gated_group_norm_sums(const float* x_in, float* x_out, void* h_out, const float* y, int64_t parts, const void* shared,
                              const float* shared_scale, const void* gate, int64_t gate_ld, const void* gate_bias, const void* post_w,
                              const void* next_w, int64_t n, int64_t width, int64_t groups, float eps, const void* y_bias, int dtype,

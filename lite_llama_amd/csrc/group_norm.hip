@@ -201,8 +201,7 @@ __device__ __forceinline__ void st4(void* p, int64_t i, f32x4 v) {
 
 // Vector form of the register-cached kernel: a thread owns pieces of four consecutive channels (16-byte residual accesses,
 // 8-byte accesses of 16-bit rows).  Needs group sizes that are multiples of 4 and at most 1024 NV channels, aligned rows.
-// SUMS: y holds `parts` fp32 planes [parts][n][width], what a split-K projection left; their sum enters rounded to 16 bits, as the
-// projection's own rows do: a step's results do not depend on which of the two comes.  (A launch that only adds planes
+// SUMS: y holds `parts` fp32 planes [parts][n][width], what a split-K projection left; their sum enters as it is.  (A launch that only adds planes
 // up, 4.8 us, is gone, and the projections whose planes were not worth that launch -- 2048 x 2048, 32 rows: 9.0 us in whole sums -- take 4.4.)
 template <int DT, int NV, bool SUMS = false>
 __global__ __launch_bounds__(256) void gated_group_norm_vec_kernel(
@@ -238,10 +237,6 @@ __global__ __launch_bounds__(256) void gated_group_norm_vec_kernel(
 #pragma unroll
           for (int p = 0; p < 4; ++p)
             if (p0 + p < parts) s += v[p];
-        }
-        if constexpr (SUMS) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) s[e] = to_f32<DT>(from_f32<DT>(s[e]));
         }
         if (y_bias) s += ld4<DT>(y_bias, i);
         if (shared) s += sscale * ld4<DT>(shared, t * (int64_t)width + i);

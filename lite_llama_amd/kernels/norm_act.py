@@ -589,8 +589,7 @@ class GatedUpdate:
 
     def __init__(self, y, post_weight, gate=None, gate_bias=None, shared=None, shared_scale=None, bias=None):
         """``bias [width]``: added to the summed rows (the bias of the projection that produced them).  ``y`` may be the
-        :class:`PartialSums` of a projection: its fp32 planes ``[parts, n, width]`` enter as the
-        rows that finishing it would leave: added up, then rounded to the storage type."""
+        :class:`PartialSums` of a projection: its fp32 planes ``[parts, n, width]`` enter the norm's sum as they are."""
         self.y = y if isinstance(y, PartialSums) or y.dim() == 3 else y.unsqueeze(1)
         self.post_weight, self.gate, self.gate_bias, self.shared, self.shared_scale = post_weight, gate, gate_bias, shared, shared_scale
         self.bias = bias

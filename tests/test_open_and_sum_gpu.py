@@ -35,13 +35,10 @@ def test_norm_over_planes(dtype, n, width, groups, planes):
         one = x[n - 1:].to(DEV)
         gated_group_norm(one, pick, None, 1e-6, groups)
         h = gated_group_norm(got_x, update, nw.to(DEV), 1e-6, groups)
-        # the planes' sum rounded to the storage type, half a unit of each (it moves the mean square by less than that), met by the gate (< 1)
-        # and the shared rows beside it: at most two units of the largest normed value; fp32 sums of at most 4096 squares and a hardware
-        # sigmoid: 1e-5; then one rounding to the storage type
-        unit = 2.0 ** (-11 if dtype == torch.float16 else -8)
-        assert (got_x.double().cpu() - want_x).abs().max() <= 2e-5 * want_x.abs().max() + 2 * unit * (want_x - x.double()).abs().max()
+        # fp32 sums of at most 4096 squares and a hardware sigmoid: 1e-5; then one rounding to the storage type
+        assert (got_x.double().cpu() - want_x).abs().max() <= 2e-5 * want_x.abs().max()
         assert torch.equal(one[0], got_x[n - 1])
-        assert (h.double().cpu() - want_h).abs().max() <= 3 * unit * want_h.abs().max()
+        assert (h.double().cpu() - want_h).abs().max() <= (6e-4 if dtype == torch.float16 else 5e-3) * want_h.abs().max()
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
@@ -56,17 +53,3 @@ def test_embedding_rows(dtype, index, n, width):
     x, first = embed_rows(ids, table)
     assert x[n - 1].isnan().all() and first.rows[n - 1].isnan().all()
     assert embed_rows(ids, table.t().contiguous().t()) is None and embed_rows(ids.cpu(), table) is None
-
-
-@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-def test_planes_and_their_finished_rows_give_the_same_bits(dtype):
-    g = torch.Generator(device=DEV).manual_seed(5)
-    y, x = torch.randn(6, 9, 2048, generator=g, device=DEV), torch.randn(9, 2048, generator=g, device=DEV)
-    pw, nw = ((1 + 0.1 * torch.randn(2048, generator=g, device=DEV)).to(dtype) for _ in range(2))
-    own = y[0].clone()
-    for p in range(1, 6):
-        own += y[p]
-    got_x, want_x = x.clone(), x.clone()
-    got = gated_group_norm(got_x, GatedUpdate(PartialSums(y, (9, 2048), dtype), pw), nw, 1e-6, 1)
-    want = gated_group_norm(want_x, GatedUpdate(own.to(dtype)[:, None], pw), nw, 1e-6, 1)
-    assert torch.equal(got, want) and torch.equal(got_x, want_x)
