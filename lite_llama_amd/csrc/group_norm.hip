@@ -201,9 +201,7 @@ __device__ __forceinline__ void st4(void* p, int64_t i, f32x4 v) {
 
 // Vector form of the register-cached kernel: a thread owns pieces of four consecutive channels (16-byte residual accesses,
 // 8-byte accesses of 16-bit rows).  Needs group sizes that are multiples of 4 and at most 1024 NV channels, aligned rows.
-// SUMS: y holds `parts` fp32 planes [parts][n][width], what a split-K projection left; their sum enters as it is.  (A launch that only adds planes
-// up, 4.8 us, is gone, and the projections whose planes were not worth that launch -- 2048 x 2048, 32 rows: 9.0 us in whole sums -- take 4.4.)
-template <int DT, int NV, bool SUMS = false>
+template <int DT, int NV>
 __global__ __launch_bounds__(256) void gated_group_norm_vec_kernel(
     const float* x_in, float* x_out, void* __restrict__ h_out, const void* __restrict__ y, int parts,
     const void* __restrict__ shared, const float* __restrict__ shared_scale, const void* __restrict__ gate, int64_t gate_ld,
@@ -226,18 +224,7 @@ __global__ __launch_bounds__(256) void gated_group_norm_vec_kernel(
       const int i = lo + 4 * (tid + 256 * k);
       f32x4 s = {0.f, 0.f, 0.f, 0.f};
       if (i < hi) {
-        for (int p0 = 0; p0 < parts; p0 += 4) {   // (four rows requested together)
-          f32x4 v[4];
-#pragma unroll
-          for (int p = 0; p < 4; ++p) {
-            const int64_t at = p0 + p < parts ? p0 + p : p0;
-            if constexpr (SUMS) v[p] = ld4<LL_F32>(y, (at * gridDim.x + t) * width + i);
-            else v[p] = ld4<DT>(y, (t * parts + at) * (int64_t)width + i);
-          }
-#pragma unroll
-          for (int p = 0; p < 4; ++p)
-            if (p0 + p < parts) s += v[p];
-        }
+        for (int p = 0; p < parts; ++p) s += ld4<DT>(y, (t * parts + p) * (int64_t)width + i);
         if (y_bias) s += ld4<DT>(y_bias, i);
         if (shared) s += sscale * ld4<DT>(shared, t * (int64_t)width + i);
         if (gate) {
@@ -409,34 +396,6 @@ extern "C" int ll_gated_group_norm(const float* x_in, float* x_out, void* h_out,
   LL_BY_DTYPE(dtype, CALL);
 #undef CALL
 #undef LL_GN_ARGS
-  return LL_LAUNCH_CHECK();
-}
-
-// ll_gated_group_norm over the planes [parts][n][width] (fp32) of a split-K projection: 16-bit weights, groups of 4 .. 4096 channels in whole
-// pieces of four, 16-byte aligned rows.
-extern "C" int ll_gated_group_norm_sums(const float* x_in, float* x_out, void* h_out, const float* y, int64_t parts, const void* shared,
-                                        const float* shared_scale, const void* gate, int64_t gate_ld, const void* gate_bias, const void* post_w,
-                                        const void* next_w, int64_t n, int64_t width, int64_t groups, float eps, const void* y_bias, int dtype,
-                                        void* stream) {
-  if (dtype != LL_F16 && dtype != LL_BF16) return LL_ERR_DTYPE;
-  if (n < 0 || width < 1 || width > (1 << 20) || groups < 1 || width % groups || parts < 1 || parts > 64) return LL_ERR_SHAPE;
-  if (n == 0) return LL_OK;
-  if (!x_in || !x_out || !y || !post_w || (shared && !shared_scale)) return LL_ERR_ARG;
-  const int64_t gs = width / groups;
-  if (gs % 4 || gs > 4096 || (gate && (gate_ld < width || gate_ld % 4))) return LL_ERR_SHAPE;
-  if (!ll_aligned16(x_in) || !ll_aligned16(x_out) || !ll_aligned16(y)) return LL_ERR_ARG;
-  for (const void* p : {(const void*)h_out, shared, gate, gate_bias, post_w, next_w, y_bias})
-    if ((uintptr_t)p & 7) return LL_ERR_ARG;
-  const dim3 grid((unsigned)n);
-  hipStream_t st = (hipStream_t)stream;
-#define CALL(DT, NV)                                                                                                                        \
-  gated_group_norm_vec_kernel<DT, NV, true><<<grid, 256, 0, st>>>(x_in, x_out, h_out, y, (int)parts, shared, shared_scale, gate, gate_ld,    \
-                                                                  gate_bias, post_w, next_w, (int)width, (int)groups, eps, y_bias)
-#define BY_SIZE(DT) \
-  if (gs <= 1024) CALL(DT, 1); else if (gs <= 2048) CALL(DT, 2); else CALL(DT, 4)
-  if (dtype == LL_F16) { BY_SIZE(LL_F16); } else { BY_SIZE(LL_BF16); }
-#undef BY_SIZE
-#undef CALL
   return LL_LAUNCH_CHECK();
 }
 

@@ -553,30 +553,6 @@ def residual_set(y: torch.Tensor, bias: torch.Tensor | None = None, out: torch.T
     return out
 
 
-class FirstRows:
-    """The rows that open a stack, in the storage dtype: what a sublayer that reads the residual stream itself reads first."""
-
-    __slots__ = ("rows",)
-
-    def __init__(self, rows: torch.Tensor):
-        self.rows = rows
-
-
-@torch.no_grad()
-def embed_rows(ids: torch.Tensor, table: torch.Tensor):
-    """``(x, FirstRows)``: embedding rows as the fp32 residual and as they are, in one launch -- ``residual_set(F.embedding(ids, table))`` and
-    the cast of it back.  ``None`` where the call is not served."""
-    if (ids.dtype not in (torch.int32, torch.int64) or ids.dim() != 1 or not ids.is_contiguous() or not ids.is_cuda or table.device != ids.device
-            or table.dtype not in (torch.float16, torch.bfloat16) or not table.is_contiguous() or not L.has("ll_embed_rows")):
-        return None
-    n, width = ids.numel(), table.shape[1]
-    x = torch.empty(n, width, dtype=torch.float32, device=ids.device)
-    h = torch.empty(n, width, dtype=table.dtype, device=ids.device)
-    L.check(L.lib().ll_embed_rows(x.data_ptr(), h.data_ptr(), table.data_ptr(), ids.data_ptr(), L.index_width(ids), n, width, table.shape[0],
-                                  L.dtype_code(table.dtype), L.stream_ptr()), "embed_rows")
-    return x, FirstRows(h)
-
-
 # ------------------------------------------------------------------------------------- #
 # sublayers between two grouped norms, with a gate on the residual branch (csrc/group_norm.hip)
 # ------------------------------------------------------------------------------------- #
@@ -588,18 +564,15 @@ class GatedUpdate:
     __slots__ = ("y", "shared", "shared_scale", "gate", "gate_bias", "post_weight", "bias")
 
     def __init__(self, y, post_weight, gate=None, gate_bias=None, shared=None, shared_scale=None, bias=None):
-        """``bias [width]``: added to the summed rows (the bias of the projection that produced them).  ``y`` may be the
-        :class:`PartialSums` of a projection: its fp32 planes ``[parts, n, width]`` enter the norm's sum as they are."""
-        self.y = y if isinstance(y, PartialSums) or y.dim() == 3 else y.unsqueeze(1)
+        """``bias [width]``: added to the summed rows (the bias of the projection that produced them)."""
+        self.y = y if y.dim() == 3 else y.unsqueeze(1)
         self.post_weight, self.gate, self.gate_bias, self.shared, self.shared_scale = post_weight, gate, gate_bias, shared, shared_scale
         self.bias = bias
 
     def rows(self, index: torch.Tensor) -> "GatedUpdate":
         """The update of the listed tokens only."""
         pick = lambda t: None if t is None else t[index].contiguous()  # noqa: E731
-        y = self.y
-        y = PartialSums(y.parts[:, index].contiguous(), (index.numel(), y.shape[-1]), y.dtype) if isinstance(y, PartialSums) else pick(y)
-        return GatedUpdate(y, self.post_weight, pick(self.gate), self.gate_bias, pick(self.shared), pick(self.shared_scale),
+        return GatedUpdate(pick(self.y), self.post_weight, pick(self.gate), self.gate_bias, pick(self.shared), pick(self.shared_scale),
                            self.bias)
 
 
@@ -621,12 +594,8 @@ def gated_group_norm(x: torch.Tensor, update: "GatedUpdate | None", next_weight,
     if next_weight is not None and (next_weight.numel() != width or not next_weight.is_contiguous()):
         raise ValueError("gated_group_norm: the norm weight has one entry per channel")
     args, y_bias = (0, 0, 0, 0, 0, 0, 0, 0), None
-    sums = u is not None and isinstance(u.y, PartialSums)
     if u is not None:
-        if sums:
-            if u.y.dtype != dt or tuple(u.y.parts.shape[1:]) != (n, width) or not u.y.parts.is_contiguous() or u.post_weight.dtype != dt:
-                raise ValueError("gated_group_norm: the update's planes are [parts, n, width] of a projection in the weights' dtype")
-        elif u.y.dtype != dt or u.y.shape[0] != n or u.y.shape[2] != width or not u.y.is_contiguous() or u.post_weight.dtype != dt:
+        if u.y.dtype != dt or u.y.shape[0] != n or u.y.shape[2] != width or not u.y.is_contiguous() or u.post_weight.dtype != dt:
             raise ValueError("gated_group_norm: the update is [n, parts, width] in the weights' dtype")
         gate_ld = 0
         if u.gate is not None:
@@ -639,13 +608,12 @@ def gated_group_norm(x: torch.Tensor, update: "GatedUpdate | None", next_weight,
         y_bias = u.bias
         if y_bias is not None and (y_bias.dtype != dt or y_bias.numel() != width or not y_bias.is_contiguous()):
             raise ValueError("gated_group_norm: the update's bias has one entry per channel, in the weights' dtype")
-        args = (*((u.y.parts.data_ptr(), u.y.parts.shape[0]) if sums else (u.y.data_ptr(), u.y.shape[1])), L.ptr(u.shared), L.ptr(u.shared_scale), L.ptr(u.gate), gate_ld, L.ptr(u.gate_bias),
+        args = (u.y.data_ptr(), u.y.shape[1], L.ptr(u.shared), L.ptr(u.shared_scale), L.ptr(u.gate), gate_ld, L.ptr(u.gate_bias),
                 u.post_weight.data_ptr())
     elif h is None:
         return None
-    run = L.lib().ll_gated_group_norm_sums if sums else L.lib().ll_gated_group_norm
-    L.check(run(x.data_ptr(), x.data_ptr(), L.ptr(h), *args, L.ptr(next_weight), n, width, int(groups),
-                float(eps), L.ptr(y_bias), L.dtype_code(dt), L.stream_ptr()), "gated_group_norm")
+    L.check(L.lib().ll_gated_group_norm(x.data_ptr(), x.data_ptr(), L.ptr(h), *args, L.ptr(next_weight), n, width, int(groups),
+                                        float(eps), L.ptr(y_bias), L.dtype_code(dt), L.stream_ptr()), "gated_group_norm")
     return h
 
 

@@ -65,21 +65,17 @@ from dataclasses import dataclass, field
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
-from torch.nn.modules import module as _nn
 
-from . import _lib as L
 from .distributed.parallel_state import get_tp_world_size
 from .kernels.activations import xielu
 from .kernels.attention import (conv_rope_cache, latent_kv_prep, qk_norm_cache, ragged_attention, rotate_pairs, rotation_table,
                                 rownorm_rope_cache)
 from .kernels.fused_moe import group_router, sparse_glu_experts, sparse_square_experts
-from .kernels.norm_act import (FirstRows, GatedUpdate, StreamUpdate, SummedUpdate, add_rmsnorm_shift, cast_pair, embed_pair, embed_rows,
-                               gated_group_norm, glu_act, relu_square, residual_set, softcap_, stream_norm)
+from .kernels.norm_act import (GatedUpdate, StreamUpdate, SummedUpdate, add_rmsnorm_shift, cast_pair, embed_pair, gated_group_norm,
+                               glu_act, relu_square, residual_set, softcap_, stream_norm)
 from .kernels.recurrent import (conv_act, delta_scan, gated_linear_scan, gated_out_norm, linear_scan, mingru_scan, retention,
                                 rglru_scan)
 from .linear import ReplicatedLinear
-from .prefill_layers import _plain
-from .quantization.methods import UnquantizedLinearMethod
 
 
 # ------------------------------------------------------------------------------------- #
@@ -588,19 +584,6 @@ def _linear(inp: int, out: int) -> ReplicatedLinear:
     return ReplicatedLinear(inp, out)
 
 
-def _for_the_norm(linear: ReplicatedLinear, x: torch.Tensor):
-    """``linear(x)`` for a norm launch that adds split-K sums up itself (:class:`GatedUpdate`): for up to 64 rows the sums of the projection, where
-    nothing but that launch would see its output -- or the output."""
-    w = linear.weight
-    if (0 < x.shape[0] <= 64 and x.is_cuda and w.device == x.device and w.shape[0] % 4 == 0 and w.shape[0] <= 4096 and linear.bias is None
-            and _plain(linear, ReplicatedLinear) and type(linear.quant_method) is UnquantizedLinearMethod and not _nn._global_forward_hooks
-            and not _nn._global_forward_pre_hooks and L.has("ll_dense_partials") and L.has("ll_gated_group_norm_sums")):
-        sums = linear.quant_method.apply_partials(linear, x)
-        if sums is not None:
-            return sums
-    return linear(x)
-
-
 def _padded_linear(inp: int, out: int, used_rows: int, bias_rows: int = 0) -> ReplicatedLinear:
     """A projection fused from members that start on 16-byte borders: ``out`` rows of which the members fill ``used_rows``, the rest
     are zeros that no checkpoint tensor fills.  ``bias_rows``: how many rows belong to members with a bias (0: there is none)."""
@@ -984,8 +967,6 @@ class WindowAttentionSSD(nn.Module):
     State-space branch: ``u B C`` through a causal convolution and silu, then per head ``S <- exp(-exp(A_log) dt) S + dt B u^T``,
     ``y = S^T C + D u`` (B, C shared by the heads of a group), ``y silu(z)`` RMS-normed in equal parts."""
 
-    leaves_sums = False   # what reads the result adds split-K sums up itself
-
     def __init__(self, width: int, spec: MixerSpec, eps: float):
         super().__init__()
         self.spec, self.eps = spec, eps
@@ -1030,14 +1011,12 @@ class WindowAttentionSSD(nn.Module):
                         skip=self.skip)
         gated_out_norm(o, self.ssd_norm_weight, self.eps, parts=r.norm_groups, gate=rows[:, self.z_off:self.conv_off],
                        gate_kind="silu", gate_first=True, scale=s.branch_scales[1], out=mixed[:, self.heads_width:])
-        return _for_the_norm(self.out_proj, mixed) if self.leaves_sums else self.out_proj(mixed)
+        return self.out_proj(mixed)
 
 
 class DecayLinearAttention(nn.Module):
     """``q | k | v | g`` in one projection; per head ``S <- decay_h S + silu(k) silu(v)^T``, ``o = S^T silu(q)`` over the fp32
     state slots; the heads side by side RMS-normed together, times ``sigmoid(g)``; output projection."""
-
-    leaves_sums = False   # what reads the result adds split-K sums up itself
 
     def __init__(self, width: int, spec: MixerSpec, eps: float):
         super().__init__()
@@ -1058,8 +1037,7 @@ class DecayLinearAttention(nn.Module):
             self._decay = torch.tensor(s.decay, dtype=torch.float64).to(torch.float32).to(h.device)
         o = linear_scan(rows[:, :qk], rows[:, qk:2 * qk], rows[:, 2 * qk:2 * qk + v], s.heads, s.dim, s.vdim, step,
                         cache.recurrent[run], act=True, head_decay=self._decay)
-        o = gated_out_norm(o, self.out_norm_weight, self.eps, gate=rows[:, 2 * qk + v:], gate_kind="sigmoid")
-        return _for_the_norm(self.o_proj, o) if self.leaves_sums else self.o_proj(o)
+        return self.o_proj(gated_out_norm(o, self.out_norm_weight, self.eps, gate=rows[:, 2 * qk + v:], gate_kind="sigmoid"))
 
 
 class Retention(nn.Module):
@@ -1101,8 +1079,6 @@ class GatedLinearAttention(nn.Module):
     ``S <- diag(alpha) S + k v^T``, ``o = S^T q / sqrt(dim)`` with ``alpha = sigmoid(W_a2 a + b)^(1 / tau)`` per key entry;
     every head RMS-normed with one shared weight, times ``silu(g)``; output projection."""
 
-    leaves_sums = False   # what reads the result adds split-K sums up itself
-
     def __init__(self, width: int, spec: MixerSpec, eps: float):
         super().__init__()
         self.spec, self.eps = spec, eps
@@ -1124,15 +1100,13 @@ class GatedLinearAttention(nn.Module):
         logits = self.decay_proj(low if low.shape[0] <= 64 and rows.shape[1] % 8 == 0 else low.contiguous())
         o = linear_scan(rows[:, :qk], rows[:, qk:2 * qk], rows[:, 2 * qk:2 * qk + v], s.heads, s.dim, s.vdim, step,
                         cache.recurrent[run], q_scale=s.dim ** -0.5, gate=logits, gate_bias=self.decay_bias, tau=s.tau)
-        o = gated_out_norm(o, self.out_norm_weight, self.eps, parts=s.heads, gate=rows[:, 2 * qk + v:2 * qk + 2 * v], gate_kind="silu")
-        return _for_the_norm(self.o_proj, o) if self.leaves_sums else self.o_proj(o)
+        return self.o_proj(gated_out_norm(o, self.out_norm_weight, self.eps, parts=s.heads, gate=rows[:, 2 * qk + v:2 * qk + 2 * v],
+                                          gate_kind="silu"))
 
 
 class BiasedGatedMLP(nn.Module):
     """``down(silu(gate h + b_g) * (up h + b_u)) + b_d``; ``gate | up`` are one projection.  The down projection's bias is
     not added here: it rides with the result into the norm launch that follows."""
-
-    leaves_sums = False   # what reads the result adds split-K sums up itself
 
     def __init__(self, width: int, ff: int):
         super().__init__()
@@ -1142,8 +1116,7 @@ class BiasedGatedMLP(nn.Module):
         self.down_bias = _vector(width)
 
     def forward(self, h):
-        act = glu_act(self.in_proj(h), self.ff, "silu")
-        return (_for_the_norm(self.down_proj, act) if self.leaves_sums else self.down_proj(act)), self.down_bias, None, None
+        return self.down_proj(glu_act(self.in_proj(h), self.ff, "silu")), self.down_bias, None, None
 
 
 class CorrectedSoftmaxMoE(nn.Module):
@@ -1433,14 +1406,11 @@ class PostNormLayer(nn.Module):
         if spec.mlp is not None:
             self.norm2_weight = _vector(w)
             self.mlp = CorrectedSoftmaxMoE(w, spec.mlp) if spec.mlp.kind == "moe" else BiasedGatedMLP(w, spec.mlp.ff)
-        self.mixer.leaves_sums = True
-        if isinstance(self.mlp, BiasedGatedMLP):
-            self.mlp.leaves_sums = True
 
     def forward(self, x, pending, step, cache, run: int, token_table):
         """``(x, pending)``: the fp32 residual (updated in place) and the update still to enter it.  Returns the same pair."""
         dt = self.norm1_weight.dtype
-        h = pending.rows if isinstance(pending, FirstRows) else gated_group_norm(x, pending, None, self.eps, plain=dt)
+        h = gated_group_norm(x, pending, None, self.eps, plain=dt)
         pending = GatedUpdate(self.mixer(h, step, cache, run, token_table), self.norm1_weight)
         if self.mlp is not None:
             h = gated_group_norm(x, pending, None, self.eps, plain=dt)
@@ -1537,12 +1507,6 @@ class LayeredLM(nn.Module):
             runs.append(run)
         return runs
 
-    def _reads_stream(self) -> bool:
-        """Whether the first layer reads the embedded rows as they are, and nothing else looks at what it is handed."""
-        return (self.geo.post_norm and not (self.geo.looped and self.geo.loop_mix) and len(self.run_order) > 0
-                and _plain(self.layers[self.run_order[0][0]], PostNormLayer) and not _nn._global_forward_hooks
-                and not _nn._global_forward_pre_hooks and self.embed_tokens.weight.dtype == self.norm_weight.dtype)
-
     @torch.no_grad()
     def forward(self, token_ids, step, cache, token_table, logits_rows=None, collect_layers: list | None = None):
         """``token_ids [n]`` int64 of the step's flat token array.  ``logits_rows``: int64 indices into it, ``"all"`` for every row in order
@@ -1551,12 +1515,10 @@ class LayeredLM(nn.Module):
         if self.geo.pair_buckets or self.geo.embed_scale != 1.0:
             x0 = embed_pair(token_ids, self.embed_tokens.weight, self.geo.embed_scale, self.pair_table if self.geo.pair_buckets else None,
                             self.geo.pair_mul_prev, self.geo.pair_mul_cur, step, cache.prev_token)
-            opened = None
         else:
-            opened = embed_rows(token_ids, self.embed_tokens.weight) if self._reads_stream() else None
-            x0, opened = opened if opened is not None else (residual_set(F.embedding(token_ids, self.embed_tokens.weight)), None)
+            x0 = residual_set(F.embedding(token_ids, self.embed_tokens.weight))
         loop_mix = self.geo.looped and self.geo.loop_mix
-        x, delta = (x0.clone() if loop_mix else x0), opened  # (layers update the residual in place; x0 is read again)
+        x, delta = (x0.clone() if loop_mix else x0), None  # (layers update the residual in place; x0 is read again)
         for run, (index, pass_no, first) in enumerate(self.run_order):
             if first and loop_mix:
                 y = self.loop_in(cast_pair(x, x0, self.dtype, a_delta=delta))
