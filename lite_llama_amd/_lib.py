@@ -144,6 +144,7 @@ SIGNATURES = {
     "ll_ragged_attention_partition": [],
     "ll_ragged_attention_mfma": [P, P, P, P, L, P, P, P, P, F, P, L, L, L, L, I, P, L, L, L, L, L, L, L, L, L, F, P, L, P, L, I, P],
     "ll_gated_group_norm": [P, P, P, P, L, P, P, P, L, P, P, P, L, L, L, F, P, I, P],
+    "ll_embed_rows": [P, P, P, P, I, L, L, L, I, P],
     "ll_glu_act": [P, L, P, L, P, L, L, L, I, F, F, I, P],
     "ll_softcap": [P, L, F, I, P],
     "ll_mingru_scan_scratch_floats": [L, L, L],

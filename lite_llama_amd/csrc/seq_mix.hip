@@ -344,6 +344,37 @@ __global__ __launch_bounds__(256) void residual_set_kernel(float* __restrict__ x
   }
 }
 
+// A workgroup per token: its embedding row as it is and as the fp32 residual (a row that the table does not have: NaN).  VEC: 8-value pieces.
+template <int DT, bool VEC>
+__global__ __launch_bounds__(256) void embed_rows_kernel(float* __restrict__ x, uint16_t* __restrict__ h, const uint16_t* __restrict__ table,
+                                                         const void* __restrict__ ids, int id_w, int64_t vocab, int width) {
+  const int64_t t = blockIdx.x, id = id_w == LL_I32 ? (int64_t)((const int32_t*)ids)[t] : ((const int64_t*)ids)[t];
+  const bool known = id >= 0 && id < vocab;
+  const uint16_t* from = table + (known ? id : 0) * width;
+  if constexpr (VEC) {
+    for (int i = threadIdx.x * 8; i < width; i += 2048) {
+      U16x8 v = *reinterpret_cast<const U16x8*>(from + i);
+      f32x4 lo, hi;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v.v[e] = known ? v.v[e] : (uint16_t)0x7fff;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        lo[e] = to_f32<DT>(v.v[e]);
+        hi[e] = to_f32<DT>(v.v[4 + e]);
+      }
+      *reinterpret_cast<U16x8*>(h + t * width + i) = v;
+      *reinterpret_cast<f32x4*>(x + t * width + i) = lo;
+      *reinterpret_cast<f32x4*>(x + t * width + i + 4) = hi;
+    }
+  } else {
+    for (int i = threadIdx.x; i < width; i += 256) {
+      const uint16_t v = known ? from[i] : (uint16_t)0x7fff;
+      h[t * width + i] = v;
+      x[t * width + i] = to_f32<DT>(v);
+    }
+  }
+}
+
 // One workgroup per token: x = embed[token] * scale + pair[row], row = (previous token * mul_prev + token * mul_cur) mod buckets,
 // or row `buckets` (the table's last) for a sequence's first token.  The previous token of a run's first token comes from the
 // sequence's state slot (half seq_parity is read); a run's last token leaves itself in the other half.  pair == NULL: no table.
@@ -888,6 +919,23 @@ extern "C" int ll_residual_set(float* x, const void* y, const void* bias, int64_
   if (!x || !y) return LL_ERR_ARG;
 #define CALL(DT) residual_set_kernel<DT><<<dim3(flat_grid(n * width)), 256, 0, (hipStream_t)stream>>>(x, y, bias, n, (int)width)
   LL_BY_DTYPE(dtype, CALL);
+#undef CALL
+  return LL_LAUNCH_CHECK();
+}
+
+extern "C" int ll_embed_rows(float* x, void* h, const void* table, const void* ids, int id_width, int64_t n, int64_t width, int64_t vocab,
+                             int dtype, void* stream) {
+  if (dtype != LL_F16 && dtype != LL_BF16) return LL_ERR_DTYPE;
+  if (id_width != LL_I32 && id_width != LL_I64) return LL_ERR_DTYPE;
+  if (n < 0 || width < 1 || width > (1 << 20) || vocab < 1) return LL_ERR_SHAPE;
+  if (n == 0) return LL_OK;
+  if (!x || !h || !table || !ids) return LL_ERR_ARG;
+  hipStream_t st = (hipStream_t)stream;
+  const bool vec = width % 8 == 0 && ll_aligned16(x) && ll_aligned16(h) && ll_aligned16(table);
+#define CALL(DT, VEC) \
+  embed_rows_kernel<DT, VEC><<<dim3((unsigned)n), 256, 0, st>>>(x, (uint16_t*)h, (const uint16_t*)table, ids, id_width, vocab, (int)width)
+  if (dtype == LL_F16) { if (vec) CALL(LL_F16, true); else CALL(LL_F16, false); }
+  else { if (vec) CALL(LL_BF16, true); else CALL(LL_BF16, false); }
 #undef CALL
   return LL_LAUNCH_CHECK();
 }

@@ -553,6 +553,30 @@ def residual_set(y: torch.Tensor, bias: torch.Tensor | None = None, out: torch.T
     return out
 
 
+class FirstRows:
+    """The rows that open a stack, in the storage dtype: what a sublayer that reads the residual stream itself reads first."""
+
+    __slots__ = ("rows",)
+
+    def __init__(self, rows: torch.Tensor):
+        self.rows = rows
+
+
+@torch.no_grad()
+def embed_rows(ids: torch.Tensor, table: torch.Tensor):
+    """``(x, FirstRows)``: embedding rows as the fp32 residual and as they are, in one launch -- ``residual_set(F.embedding(ids, table))`` and
+    the cast of it back.  ``None`` where the call is not served."""
+    if (ids.dtype not in (torch.int32, torch.int64) or ids.dim() != 1 or not ids.is_contiguous() or not ids.is_cuda or table.device != ids.device
+            or table.dtype not in (torch.float16, torch.bfloat16) or not table.is_contiguous() or not L.has("ll_embed_rows")):
+        return None
+    n, width = ids.numel(), table.shape[1]
+    x = torch.empty(n, width, dtype=torch.float32, device=ids.device)
+    h = torch.empty(n, width, dtype=table.dtype, device=ids.device)
+    L.check(L.lib().ll_embed_rows(x.data_ptr(), h.data_ptr(), table.data_ptr(), ids.data_ptr(), L.index_width(ids), n, width, table.shape[0],
+                                  L.dtype_code(table.dtype), L.stream_ptr()), "embed_rows")
+    return x, FirstRows(h)
+
+
 # ------------------------------------------------------------------------------------- #
 # sublayers between two grouped norms, with a gate on the residual branch (csrc/group_norm.hip)
 # ------------------------------------------------------------------------------------- #

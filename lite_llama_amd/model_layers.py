@@ -65,17 +65,19 @@ from dataclasses import dataclass, field
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.nn.modules import module as _nn
 
 from .distributed.parallel_state import get_tp_world_size
 from .kernels.activations import xielu
 from .kernels.attention import (conv_rope_cache, latent_kv_prep, qk_norm_cache, ragged_attention, rotate_pairs, rotation_table,
                                 rownorm_rope_cache)
 from .kernels.fused_moe import group_router, sparse_glu_experts, sparse_square_experts
-from .kernels.norm_act import (GatedUpdate, StreamUpdate, SummedUpdate, add_rmsnorm_shift, cast_pair, embed_pair, gated_group_norm,
-                               glu_act, relu_square, residual_set, softcap_, stream_norm)
+from .kernels.norm_act import (FirstRows, GatedUpdate, StreamUpdate, SummedUpdate, add_rmsnorm_shift, cast_pair, embed_pair, embed_rows,
+                               gated_group_norm, glu_act, relu_square, residual_set, softcap_, stream_norm)
 from .kernels.recurrent import (conv_act, delta_scan, gated_linear_scan, gated_out_norm, linear_scan, mingru_scan, retention,
                                 rglru_scan)
 from .linear import ReplicatedLinear
+from .prefill_layers import _plain
 
 
 # ------------------------------------------------------------------------------------- #
@@ -1410,7 +1412,7 @@ class PostNormLayer(nn.Module):
     def forward(self, x, pending, step, cache, run: int, token_table):
         """``(x, pending)``: the fp32 residual (updated in place) and the update still to enter it.  Returns the same pair."""
         dt = self.norm1_weight.dtype
-        h = gated_group_norm(x, pending, None, self.eps, plain=dt)
+        h = pending.rows if isinstance(pending, FirstRows) else gated_group_norm(x, pending, None, self.eps, plain=dt)
         pending = GatedUpdate(self.mixer(h, step, cache, run, token_table), self.norm1_weight)
         if self.mlp is not None:
             h = gated_group_norm(x, pending, None, self.eps, plain=dt)
@@ -1507,6 +1509,12 @@ class LayeredLM(nn.Module):
             runs.append(run)
         return runs
 
+    def _reads_stream(self) -> bool:
+        """Whether the first layer reads the embedded rows as they are, and nothing else looks at what it is handed."""
+        return (self.geo.post_norm and not (self.geo.looped and self.geo.loop_mix) and len(self.run_order) > 0
+                and _plain(self.layers[self.run_order[0][0]], PostNormLayer) and not _nn._global_forward_hooks
+                and not _nn._global_forward_pre_hooks and self.embed_tokens.weight.dtype == self.norm_weight.dtype)
+
     @torch.no_grad()
     def forward(self, token_ids, step, cache, token_table, logits_rows=None, collect_layers: list | None = None):
         """``token_ids [n]`` int64 of the step's flat token array.  ``logits_rows``: int64 indices into it, ``"all"`` for every row in order
@@ -1515,10 +1523,12 @@ class LayeredLM(nn.Module):
         if self.geo.pair_buckets or self.geo.embed_scale != 1.0:
             x0 = embed_pair(token_ids, self.embed_tokens.weight, self.geo.embed_scale, self.pair_table if self.geo.pair_buckets else None,
                             self.geo.pair_mul_prev, self.geo.pair_mul_cur, step, cache.prev_token)
+            opened = None
         else:
-            x0 = residual_set(F.embedding(token_ids, self.embed_tokens.weight))
+            opened = embed_rows(token_ids, self.embed_tokens.weight) if self._reads_stream() else None
+            x0, opened = opened if opened is not None else (residual_set(F.embedding(token_ids, self.embed_tokens.weight)), None)
         loop_mix = self.geo.looped and self.geo.loop_mix
-        x, delta = (x0.clone() if loop_mix else x0), None  # (layers update the residual in place; x0 is read again)
+        x, delta = (x0.clone() if loop_mix else x0), opened  # (layers update the residual in place; x0 is read again)
         for run, (index, pass_no, first) in enumerate(self.run_order):
             if first and loop_mix:
                 y = self.loop_in(cast_pair(x, x0, self.dtype, a_delta=delta))
