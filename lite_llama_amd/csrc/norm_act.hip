@@ -128,7 +128,7 @@ __global__ __launch_bounds__(256) void skip_rmsnorm_cached(uint16_t* __restrict_
     if (ok[v]) {
       U16x8 yv;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) yv.v[i] = mul_storage<DT>(from_f32<DT>(s[v][i] * rrms), wv[v].v[i]);
+      for (int i = 0; i < 8; ++i) yv.v[i] = mul_storage<DT>(from_f32<DT>(ll_pinned(s[v][i] * rrms)), wv[v].v[i]);   // (the same values, gathered or not)
       *reinterpret_cast<U16x8*>(y + row * n + (v * TPR + tr) * 8) = yv;
     }
   }

@@ -36,6 +36,20 @@ def test_first_norm_reads_the_table(dtype, rows, n):
     assert not EmbeddedRows.served(ids.int(), table) and not EmbeddedRows.served(ids, table[:, 1:]) and not EmbeddedRows.served(ids, table.t())
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n", [896, 1536, 2048, 2056, 3584, 4096, 4104, 5120, 8192])
+def test_a_wide_first_norm_rounds_as_the_norm_of_rows_does(dtype, n):
+    """Rows in one, two and four pieces of 2048 columns, values enough that a product rounded once instead of twice shows (about one in 2^13 does)."""
+    g = torch.Generator(device=DEV).manual_seed(n)
+    table = torch.randn(500, n, generator=g, device=DEV).to(dtype)
+    weight = (1 + 0.1 * torch.randn(n, generator=g, device=DEV)).to(dtype)
+    ids = torch.randperm(500, generator=g, device=DEV)[:200].view(200, 1)
+    y, r = embed_rmsnorm(EmbeddedRows(ids, table), weight, 1e-6)
+    x = F.embedding(ids, table)
+    want, _ = skip_rmsnorm(x, None, weight, 1e-6)
+    assert torch.equal(r, x) and torch.equal(y, want)
+
+
 def test_copies_of_a_steps_inputs():
     src = [torch.randint(0, 1 << 20, (n,), device=DEV, dtype=dt) for n, dt in ((1, torch.int64), (64, torch.int64), (300, torch.int32), (7, torch.int32))]
     dst = [torch.full((s.numel() + 1,), -5, device=DEV, dtype=s.dtype) for s in src]
