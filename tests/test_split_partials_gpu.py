@@ -62,3 +62,39 @@ def test_plane_count_does_not_depend_on_the_rows(fmt, n, k):
         counts = {L.lib().ll_dense_partials_count(m, n, k, fmt, cap) for m in (1, 31, 32, 33, 64)}
         assert len(counts) == 1 and max(counts) <= cap
     assert L.lib().ll_dense_partials_count(65, n, k, fmt, 12) == 0
+
+
+@pytest.mark.parametrize("fmt", [FP8, I8])
+def test_contractions_of_whole_64_columns_leave_planes(fmt):
+    for n, k in ((2048, 4160), (1024, 2112), (4096, 1088)):
+        assert 1 <= L.lib().ll_dense_partials_count(33, n, k, fmt, 12) <= 12
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", [FP8, I8])
+@pytest.mark.parametrize("m,n,k", [(64, 2048, 4160), (7, 2048, 4160), (33, 1024, 2112), (33, 2048, 4096), (64, 5120, 2048), (9, 4096, 2432), (32, 96, 640)])
+@pytest.mark.parametrize("group_n", [1, 32, 128])
+@pytest.mark.parametrize("group_k", [64, 128, 192, 0])
+def test_scales_of_a_block_meet_its_columns_alone(fmt, m, n, k, group_n, group_k):
+    """Blocks of half a unit of the contraction, of one, of one and a half and of all of it (0); the last block of 192 columns is a partial one."""
+    gk = group_k or k
+    g = torch.Generator(device=DEV).manual_seed(n + k + group_n + gk)
+    x = torch.randn(m, k, generator=g, device=DEV).half()
+    if fmt == FP8:
+        w = torch.randn(n, k, generator=g, device=DEV).to(torch.float8_e4m3fn)
+        wide, w = w.double(), w.view(torch.uint8)
+    else:
+        w = torch.randint(-127, 128, (n, k), generator=g, device=DEV, dtype=torch.int8)
+        wide = w.double()
+    blocks = (-(-n // group_n), -(-k // gk))
+    scales = 2.0 ** torch.randint(-6, 5, blocks, generator=g, device=DEV).float()   # (powers of two: a widened weight is exact in fp16)
+    wide *= scales.double().repeat_interleave(group_n, 0)[:n].repeat_interleave(gk, 1)[:, :k]
+    count = L.lib().ll_dense_partials_count(m, n, k, fmt, 12)
+    assert 1 <= count <= 12
+    planes = torch.full((count, m, n), float("nan"), device=DEV)
+    got = L.lib().ll_dense_partials(planes.data_ptr(), x.data_ptr(), w.data_ptr(), scales.data_ptr(), m, n, k, group_n, gk, fmt, k, k, scales.stride(0),
+                                    scales.stride(1), 12, L.stream_ptr())
+    assert got == count
+    # fp32 sums of k exact products, in whatever order
+    bound = k * 2.0 ** -24 * (x.double().abs() @ wide.abs().T) + 1e-30
+    assert ((planes.double().sum(0) - x.double() @ wide.T).abs() <= bound).all()
