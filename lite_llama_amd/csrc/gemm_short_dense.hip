@@ -1,4 +1,4 @@
-// SHORT-STREAM decode GEMM for the ROW-MAJOR weight formats (round 6): split-K partial launches of a few tens of KB per CU over
+// SHORT-STREAM decode GEMM for the ROW-MAJOR weight formats: split-K partial launches of a few tens of KB per CU over
 // fp8-e4m3 / int8 weights with block scales (a9, lite_llama/kernels/quantization/w8a16.py:155-216) and unquantised fp16 / bf16
 // weights (the reference's F.linear, methods/unquantized.py:21-22) -- the dense q|k|v / o projections of Qwen3-30B-A3B (fp8, 10.5 /
 // 8.4 MB), the narrow projections of a 1.5B bf16 model, every projection of a TP >= 4 shard.  Same shape as gemm_short.hip (the
@@ -9,7 +9,7 @@
 // stages); a piece is widened (the decode engines' exact bit surgery, gemm_w8_common.h, block scale folded in) and multiplied as it
 // lands; the k-interleaves of a row group meet through LDS in wave order and leave as whole 128-byte lines of the fp32 plane
 // [slice][m][n] -- the planes ll_dense_partials documents, for ll_skip_rmsnorm_partials / ll_decode_attention_partials.
-// The launches this plan declines (long streams, shapes off its grid) stay on gemm_w8_skinny.hip.
+// The launches this plan declines (long streams, shapes off its grid) stay on gemm_split.hip and gemm_w8_skinny.hip.
 #include <stdlib.h>
 
 #include "common.h"
@@ -303,7 +303,7 @@ static SDPlan sd_plan(int64_t m, int64_t n, int64_t k, int wfmt, int max_splits)
   }
   // a launch that would leave more than a third of the CUs idle stays on the streaming engine
   if (best.ok && best.total * 3 < cus * 2) best.ok = 0;
-  // Measured (benchmarks/gemm_short_dense.py, same box, us per launch short-stream / streaming engine; DESIGN_NOTEBOOK.md 8.7):
+  // Measured (benchmarks/gemm_short_dense.py, same box, us per launch short-stream / streaming engine):
   // fp8 2048 x 4096 7.4 / 11.2, int8 4096 x 1024 5.4 / 6.6 -- but fp8 5120 x 2048 (10.5 MB) 10.6 / 10.1 under every plan, and
   // the 16-bit formats 7.2 - 8.1 / 6.0 - 6.5: a lane's 32 - 64 contiguous bytes per row make every load instruction touch 32+ cache
   // lines (the int4 engine's pre-packed pieces are 1 KB contiguous).  Default: 8-bit weights of at most 9 MB; LL_DENSE_SS=2 lifts it.

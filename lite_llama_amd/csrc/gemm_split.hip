@@ -6,14 +6,14 @@
 //   * Four LOADER waves bring units of 128 bytes of every weight row (whole lines, non-temporal) and the same columns of the activations into a
 //     ring of LDS slots by LDS-DMA, up to 11 units ahead: most shares are on their way at once.  16-byte slot s of a row stands at
 //     s ^ ((row >> 1) & 7) (activations in 256-byte rows: s ^ (row & 15)), through the SOURCE address: fragment reads are conflict free.
-//   * One CONSUMER wave per row group runs the unit's MFMAs 32x32x16 (int8 x int8 32x32x32) from LDS fragments; 8-bit weights under fp16
-//     activations, whose widening is most of the work, have two, which share a unit's columns.
+//   * One CONSUMER wave per row group runs the unit's MFMAs 32x32x16 (int8 x int8 32x32x32) from LDS fragments.
 //   * The sums pass through the idle ring and leave as whole lines.
-// Bound by the ramp of a launch (about 3 us), then by what a CU can take in, about 27 KB/us.  A kernel that parks one 16 KB chunk per workgroup in
-// registers took (us, calls that follow each other over 0.7 GB of weights, before -> here): 1536 x 8960 bf16, 27 rows 14.5 -> 7.9; 1536 x 1536 4.9 ->
-// 3.7; 896 x 4864 fp16, 37 rows 10.5 -> 5.8; int8 x int8, 30 rows 4096 x 14336 18.4 -> 13.0, 6144 x 4096 9.0 -> 7.5; fp8, 64 rows 5120 x 2048 10.0 ->
-// 7.8, 4096 x 14336 29.1 -> 19.1.  Weights requested straight into registers, as the packed int4 words are: fp8 2048 x 4096, 64 rows 7.2 -> 6.9, 5
-// rows 6.1 -> 5.0 (a lane's piece of a row is half a line there).
+// Bound by the ramp of a launch (about 3 us), then by what a CU can take in, about 27 KB/us.  us, the kernel that parks one 16 KB chunk per workgroup in
+// registers -> here, the same bits (calls that follow each other over 0.7 GB of weights): 1536 x 8960 bf16, 27 rows 14.6 -> 8.6, 64 rows 17.7 -> 9.8; 1536 x
+// 1536 4.8 -> 4.0; 896 x 4864 fp16, 37 rows 10.6 -> 5.7; 4096 x 4096, 64 rows 13.6 -> 11.4, x 14336, one row 27.6 -> 21.7; int8 x int8, 30 rows 4096 x 14336 17.2 -> 12.5, 6144 x 4096 8.9 -> 8.0; fp8, 64 rows 5120
+// x 2048 10.0 -> 8.8, 4096 x 14336 27.6 -> 20.1.  In slices of its own choice, whose sums round otherwise, the bf16 and fp8 products take up to 0.9 us
+// less.  Weights requested straight into registers, as the packed int4 words are: fp8, 5 rows 2048 x 4096 6.1 -> 5.0 (a lane's piece of a row is half a
+// line there; gemm_short_dense.hip has the small 8-bit ones).
 #include "common.h"
 #include "gemm_w4_common.h"
 #include "gemm_w8_common.h"
@@ -24,6 +24,10 @@ typedef __bf16 sk_bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int SK_FP8 = 1, SK_I8 = 2, SK_I8I8 = 3, SK_F16 = 4, SK_BF16 = 5;
 
+// row groups that a tile of a format may have (a consumer wave each; eight leave a ring of three or four)
+constexpr int SK_MOST_GROUPS = 8;
+constexpr bool sk_tile(int wfmt, int groups) { return groups == 1 || groups == 2 || groups == 4 || (wfmt != SK_I8I8 && (groups == 3 || groups == 8)); }
+
 template <int WF, int MT, int GROUPS>
 struct SkLds {
   static constexpr bool W8A16 = WF == SK_FP8 || WF == SK_I8;
@@ -31,13 +35,12 @@ struct SkLds {
   static constexpr int XKB = W8A16 ? 256 : 128;     // bytes of an activation row per unit
   static constexpr int W_BYTES = GROUPS * 32 * KB, X_BYTES = MT * 32 * XKB, SLOT = W_BYTES + X_BYTES;
   static constexpr int FIT = 160 * 1024 / SLOT, R = FIT < 12 ? FIT : 12;
-  static constexpr int KQ = W8A16 ? 2 : 1;          // consumers of a row group: each widens and multiplies its share of a unit's columns
-  static constexpr int THREADS = 64 * (GROUPS * KQ + 4);
+  static constexpr int THREADS = 64 * (GROUPS + 4);
   static constexpr int WOPS = GROUPS, XOPS = X_BYTES / 4096, OPS = WOPS + XOPS;   // LDS-DMA operations per loader wave and unit
   static constexpr int OSTR = GROUPS * 32 + 4;      // words per row of the finished sums
   static constexpr int BYTES = R * SLOT;
-  static constexpr int SUMS = MT * 32 * OSTR * 4;   // bytes of a consumer set's sums
-  static_assert(KQ * SUMS <= BYTES && (R - 1) * OPS <= 63, "ring");
+  static constexpr int SUMS = MT * 32 * OSTR * 4;   // bytes of the tile's sums
+  static_assert(SUMS <= BYTES && (R - 1) * OPS <= 63, "ring");
 };
 
 struct SkParams {
@@ -49,7 +52,7 @@ struct SkParams {
   int64_t s_stride_n, s_stride_k;
   int m, group_n, group_k;
   int tiles, total, cap;           // items = slice * tiles + tile; workgroup b takes item (b % 8) * cap + b / 8
-  int ubase, urem;                 // slice s owns units [s * ubase + min(s, urem), + ubase + (s < urem))
+  int units, each;                 // slice s owns units [s * each, + each) of them
 };
 
 template <int N>
@@ -80,12 +83,12 @@ __global__ __launch_bounds__((SkLds<WF, MT, GROUPS>::THREADS)) void split_kernel
   const int item = ((int)blockIdx.x & 7) * p.cap + ((int)blockIdx.x >> 3);
   if ((int)blockIdx.x >> 3 >= p.cap || item >= p.total) return;
   const int slice = item / p.tiles, tile = item - slice * p.tiles;
-  const int u0 = slice * p.ubase + (slice < p.urem ? slice : p.urem), units = p.ubase + (slice < p.urem ? 1 : 0);
+  const int u0 = slice * p.each, units = p.units - u0 < p.each ? p.units - u0 : p.each;
   const int64_t row0 = (int64_t)tile * GROUPS * 32;
 
-  if (wv >= GROUPS * LD::KQ) {
+  if (wv >= GROUPS) {
     // ======================================== loaders ======================================== //
-    const int L = wv - GROUPS * LD::KQ;
+    const int L = wv - GROUPS;
     uint32_t woff[LD::WOPS], xoff[LD::XOPS];
 #pragma unroll
     for (int j = 0; j < LD::WOPS; ++j) {
@@ -125,8 +128,7 @@ __global__ __launch_bounds__((SkLds<WF, MT, GROUPS>::THREADS)) void split_kernel
     }
   } else {
     // ======================================= consumers ======================================= //
-    const int nl = lane & 31, h = lane >> 5;
-    const int rg = LD::KQ == 2 ? wv >> 1 : wv, kq = LD::KQ == 2 ? wv & 1 : 0;
+    const int nl = lane & 31, h = lane >> 5, rg = wv;
     f32x16 accf[MT];
     i32x16 acci[MT];
 #pragma unroll
@@ -137,8 +139,8 @@ __global__ __launch_bounds__((SkLds<WF, MT, GROUPS>::THREADS)) void split_kernel
     const unsigned char* xrow = lds + LD::W_BYTES + nl * XKB;
     const float* srow = nullptr;
     if constexpr (W8A16) srow = p.scales + ((row0 + rg * 32 + nl) / p.group_n) * p.s_stride_n;
-    auto scale_at = [&](int u) {  // of this wave's 64 columns of a unit (the last unit's again past it)
-      return srow[(int64_t)(((u0 + (u < units ? u : units - 1)) * 128 + kq * 64) / p.group_k) * p.s_stride_k];
+    auto scale_at = [&](int u) {  // of this lane's 64 columns of a unit (the last unit's again past it)
+      return srow[(int64_t)(((u0 + (u < units ? u : units - 1)) * 128 + h * 64) / p.group_k) * p.s_stride_k];
     };
     float sc = 0.f;
     if constexpr (W8A16) sc = scale_at(0);
@@ -147,32 +149,36 @@ __global__ __launch_bounds__((SkLds<WF, MT, GROUPS>::THREADS)) void split_kernel
     for (int u = 0; u < units; ++u) {
       float next = 0.f;
       if constexpr (W8A16) next = scale_at(u + 1);   // on its way under this unit's products
+      if constexpr (W8A16) {
+        // a lane half holds 64 columns of its row; a product takes eight of either half
+        const uint32_t sp = d8_bcast(WF == SK_FP8 ? sc * 256.0f : sc);
 #pragma unroll
-      for (int i = 0; i < 4 / LD::KQ; ++i) {
-        const int s = kq * (4 / LD::KQ) + i;
-        const u32x4 wf = *reinterpret_cast<const u32x4*>(wrow + slot + (((2 * s + h) ^ ((nl >> 1) & 7)) * 16));
-        if constexpr (W8A16) {
-          const uint32_t sp = d8_bcast(WF == SK_FP8 ? sc * 256.0f : sc);
+        for (int j = 0; j < 4; ++j) {
+          const u32x4 wf = *reinterpret_cast<const u32x4*>(wrow + slot + (((4 * h + j) ^ ((nl >> 1) & 7)) * 16));
           u32x4 a, b;
           uint32_t lo, hi;
-#define SK_WIDEN(D, W) if constexpr (WF == SK_FP8) d8_fp8(W, sp, lo, hi); else d8_i8(W, sp, lo, hi);
-          SK_WIDEN(a, wf.x) a.x = lo; a.y = hi;
-          SK_WIDEN(a, wf.y) a.z = lo; a.w = hi;
-          SK_WIDEN(b, wf.z) b.x = lo; b.y = hi;
-          SK_WIDEN(b, wf.w) b.z = lo; b.w = hi;
+#define SK_WIDEN(W) if constexpr (WF == SK_FP8) d8_fp8(W, sp, lo, hi); else d8_i8(W, sp, lo, hi);
+          SK_WIDEN(wf.x) a.x = lo; a.y = hi;
+          SK_WIDEN(wf.y) a.z = lo; a.w = hi;
+          SK_WIDEN(wf.z) b.x = lo; b.y = hi;
+          SK_WIDEN(wf.w) b.z = lo; b.w = hi;
 #undef SK_WIDEN
 #pragma unroll
           for (int mt = 0; mt < MT; ++mt) {
             const unsigned char* xb = xrow + slot + mt * 32 * XKB;
-            const u32x4 xa = *reinterpret_cast<const u32x4*>(xb + ((((2 * s + h) * 2) ^ (nl & 15)) * 16));
-            const u32x4 xc = *reinterpret_cast<const u32x4*>(xb + ((((2 * s + h) * 2 + 1) ^ (nl & 15)) * 16));
+            const u32x4 xa = *reinterpret_cast<const u32x4*>(xb + (((8 * h + 2 * j) ^ (nl & 15)) * 16));
+            const u32x4 xc = *reinterpret_cast<const u32x4*>(xb + (((8 * h + 2 * j + 1) ^ (nl & 15)) * 16));
             accf[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, xa), accf[mt], 0, 0, 0);
             accf[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, b), __builtin_bit_cast(f16x8, xc), accf[mt], 0, 0, 0);
           }
-        } else {
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const u32x4 wf = *reinterpret_cast<const u32x4*>(wrow + slot + (((2 * j + h) ^ ((nl >> 1) & 7)) * 16));
 #pragma unroll
           for (int mt = 0; mt < MT; ++mt) {
-            const u32x4 xf = *reinterpret_cast<const u32x4*>(xrow + slot + mt * 32 * XKB + (((2 * s + h) ^ ((nl >> 1) & 7)) * 16));
+            const u32x4 xf = *reinterpret_cast<const u32x4*>(xrow + slot + mt * 32 * XKB + (((2 * j + h) ^ ((nl >> 1) & 7)) * 16));
             if constexpr (WF == SK_F16)
               accf[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, wf), __builtin_bit_cast(f16x8, xf), accf[mt], 0, 0, 0);
             else if constexpr (WF == SK_BF16)
@@ -198,7 +204,7 @@ __global__ __launch_bounds__((SkLds<WF, MT, GROUPS>::THREADS)) void split_kernel
           if constexpr (I8A) v[e] = acci[mt][4 * g + e];
           else v[e] = (int)__float_as_uint(accf[mt][4 * g + e]);
         }
-        *reinterpret_cast<i32x4*>(lds + kq * LD::SUMS + ((mt * 32 + nl) * LD::OSTR + rg * 32 + 8 * g + 4 * h) * 4) = v;
+        *reinterpret_cast<i32x4*>(lds + ((mt * 32 + nl) * LD::OSTR + rg * 32 + 8 * g + 4 * h) * 4) = v;
       }
   }
   __syncthreads();
@@ -207,9 +213,7 @@ __global__ __launch_bounds__((SkLds<WF, MT, GROUPS>::THREADS)) void split_kernel
   for (int i = tid; i < p.m * QUADS; i += LD::THREADS) {
     const int r = i / QUADS, q = i - r * QUADS;
     const unsigned char* from = lds + (r * LD::OSTR + q * 4) * 4;
-    if constexpr (LD::KQ == 2)
-      *reinterpret_cast<f32x4*>(out + r * p.n + q * 4) = *reinterpret_cast<const f32x4*>(from) + *reinterpret_cast<const f32x4*>(from + LD::SUMS);
-    else *reinterpret_cast<i32x4*>(out + r * p.n + q * 4) = *reinterpret_cast<const i32x4*>(from);
+    *reinterpret_cast<i32x4*>(out + r * p.n + q * 4) = *reinterpret_cast<const i32x4*>(from);
   }
 }
 
@@ -225,31 +229,37 @@ int sk_num_cus() {
 }
 
 struct SkPlan {
-  int groups = 0, slices = 0;
+  int groups = 0, slices = 0, each = 0;   // each: units of a slice
 };
 
-// Row groups of a tile and slices.  us: a unit of GROUPS row groups at 27 KB/us, its activations at 130 KB/us and its barrier -- or, where weights are
-// widened, the consumers' time for it, which hardly depends on the groups -- and what a plane costs here and where it is added up.  At most a
-// workgroup per CU: two rounds double the ramp.
+// Row groups of a tile, slices and their units.  At most a workgroup per CU: two rounds double the ramp.
+// Floating sums round in the order they are formed in, and that order is the one of the kernel that parks a chunk per workgroup (gemm_w8_skinny.hip), which has
+// the shapes that are not served here: its slices, and within a unit its products -- a call's values do not depend on which of the two runs.  The tile is then the
+// narrowest that leaves no CU two.  Whole numbers have one sum: slices as they cost least.  us: a unit of GROUPS row groups at 27 KB/us, its
+// activations at 130 KB/us and its barrier, and what a plane costs here and where it is added up.
 SkPlan sk_plan(int64_t m, int64_t n, int64_t k, int wfmt, int max_splits) {
   SkPlan best;
   const bool w16 = wfmt == SK_F16 || wfmt == SK_BF16;
   if (wfmt < SK_FP8 || wfmt > SK_BF16 || m < 1 || m > 64 || n < 32 || n % 32 != 0 || max_splits < 1) return best;
   const int64_t row = w16 ? k * 2 : k;
   if (row < 128 || row % 128 != 0 || n >= (1 << 30) || k >= (1 << 24)) return best;
-  const int64_t units = row / 128, rgs = n / 32;
-  const int cus = sk_num_cus();
+  const int units = (int)(row / 128), cus = sk_num_cus();
+  const int64_t rgs = n / 32;
+  if (wfmt != SK_I8I8) {
+    const int s = d8_splits(n, k, w16 ? 64 : 128, max_splits), each = (units + s - 1) / s, slices = (units + each - 1) / each;
+    for (int g = 1; g <= SK_MOST_GROUPS; ++g)
+      if (sk_tile(wfmt, g) && rgs % g == 0 && rgs / g * slices <= cus) return SkPlan{g, slices, each};
+    return best;
+  }
   double least = 1e30;
   for (int g = 4; g >= 1; g /= 2) {
     if (rgs % g) continue;
     for (int s = 1; s <= max_splits && s <= units && rgs / g * s <= cus; ++s) {
-      const int64_t each = (units + s - 1) / s;
-      const double unit = wfmt < SK_I8I8 ? 0.5 + 0.05 * g : g * 4.0 / 27 + 4.0 / 130 + 0.05;
-      const double cost = each * unit + 0.15 * s;
+      const int each = (units + s - 1) / s;
+      const double cost = each * (g * 4.0 / 27 + 4.0 / 130 + 0.05) + 0.15 * s;
       if (cost < least) {
         least = cost;
-        best.groups = g;
-        best.slices = s;
+        best = SkPlan{g, (units + each - 1) / each, each};
       }
     }
   }
@@ -267,8 +277,8 @@ void sk_go(const SkParams& p, hipStream_t st) {
     (void)hipFuncSetAttribute((const void*)split_kernel<WF, MT, GROUPS>, hipFuncAttributeMaxDynamicSharedMemorySize, LD::BYTES);
     attr[dev] = true;
   }
-  const int units = p.ubase + (p.urem ? 1 : 0), sums = LD::KQ * LD::SUMS, ring = (units < LD::R ? units : LD::R) * LD::SLOT;
-  split_kernel<WF, MT, GROUPS><<<dim3((unsigned)(p.cap * 8)), LD::THREADS, ring > sums ? ring : sums, st>>>(p);
+  const int ring = (p.each < LD::R ? p.each : LD::R) * LD::SLOT;
+  split_kernel<WF, MT, GROUPS><<<dim3((unsigned)(p.cap * 8)), LD::THREADS, ring > LD::SUMS ? ring : LD::SUMS, st>>>(p);
 }
 
 }  // namespace
@@ -282,25 +292,21 @@ int sk_launch(void* out, const void* x, const void* w, const float* scales, int6
   const SkPlan pl = sk_plan(m, n, k, wfmt, max_splits);
   if (!pl.slices) return 0;
   if (w_stride % 16 || x_stride % 16 || !ll_aligned16(w) || !ll_aligned16(x) || !ll_aligned16(out)) return 0;
-  if (128 * w_stride >= (1ll << 31) || m * x_stride >= (1ll << 31)) return 0;
+  if (SK_MOST_GROUPS * 32 * w_stride >= (1ll << 31) || m * x_stride >= (1ll << 31)) return 0;
   SkParams p{};
   p.part = out; p.x = (const unsigned char*)x; p.w = (const unsigned char*)w; p.scales = scales;
   p.n = n; p.x_stride = x_stride; p.w_stride = w_stride; p.s_stride_n = s_stride_n; p.s_stride_k = s_stride_k;
   p.m = (int)m; p.group_n = group_n > 0 ? group_n : 1;
   p.group_k = group_k > 0 && group_k < k ? (int)group_k : (int)k;
-  const bool w16 = wfmt == SK_F16 || wfmt == SK_BF16;
-  const int units = (int)((w16 ? k * 2 : k) / 128);
+  p.units = (int)((wfmt == SK_F16 || wfmt == SK_BF16 ? k * 2 : k) / 128);
+  p.each = pl.each;
   p.tiles = (int)(n / (32 * pl.groups));
   p.total = p.tiles * pl.slices;
   p.cap = (p.total + 7) / 8;
-  p.ubase = units / pl.slices;
-  p.urem = units % pl.slices;
   hipStream_t st = (hipStream_t)stream;
-#define SK_G(WF, MT)                                       \
-  if (pl.groups == 4) sk_go<WF, MT, 4>(p, st);             \
-  else if (pl.groups == 2) sk_go<WF, MT, 2>(p, st);        \
-  else sk_go<WF, MT, 1>(p, st)
-#define SK_M(WF) if (m > 32) { SK_G(WF, 2); } else { SK_G(WF, 1); }
+#define SK_T(WF, MT, G) if constexpr (sk_tile(WF, G)) { if (pl.groups == G) sk_go<WF, MT, G>(p, st); }
+#define SK_G(WF, MT) SK_T(WF, MT, 1) SK_T(WF, MT, 2) SK_T(WF, MT, 3) SK_T(WF, MT, 4) SK_T(WF, MT, 8)
+#define SK_M(WF) if (m > 32) { SK_G(WF, 2) } else { SK_G(WF, 1) }
   switch (wfmt) {
     case SK_FP8: SK_M(SK_FP8) break;
     case SK_I8: SK_M(SK_I8) break;
@@ -310,5 +316,6 @@ int sk_launch(void* out, const void* x, const void* w, const float* scales, int6
   }
 #undef SK_M
 #undef SK_G
+#undef SK_T
   return hipGetLastError() == hipSuccess ? pl.slices : LL_ERR_LAUNCH;
 }

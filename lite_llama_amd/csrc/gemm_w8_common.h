@@ -29,3 +29,12 @@ __device__ __forceinline__ void d8_fp8(uint32_t w, uint32_t s256, uint32_t& o0, 
   o1 = d8_mul(p1, s256);
 }
 
+// slices of a split-K projection over chunks of 128 bytes of every weight row (gemm_w8_skinny.hip, gemm_split.hip: the order of a sum)
+inline int d8_splits(int64_t n, int64_t k, int kch = 128, int cap = 1 << 30) {
+  const int tiles = (int)((n + 127) / 128), chunks = (int)(k / kch);
+  int s = (768 + tiles - 1) / tiles;   // ~3 resident workgroups per CU ...
+  if (s > chunks / 2) s = chunks / 2;  // ... of at least two chunks each (the tile prefetch needs something to hide behind)
+  if (s > cap) s = cap;                // (partial mode: what the consumer of the planes adds up in one pass)
+  if (s < 1) s = 1;
+  return s;
+}

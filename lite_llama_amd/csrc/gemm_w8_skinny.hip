@@ -16,7 +16,8 @@
 #include "common.h"
 #include "gemm_w8_common.h"
 
-// the form that streams a CU's whole share through LDS (gemm_split.hip): rows of whole 128-byte lines, n % 32 == 0
+// the form that streams a CU's whole share through LDS (gemm_split.hip): rows of whole 128-byte lines, n % 32 == 0.  Floating sums are formed in one order in
+// both, so that rounding does not depend on the form
 int sk_partials_slices(int64_t m, int64_t n, int64_t k, int wfmt, int max_splits);
 int sk_launch(void* out, const void* x, const void* w, const float* scales, int64_t m, int64_t n, int64_t k, int group_n, int64_t group_k,
               int wfmt, int64_t x_stride, int64_t w_stride, int64_t s_stride_n, int64_t s_stride_k, int max_splits, void* stream);
@@ -267,15 +268,6 @@ __global__ __launch_bounds__(256) void dense8_finish(uint16_t* __restrict__ out,
   *reinterpret_cast<uint2*>(out + i) = uint2{(uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16)};
 }
 
-int d8_splits(int64_t n, int64_t k, int kch = 128, int cap = 1 << 30) {
-  const int tiles = (int)((n + 127) / 128), chunks = (int)(k / kch);
-  int s = (768 + tiles - 1) / tiles;   // ~3 resident workgroups per CU ...
-  if (s > chunks / 2) s = chunks / 2;  // ... of at least two chunks each (the tile prefetch needs something to hide behind)
-  if (s > cap) s = cap;                // (partial mode: what the consumer of the planes adds up in one pass)
-  if (s < 1) s = 1;
-  return s;
-}
-
 }  // namespace
 
 // shapes the skinny engine takes (the dispatchers of gemm_wq.hip ask; also sizes the partial planes in ll_gemm_workspace)
@@ -366,8 +358,6 @@ extern "C" int ll_dense16_matmul(void* out, const void* x, const void* w, const 
     p.direct_out = (uint16_t*)out;
     p.direct_bias = (const uint16_t*)bias;
   }
-  // (The planes of gemm_split.hip would take 3 us less at 32 rows of 2048 x 4096, 14.2 with the finish.  They are added up in another order, and near
-  // ties of a router further on turn that into other experts: these finished rows keep theirs.)
   if (dtype == LL_F16) {
     if (m > 32) dense8_kernel<D8_F16, 2><<<grid, 256, 0, st>>>(p);
     else dense8_kernel<D8_F16, 1><<<grid, 256, 0, st>>>(p);
@@ -432,9 +422,9 @@ extern "C" int ll_dense_partials(float* partials, const void* x, const void* w, 
   if (sd_partials_slices(m, n, k, wfmt, max_splits))  // (declines -- 0 -- exactly where the engines below would)
     return sd_launch(partials, x, w, scales, m, n, k, group_n, group_k, wfmt, x_stride, w_stride * eb, s_stride_n, s_stride_k,
                      max_splits, stream);
-  if (sk_partials_slices(m, n, k, wfmt, max_splits))
-    return sk_launch(partials, x, w, scales, m, n, k, group_n, group_k, wfmt, x_stride * (i8a ? 1 : 2), w_stride * eb, s_stride_n, s_stride_k,
-                     max_splits, stream);
+  if (const int r = sk_launch(partials, x, w, scales, m, n, k, group_n, group_k, wfmt, x_stride * (i8a ? 1 : 2), w_stride * eb, s_stride_n,
+                              s_stride_k, max_splits, stream))
+    return r;
   D8Params p{};
   p.part = partials; p.x = x; p.w = (const unsigned char*)w; p.scales = scales;
   p.m = m; p.n = n; p.k = k; p.x_stride = x_stride; p.w_stride = w_stride * eb;

@@ -98,3 +98,31 @@ def test_scales_of_a_block_meet_its_columns_alone(fmt, m, n, k, group_n, group_k
     # fp32 sums of k exact products, in whatever order
     bound = k * 2.0 ** -24 * (x.double().abs() @ wide.abs().T) + 1e-30
     assert ((planes.double().sum(0) - x.double() @ wide.T).abs() <= bound).all()
+
+
+# tiles of one, two, three, four and eight row groups; slices of one unit, of many, a short last one
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt,m,n,k,cap", [(f, *s) for f in (F16, BF16) for s in (
+    (27, 1536, 8960, 12), (64, 1536, 1536, 12), (27, 2048, 1536, 8), (37, 896, 4864, 12), (37, 896, 896, 12), (33, 1024, 4096, 12), (5, 2048, 2048, 12),
+    (7, 256, 2048, 12), (1, 128, 64, 12), (64, 4096, 4096, 12), (32, 4096, 1216, 12))] + [(f, *s) for f in (FP8, I8) for s in (
+        (64, 5120, 2048, 8), (7, 5120, 2048, 12), (31, 4096, 14336, 12), (64, 4096, 14336, 12), (9, 1536, 8960, 12), (33, 1024, 12288, 8), (64, 2048, 8192, 8))])
+def test_sums_are_formed_in_one_order(fmt, m, n, k, cap):
+    """The same planes, bit for bit, where four weight rows less put the call on the kernel of gemm_w8_skinny.hip: as many slices, and every sum in its order."""
+    g = torch.Generator(device=DEV).manual_seed(n + k + m)
+    scales, gk = None, k
+    if fmt in (F16, BF16):
+        dt = torch.float16 if fmt == F16 else torch.bfloat16
+        w, x = torch.randn(n, k, generator=g, device=DEV).to(dt), torch.randn(m, k, generator=g, device=DEV).to(dt)
+    else:
+        x, gk = torch.randn(m, k, generator=g, device=DEV).half(), 64
+        w = (torch.randn(n, k, generator=g, device=DEV).to(torch.float8_e4m3fn).view(torch.uint8) if fmt == FP8 else
+             torch.randint(-127, 128, (n, k), generator=g, device=DEV, dtype=torch.int8))
+        scales = 0.5 + torch.rand(-(-n // 32), k // gk, generator=g, device=DEV)
+    got = []
+    for rows in (n, n - 4):
+        count = L.lib().ll_dense_partials_count(m, rows, k, fmt, cap)
+        planes = torch.full((count, m, rows), float("nan"), device=DEV)
+        assert L.lib().ll_dense_partials(planes.data_ptr(), x.data_ptr(), w.data_ptr(), L.ptr(scales), m, rows, k, 32, gk, fmt, k, k,
+                                         0 if scales is None else scales.stride(0), 0 if scales is None else 1, cap, L.stream_ptr()) == count
+        got.append(planes[:, :, :n - 4])
+    assert torch.equal(*got)
