@@ -384,15 +384,19 @@ def add_norm(hidden_states, residual, weight, eps, q8: bool = False):
 
 
 def _rows_of(hidden_states, residual, rows):
-    """``(whether it could be done, update, residual)`` of the listed rows alone."""
+    """``(whether it could be done, update, residual)`` of the rows that ``rows`` picks (whatever indexes a tensor's first dimension) alone."""
     width = residual.shape[-1]
+    picked = residual.reshape(-1, width)[rows]
+    if picked.numel() == 0:
+        return False, hidden_states, residual
     if torch.is_tensor(hidden_states):
-        hidden_states = hidden_states.view(-1, width)[rows]
+        hidden_states = hidden_states.reshape(-1, width)[rows]
     elif type(hidden_states) is SlotSums:
-        hidden_states = SlotSums(hidden_states.parts[rows], (rows.numel(), width))
+        parts = hidden_states.parts
+        hidden_states = SlotSums(parts[rows].reshape(-1, *parts.shape[1:]).contiguous(), tuple(picked.shape))
     else:
         return False, hidden_states, residual
-    return True, hidden_states, residual.view(-1, width)[rows]
+    return True, hidden_states, picked
 
 
 class FusedMLP(nn.Module):
