@@ -224,9 +224,9 @@ extern "C" int ll_embed_rmsnorm(void* y, void* residual, const void* table, cons
                                 int64_t table_rows, float eps, int dtype, void* stream) {
   if (dtype != LL_F16 && dtype != LL_BF16) return LL_ERR_DTYPE;
   if (rows < 0 || n <= 0 || n % 8 != 0 || n > 8192 || table_rows < 1) return LL_ERR_SHAPE;
+  if (rows == 0) return LL_OK;
   if (!y || !residual || !table || !ids || !weight || !ll_aligned16(y) || !ll_aligned16(residual) || !ll_aligned16(table) || !ll_aligned16(weight))
     return LL_ERR_ARG;
-  if (rows == 0) return LL_OK;
   hipStream_t st = (hipStream_t)stream;
   const int nv = (int)(n / 8);
 #define LL_EMBED_CASE(DT, TPR, VPT)                                                                                      \

@@ -283,9 +283,9 @@ extern "C" int ll_skip_rmsnorm_q8(void* y, int8_t* q, float* q_scale, const void
 extern "C" int ll_embed_rmsnorm_q8(void* y, int8_t* q, float* q_scale, void* residual, const void* table, const int64_t* ids, const void* weight,
                                    int64_t rows, int64_t n, int64_t table_rows, float eps, void* stream) {
   if (rows < 0 || n <= 0 || n % 8 != 0 || n > 8192 || table_rows < 1) return LL_ERR_SHAPE;
+  if (rows == 0) return LL_OK;
   if (!residual || !table || !ids || !weight || (!y && !q) || (q && !q_scale)) return LL_ERR_ARG;
   if (!ll_aligned16(y) || !ll_aligned16(residual) || !ll_aligned16(table) || !ll_aligned16(weight) || ((uintptr_t)q & 7) != 0) return LL_ERR_ARG;
-  if (rows == 0) return LL_OK;
   hipStream_t st = (hipStream_t)stream;
   const int nv = (int)(n / 8);
 #define LL_Q8_EMBED(VPT)                                                                                                              \

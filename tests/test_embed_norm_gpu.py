@@ -50,6 +50,18 @@ def test_a_wide_first_norm_rounds_as_the_norm_of_rows_does(dtype, n):
     assert torch.equal(r, x) and torch.equal(y, want)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_a_step_without_rows(dtype):
+    table, weight = torch.randn(50, 128, device=DEV).to(dtype), torch.ones(128, dtype=dtype, device=DEV)
+    for shape in ((0, 1), (3, 0)):
+        rows = EmbeddedRows(torch.zeros(shape, dtype=torch.int64, device=DEV), table)
+        y, r = embed_rmsnorm(rows, weight, 1e-6)
+        assert y.shape == r.shape == (*shape, 128)
+        if dtype == torch.float16:
+            got, r = skip_rmsnorm_q8(rows, None, weight, 1e-6)
+            assert got.q.shape == (0, 128) and got.scale.shape == (0,) and r.shape == (*shape, 128)
+
+
 def test_copies_of_a_steps_inputs():
     src = [torch.randint(0, 1 << 20, (n,), device=DEV, dtype=dt) for n, dt in ((1, torch.int64), (64, torch.int64), (300, torch.int32), (7, torch.int32))]
     dst = [torch.full((s.numel() + 1,), -5, device=DEV, dtype=s.dtype) for s in src]
