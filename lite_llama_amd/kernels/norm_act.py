@@ -103,6 +103,8 @@ def embed_rmsnorm(X: EmbeddedRows, weight, eps=1e-5, *, q8: bool = False):
         L.check(L.lib().ll_embed_rmsnorm_q8(0, q.data_ptr(), scale.data_ptr(), residual.data_ptr(), X.table.data_ptr(), X.ids.data_ptr(),
                                             weight.data_ptr(), rows, n, X.table.shape[0], float(eps), L.stream_ptr()), "embed_rmsnorm_q8")
         return Int8Rows(q, scale, X.shape), residual.view(X.shape)
+    if weight.data_ptr() % 16:   # (inside a flat tensor: the kernel reads whole pieces)
+        weight = weight.clone()
     Y = torch.empty_like(residual)
     L.check(L.lib().ll_embed_rmsnorm(Y.data_ptr(), residual.data_ptr(), X.table.data_ptr(), X.ids.data_ptr(), weight.data_ptr(), rows, n,
                                      X.table.shape[0], float(eps), L.dtype_code(X.dtype), L.stream_ptr()), "embed_rmsnorm")

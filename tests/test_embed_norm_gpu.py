@@ -62,6 +62,18 @@ def test_a_step_without_rows(dtype):
             assert got.q.shape == (0, 128) and got.scale.shape == (0,) and r.shape == (*shape, 128)
 
 
+@pytest.mark.parametrize("n", [128, 3584])
+def test_a_norms_weight_inside_a_flat_tensor(n):
+    """Weights that begin where no 16-byte piece does."""
+    table, flat = torch.randn(50, n, device=DEV).half(), 1 + 0.1 * torch.randn(n + 8, device=DEV).half()
+    ids = torch.arange(20, device=DEV).view(20, 1)
+    for at in (1, 2, 4):
+        weight = flat[at:at + n]
+        y, r = embed_rmsnorm(EmbeddedRows(ids, table), weight, 1e-6)
+        want, _ = skip_rmsnorm(F.embedding(ids, table), None, weight.clone(), 1e-6)
+        assert torch.equal(y, want)
+
+
 def test_copies_of_a_steps_inputs():
     src = [torch.randint(0, 1 << 20, (n,), device=DEV, dtype=dt) for n, dt in ((1, torch.int64), (64, torch.int64), (300, torch.int32), (7, torch.int32))]
     dst = [torch.full((s.numel() + 1,), -5, device=DEV, dtype=s.dtype) for s in src]
