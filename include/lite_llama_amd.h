@@ -742,7 +742,7 @@ int ll_gated_group_norm(const float* x_in, float* x_out, void* h_out, const void
                         const float* shared_scale, const void* gate, int64_t gate_ld, const void* gate_bias,
                         const void* post_w, const void* next_w, int64_t n, int64_t width, int64_t groups, float eps,
                         const void* y_bias, int dtype, void* stream);
-/* h [n][width] = table[ids] (16 bit, a row that the table does not have: NaN) and x = the same in fp32. */
+/* h [n][width] = table[ids] (16 bit, a row that the table does not have: NaN) and, unless NULL, x = the same in fp32. */
 int ll_embed_rows(float* x, void* h, const void* table, const void* ids, int id_width, int64_t n, int64_t width, int64_t vocab, int dtype,
                   void* stream);
 /* out [n, ff] (rows of stride out_ld) = act(gate[t][j]) * up[t][j], gate / up rows of stride gate_ld / up_ld; kind 0: silu,

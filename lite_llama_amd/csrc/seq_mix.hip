@@ -344,7 +344,7 @@ __global__ __launch_bounds__(256) void residual_set_kernel(float* __restrict__ x
   }
 }
 
-// A workgroup per token: its embedding row as it is and as the fp32 residual (a row that the table does not have: NaN).  VEC: 8-value pieces.
+// A workgroup per token: its embedding row as it is and, if asked for, as the fp32 residual (a row that the table does not have: NaN).  VEC: 8-value pieces.
 template <int DT, bool VEC>
 __global__ __launch_bounds__(256) void embed_rows_kernel(float* __restrict__ x, uint16_t* __restrict__ h, const uint16_t* __restrict__ table,
                                                          const void* __restrict__ ids, int id_w, int64_t vocab, int width) {
@@ -363,14 +363,16 @@ __global__ __launch_bounds__(256) void embed_rows_kernel(float* __restrict__ x, 
         hi[e] = to_f32<DT>(v.v[4 + e]);
       }
       *reinterpret_cast<U16x8*>(h + t * width + i) = v;
-      *reinterpret_cast<f32x4*>(x + t * width + i) = lo;
-      *reinterpret_cast<f32x4*>(x + t * width + i + 4) = hi;
+      if (x) {
+        *reinterpret_cast<f32x4*>(x + t * width + i) = lo;
+        *reinterpret_cast<f32x4*>(x + t * width + i + 4) = hi;
+      }
     }
   } else {
     for (int i = threadIdx.x; i < width; i += 256) {
       const uint16_t v = known ? from[i] : (uint16_t)0x7fff;
       h[t * width + i] = v;
-      x[t * width + i] = to_f32<DT>(v);
+      if (x) x[t * width + i] = to_f32<DT>(v);
     }
   }
 }
@@ -929,7 +931,7 @@ extern "C" int ll_embed_rows(float* x, void* h, const void* table, const void* i
   if (id_width != LL_I32 && id_width != LL_I64) return LL_ERR_DTYPE;
   if (n < 0 || width < 1 || width > (1 << 20) || vocab < 1) return LL_ERR_SHAPE;
   if (n == 0) return LL_OK;
-  if (!x || !h || !table || !ids) return LL_ERR_ARG;
+  if (!h || !table || !ids) return LL_ERR_ARG;
   hipStream_t st = (hipStream_t)stream;
   const bool vec = width % 8 == 0 && ll_aligned16(x) && ll_aligned16(h) && ll_aligned16(table);
 #define CALL(DT, VEC) \

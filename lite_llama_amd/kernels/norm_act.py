@@ -555,6 +555,21 @@ def residual_set(y: torch.Tensor, bias: torch.Tensor | None = None, out: torch.T
     return out
 
 
+@torch.no_grad()
+def embedding(ids: torch.Tensor, table: torch.Tensor):
+    """``F.embedding(ids, table)``; an id that the table does not have is answered with NaN, as :func:`embed_rmsnorm` does.  ``None`` where the
+    call is not served."""
+    if (type(ids) is not torch.Tensor or not ids.is_cuda or ids.dtype not in (torch.int32, torch.int64) or table.device != ids.device
+            or table.dtype not in (torch.float16, torch.bfloat16) or table.dim() != 2 or not table.is_contiguous() or table.shape[0] < 1
+            or not 0 < table.shape[1] <= 1 << 20 or not L.has("ll_embed_rows")):
+        return None
+    ids = ids.contiguous()
+    h = torch.empty(*ids.shape, table.shape[1], dtype=table.dtype, device=ids.device)
+    L.check(L.lib().ll_embed_rows(0, h.data_ptr(), table.data_ptr(), ids.data_ptr(), L.index_width(ids), ids.numel(), table.shape[1], table.shape[0],
+                                  L.dtype_code(table.dtype), L.stream_ptr()), "embed_rows")
+    return h
+
+
 class FirstRows:
     """The rows that open a stack, in the storage dtype: what a sublayer that reads the residual stream itself reads first."""
 

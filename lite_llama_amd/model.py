@@ -28,7 +28,7 @@ from .distributed.parallel_state import all_reduce_tp, divide, get_tp_rank, get_
 from .distributed.partition import ShardPlan, make_plan, scale_unit, set_active_plan
 from .kernels.attention import decode_attention, decode_attention_partials, decode_attention_partials_supported
 from .kernels.kv_cache import pack_prompts
-from .kernels.norm_act import (EmbeddedRows, Int8Rows, PartialSums, ScaledInt32Partials, SlotSums, embed_rmsnorm, norm_rope_and_cache_supported,
+from .kernels.norm_act import (EmbeddedRows, Int8Rows, PartialSums, ScaledInt32Partials, SlotSums, embed_rmsnorm, embedding, norm_rope_and_cache_supported,
                                rope_and_cache, rotary_rows, skip_rmsnorm_partials, skip_rmsnorm_q8)
 from .kernels import (
     flash_attention2_no_pad,
@@ -660,13 +660,17 @@ class CausalLM(nn.Module):
 
     def _embed(self, input_ids):
         """The embedding -- left to the first layer's norm where nothing but that would see it, and the pass is not one of the short prefills
-        that run their layers by a host call each."""
+        that run their layers by a host call each.  An id that the table does not have is NaN on either way; a module that something looks on, and one of
+        another kind, answers for itself."""
         embed = self.embed_tokens
-        if (not self.layers or not (input_ids.dim() == 2 and (input_ids.shape[1] == 1 or input_ids.numel() > ShortPrefill.MAX_TOKENS))
-                or not _plain(embed, nn.Embedding) or embed.max_norm is not None or not _plain(self.layers[0], DecoderLayer)
-                or not _plain(self.rotary_emb, RotaryEmbedding) or _nn._global_forward_hooks or _nn._global_forward_pre_hooks
-                or _nn._global_backward_hooks or _nn._global_backward_pre_hooks or not EmbeddedRows.served(input_ids, embed.weight)):
+        if (not _plain(embed, nn.Embedding) or embed.max_norm is not None or _nn._global_forward_hooks or _nn._global_forward_pre_hooks
+                or _nn._global_backward_hooks or _nn._global_backward_pre_hooks):
             return embed(input_ids)
+        if (not self.layers or not (input_ids.dim() == 2 and (input_ids.shape[1] == 1 or input_ids.numel() > ShortPrefill.MAX_TOKENS))
+                or not _plain(self.layers[0], DecoderLayer) or not _plain(self.rotary_emb, RotaryEmbedding)
+                or not EmbeddedRows.served(input_ids, embed.weight)):
+            rows = embedding(input_ids, embed.weight)
+            return rows if rows is not None else embed(input_ids)
         return EmbeddedRows(input_ids, embed.weight)
 
     @torch.no_grad()

@@ -2,8 +2,9 @@
 
 import pytest
 import torch
+import torch.nn.functional as F
 
-from lite_llama_amd.kernels.norm_act import embed_rows
+from lite_llama_amd.kernels.norm_act import EmbeddedRows, embed_rows, embedding
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -21,3 +22,33 @@ def test_embedding_rows(dtype, index, n, width):
     x, first = embed_rows(ids, table)
     assert x[n - 1].isnan().all() and first.rows[n - 1].isnan().all()
     assert embed_rows(ids, table.t().contiguous().t()) is None and embed_rows(ids.cpu(), table) is None
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("index", [torch.int32, torch.int64])
+@pytest.mark.parametrize("width", [8, 12, 2056])
+def test_rows_without_the_residual(dtype, index, width):
+    table = torch.randn(9, width, device=DEV).to(dtype)
+    for ids in (torch.randint(0, 9, (2, 5), device=DEV, dtype=index), torch.arange(8, device=DEV, dtype=index).view(2, 4).t(),
+                torch.tensor(3, device=DEV, dtype=index), torch.zeros(0, 3, device=DEV, dtype=index)):
+        assert torch.equal(embedding(ids, table), F.embedding(ids, table))
+    assert embedding(ids.cpu(), table) is None and embedding(ids, table.float()) is None and embedding(ids, table[:, 1:]) is None
+
+
+@pytest.mark.parametrize("index", [torch.int32, torch.int64])
+@pytest.mark.parametrize("shape", [(2, 1), (2, 3), (1, 200), (7,)])
+def test_an_id_outside_the_table_is_nan_on_every_route(index, shape):
+    """Decoded tokens, short prefills, long ones: no route reads past the table."""
+    from lite_llama_amd.model import CausalLM, tiny_geometry
+
+    with torch.device(DEV):
+        model = CausalLM(tiny_geometry(hidden_size=64, intermediate_size=128, num_layers=1, num_heads=4, num_kv_heads=2, head_dim=16, vocab_size=32))
+    ids = torch.randint(0, 32, shape, device=DEV, dtype=index)
+    for odd in (32, -1, 1 << 30):
+        ids.view(-1)[0] = odd
+        rows = model._embed(ids)
+        if isinstance(rows, EmbeddedRows):
+            assert index == torch.int64 and len(shape) == 2 and (shape[1] == 1 or shape[1] > 192)   # (left to the first norm: tests/test_embed_norm_gpu.py)
+            continue
+        assert rows.shape == (*shape, 64)
+        assert rows.view(-1, 64)[0].isnan().all() and torch.equal(rows.view(-1, 64)[1:], model.embed_tokens.weight[ids.view(-1)[1:].long()])
