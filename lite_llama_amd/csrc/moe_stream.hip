@@ -20,8 +20,8 @@
 //     groups, two workgroups per CU for 8-bit weights, which this replaces: the second one of a CU came 10 us late, and a tile of one group
 //     took as long as one of four.  us for both products, that -> here: 8-bit floats, 128 experts of 2048 / 768, top 8: 1 token 34 -> 29.9,
 //     8 70 -> 65, 32 108 -> 102, 64 124 -> 119 (604 MB: 5.1 TB/s), 128 140 -> 136, 200 169 -> 151, 256 174 -> 155, 320 191 -> 192; bf16, 34 of
-//     2048 / 704, top 4: 1 21.2 -> 21.1, 4 42 -> 33, 32 63 -> 59, 128 68 -> 62, 262 81 -> 67; 68 of 3072 / 512, top 8: 1 27.8 -> 29.1 (24 units
-//     of two groups in a row: latency), 6 69 -> 67, 32 119 -> 114, 128 133 -> 124, 262 159 -> 135.
+//     2048 / 704, top 4: 1 21.2 -> 21.1, 4 42 -> 33, 32 63 -> 59, 128 68 -> 62, 262 81 -> 67; 68 of 3072 / 512, top 8: 1 27.8 -> 28.0 (24 units
+//     of two groups in a row: latency; tiles of up to two groups have a ring of six, with one of four 29.1), 6 69 -> 67, 32 119 -> 114, 128 133 -> 124, 262 159 -> 135.
 //   Lines against the tiles (before that change; us, tiles -> streams): 8-bit floats, 128 of 2048 / 768: 1 token 42 -> 24, 64 137 -> 117, 320 181 ->
 //   168, 400 186 -> 191; bf16, 34 of 2048 / 704, top 4: 1 token 33 -> 17, 128 78 -> 65, 300 (35 rows per expert) 78.5 -> 77, 400 (47) 80 -> 85; 68 of
 //   3072 / 512: 262 (31) 165 -> 150: up to 36 rows per expert in ll_moe_rows_gemm.  ll_moe_gemm has other tiles and lines of its own (moe.hip).
@@ -46,7 +46,8 @@ struct MsLds {
   static constexpr int XB = KU * 2;                            // bytes of an activation row per unit
   static constexpr int X_BYTES = ROWS * XB;
   static constexpr int S_BYTES = WF == MS_W16 ? 0 : 8 * 4 * 16 * 4;   // scales: [row group][64-column step][16 rows], or, alike in 16 rows, [row group][step]
-  static constexpr int slot(int groups) { return groups * 16 * MS_KB + X_BYTES + S_BYTES; }   // of the ring: three units of eight row groups, four of four
+  static constexpr int slot(int groups) { return groups * 16 * MS_KB + X_BYTES + S_BYTES; }   // of the ring: three units of eight row groups, four of four, six of two
+  static constexpr int ring(int groups) { return groups == 8 ? 3 : groups == 4 ? 4 : 3 * slot(8) < 6 * slot(2) ? 5 : 6; }
   static constexpr int LIST = 3 * slot(8);                  // int32 [MS_LIST]: row block | expert << 16
   static constexpr int SLOTS = LIST + MS_LIST * 4;             // int32 [MS_OWN][ROWS]
   static constexpr int FROM = SLOTS + MS_OWN * ROWS * 4;       // uint32 [MS_OWN][ROWS]: where the slot's activations begin, bytes
@@ -55,7 +56,8 @@ struct MsLds {
   static constexpr int BYTES = COUNTS + 16;                    // (nothing static: the ring begins at LDS byte 0)
   static_assert(BYTES <= 160 * 1024, "LDS");
   static constexpr int XOPS = X_BYTES / 4096;                  // activation operations per loader and unit, at most
-  static_assert(4 * slot(4) <= LIST && 8 + 2 + XOPS <= 18 && 2 * (4 + 1 + XOPS) <= 18, "the ring, the waits");
+  static_assert(ring(4) * slot(4) <= LIST && ring(2) * slot(2) <= LIST && 8 + 2 + XOPS <= 24 && 2 * (4 + 1 + XOPS) <= 24 &&
+                    (ring(2) - 2) * (2 + (WF != MS_W16) + XOPS) <= 24, "the ring, the waits");
 };
 
 __device__ const uint32_t ms_zeros[4] __attribute__((aligned(16))) = {0, 0, 0, 0};   // what pieces without an entry read
@@ -72,6 +74,7 @@ __device__ __forceinline__ void ms_wait(int k) {   // at most k operations may s
 #define MS_C(K) case K: v3_vmcnt<K>(); break;
   switch (k) {
     MS_C(1) MS_C(2) MS_C(3) MS_C(4) MS_C(5) MS_C(6) MS_C(7) MS_C(8) MS_C(9) MS_C(10) MS_C(11) MS_C(12) MS_C(13) MS_C(14) MS_C(15) MS_C(16) MS_C(17) MS_C(18)
+    MS_C(19) MS_C(20) MS_C(21) MS_C(22) MS_C(23) MS_C(24)
     default: v3_vmcnt<0>(); break;
   }
 #undef MS_C
@@ -145,7 +148,8 @@ template <int WF, int MT, int MODE, int GROUPS>
 __device__ __forceinline__ void ms_load(const MoeStreamParams& p, unsigned char* lds, int L, int lane, MsWalk run, int rgs, int i0, int units, int total) {
   using LD = MsLds<WF, MT>;
   constexpr int KU = LD::KU, EB = WF == MS_W16 ? 2 : 1, ROWS = LD::ROWS, XOPS = LD::XOPS, XL = LD::XB / 16;   // lanes of an activation row
-  constexpr int RING = GROUPS == 4 ? 4 : 3, W_BYTES = GROUPS * 16 * MS_KB, SLOT = LD::slot(GROUPS);
+  constexpr int RING = LD::ring(GROUPS), W_BYTES = GROUPS * 16 * MS_KB, SLOT = LD::slot(GROUPS);
+  constexpr int SOPS = GROUPS == 8 ? 2 : 1;   // requests of a unit's scales, where not all 16 rows share them
   const uint32_t* list = reinterpret_cast<const uint32_t*>(lds + LD::LIST);
   const int32_t* rows = reinterpret_cast<const int32_t*>(lds + LD::FROM);
   const int row_bytes = p.K * EB;
@@ -176,7 +180,7 @@ __device__ __forceinline__ void ms_load(const MoeStreamParams& p, unsigned char*
       if constexpr (WF != MS_W16) {
         sbase = (const char*)(p.scales + (int64_t)e * p.s_stride_e);
 #pragma unroll
-        for (int j = 0; j < GROUPS / 4; ++j) {
+        for (int j = 0; j < SOPS; ++j) {
           int row = p.rows16 ? 16 * (r0 + (lane >> 2)) : 16 * (r0 + 4 * j + L) + (lane & 15);
           row = row < p.N ? row : p.N - 1;
           soff[j] = (uint32_t)(p.n_shift >= 0 ? row >> p.n_shift : row / (int)p.group_n) * (uint32_t)(p.s_stride_n * 4);
@@ -199,7 +203,7 @@ __device__ __forceinline__ void ms_load(const MoeStreamParams& p, unsigned char*
       int k = wunit * KU + (p.rows16 ? lane & 3 : lane >> 4) * 64;
       k = k < p.K ? k : p.K - 1;
 #pragma unroll
-      for (int j = 0; j < GROUPS / 4; ++j)
+      for (int j = 0; j < SOPS; ++j)
         if (p.rows16 ? j == 0 && L == 3 : 4 * j + L < groups) v3_dma4<false>(wdst + W_BYTES + LD::X_BYTES + (p.rows16 ? 0 : (4 * j + L) * 256), sbase, soff[j] + (uint32_t)(k >> p.k_shift) * (uint32_t)(p.s_stride_k * 4));
     }
     if (++wunit == units) wunit = 0;
@@ -249,18 +253,22 @@ __device__ __forceinline__ void ms_load(const MoeStreamParams& p, unsigned char*
   for (int i = 0; i < pre; ++i) activations();
   ms_wait((pre - 1) * xops);   // (the activations of the first ring follow all its weights)
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // P0: unit 0 has landed
-  int ops = 0, before = 0;   // requests of the last unit and the one before it
+  int ops[RING - 2];   // requests of the last units, the latest first (of the first ring's: those behind its weights)
+#pragma unroll
+  for (int i = 0; i < RING - 2; ++i) ops[i] = xops;
   for (int u = 0; u < total; ++u) {
-    const bool more = u + RING - 1 < total;
-    if (more) {   // into the slot of unit u - 1, free since the barrier that ended it
+    if (u + RING - 1 < total) {   // into the slot of unit u - 1, free since the barrier that ended it
       weights();
       activations();
-      before = ops;
-      ops = groups + xops + (WF == MS_W16 ? 0 : p.rows16 ? L == 3 : (groups > L) + (groups > 4 + L));
+#pragma unroll
+      for (int i = RING - 3; i > 0; --i) ops[i] = ops[i - 1];
+      ops[0] = groups + xops + (WF == MS_W16 ? 0 : p.rows16 ? L == 3 : (groups > L) + (groups > 4 + L));
     }
-    // unit u + 1 has landed before the consumers are released into it: behind it are the last RING - 2
-    if constexpr (RING == 3) ms_wait(more ? ops : 0);
-    else ms_wait(more ? ops + (u > 0 ? before : 0) : u + 3 == total && u > 0 ? ops : 0);
+    // unit u + 1 has landed before the consumers are released into it: behind it are the units that follow it, at most RING - 2
+    int later = 0;
+#pragma unroll
+    for (int i = 0; i < RING - 2; ++i) later += i < total - 2 - u ? ops[i] : 0;
+    ms_wait(later);
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // B_u
   }
 }
@@ -352,14 +360,16 @@ __global__ __launch_bounds__((MsLds<WF, MT>::THREADS)) __attribute__((amdgpu_wav
     own = lo < hi ? ms_over(hi - 1, p.per_block) - i0 + 1 : 0;
   }
   MsWalk run{i0, lo - i0 * rgs, hi - lo};
-  const bool small = run.left <= 4;
-  const int slot_bytes = small ? LD::slot(4) : LD::slot(8), w_bytes = slot_bytes - LD::X_BYTES - LD::S_BYTES, ring = small ? 4 : 3;
+  const int widest = run.left <= 2 ? 2 : run.left <= 4 ? 4 : 8;   // (row groups of a tile: narrow ones in a ring of more units)
+  const int slot_bytes = widest == 2 ? LD::slot(2) : widest == 4 ? LD::slot(4) : LD::slot(8), w_bytes = slot_bytes - LD::X_BYTES - LD::S_BYTES;
+  const int ring = widest == 2 ? LD::ring(2) : widest == 4 ? LD::ring(4) : LD::ring(8);
   if (wv >= 8) {
     if (lo >= hi) return;   // (as a whole: the consumers behind their zeros)
     __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0), for the compiler: it would wait for the lists' registers between the requests
     const int head = rgs - run.r0 < run.left ? rgs - run.r0 : run.left, tail = run.left - head - (own - 2) * rgs;
     const int total = units * ((head + 7) / 8 + (own > 1 ? (own - 2) * ((rgs + 7) / 8) + (tail + 7) / 8 : 0));
-    if (small) ms_load<WF, MT, MODE, 4>(p, lds, wv - 8, lane, run, rgs, i0, units, total);
+    if (widest == 2) ms_load<WF, MT, MODE, 2>(p, lds, wv - 8, lane, run, rgs, i0, units, total);
+    else if (widest == 4) ms_load<WF, MT, MODE, 4>(p, lds, wv - 8, lane, run, rgs, i0, units, total);
     else ms_load<WF, MT, MODE, 8>(p, lds, wv - 8, lane, run, rgs, i0, units, total);
     return;
   }

@@ -147,3 +147,35 @@ def test_runs_of_row_groups(experts, groups):
     want = torch.stack([down[e].double() @ act[t] for t, e in enumerate(ids[:, 0].tolist())])
     # the activations' rounding, met by weights of deviation ff^-1/2 (6 deviations), and the result's own
     assert ((got - want).abs() <= 2.0 ** -8 * (want.abs() + 6 * act.norm(dim=1, keepdim=True) * ff ** -0.5)).all()
+
+
+@pytest.mark.parametrize("units", [1, 2, 4, 5, 6, 7, 24])
+@pytest.mark.parametrize("groups", [1, 2])
+@pytest.mark.parametrize("tokens", [1, 3])
+def test_narrow_runs_of_any_length(units, groups, tokens):
+    """Runs of one and two row groups, whose units stand in a ring of six: contractions shorter than it, as long, longer; rows in one piece and in two."""
+    from lite_llama_amd.kernels.fused_moe import sparse_square_experts
+
+    cus, experts = torch.cuda.get_device_properties(0).multi_processor_count, 16
+    width, ff = 128 * units - 8, 16 * (cus * groups // experts)
+    g = torch.Generator(device=DEV).manual_seed(units + groups)
+    up, down = ((torch.randn(experts, *s, generator=g, device=DEV) * s[1] ** -0.5).bfloat16() for s in ((ff, width), (width, ff)))
+    h = torch.randn(tokens, width, generator=g, device=DEV).bfloat16()
+    ids = torch.stack([torch.randperm(experts, generator=g, device=DEV) for _ in range(tokens)]).to(torch.int32)
+    weights = torch.rand(tokens, experts, generator=g, device=DEV) + 0.1
+    got = sparse_square_experts(h, up, down, ids, weights).double()
+    for t in range(tokens):
+        for k, e in enumerate(ids[t].tolist()):
+            act = torch.relu(up[e].double() @ h[t].double() * weights[t, k].double()) ** 2
+            want = down[e].double() @ act
+            # the activations' rounding, met by weights of deviation ff^-1/2 (6 deviations), and the result's own
+            assert ((got[t, k] - want).abs() <= 2.0 ** -8 * (want.abs() + 6 * act.norm() * ff ** -0.5)).all()
+
+
+@pytest.mark.parametrize("fmt", ["fp8", "int8"])
+@pytest.mark.parametrize("width", [256, 768, 1280, 1536, 3072])
+@pytest.mark.parametrize("tokens,group", [(1, 128), (2, 4096), (24, 128)])
+@pytest.mark.parametrize("interleaved", [False, True])
+def test_narrow_runs_of_8_bit_experts(fmt, width, tokens, group, interleaved):
+    """The same in 8 bits, scales per row and alike in 16 rows, rows in pieces of 16 and of 32."""
+    test_8_bit_experts(fmt, width, 256, 4 if tokens > 2 else 8, tokens, 2, group, interleaved)
