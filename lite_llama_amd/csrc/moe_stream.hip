@@ -20,8 +20,8 @@
 //     groups, two workgroups per CU for 8-bit weights, which this replaces: the second one of a CU came 10 us late, and a tile of one group
 //     took as long as one of four.  us for both products, that -> here: 8-bit floats, 128 experts of 2048 / 768, top 8: 1 token 34 -> 29.9,
 //     8 70 -> 65, 32 108 -> 102, 64 124 -> 119 (604 MB: 5.1 TB/s), 128 140 -> 136, 200 169 -> 151, 256 174 -> 155, 320 191 -> 192; bf16, 34 of
-//     2048 / 704, top 4: 1 21.2 -> 21.1, 4 42 -> 33, 32 63 -> 59, 128 68 -> 62, 262 81 -> 67; 68 of 3072 / 512, top 8: 1 27.8 -> 28.0 (24 units
-//     of two groups in a row: latency; tiles of up to two groups have a ring of six, with one of four 29.1), 6 69 -> 67, 32 119 -> 114, 128 133 -> 124, 262 159 -> 135.
+//     2048 / 704, top 4: 1 21.2 -> 21.1, 4 42 -> 33, 32 63 -> 59, 128 68 -> 62, 262 81 -> 67; 68 of 3072 / 512, top 8: 1 27.8 -> 29.1 (24 units
+//     of two groups in a row: latency), 1 less since tiles of up to two groups have a ring of six instead of four, 6 69 -> 67, 32 119 -> 114, 128 133 -> 124, 262 159 -> 135.
 //   Lines against the tiles (before that change; us, tiles -> streams): 8-bit floats, 128 of 2048 / 768: 1 token 42 -> 24, 64 137 -> 117, 320 181 ->
 //   168, 400 186 -> 191; bf16, 34 of 2048 / 704, top 4: 1 token 33 -> 17, 128 78 -> 65, 300 (35 rows per expert) 78.5 -> 77, 400 (47) 80 -> 85; 68 of
 //   3072 / 512: 262 (31) 165 -> 150: up to 36 rows per expert in ll_moe_rows_gemm.  ll_moe_gemm has other tiles and lines of its own (moe.hip).

@@ -78,3 +78,36 @@ def test_row_group_runs(n, k, m, swiglu):
         qa, a = quantize_activations_int8(x)
         sums = qa.float() @ codes.float().T                 # (whole numbers below 2^24: exact)
         assert torch.equal(smoothquant_rows_matmul(x, codes, scale), ((sums * a.view(-1, 1)) * scale.view(1, -1)).half())
+
+
+# 64 to 256 MB: workgroups begin in other steps than above; six and seven row groups per CU (tiles of up to four, of up to eight for more than 32 rows), one and two
+MIDDLE = [(49152 + 32, 2048), (8192 + 32, 8192), (14336, 4096)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n,k", MIDDLE)
+def test_staggered_rows_of_streams_of_middle_length(dtype, n, k):
+    from lite_llama_amd.kernels.quantization import dense16_rows_linear
+
+    g = torch.Generator(device=DEV).manual_seed(n + k)
+    w = (torch.randn(n, k, generator=g, device=DEV) * k ** -0.5).to(dtype)
+    x = torch.randn(64, k, generator=g, device=DEV).to(dtype)
+    every, want = dense16_rows_linear(x, w), x.float() @ w.float().T
+    unit = 2.0 ** (-11 if dtype == torch.float16 else -8)   # as above
+    assert ((every.float() - want).abs() <= unit * want.abs() + 2.0 ** -14).all()
+    for m in (1, 32, 33):
+        assert torch.equal(dense16_rows_linear(x[:m], w), every[:m])
+
+
+@pytest.mark.parametrize("m", [30, 33, 64])
+@pytest.mark.parametrize("n,k", [(40960 + 32, 4096), (16384, 8192)])
+def test_staggered_int8_rows_in_all_tiles(m, n, k):
+    from lite_llama_amd.kernels.quantization import quantize_activations_int8, smoothquant_rows_matmul
+
+    g = torch.Generator(device=DEV).manual_seed(n + m)
+    w = torch.randint(-127, 128, (n, k), generator=g, device=DEV, dtype=torch.int8)
+    scale = torch.rand(n, generator=g, device=DEV) * 1e-3
+    x = torch.randn(m, k, generator=g, device=DEV).half()
+    qa, each = quantize_activations_int8(x)
+    sums = torch.cat([qa.double() @ part.double().T for part in w.split(8192)], dim=1).float()   # (whole numbers: one value, whatever the order)
+    assert torch.equal(smoothquant_rows_matmul(x, w, scale), ((sums * each.view(-1, 1)) * scale.view(1, -1)).half())
