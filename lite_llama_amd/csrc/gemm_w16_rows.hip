@@ -10,14 +10,13 @@
 //     address: fragment reads are conflict free; weights non-temporal.  CONSUMERS, one per row group of the tile, run the unit's MFMA
 //     32x32x16 from LDS fragments and keep the tile's accumulators (16 x MT registers) for the whole K loop: no cross-wave exchange.
 //     The loaders run ahead ACROSS tile boundaries, so a tile's epilogue overlaps the next tile's first units.
-//   * Long streams of rows a multiple of 4 KB long: workgroup b begins every tile b steps of 256 bytes into its rows and wraps; streams under 256 MB
+//   * Long streams of rows a multiple of 4 KB long: workgroup b begins every tile b steps of 256 bytes into its rows and wraps; int8 streams under 256 MB
 //     5 b steps.  All of them beginning at column 0 ask the same few memory channels, and so do runs of a power of two rows whose steps of b keep
 //     pace with them.  us for 600 MB, 1 row, all from column 0 -> staggered: K = 2048 113 -> 94, 4096 127 -> 98, 8192 139 -> 124; staggered within
-//     an XCD instead, b / 8: 98, 106, 124; K = 3584: 90 -> 91, 37888 rows of it 50 -> 52.  32 rows, column 0 / b / 5 b: 16384 x 2048 16.3 / 14.6 / 14.6,
-//     32768 x 2048 32.7 / 29.5 / 25.6, 49152 x 2048 45 / 36 / 36, 14336 x 4096 25.6 / 30.9 / 24.5, 16384 x 4096 29.6 / 36.6 / 26.2, 28672 x 4096
-//     50 / 42 / 43, 8192 x 8192 37 / 32 / 28, int8 28672 x 4096 - / 23.8 / 23.1, 16384 x 8192 - / 36.3 / 25.7; 7 b: 28672 x 4096 47; 11 b: 16384 x
-//     4096 29.4; b's bits reversed: 32000 x 4096 57 (b 46).  From 256 MB on b and 5 b are within 2 % of each other, either way.  Sums of 16-bit products
-//     in another order round otherwise, so streams under 64 MB, which gain less (8192 x 2048 10.7 -> 9.9), keep the ascending one; int8 sums are exact.
+//     an XCD instead, b / 8: 98, 106, 124; K = 3584: 90 -> 91, 37888 rows of it 50 -> 52.  b / 5 b steps: int8 28672 x 4096 23.8 / 23.1, 16384 x 8192 36.3 /
+//     25.7; from 256 MB on b and 5 b are within 2 % of each other, either way.  Sums of 16-bit products in another order round otherwise, which travels
+//     through all that follows, so 16-bit streams under 256 MB keep the ascending one (in 5 b steps 32 rows of 32768 x 2048 take 25.6 instead of 32.7, 14336 x 4096
+//     24.5 instead of 25.6, 28672 x 4096 43 instead of 50); int8 sums are exact, and staggered from 64 MB.
 //   * one s_barrier per unit.  Of every row group each loader requests a quarter, and nothing is requested that no one reads: neither groups that a
 //     tile lacks nor activations behind the last row; the waits count what was.  (Loaders of one group each, which pointed the requests of
 //     groups that were not there at one cached KB so that the count stayed the same, took as long for a tile of one group as for four.  us,
@@ -323,7 +322,7 @@ extern "C" int ll_dense16_rows_matmul(void* out, const void* x, const void* w, c
   R16Params p{};
   p.out = (uint16_t*)out; p.x = (const uint16_t*)x; p.w = (const uint16_t*)w; p.bias = (const uint16_t*)bias;
   p.m = m; p.n = n; p.k = k; p.x_stride = x_stride_m; p.w_stride = w_stride_n;
-  p.stagger = w_stride_n % 2048 || n * k * 2 < (1ll << 26) ? 0 : n * k * 2 < (1ll << 28) ? 5 : 1;
+  p.stagger = w_stride_n % 2048 == 0 && n * k * 2 >= (1ll << 28);
   p.epi = epilogue;
   const int64_t rgs = n / 32;
   int grid = r16_num_cus();

@@ -80,13 +80,14 @@ def test_row_group_runs(n, k, m, swiglu):
         assert torch.equal(smoothquant_rows_matmul(x, codes, scale), ((sums * a.view(-1, 1)) * scale.view(1, -1)).half())
 
 
-# 64 to 256 MB: workgroups begin in other steps than above; six and seven row groups per CU (tiles of up to four, of up to eight for more than 32 rows), one and two
+# 64 to 256 MB: six and seven row groups per CU (tiles of up to four, of up to eight for more than 32 rows), one and two
 MIDDLE = [(49152 + 32, 2048), (8192 + 32, 8192), (14336, 4096)]
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("n,k", MIDDLE)
-def test_staggered_rows_of_streams_of_middle_length(dtype, n, k):
+def test_sums_of_streams_of_middle_length(dtype, n, k):
+    """In the order of columns, as those of short streams: 32 MB of the same weights give the same bits."""
     from lite_llama_amd.kernels.quantization import dense16_rows_linear
 
     g = torch.Generator(device=DEV).manual_seed(n + k)
@@ -97,6 +98,8 @@ def test_staggered_rows_of_streams_of_middle_length(dtype, n, k):
     assert ((every.float() - want).abs() <= unit * want.abs() + 2.0 ** -14).all()
     for m in (1, 32, 33):
         assert torch.equal(dense16_rows_linear(x[:m], w), every[:m])
+    part = (1 << 24) // k
+    assert torch.equal(dense16_rows_linear(x, w[:part]), every[:, :part])
 
 
 @pytest.mark.parametrize("m", [30, 33, 64])
