@@ -264,6 +264,12 @@ static SDPlan sd_plan(int64_t m, int64_t n, int64_t k, int wfmt, int max_splits)
   static const int force_s = getenv("LL_DENSE_SS_S") ? atoi(getenv("LL_DENSE_SS_S")) : 0;
   const bool w16 = wfmt == 4 || wfmt == 5;
   if (off || (wfmt != 1 && wfmt != 2 && !w16) || m < 1 || m > 64 || n < 32 || n % 32 != 0 || k < 64 || k % 64 != 0) return best;
+  // Measured (benchmarks/gemm_short_dense.py, same box, us per launch short-stream / streaming engine):
+  // fp8 2048 x 4096 7.4 / 11.2, int8 4096 x 1024 5.4 / 6.6 -- but fp8 5120 x 2048 (10.5 MB) 10.6 / 10.1 under every plan, and
+  // the 16-bit formats 7.2 - 8.1 / 6.0 - 6.5: a lane's 32 - 64 contiguous bytes per row make every load instruction touch 32+ cache
+  // lines (the int4 engine's pre-packed pieces are 1 KB contiguous).  Default: 8-bit weights of at most 9 MB; LL_DENSE_SS=2 lifts it.
+  static const bool all = getenv("LL_DENSE_SS") != nullptr && atoi(getenv("LL_DENSE_SS")) == 2;
+  if (!all && (w16 || n * k > 9000000)) return best;   // (in front of the loops: a call asks several times)
   if (n * k * (w16 ? 2 : 1) >= (1ll << 31) || (int64_t)(m - 1) * k * 2 + k * 2 >= (1ll << 31)) return best;  // 32-bit offsets
   const int cus = sd_num_cus();
   const int rgs = (int)(n / 32), kbs = (int)(k / 64);
@@ -303,12 +309,6 @@ static SDPlan sd_plan(int64_t m, int64_t n, int64_t k, int wfmt, int max_splits)
   }
   // a launch that would leave more than a third of the CUs idle stays on the streaming engine
   if (best.ok && best.total * 3 < cus * 2) best.ok = 0;
-  // Measured (benchmarks/gemm_short_dense.py, same box, us per launch short-stream / streaming engine):
-  // fp8 2048 x 4096 7.4 / 11.2, int8 4096 x 1024 5.4 / 6.6 -- but fp8 5120 x 2048 (10.5 MB) 10.6 / 10.1 under every plan, and
-  // the 16-bit formats 7.2 - 8.1 / 6.0 - 6.5: a lane's 32 - 64 contiguous bytes per row make every load instruction touch 32+ cache
-  // lines (the int4 engine's pre-packed pieces are 1 KB contiguous).  Default: 8-bit weights of at most 9 MB; LL_DENSE_SS=2 lifts it.
-  static const bool all = getenv("LL_DENSE_SS") != nullptr && atoi(getenv("LL_DENSE_SS")) == 2;
-  if (best.ok && !all && (w16 || n * k > 9000000)) best.ok = 0;
   return best;
 }
 
