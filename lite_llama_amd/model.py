@@ -185,7 +185,9 @@ class RotaryEmbedding(nn.Module):
             # decode: hand out the position-indexed tables themselves; the fused rope kernel reads row
             # positions[i] (callers guarantee positions < the size given to ``ensure``)
             return RopeTables(c[0], c[1], position_ids.reshape(-1))
-        rows = rotary_rows(position_ids, self.inv_freq, x.dtype)   # (the same values)
+        rows = None
+        if type(self)._tables is RotaryEmbedding._tables and "_tables" not in self.__dict__:   # (angles of another kind come from their own tables)
+            rows = rotary_rows(position_ids, self.inv_freq, x.dtype)   # (the same values)
         return rows if rows is not None else self._tables(position_ids, x.dtype)
 
 

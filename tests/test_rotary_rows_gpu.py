@@ -26,6 +26,22 @@ def test_rows_are_those_of_the_tensor_operations(dtype, index, batch, seq, half)
     assert rotary_rows(pos, rope.inv_freq.double(), dtype) is None and rotary_rows(pos.cpu(), rope.inv_freq, dtype) is None
 
 
+def test_tables_of_another_kind_are_asked():
+    class Scaled(RotaryEmbedding):
+        def _tables(self, pos, dtype):
+            cos, sin = super()._tables(pos, torch.float32)
+            return (1.5 * cos).to(dtype), (1.5 * sin).to(dtype)
+
+    geo = tiny_geometry(head_dim=64)
+    plain, scaled, patched = RotaryEmbedding(geo).to(DEV), Scaled(geo).to(DEV), RotaryEmbedding(geo).to(DEV)
+    patched._tables = scaled._tables
+    x, pos = torch.zeros(1, device=DEV, dtype=torch.float16), torch.arange(37, device=DEV)[None]
+    for rope in (scaled, patched):
+        for got, want in zip(rope(x, pos), scaled._tables(pos, torch.float16)):
+            assert torch.equal(got, want)
+    assert torch.equal(plain(x, pos)[0], plain._tables(pos, torch.float16)[0]) and not torch.equal(plain(x, pos)[0], scaled(x, pos)[0])
+
+
 def _prompt(seq, **kw):
     """A model and a prompt of ``seq`` tokens: what its ``forward`` takes."""
     geo = tiny_geometry(hidden_size=128, intermediate_size=256, num_layers=2, num_heads=4, num_kv_heads=2, head_dim=32, vocab_size=64, **kw)
