@@ -70,6 +70,9 @@ class PartialSums:
         return out
 
 
+_TABLES = (torch.Tensor, torch.nn.Parameter)   # (a table of another class may be more than what it points at)
+
+
 class EmbeddedRows:
     """Rows ``ids`` of an embedding table that are not looked up yet: the first norm of a step reads them from the table and leaves
     them as the residual (:func:`embed_rmsnorm`)."""
@@ -83,7 +86,7 @@ class EmbeddedRows:
 
     @staticmethod
     def served(ids: torch.Tensor, table: torch.Tensor) -> bool:
-        return (type(ids) is torch.Tensor and ids.is_cuda and ids.dtype == torch.int64 and ids.is_contiguous() and table.device == ids.device
+        return (type(ids) is torch.Tensor and type(table) in _TABLES and ids.is_cuda and ids.dtype == torch.int64 and ids.is_contiguous() and table.device == ids.device
                 and table.dtype in (torch.float16, torch.bfloat16) and table.dim() == 2 and table.is_contiguous() and table.shape[0] > 0
                 and table.shape[1] % 8 == 0 and 0 < table.shape[1] <= 8192 and table.data_ptr() % 16 == 0 and L.has("ll_embed_rmsnorm_q8"))
 
@@ -559,7 +562,7 @@ def residual_set(y: torch.Tensor, bias: torch.Tensor | None = None, out: torch.T
 def embedding(ids: torch.Tensor, table: torch.Tensor):
     """``F.embedding(ids, table)``; an id that the table does not have is answered with NaN, as :func:`embed_rmsnorm` does.  ``None`` where the
     call is not served."""
-    if (type(ids) is not torch.Tensor or not ids.is_cuda or ids.dtype not in (torch.int32, torch.int64) or table.device != ids.device
+    if (type(ids) is not torch.Tensor or type(table) not in _TABLES or not ids.is_cuda or ids.dtype not in (torch.int32, torch.int64) or table.device != ids.device
             or table.dtype not in (torch.float16, torch.bfloat16) or table.dim() != 2 or not table.is_contiguous() or table.shape[0] < 1
             or not 0 < table.shape[1] <= 1 << 20 or not L.has("ll_embed_rows")):
         return None
@@ -583,7 +586,7 @@ class FirstRows:
 def embed_rows(ids: torch.Tensor, table: torch.Tensor):
     """``(x, FirstRows)``: embedding rows as the fp32 residual and as they are, in one launch -- ``residual_set(F.embedding(ids, table))`` and
     the cast of it back.  ``None`` where the call is not served."""
-    if (ids.dtype not in (torch.int32, torch.int64) or ids.dim() != 1 or not ids.is_contiguous() or not ids.is_cuda or table.device != ids.device
+    if (type(table) not in _TABLES or ids.dtype not in (torch.int32, torch.int64) or ids.dim() != 1 or not ids.is_contiguous() or not ids.is_cuda or table.device != ids.device
             or table.dtype not in (torch.float16, torch.bfloat16) or not table.is_contiguous() or not L.has("ll_embed_rows")):
         return None
     n, width = ids.numel(), table.shape[1]

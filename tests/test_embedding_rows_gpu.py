@@ -52,3 +52,26 @@ def test_an_id_outside_the_table_is_nan_on_every_route(index, shape):
             continue
         assert rows.shape == (*shape, 64)
         assert rows.view(-1, 64)[0].isnan().all() and torch.equal(rows.view(-1, 64)[1:], model.embed_tokens.weight[ids.view(-1)[1:].long()])
+
+
+class Halved(torch.Tensor):
+    """A table that means half of what it holds."""
+
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        out = super().__torch_function__(func, types, args, kwargs or {})
+        return out.as_subclass(torch.Tensor) * 0.5 if func is F.embedding else out
+
+
+def test_a_table_of_another_class_answers_for_itself():
+    from lite_llama_amd.model import CausalLM, tiny_geometry
+
+    with torch.device(DEV):
+        model = CausalLM(tiny_geometry(hidden_size=64, intermediate_size=128, num_layers=1, num_heads=4, num_kv_heads=2, head_dim=16, vocab_size=32))
+    plain = model.embed_tokens.weight.detach().clone().normal_()
+    table = plain.as_subclass(Halved)
+    model.embed_tokens._parameters["weight"] = table
+    for shape in ((3, 1), (2, 5), (1, 200)):
+        ids = torch.randint(0, 32, shape, device=DEV)
+        assert embedding(ids, table) is None and embed_rows(ids.view(-1), table) is None and not EmbeddedRows.served(ids, table)
+        assert torch.equal(model._embed(ids), plain[ids] * 0.5)
