@@ -6,7 +6,7 @@
 // activation in its epilogue, down as partials.  (The eager route asks the library for q|k|v and o; here they stay on the narrow kernel or
 // the row-group loop and on the split-K engine: 5 - 9 us each against 8, without 24 us of the library's host side.)
 // These engines take 64 rows: more go through them in parts of equal size, whose weights the Infinity Cache
-// holds between them, if the layer's are no more than 100 MB.  us, eager -> here: 12 layers of 896 / 4864, 37 tokens 2290 -> 790 (534 since: fewer checks, the rotation in the attention's launch), 100 2850 -> 1090, 200
+// holds between them, if the layer's are no more than 100 MB.  us, eager -> here: 12 layers of 896 / 4864, 37 tokens 2290 -> 790 (519 since: fewer checks, the rotation in the attention's launch, plans told apart early), 100 2850 -> 1090, 200
 // (four parts) 2790 -> 1530; 4 layers of 1536 / 8960 (94 MB each), 64 tokens 850 -> 374, 100 1020 -> 616, 180 1034 -> 858, 256 1025 -> 1096.
 #include "common.h"
 
