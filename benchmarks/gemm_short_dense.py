@@ -1,5 +1,5 @@
-"""Short-stream engine for the row-major weight formats (csrc/gemm_short_dense.hip) against the streaming split-K engine
-(gemm_w8_skinny.hip): split-K partial launches at the dense projection shapes of Qwen3-30B-A3B (fp8 128 x 128 blocks), of a 1.5B
+"""Short-stream engine for the row-major weight formats (csrc/gemm_short_dense.hip) against the streaming split-K engines
+(gemm_split.hip, gemm_w8_skinny.hip): split-K partial launches at the dense projection shapes of Qwen3-30B-A3B (fp8 128 x 128 blocks), of a 1.5B
 bf16 model and of TP shards.  us per launch (hipGraph replays over ~600 MB of rotating weights), planes, max error vs fp32.
 The engine is chosen once per process: run once as is and once with LL_DENSE_SS=0.  One JSON line.
 
