@@ -79,13 +79,18 @@ __global__ __launch_bounds__(1024 / MF) __attribute__((amdgpu_waves_per_eu(4 / M
   // ---- loader roles ----
   // activations: 32 pieces of 8 rows x 128 B, eight per wave; lane -> (row, physical slot), the swizzle in the SOURCE address
   uint32_t xoff[XP];
-  // GROUPED: row r of row block m is the slot sorted_ids[m + r] (num_slots: none), its input row slot / top_k; the slots of the tile that is
-  // requested next are fetched a tile ahead
-  int slot1[GROUPED ? XP : 1];
-  auto fetch_slots = [&](int m) {
+  // GROUPED: row r of row block m is the slot sorted_ids[m + r] (num_slots: none), its input row slot / top_k.  A tile's slots stand in LDS
+  // behind the operands, requested a tile ahead into a ring of three (a wave may still read those of the tile in front of the one another wave
+  // has begun): in registers they were spilled, and read from memory where they are used they waited for the stores of the tile before.  us of
+  // fused_moe with both products, in registers -> here (with the fragments' addresses formed in the loop and fewer operations per widened fp8
+  // weight): fp8, 128 experts of 2048 / 768, top 8, 3000 tokens 497 -> 485, 4096 683 -> 653, 8192 1151 -> 1104; 8 of 4096 / 14336, top 2, 600 tokens
+  // 878 -> 825, 4096 3478 -> 3324.  What is left per tile of 12 steps (cycles): 12 500 of epilogue, 9000 until its stores are out, 34 000 of steps.
+  constexpr int ST = 4 * OPND;
+  const int* slots = reinterpret_cast<const int*>(lds + ST);
+  int turn = 0, turn1 = 0;  // where the slots of the tile that is multiplied begin, and those of the tile after it
+  auto fetch_slots = [&](int m, int into) {
     if constexpr (GROUPED) {
-#pragma unroll
-      for (int j = 0; j < XP; ++j) slot1[j] = p.sorted_ids[m + (wv * XP + j) * 8 + (lane >> 3)];
+      if (wv < 4) v3_dma4<false>((uint32_t)(ST + (into + wv * 64) * 4), p.sorted_ids + m, (uint32_t)(wv * 256 + lane * 4));
     }
   };
   auto aim_x = [&](int m) {
@@ -93,7 +98,8 @@ __global__ __launch_bounds__(1024 / MF) __attribute__((amdgpu_waves_per_eu(4 / M
     for (int j = 0; j < XP; ++j) {
       const int r = (wv * XP + j) * 8 + (lane >> 3);
       if constexpr (GROUPED) {
-        const uint32_t row = slot1[j] < p.num_slots ? (uint32_t)slot1[j] / (uint32_t)p.top_k : 0;  // (no slot: feeds only unstored outputs)
+        const int slot = slots[turn1 + r];
+        const uint32_t row = (uint32_t)(slot < p.num_slots ? slot : p.num_slots - 1) / (uint32_t)p.top_k;  // (no slot: feeds only unstored outputs)
         xoff[j] = row * (uint32_t)p.x_stride + swz(r, lane & 7) * 16;
         continue;
       }
@@ -108,7 +114,7 @@ __global__ __launch_bounds__(1024 / MF) __attribute__((amdgpu_waves_per_eu(4 / M
   const char* sbase = WF == 0 ? (const char*)p.sp : (const char*)p.scales;
   auto aim_w = [&](int m, int n) {
     if constexpr (GROUPED) {
-      const int64_t expert = __builtin_amdgcn_readfirstlane(p.expert_ids[m >> 8]);
+      const int64_t expert = ((const __attribute__((address_space(4))) int32_t*)p.expert_ids)[m >> 8];  // (a scalar load)
       wbase = p.w + expert * p.w_stride_e;
       sbase = (const char*)p.scales + expert * p.s_stride_e * 4;
     }
@@ -226,19 +232,16 @@ __global__ __launch_bounds__(1024 / MF) __attribute__((amdgpu_waves_per_eu(4 / M
   // (waves v and v + 4 share a SIMD: eight waves give it two different token parts, so a grouped tile whose rows end in its first half keeps
   // every SIMD at half its products instead of two SIMDs at all of theirs)
   const int wn = wv / MP, wm = MF == 2 ? (wv + 2 * wn) % MP : wv % MP;
-  const unsigned char *xsrc[4], *wsrc[4];  // per MFMA step kk of a step: 16-byte slot kk * 2 + h (rows nl + a multiple of 32 share the swizzle)
-#pragma unroll
-  for (int kk = 0; kk < 4; ++kk) {
-    xsrc[kk] = lds + (wm * MF * 32 + nl) * 128 + swz(nl, kk * 2 + h) * 16;
-    wsrc[kk] = lds + WT + (wn * 128 + nl) * 128 + swz(nl, kk * 2 + h) * 16;
-  }
+  // per MFMA step kk of a step: 16-byte slot kk * 2 + h (rows nl + a multiple of 32 share the swizzle) = where slot h stands, its bits 5 and 6
+  // exchanged by kk
+  uint32_t xsrc = (wm * MF * 32 + nl) * 128 + swz(nl, h) * 16, wsrc = WT + (wn * 128 + nl) * 128 + swz(nl, h) * 16;
   i32x4 xf[2][MF], wf[2][4];
   auto read_frag = [&](auto B, int kk, int set, int i) {
     constexpr int buf = decltype(B)::value;
     // in the order in which the MFMAs ask for them: the first weight fragment, the activations, the other weight fragments
     const int w = i == 0 ? 0 : i - MF, x = i - 1;
-    if (i == 0 || i > MF) wf[set][w] = *reinterpret_cast<const i32x4*>(wsrc[kk] + buf * OPND + w * 4096);
-    else xf[set][x] = *reinterpret_cast<const i32x4*>(xsrc[kk] + buf * OPND + x * 4096);
+    if (i == 0 || i > MF) wf[set][w] = *reinterpret_cast<const i32x4*>(lds + (wsrc ^ (kk * 32)) + buf * OPND + w * 4096);
+    else xf[set][x] = *reinterpret_cast<const i32x4*>(lds + (xsrc ^ (kk * 32)) + buf * OPND + x * 4096);
   };
   using Acc = typename std::conditional<I8A, i32x16, f32x16>::type;
   Acc acc[4][MF];
@@ -253,7 +256,11 @@ __global__ __launch_bounds__(1024 / MF) __attribute__((amdgpu_waves_per_eu(4 / M
   constexpr integral_constant<int, 0> Q0{};
   constexpr integral_constant<int, 1> Q1{};
   WRegs rA, rB;  // weights of odd / even steps ahead
-  fetch_slots(m0);
+  if constexpr (GROUPED) {
+    fetch_slots(m0, 0);
+    __builtin_amdgcn_s_waitcnt(0x0070);
+    __builtin_amdgcn_s_barrier();
+  }
   aim_x(m0);
   aim_w(m0, n0);
   m1 = m0;
@@ -279,6 +286,9 @@ __global__ __launch_bounds__(1024 / MF) __attribute__((amdgpu_waves_per_eu(4 / M
   if constexpr (ND > 0) { _Pragma("unroll") for (int e = 0; e < ND; ++e) issue(buf, from + (g & 3) * ND + e); }      \
   else if (g % 2 == 0) issue(buf, from + (g & 3) / 2);
 #define T2_STEP(R, cur, nxt, MULS)                                                                           \
+  /* (GROUPED: the addresses of kk 1 .. 3 are formed where they are used; kept over the loop they were spilled, and every reload waited for \
+     all that was requested before it) */                                                                \
+  if constexpr (GROUPED) asm volatile("" : "+v"(xsrc), "+v"(wsrc));                                      \
   _Pragma("unroll") for (int g = 0; g < 16; ++g) {                                                       \
     const int q = g >> 2, set = q & 1, i0 = (g & 3) * MF;                                                \
     if (g == 12) {                                                                                       \
@@ -312,12 +322,8 @@ __global__ __launch_bounds__(1024 / MF) __attribute__((amdgpu_waves_per_eu(4 / M
   for (;;) {
   const bool more = !SPLIT && t + stride < tend;
   if (more) tile_of(t + stride, m1, n1);  // (else: the same tile's first steps once more, never multiplied)
-  fetch_slots(m1);
-  int slot0[GROUPED ? MF : 1];
-  if constexpr (GROUPED) {
-#pragma unroll
-    for (int mi = 0; mi < MF; ++mi) slot0[mi] = p.sorted_ids[m0 + (wm * MF + mi) * 32 + nl];
-  }
+  turn1 = turn == 512 ? 0 : turn + 256;
+  fetch_slots(m1, turn1);
 #pragma unroll
   for (int ni = 0; ni < 4; ++ni)
 #pragma unroll
@@ -326,7 +332,7 @@ __global__ __launch_bounds__(1024 / MF) __attribute__((amdgpu_waves_per_eu(4 / M
       for (int e = 0; e < 16; ++e) acc[ni][mi][e] = 0;
   int left = ksteps;
   // (an even number of steps: one exit, or the accumulators' registers do not line up)
-  if (!GROUPED || __builtin_amdgcn_readfirstlane(slot0[0]) < p.num_slots) {
+  if (!GROUPED || __builtin_amdgcn_readfirstlane(slots[turn + wm * MF * 32]) < p.num_slots) {
     do {
       T2_STEP(rA, Q0, Q1, true)
       T2_STEP(rB, Q1, Q0, true)
@@ -368,7 +374,7 @@ __global__ __launch_bounds__(1024 / MF) __attribute__((amdgpu_waves_per_eu(4 / M
     a = r[0];
     b = r[1];
   };
-  const bool has_bias = p.bias != nullptr;
+  const bool has_bias = !GROUPED && p.bias != nullptr;
   float as[MF];
   f32x4 ws[I8A ? 4 : 1][4];
   uint2 bb[4][4];
@@ -393,7 +399,10 @@ __global__ __launch_bounds__(1024 / MF) __attribute__((amdgpu_waves_per_eu(4 / M
     __builtin_amdgcn_s_waitcnt(0x0f70);
   }
   float rw[GROUPED ? MF : 1];
+  int slot0[GROUPED ? MF : 1];
   if constexpr (GROUPED) {
+#pragma unroll
+    for (int mi = 0; mi < MF; ++mi) slot0[mi] = slots[turn + (wm * MF + mi) * 32 + nl];
 #pragma unroll
     for (int mi = 0; mi < MF; ++mi) rw[mi] = p.topk_w ? f16_bits_to_f32(p.topk_w[slot0[mi] < p.num_slots ? slot0[mi] : 0]) : 1.f;
   }
@@ -477,6 +486,7 @@ __global__ __launch_bounds__(1024 / MF) __attribute__((amdgpu_waves_per_eu(4 / M
   t += stride;
   m0 = m1;
   n0 = n1;
+  turn = turn1;
   }
 #undef T2_STEP
 #undef T2_DMA
@@ -638,7 +648,7 @@ int tile256_wants(int64_t m, int64_t n, int64_t k, int wf, bool split) {
 
 template <int WF, int MF, bool GROUPED, bool SPLIT>
 static int t2_go(const T2Params& p, unsigned grid, hipStream_t st) {
-  constexpr int bytes = 4 * 256 * 128;
+  constexpr int bytes = 4 * 256 * 128 + (GROUPED ? 3 * 256 * 4 : 0);
   static bool attr[16] = {false};
   int dev = 0;
   (void)hipGetDevice(&dev);

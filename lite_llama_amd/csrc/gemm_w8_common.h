@@ -21,12 +21,11 @@ __device__ __forceinline__ void d8_i8(uint32_t w, uint32_t s, uint32_t& o0, uint
 }
 // 4 fp8 e4m3 bytes -> 2 x (2 fp16) * (s * 256): the reference's bit surgery (w8a16.py:48-62)
 __device__ __forceinline__ void d8_fp8(uint32_t w, uint32_t s256, uint32_t& o0, uint32_t& o1) {
-  uint32_t p0 = __builtin_amdgcn_perm(0u, w, 0x010C000Cu);
-  uint32_t p1 = __builtin_amdgcn_perm(0u, w, 0x030C020Cu);
-  p0 = (p0 & 0x80008000u) | ((p0 >> 1) & 0x3F803F80u);
-  p1 = (p1 & 0x80008000u) | ((p1 >> 1) & 0x3F803F80u);
-  o0 = d8_mul(p0, s256);
-  o1 = d8_mul(p1, s256);
+  // a byte in the upper half of each 16 bits, shifted by one behind its sign (the copy of the sign is masked out)
+  const s16x2 p0 = __builtin_bit_cast(s16x2, __builtin_amdgcn_perm(0u, w, 0x010C000Cu)) >> 1;
+  const s16x2 p1 = __builtin_bit_cast(s16x2, __builtin_amdgcn_perm(0u, w, 0x030C020Cu)) >> 1;
+  o0 = d8_mul(__builtin_bit_cast(uint32_t, p0) & 0xBF80BF80u, s256);
+  o1 = d8_mul(__builtin_bit_cast(uint32_t, p1) & 0xBF80BF80u, s256);
 }
 
 // slices of a split-K projection over chunks of 128 bytes of every weight row (gemm_w8_skinny.hip, gemm_split.hip: the order of a sum)
