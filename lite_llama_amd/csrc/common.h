@@ -62,6 +62,13 @@ __device__ __forceinline__ uint16_t mul_storage(uint16_t a, uint16_t b) {
   return from_f32<DT>(to_f32<DT>(a) * to_f32<DT>(b));
 }
 
+// i / d for 0 <= i < most (one value for the whole launch), d > 0: a 64-bit division by a run-time value is some 100 dependent instructions, and no row
+// of few tokens needs it
+__device__ __forceinline__ int64_t ll_div(int64_t i, int d, int64_t most) {
+  if (most <= 0x7fffffff) return (int64_t)((uint32_t)i / (uint32_t)d);
+  return i / d;
+}
+
 struct alignas(16) U16x8 {
   uint16_t v[8];
 };

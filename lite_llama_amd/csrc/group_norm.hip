@@ -199,39 +199,94 @@ __device__ __forceinline__ void st4(void* p, int64_t i, f32x4 v) {
   }
 }
 
+// ... as they are stored, so that a piece can be on its way while nothing waits for it
+template <int DT>
+struct Piece4 {
+  using Bits = uint2;
+};
+template <>
+struct Piece4<LL_F32> {
+  using Bits = f32x4;
+};
+template <int DT>
+__device__ __forceinline__ typename Piece4<DT>::Bits bits4(const void* p, int64_t i) {
+  using Bits = typename Piece4<DT>::Bits;
+  if constexpr (DT == LL_F32) return *reinterpret_cast<const Bits*>((const float*)p + i);
+  else return *reinterpret_cast<const Bits*>((const uint16_t*)p + i);
+}
+template <int DT>
+__device__ __forceinline__ f32x4 val4(const typename Piece4<DT>::Bits& u) {
+  if constexpr (DT == LL_F32) return u;
+  else
+    return f32x4{to_f32<DT>((uint16_t)(u.x & 0xffff)), to_f32<DT>((uint16_t)(u.x >> 16)), to_f32<DT>((uint16_t)(u.y & 0xffff)),
+                 to_f32<DT>((uint16_t)(u.y >> 16))};
+}
+
 // Vector form of the register-cached kernel: a thread owns pieces of four consecutive channels (16-byte residual accesses,
 // 8-byte accesses of 16-bit rows).  Needs group sizes that are multiples of 4 and at most 1024 NV channels, aligned rows.
-template <int DT, int NV>
+// Everything that a group needs is requested at its start, unconditionally: the first PB rows of the result, the residual and both weights (EX: the
+// shared row, the gate and its bias, the result's bias; one that is not given is read from x_in and dropped).  A decoded token's row is bound by the
+// launch and one trip to memory; asked for where it was used it took one trip per row of the result, and one behind each of the two sums.
+// us a launch, bf16, before -> now: 32 rows of 2048 5.8 -> 5.1 (one row of result), 5.5 (four); rows of 3072 8.7 -> 5.8 (one), 6.2 (one with a shared row)
+template <int DT, int NV, int PB, bool EX>
 __global__ __launch_bounds__(256) void gated_group_norm_vec_kernel(
     const float* x_in, float* x_out, void* __restrict__ h_out, const void* __restrict__ y, int parts,
     const void* __restrict__ shared, const float* __restrict__ shared_scale, const void* __restrict__ gate, int64_t gate_ld,
     const void* __restrict__ gate_bias, const void* __restrict__ post_w, const void* __restrict__ next_w, int width, int groups,
     float eps, const void* __restrict__ y_bias) {
   constexpr bool EXACT = DT == LL_F32;
+  using Bits = typename Piece4<DT>::Bits;
   __shared__ float red[4];
   const int64_t t = blockIdx.x;
   const int tid = threadIdx.x;
   const int gs = width / groups;
   const float* xr = x_in + t * width;
   float* xo = x_out + t * width;
-  const float sscale = shared ? shared_scale[t] : 0.f;
+  const void* nwp = next_w ? next_w : post_w;
+  const float sscale = EX ? (shared ? shared_scale : x_in)[t] : 0.f;
   for (int g = 0; g < groups; ++g) {
     const int lo = g * gs, hi = lo + gs;
+    int at[NV];
+    Bits yr[NV][PB], pw[NV], nw[NV], sh[EX ? NV : 1], gt[EX ? NV : 1], gb[EX ? NV : 1], yb[EX ? NV : 1];
+    f32x4 xv[NV];
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      const int i = lo + 4 * (tid + 256 * k);
+      at[k] = i < hi ? i : lo;   // (pieces past the group: read, never used)
+#pragma unroll
+      for (int p = 0; p < PB; ++p) yr[k][p] = bits4<DT>(y, (t * parts + (p < parts ? p : parts - 1)) * (int64_t)width + at[k]);
+      if constexpr (EX) {
+        yb[k] = bits4<DT>(y_bias ? y_bias : x_in, at[k]);
+        sh[k] = bits4<DT>(shared ? shared : x_in, t * (int64_t)width + at[k]);
+        gt[k] = bits4<DT>(gate ? gate : x_in, t * (gate ? gate_ld : (int64_t)width) + at[k]);
+        gb[k] = bits4<DT>(gate_bias ? gate_bias : x_in, at[k]);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      xv[k] = *reinterpret_cast<const f32x4*>(xr + at[k]);
+      pw[k] = bits4<DT>(post_w, at[k]);
+      nw[k] = bits4<DT>(nwp, at[k]);
+    }
     f32x4 val[NV];
     float ss = 0.f;
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
-      const int i = lo + 4 * (tid + 256 * k);
       f32x4 s = {0.f, 0.f, 0.f, 0.f};
-      if (i < hi) {
-        for (int p = 0; p < parts; ++p) s += ld4<DT>(y, (t * parts + p) * (int64_t)width + i);
-        if (y_bias) s += ld4<DT>(y_bias, i);
-        if (shared) s += sscale * ld4<DT>(shared, t * (int64_t)width + i);
-        if (gate) {
-          f32x4 r = ld4<DT>(gate, t * gate_ld + i);
-          if (gate_bias) r += ld4<DT>(gate_bias, i);
+      if (lo + 4 * (tid + 256 * k) < hi) {
 #pragma unroll
-          for (int e = 0; e < 4; ++e) s[e] *= sigmoid_f<EXACT>(r[e]);
+        for (int p = 0; p < PB; ++p)
+          if (p < parts) s += val4<DT>(yr[k][p]);
+        for (int p = PB; p < parts; ++p) s += ld4<DT>(y, (t * parts + p) * (int64_t)width + at[k]);
+        if constexpr (EX) {
+          if (y_bias) s += val4<DT>(yb[k]);
+          if (shared) s += sscale * val4<DT>(sh[k]);
+          if (gate) {
+            f32x4 r = val4<DT>(gt[k]);
+            if (gate_bias) r += val4<DT>(gb[k]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[e] *= sigmoid_f<EXACT>(r[e]);
+          }
         }
       }
       val[k] = s;
@@ -243,14 +298,12 @@ __global__ __launch_bounds__(256) void gated_group_norm_vec_kernel(
     float s2 = 0.f;
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
-      const int i = lo + 4 * (tid + 256 * k);
       f32x4 v = {0.f, 0.f, 0.f, 0.f};
-      if (i < hi) {
-        const f32x4 pw = ld4<DT>(post_w, i);
-        const f32x4 xv = *reinterpret_cast<const f32x4*>(xr + i);
+      if (lo + 4 * (tid + 256 * k) < hi) {
+        const f32x4 w = val4<DT>(pw[k]);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = xv[e] + val[k][e] * inv * pw[e];
-        *reinterpret_cast<f32x4*>(xo + i) = v;
+        for (int e = 0; e < 4; ++e) v[e] = xv[k][e] + val[k][e] * inv * w[e];
+        *reinterpret_cast<f32x4*>(xo + at[k]) = v;
       }
       val[k] = v;
 #pragma unroll
@@ -261,15 +314,14 @@ __global__ __launch_bounds__(256) void gated_group_norm_vec_kernel(
       const float inv2 = 1.0f / sqrtf(s2 / (float)gs + eps);
 #pragma unroll
       for (int k = 0; k < NV; ++k) {
-        const int i = lo + 4 * (tid + 256 * k);
-        if (i < hi) {
+        if (lo + 4 * (tid + 256 * k) < hi) {
           f32x4 o = val[k];   // (no next weight: the new residual itself, cast)
           if (next_w) {
-            const f32x4 nw = ld4<DT>(next_w, i);
+            const f32x4 w = val4<DT>(nw[k]);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] = val[k][e] * inv2 * nw[e];
+            for (int e = 0; e < 4; ++e) o[e] = val[k][e] * inv2 * w[e];
           }
-          st4<DT>(h_out, t * (int64_t)width + i, o);
+          st4<DT>(h_out, t * (int64_t)width + at[k], o);
         }
       }
     }
@@ -325,7 +377,7 @@ __global__ __launch_bounds__(256) void glu_act_vec_kernel(void* __restrict__ out
   const int pieces = ff / VEC;
   const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (idx >= n * pieces) return;
-  const int64_t t = idx / pieces;
+  const int64_t t = ll_div(idx, pieces, n * pieces);
   const int j = (int)(idx - t * pieces) * VEC;
   if constexpr (DT == LL_F32) {
     const f32x4 g = *reinterpret_cast<const f32x4*>((const float*)gate + t * gate_ld + j);
@@ -385,16 +437,28 @@ extern "C" int ll_gated_group_norm(const float* x_in, float* x_out, void* h_out,
   auto ok = [&](const void* p) { return !p || (reinterpret_cast<uintptr_t>(p) % al) == 0; };
   const bool vec = y && gs % 4 == 0 && gs <= 4096 && (!gate || gate_ld % 4 == 0) && ll_aligned16(x_in) && ll_aligned16(x_out) && ok(h_out) &&
                    ok(y) && ok(shared) && ok(gate) && ok(gate_bias) && ok(post_w) && ok(next_w) && ok(y_bias);
+  const bool extra = shared || gate || y_bias;
+#define LL_GN_VEC_P(DT, NV, PB)                                                                           \
+  if (extra) gated_group_norm_vec_kernel<DT, NV, PB, true><<<grid, 256, 0, st>>>(LL_GN_ARGS);             \
+  else gated_group_norm_vec_kernel<DT, NV, PB, false><<<grid, 256, 0, st>>>(LL_GN_ARGS)
+#define LL_GN_VEC(DT, NV)                                                                                 \
+  do {                                                                                                    \
+    if (parts == 1) { LL_GN_VEC_P(DT, NV, 1); }                                                           \
+    else if (parts <= 4) { LL_GN_VEC_P(DT, NV, 4); }                                                      \
+    else { LL_GN_VEC_P(DT, NV, 8); }                                                                      \
+  } while (0)
 #define CALL(DT)                                                                                          \
-  if (vec && gs <= 1024) gated_group_norm_vec_kernel<DT, 1><<<grid, 256, 0, st>>>(LL_GN_ARGS);            \
-  else if (vec && gs <= 2048) gated_group_norm_vec_kernel<DT, 2><<<grid, 256, 0, st>>>(LL_GN_ARGS);       \
-  else if (vec) gated_group_norm_vec_kernel<DT, 4><<<grid, 256, 0, st>>>(LL_GN_ARGS);                     \
+  if (vec && gs <= 1024) LL_GN_VEC(DT, 1);                                                                \
+  else if (vec && gs <= 2048) LL_GN_VEC(DT, 2);                                                           \
+  else if (vec) LL_GN_VEC(DT, 4);                                                                         \
   else if (y && gs <= 256) gated_group_norm_cached_kernel<DT, 1><<<grid, 256, 0, st>>>(LL_GN_ARGS);       \
   else if (y && gs <= 1024) gated_group_norm_cached_kernel<DT, 4><<<grid, 256, 0, st>>>(LL_GN_ARGS);      \
   else if (y && gs <= 4096) gated_group_norm_cached_kernel<DT, 16><<<grid, 256, 0, st>>>(LL_GN_ARGS);     \
   else gated_group_norm_kernel<DT><<<grid, 256, 0, st>>>(LL_GN_ARGS)
   LL_BY_DTYPE(dtype, CALL);
 #undef CALL
+#undef LL_GN_VEC
+#undef LL_GN_VEC_P
 #undef LL_GN_ARGS
   return LL_LAUNCH_CHECK();
 }
