@@ -14,6 +14,8 @@
 //                     stacked in one matrix per expert), out = (a W_e^T) * slot weight, or act = relu((slot weight * a) W_e^T)^2 (experts
 //                     without a gate whose weight multiplies their INPUT), fp32 accumulation.  MFMA form for
 //                     16-bit storage with contraction widths that are multiples of 8, a plain tiled form otherwise.
+#include <type_traits>
+
 #include "common.h"
 #include "moe_stream.h"
 
@@ -556,8 +558,10 @@ struct alignas(16) Q4 {
 //   * Tiles are dealt to the XCDs in contiguous ranges of the tiles that exist (num_post, a device value), four blocks side by side under
 //     one weight tile: blocks of one expert read it from the XCD's own L2.
 // us for both products, 32 experts of 2048 / 704 with 384 / 706 rows each: 362 / 602 with one buffer filled through registers and two barriers
-// per step, 254 / 427 here (0.48 PFLOP/s: two operand tiles per 128 x 128 results through L2); at 70 rows each 95 us, of which the weights
-// alone need 55.
+// per step, 254 / 427 with a step's requests in front of its products (0.48 PFLOP/s: two operand tiles per 128 x 128 results through L2); at 70 rows
+// each 95 us, of which the weights alone need 55.  With the requests between the products, from 32-bit offsets, before -> now: 32 experts of 2048 / 704,
+// 1500 tokens with 4 experts each 146 -> 137, 3100 236 -> 209, 4096 280 -> 243; 64 of 3072 / 512 with 8 each, 1500 tokens 335 -> 291, 4096 627 -> 577;
+// up to 1000 tokens of either as before (the weights' stream).
 // ------------------------------------------------------------------------------------------------------------------------
 __device__ const uint32_t moe_zeros[4] __attribute__((aligned(16))) = {0, 0, 0, 0};   // what pieces behind the contraction's end read
 
@@ -568,6 +572,16 @@ __device__ __forceinline__ void dma16(uint32_t dst, const void* src) {
   asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\ts_mov_b32 m0, %0"
                : "=&s"(keep) : "s"(dst), "v"(src) : "memory");
 }
+// ... from a wave-uniform address and 32-bit offsets
+__device__ __forceinline__ void dma16(uint32_t dst, const void* base, uint32_t off) {
+  dst = __builtin_amdgcn_readfirstlane(dst);
+  const uint64_t at = (uint64_t)base;
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)at), hi = __builtin_amdgcn_readfirstlane((uint32_t)(at >> 32));   // (each back in 32 bits)
+  base = (const void*)(((uint64_t)hi << 32) | lo);
+  uint32_t keep;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep) : "s"(dst), "v"(off), "s"(base) : "memory");
+}
 template <int DT>
 __device__ __forceinline__ f32x16 mfma32(const Q4& a, const Q4& b, f32x16 c) {
   if constexpr (DT == LL_F16)
@@ -576,7 +590,7 @@ __device__ __forceinline__ f32x16 mfma32(const Q4& a, const Q4& b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
 }
 
-template <int DT, int MODE>
+template <int DT, int MODE, bool FAR>
 __global__ __launch_bounds__(256, 2) void moe_rows_gemm_tiled_kernel(const uint16_t* __restrict__ a, int64_t a_ld, int a_div,
                                                                      const uint16_t* __restrict__ w, int64_t w_stride_e, int K, int N,
                                                                      const float* __restrict__ slot_weight, uint16_t* __restrict__ out,
@@ -624,29 +638,35 @@ __global__ __launch_bounds__(256, 2) void moe_rows_gemm_tiled_kernel(const uint1
     }
     return;
   }
-  // what this thread requests of a step: row (and weight row) 8 (4 wave + j) + lane / 8, one swizzled 16-byte piece of it
-  const char* aptr[4];
-  const char* wptr[4];
-  int piece[4];
+  // what this thread requests of a step: row (and weight row) 8 (4 wave + j) + lane / 8, one swizzled 16-byte piece of it: offsets from the
+  // operand's (the expert's) first byte, in 32 bits where the host has seen that they fit
+  using Off = std::conditional_t<FAR, uint64_t, uint32_t>;
+  const char* abase = (const char*)a;
+  const char* wbase = (const char*)(w + (int64_t)e * w_stride_e);
+  Off aoff[4], woff[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    const int r = (wave * 4 + j) * 8 + (lane >> 3);
-    piece[j] = ((lane & 7) ^ ((r >> 1) & 7)) * 8;
+    const int r = (wave * 4 + j) * 8 + (lane >> 3), piece = ((lane & 7) ^ ((r >> 1) & 7)) * 16;
     const int slot = own[j];   // (rows without a slot read row 0, columns >= N the last: they feed only unstored results)
-    aptr[j] = (const char*)(a + (slot < num_slots ? (int64_t)(slot / a_div) * a_ld : 0) + piece[j]);
+    aoff[j] = (slot < num_slots ? (Off)(slot / a_div) : (Off)0) * (Off)(a_ld * 2) + piece;
     int col = GLU ? n0 + (r & 63) : n0 + r;
     col = col < N ? col : N - 1;
-    wptr[j] = (const char*)(w + (int64_t)e * w_stride_e + (GLU && r >= 64 ? (int64_t)N + col : (int64_t)col) * K + piece[j]);
+    woff[j] = (Off)(GLU && r >= 64 ? (Off)N + col : (Off)col) * ((Off)K * 2) + piece;
   }
-  auto get_a = [&](int s) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      dma16((uint32_t)((s & 1) * TILE + (wave * 4 + j) * 1024), s * 64 + piece[j] < K ? aptr[j] + (int64_t)s * 128 : (const char*)moe_zeros);
+  // request j of step s; the pieces of a last, partial step that lie behind the contraction read zeros, and so do steps behind the last one
+  const int whole = K / 64;
+  auto get = [&](uint32_t dst, const char* base, Off off, int j, int s, bool inside) {
+    if (inside || s < whole) {
+      if constexpr (FAR) dma16(dst, base + (int64_t)s * 128 + off);
+      else dma16(dst, base + (int64_t)s * 128, off);
+    } else {
+      const int r = (wave * 4 + j) * 8 + (lane >> 3), piece = ((lane & 7) ^ ((r >> 1) & 7)) * 8;
+      dma16(dst, s * 64 + piece < K ? base + (int64_t)s * 128 + off : (const char*)moe_zeros);
+    }
   };
-  auto get_w = [&](int s, int buf) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      dma16((uint32_t)((2 + buf) * TILE + (wave * 4 + j) * 1024), s * 64 + piece[j] < K ? wptr[j] + (int64_t)s * 128 : (const char*)moe_zeros);
+  auto get_a = [&](int s, int j, bool inside) { get((uint32_t)((s & 1) * TILE + (wave * 4 + j) * 1024), abase, aoff[j], j, s, inside); };
+  auto get_w = [&](int s, int j, int buf, bool inside) {
+    get((uint32_t)((2 + buf) * TILE + (wave * 4 + j) * 1024), wbase, woff[j], j, s, inside);
   };
   const bool act0 = srt[32 * wr] < num_slots, act1 = srt[32 * (wr + 2)] < num_slots;   // (an expert's empty rows stand last)
   f32x16 acc[2][2];
@@ -660,49 +680,63 @@ __global__ __launch_bounds__(256, 2) void moe_rows_gemm_tiled_kernel(const uint1
   const unsigned char* arow = tile_lds + (32 * wr + tl) * 128;
   const unsigned char* wrow0 = tile_lds + 2 * TILE + ((GLU ? 32 * wc : 64 * wc) + tl) * 128;
   const int wrow1 = (GLU ? 64 : 32) * 128;
-  get_a(0);
-  get_w(0, 0);
-  get_w(1, 1);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) get_a(0, j, false);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) get_w(0, j, 0, false);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) get_w(1, j, 1, false);
   const int steps = (K + 63) / 64;
-  int buf = 0;
-  for (int s = 0; s < steps; ++s) {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(0x0074);   // all but the last four requests (the weights of step s + 1); own fragment reads
-    __builtin_amdgcn_s_barrier();
-    get_a(s + 1);
-    get_w(s + 2, buf == 0 ? 2 : buf - 1);   // (the buffer step s - 1 has been read from)
-    const unsigned char* ap = arow + (s & 1) * TILE;
-    const unsigned char* wp = wrow0 + buf * TILE;
-    if (act0) {
-      Q4 w0[4], w1[4], a0[4];
+  // A step in four quarters of 16 columns: the fragments of the next quarter are read and two of the eight requests are issued between the products
+  // of this one (a request occupies its wave for some 80 cycles: in front of the step's fragments, as they were, eight of them kept the
+  // matrix cores waiting for longer than the products take).  MI: row tiles of this wave that hold a slot
+  auto walk = [&](auto tag) {
+    constexpr int MI = decltype(tag)::value;
+    int buf = 0;
+    auto step = [&](int s, auto inside) {   // (inside: what the step requests lies in whole steps)
+      constexpr bool IN = decltype(inside)::value;
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_waitcnt(0x0074);   // all but the last four requests (the weights of step s + 1); own fragment reads
+      __builtin_amdgcn_s_barrier();
+      const unsigned char* ap = arow + (s & 1) * TILE;
+      const unsigned char* wp = wrow0 + buf * TILE;
+      const int wbuf = buf == 0 ? 2 : buf - 1;   // (the buffer step s - 1 has been read from)
+      Q4 wf[2][2], af[2][2];
+      auto read = [&](int q) {
+        const int o = ((2 * q + h) ^ sw) * 16;
+        if constexpr (MI > 0) {
+          wf[q & 1][0] = *reinterpret_cast<const Q4*>(wp + o);
+          af[q & 1][0] = *reinterpret_cast<const Q4*>(ap + o);
+          wf[q & 1][1] = *reinterpret_cast<const Q4*>(wp + wrow1 + o);
+          if constexpr (MI > 1) af[q & 1][1] = *reinterpret_cast<const Q4*>(ap + 64 * 128 + o);
+        }
+      };
+      read(0);
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int o = ((2 * q + h) ^ sw) * 16;
-        w0[q] = *reinterpret_cast<const Q4*>(wp + o);
-        w1[q] = *reinterpret_cast<const Q4*>(wp + wrow1 + o);
-        a0[q] = *reinterpret_cast<const Q4*>(ap + o);
-      }
-      if (act1) {
-        Q4 a1[4];
+        if (q < 3) read(q + 1);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) a1[q] = *reinterpret_cast<const Q4*>(ap + 64 * 128 + ((2 * q + h) ^ sw) * 16);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          acc[0][0] = mfma32<DT>(w0[q], a0[q], acc[0][0]);
-          acc[0][1] = mfma32<DT>(w1[q], a0[q], acc[0][1]);
-          acc[1][0] = mfma32<DT>(w0[q], a1[q], acc[1][0]);
-          acc[1][1] = mfma32<DT>(w1[q], a1[q], acc[1][1]);
-        }
-      } else {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          acc[0][0] = mfma32<DT>(w0[q], a0[q], acc[0][0]);
-          acc[0][1] = mfma32<DT>(w1[q], a0[q], acc[0][1]);
+        for (int i = 0; i < 2; ++i) {   // (the rows' four requests in front of the weights': the wait above counts on it)
+          if constexpr (MI > 0) {
+            acc[0][i] = mfma32<DT>(wf[q & 1][i], af[q & 1][0], acc[0][i]);
+            if constexpr (MI > 1) acc[1][i] = mfma32<DT>(wf[q & 1][i], af[q & 1][1], acc[1][i]);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          if (q < 2) get_a(s + 1, 2 * q + i, IN);
+          else get_w(s + 2, 2 * (q - 2) + i, wbuf, IN);
+          __builtin_amdgcn_sched_barrier(0);
         }
       }
-    }
-    buf = buf == 2 ? 0 : buf + 1;
-  }
+      buf = buf == 2 ? 0 : buf + 1;
+    };
+    int s = 0;
+    for (; s + 2 < whole; ++s) step(s, std::true_type{});
+    for (; s < steps; ++s) step(s, std::false_type{});
+  };
+  if (!act0) walk(std::integral_constant<int, 0>{});
+  else if (!act1) walk(std::integral_constant<int, 1>{});
+  else walk(std::integral_constant<int, 2>{});
   __builtin_amdgcn_s_waitcnt(0x0070);   // (requests past the end have landed before the LDS is given back)
   if (!act0) return;
 #pragma unroll
@@ -895,23 +929,29 @@ extern "C" int ll_moe_rows_gemm(const void* a, int64_t a_ld, int64_t a_div, cons
     const unsigned grid = (unsigned)(few ? max_tiles : (max_tiles + 7) / 8 * 8 + 8);   // (a range of an XCD may hold one tile more than an eighth)
     const int wide = N % 4 == 0 && out_ld % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & 7u) == 0;
     constexpr int bytes = 5 * 128 * 128;
+    // rows and one expert's weights within 32-bit offsets, as all but the very largest are
+    const bool near = (num_slots / a_div + 1) * a_ld * 2 < (1ll << 32) && (mode == 1 ? 2 : 1) * N * K * 2 < (1ll << 32);
     int dev = 0;
     (void)hipGetDevice(&dev);
-#define CALL_T(DT, G)                                                                                                             \
+#define CALL_F(DT, G, FAR)                                                                                                         \
   do {                                                                                                                            \
     static bool attr[16] = {false};                                                                                               \
     if (dev >= 0 && dev < 16 && !attr[dev]) {                                                                                     \
-      (void)hipFuncSetAttribute((const void*)moe_rows_gemm_tiled_kernel<DT, G>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes); \
+      (void)hipFuncSetAttribute((const void*)moe_rows_gemm_tiled_kernel<DT, G, FAR>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes); \
       attr[dev] = true;                                                                                                           \
     }                                                                                                                             \
-    moe_rows_gemm_tiled_kernel<DT, G><<<dim3(grid), 256, bytes, st>>>((const uint16_t*)a, a_ld, (int)a_div, (const uint16_t*)w,   \
+    moe_rows_gemm_tiled_kernel<DT, G, FAR><<<dim3(grid), 256, bytes, st>>>((const uint16_t*)a, a_ld, (int)a_div, (const uint16_t*)w,   \
                                                                       w_stride_e, (int)K, (int)N, slot_weight, (uint16_t*)out, out_ld, \
                                                                       sorted, block_expert, num_post, (int)num_slots, glu_limit, \
                                                                       (int)tiles_n, wide, few, (int)((num_slots + experts * 127) / 128)); \
   } while (0)
-    if (dtype == LL_F16) { if (mode == 1) CALL_T(LL_F16, 1); else if (mode == 2) CALL_T(LL_F16, 2); else CALL_T(LL_F16, 0); }
-    else { if (mode == 1) CALL_T(LL_BF16, 1); else if (mode == 2) CALL_T(LL_BF16, 2); else CALL_T(LL_BF16, 0); }
+#define CALL_T(DT, G)             \
+  if (near) CALL_F(DT, G, false); \
+  else CALL_F(DT, G, true)
+    if (dtype == LL_F16) { if (mode == 1) { CALL_T(LL_F16, 1); } else if (mode == 2) { CALL_T(LL_F16, 2); } else { CALL_T(LL_F16, 0); } }
+    else { if (mode == 1) { CALL_T(LL_BF16, 1); } else if (mode == 2) { CALL_T(LL_BF16, 2); } else { CALL_T(LL_BF16, 0); } }
 #undef CALL_T
+#undef CALL_F
     return LL_LAUNCH_CHECK();
   }
   const int64_t max_blocks = most * (block / 32);   // (the plain form takes either order)

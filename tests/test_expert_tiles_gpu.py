@@ -53,6 +53,32 @@ def test_experts_of_every_load(dtype, width, ff, form):
     assert ((got.to(F64) - want).abs() <= unit * (want.abs() + 6 * mid) + 2.0 ** -14 * unit).all()
 
 
+def test_rows_beyond_32_bit_offsets():
+    from lite_llama_amd import _lib as L
+
+    tokens, experts, width, ff, ld = 300, 2, 200, 136, (1 << 23) + 8      # (rows 16 MB apart: the last ones lie 5 GB in)
+    g = torch.Generator(device=DEV).manual_seed(3)
+    rows = torch.empty((tokens - 1) * ld + width, dtype=torch.bfloat16, device=DEV).as_strided((tokens, width), (ld, 1))
+    rows.copy_(torch.randn(tokens, width, generator=g, device=DEV))
+    w = (torch.randn(experts, ff, width, generator=g, device=DEV) * width ** -0.5).to(torch.bfloat16)
+    ids = torch.randint(0, experts, (tokens, 1), generator=g, device=DEV, dtype=torch.int32)
+    block = 128
+    padded = tokens + experts * (block - 1)
+    meta = torch.empty(experts + padded + -(-padded // block) + 1, dtype=torch.int32, device=DEV)
+    srt, owner, post = meta[experts:experts + padded], meta[experts + padded:-1], meta[-1:]
+    L.check(L.lib().ll_moe_sort(ids.data_ptr(), tokens, experts, block, meta[:experts].data_ptr(), srt.data_ptr(), owner.data_ptr(),
+                                post.data_ptr(), L.stream_ptr()), "moe_sort")
+    out = {}
+    for name, a in (("far", rows), ("near", rows.contiguous())):
+        out[name] = torch.empty(tokens, ff, dtype=torch.bfloat16, device=DEV)
+        L.check(L.lib().ll_moe_rows_gemm(a.data_ptr(), a.stride(0), 1, w.data_ptr(), w.stride(0), width, ff, 0, 0, out[name].data_ptr(), ff,
+                                         srt.data_ptr(), owner.data_ptr(), post.data_ptr(), tokens, experts, block, 0.0,
+                                         L.dtype_code(torch.bfloat16), L.stream_ptr()), "moe_rows_gemm")
+    assert torch.equal(out["far"], out["near"])
+    want = (rows.to(F64)[:, None] @ w[ids[:, 0].long()].to(F64).transpose(1, 2).contiguous())[:, 0]
+    assert ((out["near"].to(F64) - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -18).all()
+
+
 @pytest.mark.parametrize("slots,experts,block", [(1, 1, 32), (7, 5, 32), (256, 34, 128), (257, 300, 32), (5000, 64, 128), (13057, 3, 128), (900, 9000, 32)])
 @pytest.mark.parametrize("skipped", [False, True])
 def test_slots_sorted_by_expert(slots, experts, block, skipped):
