@@ -805,6 +805,9 @@ int ll_rotate_pairs(const void* q, int64_t q_tok_stride, int64_t q_head_stride, 
  * [experts]; sorted [num_slots + experts (block - 1)], block_expert [ceil(that / block)], num_post [1]).  ll_moe_sort_skipped (up to 8192
  * experts): slots whose id lies outside 0 .. experts - 1 follow in a run of their own under expert -1 (arrays for experts + 1 runs);
  * ll_moe_rows_gemm writes zeros for them where glu == 0 or 3, nothing where it makes gated activations.
+ * ll_group_router_sorted: ll_group_router, and its slots sorted over `sorted_experts` experts as ll_moe_sort (skipped: ll_moe_sort_skipped)
+ * sorts them; for few tokens the logits are
+ * spread over the chip and every expert's workgroup makes the choices for itself.
  * ll_moe_rows_gemm: glu != 0: w [experts][2 N][K] (gate rows, then up rows), out[slot] = silu(a Wg^T) * (a Wu^T) with
  * a = row slot / a_div (glu == 2: g' sigmoid(1.702 g') (u' + 1) with g' = min(g, limit), u' = clamp(u, -limit, limit));
  * glu == 0: w [experts][N][K], out[slot] = (a W^T) * slot_weight[slot]; glu == 3: w [experts][N][K],
@@ -813,6 +816,11 @@ int ll_group_router(const void* h, int64_t h_ld, const void* w_router, const voi
                     int64_t experts, int64_t top, int64_t group_count, int64_t group_keep, float route_scale, int scoring,
                     int32_t* ids, float* weights, float* extra_scale, float* logits, const void* correction, int64_t identity,
                     int dtype, void* stream);
+int ll_group_router_sorted(const void* h, int64_t h_ld, const void* w_router, const void* w_extra, int64_t n, int64_t width,
+                           int64_t experts, int64_t top, int64_t group_count, int64_t group_keep, float route_scale, int scoring,
+                           int32_t* ids, float* weights, float* extra_scale, float* logits, const void* correction, int64_t identity,
+                           int64_t sorted_experts, int64_t block, int skipped, int32_t* counts, int32_t* sorted,
+                           int32_t* block_expert, int32_t* num_post, int dtype, void* stream);
 int64_t ll_moe_rows_block(int64_t num_slots, int64_t experts, int64_t width, int64_t ff, int dtype);
 int ll_moe_sort(const int32_t* ids, int64_t num_slots, int64_t experts, int64_t block, int32_t* counts, int32_t* sorted,
                 int32_t* block_expert, int32_t* num_post, void* stream);

@@ -152,6 +152,7 @@ SIGNATURES = {
     "ll_latent_kv_prep": [P, L, L, L, L, P, F, P, L, F, P, P, P, L, L, L, P, P, L, I, P],
     "ll_rotate_pairs": [P, L, L, L, L, P, L, F, P, P, L, L, L, L, I, P],
     "ll_group_router": [P, L, P, P, L, L, L, L, L, L, F, I, P, P, P, P, P, L, I, P],
+    "ll_group_router_sorted": [P, L, P, P, L, L, L, L, L, L, F, I, P, P, P, P, P, L, L, L, I, P, P, P, P, I, P],
     "ll_moe_rows_block": [L, L, L, L, I],
     "ll_moe_sort": [P, L, L, L, P, P, P, P, P],
     "ll_moe_sort_skipped": [P, L, L, L, P, P, P, P, P],

@@ -152,9 +152,108 @@ __host__ __device__ static inline size_t select_floats(int scoring, int experts,
 
 __device__ __forceinline__ void select_settle() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
+__device__ __forceinline__ float lane_value(float v, int lane) {
+  return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), lane));
+}
+
+// ... where neither groups nor many slots are asked for: a lane holds the scores of EL experts in registers, and the best is taken `top` times.
+// Ranking every expert against every other takes experts^2 / 64 compares per token (68 experts: some 600 vector instructions, of which this needs
+// some 250); sums in the same order, the same choices.  (A NaN ranks behind every number here, so that every slot gets an expert.)  us of router and
+// sort in a graph, ranks -> this: 34 rows, top 4, 32 tokens 13.6 -> 13.1, 3264 33.0 -> 31.9; 68 rows, top 8, 32 tokens 18.5 -> 16.1, 3264 70.3 -> 66.7
+constexpr int kSmallTop = 16;
+
+template <int SCORING, int DT, int EL>
+__device__ __forceinline__ void select_small(const SelectArgs& p, const float* z, int64_t t, int lane) {
+  const int experts = p.experts, top = p.top;
+  float zv[EL], shift[EL], plain[EL], score[EL];
+#pragma unroll
+  for (int i = 0; i < EL; ++i) {
+    const int e = lane + 64 * i < experts ? lane + 64 * i : experts - 1;
+    zv[i] = z[e];
+    shift[i] = SCORING == 2 && p.correction ? ldv<DT>(p.correction, e) : 0.f;
+  }
+  float extra = 0.f;
+  if (SCORING != 2 && p.extra_scale) extra = z[p.rows - 1];
+  if constexpr (SCORING == 2 || SCORING == 4) {
+    float top_z = zv[0];   // (a clamped lane repeats the last expert's)
+#pragma unroll
+    for (int i = 1; i < EL; ++i) top_z = fmaxf(top_z, zv[i]);
+    top_z = wave_max(top_z);
+    float total = 0.f;
+#pragma unroll
+    for (int i = 0; i < EL; ++i) {
+      plain[i] = expf(zv[i] - top_z);
+      const float term = lane + 64 * i < experts ? plain[i] : 0.f;   // (in index order, eight at a time: the last ones past the end add zeros)
+      for (int e = 0; e < 64 && e + 64 * i < experts; e += 8)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) total += lane_value(term, e + j);
+    }
+#pragma unroll
+    for (int i = 0; i < EL; ++i) {
+      plain[i] /= total;
+      score[i] = SCORING == 2 && p.correction ? plain[i] + shift[i] : plain[i];
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < EL; ++i) plain[i] = score[i] = SCORING == 1 ? zv[i] : sigmoid_exact(zv[i]);
+  }
+  if (SCORING != 2 && p.rows > experts && lane == 0) p.extra_scale[t] = sigmoid_exact(extra);
+  bool left[EL];
+#pragma unroll
+  for (int i = 0; i < EL; ++i) left[i] = lane + 64 * i < experts;
+  int id = 0;
+  float own = 0.f, mine = 0.f, sum = 0.f, first = 0.f;   // lane k: slot k's expert and score; sums in the slots' order
+  for (int k = 0; k < top; ++k) {
+    float best = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < EL; ++i) best = left[i] ? fmaxf(best, score[i]) : best;
+    best = wave_max(best);
+    unsigned long long mask[EL];
+#pragma unroll
+    for (int i = 0; i < EL; ++i) mask[i] = __ballot(left[i] && score[i] == best);
+    bool any = mask[0] != 0;
+#pragma unroll
+    for (int i = 1; i < EL; ++i) any = any || mask[i] != 0;
+    if (!any) {   // only NaN is left
+#pragma unroll
+      for (int i = 0; i < EL; ++i) mask[i] = __ballot(left[i]);
+    }
+    int e = 0;
+    float value = 0.f;
+#pragma unroll
+    for (int i = EL - 1; i >= 0; --i) {
+      if (mask[i]) {
+        const int l = __ffsll(mask[i]) - 1;
+        e = l + 64 * i;
+        value = lane_value(plain[i], l);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < EL; ++i) left[i] = left[i] && e != lane + 64 * i;
+    if (SCORING == 2) own += e >= experts - p.identity ? value : 0.f;
+    else if (SCORING == 1) {
+      first = k == 0 ? value : first;
+      value = expf(value - first);
+      sum += value;
+    } else sum += value;
+    id = lane == k ? e : id;
+    mine = lane == k ? value : mine;
+  }
+  if (SCORING == 2 && p.extra_scale && lane == 0) p.extra_scale[t] = own * p.route_scale;
+  if (lane < top) {
+    p.ids[t * top + lane] = id;
+    p.weights[t * top + lane] = (SCORING == 1 ? mine / sum : SCORING == 2 || SCORING == 3 ? mine : mine / (sum + 1e-20f)) * p.route_scale;
+  }
+}
+
 template <int SCORING, int DT>
 __device__ __forceinline__ void select_token(const SelectArgs& p, const float* z, int64_t t, float* lds, int lane) {
   const int experts = p.experts, top = p.top;
+  if (p.group_count == 1 && experts <= 128 && top <= kSmallTop) {
+    if (experts <= 64) select_small<SCORING, DT, 1>(p, z, t, lane);
+    else select_small<SCORING, DT, 2>(p, z, t, lane);
+    return;
+  }
   float* score = lds;
   float* gscore = score + experts;
   float* gkeep = gscore + p.group_count;
@@ -377,10 +476,10 @@ __global__ __launch_bounds__(64 * NW) void router_kernel(const void* __restrict_
 // ------------------------------------------------------------------------------------------------------------------------
 constexpr int kSortExperts = 8192;
 
-__global__ __launch_bounds__(1024) void moe_sort_kernel(const int32_t* __restrict__ ids, int num_slots, int experts, int block_m, int skipped,
-                                                       int32_t* __restrict__ counts, int32_t* __restrict__ sorted,
-                                                       int32_t* __restrict__ block_expert, int32_t* __restrict__ num_post) {
-  extern __shared__ int hist[];   // [experts]: counts of the experts in front of this workgroup's
+// hist: LDS [experts], counts of the experts in front of this workgroup's
+__device__ __forceinline__ void sort_expert(const int32_t* ids, int num_slots, int experts, int block_m, int skipped, int* hist,
+                                            int32_t* __restrict__ counts, int32_t* __restrict__ sorted, int32_t* __restrict__ block_expert,
+                                            int32_t* __restrict__ num_post) {
   __shared__ int part[16], start[16];
   const int e = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, threads = blockDim.x, waves = threads >> 6;
   for (int i = tid; i < e; i += threads) hist[i] = 0;
@@ -425,6 +524,108 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(const int32_t* __restric
     if (e < experts) counts[e] = total;
     if (e == experts - 1 + skipped) num_post[0] = base + padded;
   }
+}
+
+__global__ __launch_bounds__(1024) void moe_sort_kernel(const int32_t* __restrict__ ids, int num_slots, int experts, int block_m, int skipped,
+                                                       int32_t* __restrict__ counts, int32_t* __restrict__ sorted,
+                                                       int32_t* __restrict__ block_expert, int32_t* __restrict__ num_post) {
+  extern __shared__ int hist[];
+  sort_expert(ids, num_slots, experts, block_m, skipped, hist, counts, sorted, block_expert, num_post);
+}
+
+// ------------------------------------------------------------------------------------------------------------------------
+// router and sort of few tokens (up to kRouteTokens): the logits by a wave per token and two rows, all over the chip, then ONE launch in which
+// each expert's workgroup chooses for every token by itself (the choices stay in LDS; the first workgroup writes them out) and sorts its slots.
+// In a workgroup per token as above the weights come through one CU each, 20 - 25 KB/us where they are not in its L2: at few tokens
+// that, and not the choice, was the launch's time.  Sums in router_kernel's order: the same bits.
+// ------------------------------------------------------------------------------------------------------------------------
+constexpr int kRouteTokens = 16;
+
+template <int DT, int VEC>
+__global__ __launch_bounds__(64) void route_logits_kernel(const void* __restrict__ h, int64_t h_ld, const void* __restrict__ w_router,
+                                                          const void* __restrict__ w_extra, int width, int experts, int rows,
+                                                          float* __restrict__ logits) {
+  constexpr int EW = 2, PU = 8;   // rows of weights; pieces of the width that are requested together
+  const int lane = threadIdx.x, e0 = blockIdx.x * EW;
+  const int64_t hat = (int64_t)blockIdx.y * h_ld;
+  const void* wp[EW];
+  int64_t wat[EW];
+#pragma unroll
+  for (int j = 0; j < EW; ++j) {
+    const int e = e0 + j < rows ? e0 + j : rows - 1;
+    wp[j] = e < experts ? w_router : w_extra;
+    wat[j] = e < experts ? (int64_t)e * width : 0;
+  }
+  float acc[EW] = {};
+  for (int p0 = lane * VEC; p0 < width; p0 += 64 * VEC * PU) {
+    float hv[PU][VEC], wv[PU][EW][VEC];
+#pragma unroll
+    for (int u = 0; u < PU; ++u) {
+      const int at = p0 + u * 64 * VEC;
+      const bool in = at < width;
+#pragma unroll
+      for (int j = 0; j < EW; ++j) load_piece<DT, VEC>(wp[j], wat[j] + (in ? at : p0), wv[u][j]);
+      load_piece<DT, VEC>(h, hat + (in ? at : p0), hv[u]);
+#pragma unroll
+      for (int k = 0; k < VEC; ++k) {
+        hv[u][k] = in ? hv[u][k] : 0.f;
+#pragma unroll
+        for (int j = 0; j < EW; ++j) wv[u][j][k] = in ? wv[u][j][k] : 0.f;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < PU; ++u)
+#pragma unroll
+      for (int j = 0; j < EW; ++j)
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) {
+          if constexpr (DT == LL_F32) acc[j] += hv[u][k] * wv[u][j][k];
+          else acc[j] = __builtin_fmaf(hv[u][k], wv[u][j][k], acc[j]);
+        }
+  }
+#pragma unroll
+  for (int j = 0; j < EW; ++j) {
+    const float v = wave_sum(acc[j]);
+    if (lane == 0 && e0 + j < rows) logits[(int64_t)blockIdx.y * rows + e0 + j] = v;
+  }
+}
+
+// sorted_experts: those with weights (ids beyond them are identity experts); LDS: hist [sorted_experts], the choices' ids and weights [n top] and
+// extra [n], then what select_token wants, once per wave
+template <int SCORING, int DT>
+__global__ __launch_bounds__(1024) void route_sort_kernel(const float* __restrict__ logits, const SelectArgs p, int n, int sorted_experts, int block_m,
+                                                          int skipped, int32_t* __restrict__ counts, int32_t* __restrict__ sorted,
+                                                          int32_t* __restrict__ block_expert, int32_t* __restrict__ num_post) {
+  extern __shared__ int route_lds[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), waves = (int)blockDim.x >> 6;
+  const int slots = n * p.top;
+  int32_t* ids = route_lds + sorted_experts;
+  float* weights = (float*)(ids + slots);
+  float* extra = weights + slots;
+  float* scratch = extra + n + (size_t)wave * select_floats(SCORING, p.experts, p.group_count, p.top);
+  SelectArgs q = p;
+  q.ids = ids;
+  q.weights = weights;
+  q.extra_scale = p.extra_scale ? extra : nullptr;
+  for (int i = threadIdx.x; i < slots; i += blockDim.x) {   // (a slot that NaN logits leave without an expert is one that no expert serves)
+    ids[i] = -1;
+    weights[i] = 0.f;
+  }
+  __syncthreads();
+  for (int t = wave; t < n; t += waves) {
+    select_token<SCORING, DT>(q, logits + (int64_t)t * p.rows, t, scratch, lane);
+    select_settle();   // (the next token's scores take this one's place)
+  }
+  __syncthreads();
+  if (blockIdx.x == 0) {
+    for (int i = threadIdx.x; i < slots; i += blockDim.x) {
+      p.ids[i] = ids[i];
+      p.weights[i] = weights[i];
+    }
+    if (p.extra_scale)
+      for (int i = threadIdx.x; i < n; i += blockDim.x) p.extra_scale[i] = extra[i];
+  }
+  sort_expert(ids, slots, sorted_experts, block_m, skipped, route_lds, counts, sorted, block_expert, num_post);
 }
 
 // more experts: a workgroup per expert, twice (count, then place)
@@ -776,11 +977,15 @@ __global__ __launch_bounds__(256, 2) void moe_rows_gemm_tiled_kernel(const uint1
     else { CALL(LL_F32); }                   \
   } while (0)
 
-// logits: fp32 scratch [n][experts + (w_extra ? 1 : 0)], written where the router takes two launches (more than kRouterRows rows)
-extern "C" int ll_group_router(const void* h, int64_t h_ld, const void* w_router, const void* w_extra, int64_t n, int64_t width,
-                               int64_t experts, int64_t top, int64_t group_count, int64_t group_keep, float route_scale, int scoring,
-                               int32_t* ids, float* weights, float* extra_scale, float* logits, const void* correction, int64_t identity,
-                               int dtype, void* stream) {
+struct RouterCall {
+  SelectArgs p;
+  size_t each;   // floats of LDS for one token's choice
+  bool aligned;
+};
+
+static int router_call(RouterCall& c, const void* h, int64_t h_ld, const void* w_router, const void* w_extra, int64_t n, int64_t width,
+                       int64_t experts, int64_t top, int64_t group_count, int64_t group_keep, float route_scale, int scoring, int32_t* ids,
+                       float* weights, float* extra_scale, float* logits, const void* correction, int64_t identity, int dtype) {
   if (dtype != LL_F16 && dtype != LL_BF16 && dtype != LL_F32) return LL_ERR_DTYPE;
   if (scoring == 2 && (group_count != 1 || w_extra || identity < 0 || identity > experts || (identity > 0 && !extra_scale)))
     return LL_ERR_SHAPE;
@@ -789,14 +994,29 @@ extern "C" int ll_group_router(const void* h, int64_t h_ld, const void* w_router
       experts % group_count || group_keep < 1 || group_keep > group_count || group_keep * (experts / group_count) < top ||
       scoring < 0 || scoring > 4 || (scoring == 1 && group_count != 1))
     return LL_ERR_SHAPE;
-  if (n == 0) return LL_OK;
-  if (!h || !w_router || !ids || !weights || !logits || (w_extra && !extra_scale)) return LL_ERR_ARG;
+  if (n > 0 && (!h || !w_router || !ids || !weights || !logits || (w_extra && !extra_scale))) return LL_ERR_ARG;
   const int rows = (int)experts + (w_extra ? 1 : 0);
   const int vec = dtype == LL_F32 ? 4 : 8;
-  const bool aligned = width % vec == 0 && h_ld % vec == 0 && ll_aligned16(h) && ll_aligned16(w_router) && (!w_extra || ll_aligned16(w_extra));
+  c.aligned = width % vec == 0 && h_ld % vec == 0 && ll_aligned16(h) && ll_aligned16(w_router) && (!w_extra || ll_aligned16(w_extra));
+  c.p = SelectArgs{rows, (int)experts, (int)top, (int)group_count, (int)group_keep, (int)identity, route_scale, ids, weights, extra_scale, correction};
+  c.each = select_floats(scoring, (int)experts, (int)group_count, (int)top);
+  return LL_OK;
+}
+
+// logits: fp32 scratch [n][experts + (w_extra ? 1 : 0)], written where the router takes two launches (more than kRouterRows rows)
+extern "C" int ll_group_router(const void* h, int64_t h_ld, const void* w_router, const void* w_extra, int64_t n, int64_t width,
+                               int64_t experts, int64_t top, int64_t group_count, int64_t group_keep, float route_scale, int scoring,
+                               int32_t* ids, float* weights, float* extra_scale, float* logits, const void* correction, int64_t identity,
+                               int dtype, void* stream) {
+  RouterCall c;
+  const int bad = router_call(c, h, h_ld, w_router, w_extra, n, width, experts, top, group_count, group_keep, route_scale, scoring, ids, weights,
+                              extra_scale, logits, correction, identity, dtype);
+  if (bad || n == 0) return bad;
+  const SelectArgs& p = c.p;
+  const int rows = p.rows;
+  const size_t each = c.each;
+  const bool aligned = c.aligned;
   hipStream_t st = (hipStream_t)stream;
-  const SelectArgs p{rows, (int)experts, (int)top, (int)group_count, (int)group_keep, (int)identity, route_scale, ids, weights, extra_scale, correction};
-  const size_t each = select_floats(scoring, (int)experts, (int)group_count, (int)top);
   if (rows <= kRouterRows) {
     const int tw = n > 256 ? 4 : 1, nw = tw == 1 && rows > 40 ? 16 : 8;   // tokens per workgroup; waves
     const dim3 grid((unsigned)((n + tw - 1) / tw));
@@ -887,6 +1107,60 @@ extern "C" int ll_moe_sort(const int32_t* ids, int64_t num_slots, int64_t expert
 extern "C" int ll_moe_sort_skipped(const int32_t* ids, int64_t num_slots, int64_t experts, int64_t block, int32_t* counts, int32_t* sorted,
                                    int32_t* block_expert, int32_t* num_post, void* stream) {
   return moe_sort(ids, num_slots, experts, block, 1, counts, sorted, block_expert, num_post, stream);
+}
+
+// ll_group_router, and its choices sorted as ll_moe_sort (`skipped`: ll_moe_sort_skipped) sorts them: `sorted_experts` experts in blocks of `block`
+extern "C" int ll_group_router_sorted(const void* h, int64_t h_ld, const void* w_router, const void* w_extra, int64_t n, int64_t width,
+                                      int64_t experts, int64_t top, int64_t group_count, int64_t group_keep, float route_scale, int scoring,
+                                      int32_t* ids, float* weights, float* extra_scale, float* logits, const void* correction, int64_t identity,
+                                      int64_t sorted_experts, int64_t block, int skipped, int32_t* counts, int32_t* sorted,
+                                      int32_t* block_expert, int32_t* num_post, int dtype, void* stream) {
+  RouterCall c;
+  const int bad = router_call(c, h, h_ld, w_router, w_extra, n, width, experts, top, group_count, group_keep, route_scale, scoring, ids, weights,
+                              extra_scale, logits, correction, identity, dtype);
+  if (bad) return bad;
+  const int rows = c.p.rows;
+  const size_t lds = sizeof(float) * (sorted_experts + 2 * n * top + n + 16 * c.each);
+  // us of router and sort in a graph, weights not in L2, workgroups per token and per expert -> here: 34 rows of 2048, top 4: 1 token 12.8 -> 9.5,
+  // 4 13.3 -> 9.8, 8 13.6 -> 10.4, 16 13.2 -> 12.3, 24 13.1 -> 13.2 (every workgroup chooses for every token); 68 rows of 3072, top 8: 1 15.9 -> 11.1,
+  // 4 16.5 -> 11.6, 8 16.5 -> 12.3, 16 16.5 -> 15.1, 24 16.3 -> 16.7
+  if (n < 1 || n > kRouteTokens || rows > kRouterRows || sorted_experts < 1 || sorted_experts > experts || (block != 32 && block != 128) ||
+      lds > 65536) {
+    const int rc = ll_group_router(h, h_ld, w_router, w_extra, n, width, experts, top, group_count, group_keep, route_scale, scoring, ids, weights,
+                                   extra_scale, logits, correction, identity, dtype, stream);
+    return rc ? rc : moe_sort(ids, n * top, sorted_experts, block, skipped ? 1 : 0, counts, sorted, block_expert, num_post, stream);
+  }
+  if (!counts || !sorted || !block_expert || !num_post) return LL_ERR_ARG;
+  hipStream_t st = (hipStream_t)stream;
+  const dim3 grid((unsigned)((rows + 1) / 2), (unsigned)n);
+#define LL_RL(DT, V) route_logits_kernel<DT, V><<<grid, 64, 0, st>>>(h, h_ld, w_router, w_extra, (int)width, (int)experts, rows, logits)
+  if (!c.aligned) {
+#define CALL(DT) LL_RL(DT, 1)
+    LL_BY_DTYPE(dtype, CALL);
+#undef CALL
+  } else if (dtype == LL_F32) {
+    LL_RL(LL_F32, 4);
+  } else if (dtype == LL_F16) {
+    LL_RL(LL_F16, 8);
+  } else {
+    LL_RL(LL_BF16, 8);
+  }
+#undef LL_RL
+  const unsigned threads = n <= 4 ? 256 : n <= 8 ? 512 : 1024;   // a wave per token
+#define LL_GS(S, DT)                                                                                                                          \
+  route_sort_kernel<S, DT><<<dim3((unsigned)(sorted_experts + (skipped ? 1 : 0))), threads, lds, st>>>(logits, c.p, (int)n, (int)sorted_experts, \
+                                                                                                     (int)block, skipped ? 1 : 0, counts, sorted, \
+                                                                                                     block_expert, num_post)
+  if (scoring == 2) {
+#define CALL(DT) LL_GS(2, DT)
+    LL_BY_DTYPE(dtype, CALL);
+#undef CALL
+  } else if (scoring == 1) LL_GS(1, LL_F32);
+  else if (scoring == 4) LL_GS(4, LL_F32);
+  else if (scoring == 3) LL_GS(3, LL_F32);
+  else LL_GS(0, LL_F32);
+#undef LL_GS
+  return LL_LAUNCH_CHECK();
 }
 
 // glu != 0: w [experts][2 N][K] (gate rows, then up rows), out[slot][N] = silu(a_row Wg^T) * (a_row Wu^T) with a_row =

@@ -281,7 +281,7 @@ def moe_router(x: torch.Tensor, gate_weight: torch.Tensor, top_k: int, norm_topk
 @torch.no_grad()
 def group_router(h: torch.Tensor, router_weight: torch.Tensor, top: int, group_count: int = 1, group_keep: int = 1,
                  route_scale: float = 1.0, extra_weight: torch.Tensor | None = None, scoring: str = "sigmoid",
-                 correction: torch.Tensor | None = None, identity: int = 0):
+                 correction: torch.Tensor | None = None, identity: int = 0, sort_for: torch.Tensor | None = None, skipped: bool = False):
     """``scores = sigmoid(router_weight h)`` in fp32 (``h`` in its storage dtype); the experts form ``group_count`` equal groups
     of neighbours, a group's score is the sum of its two best, the best ``group_keep`` groups stay eligible; the ``top`` best
     eligible experts are chosen.  Returns ``(ids int32 [n, top], weights fp32 [n, top], extra)``: weights = chosen scores /
@@ -294,7 +294,9 @@ def group_router(h: torch.Tensor, router_weight: torch.Tensor, top: int, group_c
     ids ``>= experts - identity`` (which :func:`sparse_glu_experts` leaves as zero rows) and ``extra`` is the sum of their
     scores per token -- the factor of ``h`` itself in the sublayer's result.  ``scoring="sigmoid_plain"``: as ``"sigmoid"``, but the
     weights are the chosen scores themselves (times ``route_scale``), not divided by their sum.  ``scoring="softmax_groups"``: scores are
-    the softmax over all router outputs, a group's score is its LARGEST, the weights are divided by their sum as in ``"sigmoid"``."""
+    the softmax over all router outputs, a group's score is its LARGEST, the weights are divided by their sum as in ``"sigmoid"``.
+    ``sort_for``: the second product's weights ``[experts, width, ff]`` of the experts that will serve the slots (``skipped``: some
+    slots may be served by none): the slots are sorted as well, and a fourth value returned for the products' ``order``."""
     L.require_cuda(h, router_weight, extra_weight, correction)
     n, width = h.shape
     experts = router_weight.shape[0]
@@ -310,43 +312,55 @@ def group_router(h: torch.Tensor, router_weight: torch.Tensor, top: int, group_c
         raise ValueError("group_router: corrections and identity experts belong to the softmax_all scoring")
     extra = torch.empty(n, dtype=torch.float32, device=h.device) if (extra_weight is not None or identity) else None
     logits = torch.empty(n, experts + (1 if extra_weight is not None else 0), dtype=torch.float32, device=h.device)
-    L.check(L.lib().ll_group_router(h.data_ptr(), h.stride(0), router_weight.data_ptr(), L.ptr(extra_weight), n, width, experts,
-                                    int(top), int(group_count), int(group_keep), float(route_scale),
-                                    {"sigmoid": 0, "softmax_chosen": 1, "softmax_all": 2, "sigmoid_plain": 3, "softmax_groups": 4}[scoring], ids.data_ptr(),
-                                    weights.data_ptr(), L.ptr(extra), logits.data_ptr(), L.ptr(correction), int(identity),
-                                    L.dtype_code(h.dtype), L.stream_ptr()),
-            "group_router")
+    scorings = {"sigmoid": 0, "softmax_chosen": 1, "softmax_all": 2, "sigmoid_plain": 3, "softmax_groups": 4}
+    args = (h.data_ptr(), h.stride(0), router_weight.data_ptr(), L.ptr(extra_weight), n, width, experts, int(top), int(group_count),
+            int(group_keep), float(route_scale), scorings[scoring], ids.data_ptr(), weights.data_ptr(), L.ptr(extra), logits.data_ptr(),
+            L.ptr(correction), int(identity))
+    if sort_for is not None:
+        served, _, ff = sort_for.shape
+        run = skipped and served <= _SKIPPED_RUN
+        order, counts = _slot_lists(ids, n * top, served, width, ff, h.dtype, run)
+        block, sorted_ids, block_expert, num_post = order
+        L.check(L.lib().ll_group_router_sorted(*args, served, block, run, counts.data_ptr(), sorted_ids.data_ptr(), block_expert.data_ptr(),
+                                               num_post.data_ptr(), L.dtype_code(h.dtype), L.stream_ptr()), "group_router_sorted")
+        return ids, weights, extra, order
+    L.check(L.lib().ll_group_router(*args, L.dtype_code(h.dtype), L.stream_ptr()), "group_router")
     return ids, weights, extra
 
 
 _SKIPPED_RUN = 8192   # most experts beside which ll_moe_sort_skipped sorts skipped slots
 
 
+def _slot_lists(ids: torch.Tensor, slots: int, experts: int, width: int, ff: int, dt, skipped: bool):
+    """Room for slots sorted by expert in row blocks: ``((rows per block, sorted slots, expert of every block, [padded count]), counts)``."""
+    block = int(L.lib().ll_moe_rows_block(slots, experts, width, ff, L.dtype_code(dt)))
+    padded = slots + (experts + (1 if skipped else 0)) * (block - 1)
+    meta = torch.empty(experts + padded + -(-padded // block) + 1, dtype=torch.int32, device=ids.device)
+    return (block, meta[experts:experts + padded], meta[experts + padded:-1], meta[-1:]), meta[:experts]
+
+
 def _sort_slots(ids: torch.Tensor, slots: int, experts: int, width: int, ff: int, dt, skipped: bool = False):
     """Slots sorted by expert in row blocks: ``(rows per block, sorted slots, expert of every block, [padded count])``.  ``skipped``:
     slots whose id is no expert's follow in blocks of expert -1."""
     lib = L.lib()
-    block = int(lib.ll_moe_rows_block(slots, experts, width, ff, L.dtype_code(dt)))
-    padded = slots + (experts + (1 if skipped else 0)) * (block - 1)
-    meta = torch.empty(experts + padded + -(-padded // block) + 1, dtype=torch.int32, device=ids.device)
-    counts, sorted_ids = meta[:experts], meta[experts:experts + padded]
-    block_expert, num_post = meta[experts + padded:-1], meta[-1:]
+    order, counts = _slot_lists(ids, slots, experts, width, ff, dt, skipped)
+    block, sorted_ids, block_expert, num_post = order
     sort = lib.ll_moe_sort_skipped if skipped else lib.ll_moe_sort
     L.check(sort(ids.data_ptr(), slots, experts, block, counts.data_ptr(), sorted_ids.data_ptr(), block_expert.data_ptr(),
                  num_post.data_ptr(), L.stream_ptr()), "moe_sort")
-    return block, sorted_ids, block_expert, num_post
+    return order
 
 
 @torch.no_grad()
 def sparse_glu_experts(h: torch.Tensor, w_gate_up: torch.Tensor, w_down: torch.Tensor, ids: torch.Tensor,
-                       weights: torch.Tensor, *, limit: float | None = None, skipped_ids: bool = False) -> torch.Tensor:
+                       weights: torch.Tensor, *, limit: float | None = None, skipped_ids: bool = False, order=None) -> torch.Tensor:
     """Per slot (token, k): ``weights * down_e(silu(gate_e h) * up_e h)`` with ``e = ids[token, k]``; ``w_gate_up
     [experts, 2 ff, width]`` (gate rows, then up rows), ``w_down [experts, width, ff]``.  Returns the slots' rows
     ``[n, top, width]`` in the storage dtype (their sum over k is the caller's: the norm that follows adds them in fp32).
     Slots are sorted by expert on the device; every product accumulates in fp32.  ``limit``: the clamped pair
     ``g' sigmoid(1.702 g') (u' + 1)`` with ``g' = min(gate, limit)``, ``u' = clamp(up, -limit, limit)`` instead of
     ``silu(gate) up``.  ``skipped_ids``: some ids may lie beyond the experts (slots that no expert serves): their rows are
-    zeros."""
+    zeros.  ``order``: these slots as :func:`group_router` sorted them (for ``w_down`` and the same ``skipped``); by default they are sorted here."""
     L.require_cuda(h, w_gate_up, w_down, ids, weights)
     n, width = h.shape
     experts, two_ff, _ = w_gate_up.shape
@@ -361,7 +375,7 @@ def sparse_glu_experts(h: torch.Tensor, w_gate_up: torch.Tensor, w_down: torch.T
     lib = L.lib()
     slots = n * top
     run = skipped_ids and experts <= _SKIPPED_RUN    # (the last product writes the skipped slots' zeros)
-    block, sorted_ids, block_expert, num_post = _sort_slots(ids, slots, experts, width, ff, dt, run)
+    block, sorted_ids, block_expert, num_post = order or _sort_slots(ids, slots, experts, width, ff, dt, run)
     act = torch.empty(slots, ff, dtype=dt, device=h.device)
     out = (torch.zeros if skipped_ids and not run else torch.empty)(n, top, width, dtype=dt, device=h.device)
     code, st = L.dtype_code(dt), L.stream_ptr()
@@ -377,11 +391,12 @@ def sparse_glu_experts(h: torch.Tensor, w_gate_up: torch.Tensor, w_down: torch.T
 
 @torch.no_grad()
 def sparse_square_experts(h: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor, ids: torch.Tensor,
-                          weights: torch.Tensor) -> torch.Tensor:
+                          weights: torch.Tensor, order=None) -> torch.Tensor:
     """Per slot (token, k): ``down_e(relu(up_e (weights * h))^2)`` with ``e = ids[token, k]`` -- experts without a gate, whose weight
     multiplies their INPUT (it is applied to the fp32 sums of the first product, which are linear in the input).  ``w_up
     [experts, ff, width]``, ``w_down [experts, width, ff]``.  Returns the slots' rows ``[n, top, width]`` in the storage dtype (their
-    sum over k is the caller's).  Slots are sorted by expert on the device; every product accumulates in fp32."""
+    sum over k is the caller's).  Slots are sorted by expert on the device (``order``: by :func:`group_router` already); every product
+    accumulates in fp32."""
     L.require_cuda(h, w_up, w_down, ids, weights)
     n, width = h.shape
     experts, ff, _ = w_up.shape
@@ -394,7 +409,7 @@ def sparse_square_experts(h: torch.Tensor, w_up: torch.Tensor, w_down: torch.Ten
         raise ValueError("sparse_square_experts: int32 ids and fp32 weights [n, top]")
     lib = L.lib()
     slots = n * top
-    block, sorted_ids, block_expert, num_post = _sort_slots(ids, slots, experts, width, ff, dt)
+    block, sorted_ids, block_expert, num_post = order or _sort_slots(ids, slots, experts, width, ff, dt)
     act = torch.empty(slots, ff, dtype=dt, device=h.device)
     out = torch.empty(n, top, width, dtype=dt, device=h.device)
     code, st = L.dtype_code(dt), L.stream_ptr()

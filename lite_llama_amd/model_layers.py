@@ -844,9 +844,9 @@ class SparseMoE(nn.Module):
 
     def forward(self, h):
         s = self.spec
-        ids, weights, scale = group_router(h, self.router_weight, s.top, s.group_count, s.group_keep, s.route_scale,
-                                           extra_weight=self.shared_scale_weight if s.shared_ff else None)
-        y = sparse_glu_experts(h, self.gate_up_weight, self.down_weight, ids, weights)
+        ids, weights, scale, order = group_router(h, self.router_weight, s.top, s.group_count, s.group_keep, s.route_scale,
+                                                  extra_weight=self.shared_scale_weight if s.shared_ff else None, sort_for=self.down_weight)
+        y = sparse_glu_experts(h, self.gate_up_weight, self.down_weight, ids, weights, order=order)
         rows = self.in_proj(h) if (s.shared_ff or self.extra) else None
         shared = self.shared_down_proj(glu_act(rows, s.shared_ff, "silu")) if s.shared_ff else None
         return y, (rows[:, 2 * s.shared_ff:] if self.extra else None), shared, scale
@@ -907,8 +907,8 @@ class ChosenSoftmaxMoE(nn.Module):
         self.down_weight = nn.Parameter(torch.zeros(spec.experts, width, spec.ff, dtype=torch.float16), requires_grad=False)
 
     def forward(self, h):
-        ids, weights, _ = group_router(h, self.router_weight, self.spec.top, scoring=self.spec.scoring)
-        return sparse_glu_experts(h, self.gate_up_weight, self.down_weight, ids, weights)
+        ids, weights, _, order = group_router(h, self.router_weight, self.spec.top, scoring=self.spec.scoring, sort_for=self.down_weight)
+        return sparse_glu_experts(h, self.gate_up_weight, self.down_weight, ids, weights, order=order)
 
 
 class GroupSoftmaxMoE(ChosenSoftmaxMoE):
@@ -918,8 +918,9 @@ class GroupSoftmaxMoE(ChosenSoftmaxMoE):
 
     def forward(self, h):
         s = self.spec
-        ids, weights, _ = group_router(h, self.router_weight, s.top, s.group_count, s.group_keep, scoring=s.scoring)
-        return sparse_glu_experts(h, self.gate_up_weight, self.down_weight, ids, weights)
+        ids, weights, _, order = group_router(h, self.router_weight, s.top, s.group_count, s.group_keep, scoring=s.scoring,
+                                              sort_for=self.down_weight)
+        return sparse_glu_experts(h, self.gate_up_weight, self.down_weight, ids, weights, order=order)
 
 
 class GatedWindowAttention(nn.Module):
@@ -1138,9 +1139,10 @@ class CorrectedSoftmaxMoE(nn.Module):
 
     def forward(self, h):
         s = self.spec
-        ids, weights, own = group_router(h, self.router_weight, s.top, scoring=s.scoring, correction=self.correction,
-                                         identity=s.identity)
-        y = sparse_glu_experts(h, self.gate_up_weight, self.down_weight, ids, weights, limit=s.limit, skipped_ids=s.identity > 0)
+        skipped = s.identity > 0
+        ids, weights, own, order = group_router(h, self.router_weight, s.top, scoring=s.scoring, correction=self.correction,
+                                                identity=s.identity, sort_for=self.down_weight, skipped=skipped)
+        y = sparse_glu_experts(h, self.gate_up_weight, self.down_weight, ids, weights, limit=s.limit, skipped_ids=skipped, order=order)
         return y, None, (h if s.identity else None), own
 
 
@@ -1285,9 +1287,9 @@ class SquareMoE(nn.Module):
     def forward(self, h):
         """``(slots' rows [n, top, width], shared row or None, its scale or None)``."""
         s = self.spec
-        ids, weights, scale = group_router(h, self.router_weight, s.top, scoring=s.scoring,
-                                           extra_weight=self.shared_scale_weight if s.shared_ff else None)
-        y = sparse_square_experts(h, self.up_weight, self.down_weight, ids, weights)
+        ids, weights, scale, order = group_router(h, self.router_weight, s.top, scoring=s.scoring,
+                                                  extra_weight=self.shared_scale_weight if s.shared_ff else None, sort_for=self.down_weight)
+        y = sparse_square_experts(h, self.up_weight, self.down_weight, ids, weights, order=order)
         shared = self.shared_down_proj(relu_square(self.shared_up_proj(h), s.shared_ff)) if s.shared_ff else None
         return y, shared, scale
 

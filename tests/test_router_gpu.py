@@ -70,3 +70,31 @@ def test_the_largest_choices(scoring, experts, top):
     if scoring == "softmax_all":
         mine = torch.where(want >= experts - (1000 if experts > 1000 else 5), chosen, torch.zeros_like(chosen)).sum(-1)
         assert (own[clear].to(F64) - mine[clear]).abs().max() <= 2e-5
+
+
+@pytest.mark.parametrize("n,width,experts,top", [(1, 40, 5, 1), (1, 3072, 68, 8), (4, 2048, 34, 4), (5, 520, 34, 4), (31, 136, 130, 3), (32, 3080, 65, 4),
+                                                 (33, 264, 40, 4), (2, 520, 512, 9), (8, 72, 513, 2), (32, 64, 511, 64)])
+@pytest.mark.parametrize("scoring", ["sigmoid", "softmax_chosen", "softmax_all", "sigmoid_plain", "softmax_groups"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_choices_sorted_for_the_products_are_those_of_two_calls(n, width, experts, top, scoring, dtype):
+    """Bit for bit, on both sides of the largest step whose choices every expert's workgroup makes; slots in their order, every list's tail."""
+    from lite_llama_amd.kernels.fused_moe import _sort_slots, group_router
+
+    g = torch.Generator(device=DEV).manual_seed(n + width + experts)
+    h = torch.randn(n, width + 8, generator=g, device=DEV).to(dtype)[:, :width]
+    w = (torch.randn(experts, width, generator=g, device=DEV) * 2 * width ** -0.5).to(dtype)
+    identity = 2 if scoring == "softmax_all" and experts > 5 else 0
+    served = experts - identity
+    kw = {"scoring": scoring, "route_scale": 1.25}
+    if scoring == "softmax_all":
+        kw.update(correction=(torch.randn(experts, generator=g, device=DEV) * 0.02).to(dtype), identity=identity)
+    elif n % 2:
+        kw.update(extra_weight=(torch.randn(width, generator=g, device=DEV) * width ** -0.5).to(dtype))
+    ids, weights, extra = group_router(h, w, top, **kw)
+    block, srt, owner, post = _sort_slots(ids, n * top, served, width, 24, dtype, identity > 0)
+    got = group_router(h, w, top, sort_for=torch.empty(served, width, 24, dtype=dtype, device=DEV), skipped=identity > 0, **kw)
+    assert torch.equal(got[0], ids) and torch.equal(got[1], weights)
+    assert (extra is None and got[2] is None) or torch.equal(got[2], extra)
+    used = int(post)
+    assert got[3][0] == block and int(got[3][3]) == used
+    assert torch.equal(got[3][1][:used], srt[:used]) and torch.equal(got[3][2][:used // block], owner[:used // block])
