@@ -367,7 +367,7 @@ int ll_dense16_matmul(void* out, const void* x, const void* w, const void* bias,
 /* Round 5: the same product on the row-group loop (gemm_w16_rows.hip) -- every workgroup owns a run of 32-row groups and all of K,
  * weights and activations streamed through an LDS ring by LDS-DMA, finished outputs only (no planes, no finish launch).
  * epilogue 0: out [m][n] (+ bias); 1: the rows of w are (gate_j, up_j) pairs -> out [m][n / 2] = silu(gate) * up (swiglu_forward's
- * arithmetic on the rounded outputs).  m <= 64, n % 32 == 0, k % 128 == 0, element strides % 8 == 0. */
+ * arithmetic on the rounded outputs).  m <= 64, n % 16 == 0, n >= 32, k % 128 == 0, element strides % 8 == 0. */
 int ll_dense16_rows_supported(int64_t m, int64_t n, int64_t k, int epilogue); /* 1 / 0 */
 int ll_dense16_rows_matmul(void* out, const void* x, const void* w, const void* bias, int64_t m, int64_t n, int64_t k,
                            int64_t x_stride_m, int64_t w_stride_n, int dtype, int epilogue, void* stream);

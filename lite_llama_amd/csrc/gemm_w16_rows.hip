@@ -1,7 +1,7 @@
 // Decode-shaped F.linear for UNQUANTISED fp16 / bf16 weights [N][K] (M <= 64 rows): the row-group loop of gemm_w4_v4.hip without
 // a dequantiser.  Reference: lite_llama/models/quantization/methods/unquantized.py:21-22 and the lm_head of models/base.py:486-489
 // are torch's library GEMM; BASELINE config 2 (Qwen2.5-1.5B bf16, batch 32) has its fused gate|up and the lm_head there.
-//   * A workgroup owns a contiguous run of 32-row groups (N / 32 groups dealt over the CUs, sizes differing by at most one) and ALL
+//   * A workgroup owns a contiguous run of 32-row groups (or, r16_deal, of halves of them; runs differ by at most one) and ALL
 //     of K; it walks its run in tiles of up to 4 groups (WIDE: 8), of equal size to within one.  Finished outputs only: no
 //     split-K planes, no finish launch, bias or the fused swiglu of a row-interleaved gate|up in the epilogue (the decode engines'
 //     epilogue, common.h::ll_silu_mul_f32).
@@ -54,7 +54,8 @@ struct R16Params {
   const uint16_t* bias;
   int64_t m, n, k, x_stride, w_stride;
   int chunks;        // units of a row: its bytes / R16Lds::KB
-  int rbase, rrem;   // workgroup b owns row groups [b * rbase + min(b, rrem), + rbase + (b < rrem))
+  int piece;         // what is dealt out: 32-row groups (2) or halves of them (1)
+  int rbase, rrem;   // workgroup b owns pieces [b * rbase + min(b, rrem), + rbase + (b < rrem))
   int stagger;       // workgroup b begins a tile that many times b steps of 256 bytes into its rows
   int epi;           // 0: out[m, n] (+ bias);  1: rows are (gate_j, up_j) pairs -> out[m, n / 2] = silu(gate) * up
   const float* a_scale;  // R16_I8 only: per-token activation scales [m], per-channel weight scales [n] (smoothquant, w8a8.py:118-149)
@@ -84,12 +85,18 @@ __global__ __launch_bounds__((R16Lds<MT, WIDE>::THREADS)) __attribute__((amdgpu_
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int b = (int)blockIdx.x;
-  const int lo = b * p.rbase + (b < p.rrem ? b : p.rrem);
+  const int lo = (b * p.rbase + (b < p.rrem ? b : p.rrem)) * p.piece;   // in halves of a group, as are the tiles' sizes
   const int cnt = p.rbase + (b < p.rrem ? 1 : 0);
   if (cnt <= 0) return;
-  // (tiles of equal size to within one: a last tile of a group or two would walk the whole contraction with little on its way)
-  const int tiles = (cnt + GROUPS - 1) / GROUPS, tbase = cnt / tiles, trem = cnt - tbase * tiles;
+  // (tiles of equal size to within one piece: a last tile of a group or two would walk the whole contraction with little on its way)
+  const int most = p.piece == 2 ? GROUPS : 2 * GROUPS;
+  const int tiles = (cnt + most - 1) / most, tbase = cnt / tiles, trem = cnt - tbase * tiles;
   const int units = tiles * p.chunks;
+  const int halves = (int)(p.n >> 4);
+  auto sized = [&](int t, int first) {   // tile t's halves (N may end inside the last group)
+    const int s = (tbase + (t < trem ? 1 : 0)) * p.piece;
+    return first + s < halves ? s : halves - first;
+  };
 
   if (wv >= GROUPS) {
     // ======================================== loaders ======================================== //
@@ -110,23 +117,24 @@ __global__ __launch_bounds__((R16Lds<MT, WIDE>::THREADS)) __attribute__((amdgpu_
     }
     int xops = ((int)p.m - L * PER + 4 * PER - 1) / (4 * PER);   // this wave's activation operations that hold a row
     xops = xops < 0 ? 0 : xops;
-    int issued = 0, t = 0, size = tbase + (trem > 0 ? 1 : 0), done = 0, c = 0, ops = 0, before = 0;   // operations of the last unit and the one before it
+    int issued = 0, t = 0, first = lo, size = sized(0, lo), done = 0, c = 0, ops = 0, before = 0;   // operations of the last unit and the one before it
     if (p.stagger) {   // (WIDE units are half as long: two of them per step, so that a row's sum begins at the same column in either form)
       c = b * p.stagger % (p.chunks * KB / 256) * (256 / KB);
     }
     const size_t group = 32 * (size_t)p.w_stride * 2;
-    const char* wt = (const char*)p.w + (size_t)lo * group;   // the tile's rows
+    const char* wt = (const char*)p.w + (size_t)lo * (group / 2);   // the tile's rows
     uint32_t dst = 0;
     auto issue = [&]() {
       const char* wb = wt + (size_t)c * KB;
       const char* xb = (const char*)p.x + (size_t)c * KB;
 #pragma unroll
       for (int g = 0; g < GROUPS; ++g) {
-        if (g >= size) break;
+        if (2 * g + 1 >= size) break;
 #pragma unroll
         for (int q = 0; q < PG; ++q) v3_dma16<true>(dst + g * 32 * KB + (4 * q + L) * 1024, wb, woff[q]);
         wb += group;
       }
+      if ((size & 1) && (PG == 2 || L < 2)) v3_dma16<true>(dst + (size >> 1) * 32 * KB + L * 1024, wb, woff[0]);   // half a group: its first 16 rows
 #pragma unroll
       for (int j = 0; j < XP; ++j) {
         if (j >= xops) break;
@@ -134,12 +142,13 @@ __global__ __launch_bounds__((R16Lds<MT, WIDE>::THREADS)) __attribute__((amdgpu_
       }
       ++issued;
       before = ops;
-      ops = size * PG + xops;
+      ops = (PG == 2 ? size : (size + (L < 2 ? 1 : 0)) >> 1) + xops;
       if (++c == p.chunks) c = 0;
       if (++done == p.chunks) {
         done = 0;
-        wt += (size_t)size * group;
-        size = tbase + (++t < trem ? 1 : 0);
+        wt += (size_t)size * (group / 2);
+        first += size;
+        size = sized(++t, first);
       }
       dst = dst + LD::SLOT == R * LD::SLOT ? 0 : dst + LD::SLOT;
     };
@@ -173,12 +182,11 @@ __global__ __launch_bounds__((R16Lds<MT, WIDE>::THREADS)) __attribute__((amdgpu_
     bb = r[1];
   };
   const bool has_bias = p.bias != nullptr;
-  int t = 0, first = lo, size = tbase + (trem > 0 ? 1 : 0), c = 0;
+  int t = 0, first = lo, size = sized(0, lo), c = 0;
   uint32_t slot = 0;
   asm volatile("s_barrier" ::: "memory");  // P0: unit 0 has landed
   for (int u = 0; u < units; ++u) {
-    const int rg = first + wv;
-    const bool mine = wv < size;
+    const bool mine = 2 * wv < size, whole = 2 * wv + 1 < size;
     if (mine) {
       const unsigned char* wb = lds + slot + wrow;
       const unsigned char* xb = lds + slot + LD::W_BYTES + nl * KB;
@@ -204,11 +212,11 @@ __global__ __launch_bounds__((R16Lds<MT, WIDE>::THREADS)) __attribute__((amdgpu_
       c = 0;
       if (mine) {
         // a lane holds, for batch row nl (+ 32 mt), the weight rows 8g + 4h .. + 3 of the group: the decode engines' epilogue
-        const int64_t ncol = (int64_t)rg * 32;
+        const int64_t ncol = (int64_t)(first + 2 * wv) * 16;
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
           const int64_t mrow = nl + mt * 32;
-          const bool row_ok = mrow < p.m;
+          const bool row_ok = mrow < p.m, store = row_ok && (whole || h == 0);
           float v[16];
           if constexpr (DT == R16_I8) {
             // (acc.f32 * a_scale[m]) * w_scale[n], each product rounded to fp32 before the next (w8a8.py:118-120): pinned so that
@@ -216,7 +224,7 @@ __global__ __launch_bounds__((R16Lds<MT, WIDE>::THREADS)) __attribute__((amdgpu_
             const float as = p.a_scale[row_ok ? mrow : 0];
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-              const f32x4 ws = *reinterpret_cast<const f32x4*>(p.w_scale + ncol + 8 * g + 4 * h);
+              const f32x4 ws = *reinterpret_cast<const f32x4*>(p.w_scale + ncol + 8 * (whole ? g : g & 1) + 4 * h);   // (rows that are not there: any that are)
 #pragma unroll
               for (int e = 0; e < 4; ++e) {
                 float f = ((float)iacc[mt][4 * g + e] * as) * ws[e];
@@ -231,7 +239,7 @@ __global__ __launch_bounds__((R16Lds<MT, WIDE>::THREADS)) __attribute__((amdgpu_
           if (has_bias) {
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-              const uint2 bb = *reinterpret_cast<const uint2*>(p.bias + ncol + 8 * g + 4 * h);
+              const uint2 bb = *reinterpret_cast<const uint2*>(p.bias + ncol + 8 * (whole ? g : g & 1) + 4 * h);
               v[4 * g + 0] += to_f32<ODT>((uint16_t)(bb.x & 0xffffu));
               v[4 * g + 1] += to_f32<ODT>((uint16_t)(bb.x >> 16));
               v[4 * g + 2] += to_f32<ODT>((uint16_t)(bb.y & 0xffffu));
@@ -258,13 +266,13 @@ __global__ __launch_bounds__((R16Lds<MT, WIDE>::THREADS)) __attribute__((amdgpu_
           if (p.epi) {
             swap32(sw[0], sw[2]);
             swap32(sw[1], sw[3]);
-            if (row_ok) *reinterpret_cast<u32x4*>(p.out + mrow * (p.n >> 1) + (nn >> 1)) = u32x4{sw[0], sw[2], sw[1], sw[3]};
+            if (store) *reinterpret_cast<u32x4*>(p.out + mrow * (p.n >> 1) + (nn >> 1)) = u32x4{sw[0], sw[2], sw[1], sw[3]};
           } else {
             swap32(lo2[0], lo2[2]);
             swap32(hi2[0], hi2[2]);
             swap32(lo2[1], lo2[3]);
             swap32(hi2[1], hi2[3]);
-            if (row_ok) {
+            if (store) {
               *reinterpret_cast<u32x4*>(p.out + mrow * p.n + nn) = u32x4{lo2[0], hi2[0], lo2[2], hi2[2]};
               *reinterpret_cast<u32x4*>(p.out + mrow * p.n + nn + 8) = u32x4{lo2[1], hi2[1], lo2[3], hi2[3]};
             }
@@ -274,7 +282,7 @@ __global__ __launch_bounds__((R16Lds<MT, WIDE>::THREADS)) __attribute__((amdgpu_
         }
       }
       first += size;
-      size = tbase + (++t < trem ? 1 : 0);
+      size = sized(++t, first);
     }
   }
 }
@@ -288,6 +296,23 @@ static int r16_num_cus() {
     cus[dev] = hipGetDeviceProperties(&prop, dev) == hipSuccess && prop.multiProcessorCount > 0 ? prop.multiProcessorCount : 256;
   }
   return cus[dev];
+}
+
+// Deals n / 16 halves of 32-row groups out to the CUs: in groups, or in halves where a few workgroups would have a group more than the rest -- they
+// take that much longer -- and where rows keep the column that their workgroup begins at.  us, groups -> halves, 6 / 32 rows: 8224 x 2048 11.3 -> 11.0 /
+// 12.1 -> 11.7, 9248 x 3072 15.2 -> 14.4 / 17.3 -> 15.9, 9216 x 4096 21.2 -> 20.0 / 22.9 -> 20.9, 17920 x 1536 13.9 -> 13.4 / 14.4 -> 13.9; where more
+// than a third of the workgroups has one group more, 11264 x 2048 12.9 -> 13.1 / 13.8 -> 13.6, and below a group per CU, 4096 x 2048 8.9 -> 9.2 /
+// 9.2 -> 9.5: groups.  Returns the workgroups.
+static int r16_deal(R16Params& p, int* groups) {
+  const int cus = r16_num_cus();
+  const int64_t halves = p.n / 16, rgs = (halves + 1) / 2;
+  const bool few = rgs > cus && rgs % cus > 0 && rgs % cus <= cus / 3;
+  p.piece = few && (halves + cus - 1) / cus < (rgs + cus - 1) / cus * 2 && !p.stagger ? 1 : 2;
+  const int64_t pieces = p.piece == 1 ? halves : rgs;
+  const int grid = (int)(pieces < cus ? pieces : cus);
+  p.rbase = (int)(pieces / grid); p.rrem = (int)(pieces % grid);
+  *groups = (int)((p.rbase + (p.rrem > 0)) * p.piece + 1) / 2;   // of the fullest workgroup
+  return grid;
 }
 
 // the row-group loop needs R16Lds::BYTES of LDS per workgroup (160 KB at MT = 1): callers fall back when the device's opt-in
@@ -304,13 +329,13 @@ static bool r16_lds_fits(int64_t m) {
 }
 
 extern "C" int ll_dense16_rows_supported(int64_t m, int64_t n, int64_t k, int epilogue) {
-  if (m < 1 || m > 64 || n < 32 || n % 32 != 0 || k < 128 || k % 128 != 0) return 0;
+  if (m < 1 || m > 64 || n < 32 || n % 16 != 0 || k < 128 || k % 128 != 0) return 0;
   if (epilogue != 0 && epilogue != 1) return 0;
   return r16_lds_fits(m) ? 1 : 0;
 }
 
 // out [m][n] (epilogue 0, + bias) or [m][n / 2] (epilogue 1: rows of w interleaved (gate_j, up_j)) = x [m][k] @ w [n][k]^T for an
-// unquantised fp16 / bf16 weight; m <= 64, n % 32 == 0, k % 128 == 0, rows 16-byte aligned.  Returns LL_OK, or an error code.
+// unquantised fp16 / bf16 weight; m <= 64, n % 16 == 0, k % 128 == 0, rows 16-byte aligned.  Returns LL_OK, or an error code.
 extern "C" int ll_dense16_rows_matmul(void* out, const void* x, const void* w, const void* bias, int64_t m, int64_t n, int64_t k,
                                       int64_t x_stride_m, int64_t w_stride_n, int dtype, int epilogue, void* stream) {
   if (dtype != LL_F16 && dtype != LL_BF16) return LL_ERR_DTYPE;
@@ -324,11 +349,9 @@ extern "C" int ll_dense16_rows_matmul(void* out, const void* x, const void* w, c
   p.m = m; p.n = n; p.k = k; p.x_stride = x_stride_m; p.w_stride = w_stride_n;
   p.stagger = w_stride_n % 2048 == 0 && n * k * 2 >= (1ll << 28);
   p.epi = epilogue;
-  const int64_t rgs = n / 32;
-  int grid = r16_num_cus();
-  if (grid > rgs) grid = (int)rgs;
-  p.rbase = (int)(rgs / grid); p.rrem = (int)(rgs % grid);
-  const bool wide = m > 32 && rgs > 4 * (int64_t)grid;
+  int groups = 0;
+  const int grid = r16_deal(p, &groups);
+  const bool wide = m > 32 && groups > 4;
   p.chunks = (int)(k * 2 / (wide ? 128 : 256));
   hipStream_t st = (hipStream_t)stream;
 #define R16_GO(MT, DT, WIDE)                                                                                                   \
@@ -378,11 +401,9 @@ extern "C" int ll_w8a8_rows_matmul(void* out, const int8_t* qa, const float* a_s
   p.x_stride = qa_stride_m / 2; p.w_stride = qw_stride_n / 2;  // the kernel addresses rows in 2-byte units
   p.stagger = qw_stride_n % 4096 || n * k < (1ll << 26) ? 0 : n * k < (1ll << 28) ? 5 : 1;
   p.epi = epilogue;
-  const int64_t rgs = n / 32;
-  int grid = r16_num_cus();
-  if (grid > rgs) grid = (int)rgs;
-  p.rbase = (int)(rgs / grid); p.rrem = (int)(rgs % grid);
-  const bool wide = m > 32 && rgs > 4 * (int64_t)grid;
+  int groups = 0;
+  const int grid = r16_deal(p, &groups);
+  const bool wide = m > 32 && groups > 4;
   p.chunks = (int)(k / (wide ? 128 : 256));
   hipStream_t st = (hipStream_t)stream;
 #define R16_GO8(MT, WIDE)                                                                                                      \

@@ -580,6 +580,16 @@ def dense16_rows_wins(m: int, n: int, k: int) -> bool:
     return 1 <= m <= 64 and n >= 8192 and n % 32 == 0 and k % 128 == 0
 
 
+def dense16_rows_narrower_wins(m: int, n: int, k: int) -> bool:
+    """... and of rows that end inside a 32-row group, or too few for a group per CU, on contractions short enough (us per launch rows /
+    library, bf16, hipGraph replays over rotating weights): 12080 x 3072 6 rows 16.8 / 22.0, 32 rows 16.9 / 19.6, 48 rows 19.4 / 21.7, 64 rows
+    22.9 / 22.0; 6176 x 2048 32 rows 9.9 / 13.0, 48 rows 12.9 / 13.6; 4096 x 2048 32 rows 9.5 / 12.0, 48 rows 12.5 / 12.3; 5120 x 1024 32 rows
+    6.7 / 11.7; 7168 x 3072 6 rows 12.9 / 13.3, 32 rows 13.2 / 14.0; 6144 x 3072 16 rows 12.7 / 12.7, 4096 x 3072 32 rows 12.2 / 11.3,
+    6144 x 4096 32 rows 16.5 / 16.4."""
+    wide = n >= 8192 or (k <= 3072 and n >= 7168) or (k <= 2048 and n >= (4096 if m <= 32 else 5120))
+    return 1 <= m <= 48 and wide and n % 16 == 0 and k % 128 == 0
+
+
 def _on_one_device(x: torch.Tensor, weight: torch.Tensor, bias) -> bool:
     """Whether all operands are where ``x`` is: a kernel is handed their addresses, whatever they point at."""
     here = x.device

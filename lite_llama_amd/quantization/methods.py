@@ -17,7 +17,7 @@ import torch.nn.functional as F
 from ..kernels import fused_moe, smoothquant_matmul, w4a16_matmul, w8a16_matmul
 from ..kernels.quantization import (smoothquant_gate_up_swiglu, smoothquant_matmul_partials, smoothquant_prefill_swiglu,
                                      smoothquant_rows_matmul)
-from ..kernels.quantization import (dense16_linear, dense16_narrow_linear, dense16_rows_linear, dense16_rows_wins, dense_matmul_partials, pack_w4a16_scales, pack_w4a16_weights, unpack_w4a16_weights, w4a16_matmul_partials,
+from ..kernels.quantization import (_is_followed as is_followed, dense16_linear, dense16_narrow_linear, dense16_rows_linear, dense16_rows_narrower_wins, dense16_rows_wins, dense_matmul_partials, pack_w4a16_scales, pack_w4a16_weights, unpack_w4a16_weights, w4a16_matmul_partials,
                                     w4a16_matmul_prepacked_rows, w4a16_mtiled_supported,
                                     w4a16_matmul_prepacked, w4a16_prepacked_supported)
 from .config import FP8, INT4, INT8, SMOOTHQUANT, QuantConfig
@@ -72,6 +72,11 @@ class UnquantizedLinearMethod(LinearQuantMethod):
             out = dense16_rows_linear(x, layer.weight, layer.bias)
             if out is not None:
                 return out
+        elif dense16_rows_narrower_wins(m, layer.weight.shape[0], layer.weight.shape[1]) and not is_followed(x, layer.weight, layer.bias):
+            if layer.bias is None or (layer.bias.is_contiguous() and layer.bias.data_ptr() % 8 == 0):
+                out = dense16_rows_linear(x, layer.weight, layer.bias)
+                if out is not None:
+                    return out
         out = dense16_linear(x, layer.weight, layer.bias, policy="auto")  # decode shapes where the own kernel measured faster
         return out if out is not None else F.linear(x, layer.weight, layer.bias)
 

@@ -114,3 +114,26 @@ def test_staggered_int8_rows_in_all_tiles(m, n, k):
     qa, each = quantize_activations_int8(x)
     sums = torch.cat([qa.double() @ part.double().T for part in w.split(8192)], dim=1).float()   # (whole numbers: one value, whatever the order)
     assert torch.equal(smoothquant_rows_matmul(x, w, scale), ((sums * each.view(-1, 1)) * scale.view(1, -1)).half())
+
+
+# (rows of weights, contraction): half a group at the end, runs dealt in halves (a CU with three), both, one workgroup
+@pytest.mark.parametrize("n,k", [(48, 128), (8208, 128), (8224, 256), (12080, 384), (17936, 128), (4112, 640)])
+@pytest.mark.parametrize("m", [1, 32, 33, 64])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_halves_of_row_groups(n, k, m, dtype):
+    from lite_llama_amd.kernels.quantization import dense16_rows_linear
+
+    g = torch.Generator(device=DEV).manual_seed(n + m)
+    x = torch.randn(m, k, generator=g, device=DEV).to(dtype)
+    w = (torch.randn(n, k, generator=g, device=DEV) * k ** -0.5).to(dtype)
+    bias = torch.randn(n + 16, generator=g, device=DEV).to(dtype)[:n]
+    # exact 16-bit products summed in fp32 (k 2^-24 of their magnitudes' sum, which stays below 40 deviations), rounded once
+    unit, slack = 2.0 ** (-11 if dtype == torch.float16 else -8), k * 2.0 ** -24 * 40 + 2.0 ** -24
+    want = x.double() @ w.double().T + bias.double()
+    got = dense16_rows_linear(x, w, bias)
+    assert ((got.double() - want).abs() <= unit * want.abs() + slack).all()
+    plain = dense16_rows_linear(x, w)
+    pairs = dense16_rows_linear(x, w, gate_up_swiglu=True)
+    gate, up = plain[:, 0::2].double(), plain[:, 1::2].double()
+    act = torch.nn.functional.silu(gate) * up
+    assert ((pairs.double() - act).abs() <= unit * act.abs() + 2.0 ** -20 * (gate * up).abs() + 2.0 ** -24).all()
