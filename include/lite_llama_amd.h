@@ -831,6 +831,13 @@ int ll_moe_rows_gemm(const void* a, int64_t a_ld, int64_t a_div, const void* w, 
                      const int32_t* block_expert, const int32_t* num_post, int64_t num_slots, int64_t experts, int64_t block,
                      float limit, int dtype, void* stream);
 
+/* ---- one layer of a step of decoded tokens (csrc/layered_decode.hip) -----------------------------------------------------------
+ * The launches of a layer whose norms sit on its sublayers' results, from two packed arrays (the fields of LayeredDecode and
+ * LayeredDecodeFloats in their order).  ..._bytes: scratch of such a call, or 0 where a part of it is not served. */
+int64_t ll_layered_decode_bytes(const int64_t* args, int64_t count, const double* floats, int64_t float_count);
+int ll_layered_decode(const int64_t* args, int64_t count, const double* floats, int64_t float_count, void* scratch, int64_t bytes,
+                      void* stream);
+
 /* ---- linear attention with a decay, and what stands around it (csrc/linear_mix.hip) -----------------------------------------
  * ll_linear_scan: per head S_t = diag(a_t) S_(t-1) + k_t (b_t v_t)^T, o_t = S_t^T q_t (+ skip_h v_t), fp32 state
  * [slots, heads, dk, dv]; value head h reads query / key head h / qk_rep of rows q / k (strides q_ld / k_ld), its values at

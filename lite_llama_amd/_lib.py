@@ -7,6 +7,7 @@ this module raises, loudly.  Build it with ``python -m lite_llama_amd.build``.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 from ctypes import c_float, c_int, c_int64, c_void_p
 
@@ -157,6 +158,8 @@ SIGNATURES = {
     "ll_moe_sort": [P, L, L, L, P, P, P, P, P],
     "ll_moe_sort_skipped": [P, L, L, L, P, P, P, P, P],
     "ll_moe_rows_gemm": [P, L, L, P, L, L, L, I, P, P, L, P, P, P, L, L, L, F, I, P],
+    "ll_layered_decode_bytes": [P, L, P, L],
+    "ll_layered_decode": [P, L, P, L, P, L, P],
     "ll_linear_scan_supported": [L, L],
     "ll_linear_scan": [P, L, P, L, P, L, L, L, L, L, I, I, F, P, P, L, P, F, P, L, P, P, P, P, L, P, P, P, P, P, L, L, I, P],
     "ll_linear_scan_walk_floats": [L, L, L, L, L, L, I, L],
@@ -174,7 +177,7 @@ SIGNATURES = {
     "ll_stream_norm": [P, L, L, P, P, L, P, P, P, P, P, P, P, F, F, P, L, L, L, I, P],
 }
 
-_RETURNS_I64 = {"ll_tile256_split_bytes", "ll_linear_scan_walk_floats", "ll_rglru_scan_scratch_floats", "ll_delta_scan_scratch_floats", "ll_ragged_attention_partition", "ll_mingru_scan_scratch_floats", "ll_moe_rows_block", "ll_kv_alloc_scratch_bytes", "ll_tp_oneshot_flag_words", "ll_moe_router_workspace_floats", "ll_moe_align_workspace_ints"}
+_RETURNS_I64 = {"ll_tile256_split_bytes", "ll_layered_decode_bytes", "ll_linear_scan_walk_floats", "ll_rglru_scan_scratch_floats", "ll_delta_scan_scratch_floats", "ll_ragged_attention_partition", "ll_mingru_scan_scratch_floats", "ll_moe_rows_block", "ll_kv_alloc_scratch_bytes", "ll_tp_oneshot_flag_words", "ll_moe_router_workspace_floats", "ll_moe_align_workspace_ints"}
 _lib = None
 
 
@@ -229,6 +232,18 @@ def stream_ptr(index: int | None = None) -> int:
     """The current stream of the device ``index`` (the current device).  The handle straight from the runtime: building a
     ``torch.cuda.Stream`` around it costs about 5 us, on every launch."""
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+
+
+def without_grad(fn):
+    """``torch.no_grad()`` around ``fn``, entered only where gradients are on: under a model's own ``no_grad`` a launch does not pay the 2 us
+    again."""
+    @functools.wraps(fn)
+    def call(*args, **kwargs):
+        if not torch.is_grad_enabled():
+            return fn(*args, **kwargs)
+        with torch.no_grad():
+            return fn(*args, **kwargs)
+    return call
 
 
 def dtype_code(dt: torch.dtype) -> int:

@@ -20,27 +20,27 @@ def _apply(x: torch.Tensor, kind: int, what: str) -> torch.Tensor:
     return y.view(x.shape)
 
 
-@torch.no_grad()
+@L.without_grad
 def relu(x):
     return _apply(x, 0, "relu")
 
 
-@torch.no_grad()
+@L.without_grad
 def leaky_relu(x):
     return _apply(x, 1, "leaky_relu")
 
 
-@torch.no_grad()
+@L.without_grad
 def tanh(x):
     return _apply(x, 2, "tanh")
 
 
-@torch.no_grad()
+@L.without_grad
 def gelu(x):
     return _apply(x, 3, "gelu")
 
 
-@torch.no_grad()
+@L.without_grad
 def xielu(z: torch.Tensor, pq: torch.Tensor) -> torch.Tensor:
     """xIELU with its two learned numbers ``pq = (p, q)``: ``softplus(p) z^2 + z / 2`` for ``z > 0``, else
     ``(1/2 + softplus(q)) (exp(z) - 1 - z) + z / 2``; fp32 arithmetic, one rounding to the storage dtype (fp16 / bf16 / fp32)."""

@@ -37,7 +37,7 @@ def _merge_counters(device, entries: int):
     return _grow_counters(key, device, entries)
 
 
-@torch.no_grad()
+@L.without_grad
 def flash_decoding(
     q,
     k_cache,
@@ -88,7 +88,7 @@ def flash_decoding(
     return out
 
 
-@torch.no_grad()
+@L.without_grad
 def flash_decoding_fp8kv(q, k_cache, v_cache, qk_scale, b_req_tokens_table, b_req_idx, b_seq_len, max_actual_seq_len,
                          k_scale: float = 1.0, v_scale: float = 1.0):
     """``flash_decoding`` over an fp8 (OCP e4m3) pool written by ``update_kv_buffer_fp8`` (extension): ``k_cache`` /
@@ -134,7 +134,7 @@ def decode_attention_supported(q, kv, cos, n_kv_heads: int) -> bool:
             and q.dtype in (torch.float16, torch.bfloat16) and q.stride(0) % 8 == 0 and kv.stride(0) % 8 == 0)
 
 
-@torch.no_grad()
+@L.without_grad
 def _head_norm_ok(qk_norm, head_dim: int, dtype) -> bool:
     if qk_norm is None:
         return True
@@ -143,7 +143,7 @@ def _head_norm_ok(qk_norm, head_dim: int, dtype) -> bool:
                                     for w in (qw, kw)))
 
 
-@torch.no_grad()
+@L.without_grad
 def decode_attention(q, kv, cos_table, sin_table, positions, select_index, kv_buffer, qk_scale, b_req_tokens_table,
                      b_req_idx, b_seq_len, max_actual_seq_len, qk_norm=None):
     """Extension: ``rope_and_cache(q, kv, tables, positions)`` + ``flash_decoding(...)`` in ONE launch
@@ -206,7 +206,7 @@ def _partials_waves(max_len: int, num_heads: int, num_kv_heads: int, head_dim: i
     return waves if (rep + 2) * head_dim // 4 <= 128 * waves else 0
 
 
-@torch.no_grad()
+@L.without_grad
 def decode_attention_partials(parts, bias, num_heads: int, num_kv_heads: int, head_dim: int, cos_table, sin_table,
                               positions, select_index, kv_buffer, qk_scale, b_req_tokens_table, b_req_idx, b_seq_len,
                               max_actual_seq_len, qk_norm=None):
@@ -267,7 +267,7 @@ def decode_attention_partials(parts, bias, num_heads: int, num_kv_heads: int, he
     return out
 
 
-@torch.no_grad()
+@L.without_grad
 def flash_attention2_no_pad(q, k, v, sm_scale, b_start_loc, b_seq_len, max_seq_len):
     """Varlen causal prefill attention (``sm_scale`` must already include log2(e); the
     kernel evaluates exp2).  fp32 inputs are cast to fp16 like the reference's
@@ -300,7 +300,7 @@ def flash_attention2_no_pad(q, k, v, sm_scale, b_start_loc, b_seq_len, max_seq_l
 # ------------------------------------------------------------------------------------- #
 # ragged steps against a paged cache with separate key / value widths (csrc/ragged_attn.hip)
 # ------------------------------------------------------------------------------------- #
-@torch.no_grad()
+@L.without_grad
 def qk_norm_cache(qkv, heads: int, kv_heads: int, dk: int, dv: int, q_weight, k_weight, eps: float, temp_coef: float,
                   temp_every: int, step, k_cache, v_cache):
     """Fused projection rows ``[q | k | v]`` -> queries ``[n, heads, dk]`` (per-head RMS norm, then the position temperature
@@ -325,7 +325,7 @@ def qk_norm_cache(qkv, heads: int, kv_heads: int, dk: int, dv: int, q_weight, k_
     return q
 
 
-@torch.no_grad()
+@L.without_grad
 def rotation_table(step, freq, pairs: int, amp: float = 1.0):
     """fp32 ``[n, 2 * pairs4]`` (``pairs4``: ``pairs`` rounded up to a multiple of 4, the padding zero): per token of the step and
     entry pair ``(cos(position * freq[i]) * amp, sin(position * freq[i]) * amp)``."""
@@ -338,7 +338,7 @@ def rotation_table(step, freq, pairs: int, amp: float = 1.0):
     return out
 
 
-@torch.no_grad()
+@L.without_grad
 def conv_rope_cache(qkv, heads: int, kv_heads: int, dk: int, dv: int, step, k_cache, v_cache, *, bias=None, conv_weight=None,
                     conv_state=None, freq=None, pairs: int = 0, amp: float = 1.0, unit_norm: bool = False, eps: float = 0.0,
                     v_source=None, v_blend=None, rot_table=None):
@@ -393,7 +393,7 @@ def conv_rope_cache(qkv, heads: int, kv_heads: int, dk: int, dv: int, step, k_ca
     return q
 
 
-@torch.no_grad()
+@L.without_grad
 def rownorm_rope_cache(qkv, heads: int, kv_heads: int, dk: int, dv: int, step, k_cache, v_cache, *, q_weight=None, k_weight=None,
                        eps: float = 0.0, freq=None, pairs: int = 0, value_scale: float = 1.0):
     """Fused projection rows ``[q | k | v]`` -> queries ``[n, heads, dk]``; keys and values land in the cache rows
@@ -423,7 +423,7 @@ def rownorm_rope_cache(qkv, heads: int, kv_heads: int, dk: int, dv: int, step, k
     return q
 
 
-@torch.no_grad()
+@L.without_grad
 def ragged_attention(q, k_cache, v_cache, scale: float, step, token_table, sink=None, window: int = 0, keep_first: int = 0,
                      out=None, cap: float = 0.0, dist_bias=None, head_gate=None):
     """Causal softmax attention of every token of a ragged step against positions ``0 .. its own`` of its sequence, keys and
@@ -494,7 +494,7 @@ def ragged_attention(q, k_cache, v_cache, scale: float, step, token_table, sink=
 # ------------------------------------------------------------------------------------- #
 # attention over a shared latent (csrc/latent_attn.hip): what surrounds the projections
 # ------------------------------------------------------------------------------------- #
-@torch.no_grad()
+@L.without_grad
 def latent_kv_prep(rows, kv_off: int, rank: int, rot: int, kv_norm_weight, eps: float, freq, pairs: int, amp: float, step, cache,
                    q_off: int = 0, q_rank: int = 0, q_norm_weight=None):
     """Rows of the fused input projection hold the key/value latent ``[rank]`` followed by the shared rotated key part
@@ -520,7 +520,7 @@ def latent_kv_prep(rows, kv_off: int, rank: int, rot: int, kv_norm_weight, eps: 
     return q_out
 
 
-@torch.no_grad()
+@L.without_grad
 def rotate_pairs(q, q_off: int, rot: int, freq, pairs: int, amp: float, step, out, out_off: int):
     """``q [n, heads, w]`` (unit inner stride): the ``rot`` entries at ``q_off`` of every head, rotated pair by pair at the
     token's position, land at ``out[n, heads, w'][..., out_off : out_off + rot]`` (``out`` contiguous; it may be ``q`` itself

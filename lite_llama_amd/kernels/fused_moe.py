@@ -218,7 +218,7 @@ def fused_moe(
     return out
 
 
-@torch.no_grad()
+@L.without_grad
 def moe_route_topk(router_logits: torch.Tensor, top_k: int, norm_topk_prob: bool = True):
     """Extension (decode-step launch count): the router's tail -- fp32 softmax over all experts, top-k, optional
     renormalisation, cast to the activation dtype (models/qwen3_moe.py:95-100) -- as ONE launch instead of four tensor
@@ -237,7 +237,7 @@ def moe_route_topk(router_logits: torch.Tensor, top_k: int, norm_topk_prob: bool
     return w, ids
 
 
-@torch.no_grad()
+@L.without_grad
 def moe_router(x: torch.Tensor, gate_weight: torch.Tensor, top_k: int, norm_topk_prob: bool = True, align_block: int = 0):
     """Extension (round 6): the WHOLE router of a decode batch without a library GEMM -- ``F.linear(x, gate_weight)`` (the
     reference's unquantised fp16 gate, models/qwen3_moe.py:102-111) as split-K fp32 planes from a grid of one-wave MFMA
@@ -278,7 +278,7 @@ def moe_router(x: torch.Tensor, gate_weight: torch.Tensor, top_k: int, norm_topk
 # ------------------------------------------------------------------------------------- #
 # sigmoid router over expert groups + grouped expert products for 16-bit and 32-bit storage (csrc/moe_sparse.hip)
 # ------------------------------------------------------------------------------------- #
-@torch.no_grad()
+@L.without_grad
 def group_router(h: torch.Tensor, router_weight: torch.Tensor, top: int, group_count: int = 1, group_keep: int = 1,
                  route_scale: float = 1.0, extra_weight: torch.Tensor | None = None, scoring: str = "sigmoid",
                  correction: torch.Tensor | None = None, identity: int = 0, sort_for: torch.Tensor | None = None, skipped: bool = False):
@@ -351,7 +351,7 @@ def _sort_slots(ids: torch.Tensor, slots: int, experts: int, width: int, ff: int
     return order
 
 
-@torch.no_grad()
+@L.without_grad
 def sparse_glu_experts(h: torch.Tensor, w_gate_up: torch.Tensor, w_down: torch.Tensor, ids: torch.Tensor,
                        weights: torch.Tensor, *, limit: float | None = None, skipped_ids: bool = False, order=None) -> torch.Tensor:
     """Per slot (token, k): ``weights * down_e(silu(gate_e h) * up_e h)`` with ``e = ids[token, k]``; ``w_gate_up
@@ -389,7 +389,7 @@ def sparse_glu_experts(h: torch.Tensor, w_gate_up: torch.Tensor, w_down: torch.T
     return out
 
 
-@torch.no_grad()
+@L.without_grad
 def sparse_square_experts(h: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor, ids: torch.Tensor,
                           weights: torch.Tensor, order=None) -> torch.Tensor:
     """Per slot (token, k): ``down_e(relu(up_e (weights * h))^2)`` with ``e = ids[token, k]`` -- experts without a gate, whose weight

@@ -8,7 +8,7 @@ import torch
 from .. import _lib as L
 
 
-@torch.no_grad()
+@L.without_grad
 def update_kv_buffer(KV_Values, Select_Index, KV_Buffer):
     """``KV_Buffer[Select_Index[i], :, :] = KV_Values[i, :, :]``; other rows untouched."""
     L.require_cuda(KV_Values, Select_Index, KV_Buffer)
@@ -32,7 +32,7 @@ def update_kv_buffer(KV_Values, Select_Index, KV_Buffer):
 FP8_KV_DTYPES = (torch.uint8, torch.float8_e4m3fn)
 
 
-@torch.no_grad()
+@L.without_grad
 def update_kv_buffer_fp8(KV_Values, Select_Index, KV_Buffer, num_k_heads: int, k_scale: float = 1.0, v_scale: float = 1.0):
     """``update_kv_buffer`` into an fp8 (OCP e4m3) pool (extension): ``KV_Buffer[Select_Index[i]] = e4m3(KV_Values[i] /
     scale)`` with ``k_scale`` for the first ``num_k_heads`` heads of a row and ``v_scale`` for the rest; values are
@@ -54,7 +54,7 @@ def update_kv_buffer_fp8(KV_Values, Select_Index, KV_Buffer, num_k_heads: int, k
     )
 
 
-@torch.no_grad()
+@L.without_grad
 def update_kv_index(req_to_token_indexs, b_req_idx, b_seq_len, select_index):
     """``table[b_req_idx[i], b_seq_len[i] - 1] = select_index[i]``."""
     L.require_cuda(req_to_token_indexs, b_req_idx, b_seq_len, select_index)
@@ -74,7 +74,7 @@ def update_kv_index(req_to_token_indexs, b_req_idx, b_seq_len, select_index):
     return
 
 
-@torch.no_grad()
+@L.without_grad
 def pack_prompts(input_ids, position_ids, select_index, b_seq_len, total: int, rows):
     """Prompts on a padded grid ``[batch, longest]`` -> the tokens of all prompts one after the other (``total`` = the sum of their
     lengths): ``(ids [1, total], positions [1, total], select_index [total], starts int32 [batch], lengths int64 [batch], rows)``, with

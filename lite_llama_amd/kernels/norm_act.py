@@ -23,7 +23,7 @@ def _check_row(n: int) -> None:
         )
 
 
-@torch.no_grad()
+@L.without_grad
 def skip_rmsnorm(X, residual, weight, eps=1e-5):
     """``(Y, residual)``: residual is updated IN PLACE with ``x + residual`` and returned
     (same storage); ``residual=None`` -> plain RMSNorm, returns ``(Y, X)``."""
@@ -91,7 +91,7 @@ class EmbeddedRows:
                 and table.shape[1] % 8 == 0 and 0 < table.shape[1] <= 8192 and table.data_ptr() % 16 == 0 and L.has("ll_embed_rmsnorm_q8"))
 
 
-@torch.no_grad()
+@L.without_grad
 def embed_rmsnorm(X: EmbeddedRows, weight, eps=1e-5, *, q8: bool = False):
     """``skip_rmsnorm(table[ids], None, weight)`` -- with ``q8`` ``skip_rmsnorm_q8`` -- in one launch: ``(Y | Int8Rows, residual)``."""
     n, rows = X.table.shape[1], X.ids.numel()
@@ -203,7 +203,7 @@ class ScaledInt32Partials(PartialSums):
         return out.to(self.dtype).view(self.shape)
 
 
-@torch.no_grad()
+@L.without_grad
 def skip_rmsnorm_q8(X, residual, weight, eps=1e-5, *, quantize: bool = True, keep_y: bool = False):
     """:func:`skip_rmsnorm` of a smoothquant block in ONE launch (csrc/w8a8_fused.hip): ``X`` is an fp16 tensor or the
     :class:`ScaledInt32Partials` of the previous W8A8 projection (its scale epilogue runs here); with ``quantize`` the
@@ -255,7 +255,7 @@ def skip_rmsnorm_q8(X, residual, weight, eps=1e-5, *, quantize: bool = True, kee
     return (rows if quantize else Y.view(shape)), res_out
 
 
-@torch.no_grad()
+@L.without_grad
 def skip_rmsnorm_partials(X: PartialSums, residual, weight, eps=1e-5):
     """:func:`skip_rmsnorm` over a :class:`PartialSums` input: ``x = fp16(sum of the partials)`` -- the value the
     projection itself would have stored -- then the same add-and-normalise.  ``residual`` is required.
@@ -377,7 +377,7 @@ def norm_rope_and_cache_supported(q, kv, kv_buffer, q_weight, k_weight) -> bool:
             and all(t.stride(0) % 8 == 0 and t.stride(1) % 8 == 0 and t.stride(2) == 1 for t in (q, kv, kv_buffer)))
 
 
-@torch.no_grad()
+@L.without_grad
 def rope_and_cache(q, kv, cos, sin, batch_size, seq_len, select_index, kv_buffer, positions=None, qk_norm=None):
     """Extension (one launch instead of two): ``rope_emb_forward(q, k)`` + ``update_kv_buffer(cat(k, v))``
     where ``kv [N, 2*Hkv, D]`` holds this step's K heads then V heads (typically a strided view of the
@@ -452,7 +452,7 @@ class SummedUpdate:
         return out + self.row.float() if self.row is not None else out
 
 
-@torch.no_grad()
+@L.without_grad
 def add_rmsnorm_shift(x_in, delta, weight, eps, *, x_out=None, shift=None, step=None, state=None, out_scale: float = 1.0):
     """``s = x_in + delta`` (fp32 residual ``[n, width]``; ``delta`` in the storage dtype, a :class:`SummedUpdate`, or ``None``),
     RMS norm with ``weight``,
@@ -497,7 +497,7 @@ def add_rmsnorm_shift(x_in, delta, weight, eps, *, x_out=None, shift=None, step=
     return y, (x_out if updated else x_in)
 
 
-@torch.no_grad()
+@L.without_grad
 def embed_pair(tokens: torch.Tensor, embed: torch.Tensor, scale: float = 1.0, pair: torch.Tensor | None = None,
                mul_prev: int = 0, mul_cur: int = 0, step=None, state: torch.Tensor | None = None) -> torch.Tensor:
     """The fp32 residual stream of a step's tokens: ``embed[token] * scale`` plus, with ``pair [buckets + 1, width]``, the row
@@ -528,7 +528,7 @@ def embed_pair(tokens: torch.Tensor, embed: torch.Tensor, scale: float = 1.0, pa
     return x
 
 
-@torch.no_grad()
+@L.without_grad
 def cast_pair(a: torch.Tensor, b: torch.Tensor, dtype, a_delta: torch.Tensor | None = None) -> torch.Tensor:
     """``[a + a_delta | b]`` of two fp32 ``[n, width]`` tensors (``a_delta``: a pending residual update in ``dtype``), cast to
     ``dtype``: the input of a projection over the pair."""
@@ -544,7 +544,7 @@ def cast_pair(a: torch.Tensor, b: torch.Tensor, dtype, a_delta: torch.Tensor | N
     return out
 
 
-@torch.no_grad()
+@L.without_grad
 def residual_set(y: torch.Tensor, bias: torch.Tensor | None = None, out: torch.Tensor | None = None) -> torch.Tensor:
     """A projection's rows ``y`` (+ ``bias [width]``) become the fp32 residual stream."""
     L.require_cuda(y)
@@ -558,7 +558,7 @@ def residual_set(y: torch.Tensor, bias: torch.Tensor | None = None, out: torch.T
     return out
 
 
-@torch.no_grad()
+@L.without_grad
 def embedding(ids: torch.Tensor, table: torch.Tensor):
     """``F.embedding(ids, table)``; an id that the table does not have is answered with NaN, as :func:`embed_rmsnorm` does.  ``None`` where the
     call is not served."""
@@ -582,7 +582,7 @@ class FirstRows:
         self.rows = rows
 
 
-@torch.no_grad()
+@L.without_grad
 def embed_rows(ids: torch.Tensor, table: torch.Tensor):
     """``(x, FirstRows)``: embedding rows as the fp32 residual and as they are, in one launch -- ``residual_set(F.embedding(ids, table))`` and
     the cast of it back.  ``None`` where the call is not served."""
@@ -620,7 +620,7 @@ class GatedUpdate:
                            self.bias)
 
 
-@torch.no_grad()
+@L.without_grad
 def gated_group_norm(x: torch.Tensor, update: "GatedUpdate | None", next_weight, eps: float, groups: int = 1, plain=None):
     """``x`` (fp32 residual ``[n, width]``, updated IN PLACE): ``x += groupnorm(update) * post_weight`` -- the update's rows
     summed, scaled by the sigmoid of its gate --, then ``h = groupnorm(x) * next_weight`` in the storage dtype
@@ -664,7 +664,7 @@ def gated_group_norm(x: torch.Tensor, update: "GatedUpdate | None", next_weight,
 _GLU_KINDS = {"silu": 0, "gelu_tanh": 1, "sigmoid": 2, "clamped": 3}
 
 
-@torch.no_grad()
+@L.without_grad
 def glu_act(gate: torch.Tensor, ff: int, kind: str, up: torch.Tensor | None = None, *, limit: float = 0.0, slope: float = 1.0,
             out: torch.Tensor | None = None) -> torch.Tensor:
     """``act(gate[:, :ff]) * up[:, :ff]``; without ``up`` the rows of ``gate`` hold ``[gate | up]``.  Both may be wider,
@@ -690,7 +690,7 @@ def glu_act(gate: torch.Tensor, ff: int, kind: str, up: torch.Tensor | None = No
     return out
 
 
-@torch.no_grad()
+@L.without_grad
 def relu_square(x: torch.Tensor, ff: int, out: torch.Tensor | None = None) -> torch.Tensor:
     """``relu(x[:, :ff])^2`` of row-strided rows (fp32 arithmetic, one rounding to the storage dtype).  ``out``: a ``[n, ff]`` view
     with a unit inner stride (a column range of the next projection's input)."""
@@ -706,7 +706,7 @@ def relu_square(x: torch.Tensor, ff: int, out: torch.Tensor | None = None) -> to
     return out
 
 
-@torch.no_grad()
+@L.without_grad
 def softcap_(x: torch.Tensor, cap: float) -> torch.Tensor:
     """``x <- cap * tanh(x / cap)`` in place (fp32 arithmetic)."""
     L.require_cuda(x)
@@ -736,7 +736,7 @@ class StreamUpdate:
         return StreamUpdate(pick(self.y), self.scale, self.mix, self.out, pick(self.shared), pick(self.shared_scale))
 
 
-@torch.no_grad()
+@L.without_grad
 def stream_norm(x: torch.Tensor, update: "StreamUpdate | None", streams: int, gather, weight, eps: float, weight_base: float = 0.0):
     """``x``: the fp32 residual streams ``[n, streams, width]``, or one row per token ``[n, width]`` that every stream starts from.  The
     pending ``update`` (or ``None``) enters and mixes the streams; then ``h = rmsnorm(sum_s gather[s] x_s) * (weight_base + weight)`` in

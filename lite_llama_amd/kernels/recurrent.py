@@ -12,7 +12,7 @@ def gated_linear_scan_supported(dk: int, dv: int) -> bool:
     return bool(L.lib().ll_gated_linear_scan_supported(dk, dv))
 
 
-@torch.no_grad()
+@L.without_grad
 def gated_linear_scan(qfv: torch.Tensor, heads: int, dk: int, dv: int, f_bias, lower, norm_weight, eps: float, step,
                       state: torch.Tensor) -> torch.Tensor:
     """HGRN2-style gated linear attention.  ``qfv [n, 2 heads dk + heads dv]`` = the fused projection rows
@@ -49,7 +49,7 @@ def gated_linear_scan(qfv: torch.Tensor, heads: int, dk: int, dv: int, f_bias, l
     return out
 
 
-@torch.no_grad()
+@L.without_grad
 def mingru_scan(zxg: torch.Tensor, width: int, z_bias, x_bias, step, state: torch.Tensor) -> torch.Tensor:
     """minGRU over a ragged step.  ``zxg [n, >= 3 width]`` = fused projection rows ``[z_raw | x_raw | g_raw]``; per channel
     ``z = sigmoid(z_raw + z_bias)``, ``u = x_raw + x_bias``, candidate ``u + 1/2`` where ``u >= 0`` and ``sigmoid(u)`` below,
@@ -78,7 +78,7 @@ def mingru_scan(zxg: torch.Tensor, width: int, z_bias, x_bias, step, state: torc
     return out
 
 
-@torch.no_grad()
+@L.without_grad
 def rglru_scan(u: torch.Tensor, gates: torch.Tensor, r_bias, i_bias, lam, y: torch.Tensor, step, state: torch.Tensor) -> torch.Tensor:
     """RG-LRU over a ragged step: per channel ``r = sigmoid(r_raw + r_bias)``, ``i = sigmoid(i_raw + i_bias)``,
     ``log a = -8 r softplus(lam)``, ``S <- a S + sqrt(1 - a^2) i u``; returns ``S * gelu(y)`` (tanh form) ``[n, width]`` in the
@@ -116,7 +116,7 @@ def delta_scan_supported(dk: int, dv: int) -> bool:
     return bool(L.lib().ll_delta_scan_supported(dk, dv))
 
 
-@torch.no_grad()
+@L.without_grad
 def delta_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, heads: int, dk: int, dv: int, step, state: torch.Tensor, *,
                gate: torch.Tensor, dt_bias: torch.Tensor, a_log: torch.Tensor, beta: torch.Tensor, qk_heads: int | None = None,
                q_scale: float = 1.0, unit_eps: float = 1e-6) -> torch.Tensor:
@@ -169,7 +169,7 @@ def _rows(t: torch.Tensor, cols: int, what: str) -> None:
         raise ValueError(f"linear_scan: {what} rows are [n, >= {cols}] with a unit inner stride")
 
 
-@torch.no_grad()
+@L.without_grad
 def linear_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, heads: int, dk: int, dv: int, step, state: torch.Tensor, *,
                 qk_heads: int | None = None, act: bool = False, q_scale: float = 1.0, head_decay: torch.Tensor | None = None,
                 gate: torch.Tensor | None = None, gate_bias: torch.Tensor | None = None, tau: float = 1.0,
@@ -251,7 +251,7 @@ def retention_supported(dk: int, dv: int) -> bool:
     return bool(L.lib().ll_retention_supported(dk, dv))
 
 
-@torch.no_grad()
+@L.without_grad
 def retention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, heads: int, dk: int, dv: int, step, state: torch.Tensor, *,
               decay: torch.Tensor, gate: torch.Tensor, eps: float, k_scale: float = 1.0, half: int = 0,
               rot_table: torch.Tensor | None = None, out: torch.Tensor | None = None) -> torch.Tensor:
@@ -301,7 +301,7 @@ def retention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, heads: int, dk:
 _GATES = {None: 0, "silu": 1, "sigmoid": 2}
 
 
-@torch.no_grad()
+@L.without_grad
 def gated_out_norm(o: torch.Tensor, weight: torch.Tensor | None, eps: float, *, parts: int = 1, gate: torch.Tensor | None = None,
                    gate_kind: str | None = None, gate_first: bool = False, scale: float = 1.0, out: torch.Tensor | None = None,
                    dtype=None) -> torch.Tensor:
@@ -332,7 +332,7 @@ def gated_out_norm(o: torch.Tensor, weight: torch.Tensor | None, eps: float, *, 
     return out
 
 
-@torch.no_grad()
+@L.without_grad
 def conv_act(rows: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, step, state: torch.Tensor | None,
              act: str | None = "silu") -> torch.Tensor:
     """``act(bias + causal convolution)`` per channel (``act``: silu, or ``None``) over a ragged step: ``rows [n, channels]`` (a row-strided view),

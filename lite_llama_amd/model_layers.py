@@ -71,6 +71,7 @@ from .distributed.parallel_state import get_tp_world_size
 from .kernels.activations import xielu
 from .kernels.attention import (conv_rope_cache, latent_kv_prep, qk_norm_cache, ragged_attention, rotate_pairs, rotation_table,
                                 rownorm_rope_cache)
+from .layered_decode import _attention_ssd, _dense, _entry_decay, _fixed_decay, _routed, decode_layer
 from .kernels.fused_moe import group_router, sparse_glu_experts, sparse_square_experts
 from .kernels.norm_act import (FirstRows, GatedUpdate, StreamUpdate, SummedUpdate, add_rmsnorm_shift, cast_pair, embed_pair, embed_rows,
                                gated_group_norm, glu_act, relu_square, residual_set, softcap_, stream_norm)
@@ -996,15 +997,18 @@ class WindowAttentionSSD(nn.Module):
         return {"kind": "attention", "kv_heads": s.kv_heads, "dk": s.dim, "dv": s.vdim, "state": (r.heads, r.state, r.vdim),
                 "conv_taps": r.conv_taps, "conv_channels": r.conv_channels}
 
+    def frequencies(self, device):
+        if self.pairs and (self._freq is None or self._freq.device != device):
+            self._freq = torch.tensor(self._freq_values, dtype=torch.float64).to(torch.float32).to(device)
+        return self._freq
+
     def forward(self, h, step, cache, run: int, token_table):
         s, r = self.spec, self.spec.ssd
         rows = self.in_proj(h)
-        if self.pairs and (self._freq is None or self._freq.device != h.device):
-            self._freq = torch.tensor(self._freq_values, dtype=torch.float64).to(torch.float32).to(h.device)
         mixed = torch.empty(h.shape[0], self.heads_width + r.inner, dtype=h.dtype, device=h.device)
         k_cache, v_cache = cache.kv_buffer[run]
         q = rownorm_rope_cache(rows, s.heads, s.kv_heads, s.dim, s.vdim, step, k_cache, v_cache, q_weight=self.q_norm_weight,
-                               k_weight=self.k_norm_weight, eps=self.eps, freq=self._freq, pairs=self.pairs,
+                               k_weight=self.k_norm_weight, eps=self.eps, freq=self.frequencies(h.device), pairs=self.pairs,
                                value_scale=s.branch_scales[0])
         ragged_attention(q, k_cache, v_cache, s.scale, step, token_table, window=s.window, out=mixed[:, :self.heads_width])
         ubc = conv_act(rows[:, self.conv_off:self.dt_off], self.conv_weight, self.conv_bias, step, cache.conv[run])
@@ -1033,13 +1037,16 @@ class DecayLinearAttention(nn.Module):
     def cache_run(self) -> dict:
         return {"kind": "recurrent", "heads": self.spec.heads, "dk": self.spec.dim, "dv": self.spec.vdim}
 
+    def decays(self, device):
+        if self._decay is None or self._decay.device != device:
+            self._decay = torch.tensor(self.spec.decay, dtype=torch.float64).to(torch.float32).to(device)
+        return self._decay
+
     def forward(self, h, step, cache, run: int, token_table):
         s, qk, v = self.spec, self.qk, self.v
         rows = self.in_proj(h)
-        if self._decay is None or self._decay.device != h.device:
-            self._decay = torch.tensor(s.decay, dtype=torch.float64).to(torch.float32).to(h.device)
         o = linear_scan(rows[:, :qk], rows[:, qk:2 * qk], rows[:, 2 * qk:2 * qk + v], s.heads, s.dim, s.vdim, step,
-                        cache.recurrent[run], act=True, head_decay=self._decay)
+                        cache.recurrent[run], act=True, head_decay=self.decays(h.device))
         return self.o_proj(gated_out_norm(o, self.out_norm_weight, self.eps, gate=rows[:, 2 * qk + v:], gate_kind="sigmoid"))
 
 
@@ -1395,6 +1402,10 @@ class ParallelLayer(nn.Module):
         return x, SummedUpdate(row, self.experts(h) if self.experts is not None else None)
 
 
+DECODED_MIXERS = {WindowAttentionSSD: _attention_ssd, DecayLinearAttention: _fixed_decay, GatedLinearAttention: _entry_decay}
+DECODED_FEED_FORWARDS = {BiasedGatedMLP: _dense, CorrectedSoftmaxMoE: _routed}
+
+
 class PostNormLayer(nn.Module):
     """``x <- x + norm_1(mixer(x))``, then ``x <- x + norm_2(feed_forward(x))``: sublayers read the residual stream itself (cast
     to the storage dtype), the norm sits on each sublayer's RESULT.  A result is carried as a :class:`GatedUpdate` into the
@@ -1413,6 +1424,9 @@ class PostNormLayer(nn.Module):
 
     def forward(self, x, pending, step, cache, run: int, token_table):
         """``(x, pending)``: the fp32 residual (updated in place) and the update still to enter it.  Returns the same pair."""
+        done = decode_layer(self, x, pending, step, cache, run, token_table, DECODED_MIXERS, DECODED_FEED_FORWARDS)
+        if done is not None:
+            return done
         dt = self.norm1_weight.dtype
         h = pending.rows if isinstance(pending, FirstRows) else gated_group_norm(x, pending, None, self.eps, plain=dt)
         pending = GatedUpdate(self.mixer(h, step, cache, run, token_table), self.norm1_weight)
