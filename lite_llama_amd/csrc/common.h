@@ -53,6 +53,17 @@ __device__ __forceinline__ uint16_t from_f32(float f) {
   else return f32_to_bf16_bits(f);
 }
 
+// Two values side by side in one conversion (v_cvt_pk_f16_f32, v_cvt_pk_bf16_f32: the rounding of the single ones), `lo` in the lower half.  Not for an
+// fp16 product that has to be rounded twice, unless it is ll_pinned.
+template <int DT>
+__device__ __forceinline__ uint32_t ll_pack2(float lo, float hi) {
+  typedef float v2 __attribute__((ext_vector_type(2)));
+  typedef f16 h2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+  if constexpr (DT == LL_F16) return __builtin_bit_cast(uint32_t, __builtin_convertvector((v2{lo, hi}), h2));
+  else return __builtin_bit_cast(uint32_t, __builtin_convertvector((v2{lo, hi}), b2));
+}
+
 // Product of two storage-dtype values rounded once to the storage dtype (what
 // a fp16*fp16 / bf16*bf16 multiply yields: the fp32 product is exact).
 template <int DT>

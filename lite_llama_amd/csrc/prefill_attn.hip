@@ -30,7 +30,7 @@ __device__ __forceinline__ f32x4 mfma16(const Q4& a, const Q4& b, f32x4 c) {
 
 template <int DT>
 __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-  return (uint32_t)from_f32<DT>(lo) | ((uint32_t)from_f32<DT>(hi) << 16);
+  return ll_pack2<DT>(lo, hi);
 }
 
 __device__ __forceinline__ int64_t pa_load_idx(const void* p, int64_t i, int w) {
@@ -171,6 +171,9 @@ __global__ __launch_bounds__(64) void fa_prefill(
 // L2 traffic at batch 64 x 512).  Each wave keeps 16 * QB query columns: K fragments are read from LDS once per tile
 // and used for QB query blocks, V^T fragments come from transposing LDS reads (ds_read_b64_tr_b16), the online softmax
 // runs once per 64 keys (one rescale of O per tile, skipped when no running maximum moved).
+// Two tiles stand in LDS, so that one barrier per tile is enough; it waits for LDS alone.  A row's address is its number, clamped in 32 bits, times the
+// stride: in 64 bits throughout, the eight requests of a tile took 120 of the walk's 530 instructions.  us, before -> now, bit for bit, heads of 128: 16 prompts of
+// 255 - 509, 28 on 4, 82.6 -> 76.0; 5 of 500 - 1000, 32 on 8, 101.4 -> 94.1
 // ROPE (the type of the rotary tables' entries; -1: none): q and k come as the projection left them and are rotated on the way in, rounded as
 // rope_cache_kernel rounds them; what that kernel writes to the cache is written by workgroups of their own beside these (blockIdx.z past
 // the sequences), for every token and whatever the sequences cover.  A launch less per layer of a short prefill, whose launches are
@@ -204,8 +207,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
   constexpr int NS = D / 32, NT = D / 16, STR = D + 8, TK = 64;
   constexpr int CS = ROPE < 0 ? LL_F16 : ROPE;
   constexpr int TPR = D / 8, RPP = 256 / TPR, PASSES = TK / RPP;  // 16-byte pieces per row, rows per pass
-  __shared__ __attribute__((aligned(16))) uint16_t lds_k[TK * STR];
-  __shared__ __attribute__((aligned(16))) uint16_t lds_v[TK * STR];
+  extern __shared__ __attribute__((aligned(16))) uint16_t lds[];   // [2][keys, then values][TK * STR] (fa2_lds)
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int t = lane & 15, c = lane >> 4;
@@ -242,15 +244,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
   }
   const int64_t seq_len = pa_load_idx(b_seq_len, b, seq_w);
   const int64_t start = pa_load_idx(b_start_loc, b, start_w);
-  const int64_t q0 = (int64_t)(gridDim.x - 1 - blockIdx.x) * (64 * QB);  // the longest key ranges are dispatched first
-  if (q0 >= seq_len) return;
-  const int64_t qw = q0 + wave * (16 * QB);  // this wave's first query
+  const int64_t first = (int64_t)(gridDim.x - 1 - blockIdx.x) * (64 * QB);  // the longest key ranges are dispatched first
+  if (first >= seq_len) return;
+  const int q0 = (int)first, keys = seq_len < 0x7fffff00 ? (int)seq_len : 0x7fffff00;   // (positions of a sequence are 32-bit numbers from here on)
+  const int qw = q0 + wave * (16 * QB);  // this wave's first query
 
   Q4 qf[QB][NS];
 #pragma unroll
   for (int qb = 0; qb < QB; ++qb) {
-    const int64_t qi = qw + qb * 16 + t;
-    const int64_t qrow = qi < seq_len ? qi : seq_len - 1;  // rows past the end: a valid row, never stored
+    const int qi = qw + qb * 16 + t;
+    const int qrow = qi < keys ? qi : keys - 1;  // rows past the end: a valid row, never stored
 #pragma unroll
     for (int s = 0; s < NS; ++s)
       qf[qb][s] = *reinterpret_cast<const Q4*>(q + (start + qrow) * q_st + (int64_t)head * q_sh + s * 32 + c * 8);
@@ -276,49 +279,59 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
     for (int i = 0; i < NT; ++i) ot[qb][i] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
 
-  const int64_t kend = q0 + 64 * QB < seq_len ? q0 + 64 * QB : seq_len;  // causal: the workgroup needs keys < kend
+  const int kend = q0 + 64 * QB < keys ? q0 + 64 * QB : keys;  // causal: the workgroup needs keys < kend
   const int lrow = tid / TPR, lcol = (tid % TPR) * 8;
   constexpr int ROT = ROPE < 0 ? 1 : PASSES;
   [[maybe_unused]] const bool low = lcol < D / 2;
   [[maybe_unused]] const int lj = low ? lcol : lcol - D / 2;
   [[maybe_unused]] i32x4 ko[ROT], kc[ROT], ks[ROT];   // the other half's entries, the tables' entries
   i32x4 kr[PASSES], vr[PASSES];  // (vector type, not the Q4 struct: the struct copy into LDS kept the array in scratch)
-  auto fetch = [&](int64_t p0) {
+  const uint16_t *kbase = k + start * k_st + (int64_t)kvh * k_sh, *vbase = v + start * v_st + (int64_t)kvh * v_sh + lcol;
+  auto fetch = [&](int p0) {
 #pragma unroll
     for (int ps = 0; ps < PASSES; ++ps) {
-      int64_t key = p0 + ps * RPP + lrow;
-      if (key >= seq_len) key = seq_len - 1;
-      kr[ps] = *reinterpret_cast<const i32x4*>(k + (start + key) * k_st + (int64_t)kvh * k_sh + lcol);
-      vr[ps] = *reinterpret_cast<const i32x4*>(v + (start + key) * v_st + (int64_t)kvh * v_sh + lcol);
+      const int want = p0 + ps * RPP + lrow;
+      const uint32_t key = (uint32_t)(want < keys ? want : keys - 1);
+      kr[ps] = *reinterpret_cast<const i32x4*>(kbase + lcol + key * (uint64_t)k_st);
+      vr[ps] = *reinterpret_cast<const i32x4*>(vbase + key * (uint64_t)v_st);
       if constexpr (ROPE >= 0) {
         int64_t cb, sb;
-        tables((int)(start + key), cb, sb);
-        ko[ps] = at(k + (start + key) * k_st + (int64_t)kvh * k_sh + (low ? lcol + D / 2 : lj));
+        tables((int)start + (int)key, cb, sb);
+        ko[ps] = at(kbase + (low ? lcol + D / 2 : lj) + key * (uint64_t)k_st);
         kc[ps] = at(rp.cos_t + cb + lj);
         ks[ps] = at(rp.sin_t + sb + lj);
       }
     }
   };
-  auto stage = [&](int64_t p0) {
+  auto stage = [&](int p0, int buf) {
+    uint16_t *lds_k = lds + buf * (2 * TK * STR), *lds_v = lds_k + TK * STR;
 #pragma unroll
     for (int ps = 0; ps < PASSES; ++ps) {
-      const int row = ps * RPP + lrow;
       if constexpr (ROPE >= 0) kr[ps] = fa_rotated<DT, CS>(kr[ps], ko[ps], kc[ps], ks[ps], low);
-      *reinterpret_cast<i32x4*>(&lds_k[row * STR + lcol]) = kr[ps];
+      *reinterpret_cast<i32x4*>(&lds_k[(ps * RPP + lrow) * STR + lcol]) = kr[ps];
+    }
+    if (p0 + TK <= keys) {   // (wave-uniform)
+#pragma unroll
+      for (int ps = 0; ps < PASSES; ++ps) *reinterpret_cast<i32x4*>(&lds_v[(ps * RPP + lrow) * STR + lcol]) = vr[ps];
+    } else {
       // rows past the sequence end are multiplied by p = 0: they must not hold NaN / Inf bit patterns
-      *reinterpret_cast<i32x4*>(&lds_v[row * STR + lcol]) = p0 + row < seq_len ? vr[ps] : i32x4{0, 0, 0, 0};
+#pragma unroll
+      for (int ps = 0; ps < PASSES; ++ps)
+        *reinterpret_cast<i32x4*>(&lds_v[(ps * RPP + lrow) * STR + lcol]) = p0 + ps * RPP + lrow < keys ? vr[ps] : i32x4{0, 0, 0, 0};
     }
   };
-  const uint16_t* vtr = lds_v + (4 * c + (t >> 2)) * STR + (t & 3) * 4;
+  auto meet = [&]() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };   // (only LDS is exchanged)
 
   fetch(0);
-  for (int64_t p0 = 0; p0 < kend; p0 += TK) {
-    __syncthreads();  // the previous tile's fragment reads are done
-    stage(p0);
-    __syncthreads();
-    fetch(p0 + TK < kend ? p0 + TK : p0);  // in flight under this tile's arithmetic (unconditional: a branch around
-                                           // loads parks the prefetch registers in scratch)
-    if (p0 >= qw + 16 * QB) continue;    // every key of the tile lies after this wave's last query
+  stage(0, 0);
+  int buf = 0;
+  for (int p0 = 0; p0 < kend; p0 += TK, buf ^= 1) {
+    const uint16_t* lds_k = lds + buf * (2 * TK * STR);
+    const uint16_t* vtr = lds_k + TK * STR + (4 * c + (t >> 2)) * STR + (t & 3) * 4;
+    meet();  // this tile is in LDS, and the fragment reads of the one before are done
+    const int p1 = p0 + TK < kend ? p0 + TK : p0;   // in flight under this tile's arithmetic (unconditional: a branch around
+    fetch(p1);                                       // loads parks the prefetch registers in scratch)
+    if (p0 < qw + 16 * QB) {    // (else every key of the tile lies after this wave's last query)
     // S^T blocks for all QB query blocks from ONE read of each K fragment: rows = keys p0 + 16 kb + 4c + r, column =
     // query qw + 16 qb + t.  (A query block that lies entirely before the tile gets all-masked scores: p = 0, alpha = 1.)
     f32x4 sacc[QB][4];
@@ -338,7 +351,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
     Q4 pf[QB][2];
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
-      const int64_t qfirst = qw + qb * 16;
+      const int qfirst = qw + qb * 16;
       // scores stay raw until the exponent: p = exp2(s * scale - m) is one fma + one v_exp per key (scale > 0, so the
       // maximum is taken over the raw scores); masked keys hold the raw value whose scaled form is the reference's -1e8
       float sc[16];
@@ -347,11 +360,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
 #pragma unroll
         for (int j = 0; j < 16; ++j) sc[j] = sacc[qb][j >> 2][j & 3];
       } else {
-        const int64_t qi = qfirst + t;
+        const int qi = qfirst + t;
         const float masked = -1.0e8f / sm_scale;
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
-          const int64_t key = p0 + 16 * (j >> 2) + 4 * c + (j & 3);
+          const int key = p0 + 16 * (j >> 2) + 4 * c + (j & 3);
           sc[j] = key <= qi ? sacc[qb][j >> 2][j & 3] : masked;  // reference: where(causal, qk * scale, -1e8)
         }
       }
@@ -402,12 +415,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
         for (int qb = 0; qb < QB; ++qb) ot[qb][dt] = mfma16<DT>(vf, pf[qb][hf], ot[qb][dt]);
       }
     }
+    }
+    if (p0 + TK < kend) stage(p1, buf ^ 1);
   }
 
 #pragma unroll
   for (int qb = 0; qb < QB; ++qb) {
-    const int64_t qi = qw + qb * 16 + t;
-    if (qi < seq_len) {
+    const int qi = qw + qb * 16 + t;
+    if (qi < keys) {
       const float inv = 1.0f / d_i[qb];
       uint16_t* o = out + (start + qi) * o_st + (int64_t)head * o_sh;
 #pragma unroll
@@ -421,6 +436,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
   }
 }
 
+constexpr int fa2_lds(int d) { return 2 * 2 * 64 * (d + 8) * 2; }
+// (more than a launch may have without being asked for)
+template <int DT, int D, int QB, int ROPE = -1>
+static bool fa2_ready() {
+  static const hipError_t wide = hipFuncSetAttribute((const void*)fa_prefill2<DT, D, QB, ROPE>, hipFuncAttributeMaxDynamicSharedMemorySize, fa2_lds(D));
+  return wide == hipSuccess;
+}
+
 template <int DT>
 static int launch_fa(void* out, const void* q, const void* k, const void* v, const void* start, const void* seq,
                      int batch, int hq, int hkv, int d, int64_t max_seq_len, float sm_scale, int64_t q_st,
@@ -430,14 +453,17 @@ static int launch_fa(void* out, const void* q, const void* k, const void* v, con
     static const int qb_env = getenv("LL_FA_QB") ? atoi(getenv("LL_FA_QB")) : 0;  // debug knob, read once
     const int qb = qb_env == 1 || qb_env == 2 ? qb_env : (max_seq_len > 64 ? 2 : 1);
     dim3 grid2((unsigned)((max_seq_len + 64 * qb - 1) / (64 * qb)), (unsigned)hq, (unsigned)batch);
-#define LL_FA2(DD, QQ)                                                                                          \
-  fa_prefill2<DT, DD, QQ><<<grid2, 256, 0, st>>>((uint16_t*)out, (const uint16_t*)q, (const uint16_t*)k,        \
-                                                 (const uint16_t*)v, start, seq, hq, hkv, sm_scale, q_st, q_sh, \
-                                                 k_st, k_sh, v_st, v_sh, o_st, o_sh, start_w, seq_w, FaRope{})
+#define LL_FA2(DD, QQ)                                                                                                  \
+  {                                                                                                                     \
+    if (!fa2_ready<DT, DD, QQ>()) return LL_ERR_LAUNCH;                                                                 \
+    fa_prefill2<DT, DD, QQ><<<grid2, 256, fa2_lds(DD), st>>>((uint16_t*)out, (const uint16_t*)q, (const uint16_t*)k,     \
+                                                             (const uint16_t*)v, start, seq, hq, hkv, sm_scale, q_st, q_sh, \
+                                                             k_st, k_sh, v_st, v_sh, o_st, o_sh, start_w, seq_w, FaRope{}); \
+  }
     if (d == 64) {
-      if (qb == 2) LL_FA2(64, 2); else LL_FA2(64, 1);
+      if (qb == 2) LL_FA2(64, 2) else LL_FA2(64, 1)
     } else {
-      if (qb == 2) LL_FA2(128, 2); else LL_FA2(128, 1);
+      if (qb == 2) LL_FA2(128, 2) else LL_FA2(128, 1)
     }
 #undef LL_FA2
     return LL_LAUNCH_CHECK();
@@ -499,9 +525,12 @@ int fa_rope_launch(void* out, const void* qkv, int64_t row, const void* cos_t, c
   const int qb = max_len > 64 && d == 64 ? 2 : 1;   // (128 query entries and the tables' beside them do not fit the registers twice)
   const uint16_t *q = (const uint16_t*)qkv, *k = q + (int64_t)heads * d, *v = k + (int64_t)kv_heads * d;
   const dim3 grid((unsigned)((max_len + 64 * qb - 1) / (64 * qb)), (unsigned)heads, (unsigned)prompts + 1);
-#define LL_FAR(DT, DD, QQ, CS)                                                                                                               \
-  fa_prefill2<DT, DD, QQ, CS><<<grid, 256, 0, st>>>((uint16_t*)out, q, k, v, starts, lens, heads, kv_heads, sm_scale, row, d, row, d, row, d, \
-                                                    (int64_t)heads * d, d, start_width, len_width, rp)
+#define LL_FAR(DT, DD, QQ, CS)                                                                                                                       \
+  do {                                                                                                                                               \
+    if (!fa2_ready<DT, DD, QQ, CS>()) return LL_ERR_LAUNCH;                                                                                           \
+    fa_prefill2<DT, DD, QQ, CS><<<grid, 256, fa2_lds(DD), st>>>((uint16_t*)out, q, k, v, starts, lens, heads, kv_heads, sm_scale, row, d, row, d, row, \
+                                                                d, (int64_t)heads * d, d, start_width, len_width, rp);                                \
+  } while (0)
 #define LL_FAR_Q(DT, DD, CS) do { if (qb == 2) LL_FAR(DT, DD, 2, CS); else LL_FAR(DT, DD, 1, CS); } while (0)
 #define LL_FAR_D(DT, CS) do { if (d == 64) LL_FAR_Q(DT, 64, CS); else LL_FAR(DT, 128, 1, CS); } while (0)
 #define LL_FAR_C(DT) do { if (cs_dtype == LL_F16) LL_FAR_D(DT, LL_F16); else LL_FAR_D(DT, LL_BF16); } while (0)
