@@ -1040,14 +1040,24 @@ extern "C" int ll_flash_decoding_num_partitions(int64_t max_len) {
 // 200 - 270 on 8 KV heads of 4 134 / 239 / 47.
 // Heads of 256 spill 400 registers in a grouped workgroup (27 rows on 4 KV heads of 4, 3000 tokens 55 / 140): they take it only where the
 // last arriver alone would merge very many partitions (2 pairs, 32 768 tokens 160 / 75; 16 pairs, 16 384 140 / 118).
+// Five to eight partitions at up to 64 pairs, heads of 128: workgroups of four waves, as many per pair as leave each a CU to itself -- a CU takes in
+// some 27 KB a microsecond whatever its waves, and a row of 1000 tokens is 512 KB.  us, one workgroup / here, longest row 520 | 700 | 1000 tokens:
+// 4 pairs of 7 heads 12.1 / 10.5 | 15.3 / 10.8 | 19.2 / 10.6; 64 of 7 12.3 / 11.4 | 15.6 / 12.2 | 19.7 / 12.4; 64 of 8 11.9 / 11.1 | 15.8 / 12.1 |
+// 20.0 / 12.6.  Not from 100 pairs on (12.5 / 13.2 at 520), not for heads of 64 (7.6 / 7.8 at 8 pairs, 7.7 / 8.8 at 120), not up to four partitions
+// (300 tokens 9.0 / 10.2).
 #define FD_LOOP_MAX 256  // partitions (32 768 tokens)
 struct FdPlan {
   int waves, splits;
 };
-static FdPlan fd_plan(int64_t max_len, int64_t pairs, int heads, int d, bool planes) {
+// (planes: q|k|v come as sums to be added up, two float4 slots a lane; merge: the caller lends the scratch that workgroups of a pair meet in)
+static FdPlan fd_plan(int64_t max_len, int64_t pairs, int heads, int d, bool planes, bool merge) {
   const int64_t np = (max_len + FD_PART - 1) / FD_PART;
   if (np < 2 || np > FD_LOOP_MAX || pairs < 1) return {0, 0};
-  if (np <= FD_GROUP_MAX) return {(int)np, 1};
+  if (np <= FD_GROUP_MAX) {
+    const int64_t room = 256 / pairs, most = (np + 1) / 2;
+    if (np > 4 && pairs <= 64 && d == 128 && merge && (!planes || (heads + 2) * d / 4 <= 128 * 4)) return {4, (int)(room < most ? room : most)};
+    return {(int)np, 1};
+  }
   static const bool no_loop = getenv("LL_FD_NO_LOOP") != nullptr;  // A/B knob, read once
   if (no_loop) return {0, 0};
   if (pairs >= 128) return {FD_GROUP_MAX, 1};
@@ -1064,7 +1074,7 @@ static FdPlan fd_plan(int64_t max_len, int64_t pairs, int heads, int d, bool pla
 // Waves of a workgroup where the grouped form also takes q|k|v as split-K partials (every workgroup of a pair adds them up again:
 // past FD_GROUP_MAX partitions that is declined below 64 pairs); 0: it does not.
 extern "C" int ll_flash_decoding_group_waves(int64_t max_len, int64_t workgroups) {
-  const FdPlan pl = fd_plan(max_len, workgroups, 1, 128, true);
+  const FdPlan pl = fd_plan(max_len, workgroups, 1, 128, true, false);   // (up to FD_GROUP_MAX partitions the most waves that it may take)
   return pl.splits > 1 && workgroups < 64 ? 0 : pl.waves;
 }
 
@@ -1088,7 +1098,7 @@ static int launch_fd(void* out, const void* q, const void* kc, const void* vc, c
   const bool qkn = rope && (rp.qnw || rp.knw);
   if (qkn && (!rp.qnw || !rp.knw || d != 128 || kv8 || !(rp.nrm_eps >= 0.f))) return LL_ERR_SHAPE;
   const int64_t pairs = (int64_t)batch * hkv * hgroups;
-  FdPlan plan = fd_plan(max_len, pairs, groups < 16 ? groups : 16, d, rope && rp.qp);
+  FdPlan plan = fd_plan(max_len, pairs, groups < 16 ? groups : 16, d, rope && rp.qp, mid_o && mid_lse);
   // (planes without the scratch of a merge between workgroups: one workgroup walks a pair's whole context, as from 128 pairs on)
   if (rope && rp.qp && !(mid_o && mid_lse)) plan.splits = 1;
   const int gw = plan.waves;  // waves of a grouped workgroup; 0: not grouped

@@ -242,10 +242,13 @@ def decode_attention_partials(parts, bias, num_heads: int, num_kv_heads: int, he
     k_cache, v_cache = kv_buffer[:, :num_kv_heads], kv_buffer[:, num_kv_heads:]
     out = torch.empty((batchs, num_heads, head_dim), dtype=dt, device=p.device)
     fn, merge = L.lib().ll_decode_attention_partials, ()
-    if max_len > 1024 and batchs * num_kv_heads < 128:  # several workgroups share a row: scratch of their merge
-        counters = _merge_counters(p.device, batchs * num_kv_heads)
-        if counters is None:
+    pairs = batchs * num_kv_heads
+    counters = None   # several workgroups share a row: scratch of their merge
+    if (max_len > 1024 and pairs < 128) or (max_len > 512 and pairs <= 64 and head_dim == 128):
+        counters = _merge_counters(p.device, pairs)
+        if counters is None and max_len > 1024:
             return None
+    if counters is not None:
         nparts = L.lib().ll_flash_decoding_num_partitions(max_len)
         mid_o = torch.empty((batchs, num_heads, nparts, head_dim), dtype=torch.float32, device=p.device)
         mid_lse = torch.empty((batchs, num_heads, nparts, 32), dtype=torch.float32, device=p.device)

@@ -167,3 +167,48 @@ def test_projection_planes_are_taken_from_64_pairs_on():
     assert torch.equal(pool_a, pool_b) and torch.equal(got, want)
     assert decode_attention_partials_supported(longest, hq, hkv, d, batch=32)
     assert not decode_attention_partials_supported(longest, hq, hkv, d, batch=31)
+
+
+# five to eight partitions: several workgroups of four waves per pair up to 64 pairs of heads of 128, one workgroup beside that line and without scratch
+@pytest.mark.parametrize("b,hkv,rep,d,longest,bound", [(1, 1, 1, 128, 513, 640), (1, 4, 7, 128, 1000, 1024), (3, 2, 16, 128, 1024, 1024), (16, 4, 8, 128, 700, 768),
+                                                       (13, 5, 3, 128, 900, 1024), (2, 2, 15, 128, 640, 640), (9, 2, 7, 64, 1000, 1024)])
+def test_middle_contexts(b, hkv, rep, d, longest, bound):
+    from lite_llama_amd.kernels import flash_decoding
+    from lite_llama_amd.kernels.attention import _fd_counters
+
+    g = torch.Generator(device=DEV).manual_seed(longest)
+    lens = [longest if i == b // 2 else (131 * i) % longest + 1 for i in range(b)]
+    pool = torch.randn(sum(lens), 2 * hkv, d, generator=g, device=DEV).half()
+    table = torch.zeros(b, bound, dtype=torch.int32, device=DEV)
+    for i, rows in enumerate(torch.randperm(sum(lens), generator=g, device=DEV).to(torch.int32).split(lens)):
+        table[i, :lens[i]] = rows
+    q = torch.randn(b, hkv * rep, d, generator=g, device=DEV).half()
+    seq, req = torch.tensor(lens, dtype=torch.int32, device=DEV), torch.arange(b, dtype=torch.int32, device=DEV)
+    args = (q, pool[:, :hkv], pool[:, hkv:], 2.0 / math.sqrt(d), table, req)
+    got = flash_decoding(*args, seq, bound)
+    # probabilities and the result are rounded to the storage type: half a unit each, on values of up to about 4
+    assert (got.double() - reference(q, pool[:, :hkv], pool[:, hkv:], 2.0 / math.sqrt(d), table, seq)).abs().max().item() < 4 * 2.0 ** -10
+    for _ in range(3):
+        assert torch.equal(flash_decoding(*args, seq, bound), got)
+    empty = seq.clone()
+    empty[0] = 0
+    again = flash_decoding(*args, empty, bound)
+    assert again[0].isnan().all() and torch.equal(again[1:], got[1:])
+    assert all(int(c.abs().sum()) == 0 for c in _fd_counters.values())
+
+
+@pytest.mark.parametrize("b,longest", [(1, 513), (7, 900), (27, 1024)])
+def test_planes_at_middle_contexts(b, longest):
+    """q | k | v as split-K planes == the finished projection where several workgroups share a row, bit for bit, output and written cache rows."""
+    from lite_llama_amd.kernels.attention import decode_attention, decode_attention_partials
+
+    parts, hq, hkv, d, cos, sin, pos, sel, pool, table, req, seq = _planes(b, longest, b)
+    pool_a, pool_b = pool.clone(), pool.clone()
+    got = decode_attention_partials(parts, None, hq, hkv, d, cos, sin, pos, sel, pool_a, 0.1, table, req, seq, longest)
+    sums = parts.parts[0].clone()
+    for p in parts.parts[1:]:
+        sums = sums + p                                               # (planes are added in order, in 32 bits)
+    rows = sums.to(torch.bfloat16)
+    q, kv = rows[:, :hq * d].view(b, hq, d), rows[:, hq * d:].view(b, 2 * hkv, d)
+    want = decode_attention(q.contiguous(), kv.contiguous(), cos, sin, pos, sel, pool_b, 0.1, table, req, seq, longest)
+    assert torch.equal(pool_a, pool_b) and torch.equal(got.reshape(-1), want.reshape(-1))
