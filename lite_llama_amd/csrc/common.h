@@ -1,5 +1,6 @@
 // Shared device helpers for the gfx950 kernels (wave64, 16-byte vector I/O).
 #pragma once
+#include <atomic>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -159,6 +160,16 @@ __device__ __forceinline__ float ll_silu_mul_f32(float g, float u) {
 
 static inline bool ll_aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
+// More LDS than a launch has unasked: asked for once per kernel and device (`asked`: the devices, of this kernel)
+static inline bool ll_wide_lds(const void* kernel, int bytes, std::atomic<uint64_t>& asked) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return false;
+  const uint64_t bit = 1ull << (dev & 63);
+  if (dev < 64 && (asked.load(std::memory_order_relaxed) & bit)) return true;
+  if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) return false;
+  asked.fetch_or(bit, std::memory_order_relaxed);
+  return true;
+}
 #define LL_LAUNCH_CHECK() (hipGetLastError() == hipSuccess ? LL_OK : LL_ERR_LAUNCH)
 
 // Reductions over the four 16-lane rows of a wave (lanes t, t + 16, t + 32, t + 48) with the gfx950 row-swap VALU

@@ -83,6 +83,7 @@ struct FdRope {
   // QI32 (smoothquant q|k|v): the planes at qp are EXACT int32 sums; value = fp16(((float)sum * q_as[row]) * q_ws[col] (+ bias))
   const float* q_as;          // [batch] per-token activation scales
   const float* q_ws;          // [row_w] per-channel weight scales
+  int whole;                  // > 0: several workgroups per pair, this many waves of each keep one whole partition, and every wave's record is merged
 };
 #define FD_QS_MAX 8
 
@@ -251,8 +252,10 @@ __global__ __launch_bounds__(GROUPED ? 64 * FD_GROUP_MAX : 64, GROUPED && D == 6
   const int t = lane & 15, c = lane >> 4;
   // GROUPED: gridDim.x workgroups share a row's partitions (1 unless the launch would leave most of the chip idle, fd_plan): wave
   // ``part`` of all of them walks partitions part, part + walkers, ...
-  const int walkers = GROUPED ? (int)(gridDim.x * (blockDim.x >> 6)) : 1;
-  const int part = GROUPED ? (int)(blockIdx.x * (blockDim.x >> 6)) + wave : (int)blockIdx.x;
+  // (rp.whole: that many waves of a workgroup have a partition each, the others only help to add up and to merge)
+  const int held = GROUPED ? (rp.whole ? rp.whole : (int)(blockDim.x >> 6)) : 1;   // waves with a share
+  const int walkers = GROUPED ? (int)gridDim.x * held : 1;
+  const int part = GROUPED ? (int)blockIdx.x * held + wave : (int)blockIdx.x;
   const int kvh = blockIdx.y % hkv;
   const int hg = blockIdx.y / hkv;
   const int b = blockIdx.z;
@@ -358,18 +361,19 @@ __global__ __launch_bounds__(GROUPED ? 64 * FD_GROUP_MAX : 64, GROUPED && D == 6
   // where smaller ones lost (batch 1 x ctx 300: 697 -> 712 us, batch 64 x ctx 700: 972 -> 981).
   int ptok = FD_PART;
   if constexpr (GROUPED) {
-    if (gridDim.x > 1) ptok = (((int)seq_len + walkers * 32 - 1) / (walkers * 32)) * 32;
+    if (gridDim.x > 1 && !rp.whole) ptok = (((int)seq_len + walkers * 32 - 1) / (walkers * 32)) * 32;
   }
   int64_t start = (int64_t)part * ptok;  // (GROUPED: the wave's FIRST partition; it walks part, part + walkers, ... below)
   if constexpr (GROUPED) {
     if (blockIdx.x > 0 && start - (int64_t)wave * ptok >= seq_len) return;  // a split past the row's end: no wave has work, none merges
+    if (wave >= held) start = seq_len;
   }
   if (start >= seq_len) {  // empty partition stores nothing (flashdecoding.py:141-161)
     publish_q();
     if constexpr (FUSE) {
       // a zero-length row has no merging wave: its first partition writes the 0/0 the reference's
       // stage 2 computes for it (:264-287)
-      if (part == 0 && head_ok) {
+      if (part == 0 && head_ok) {  // (seq_len 0: all waves' starts lie behind it)
         const float nan = __builtin_nanf("");
         for (int dd = c; dd < D; dd += 4) out[b * o_sb + (int64_t)head * o_sh + dd] = from_f32<DT>(nan);
       }
@@ -890,7 +894,7 @@ __global__ __launch_bounds__(GROUPED ? 64 * FD_GROUP_MAX : 64, GROUPED && D == 6
     // serial chain (two expf per record) runs once per thread -- on wave 0 alone it ran 4 times (GQA 7), 1.4 us of the launch's tail.
     constexpr int D4 = D / 4;
     constexpr int REC = 32 * VSTR / 2;
-    const int W = (int)(blockDim.x >> 6);
+    const int W = held;
     const bool shared = gridDim.x > 1;  // (one workgroup keeps whole partitions: no division by ptok)
     const int np = seq_len <= 0 ? 0 : shared ? ((int)seq_len + ptok - 1) / ptok : (int)(seq_len + FD_PART - 1) / FD_PART;
     const int first = (int)blockIdx.x * W;
@@ -905,6 +909,19 @@ __global__ __launch_bounds__(GROUPED ? 64 * FD_GROUP_MAX : 64, GROUPED && D == 6
     const int64_t hr0 = ((int64_t)b * hq + head0) * nparts + blockIdx.x;  // this split's record of the group's first head
     for (int sidx = (int)threadIdx.x; sidx < nvalid * D4; sidx += (int)blockDim.x) {
       const int hl_s = sidx / D4, d4 = sidx % D4;
+      if (rp.whole && splits > 1) {   // the waves' records as they are
+        for (int pp = 0; pp < nrec; ++pp) {
+          const float* rec = recs + pp * REC;
+          const int64_t at = hr0 + (int64_t)hl_s * nparts - (int)blockIdx.x + first + pp;
+          unsigned long long* mo = reinterpret_cast<unsigned long long*>(mid_o + at * D + d4 * 4);
+#pragma unroll
+          for (int e = 0; e < 4; e += 2)
+            __hip_atomic_store(mo + e / 2, *reinterpret_cast<const unsigned long long*>(rec + hl_s * D + d4 * 4 + e), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+          if (d4 == 0) __hip_atomic_store(mid_lse + at * FD_LSE_PAD, rec[16 * D + hl_s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        continue;
+      }
       float mm = -INFINITY, dd = 0.f;
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
       for (int pp = 0; pp < nrec; ++pp) {
@@ -950,17 +967,18 @@ __global__ __launch_bounds__(GROUPED ? 64 * FD_GROUP_MAX : 64, GROUPED && D == 6
     __syncthreads();
     if (*lds_old != splits - 1) return;
     const int64_t hra = ((int64_t)b * hq + head0) * nparts;
+    const int records = rp.whole ? np : splits;
     for (int sidx = (int)threadIdx.x; sidx < nvalid * D4; sidx += (int)blockDim.x) {
       const int hl_s = sidx / D4, d4 = sidx % D4;
       float mm = -INFINITY, dd = 0.f;
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
       constexpr int PB = 8;  // records requested together: one memory round trip per eight splits
-      for (int p0 = 0; p0 < splits; p0 += PB) {
+      for (int p0 = 0; p0 < records; p0 += PB) {
         unsigned long long v[PB][2];
         float l[PB];
 #pragma unroll
         for (int u = 0; u < PB; ++u) {
-          const int64_t rr = hra + (int64_t)hl_s * nparts + (p0 + u < splits ? p0 + u : splits - 1);  // clamped; dropped below
+          const int64_t rr = hra + (int64_t)hl_s * nparts + (p0 + u < records ? p0 + u : records - 1);  // clamped; dropped below
           const unsigned long long* mo = reinterpret_cast<const unsigned long long*>(mid_o + rr * D + d4 * 4);
           v[u][0] = __hip_atomic_load(mo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           v[u][1] = __hip_atomic_load(mo + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -968,7 +986,7 @@ __global__ __launch_bounds__(GROUPED ? 64 * FD_GROUP_MAX : 64, GROUPED && D == 6
         }
 #pragma unroll
         for (int u = 0; u < PB; ++u) {
-          if (p0 + u >= splits) break;
+          if (p0 + u >= records) break;
           const float m_new = fmaxf(mm, l[u]);
           const float alpha = expf(mm - m_new), w = expf(l[u] - m_new);
 #pragma unroll
@@ -1040,22 +1058,24 @@ extern "C" int ll_flash_decoding_num_partitions(int64_t max_len) {
 // 200 - 270 on 8 KV heads of 4 134 / 239 / 47.
 // Heads of 256 spill 400 registers in a grouped workgroup (27 rows on 4 KV heads of 4, 3000 tokens 55 / 140): they take it only where the
 // last arriver alone would merge very many partitions (2 pairs, 32 768 tokens 160 / 75; 16 pairs, 16 384 140 / 118).
-// Five to eight partitions at up to 64 pairs, heads of 128: workgroups of four waves, as many per pair as leave each a CU to itself -- a CU takes in
-// some 27 KB a microsecond whatever its waves, and a row of 1000 tokens is 512 KB.  us, one workgroup / here, longest row 520 | 700 | 1000 tokens:
-// 4 pairs of 7 heads 12.1 / 10.5 | 15.3 / 10.8 | 19.2 / 10.6; 64 of 7 12.3 / 11.4 | 15.6 / 12.2 | 19.7 / 12.4; 64 of 8 11.9 / 11.1 | 15.8 / 12.1 |
-// 20.0 / 12.6.  Not from 100 pairs on (12.5 / 13.2 at 520), not for heads of 64 (7.6 / 7.8 at 8 pairs, 7.7 / 8.8 at 120), not up to four partitions
-// (300 tokens 9.0 / 10.2).
+// Five to eight partitions, heads of 128, few pairs: a wave per partition as before, but two to a workgroup, as long as every workgroup finds a CU of its
+// own -- a CU takes in some 27 KB a microsecond whatever its waves, and a row of 1000 tokens is 512 KB.  Every wave's record goes to the workgroup
+// that arrives last, which merges them in order: the bits of one workgroup.  us, one workgroup / here, longest row 520 | 600 | 700 | 1000 tokens: 4
+// pairs of 7 heads 11.8 / 11.9 | 13.0 / 12.0 | 15.4 / 12.7 | 19.3 / 13.3; 64 of 7 12.3 / 13.2 | 13.5 / 13.1 | 15.8 / 13.8 | 19.7 / 14.8; 64 of 4 12.2 /
+// 11.7 | 14.1 / 11.8 | 15.9 / 12.1 | 19.7 / 12.6.  Even shares of four waves each, in whose order sums round otherwise: 19.2 / 10.6 at 1000.  Not up to
+// four partitions (300 tokens 9.0 / 10.2), not for heads of 64 (500 tokens 7.4 / 8.4).
 #define FD_LOOP_MAX 256  // partitions (32 768 tokens)
 struct FdPlan {
   int waves, splits;
+  int whole = 0;  // > 0: several workgroups, that many of whose waves keep whole partitions
 };
 // (planes: q|k|v come as sums to be added up, two float4 slots a lane; merge: the caller lends the scratch that workgroups of a pair meet in)
 static FdPlan fd_plan(int64_t max_len, int64_t pairs, int heads, int d, bool planes, bool merge) {
   const int64_t np = (max_len + FD_PART - 1) / FD_PART;
   if (np < 2 || np > FD_LOOP_MAX || pairs < 1) return {0, 0};
   if (np <= FD_GROUP_MAX) {
-    const int64_t room = 256 / pairs, most = (np + 1) / 2;
-    if (np > 4 && pairs <= 64 && d == 128 && merge && (!planes || (heads + 2) * d / 4 <= 128 * 4)) return {4, (int)(room < most ? room : most)};
+    const int64_t splits = (np + 1) / 2, waves = ((heads + 2) * d / 4 + 127) / 128;   // (q|k|v as planes: two float4 slots a lane)
+    if (np > 4 && pairs * splits <= 256 && d == 128 && merge) return {(int)(waves < 2 ? 2 : waves), (int)splits, 2};
     return {(int)np, 1};
   }
   static const bool no_loop = getenv("LL_FD_NO_LOOP") != nullptr;  // A/B knob, read once
@@ -1101,6 +1121,7 @@ static int launch_fd(void* out, const void* q, const void* kc, const void* vc, c
   FdPlan plan = fd_plan(max_len, pairs, groups < 16 ? groups : 16, d, rope && rp.qp, mid_o && mid_lse);
   // (planes without the scratch of a merge between workgroups: one workgroup walks a pair's whole context, as from 128 pairs on)
   if (rope && rp.qp && !(mid_o && mid_lse)) plan.splits = 1;
+  rp.whole = plan.splits > 1 ? plan.whole : 0;
   const int gw = plan.waves;  // waves of a grouped workgroup; 0: not grouped
   const bool grouped_ok = fuse && gw >= 2 && (plan.splits == 1 || (mid_o && mid_lse));
   // split-K partial inputs need the grouped form and two float4 slots per lane: (groups + 2) * d / 4 <= 2 * 64 * waves

@@ -437,11 +437,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
 }
 
 constexpr int fa2_lds(int d) { return 2 * 2 * 64 * (d + 8) * 2; }
-// (more than a launch may have without being asked for)
 template <int DT, int D, int QB, int ROPE = -1>
 static bool fa2_ready() {
-  static const hipError_t wide = hipFuncSetAttribute((const void*)fa_prefill2<DT, D, QB, ROPE>, hipFuncAttributeMaxDynamicSharedMemorySize, fa2_lds(D));
-  return wide == hipSuccess;
+  static std::atomic<uint64_t> asked{0};
+  return ll_wide_lds((const void*)fa_prefill2<DT, D, QB, ROPE>, fa2_lds(D), asked);
 }
 
 template <int DT>

@@ -82,9 +82,10 @@ __device__ __forceinline__ float shaped_score(float dot, const ScoreShape& sh, f
 // from all maxima, the weights; (3) a wave each takes 16 channels of the result through all tiles in order.  Every sum is formed in the order
 // of the walk: the bits are those of one wave.  Reads are unconditional -- rows behind the range repeat its last one, channels behind the width its
 // first, cleared in registers where they would count -- since a read inside a branch is waited for there.
-// us a launch, one wave per partition -> here, bit for bit: 32 sequences of 60 - 144 tokens, 16 heads of 128 on 4 17.5 -> 7.4; 8 of 256 - 512 27.5 -> 14.0;
-// 64 of 1000 - 2000 (fp16) 79.5 -> 73.3; heads of 256, 9 of up to 2700 69.7 -> 53.2; a latent of 256, 9 of up to 1700 42.9 -> 23.0.  (One wave with
-// unconditional reads, two tiles in flight: 14.1, 22.1, 60.7, 72.7, 36.2.)
+// us a launch, one wave per partition -> here, bit for bit: 32 sequences of 60 - 144 tokens, 16 heads of 128 on 4 17.5 -> 6.7; 8 of 256 - 512 27.5 -> 13.2;
+// 64 of 1000 - 2000 (fp16) 79.5 -> 58.3; heads of 256, 9 of up to 2700 69.7 -> 50.2; a latent of 256, 9 of up to 1700 42.9 -> 22.3.  (One wave with
+// unconditional reads, two tiles in flight: 14.1, 22.1, 60.7, 72.7, 36.2.  Keys of every width in one form: registers spill in front of the products,
+// 7.4, 14.0, 73.3, 53.2, 23.0.)
 constexpr int kTiles = kPart / 32;   // and waves of a workgroup
 
 // LDS: value rows of all tiles, [tile][32][VSTR]; weights in two 16-bit parts, [tile][part][c][columns] x 16 B; per tile and column the
@@ -95,7 +96,8 @@ __host__ __device__ constexpr int decode_lds(int group) {
   return kTiles * 32 * (NTM * 16 + 8) * 2 + kTiles * 2 * 4 * decode_columns(group) * 16 + 3 * kTiles * 16 * 4;
 }
 
-template <int DT, int NSM, int NTM, bool BIASED, bool SHARED>
+// FULL: keys as wide as the form, all pieces of a row at fixed distances from one address
+template <int DT, int NSM, int NTM, bool BIASED, bool SHARED, bool FULL>
 __global__ __launch_bounds__(64 * kTiles, NSM <= 4 ? 4 : 2) void ragged_attention_mfma_decode_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
     const int32_t* __restrict__ token_table, int64_t tt_stride, const int32_t* __restrict__ seq_req,
@@ -169,26 +171,22 @@ __global__ __launch_bounds__(64 * kTiles, NSM <= 4 ? 4 : 2) void ragged_attentio
     const uint16_t* kB = k_cache + rb * k_stride + (int64_t)g * dk;
     const uint16_t* vA = v_cache + ra * v_stride + (int64_t)g * dv;
     const uint16_t* vB = v_cache + rb * v_stride + (int64_t)g * dv;
-    auto load = [&](auto full) {   // full: heads as wide as the form, all pieces of a row at fixed distances from one address
 #pragma unroll
-      for (int s = 0; s < NSM; ++s) {
-        const int ch = 8 * (4 * s + c), at = full.value || ch < dk ? ch : 0;
-        qf[s] = *reinterpret_cast<const Q4*>(qrow + at);
-        ka[s] = *reinterpret_cast<const Q4*>(kA + at);
-        kb[s] = *reinterpret_cast<const Q4*>(kB + at);
-      }
-      if constexpr (!SHARED) {
+    for (int s = 0; s < NSM; ++s) {
+      const int ch = 8 * (4 * s + c), at = FULL || ch < dk ? ch : 0;
+      qf[s] = *reinterpret_cast<const Q4*>(qrow + at);
+      ka[s] = *reinterpret_cast<const Q4*>(kA + at);
+      kb[s] = *reinterpret_cast<const Q4*>(kB + at);
+    }
+    if constexpr (!SHARED) {
 #pragma unroll
-        for (int s = 0; s < NTM / 2; ++s) {
-          const int ch = 8 * (4 * s + c), at = full.value || ch < dv ? ch : 0;
-          va[s] = *reinterpret_cast<const Q4*>(vA + at);
-          vb[s] = *reinterpret_cast<const Q4*>(vB + at);
-        }
+      for (int s = 0; s < NTM / 2; ++s) {
+        const int ch = 8 * (4 * s + c), at = ch < dv ? ch : 0;
+        va[s] = *reinterpret_cast<const Q4*>(vA + at);
+        vb[s] = *reinterpret_cast<const Q4*>(vB + at);
       }
-    };
-    if (dk == 32 * NSM && (SHARED || dv == 16 * NTM)) load(std::true_type{});
-    else load(std::false_type{});
-    if (dk & 31) {   // (past the width a query is zero, and so must the key be: 0 times infinity is no number)
+    }
+    if constexpr (!FULL) {   // (past the width a query is zero, and so must the key be: 0 times infinity is no number)
 #pragma unroll
       for (int s = 0; s < NSM; ++s) {
         const uint32_t in = 8 * (4 * s + c) < dk ? ~0u : 0u;
@@ -659,11 +657,11 @@ extern "C" int ll_ragged_attention_mfma(const void* q, const void* k_cache, cons
   const HeadGate gate = {(const uint16_t*)head_gate, gate_ld};
   const ScoreShape shape = {scale, cap, dist_bias, dist_bias ? (int)dist_n : 1};
 #define CALL_DB(DT, NS, NT, B) if (shared_kv) { CALL_DS(DT, NS, NT, B, true); } else { CALL_DS(DT, NS, NT, B, false); }
-#define CALL_DS(DT, NS, NT, B, S)                                                                                                \
-  static const hipError_t wide_ = hipFuncSetAttribute((const void*)ragged_attention_mfma_decode_kernel<DT, NS, NT, B, S>,          \
-                                                      hipFuncAttributeMaxDynamicSharedMemorySize, decode_lds<NT>(16));           \
-  if (wide_ != hipSuccess) return LL_ERR_LAUNCH;                                                                                 \
-  ragged_attention_mfma_decode_kernel<DT, NS, NT, B, S><<<grid, 64 * kTiles, decode_lds<NT>(group), st>>>(                        \
+#define CALL_DS(DT, NS, NT, B, S) if (dk == 32 * NS) { CALL_DF(DT, NS, NT, B, S, true); } else { CALL_DF(DT, NS, NT, B, S, false); }
+#define CALL_DF(DT, NS, NT, B, S, F)                                                                                             \
+  static std::atomic<uint64_t> asked_{0};                                                                                        \
+  if (!ll_wide_lds((const void*)ragged_attention_mfma_decode_kernel<DT, NS, NT, B, S, F>, decode_lds<NT>(16), asked_)) return LL_ERR_LAUNCH; \
+  ragged_attention_mfma_decode_kernel<DT, NS, NT, B, S, F><<<grid, 64 * kTiles, decode_lds<NT>(group), st>>>(                        \
       (const uint16_t*)q, (const uint16_t*)k_cache, (const uint16_t*)v_cache, token_table, tt_stride, seq_req, seq_start,    \
       seq_first_pos, (const uint16_t*)sink, scale_log2, (uint16_t*)out, partials, max_parts, (int)heads, (int)kv_heads, (int)dk, \
       (int)dv, k_stride, v_stride, (int)window, (int)keep_first, out_stride, shape, gate)
@@ -701,6 +699,7 @@ extern "C" int ll_ragged_attention_mfma(const void* q, const void* k_cache, cons
 #undef CALL_D
 #undef CALL_DB
 #undef CALL_DS
+#undef CALL_DF
   if (decode && max_parts > 1) {
     const int64_t waves = n * heads;
     if (dtype == LL_F16)

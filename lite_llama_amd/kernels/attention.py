@@ -244,7 +244,7 @@ def decode_attention_partials(parts, bias, num_heads: int, num_kv_heads: int, he
     fn, merge = L.lib().ll_decode_attention_partials, ()
     pairs = batchs * num_kv_heads
     counters = None   # several workgroups share a row: scratch of their merge
-    if (max_len > 1024 and pairs < 128) or (max_len > 512 and pairs <= 64 and head_dim == 128):
+    if (max_len > 1024 and pairs < 128) or (max_len > 512 and pairs <= 85 and head_dim == 128):
         counters = _merge_counters(p.device, pairs)
         if counters is None and max_len > 1024:
             return None

@@ -169,7 +169,7 @@ def test_projection_planes_are_taken_from_64_pairs_on():
     assert not decode_attention_partials_supported(longest, hq, hkv, d, batch=31)
 
 
-# five to eight partitions: several workgroups of four waves per pair up to 64 pairs of heads of 128, one workgroup beside that line and without scratch
+# five to eight partitions: several workgroups of two partitions per pair where all of them find a CU (heads of 128), one workgroup beside that line
 @pytest.mark.parametrize("b,hkv,rep,d,longest,bound", [(1, 1, 1, 128, 513, 640), (1, 4, 7, 128, 1000, 1024), (3, 2, 16, 128, 1024, 1024), (16, 4, 8, 128, 700, 768),
                                                        (13, 5, 3, 128, 900, 1024), (2, 2, 15, 128, 640, 640), (9, 2, 7, 64, 1000, 1024)])
 def test_middle_contexts(b, hkv, rep, d, longest, bound):
