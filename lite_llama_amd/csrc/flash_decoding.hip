@@ -1070,7 +1070,7 @@ struct FdPlan {
   int whole = 0;  // > 0: several workgroups, that many of whose waves keep whole partitions
 };
 // (planes: q|k|v come as sums to be added up, two float4 slots a lane; merge: the caller lends the scratch that workgroups of a pair meet in)
-static FdPlan fd_plan(int64_t max_len, int64_t pairs, int heads, int d, bool planes, bool merge) {
+static FdPlan fd_plan(int64_t max_len, int64_t pairs, int heads, int d, bool planes, bool merge = false) {
   const int64_t np = (max_len + FD_PART - 1) / FD_PART;
   if (np < 2 || np > FD_LOOP_MAX || pairs < 1) return {0, 0};
   if (np <= FD_GROUP_MAX) {
