@@ -83,10 +83,10 @@ struct FdRope {
   // QI32 (smoothquant q|k|v): the planes at qp are EXACT int32 sums; value = fp16(((float)sum * q_as[row]) * q_ws[col] (+ bias))
   const float* q_as;          // [batch] per-token activation scales
   const float* q_ws;          // [row_w] per-channel weight scales
-  int whole;                  // > 0: several workgroups per pair, this many waves of each keep one whole partition, and every wave's record is merged
 };
 #define FD_QS_MAX 8
 
+#define FD_WHOLE 2  // whole partitions of a workgroup where several share up to FD_GROUP_MAX
 // grid = (nparts, hkv * head_groups, batch), block = 64 (one wave)
 // FUSE: the wave that finishes the LAST non-empty partition of its (row, KV head group) also does the
 // log-sum-exp merge and writes ``out`` (no second launch: a kernel boundary costs ~4.7 us in the
@@ -225,7 +225,9 @@ __device__ __forceinline__ void fd_head_norm(Q4 (&qf)[4], const Q4 (&wf)[4], flo
   for (int s = 0; s < 4; ++s) qf[s] = fd_scale8<DT>(qf[s], wf[s], rr);
 }
 
-template <int DT, int D, bool FUSE, bool ROPE, int GS, bool GROUPED, bool KV8 = false, bool QKN = false, bool QI32 = false>
+// WHOLE: up to FD_GROUP_MAX partitions in several workgroups; FD_WHOLE waves of each keep a whole partition, the others only help to add up and to
+// merge (a form of its own: asked at run time it cost every launch 0.9 us, through spilled scalars)
+template <int DT, int D, bool FUSE, bool ROPE, int GS, bool GROUPED, bool KV8 = false, bool QKN = false, bool QI32 = false, bool WHOLE = false>
 __global__ __launch_bounds__(GROUPED ? 64 * FD_GROUP_MAX : 64, GROUPED && D == 64 ? 4 : 1) void fd_stage1(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
     const int32_t* __restrict__ table, const void* __restrict__ b_req_idx,
@@ -252,8 +254,8 @@ __global__ __launch_bounds__(GROUPED ? 64 * FD_GROUP_MAX : 64, GROUPED && D == 6
   const int t = lane & 15, c = lane >> 4;
   // GROUPED: gridDim.x workgroups share a row's partitions (1 unless the launch would leave most of the chip idle, fd_plan): wave
   // ``part`` of all of them walks partitions part, part + walkers, ...
-  // (rp.whole: that many waves of a workgroup have a partition each, the others only help to add up and to merge)
-  const int held = GROUPED ? (rp.whole ? rp.whole : (int)(blockDim.x >> 6)) : 1;   // waves with a share
+  static_assert(!WHOLE || GROUPED, "several workgroups of waves");
+  const int held = WHOLE ? FD_WHOLE : GROUPED ? (int)(blockDim.x >> 6) : 1;   // waves with a share
   const int walkers = GROUPED ? (int)gridDim.x * held : 1;
   const int part = GROUPED ? (int)blockIdx.x * held + wave : (int)blockIdx.x;
   const int kvh = blockIdx.y % hkv;
@@ -361,12 +363,12 @@ __global__ __launch_bounds__(GROUPED ? 64 * FD_GROUP_MAX : 64, GROUPED && D == 6
   // where smaller ones lost (batch 1 x ctx 300: 697 -> 712 us, batch 64 x ctx 700: 972 -> 981).
   int ptok = FD_PART;
   if constexpr (GROUPED) {
-    if (gridDim.x > 1 && !rp.whole) ptok = (((int)seq_len + walkers * 32 - 1) / (walkers * 32)) * 32;
+    if (!WHOLE && gridDim.x > 1) ptok = (((int)seq_len + walkers * 32 - 1) / (walkers * 32)) * 32;
   }
   int64_t start = (int64_t)part * ptok;  // (GROUPED: the wave's FIRST partition; it walks part, part + walkers, ... below)
   if constexpr (GROUPED) {
     if (blockIdx.x > 0 && start - (int64_t)wave * ptok >= seq_len) return;  // a split past the row's end: no wave has work, none merges
-    if (wave >= held) start = seq_len;
+    if (WHOLE && wave >= FD_WHOLE) start = seq_len;
   }
   if (start >= seq_len) {  // empty partition stores nothing (flashdecoding.py:141-161)
     publish_q();
@@ -909,7 +911,7 @@ __global__ __launch_bounds__(GROUPED ? 64 * FD_GROUP_MAX : 64, GROUPED && D == 6
     const int64_t hr0 = ((int64_t)b * hq + head0) * nparts + blockIdx.x;  // this split's record of the group's first head
     for (int sidx = (int)threadIdx.x; sidx < nvalid * D4; sidx += (int)blockDim.x) {
       const int hl_s = sidx / D4, d4 = sidx % D4;
-      if (rp.whole && splits > 1) {   // the waves' records as they are
+      if (WHOLE && splits > 1) {   // the waves' records as they are
         for (int pp = 0; pp < nrec; ++pp) {
           const float* rec = recs + pp * REC;
           const int64_t at = hr0 + (int64_t)hl_s * nparts - (int)blockIdx.x + first + pp;
@@ -967,7 +969,7 @@ __global__ __launch_bounds__(GROUPED ? 64 * FD_GROUP_MAX : 64, GROUPED && D == 6
     __syncthreads();
     if (*lds_old != splits - 1) return;
     const int64_t hra = ((int64_t)b * hq + head0) * nparts;
-    const int records = rp.whole ? np : splits;
+    const int records = WHOLE ? np : splits;
     for (int sidx = (int)threadIdx.x; sidx < nvalid * D4; sidx += (int)blockDim.x) {
       const int hl_s = sidx / D4, d4 = sidx % D4;
       float mm = -INFINITY, dd = 0.f;
@@ -1067,15 +1069,14 @@ extern "C" int ll_flash_decoding_num_partitions(int64_t max_len) {
 #define FD_LOOP_MAX 256  // partitions (32 768 tokens)
 struct FdPlan {
   int waves, splits;
-  int whole = 0;  // > 0: several workgroups, that many of whose waves keep whole partitions
 };
 // (planes: q|k|v come as sums to be added up, two float4 slots a lane; merge: the caller lends the scratch that workgroups of a pair meet in)
 static FdPlan fd_plan(int64_t max_len, int64_t pairs, int heads, int d, bool planes, bool merge = false) {
   const int64_t np = (max_len + FD_PART - 1) / FD_PART;
   if (np < 2 || np > FD_LOOP_MAX || pairs < 1) return {0, 0};
   if (np <= FD_GROUP_MAX) {
-    const int64_t splits = (np + 1) / 2, waves = ((heads + 2) * d / 4 + 127) / 128;   // (q|k|v as planes: two float4 slots a lane)
-    if (np > 4 && pairs * splits <= 256 && d == 128 && merge) return {(int)(waves < 2 ? 2 : waves), (int)splits, 2};
+    const int64_t splits = (np + FD_WHOLE - 1) / FD_WHOLE, waves = ((heads + 2) * d / 4 + 127) / 128;   // (q|k|v as planes: two float4 slots a lane)
+    if (np > 4 && pairs * splits <= 256 && d == 128 && merge) return {(int)(waves < FD_WHOLE ? FD_WHOLE : waves), (int)splits};
     return {(int)np, 1};
   }
   static const bool no_loop = getenv("LL_FD_NO_LOOP") != nullptr;  // A/B knob, read once
@@ -1121,7 +1122,7 @@ static int launch_fd(void* out, const void* q, const void* kc, const void* vc, c
   FdPlan plan = fd_plan(max_len, pairs, groups < 16 ? groups : 16, d, rope && rp.qp, mid_o && mid_lse);
   // (planes without the scratch of a merge between workgroups: one workgroup walks a pair's whole context, as from 128 pairs on)
   if (rope && rp.qp && !(mid_o && mid_lse)) plan.splits = 1;
-  rp.whole = plan.splits > 1 ? plan.whole : 0;
+  const bool whole = plan.splits > 1 && nparts <= FD_GROUP_MAX;
   const int gw = plan.waves;  // waves of a grouped workgroup; 0: not grouped
   const bool grouped_ok = fuse && gw >= 2 && (plan.splits == 1 || (mid_o && mid_lse));
   // split-K partial inputs need the grouped form and two float4 slots per lane: (groups + 2) * d / 4 <= 2 * 64 * waves
@@ -1132,17 +1133,22 @@ static int launch_fd(void* out, const void* q, const void* kc, const void* vc, c
   const bool grouped = grouped_ok && !ungrouped_env;
 #define LL_FD1X(DD, FU, RO, GG, GR) LL_FD1XK(DD, FU, RO, GG, GR, false, false, false)
 #define LL_FD1XK(DD, FU, RO, GG, GR, K8, QN, QI)                                                            \
+  if constexpr ((GR) && (DD) == 128) {                                                                      \
+    if (whole) LL_FD1XW(DD, FU, RO, GG, GR, K8, QN, QI, true)                                               \
+    else LL_FD1XW(DD, FU, RO, GG, GR, K8, QN, QI, false)                                                    \
+  } else LL_FD1XW(DD, FU, RO, GG, GR, K8, QN, QI, false)
+#define LL_FD1XW(DD, FU, RO, GG, GR, K8, QN, QI, WH)                                                        \
   {                                                                                                  \
     constexpr int tile_bytes_ = 32 * (DD + 8) * 2;                                                   \
     if (GR) {                                                                                        \
       static bool attr_ = false;                                                                     \
       if (!attr_) {                                                                                  \
-        (void)hipFuncSetAttribute((const void*)fd_stage1<DT, DD, FU, RO, GG, GR, K8, QN, QI>,             \
+        (void)hipFuncSetAttribute((const void*)fd_stage1<DT, DD, FU, RO, GG, GR, K8, QN, QI, WH>,             \
                                   hipFuncAttributeMaxDynamicSharedMemorySize, FD_GROUP_MAX * tile_bytes_ + 18 * DD * 2); \
         attr_ = true;                                                                                \
       }                                                                                              \
     }                                                                                                \
-    fd_stage1<DT, DD, FU, RO, GG, GR, K8, QN, QI><<<(GR) ? dim3((unsigned)plan.splits, grid.y, grid.z) : grid, (GR) ? 64 * gw : 64, \
+    fd_stage1<DT, DD, FU, RO, GG, GR, K8, QN, QI, WH><<<(GR) ? dim3((unsigned)plan.splits, grid.y, grid.z) : grid, (GR) ? 64 * gw : 64, \
                                         ((GR) ? gw : 1) * tile_bytes_ + ((GR) ? 18 * DD * 2 : 0), st>>>( \
         (const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc, table, req, seq, mid_o, mid_lse, hq, hkv, nparts, \
         scale, q_sb, q_sh, k_st, k_sh, v_st, v_sh, t_sb, req_w, seq_w, (uint16_t*)out, o_sb, o_sh, counters, rp); \
@@ -1212,6 +1218,7 @@ static int launch_fd(void* out, const void* q, const void* kc, const void* vc, c
 #undef LL_FD1G
 #undef LL_FD1
 #undef LL_FD1XK
+#undef LL_FD1XW
 #undef LL_FD1X
   if (!fuse)
     fd_stage2<DT><<<dim3((unsigned)hq, (unsigned)batch), d, 0, st>>>((uint16_t*)out, mid_o, mid_lse, seq, hq, d,
