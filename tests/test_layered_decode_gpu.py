@@ -102,3 +102,73 @@ def test_what_goes_through_the_modules(monkeypatch, what):
     monkeypatch.setattr(model_layers, "decode_layer", lambda *a: None)
     want, _ = _run(model, 2)
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+class _Recorded:
+    """The library, with a native layer call that is counted and not served: nothing is launched."""
+
+    def __init__(self, lib):
+        self._lib, self.asked = lib, 0
+
+    def __getattr__(self, name):
+        return getattr(self._lib, name)
+
+    def ll_layered_decode_bytes(self, *args):
+        self.asked += 1
+        return 0
+
+
+def _places(layer, x, pending, cache, run):
+    """Every tensor that the layer's call hands on: (name, its container, its key)."""
+    out = [(f"{name}.{key}", module._parameters, key) for name, module in layer.named_modules() for key, p in module._parameters.items()
+           if p is not None and (name, key) not in (("", "norm2_weight"), ("mlp", "down_bias"))]      # (these ride on with the result)
+    for kind, group in (("recurrent", cache.recurrent), ("conv", cache.conv)):
+        if group[run] is not None:
+            out.append((kind, group, run))
+    for i in range(2 if cache.kv_buffer[run] is not None else 0):
+        out.append((f"kv {i}", cache.kv_buffer[run], i))
+    keys = ("y", "post_weight", "shared", "shared_scale", "bias") if hasattr(pending, "y") else ("rows",)
+    return out + [(key, pending, key) for key in keys if getattr(pending, key) is not None]
+
+
+@pytest.mark.parametrize("at", [0, 1, 2, 3])
+def test_an_operand_elsewhere_is_refused(monkeypatch, at):
+    """Every operand of a layer on the host in its turn: the call is refused before it is made, as the modules' wrappers refuse it."""
+    from lite_llama_amd import layered_decode, model_layers
+    from lite_llama_amd.executor.ragged import RaggedRunner
+
+    model = _model(T.CONFIGS["mix"], torch.bfloat16)
+    lib, real, checked = _Recorded(layered_decode.L.lib()), model_layers.decode_layer, []
+
+    def look(layer, x, pending, step, cache, run, table, *kinds):
+        if layer is not model.layers[at] or step.longest_run != 1:
+            return real(layer, x, pending, step, cache, run, table, *kinds)
+        cache.kv_buffer[run] = list(cache.kv_buffer[run]) if cache.kv_buffer[run] is not None else None
+        with monkeypatch.context() as m:
+            m.setattr(layered_decode.L, "lib", lambda: lib)
+            m.setattr(layered_decode.L, "has", lambda name: True)
+
+            def asked(x=x, table=table):
+                lib.asked = 0
+                assert real(layer, x, pending, step, cache, run, table, *kinds) is None
+                return lib.asked
+
+            assert asked() == 1
+            assert asked(x=x.cpu()) == 0 and asked(table=table.cpu()) == 0
+            for name, held, key in _places(layer, x, pending, cache, run):
+                own = held[key] if isinstance(held, (dict, list)) else getattr(held, key)
+                away = torch.nn.Parameter(own.detach().cpu(), requires_grad=False) if isinstance(own, torch.nn.Parameter) else own.cpu()
+                put = held.__setitem__ if isinstance(held, (dict, list)) else lambda k, v: setattr(held, k, v)
+                put(key, away)
+                assert asked() == 0, name
+                put(key, own)
+                checked.append(name)
+            assert asked() == 1
+        return real(layer, x, pending, step, cache, run, table, *kinds)
+
+    monkeypatch.setattr(model_layers, "decode_layer", look)
+    runner = RaggedRunner(model, 64, 1, block_size=16, device=DEV)
+    slot = runner.admit()
+    runner.step([(slot, [1, 2, 3])])
+    assert torch.isfinite(runner.step([(slot, [4])]).float()).all()
+    assert len(checked) >= 8
