@@ -143,6 +143,7 @@ def _decode(layer, x, pending, step, cache, run, token_table, mixers, feed_forwa
     _need(not (_nn._global_forward_hooks or _nn._global_forward_pre_hooks) and _plain(mixer, type(mixer)) and (mlp is None or _plain(mlp, type(mlp))))
     _need(forward_ad._current_level < 0 and _transform_level() is None and _dispatch_modes() == 0 and not torch.is_autocast_enabled()
           and _tracing_state() is None)
+    _need(mixer.eps == layer.eps)   # (one number for all norms of the layer)
     dt, device, here = norm.dtype, x.device, x.get_device()
     _need(here >= 0 and token_table.dtype == torch.int32 and token_table.stride(1) == 1 and token_table.get_device() == here)
     at = step.shared.get("decode")

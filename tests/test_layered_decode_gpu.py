@@ -73,7 +73,7 @@ def test_the_same_bits_as_single_launches(monkeypatch, name, batch, dtype):
     assert len(kept) == len(old) and all(torch.equal(a, b) for a, b in zip(kept, old))
 
 
-@pytest.mark.parametrize("what", ["odd", "one", "fp32", "hook", "grad", "env", "replaced"])
+@pytest.mark.parametrize("what", ["odd", "one", "fp32", "hook", "grad", "env", "replaced", "eps"])
 def test_what_goes_through_the_modules(monkeypatch, what):
     from lite_llama_amd import model_layers
 
@@ -85,6 +85,9 @@ def test_what_goes_through_the_modules(monkeypatch, what):
             layer.mixer.in_proj.register_forward_hook(lambda *a: seen.append(1))
     if what == "env":
         monkeypatch.setenv("LL_DENSE16_NARROW_OFF", "1")
+    if what == "eps":
+        for layer in model.layers:
+            layer.mixer.eps = 0.5          # (its own norms', not the layer's)
     if what == "replaced":
         first.mixer.in_proj.weight = torch.nn.Parameter(first.mixer.in_proj.weight.detach().t().contiguous().t(), requires_grad=False)
     if what == "grad":
