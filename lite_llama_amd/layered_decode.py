@@ -146,10 +146,7 @@ def _decode(layer, x, pending, step, cache, run, token_table, mixers, feed_forwa
     _need(mixer.eps == layer.eps)   # (one number for all norms of the layer)
     dt, device, here = norm.dtype, x.device, x.get_device()
     _need(here >= 0 and token_table.dtype == torch.int32 and token_table.stride(1) == 1 and token_table.get_device() == here)
-    at = step.shared.get("decode")
-    if at is None:   # (of this step's own tensors, for as long as it lives)
-        at = step.shared["decode"] = [t.data_ptr() for t in (step.tok_seq, step.tok_pos, step.select, step.seq_start, step.seq_first_pos, step.seq_slot,
-                                                             step.seq_parity)]
+    at = [t.data_ptr() for t in (step.tok_seq, step.tok_pos, step.select, step.seq_start, step.seq_first_pos, step.seq_slot, step.seq_parity)]
     norm1 = _vector(layer, "norm1_weight", here, dt, width)
     middle, scales = take(mixer, here, dt, width, step, cache, run, device)
     if mlp is None:

@@ -3,6 +3,7 @@ logits and in everything the cache keeps, over every mixer and feed-forward, eac
 plain goes through the modules."""
 
 import copy
+import ctypes
 
 import pytest
 import torch
@@ -116,8 +117,9 @@ class _Recorded:
     def __getattr__(self, name):
         return getattr(self._lib, name)
 
-    def ll_layered_decode_bytes(self, *args):
+    def ll_layered_decode_bytes(self, args, count, *floats):
         self.asked += 1
+        self.args = list((ctypes.c_int64 * count).from_address(args))
         return 0
 
 
@@ -175,3 +177,29 @@ def test_an_operand_elsewhere_is_refused(monkeypatch, at):
     runner.step([(slot, [1, 2, 3])])
     assert torch.isfinite(runner.step([(slot, [4])]).float()).all()
     assert len(checked) >= 8
+
+
+def test_a_layer_reads_the_step_as_it_is(monkeypatch):
+    """A step's vector that is replaced between two layers: the next layer is handed the new one."""
+    from lite_llama_amd import layered_decode, model_layers
+    from lite_llama_amd.executor.ragged import RaggedRunner
+
+    model = _model(T.CONFIGS["mix"], torch.bfloat16)
+    lib, real, seen = _Recorded(layered_decode.L.lib()), model_layers.decode_layer, []
+
+    def look(layer, x, pending, step, *rest):
+        if step.longest_run == 1:
+            step.tok_pos = step.tok_pos.clone()
+            seen.append(step.tok_pos)
+            with monkeypatch.context() as m:
+                m.setattr(layered_decode.L, "lib", lambda: lib)
+                assert real(layer, x, pending, step, *rest) is None
+            assert step.tok_pos.data_ptr() in lib.args
+        return None
+
+    monkeypatch.setattr(model_layers, "decode_layer", look)
+    runner = RaggedRunner(model, 64, 1, block_size=16, device=DEV)
+    slot = runner.admit()
+    runner.step([(slot, [1, 2, 3])])
+    runner.step([(slot, [4])])
+    assert len(seen) == len(model.run_order) > 1
