@@ -232,7 +232,8 @@ bool readable(const int64_t* args, int64_t count, const double* floats, int64_t 
     return false;
   const LayeredDecode& a = *reinterpret_cast<const LayeredDecode*>(args);
   return (a.dtype == LL_F16 || a.dtype == LL_BF16) && a.tokens >= 1 && a.tokens <= 64 && a.seqs == a.tokens && a.mixer >= 0 && a.mixer <= 2 &&
-         a.mlp >= 0 && a.mlp <= 2 && a.qk_heads >= 1 && a.heads % a.qk_heads == 0 && a.width >= 8 && a.width % 8 == 0;
+         a.mlp >= 0 && a.mlp <= 2 && a.qk_heads >= 1 && a.heads % a.qk_heads == 0 && a.width >= 8 && a.width % 8 == 0 &&
+         ll_aligned16(a.first);   // (what the first product reads; all other rows are this file's own)
 }
 
 }  // namespace

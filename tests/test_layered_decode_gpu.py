@@ -74,7 +74,7 @@ def test_the_same_bits_as_single_launches(monkeypatch, name, batch, dtype):
     assert len(kept) == len(old) and all(torch.equal(a, b) for a, b in zip(kept, old))
 
 
-@pytest.mark.parametrize("what", ["odd", "one", "fp32", "hook", "grad", "env", "replaced", "eps"])
+@pytest.mark.parametrize("what", ["odd", "one", "fp32", "hook", "grad", "env", "replaced", "eps", "off"])
 def test_what_goes_through_the_modules(monkeypatch, what):
     from lite_llama_amd import model_layers
 
@@ -91,6 +91,15 @@ def test_what_goes_through_the_modules(monkeypatch, what):
             layer.mixer.eps = 0.5          # (its own norms', not the layer's)
     if what == "replaced":
         first.mixer.in_proj.weight = torch.nn.Parameter(first.mixer.in_proj.weight.detach().t().contiguous().t(), requires_grad=False)
+    if what == "off":                      # (the rows that open the stack, off a 16-byte border)
+        rows_of = model_layers.embed_rows
+
+        def moved(*args):
+            x, opening = rows_of(*args)
+            room = torch.empty(opening.rows.numel() + 1, dtype=opening.rows.dtype, device=DEV)[1:].view(opening.rows.shape)
+            return x, model_layers.FirstRows(room.copy_(opening.rows))
+
+        monkeypatch.setattr(model_layers, "embed_rows", moved)
     if what == "grad":
         inner = model_layers.decode_layer
 
@@ -101,7 +110,7 @@ def test_what_goes_through_the_modules(monkeypatch, what):
         monkeypatch.setattr(model_layers, "decode_layer", with_grad)
     served = _count(monkeypatch)
     got, _ = _run(model, 2)
-    assert not any(served[0::len(model.run_order)]) if what == "replaced" else not any(served)
+    assert not any(served[0::len(model.run_order)]) if what in ("replaced", "off") else not any(served)
     assert not seen or len(seen) == len(served)
     monkeypatch.setattr(model_layers, "decode_layer", lambda *a: None)
     want, _ = _run(model, 2)
