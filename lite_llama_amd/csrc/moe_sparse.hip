@@ -475,12 +475,13 @@ __global__ __launch_bounds__(64 * NW) void router_kernel(const void* __restrict_
 // launch and a few trips to memory; us, count and place in two launches -> here: 128 slots 10.4 -> 5.5, 13 056 slots 36 -> 11.8
 // ------------------------------------------------------------------------------------------------------------------------
 constexpr int kSortExperts = 8192;
+constexpr int kSortWaves = 16;   // most waves of a workgroup
 
 // hist: LDS [experts], counts of the experts in front of this workgroup's
 __device__ __forceinline__ void sort_expert(const int32_t* ids, int num_slots, int experts, int block_m, int skipped, int* hist,
                                             int32_t* __restrict__ counts, int32_t* __restrict__ sorted, int32_t* __restrict__ block_expert,
                                             int32_t* __restrict__ num_post) {
-  __shared__ int part[16], start[16];
+  __shared__ int part[kSortWaves], start[kSortWaves];
   const int e = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, threads = blockDim.x, waves = threads >> 6;
   for (int i = tid; i < e; i += threads) hist[i] = 0;
   __syncthreads();
@@ -1125,7 +1126,7 @@ extern "C" int ll_group_router_sorted(const void* h, int64_t h_ld, const void* w
   // 4 13.3 -> 9.8, 8 13.6 -> 10.4, 16 13.2 -> 12.3, 24 13.1 -> 13.2 (every workgroup chooses for every token); 68 rows of 3072, top 8: 1 15.9 -> 11.1,
   // 4 16.5 -> 11.6, 8 16.5 -> 12.3, 16 16.5 -> 15.1, 24 16.3 -> 16.7
   if (n < 1 || n > kRouteTokens || rows > kRouterRows || sorted_experts < 1 || sorted_experts > experts || (block != 32 && block != 128) ||
-      lds > 65536) {
+      lds + 2 * sizeof(int) * kSortWaves > 65536) {   // (a launch has 64 KB unasked, with what the sort holds of its own)
     const int rc = ll_group_router(h, h_ld, w_router, w_extra, n, width, experts, top, group_count, group_keep, route_scale, scoring, ids, weights,
                                    extra_scale, logits, correction, identity, dtype, stream);
     return rc ? rc : moe_sort(ids, n * top, sorted_experts, block, skipped ? 1 : 0, counts, sorted, block_expert, num_post, stream);

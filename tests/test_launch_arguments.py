@@ -259,6 +259,14 @@ def test_every_router_that_is_accepted_fits_the_lds_of_a_launch(tmp_path):
             for tokens in (1, 300):
                 assert lib.ll_group_router(4096, 64, 4096, None, tokens, 64, experts, top, groups, groups, 1.0, scoring, *[4096] * 4, None, 0, 1, None) == 0
                 assert 0 < lib.router_lds() <= 64 * 1024, (scoring, experts, groups, tokens)
+    # ... and where the choices are sorted in the same launch, which holds 128 bytes of its own beside what it is given
+    lib.ll_group_router_sorted.argtypes = [P, L, P, P, L, L, L, L, L, L, F, I, P, P, P, P, P, L, L, L, I, P, P, P, P, I, P]
+    for scoring in range(5):
+        for experts in (34, 128, 129, *range(466, 514)):
+            for tokens, top in ((1, 8), (16, 8), (12, 12), (16, 64), (1, 64)):
+                assert lib.ll_group_router_sorted(4096, 64, 4096, None, tokens, 64, experts, min(top, experts), 1, 1, 1.0, scoring, *[4096] * 4, None, 0,
+                                                  experts, 128, 0, *[4096] * 4, 1, None) == 0
+                assert 0 < lib.router_lds() <= 64 * 1024 - 128, (scoring, experts, tokens, top)
 
 
 # (tokens, heads, key heads, key width, value width, kind): the longest steps, a little below 2^28 floats of pairs, decays and steps
