@@ -1132,6 +1132,7 @@ extern "C" int ll_group_router_sorted(const void* h, int64_t h_ld, const void* w
     return rc ? rc : moe_sort(ids, n * top, sorted_experts, block, skipped ? 1 : 0, counts, sorted, block_expert, num_post, stream);
   }
   if (!counts || !sorted || !block_expert || !num_post) return LL_ERR_ARG;
+  if (scoring != 2 && !w_extra) c.p.extra_scale = nullptr;   // (no row of weights makes it: left as it is, as ll_group_router leaves it)
   hipStream_t st = (hipStream_t)stream;
   const dim3 grid((unsigned)((rows + 1) / 2), (unsigned)n);
 #define LL_RL(DT, V) route_logits_kernel<DT, V><<<grid, 64, 0, st>>>(h, h_ld, w_router, w_extra, (int)width, (int)experts, rows, logits)

@@ -98,3 +98,26 @@ def test_choices_sorted_for_the_products_are_those_of_two_calls(n, width, expert
     used = int(post)
     assert got[3][0] == block and int(got[3][3]) == used
     assert torch.equal(got[3][1][:used], srt[:used]) and torch.equal(got[3][2][:used // block], owner[:used // block])
+
+
+@pytest.mark.parametrize("scoring", range(5))
+def test_an_extra_scale_that_nothing_makes_is_left(scoring):
+    """The C entry with ``extra_scale`` and no row of weights for it: as the entry without the sort leaves it (softmax_all writes the identity
+    experts' sum, none here)."""
+    from lite_llama_amd import _lib as L
+
+    n, width, experts, top, block = 5, 64, 12, 3, 128
+    h, w = (torch.randn(r, width, device=DEV).to(torch.bfloat16) for r in (n, experts))
+    i32, f32 = (lambda *s: torch.zeros(*s, dtype=torch.int32, device=DEV)), (lambda *s: torch.zeros(*s, device=DEV))
+    runs = n * top + experts * (block - 1)
+    out = []
+    for name in ("ll_group_router", "ll_group_router_sorted"):
+        ids, weights, extra, logits = i32(n, top), f32(n, top), f32(n) + 7.0, f32(n, experts)
+        args = (h.data_ptr(), width, w.data_ptr(), 0, n, width, experts, top, 1, 1, 1.0, scoring, ids.data_ptr(), weights.data_ptr(), extra.data_ptr(),
+                logits.data_ptr(), 0, 0)
+        lists = [i32(experts), i32(runs), i32(-(-runs // block)), i32(1)]
+        sort = (experts, block, 0, *(t.data_ptr() for t in lists)) if name.endswith("sorted") else ()
+        L.check(getattr(L.lib(), name)(*args, *sort, L.LL_BF16, L.stream_ptr()), name)
+        out.append((ids, weights, extra))
+    assert all(torch.equal(a, b) for a, b in zip(*out))
+    assert (out[1][2] == (0.0 if scoring == 2 else 7.0)).all()
