@@ -57,7 +57,7 @@ def _count(monkeypatch):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("name,batch", [("mix", 1), ("mix", 33), ("mix", 64), ("large", 1), ("large", 17), ("large", 32), ("large", 50)])
+@pytest.mark.parametrize("name,batch", [("mix", 1), ("mix", 12), ("mix", 33), ("mix", 64), ("large", 1), ("large", 16), ("large", 17), ("large", 32), ("large", 50)])
 def test_the_same_bits_as_single_launches(monkeypatch, name, batch, dtype):
     from lite_llama_amd import model_layers
 
