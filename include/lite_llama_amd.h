@@ -369,6 +369,10 @@ int ll_dense16_matmul(void* out, const void* x, const void* w, const void* bias,
  * epilogue 0: out [m][n] (+ bias); 1: the rows of w are (gate_j, up_j) pairs -> out [m][n / 2] = silu(gate) * up (swiglu_forward's
  * arithmetic on the rounded outputs).  m <= 64, n % 16 == 0, n >= 32, k % 128 == 0, element strides % 8 == 0. */
 int ll_dense16_rows_supported(int64_t m, int64_t n, int64_t k, int epilogue); /* 1 / 0 */
+/* Which routes measured faster than the library's product for m rows over unquantised weights [n][k], where the narrow one (below) does not
+ * win: bits LL_ROUTE_*, in the order in which they are to be tried; 0: the library. */
+enum { LL_ROUTE_ROWS = 1, LL_ROUTE_ROWS_NARROWER = 2, LL_ROUTE_SPLIT = 4 };
+int ll_dense16_route(int64_t m, int64_t n, int64_t k);
 int ll_dense16_rows_matmul(void* out, const void* x, const void* w, const void* bias, int64_t m, int64_t n, int64_t k,
                            int64_t x_stride_m, int64_t w_stride_n, int dtype, int epilogue, void* stream);
 /* F.linear of m <= 64 rows over a narrow unquantised weight: out [m][n] = x [m][k] @ w [n][k]^T (+ bias), finished outputs in one launch whatever n.

@@ -74,6 +74,7 @@ SIGNATURES = {
     "ll_w8a8_rows_supported": [L, L, L, I],
     "ll_w8a8_rows_matmul": [P, P, P, P, P, P, L, L, L, L, L, I, P],
     "ll_dense16_rows_supported": [L, L, L, I],
+    "ll_dense16_route": [L, L, L],
     "ll_dense16_rows_matmul": [P, P, P, P, L, L, L, L, L, I, I, P],
     "ll_dense_partials_count": [L, L, L, I, I],
     "ll_dense_partials": [P, P, P, P, L, L, L, I, L, I, L, L, L, L, I, P],

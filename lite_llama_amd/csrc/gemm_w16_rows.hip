@@ -334,6 +334,27 @@ extern "C" int ll_dense16_rows_supported(int64_t m, int64_t n, int64_t k, int ep
   return r16_lds_fits(m) ? 1 : 0;
 }
 
+// The routes of a projection of a few rows (quantization/methods.py, layered_decode.hip), us per launch, hipGraph replays over rotating weights, bf16:
+// ROWS, wide outputs on the row-group loop, rows / library / split-K engine: fused gate|up 17920 x 1536 at 32 rows incl. the swiglu 13.4 / 25.2 / 30.9;
+//   lm_head 151936 x 1536 at 32 rows 80.6 / 106.4 / 96.9 (5.8 TB/s); 152064 x 3584 at 64 rows 204.8 / 210.9 / 226.8; gate|up 37888 x 3584 fp16 at 64 rows
+//   55.7 / 76.0 / 85.3.  It needs about one 32-row group per CU to fill the chip: down 1536 x 8960 35.8 / 21.8 / 20.7.
+// ROWS_NARROWER, outputs that end inside a 32-row group, or of too few groups for a CU each, on contractions short enough, rows / library: 12080 x
+//   3072 6 rows 16.8 / 22.0, 32 rows 16.9 / 19.6, 48 rows 19.4 / 21.7, 64 rows 22.9 / 22.0; 6176 x 2048 32 rows 9.9 / 13.0, 48 rows 12.9 / 13.6;
+//   4096 x 2048 32 rows 9.5 / 12.0, 48 rows 12.5 / 12.3; 5120 x 1024 32 rows 6.7 / 11.7; 7168 x 3072 6 rows 12.9 / 13.3, 32 rows 13.2 / 14.0; 6144 x 3072
+//   16 rows 12.7 / 12.7, 4096 x 3072 32 rows 12.2 / 11.3, 6144 x 4096 32 rows 16.5 / 16.4.
+// SPLIT, long contractions or the widest outputs of up to 32 rows on the split-K engine, engine / library: down 1536 x 8960 20.4 / 21.8, lm_head 151936 x
+//   1536 94.9 / 104.1; elsewhere the library is ahead (7 / 9 on small projections, 211 / 230 on the lm_head of 3584 at 64 rows).
+extern "C" int ll_dense16_route(int64_t m, int64_t n, int64_t k) {
+  if (m < 1 || m > 64) return 0;
+  int route = 0;
+  if (k % 128 == 0) {
+    if (n >= 8192 && n % 32 == 0) route |= LL_ROUTE_ROWS;
+    else if (m <= 48 && n % 16 == 0 && (n >= 8192 || (k <= 3072 && n >= 7168) || (k <= 2048 && n >= (m <= 32 ? 4096 : 5120)))) route |= LL_ROUTE_ROWS_NARROWER;
+  }
+  if (m <= 32 && (k >= 4096 || n >= 32768)) route |= LL_ROUTE_SPLIT;
+  return route;
+}
+
 // out [m][n] (epilogue 0, + bias) or [m][n / 2] (epilogue 1: rows of w interleaved (gate_j, up_j)) = x [m][k] @ w [n][k]^T for an
 // unquantised fp16 / bf16 weight; m <= 64, n % 16 == 0, k % 128 == 0, rows 16-byte aligned.  Returns LL_OK, or an error code.
 extern "C" int ll_dense16_rows_matmul(void* out, const void* x, const void* w, const void* bias, int64_t m, int64_t n, int64_t k,

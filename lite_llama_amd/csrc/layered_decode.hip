@@ -72,10 +72,9 @@ Route linear_route(const DecodeLinear& l, int64_t m, int64_t x_ld) {
   if (x_ld % 8 || k % 8 || !ll_aligned16(l.w) || (reinterpret_cast<uintptr_t>(l.bias) & 7u)) return NOT_SERVED;
   if (ll_dense16_narrow_wins(m, n, k)) return getenv("LL_DENSE16_NARROW_OFF") ? NOT_SERVED : NARROW;
   if (x_ld != k) return NOT_SERVED;
-  const bool wide = m <= 64 && n >= 8192 && n % 32 == 0 && k % 128 == 0;
-  const bool narrower = m <= 48 && n % 16 == 0 && k % 128 == 0 && (n >= 8192 || (k <= 3072 && n >= 7168) || (k <= 2048 && n >= (m <= 32 ? 4096 : 5120)));
-  if (wide || narrower) return getenv("LL_DENSE16_ROWS_OFF") || !ll_dense16_rows_supported(m, n, k, 0) ? NOT_SERVED : ROWS;
-  if (m <= 32 && (k >= 4096 || n >= 32768) && k % 64 == 0 && n % 4 == 0 && ll_dense16_partial_words(m, n, k) > 0 && !getenv("LL_DENSE16_OFF")) return SPLIT;
+  const int route = ll_dense16_route(m, n, k);
+  if (route & (LL_ROUTE_ROWS | LL_ROUTE_ROWS_NARROWER)) return getenv("LL_DENSE16_ROWS_OFF") || !ll_dense16_rows_supported(m, n, k, 0) ? NOT_SERVED : ROWS;
+  if ((route & LL_ROUTE_SPLIT) && k % 64 == 0 && n % 4 == 0 && ll_dense16_partial_words(m, n, k) > 0 && !getenv("LL_DENSE16_OFF")) return SPLIT;
   return NOT_SERVED;
 }
 

@@ -561,33 +561,28 @@ def dense_matmul_partials(x: torch.Tensor, weight: torch.Tensor, scales: torch.T
     return PartialSums(parts, (*x.shape[:-1], n), x.dtype)
 
 
+_ROUTE_ROWS, _ROUTE_ROWS_NARROWER, _ROUTE_SPLIT = 1, 2, 4
+
+
+def dense16_route(m: int, n: int, k: int) -> int:
+    """Which of the own kernels measured faster than the library for ``m`` rows over an unquantised ``[n, k]`` weight on the GPU
+    (``ll_dense16_route``: bits, the figures beside it); 0 where the library stays, as it does in a part library without them."""
+    return L.lib().ll_dense16_route(m, n, k) if L.has("ll_dense16_route") else 0
+
+
 def dense16_wins(m: int, n: int, k: int) -> bool:
-    """Where the hand-written kernel measured FASTER than the library GEMM on MI355X (benchmarks/dense16_shapes.py, round 3,
-    same box, hipGraph replays over rotating weights): batches of <= 32 rows with a long contraction (Qwen2.5-1.5B down
-    8960 -> 1536: 20.4 vs 21.8 us) or a very wide output written straight from the single split (lm_head 151936 x 1536: 94.9
-    vs 104.1 us).  Elsewhere hipBLASLt is ahead (7 vs 9 us on the small projections, 211 vs 230 us on the 7B lm_head at
-    batch 64) and stays -- a plain library GEMM, the reference's own choice for these layers."""
-    return m <= 32 and (k >= 4096 or n >= 32768)
+    """Long contractions and the widest outputs of up to 32 rows: the split-K engine."""
+    return bool(dense16_route(m, n, k) & _ROUTE_SPLIT)
 
 
 def dense16_rows_wins(m: int, n: int, k: int) -> bool:
-    """Where the 16-bit row-group kernel measured faster than the library GEMM and than the split-K 16-bit engine on MI355X
-    (benchmarks/dense16_rows.py, round 5, hipGraph replays over rotating weights, us per launch rows / library / split-K):
-    fused gate|up 17920 x 1536 at batch 32 incl. the swiglu 13.4 / 25.2 / 30.9; lm_head 151936 x 1536 at batch 32 80.6 / 106.4 /
-    96.9 (5.8 TB/s); lm_head 152064 x 3584 at batch 64 204.8 / 210.9 / 226.8; gate|up 37888 x 3584 fp16 at batch 64 55.7 / 76.0 /
-    85.3.  It needs about one 32-row group per CU to fill the chip: narrow outputs (down 1536 x 8960: 35.8 / 21.8 / 20.7) keep the
-    split-K engine or the library."""
-    return 1 <= m <= 64 and n >= 8192 and n % 32 == 0 and k % 128 == 0
+    """Wide outputs: the row-group loop."""
+    return bool(dense16_route(m, n, k) & _ROUTE_ROWS)
 
 
 def dense16_rows_narrower_wins(m: int, n: int, k: int) -> bool:
-    """... and of rows that end inside a 32-row group, or too few for a group per CU, on contractions short enough (us per launch rows /
-    library, bf16, hipGraph replays over rotating weights): 12080 x 3072 6 rows 16.8 / 22.0, 32 rows 16.9 / 19.6, 48 rows 19.4 / 21.7, 64 rows
-    22.9 / 22.0; 6176 x 2048 32 rows 9.9 / 13.0, 48 rows 12.9 / 13.6; 4096 x 2048 32 rows 9.5 / 12.0, 48 rows 12.5 / 12.3; 5120 x 1024 32 rows
-    6.7 / 11.7; 7168 x 3072 6 rows 12.9 / 13.3, 32 rows 13.2 / 14.0; 6144 x 3072 16 rows 12.7 / 12.7, 4096 x 3072 32 rows 12.2 / 11.3,
-    6144 x 4096 32 rows 16.5 / 16.4."""
-    wide = n >= 8192 or (k <= 3072 and n >= 7168) or (k <= 2048 and n >= (4096 if m <= 32 else 5120))
-    return 1 <= m <= 48 and wide and n % 16 == 0 and k % 128 == 0
+    """... and outputs that end inside a 32-row group, or have too few groups for a CU each, on short contractions."""
+    return bool(dense16_route(m, n, k) & _ROUTE_ROWS_NARROWER)
 
 
 def _on_one_device(x: torch.Tensor, weight: torch.Tensor, bias) -> bool:
@@ -670,9 +665,9 @@ def dense16_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | N
     ``UnquantizedLinearMethod.apply`` / lm_head are torch's library GEMM.  Returns ``None`` when the call is not served
     (other shapes, dtypes, CPU tensors, ``LL_DENSE16_OFF``) or -- ``policy="auto"`` -- where the library measured faster
     (:func:`dense16_wins`): the caller keeps ``F.linear``."""
-    if policy == "auto" and x.shape[-1] and not dense16_wins(x.numel() // x.shape[-1], weight.shape[0], weight.shape[1]):
+    if not x.is_cuda or (policy == "auto" and x.shape[-1] and not dense16_wins(x.numel() // x.shape[-1], weight.shape[0], weight.shape[1])):
         return None
-    if (not x.is_cuda or x.dtype not in (torch.float16, torch.bfloat16) or weight.dtype != x.dtype or weight.dim() != 2
+    if (x.dtype not in (torch.float16, torch.bfloat16) or weight.dtype != x.dtype or weight.dim() != 2
             or os.environ.get("LL_DENSE16_OFF") or not L.has("ll_dense16_matmul")):
         return None
     n, k = weight.shape

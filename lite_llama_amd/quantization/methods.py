@@ -17,7 +17,7 @@ import torch.nn.functional as F
 from ..kernels import fused_moe, smoothquant_matmul, w4a16_matmul, w8a16_matmul
 from ..kernels.quantization import (smoothquant_gate_up_swiglu, smoothquant_matmul_partials, smoothquant_prefill_swiglu,
                                      smoothquant_rows_matmul)
-from ..kernels.quantization import (_is_followed as is_followed, dense16_linear, dense16_narrow_linear, dense16_rows_linear, dense16_rows_narrower_wins, dense16_rows_wins, dense_matmul_partials, pack_w4a16_scales, pack_w4a16_weights, unpack_w4a16_weights, w4a16_matmul_partials,
+from ..kernels.quantization import (_ROUTE_ROWS, _ROUTE_ROWS_NARROWER, _ROUTE_SPLIT, _is_followed as is_followed, dense16_linear, dense16_narrow_linear, dense16_route, dense16_rows_linear, dense_matmul_partials, pack_w4a16_scales, pack_w4a16_weights, unpack_w4a16_weights, w4a16_matmul_partials,
                                     w4a16_matmul_prepacked_rows, w4a16_mtiled_supported,
                                     w4a16_matmul_prepacked, w4a16_prepacked_supported)
 from .config import FP8, INT4, INT8, SMOOTHQUANT, QuantConfig
@@ -56,6 +56,11 @@ class MoeQuantMethod(ABC):
         raise NotImplementedError(f"{type(self).__name__} cannot be computed from fp16 weights at load time")
 
 
+def _few_rows_route(m: int, x, weight) -> int:
+    """``dense16_route`` of the calls that its kernels serve at all; 0 elsewhere."""
+    return dense16_route(m, *weight.shape) if m <= 64 and x.is_cuda and x.dtype in (torch.float16, torch.bfloat16) else 0
+
+
 class UnquantizedLinearMethod(LinearQuantMethod):
     """fp16 weight through the library GEMM (hipBLASLt via ``F.linear``), unquantized.py:21-22."""
 
@@ -68,16 +73,17 @@ class UnquantizedLinearMethod(LinearQuantMethod):
             out = dense16_narrow_linear(x, layer.weight, layer.bias)  # a few rows over a narrow output: one launch, whole sums
             if out is not None:
                 return out
-        if dense16_rows_wins(m, layer.weight.shape[0], layer.weight.shape[1]):  # wide outputs: the row-group loop (round 5)
+        route = _few_rows_route(m, x, layer.weight)
+        if route & _ROUTE_ROWS:  # wide outputs: the row-group loop (round 5)
             out = dense16_rows_linear(x, layer.weight, layer.bias)
             if out is not None:
                 return out
-        elif dense16_rows_narrower_wins(m, layer.weight.shape[0], layer.weight.shape[1]) and not is_followed(x, layer.weight, layer.bias):
+        elif route & _ROUTE_ROWS_NARROWER and not is_followed(x, layer.weight, layer.bias):
             if layer.bias is None or (layer.bias.is_contiguous() and layer.bias.data_ptr() % 8 == 0):
                 out = dense16_rows_linear(x, layer.weight, layer.bias)
                 if out is not None:
                     return out
-        out = dense16_linear(x, layer.weight, layer.bias, policy="auto")  # decode shapes where the own kernel measured faster
+        out = dense16_linear(x, layer.weight, layer.bias) if route & _ROUTE_SPLIT else None  # decode shapes where the own kernel measured faster
         return out if out is not None else F.linear(x, layer.weight, layer.bias)
 
     def apply_gate_up_swiglu(self, layer, x):
@@ -85,7 +91,7 @@ class UnquantizedLinearMethod(LinearQuantMethod):
         of the 16-bit row-group kernel for decode shapes; ``None`` -> the caller runs the merged GEMM + ``swiglu_forward`` (which
         reads the interleaved pairs in place)."""
         m = x.numel() // x.shape[-1] if x.shape[-1] else 0
-        if layer.bias is not None or not dense16_rows_wins(m, layer.weight.shape[0], layer.weight.shape[1]):
+        if layer.bias is not None or not _few_rows_route(m, x, layer.weight) & _ROUTE_ROWS:
             return None
         return dense16_rows_linear(x, layer.weight, gate_up_swiglu=True)
 
