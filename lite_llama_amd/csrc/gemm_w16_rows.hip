@@ -338,10 +338,15 @@ extern "C" int ll_dense16_rows_supported(int64_t m, int64_t n, int64_t k, int ep
 // ROWS, wide outputs on the row-group loop, rows / library / split-K engine: fused gate|up 17920 x 1536 at 32 rows incl. the swiglu 13.4 / 25.2 / 30.9;
 //   lm_head 151936 x 1536 at 32 rows 80.6 / 106.4 / 96.9 (5.8 TB/s); 152064 x 3584 at 64 rows 204.8 / 210.9 / 226.8; gate|up 37888 x 3584 fp16 at 64 rows
 //   55.7 / 76.0 / 85.3.  It needs about one 32-row group per CU to fill the chip: down 1536 x 8960 35.8 / 21.8 / 20.7.
-// ROWS_NARROWER, outputs that end inside a 32-row group, or of too few groups for a CU each, on contractions short enough, rows / library: 12080 x
-//   3072 6 rows 16.8 / 22.0, 32 rows 16.9 / 19.6, 48 rows 19.4 / 21.7, 64 rows 22.9 / 22.0; 6176 x 2048 32 rows 9.9 / 13.0, 48 rows 12.9 / 13.6;
-//   4096 x 2048 32 rows 9.5 / 12.0, 48 rows 12.5 / 12.3; 5120 x 1024 32 rows 6.7 / 11.7; 7168 x 3072 6 rows 12.9 / 13.3, 32 rows 13.2 / 14.0; 6144 x 3072
-//   16 rows 12.7 / 12.7, 4096 x 3072 32 rows 12.2 / 11.3, 6144 x 4096 32 rows 16.5 / 16.4.
+// ROWS_NARROWER, outputs that end inside a 32-row group, or of too few groups for a CU each.  Rows / library, 1, 8, 32 and 48 rows: 8208 x 1024 5.7 / 8.7,
+//   5.8 / 8.8, 6.2 / 11.9, 7.4 / 12.6; 12080 x 3072 15.5 / 21.8, 15.6 / 20.4, 16.1 / 17.9, 17.9 / 19.7; 32752 x 3072 33.8 / 42.7 .. 35.3 / 52.9.  Rows / split-K
+//   engine, 1 and 32 rows: 8208 x 4096 15.2 / 18.8, 15.7 / 22.1; 12080 x 14336 58.6 / 72.7, 67.6 / 81.3; 32784 x 8192 88 / 124, 97 / 131; the least at 8192
+//   columns, whose rows lie 16 KB apart: 8208 35.6 / 35.0, 37.3 / 39.3 -- and there, above 32 rows, the library is ahead (48 rows of 12080 47.0 / 43.7,
+//   5120 columns 29.5 / 30.4, 14336 77 / 86) up to 16 400 outputs (49 / 69).  Of too few groups, short contractions, rows / library: 7168 x 3072 1 row
+//   12.3 / 13.1, 32 13.3 / 14.3, 48 16.9 / 19.1; 6176 x 2048 24 rows 8.7 / 12.6, 48 11.3 / 13.0; 4096 x 2048 32 rows 8.4 / 11.6; 4096 x 128 32 rows 3.3 / 4.1;
+//   5120 x 1024 32 rows 5.7 / 11.5; on the other side 6144 x 3072 16 rows 12.7 / 12.7, 4096 x 3072 32 rows 12.2 / 11.3, 6144 x 4096 32 rows 16.5 / 16.4.
+//   Sums run in the order of columns, as the library's do in most of these shapes above 16 rows; where it or the split-K engine cuts the contraction, 1 - 8 of 10 000
+//   results round the other way, and both are equally far from 64 bits (1.66e-3 of their size in bf16).
 // SPLIT, long contractions or the widest outputs of up to 32 rows on the split-K engine, engine / library: down 1536 x 8960 20.4 / 21.8, lm_head 151936 x
 //   1536 94.9 / 104.1; elsewhere the library is ahead (7 / 9 on small projections, 211 / 230 on the lm_head of 3584 at 64 rows).
 extern "C" int ll_dense16_route(int64_t m, int64_t n, int64_t k) {
@@ -349,7 +354,9 @@ extern "C" int ll_dense16_route(int64_t m, int64_t n, int64_t k) {
   int route = 0;
   if (k % 128 == 0) {
     if (n >= 8192 && n % 32 == 0) route |= LL_ROUTE_ROWS;
-    else if (m <= 48 && n % 16 == 0 && (n >= 8192 || (k <= 3072 && n >= 7168) || (k <= 2048 && n >= (m <= 32 ? 4096 : 5120)))) route |= LL_ROUTE_ROWS_NARROWER;
+    else if (m <= 48 && n % 16 == 0 && ((n >= 8192 && !(m > 32 && k % 8192 == 0 && n < 16384)) || (k <= 3072 && n >= 7168) ||
+                                        (k <= 2048 && n >= (m <= 32 ? 4096 : 5120))))
+      route |= LL_ROUTE_ROWS_NARROWER;
   }
   if (m <= 32 && (k >= 4096 || n >= 32768)) route |= LL_ROUTE_SPLIT;
   return route;

@@ -17,7 +17,10 @@ ROWS, NARROWER, SPLIT = 1, 2, 4
     (1, 8192, 128, ROWS), (64, 8192, 128, ROWS), (65, 8192, 128, 0), (0, 8192, 128, 0), (1, 8192, 192, 0), (32, 32768, 1536, ROWS | SPLIT),
     (32, 151936, 4096, ROWS | SPLIT), (33, 151936, 4096, ROWS), (32, 1536, 8960, SPLIT), (33, 1536, 8960, 0), (32, 1536, 4032, 0), (32, 33000, 64, SPLIT),
     (32, 4096, 2048, NARROWER), (33, 4096, 2048, 0), (33, 5120, 2048, NARROWER), (48, 5120, 2048, NARROWER), (49, 5120, 2048, 0), (32, 4080, 2048, 0),
-    (32, 4104, 2048, 0), (32, 6144, 2176, 0), (48, 7168, 3072, NARROWER), (48, 7152, 3072, 0), (32, 7168, 3200, 0), (48, 12080, 3072, NARROWER)])
+    (32, 4104, 2048, 0), (32, 6144, 2176, 0), (48, 7168, 3072, NARROWER), (48, 7152, 3072, 0), (32, 7168, 3200, 0), (48, 12080, 3072, NARROWER),
+    # rows of 8192 columns lie 16 KB apart: above 32 rows the library's until there are outputs enough
+    (48, 8208, 8192, 0), (33, 16368, 8192, 0), (32, 8208, 8192, NARROWER | SPLIT), (48, 16400, 8192, NARROWER), (48, 8208, 5120, NARROWER),
+    (48, 8208, 14336, NARROWER), (48, 8224, 8192, ROWS)])
 def test_the_rule(m, n, k, route):
     assert Q.dense16_route(m, n, k) == route
     assert (Q.dense16_rows_wins(m, n, k), Q.dense16_rows_narrower_wins(m, n, k), Q.dense16_wins(m, n, k)) == (
