@@ -87,6 +87,7 @@ struct FdRope {
 #define FD_QS_MAX 8
 
 #define FD_WHOLE 2  // whole partitions of a workgroup where several share up to FD_GROUP_MAX
+#define FD_ALONE 3  // ... and of one that has its row to itself there: rows of no more partitions are not spread (fd_plan)
 // grid = (nparts, hkv * head_groups, batch), block = 64 (one wave)
 // FUSE: the wave that finishes the LAST non-empty partition of its (row, KV head group) also does the
 // log-sum-exp merge and writes ``out`` (no second launch: a kernel boundary costs ~4.7 us in the
@@ -226,7 +227,7 @@ __device__ __forceinline__ void fd_head_norm(Q4 (&qf)[4], const Q4 (&wf)[4], flo
 }
 
 // WHOLE: up to FD_GROUP_MAX partitions in several workgroups; FD_WHOLE waves of each keep a whole partition, the others only help to add up and to
-// merge (a form of its own: asked at run time it cost every launch 0.9 us, through spilled scalars)
+// merge; a row of up to FD_ALONE partitions has one workgroup, and as many waves (a form of its own: asked at run time it cost every launch 0.9 us, through spilled scalars)
 template <int DT, int D, bool FUSE, bool ROPE, int GS, bool GROUPED, bool KV8 = false, bool QKN = false, bool QI32 = false, bool WHOLE = false>
 __global__ __launch_bounds__(GROUPED ? 64 * FD_GROUP_MAX : 64, GROUPED && D == 64 ? 4 : 1) void fd_stage1(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
@@ -255,9 +256,12 @@ __global__ __launch_bounds__(GROUPED ? 64 * FD_GROUP_MAX : 64, GROUPED && D == 6
   // GROUPED: gridDim.x workgroups share a row's partitions (1 unless the launch would leave most of the chip idle, fd_plan): wave
   // ``part`` of all of them walks partitions part, part + walkers, ...
   static_assert(!WHOLE || GROUPED, "several workgroups of waves");
-  const int held = WHOLE ? FD_WHOLE : GROUPED ? (int)(blockDim.x >> 6) : 1;   // waves with a share
+  int held = WHOLE ? FD_WHOLE : GROUPED ? (int)(blockDim.x >> 6) : 1;   // waves with a share
   const int walkers = GROUPED ? (int)gridDim.x * held : 1;
-  const int part = GROUPED ? (int)blockIdx.x * held + wave : (int)blockIdx.x;
+  // (WHOLE: which workgroup of a pair comes first differs from pair to pair.  Those of rows that are not spread work alone, and four to a pair, dealt out
+  // over eight XCDs, would stand on two of them.)
+  const int bx = WHOLE ? (int)((blockIdx.x + ((blockIdx.z * gridDim.y + blockIdx.y) >> 1)) % gridDim.x) : (int)blockIdx.x;
+  int part = GROUPED ? bx * held + wave : bx;
   const int kvh = blockIdx.y % hkv;
   const int hg = blockIdx.y / hkv;
   const int b = blockIdx.z;
@@ -358,6 +362,12 @@ __global__ __launch_bounds__(GROUPED ? 64 * FD_GROUP_MAX : 64, GROUPED && D == 6
     if (seq_len > (int64_t)nparts * FD_PART) seq_len = (int64_t)nparts * FD_PART;
     seq_len = __builtin_amdgcn_readfirstlane((int)seq_len);  // (scalar: everything below that derives from it is)
   }
+  if constexpr (WHOLE) {
+    if (seq_len <= FD_ALONE * FD_PART) {  // (the launch knows the longest row's bound alone, and in a captured step a bucket of it)
+      held = FD_ALONE;
+      part = bx * FD_ALONE + wave;
+    }
+  }
   // Tokens of a share.  Where several workgroups share a row every wave takes one run of tokens of the same length, in tiles of 32 (27 rows
   // of 1500 - 3000 tokens on 4 x 8 waves: 96 each; 718 us a step against 741 with whole partitions of 128); one workgroup keeps whole partitions,
   // where smaller ones lost (batch 1 x ctx 300: 697 -> 712 us, batch 64 x ctx 700: 972 -> 981).
@@ -367,8 +377,8 @@ __global__ __launch_bounds__(GROUPED ? 64 * FD_GROUP_MAX : 64, GROUPED && D == 6
   }
   int64_t start = (int64_t)part * ptok;  // (GROUPED: the wave's FIRST partition; it walks part, part + walkers, ... below)
   if constexpr (GROUPED) {
-    if (blockIdx.x > 0 && start - (int64_t)wave * ptok >= seq_len) return;  // a split past the row's end: no wave has work, none merges
-    if (WHOLE && wave >= FD_WHOLE) start = seq_len;
+    if (bx > 0 && start - (int64_t)wave * ptok >= seq_len) return;  // a split past the row's end: no wave has work, none merges
+    if (WHOLE && wave >= held) start = seq_len;
   }
   if (start >= seq_len) {  // empty partition stores nothing (flashdecoding.py:141-161)
     publish_q();
@@ -899,7 +909,7 @@ __global__ __launch_bounds__(GROUPED ? 64 * FD_GROUP_MAX : 64, GROUPED && D == 6
     const int W = held;
     const bool shared = gridDim.x > 1;  // (one workgroup keeps whole partitions: no division by ptok)
     const int np = seq_len <= 0 ? 0 : shared ? ((int)seq_len + ptok - 1) / ptok : (int)(seq_len + FD_PART - 1) / FD_PART;
-    const int first = (int)blockIdx.x * W;
+    const int first = bx * W;
     const int nrec = np - first < W ? np - first : W;                 // waves of this workgroup with tokens
     int splits = 1;                                                   // workgroups of this row with tokens
     if (shared) splits = (np + W - 1) / W < (int)gridDim.x ? (np + W - 1) / W : (int)gridDim.x;
@@ -908,13 +918,13 @@ __global__ __launch_bounds__(GROUPED ? 64 * FD_GROUP_MAX : 64, GROUPED && D == 6
     uint16_t* out_g = out + b * o_sb + (int64_t)head0 * o_sh;
     const float* recs = reinterpret_cast<const float*>(lds_all);
     if (np == 0) return;                                              // (a zero-length row: its 0/0 is written above)
-    const int64_t hr0 = ((int64_t)b * hq + head0) * nparts + blockIdx.x;  // this split's record of the group's first head
+    const int64_t hr0 = ((int64_t)b * hq + head0) * nparts + bx;  // this split's record of the group's first head
     for (int sidx = (int)threadIdx.x; sidx < nvalid * D4; sidx += (int)blockDim.x) {
       const int hl_s = sidx / D4, d4 = sidx % D4;
       if (WHOLE && splits > 1) {   // the waves' records as they are
         for (int pp = 0; pp < nrec; ++pp) {
           const float* rec = recs + pp * REC;
-          const int64_t at = hr0 + (int64_t)hl_s * nparts - (int)blockIdx.x + first + pp;
+          const int64_t at = hr0 + (int64_t)hl_s * nparts - bx + first + pp;
           unsigned long long* mo = reinterpret_cast<unsigned long long*>(mid_o + at * D + d4 * 4);
 #pragma unroll
           for (int e = 0; e < 4; e += 2)
@@ -1062,10 +1072,14 @@ extern "C" int ll_flash_decoding_num_partitions(int64_t max_len) {
 // last arriver alone would merge very many partitions (2 pairs, 32 768 tokens 160 / 75; 16 pairs, 16 384 140 / 118).
 // Five to eight partitions, heads of 128, few pairs: a wave per partition as before, but two to a workgroup, as long as every workgroup finds a CU of its
 // own -- a CU takes in some 27 KB a microsecond whatever its waves, and a row of 1000 tokens is 512 KB.  Every wave's record goes to the workgroup
-// that arrives last, which merges them in order: the bits of one workgroup.  us, one workgroup / here, longest row 520 | 600 | 700 | 1000 tokens: 4
-// pairs of 7 heads 11.8 / 11.9 | 13.0 / 12.0 | 15.4 / 12.7 | 19.3 / 13.3; 64 of 7 12.3 / 13.2 | 13.5 / 13.1 | 15.8 / 13.8 | 19.7 / 14.8; 64 of 4 12.2 /
-// 11.7 | 14.1 / 11.8 | 15.9 / 12.1 | 19.7 / 12.6.  Even shares of four waves each, in whose order sums round otherwise: 19.2 / 10.6 at 1000.  Not up to
-// four partitions (300 tokens 9.0 / 10.2), not for heads of 64 (500 tokens 7.4 / 8.4).
+// that arrives last, which merges them in order: the bits of one workgroup.  It has as many waves as the result has float4 (heads D / 4), so that
+// the merge is one round: with those that the planes need alone (three for seven heads) it took two, 1.7 us more.  Rows of up to FD_ALONE partitions are
+// not spread, whatever the launch (a captured step knows its bucket alone): the merge costs them more than it gives.  us, one workgroup / here, a step's
+// longest row 300 | 400 | 513 | 600 | 700 | 1000 tokens, bounds of 640 and 1024: 4 pairs of 7 heads 8.8 / 9.0 | 10.0 / 9.9 | 11.5 / 10.1 | 12.9 / 10.1 |
+// 14.9 / 10.2 | 18.7 / 10.5; 64 of 7 9.1 / 9.1 | 10.2 / 10.1 | 11.9 / 11.2 | 13.8 / 11.3 | 15.1 / 11.4 | 19.0 / 12.4; 64 of 4 9.3 / 9.5 | 10.2 / 10.3 | 11.9 /
+// 11.0 | 13.9 / 11.1 | 15.5 / 11.4 | 18.7 / 12.2; planes, 64 of 7 11.0 / 11.3 | 12.8 / 12.9 | 13.9 / 13.4 | 15.6 / 13.4 | 16.3 / 13.3 | 21.9 / 14.4.  Spread from three
+// partitions on 300 tokens take 10.6 (4 of 7) and 12.2 us (64 of 7), alone up to four 512 take 11.3 / 11.9 / 11.9 instead of 10.0 / 11.2 / 10.9.  Even shares
+// of four waves each, in whose order sums round otherwise: 19.2 / 10.6 at 1000.  Not for heads of 64 (500 tokens 7.4 / 8.4).
 #define FD_LOOP_MAX 256  // partitions (32 768 tokens)
 struct FdPlan {
   int waves, splits;
@@ -1075,8 +1089,8 @@ static FdPlan fd_plan(int64_t max_len, int64_t pairs, int heads, int d, bool pla
   const int64_t np = (max_len + FD_PART - 1) / FD_PART;
   if (np < 2 || np > FD_LOOP_MAX || pairs < 1) return {0, 0};
   if (np <= FD_GROUP_MAX) {
-    const int64_t splits = (np + FD_WHOLE - 1) / FD_WHOLE, waves = ((heads + 2) * d / 4 + 127) / 128;   // (q|k|v as planes: two float4 slots a lane)
-    if (np > 4 && pairs * splits <= 256 && d == 128 && merge) return {(int)(waves < FD_WHOLE ? FD_WHOLE : waves), (int)splits};
+    const int64_t splits = (np + FD_WHOLE - 1) / FD_WHOLE, waves = (heads * d / 4 + 63) / 64;   // (a float4 of the result for every lane, in one round)
+    if (np > 4 && pairs * splits <= 256 && d == 128 && merge) return {(int)(waves < FD_ALONE ? FD_ALONE : waves), (int)splits};
     return {(int)np, 1};
   }
   static const bool no_loop = getenv("LL_FD_NO_LOOP") != nullptr;  // A/B knob, read once

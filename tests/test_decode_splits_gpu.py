@@ -212,3 +212,64 @@ def test_planes_at_middle_contexts(b, longest):
     q, kv = rows[:, :hq * d].view(b, hq, d), rows[:, hq * d:].view(b, 2 * hkv, d)
     want = decode_attention(q.contiguous(), kv.contiguous(), cos, sin, pos, sel, pool_b, 0.1, table, req, seq, longest)
     assert torch.equal(pool_a, pool_b) and torch.equal(got.reshape(-1), want.reshape(-1))
+
+
+# every form of the launch; heads of one and two column tiles, and of an odd last round of the merge; five, six and eight partitions; rows at the edges of a
+# partition, of what is not spread (384) and of one workgroup's share
+@pytest.mark.parametrize("kind,hkv,rep,bound", [("rows", 2, 7, 1024), ("rows", 1, 20, 1024), ("rows", 4, 1, 640), ("rows bf16", 2, 16, 768), ("fp8", 2, 4, 1024),
+                                                ("fused", 2, 6, 1024), ("fused norm", 2, 4, 900), ("planes", 2, 7, 1024), ("planes norm", 4, 16, 640),
+                                                ("planes int32", 2, 4, 1024)])
+def test_the_bits_of_one_workgroup(kind, hkv, rep, bound):
+    """Rows whose pairs leave compute units idle are spread over several workgroups; beside so many others that the launch keeps one workgroup to a pair,
+    they are not: the same bits, in the result and in the written cache rows."""
+    from lite_llama_amd.kernels import flash_decoding
+    from lite_llama_amd.kernels.attention import decode_attention, decode_attention_partials, flash_decoding_fp8kv
+    from lite_llama_amd.kernels.norm_act import PartialSums, ScaledInt32Partials
+
+    d, hq = 128, hkv * rep
+    dt = torch.float16 if kind in ("rows", "fp8", "planes int32") else torch.bfloat16
+    g = torch.Generator(device=DEV).manual_seed(hq + bound)
+    rand = lambda *s: torch.randn(*s, generator=g, device=DEV)  # noqa: E731
+    splits, groups = -(-bound // 256), -(-rep // 16)
+    lens = [n for n in (bound, 1, 128, 129, 383, 384, 385, 512, 513, 640, 641, 700, 768, 897) if n <= bound]
+    few = len(lens)
+    assert few * hkv * groups * splits <= 256
+    lens += [(37 * i) % bound + 1 for i in range(256 // (hkv * groups * splits) + 1)]
+    rows = len(lens)
+    pool = (rand(sum(lens), 2 * hkv, d) * (0.5 if kind == "fp8" else 1.0)).to(torch.float8_e4m3fn if kind == "fp8" else dt)
+    pool = pool.view(torch.uint8) if kind == "fp8" else pool
+    table = torch.zeros(rows, bound, dtype=torch.int32, device=DEV)
+    for i, at in enumerate(torch.randperm(sum(lens), generator=g, device=DEV).to(torch.int32).split(lens)):
+        table[i, :lens[i]] = at
+    seq, req = torch.tensor(lens, dtype=torch.int64, device=DEV), torch.arange(rows, dtype=torch.int64, device=DEV)
+    pos, sel = seq - 1, table[req, seq - 1].contiguous()
+    ang = torch.arange(bound, device=DEV)[:, None] * torch.rand(d // 2, generator=g, device=DEV)[None]
+    cos, sin = (torch.cat([f(ang)] * 2, -1).to(dt) for f in (torch.cos, torch.sin))
+    norm = (1 + rand(d).to(dt) * 0.1, 1 + rand(d).to(dt) * 0.1, 1e-6) if kind.endswith("norm") else None
+    width = (hq + 2 * hkv) * d
+    q, kv, planes = rand(rows, hq, d).to(dt), rand(rows, 2 * hkv, d).to(dt), rand(5, rows, width)
+    counts = torch.randint(-3000, 3000, (5, rows, width), generator=g, device=DEV, dtype=torch.int32)
+    a_scale, w_scale = rand(rows).abs() * 0.01 + 0.001, rand(width).abs() * 0.01 + 0.001
+
+    def call(n):
+        own = pool.clone()
+        k, v, tail = own[:, :hkv], own[:, hkv:], (0.1, table[:n], req[:n], seq[:n], bound)
+        if kind.startswith("rows"):
+            return flash_decoding(q[:n], k, v, *tail), own
+        if kind == "fp8":
+            return flash_decoding_fp8kv(q[:n], k, v, *tail), own
+        at = (cos, sin, pos[:n].contiguous(), sel[:n].contiguous(), own, *tail)
+        if kind.startswith("fused"):
+            return decode_attention(q[:n], kv[:n], *at, qk_norm=norm), own
+        if kind == "planes int32":
+            parts = ScaledInt32Partials(counts[:, :n].contiguous(), (n, width), a_scale[:n].contiguous(), w_scale)
+        else:
+            parts = PartialSums(planes[:, :n].contiguous(), (n, width), dt)
+        return decode_attention_partials(parts, None, hq, hkv, d, *at, qk_norm=norm), own
+
+    (alone, pool_a), (all_rows, pool_b) = call(few), call(rows)
+    assert torch.isfinite(alone.float()).all() and torch.equal(alone, all_rows[:few])
+    written = sel[:few].long()
+    assert torch.equal(pool_a[written], pool_b[written])
+    if not kind.startswith("rows") and kind != "fp8":
+        assert not torch.equal(pool_a[written], pool[written])

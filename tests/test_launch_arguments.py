@@ -63,6 +63,12 @@ void decode_plan(int64_t max_len, int64_t pairs, int heads, int d, int planes, i
   out[0] = p.waves;
   out[1] = p.splits;
 }
+void decode_plan_merged(int64_t max_len, int64_t pairs, int heads, int d, int* out) {
+  const FdPlan p = fd_plan(max_len, pairs, heads, d, true, true);
+  out[0] = p.waves;
+  out[1] = p.splits;
+}
+int decode_alone() { return FD_ALONE * FD_PART; }
 }
 """
 
@@ -163,6 +169,24 @@ def test_decode_plans_of_other_calls(flash_decoding):
     for pairs in (1, 16, 40, 127):                                   # heads of 256 spill in a grouped workgroup
         assert _plan(flash_decoding, 1025, pairs, d=256) == (0, 0)
         assert (_plan(flash_decoding, 32768, pairs, d=256)[0] == 8) == (pairs <= 16)
+
+
+@pytest.mark.parametrize("heads", range(1, 17))
+def test_rows_of_five_to_eight_partitions_in_several_workgroups(flash_decoding, heads):
+    """Every lane of the workgroup that merges has a float4 of the result, in one round; a row that is not spread has a wave for every partition."""
+    out = (ctypes.c_int * 2)()
+    alone = flash_decoding.decode_alone()
+    assert alone == 384
+    for tokens, splits in ((513, 3), (640, 3), (641, 3), (768, 3), (769, 4), (1024, 4)):
+        for pairs in (1, 64, 256 // splits, 256 // splits + 1):
+            flash_decoding.decode_plan_merged(ctypes.c_int64(tokens), ctypes.c_int64(pairs), heads, 128, out)
+            if pairs * splits > 256:
+                assert tuple(out) == (-(-tokens // 128), 1)
+                continue
+            assert out[1] == splits and 64 * out[0] >= heads * 128 // 4 and 128 * out[0] >= alone and out[0] <= 8
+            assert 128 * out[0] >= (heads + 2) * 128 // 4             # (the planes' two pieces per lane)
+    flash_decoding.decode_plan_merged(ctypes.c_int64(1024), ctypes.c_int64(8), heads, 64, out)
+    assert tuple(out) == (8, 1)
 
 
 def test_the_switch_back_to_a_workgroup_per_partition(flash_decoding, tmp_path, monkeypatch):
