@@ -237,9 +237,9 @@ bool readable(const int64_t* args, int64_t count, const double* floats, int64_t 
 
 }  // namespace
 
-// bytes of scratch for such a layer, or 0: not served
+// bytes of scratch for such a layer, or 0: not served (LL_NO_LAYER_CALLS in the environment: none is)
 extern "C" int64_t ll_layered_decode_bytes(const int64_t* args, int64_t count, const double* floats, int64_t float_count) {
-  if (!readable(args, count, floats, float_count)) return 0;
+  if (!readable(args, count, floats, float_count) || getenv("LL_NO_LAYER_CALLS")) return 0;
   Walk w{*reinterpret_cast<const LayeredDecode*>(args), *reinterpret_cast<const LayeredDecodeFloats*>(floats), nullptr, nullptr};
   w.run();
   return w.status == LL_OK ? w.used : 0;

@@ -74,7 +74,7 @@ def test_the_same_bits_as_single_launches(monkeypatch, name, batch, dtype):
     assert len(kept) == len(old) and all(torch.equal(a, b) for a, b in zip(kept, old))
 
 
-@pytest.mark.parametrize("what", ["odd", "one", "fp32", "hook", "grad", "env", "replaced", "eps", "off"])
+@pytest.mark.parametrize("what", ["odd", "one", "fp32", "hook", "grad", "env", "switch", "replaced", "eps", "off"])
 def test_what_goes_through_the_modules(monkeypatch, what):
     from lite_llama_amd import model_layers
 
@@ -86,6 +86,8 @@ def test_what_goes_through_the_modules(monkeypatch, what):
             layer.mixer.in_proj.register_forward_hook(lambda *a: seen.append(1))
     if what == "env":
         monkeypatch.setenv("LL_DENSE16_NARROW_OFF", "1")
+    if what == "switch":
+        monkeypatch.setenv("LL_NO_LAYER_CALLS", "1")
     if what == "eps":
         for layer in model.layers:
             layer.mixer.eps = 0.5          # (its own norms', not the layer's)
