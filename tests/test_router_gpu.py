@@ -73,15 +73,20 @@ def test_the_largest_choices(scoring, experts, top):
 
 
 @pytest.mark.parametrize("n,width,experts,top", [(1, 40, 5, 1), (1, 3072, 68, 8), (4, 2048, 34, 4), (5, 520, 34, 4), (31, 136, 130, 3), (32, 3080, 65, 4),
-                                                 (33, 264, 40, 4), (2, 520, 512, 9), (8, 72, 513, 2), (32, 64, 511, 64),
-                                                 # the waves of the one launch and the largest step that takes it; the end of the choice in registers; the LDS of a launch
-                                                 (9, 520, 34, 4), (16, 3072, 68, 8), (17, 3072, 68, 8), (16, 264, 64, 16), (3, 264, 64, 17), (16, 264, 128, 16),
-                                                 (7, 264, 128, 17), (13, 264, 129, 16), (16, 64, 482, 8), (16, 64, 483, 8), (12, 64, 480, 12), (1, 64, 491, 8)])
+                                                 (33, 264, 40, 4), (2, 520, 512, 9), (8, 72, 513, 2), (32, 64, 511, 64)])
 @pytest.mark.parametrize("scoring", ["sigmoid", "softmax_chosen", "softmax_all", "sigmoid_plain", "softmax_groups"])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
 def test_choices_sorted_for_the_products_are_those_of_two_calls(n, width, experts, top, scoring, dtype):
-    """Bit for bit, on both sides of the largest step whose choices every expert's workgroup makes (16 tokens); slots in their order, every list's tail."""
+    """Bit for bit; slots in their order, every list's tail.  Up to 16 tokens every expert's workgroup makes the choices, beyond them a launch of its own."""
     _the_same_as_two_calls(n, width, experts, top, scoring, dtype)
+
+
+# the waves of the one launch and the largest step that takes it; the end of the choice in registers; the LDS of a launch
+@pytest.mark.parametrize("n,width,experts,top", [(9, 520, 34, 4), (16, 3072, 68, 8), (17, 3072, 68, 8), (16, 264, 64, 16), (3, 264, 64, 17), (16, 264, 128, 16),
+                                                 (7, 264, 128, 17), (13, 264, 129, 16), (16, 64, 482, 8), (16, 64, 483, 8), (12, 64, 480, 12), (1, 64, 491, 8)])
+@pytest.mark.parametrize("scoring", ["sigmoid", "softmax_chosen", "softmax_all", "sigmoid_plain", "softmax_groups"])
+def test_choices_at_the_edges_of_the_one_launch_are_those_of_two_calls(n, width, experts, top, scoring):
+    _the_same_as_two_calls(n, width, experts, top, scoring, torch.bfloat16)
 
 
 @pytest.mark.parametrize("n,width,experts,top,groups,keep", [(1, 520, 64, 4, 8, 2), (9, 264, 32, 5, 4, 3), (16, 264, 256, 8, 8, 4), (17, 264, 64, 4, 8, 2)])
