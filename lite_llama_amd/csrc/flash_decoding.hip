@@ -1155,12 +1155,9 @@ static int launch_fd(void* out, const void* q, const void* kc, const void* vc, c
   {                                                                                                  \
     constexpr int tile_bytes_ = 32 * (DD + 8) * 2;                                                   \
     if (GR) {                                                                                        \
-      static bool attr_ = false;                                                                     \
-      if (!attr_) {                                                                                  \
-        (void)hipFuncSetAttribute((const void*)fd_stage1<DT, DD, FU, RO, GG, GR, K8, QN, QI, WH>,             \
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, FD_GROUP_MAX * tile_bytes_ + 18 * DD * 2); \
-        attr_ = true;                                                                                \
-      }                                                                                              \
+      static std::atomic<uint64_t> asked_{0};                                                        \
+      if (!ll_wide_lds((const void*)fd_stage1<DT, DD, FU, RO, GG, GR, K8, QN, QI, WH>, FD_GROUP_MAX * tile_bytes_ + 18 * DD * 2, asked_)) \
+        return LL_ERR_LAUNCH;                                                                        \
     }                                                                                                \
     fd_stage1<DT, DD, FU, RO, GG, GR, K8, QN, QI, WH><<<(GR) ? dim3((unsigned)plan.splits, grid.y, grid.z) : grid, (GR) ? 64 * gw : 64, \
                                         ((GR) ? gw : 1) * tile_bytes_ + ((GR) ? 18 * DD * 2 : 0), st>>>( \

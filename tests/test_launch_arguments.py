@@ -26,8 +26,11 @@ hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* s, hipStream_t* s
   *g = cfg_grid; *b = cfg_block; *s = cfg_lds; *st = nullptr;
   return hipSuccess;
 }
-hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
-hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return hipSuccess; }
+static int on_device = 0, asked_on[4];
+hipError_t hipGetDevice(int* d) { *d = on_device; return hipSuccess; }
+hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { ++asked_on[on_device]; return hipSuccess; }
+void use_device(int d) { on_device = d; }
+int attributes_asked(int d) { return asked_on[d]; }
 hipError_t hipGetLastError() { return hipSuccess; }
 hipError_t hipPeekAtLastError() { return hipSuccess; }
 }
@@ -155,6 +158,18 @@ def test_a_long_row_is_spread_whatever_stands_beside_it(flash_decoding, tokens, 
         assert pairs * splits >= min(160, pairs * min(32, np_ // 2))  # .. and most CUs have a workgroup
         planes = _plan(flash_decoding, tokens, pairs, heads, planes=True)
         assert planes[0] >= 4 and planes[1] >= 1                      # (18 rows of a head fit the planes' two pieces per lane)
+
+
+def test_more_lds_than_a_launch_has_is_asked_for_on_every_device(flash_decoding):
+    """Eight waves of decode attention hold 74 KB: granted to a kernel on the device that is current, and no other."""
+    P, L, I, F = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_float
+    flash_decoding.ll_flash_decoding.argtypes = [P] * 9 + [I, I, I, I, L, F] + [L] * 9 + [I, I, I, P, P]
+    for device in (0, 1, 1, 0):
+        flash_decoding.use_device(device)
+        before = flash_decoding.attributes_asked(device)
+        assert flash_decoding.ll_flash_decoding(*[4096] * 9, 2, 16, 1, 128, 1024, 0.1, *[2048, 128] * 4, 64, 1, 0, 0, 4096, None) == 0
+        assert flash_decoding.attributes_asked(device) >= 1 and before <= flash_decoding.attributes_asked(device) <= 1
+    flash_decoding.use_device(0)
 
 
 def test_decode_plans_of_other_calls(flash_decoding):
